@@ -7,6 +7,7 @@ those stages in the reference are the identity at world size 1.  Here each matri
 streaming passes over its memory: the error add is fused into the first product, the residual
 (dense, or count-sketched) into the last.
 """
+import ctypes
 import logging
 import os
 
@@ -42,7 +43,6 @@ def orthogonalize_all(matrices, epsilon, ws_ptr, ws_len, stream, table=None):
     """Gram-Schmidt of independent [rows, r] device matrices, side by side in as few launches as
     their shapes allow.  ``table``: what an earlier call over the same matrices returned (the host
     arrays are reused while the matrices stay where they are); returns the table."""
-    import ctypes
     count = len(matrices)
     if count == 0:
         return None
@@ -65,7 +65,6 @@ def gram_schmidt_give_ups():
     resident together; with several hook streams busy that is an assumption, and this is where its
     failure shows before the NaN reaches a gradient.  Waits for the device.  With CONEF_CHECK_GS=1
     every hook call ends with this check and raises."""
-    import ctypes
     count = ctypes.c_int64(0)
     _lib.check(_lib.load().conef_gram_schmidt_give_ups(ctypes.byref(count)), "conef_gram_schmidt_give_ups")
     return count.value
@@ -97,7 +96,6 @@ def topk_sparsify_all(tensors, topk_ratio, table=None, stream=None):
     single launch over all of them.  ``table`` is what an earlier call over the same tensors
     returned: the host arrays and the workspace are reused while the tensors stay where they are.
     ``stream``: the raw stream to launch on (torch's current one if None)."""
-    import ctypes
     count = len(tensors)
     if count == 0:
         return table
@@ -129,14 +127,46 @@ class _RoundPlan:
     and layout, so that a step costs a handful of foreign calls however many tensors it has."""
     __slots__ = ("small", "sig", "errs_sig", "cs_static", "env_ahead", "env_topk_side", "env_small", "key", "shapes", "work", "passthrough", "before", "after", "total_ps", "total_qs", "arena_key", "ps",
                  "qs", "items", "count", "sketches", "fused_sketch", "batched_update", "residual_offsets",
-                 "topk_table", "q_next", "q_next_ptrs", "q_next_ready", "made", "q_next_views", "items_next", "q_next_event",
-                 "topk_event", "ws_need", "handoff_event", "gs_table", "topk_number", "q_next_number", "is_wide", "wide")
+                 "topk_table", "q_next", "q_next_ptrs", "q_next_ready", "made", "q_next_event",
+                 "topk_event", "ws_need", "handoff_event", "topk_number", "q_next_number", "is_wide", "wide", "chunks", "ef_spans")
 
 
 def _layout_signature(grads):
     """What a step compares instead of every tensor's shape: a bucket keeps its buffer, its length
     (both part of the plan's key) and its parameters for as long as DDP keeps the bucket."""
     return (len(grads), grads[0].shape, grads[-1].shape) if grads else (0, None, None)
+
+
+BATCH_ITEMS = 24        # matrices the batch entry points take into one launch
+
+
+def _chunks(count):
+    """A bucket's matrices as runs of at most BATCH_ITEMS of about the same length: (first, how many)."""
+    parts = -(-count // BATCH_ITEMS)
+    return [(count * i // parts, count * (i + 1) // parts - count * i // parts) for i in range(parts)]
+
+
+def _ef_spans(plan, base_ptr, err_ptr):
+    """The stretches of a bucket that are not compressed, neighbours joined, as the host arrays
+    ``conef_ef_passthrough_batch_f32`` reads: (x pointers, error pointers, element counts, how many)."""
+    runs = []
+    for tensor in sorted(plan.passthrough, key=lambda t: t.data_ptr()):
+        at, numel = tensor.data_ptr(), tensor.numel()
+        if numel == 0:
+            continue
+        if runs and runs[-1][0] + 4 * runs[-1][1] == at:
+            runs[-1][1] += numel
+        else:
+            runs.append([at, numel])
+    n = len(runs)
+    return ((ctypes.c_void_p * n)(*[at for at, _ in runs]),
+            (ctypes.c_void_p * n)(*[err_ptr + (at - base_ptr) for at, _ in runs]),
+            (ctypes.c_int64 * n)(*[c for _, c in runs]), n)
+
+
+def _rank_bound(rank):
+    """Floats in a row of the library's own copy of a rank-r factor (ranks above 32 have none)."""
+    return 1 << max(rank - 1, 0).bit_length()
 
 
 def _build_round(state, grads, shapes, key, error_mode):
@@ -184,13 +214,15 @@ def _build_round(state, grads, shapes, key, error_mode):
     plan.q_next_number = None       # likewise for the Gram-Schmidt of the next round's Q factors
     plan.ws_need = None             # bytes of workspace the batch entry points ask for (a function of the table's shapes)
     plan.handoff_event = None       # recorded on the hook's stream where the side stream may start (one event, reused)
-    plan.gs_table = None            # host arrays of the side stream's Gram-Schmidt call
     # Second buffer for the Q factors, orthogonalised at the end of a round for the bucket's next
     # round (conef_psgd_round_ahead_f32).  Derived data: q_memory_dict keeps what the reference
     # keeps, and the flag falls with the plan whenever the state is replaced.
     plan.q_next = plan.q_next_ptrs = None
     plan.q_next_ready = False
     plan.made = None
+    plan.q_next_event = None
+    plan.chunks = _chunks(plan.count)
+    plan.ef_spans = None            # dense error feedback: host arrays of the stretches that are not compressed
     plan.residual_offsets = []
     off = 0
     for _, n, m, _ in plan.work:
@@ -404,7 +436,9 @@ def _run_round(state, bucket, error_mode, streams=1):
     wait_for_side_topk(plan, device, lambda: _lib.current_stream(device))
     eps = float(state.orthogonalization_epsilon)
     if plan.ws_need is None:
-        plan.ws_need = plan.wide.ws_need if plan.is_wide else max(lib.conef_psgd_batch_workspace_bytes(items, count), 256)
+        plan.ws_need = plan.wide.ws_need if plan.is_wide else max(
+            [lib.conef_psgd_batch_workspace_bytes(_at(items, first), part)
+             for first, part in plan.chunks] + [256])
     ws = _workspace(device, stream, plan.ws_need)
     ws_ptr, ws_len = ws.data_ptr(), ws.numel()
     if need_randomize_qs:
@@ -421,11 +455,11 @@ def _run_round(state, bucket, error_mode, streams=1):
             errs[cnt].query(matrix.view(m, n), alpha)
     if error_mode == "ef":
         # tensors that are not compressed: g += e, and their new error is exactly zero (:361,:558)
-        for tensor in plan.passthrough:
-            off = (tensor.data_ptr() - base_ptr) // 4
-            cnt_el = tensor.numel()
-            rc = lib.conef_ef_passthrough_f32(tensor.data_ptr(), dense_err.data_ptr() + 4 * off, cnt_el, stream)
-            _lib.check(rc, "conef_ef_passthrough_f32")
+        if plan.ef_spans is None:
+            plan.ef_spans = _ef_spans(plan, base_ptr, dense_err.data_ptr())
+        if plan.ef_spans[3]:
+            rc = lib.conef_ef_passthrough_batch_f32(*plan.ef_spans, stream)
+            _lib.check(rc, "conef_ef_passthrough_batch_f32")
 
     # The round itself, one foreign call: orthogonalise all Q side by side; pass 1, the error add
     # fused into P = M Q; orthogonalise all P; pass 2, Q = M^T P; pass 3, M = P Q^T with the
@@ -464,52 +498,51 @@ def _run_round(state, bucket, error_mode, streams=1):
     elif plan.small is None or plan.small[0] != (mode1, mode3):
         # a bucket of small matrices (every one fits a workgroup's LDS with its factors): the whole round in one launch
         fits = bool(count and mode3 in (0, 1, 2) and plan.env_small
-                    and lib.conef_psgd_round_small_fits(items, count, mode1, mode3, HASH_A, HASH_B))
+                    and all(lib.conef_psgd_round_small_fits(_at(items, first), part, mode1, mode3, HASH_A, HASH_B)
+                            for first, part in plan.chunks))
         plan.small = ((mode1, mode3), fits)
+    beta3 = float(state.beta) if mode3 in (2, 3) else 0.0
     if plan.is_wide:
         pass
     elif plan.small[1]:
         plan.q_next_ready = False
-        rc = lib.conef_psgd_round_small_f32(items, count, mode1, mode3, float(alpha), float(state.beta) if mode3 == 2 else 0.0,
-                                            eps, HASH_A, HASH_B, ws_ptr, ws_len, stream)
-        _lib.check(rc, "conef_psgd_round_small_f32")
-    elif (state.matrix_approximation_rank > 8 and state.warm_start and count
-            and streams <= 1 and plan.env_ahead):
-        # Ranks on the matrix cores: the round as its separate launches, with the Gram-Schmidt of the new
-        # Q factors (which the reference runs at the start of the bucket's next round,
-        # powerSGD_hook.py:496-497: 27-35 us of dependent steps on a few workgroups) on a side stream,
-        # out of place, while this stream goes on with M = P Q^T and the sketch update.  The next round
-        # of this bucket waits for it.  CONEF_ROUND_AHEAD=0 keeps everything on one stream; so does
-        # hook_streams > 1, where buckets already run side by side (measured: the two together are slower).
-        _round_with_q_on_the_side(state, plan, lib, items, count, mode1, mode3, alpha, eps, ws_ptr, ws_len, stream,
-                                  device, q_mem, qs)
-    elif (mode3 in (0, 1, 2) and state.matrix_approximation_rank <= 8 and state.warm_start and count and count <= 24
-            and plan.env_ahead):
+        for first, part in plan.chunks:
+            rc = lib.conef_psgd_round_small_f32(_at(items, first), part, mode1, mode3, float(alpha), beta3, eps, HASH_A, HASH_B,
+                                                ws_ptr, ws_len, stream)
+            _lib.check(rc, "conef_psgd_round_small_f32")
+    elif count and state.warm_start and plan.env_ahead and (state.matrix_approximation_rank > 8 or mode3 in (0, 1, 2)):
         # The bucket's next round starts by orthogonalising the Q factors this round leaves
-        # (powerSGD_hook.py:496-497): a few workgroups and an idle machine.  Workgroups of this
-        # round's last launch do it instead, into a second buffer, where the kernel allows
-        # (CONEF_ROUND_AHEAD=0 keeps the reference's order, for comparisons).
-        import ctypes
+        # (powerSGD_hook.py:496-497): a few workgroups and an idle machine.  It is done at the end of
+        # this round instead, into a second buffer: by workgroups of the last launch at ranks up to 8, by
+        # short launches of their own above (CONEF_ROUND_AHEAD=0 keeps the reference's order, for
+        # comparisons).  Where the buckets do not run side by side (one stream), those launches go to a side
+        # stream, which the bucket's next round waits for, and overlap the next bucket.
         if plan.q_next is None:
-            plan.q_next = torch.empty_like(q_mem)
-            offs, off = [], 0
+            plan.q_next = torch.empty(sum(m * _rank_bound(rank) for _, _, m, rank in work), device=device, dtype=dtype)
+            at, ptrs = plan.q_next.data_ptr(), []
             for _, n, m, rank in work:
-                offs.append(off)
-                off += m * rank
-            plan.q_next_ptrs = (ctypes.c_void_p * count)(*[plan.q_next.data_ptr() + 4 * o for o in offs])
-            plan.made = ctypes.c_int32(0)
+                ptrs.append(at)
+                at += 4 * m * _rank_bound(rank)
+            plan.q_next_ptrs = (ctypes.c_void_p * count)(*ptrs)
+            plan.made = [ctypes.c_int32(0) for _ in plan.chunks]
             plan.q_next_ready = False
-        flags = (1 if plan.q_next_ready else 0) | 2
-        rc = lib.conef_psgd_round_ahead_f32(items, count, mode1, mode3, float(alpha), float(state.beta) if mode3 == 2 else 0.0, eps, HASH_A,
-                                            HASH_B, plan.q_next_ptrs, flags, ctypes.byref(plan.made), ws_ptr, ws_len,
-                                            stream)
-        _lib.check(rc, "conef_psgd_round_ahead_f32")
-        plan.q_next_ready = bool(plan.made.value)
+        aside = state.matrix_approximation_rank > 8 and streams <= 1
+        if aside and plan.q_next_ready:
+            _pools.side_wait(device, _lib.current_stream(device), plan.q_next_number)
+        flags = (1 if plan.q_next_ready else 0) | (0 if aside else 2)
+        for (first, part), made in zip(plan.chunks, plan.made):
+            rc = lib.conef_psgd_round_ahead_f32(_at(items, first), part, mode1, mode3, float(alpha), beta3, eps, HASH_A, HASH_B,
+                                                _at(plan.q_next_ptrs, first), flags, ctypes.byref(made), ws_ptr, ws_len, stream)
+            _lib.check(rc, "conef_psgd_round_ahead_f32")
+        plan.q_next_ready = all(made.value for made in plan.made)
+        if aside:
+            _orthogonalise_q_aside(plan, lib, items, eps, ws_len, device)
     else:
         plan.q_next_ready = False
-        rc = lib.conef_psgd_round_f32(items, count, mode1, mode3, float(alpha), float(state.beta) if mode3 in (2, 3) else 0.0,
-                                      eps, HASH_A, HASH_B, ws_ptr, ws_len, stream)
-        _lib.check(rc, "conef_psgd_round_f32")
+        for first, part in plan.chunks:
+            rc = lib.conef_psgd_round_f32(_at(items, first), part, mode1, mode3, float(alpha), beta3, eps, HASH_A, HASH_B,
+                                          ws_ptr, ws_len, stream)
+            _lib.check(rc, "conef_psgd_round_f32")
     if error_mode == "topk":
         if count and streams <= 1 and plan.env_ahead and plan.env_topk_side:
             # The sparsification only touches the error tensors, which nobody reads before this bucket's
@@ -554,55 +587,30 @@ def _run_round(state, bucket, error_mode, streams=1):
     return _bucket.completed_future(input_tensor)
 
 
-def _round_with_q_on_the_side(state, plan, lib, items, count, mode1, mode3, alpha, eps, ws_ptr, ws_len, stream, device,
-                              q_mem, qs):
-    import ctypes
-    main = _lib.current_stream(device)
-    fresh_q_next = plan.q_next is None
-    if fresh_q_next:
-        plan.q_next = torch.empty_like(q_mem)
-        plan.q_next_views, off = [], 0
-        for q in qs:
-            plan.q_next_views.append(plan.q_next[off: off + q.numel()].view(q.shape))
-            off += q.numel()
-        plan.items_next = (type(items[0]) * count)()      # the same table with the first product reading the second buffer
-        plan.q_next_event = torch.cuda.Event()
-        plan.q_next_ready = False
-    if plan.q_next_ready:
-        for k in range(count):                              # pointers of the table can move between steps (err, cs)
-            ctypes.memmove(ctypes.byref(plan.items_next[k]), ctypes.byref(items[k]), ctypes.sizeof(items[k]))
-            plan.items_next[k].q = plan.q_next_views[k].data_ptr()
-        _pools.side_wait(device, main, plan.q_next_number)
-        first = plan.items_next
-    else:
-        orthogonalize_all(qs, eps, ws_ptr, ws_len, stream)
-        first = None
-    # P = M Q, P orthogonalised, Q = M^T P
-    rc = lib.conef_psgd_products_f32(items, first, count, mode1, float(alpha), eps, HASH_A, HASH_B, ws_ptr, ws_len, stream)
-    _lib.check(rc, "conef_psgd_products_f32")
-    # the new Q is final: orthogonalise a copy of it on the side
+def _at(array, index):
+    """The ctypes array from entry ``index`` on, as an argument."""
+    return ctypes.byref(array, index * ctypes.sizeof(array._type_))
+
+
+def _orthogonalise_q_aside(plan, lib, items, eps, ws_len, device):
+    """The new Q factors of a bucket orthogonalised for its next round on the side stream."""
     if plan.handoff_event is None:
         plan.handoff_event = torch.cuda.Event()
-    plan.handoff_event.record(main)
+    plan.handoff_event.record(_lib.current_stream(device))
     side = _pools.side_stream(device, 0, 1)
     side.wait_event(plan.handoff_event)
-    if fresh_q_next:
+    if plan.q_next_event is None:
+        plan.q_next_event = torch.cuda.Event()
         plan.q_next.record_stream(side)       # memory the side stream works on must not go back to the allocator under it
     with _lib.on_stream(side):
-        plan.q_next.copy_(q_mem, non_blocking=True)
-        side_ws = _workspace(device, side.cuda_stream, max(ws_len, 256))
-    plan.gs_table = orthogonalize_all(plan.q_next_views, eps, side_ws.data_ptr(), side_ws.numel(), side.cuda_stream,
-                                      plan.gs_table)
+        ws = _workspace(device, side.cuda_stream, max(ws_len, 256))
+    for (first, part), made in zip(plan.chunks, plan.made):
+        rc = lib.conef_psgd_q_next_f32(_at(items, first), part, eps, _at(plan.q_next_ptrs, first), ctypes.byref(made),
+                                       ws.data_ptr(), ws.numel(), side.cuda_stream)
+        _lib.check(rc, "conef_psgd_q_next_f32")
     plan.q_next_event.record(side)
     plan.q_next_number = _pools.side_recorded(device, plan.q_next_event)
-    plan.q_next_ready = True
-    beta = float(state.beta) if mode3 in (2, 3) else 0.0
-    rc = lib.conef_psgd_pqt_batch_f32(items, count, 1 if mode3 == 3 else mode3, beta if mode3 == 2 else 0.0, HASH_A, HASH_B,
-                                      stream)
-    _lib.check(rc, "conef_psgd_pqt_batch_f32")
-    if mode3 == 3:
-        rc = lib.conef_psgd_sketch_update_batch_f32(items, count, beta, HASH_A, HASH_B, stream)
-        _lib.check(rc, "conef_psgd_sketch_update_batch_f32")
+    plan.q_next_ready = all(made.value for made in plan.made)
 
 
 def run_batched_round(state, bucket):

@@ -32,6 +32,47 @@ inline hipError_t conef_allow_lds(const void* kernel, size_t bytes)
     return e;
 }
 
+// ---------------------------------------------------------- 16-byte accesses ----
+// Four consecutive words from any 4-byte aligned address: global memory takes 16-byte accesses at
+// word alignment (a row of 650 floats, a view that starts 40 bytes into a bucket), at worst one more
+// cache line each.  LDS does not, and keeps its aligned accesses.
+typedef float conef_f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float conef_f2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t conef_u4u __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ void conef_ld4u(const float* p, float* v)
+{
+    const conef_f4u t = *reinterpret_cast<const conef_f4u*>(p);
+    v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+}
+__device__ __forceinline__ void conef_ld4u(const uint32_t* p, uint32_t* v)
+{
+    const conef_u4u t = *reinterpret_cast<const conef_u4u*>(p);
+    v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+}
+__device__ __forceinline__ void conef_st4u(float* p, const float* v)
+{
+    conef_f4u t = {v[0], v[1], v[2], v[3]};
+    *reinterpret_cast<conef_f4u*>(p) = t;
+}
+
+// Rows cut into column quads when their length is not a multiple of four: the last quad is moved
+// back to end with the row, so that it stays inside, and its first `dup` columns are the previous
+// quad's.  Whoever owns it ignores them (they are never stored and never counted).
+__device__ __forceinline__ int conef_quad_col(int quad, int m) { return 4 * quad + 4 <= m ? 4 * quad : m - 4; }
+
+// Stores the columns of a quad that are its own.
+__device__ __forceinline__ void conef_st4_own(float* p, const float* v, int dup)
+{
+    if (dup == 0) {
+        conef_st4u(p, v);
+    } else {
+#pragma unroll
+        for (int k = 1; k < 4; ++k)
+            if (k >= dup) p[k] = v[k];
+    }
+}
+
 // ------------------------------------------------------------------ hash ----
 // Integer mixer of the count sketch (reference: communication/compressors/CountSketch.py:7-18).
 // The reference's `h` is a signed int, so all three shifts are arithmetic; the last one always

@@ -35,19 +35,17 @@ constexpr int kMaxRank = 32;
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-__device__ __forceinline__ void ld4(const float* p, float* v)
-{
-    float4 t = *reinterpret_cast<const float4*>(p);
-    v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
-}
-__device__ __forceinline__ void st4(float* p, const float* v)
+__device__ __forceinline__ void ld4(const float* p, float* v) { conef_ld4u(p, v); }
+__device__ __forceinline__ void st4(float* p, const float* v) { conef_st4u(p, v); }
+__device__ __forceinline__ void st4_lds(float* p, const float* v)          // 16-byte aligned
 {
     *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
 }
 
-// All kernels come in a FAST form (r equals the compile-time rank bound RP, m % 4 == 0, every
-// pointer 16-byte aligned: 16-byte accesses, Q rows of a column quad are one contiguous run) and a
-// general form (any r <= RP, any alignment, 4-byte accesses).
+// All kernels come in a FAST form (r equals the compile-time rank bound RP, rows of at least four
+// columns of any alignment: 16-byte accesses, Q rows of a column quad are one contiguous run) and a
+// general form (any r <= RP, 4-byte accesses).  A round of the hooks at a rank between two bounds
+// works on copies of the factors with rows of RP floats (PaddedRound) and takes the FAST forms too.
 
 // ------------------------------------------------------------ batched launches ----
 // A gradient bucket holds several matrices whose products are independent of each other, and most
@@ -106,7 +104,7 @@ psgd_mq_body(float* __restrict__ x, const float* __restrict__ err, const float* 
         for (int c = 0; c < RP; ++c) acc[a][c] = 0.f;
 
     if (FAST) {
-        const int m4 = m >> 2;
+        const int m4 = (m + 3) >> 2;
         // column quads in flight per thread, at most: registers for more of them cost more in
         // resident waves than the extra loads in flight bring
         constexpr int UMAX = (RB * RP <= 16) ? 2 : 1;
@@ -122,22 +120,27 @@ psgd_mq_body(float* __restrict__ x, const float* __restrict__ err, const float* 
 #pragma unroll
             for (int u = 0; u < U; ++u) {               // past the last quad: a valid address, result unused
                 const int j = j0 + u * 256 < m4 ? j0 + u * 256 : m4 - 1;
+                const int col = conef_quad_col(j, m), dup = 4 * j - col;
 #pragma unroll
-                for (int a = 0; a < RB; ++a) ld4(x + rowc[a] * m + 4 * j, xv[u][a]);
+                for (int a = 0; a < RB; ++a) ld4(x + rowc[a] * m + col, xv[u][a]);
 #pragma unroll
-                for (int t = 0; t < RP; ++t) ld4(q + (int64_t)j * 4 * RP + 4 * t, qf[u] + 4 * t);
+                for (int t = 0; t < RP; ++t) ld4(q + (int64_t)col * RP + 4 * t, qf[u] + 4 * t);
+                if (dup) {                              // the previous quad's columns add nothing here
+#pragma unroll
+                    for (int t = 0; t < 4 * RP; ++t)
+                        if (t / RP < dup) qf[u][t] = 0.f;
+                }
                 if (MODE == 1) {
 #pragma unroll
-                    for (int a = 0; a < RB; ++a) ld4(err + rowc[a] * m + 4 * j, ev[u][a]);
+                    for (int a = 0; a < RB; ++a) ld4(err + rowc[a] * m + col, ev[u][a]);
                 }
                 if (MODE == 2) {
                     if (pktab) {
-                        uint4 t = reinterpret_cast<const uint4*>(pktab)[j];
-                        pk[u][0] = t.x; pk[u][1] = t.y; pk[u][2] = t.z; pk[u][3] = t.w;
+                        conef_ld4u(pktab + col, pk[u]);
                     } else {
 #pragma unroll
                         for (int k = 0; k < 4; ++k)
-                            pk[u][k] = conef_bucket_sign(4 * j + k, mod, hs.a, hs.b, hs.sa, hs.sb);
+                            pk[u][k] = conef_bucket_sign(col + k, mod, hs.a, hs.b, hs.sa, hs.sb);
                     }
                 }
             }
@@ -145,12 +148,13 @@ psgd_mq_body(float* __restrict__ x, const float* __restrict__ err, const float* 
             for (int u = 0; u < U; ++u) {
                 const int j = j0 + u * 256;
                 if (j >= m4) break;
+                const int col = conef_quad_col(j, m), dup = 4 * j - col;
                 if (MODE == 1) {
 #pragma unroll
                     for (int a = 0; a < RB; ++a) {
 #pragma unroll
                         for (int k = 0; k < 4; ++k) xv[u][a][k] = __fadd_rn(xv[u][a][k], ev[u][a][k]);
-                        if (row0 + a < n) st4(x + rowc[a] * m + 4 * j, xv[u][a]);
+                        if (row0 + a < n) conef_st4_own(x + rowc[a] * m + col, xv[u][a], dup);
                     }
                 } else if (MODE == 2) {
 #pragma unroll
@@ -159,7 +163,7 @@ psgd_mq_body(float* __restrict__ x, const float* __restrict__ err, const float* 
                         for (int k = 0; k < 4; ++k)
                             xv[u][a][k] = __fadd_rn(xv[u][a][k], conef_query_term(cells[a * w + (pk[u][k] & 0x7fffffffu)],
                                                                                    pk[u][k], alpha));
-                        if (row0 + a < n) st4(x + rowc[a] * m + 4 * j, xv[u][a]);
+                        if (row0 + a < n) conef_st4_own(x + rowc[a] * m + col, xv[u][a], dup);
                     }
                 }
 #pragma unroll
@@ -272,13 +276,17 @@ psgd_mtp_body(const float* __restrict__ x, const float* __restrict__ p, float* _
     for (int k = 0; k < 4; ++k)
 #pragma unroll
         for (int c = 0; c < RP; ++c) acc[k][c] = 0.f;
+    // FAST: the quad that would end past the row is moved back to end with it; its first `dup` columns
+    // are the previous lane's.  Lanes past the edge load the last quad, results unused.
+    int dup = 0;
     if (FAST) {
-        const int cc = c0 < m ? c0 : m - 4;         // clamped: lanes past the edge load a valid quad, results unused
+        const int cc = c0 + 4 <= m ? c0 : m - 4;
+        dup = c0 < m ? c0 - cc : 0;
         int64_t i = i0 + wave;
         for (; i + 3 * kMtpWaves < i1; i += 4 * kMtpWaves) {      // four rows in flight
             float xv[4][4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) ld4(x + (i + u * kMtpWaves) * m + cc, xv[u]);
+            for (int u = 0; u < 4; ++u) conef_ld4u(x + (i + u * kMtpWaves) * m + cc, xv[u]);
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const float* pi = p + (i + u * kMtpWaves) * RP;
@@ -292,7 +300,7 @@ psgd_mtp_body(const float* __restrict__ x, const float* __restrict__ p, float* _
         }
         for (; i < i1; i += kMtpWaves) {
             float xv[4];
-            ld4(x + i * m + cc, xv);
+            conef_ld4u(x + i * m + cc, xv);
             const float* pi = p + i * RP;
 #pragma unroll
             for (int c = 0; c < RP; ++c) {
@@ -322,7 +330,8 @@ psgd_mtp_body(const float* __restrict__ x, const float* __restrict__ p, float* _
 #pragma unroll
         for (int c = 0; c < CH; ++c)
 #pragma unroll
-            for (int k = 0; k < 4; ++k) red[wave][c][lane * 4 + k] = acc[k][cb + c];
+            for (int k = 0; k < 4; ++k)
+                if (k >= dup) red[wave][c][lane * 4 + k - dup] = acc[k][cb + c];
         __syncthreads();
         if (threadIdx.x < 256) {
             const int col = bx * 256 + threadIdx.x;
@@ -426,7 +435,7 @@ struct GramTask {
     const double* parts[kPsgdBatchMax];   // [nparts][RP (RP + 1) / 2]
     int nparts[kPsgdBatchMax];
     float* tmat[kPsgdBatchMax];           // out: b_ij row-major [RP][RP] (zero unless i < j), then 1 / d_i [RP]
-    int count;
+    int count, r;                         // r: the rank; columns from r on are zeros and their steps mean nothing
     float eps;
 };
 
@@ -591,7 +600,7 @@ __device__ __forceinline__ void store_row(float* p, const float* x)
 template <int RP, int T>
 __device__ __forceinline__ void
 gram_orthogonalise_body(const float* __restrict__ src, float* __restrict__ dst, int rows, const double* parts, int nparts,
-                        float eps)
+                        int r, float eps)
 {
     __shared__ float t_l[RP * RP + RP];
     gram_solve_lds<RP, T>(parts, nparts, eps, t_l);
@@ -606,6 +615,11 @@ gram_orthogonalise_body(const float* __restrict__ src, float* __restrict__ dst, 
         for (int u = 0; u < 4; ++u) {
             const int row = r0 + u * T;
             gram_apply_row<RP>(x[u], t_l);
+            if (r < RP) {
+#pragma unroll
+                for (int c = 0; c < RP; ++c)
+                    if (c >= r) x[u][c] = 0.f;
+            }
             if (row < rows) store_row<RP>(dst + (int64_t)row * RP, x[u]);
         }
     }
@@ -639,7 +653,21 @@ struct DeferFixItem {
     int64_t n, m;
     int slabs;
     int pblocks;             // workgroups that take rows of P; the others take rows of Q
+    // A rank r below RP: p, qsrc and q hold rows of RP floats with zeros behind the first r, and the
+    // factors the caller keeps, rows of r floats, are written here (null: r is RP, p and q are those).
+    float* pt;
+    float* qt;
+    int r;
 };
+
+// A finished row (P or Q, zeros from column r on) into the caller's [rows, r] factor.
+template <int RP>
+__device__ __forceinline__ void store_tight_row(float* dst, int64_t row, const float* x, int r)
+{
+#pragma unroll
+    for (int c = 0; c < RP; ++c)
+        if (c < r) dst[row * r + c] = x[c];
+}
 
 template <int RP>
 __global__ void __launch_bounds__(256)
@@ -680,6 +708,12 @@ psgd_defer_fix_batch_kernel(PsgdBatch<DeferFixItem> b)
     }
     __syncthreads();
     gram_apply_row<RP>(x, t_l);
+    if (it.pt) {                     // the steps of columns that are not there divide by zero
+#pragma unroll
+        for (int c = 0; c < RP; ++c)
+            if (c >= it.r) x[c] = 0.f;
+        if (row < rows) store_tight_row<RP>(is_p ? it.pt : it.qt, row, x, it.r);
+    }
     if (row < rows) store_row<RP>((is_p ? it.p : it.q) + row * RP, x);
     if (!is_p && it.qgram) {                                // uniform over the workgroup
 #pragma unroll
@@ -784,7 +818,7 @@ psgd_defer_fix_wide_batch_kernel(PsgdBatch<DeferFixItem> b)
         float acc = 0.f;
 #pragma unroll 8
         for (int i = 0; i < RP; ++i) acc = fmaf(rows_l[lr][i], t_l[i * RP + col], acc);      // T is zero below the diagonal
-        out[u] = acc;
+        out[u] = col < it.r ? acc : 0.f;
     }
     __syncthreads();
 #pragma unroll
@@ -795,6 +829,12 @@ psgd_defer_fix_wide_batch_kernel(PsgdBatch<DeferFixItem> b)
 #pragma unroll
         for (int c = 0; c < 4; ++c) o[c] = rows_l[lrow][4 * piece + c];
         st4((is_p ? it.p : it.q) + row * RP + 4 * piece, o);
+        if (it.pt) {
+            float* dst = (is_p ? it.pt : it.qt) + row * it.r + 4 * piece;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (4 * piece + c < it.r) dst[c] = o[c];
+        }
     }
 }
 
@@ -864,6 +904,14 @@ psgd_mfma_mtp_gram_batch_kernel(PsgdBatch<MfmaMtpItem> b, GramTask g)
     else psgd_mfma_mtp_body<1>(it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, ct, slab);
 }
 
+// the Gram systems alone (ranks 9 to 32): a workgroup a matrix
+template <int RP>
+__global__ void __launch_bounds__(kMfmaThreads)
+psgd_gram_solve_batch_kernel(GramTask g)
+{
+    gram_solve_body<RP, kMfmaThreads, true>(g.parts[blockIdx.x], g.nparts[blockIdx.x], g.tmat[blockIdx.x], g.eps);
+}
+
 struct MfmaPqtItem {
     float* x;
     float* err;
@@ -885,7 +933,7 @@ psgd_mfma_pqt_batch_kernel(PsgdBatch<MfmaPqtItem> b)
 
 // X += alpha * unsketch(cs) over the matrices of a bucket (DenseCS.query, CountSketch.py:51-66):
 // a thread owns a column quad of a group of rows, its (bucket, sign) words from the plan's table
-// or hashed, once for the group.  VEC: m % 4 == 0 and 16-byte aligned x (and table).
+// or hashed, once for the group.  Rows of at least four columns, any alignment.
 struct QueryItem {
     float* x;
     const float* cs;
@@ -895,7 +943,6 @@ struct QueryItem {
     ConefMod mod;
 };
 
-template <bool VEC>
 __global__ void __launch_bounds__(256)
 psgd_cs_query_batch_kernel(PsgdBatch<QueryItem> b, float alpha, ConefSeeds hs)
 {
@@ -904,34 +951,25 @@ psgd_cs_query_batch_kernel(PsgdBatch<QueryItem> b, float alpha, ConefSeeds hs)
     const int bx = local % it.col_blocks, by = local / it.col_blocks;
     const int c0 = (bx * 256 + (int)threadIdx.x) * 4;
     if (c0 >= it.m) return;
+    const int col = conef_quad_col(c0 >> 2, it.m), dup = c0 - col;
     uint32_t pk[4];
-    if (VEC && it.pktab) {
-        const uint4 t = *reinterpret_cast<const uint4*>(it.pktab + c0);
-        pk[0] = t.x; pk[1] = t.y; pk[2] = t.z; pk[3] = t.w;
+    if (it.pktab) {
+        conef_ld4u(it.pktab + col, pk);
     } else {
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-            pk[k] = c0 + k < it.m ? (it.pktab ? it.pktab[c0 + k] : conef_bucket_sign(c0 + k, it.mod, hs.a, hs.b, hs.sa, hs.sb))
-                                  : 0u;
+        for (int k = 0; k < 4; ++k) pk[k] = conef_bucket_sign(col + k, it.mod, hs.a, hs.b, hs.sa, hs.sb);
     }
     const int64_t r0 = (int64_t)by * it.rows_per_block;
     const int64_t r1 = r0 + it.rows_per_block < it.n ? r0 + it.rows_per_block : it.n;
     const int w = (int)it.mod.w;
     for (int64_t r = r0; r < r1; ++r) {
         const float* row = it.cs + r * w;
-        float* xr = it.x + r * it.m + c0;
-        if (VEC) {
-            float4 v = *reinterpret_cast<const float4*>(xr);
-            v.x = __fadd_rn(v.x, conef_query_term(row[pk[0] & 0x7fffffffu], pk[0], alpha));
-            v.y = __fadd_rn(v.y, conef_query_term(row[pk[1] & 0x7fffffffu], pk[1], alpha));
-            v.z = __fadd_rn(v.z, conef_query_term(row[pk[2] & 0x7fffffffu], pk[2], alpha));
-            v.w = __fadd_rn(v.w, conef_query_term(row[pk[3] & 0x7fffffffu], pk[3], alpha));
-            *reinterpret_cast<float4*>(xr) = v;
-        } else {
+        float* xr = it.x + r * it.m + col;
+        float v[4];
+        conef_ld4u(xr, v);
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (c0 + k < it.m) xr[k] = __fadd_rn(xr[k], conef_query_term(row[pk[k] & 0x7fffffffu], pk[k], alpha));
-        }
+        for (int k = 0; k < 4; ++k) v[k] = __fadd_rn(v[k], conef_query_term(row[pk[k] & 0x7fffffffu], pk[k], alpha));
+        conef_st4_own(xr, v, dup);
     }
 }
 
@@ -957,9 +995,76 @@ psgd_rowlist_vec_batch_kernel(PsgdBatch<RowlistVecItem> b, double one_minus_beta
 
 // ------------------------------------------------------------ M = P Q^T ----
 // MODE 0: write M.  MODE 1: also write the dense residual E = X - M (X = what M held on entry).
-// A thread owns a column quad (its 4 x r slice of Q stays in registers), the workgroup walks a slab
-// of rows; the row of P is uniform over the workgroup.
-template <int RP, int MODE, bool FAST>
+// Factors of rank RP exactly (rows of RP floats, 16-byte aligned), rows of at least four columns of
+// any alignment.  A thread owns a column quad, whose 4 x RP slice of Q stays in registers, and walks
+// rows four at a time with their loads in flight together.  A workgroup is cut into groups of
+// `lanes` threads that cover a row (or 1024 columns of it) and take rows in turn; lanes is a multiple
+// of 64 wherever a row has more than 64 quads, so that a wave's row of P is uniform and comes through
+// the scalar cache.
+struct PqtItem {
+    float* x;
+    float* err;
+    const float* p;
+    const float* q;
+    int64_t n;
+    int m, r, rows_per_slab, col_tiles;
+    int lanes;
+};
+
+inline int pqt_lanes(int64_t m)
+{
+    const int64_t m4 = (m + 3) / 4;
+    return (int)(m4 >= 256 ? 256 : m4 > 64 ? (m4 + 63) / 64 * 64 : m4);
+}
+
+template <int RP, int MODE, bool UNIFORM>
+__device__ __forceinline__ void psgd_pqt_rows(const PqtItem& it, int bx, int by)
+{
+    const int m = it.m, groups = 256 / it.lanes;
+    int grp = (int)threadIdx.x / it.lanes;
+    const int quad = bx * 256 + (int)threadIdx.x - grp * it.lanes;
+    if (UNIFORM) grp = __builtin_amdgcn_readfirstlane(grp);
+    if (grp >= groups || 4 * quad >= m) return;
+    const int col = conef_quad_col(quad, m), dup = 4 * quad - col;
+    const int64_t i0 = (int64_t)by * it.rows_per_slab;
+    const int64_t i1 = i0 + it.rows_per_slab < it.n ? i0 + it.rows_per_slab : it.n;
+    float qf[4 * RP];
+#pragma unroll
+    for (int t = 0; t < RP; ++t) conef_ld4u(it.q + (int64_t)col * RP + 4 * t, qf + 4 * t);
+    for (int64_t ib = i0 + grp; ib < i1; ib += 4 * groups) {
+        float xv[4][4];
+        if (MODE == 1) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int64_t i = ib + u * groups < i1 ? ib + u * groups : ib;
+                conef_ld4u(it.x + i * m + col, xv[u]);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t i = ib + u * groups;
+            if (i >= i1) break;
+            const float* pi = it.p + i * RP;
+            float mh[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < RP; ++c) {
+                const float pc = pi[c];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) mh[k] = fmaf(pc, qf[k * RP + c], mh[k]);
+            }
+            if (MODE == 1) {
+                float ev[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) ev[k] = __fsub_rn(xv[u][k], mh[k]);
+                conef_st4_own(it.err + i * m + col, ev, dup);
+            }
+            conef_st4_own(it.x + i * m + col, mh, dup);
+        }
+    }
+}
+
+// The general form: any rank up to RP, element by element.
+template <int RP, int MODE>
 __device__ __forceinline__ void
 psgd_pqt_body(float* __restrict__ x, float* __restrict__ err, const float* __restrict__ p,
               const float* __restrict__ q, int64_t n, int m, int r, int rows_per_slab, int bx, int by)
@@ -969,81 +1074,45 @@ psgd_pqt_body(float* __restrict__ x, float* __restrict__ err, const float* __res
     const int64_t i0 = (int64_t)by * rows_per_slab;
     const int64_t i1 = i0 + rows_per_slab < n ? i0 + rows_per_slab : n;
     float qf[4][RP];
-    if (FAST) {
-        float flat[4 * RP];
+    const int valid = m - c0 < 4 ? m - c0 : 4;
 #pragma unroll
-        for (int t = 0; t < RP; ++t) ld4(q + (int64_t)c0 * RP + 4 * t, flat + 4 * t);
+    for (int k = 0; k < 4; ++k)
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
+        for (int c = 0; c < RP; ++c) qf[k][c] = (k < valid && c < r) ? q[(int64_t)(c0 + k) * r + c] : 0.f;
+    for (int64_t i = i0; i < i1; ++i) {
+        const float* pi = p + i * r;
+        float mh[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int c = 0; c < RP; ++c) qf[k][c] = flat[k * RP + c];
-        for (int64_t ib = i0; ib < i1; ib += 4) {          // four rows in flight
-            float xv[4][4];
-            if (MODE == 1) {
+        for (int c = 0; c < RP; ++c) {
+            float pc = c < r ? pi[c] : 0.f;
 #pragma unroll
-                for (int u = 0; u < 4; ++u) ld4(x + (ib + u < i1 ? ib + u : i1 - 1) * m + c0, xv[u]);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int64_t i = ib + u;
-                if (i >= i1) break;
-                const float* pi = p + i * RP;
-                float mh[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int c = 0; c < RP; ++c) {
-                    float pc = pi[c];
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) mh[k] = fmaf(pc, qf[k][c], mh[k]);
-                }
-                if (MODE == 1) {
-                    float ev[4];
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) ev[k] = __fsub_rn(xv[u][k], mh[k]);
-                    st4(err + i * m + c0, ev);
-                }
-                st4(x + i * m + c0, mh);
-            }
+            for (int k = 0; k < 4; ++k) mh[k] = fmaf(pc, qf[k][c], mh[k]);
         }
-    } else {
-        const int valid = m - c0 < 4 ? m - c0 : 4;
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-#pragma unroll
-            for (int c = 0; c < RP; ++c) qf[k][c] = (k < valid && c < r) ? q[(int64_t)(c0 + k) * r + c] : 0.f;
-        for (int64_t i = i0; i < i1; ++i) {
-            const float* pi = p + i * r;
-            float mh[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int c = 0; c < RP; ++c) {
-                float pc = c < r ? pi[c] : 0.f;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) mh[k] = fmaf(pc, qf[k][c], mh[k]);
-            }
-            for (int k = 0; k < valid; ++k) {
-                int64_t f = i * m + c0 + k;
-                if (MODE == 1) err[f] = __fsub_rn(x[f], mh[k]);
-                x[f] = mh[k];
-            }
+        for (int k = 0; k < valid; ++k) {
+            int64_t f = i * m + c0 + k;
+            if (MODE == 1) err[f] = __fsub_rn(x[f], mh[k]);
+            x[f] = mh[k];
         }
     }
 }
 
-template <int RP, int MODE, bool FAST>
+template <int RP, int MODE>
 __global__ void __launch_bounds__(256)
 psgd_pqt_kernel(float* __restrict__ x, float* __restrict__ err, const float* __restrict__ p,
                 const float* __restrict__ q, int64_t n, int m, int r, int rows_per_slab)
 {
-    psgd_pqt_body<RP, MODE, FAST>(x, err, p, q, n, m, r, rows_per_slab, (int)blockIdx.x, (int)blockIdx.y);
+    psgd_pqt_body<RP, MODE>(x, err, p, q, n, m, r, rows_per_slab, (int)blockIdx.x, (int)blockIdx.y);
 }
 
-struct PqtItem {
-    float* x;
-    float* err;
-    const float* p;
-    const float* q;
-    int64_t n;
-    int m, r, rows_per_slab, col_tiles;
-};
+// FAST: every item of the launch has rank RP and m >= 4
+template <int RP, int MODE, bool FAST>
+__device__ __forceinline__ void psgd_pqt_item(const PqtItem& it, int local)
+{
+    const int bx = local % it.col_tiles, by = local / it.col_tiles;
+    if (!FAST) psgd_pqt_body<RP, MODE>(it.x, it.err, it.p, it.q, it.n, it.m, it.r, it.rows_per_slab, bx, by);
+    else if (it.lanes % 64 == 0) psgd_pqt_rows<RP, MODE, true>(it, bx, by);
+    else psgd_pqt_rows<RP, MODE, false>(it, bx, by);
+}
 
 template <int RP, int MODE, bool FAST>
 __global__ void __launch_bounds__(256)
@@ -1051,8 +1120,7 @@ psgd_pqt_batch_kernel(PsgdBatch<PqtItem> b)
 {
     int local;
     const PqtItem& it = b.item[psgd_batch_locate(b, &local)];
-    psgd_pqt_body<RP, MODE, FAST>(it.x, it.err, it.p, it.q, it.n, it.m, it.r, it.rows_per_slab, local % it.col_tiles,
-                                  local / it.col_tiles);
+    psgd_pqt_item<RP, MODE, FAST>(it, local);
 }
 
 // Front of the row-list sketch kernel: the value to sketch is the residual X - P Q^T, and M is
@@ -1078,7 +1146,8 @@ struct ListPsgdResidual {
             // current two are used, so that a thread has one round trip per tile, not one per step.
             __shared__ float ptile[16 * RP];              // at most 16 rows a tile
             for (int i = threadIdx.x; i < rows * RP; i += kConefRowlistThreads) ptile[i] = p[row0 * RP + i];
-            const int d4 = d >> 2;
+            const int d4 = (d + 3) >> 2;
+            const bool quad_rows = (d & 3) == 0;           // rows of LDS values start on 16 bytes
             const int lanes = d4 < kConefRowlistThreads ? d4 : kConefRowlistThreads;
             const int groups = kConefRowlistThreads / lanes, grp = threadIdx.x / lanes;
             const int step = 2 * groups;
@@ -1087,12 +1156,13 @@ struct ListPsgdResidual {
             float flat[4 * RP], flatn[4 * RP], x0n[4], x1n[4];
             auto request_rows = [&](int quad, int row) {
                 const int r1 = row + 1 < rows ? row + 1 : row;
-                ld4(base + (int64_t)row * d + 4 * quad, x0n);
-                ld4(base + (int64_t)r1 * d + 4 * quad, x1n);
+                const int col = conef_quad_col(quad, d);
+                conef_ld4u(base + (int64_t)row * d + col, x0n);
+                conef_ld4u(base + (int64_t)r1 * d + col, x1n);
             };
             if (have) {
 #pragma unroll
-                for (int v = 0; v < RP; ++v) ld4(q + (int64_t)c4 * 4 * RP + 4 * v, flat + 4 * v);
+                for (int v = 0; v < RP; ++v) conef_ld4u(q + (int64_t)conef_quad_col(c4, d) * RP + 4 * v, flat + 4 * v);
                 request_rows(c4, rw);
             }
             __syncthreads();
@@ -1116,7 +1186,7 @@ struct ListPsgdResidual {
                 if (have) {
                     if (new_quad) {
 #pragma unroll
-                        for (int v = 0; v < RP; ++v) ld4(q + (int64_t)c4 * 4 * RP + 4 * v, flatn + 4 * v);
+                        for (int v = 0; v < RP; ++v) conef_ld4u(q + (int64_t)conef_quad_col(c4, d) * RP + 4 * v, flatn + 4 * v);
                     }
                     request_rows(c4, rw);
                 }
@@ -1137,11 +1207,19 @@ struct ListPsgdResidual {
                     v0[k] = __fsub_rn(x0[k], m0[k]);
                     v1[k] = __fsub_rn(x1[k], m1[k]);
                 }
-                st4(base + (int64_t)cur_rw * d + 4 * cur_c4, m0);
-                st4(vals + cur_rw * d + 4 * cur_c4, v0);
-                if (cur_rw + 1 < rows) {
-                    st4(base + (int64_t)r1 * d + 4 * cur_c4, m1);
-                    st4(vals + r1 * d + 4 * cur_c4, v1);
+                const int col = conef_quad_col(cur_c4, d), dup = 4 * cur_c4 - col;
+                conef_st4_own(base + (int64_t)cur_rw * d + col, m0, dup);
+                if (cur_rw + 1 < rows) conef_st4_own(base + (int64_t)r1 * d + col, m1, dup);
+                if (quad_rows) {
+                    st4_lds(vals + cur_rw * d + col, v0);
+                    if (cur_rw + 1 < rows) st4_lds(vals + r1 * d + col, v1);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (k >= dup) {
+                            vals[cur_rw * d + col + k] = v0[k];
+                            if (cur_rw + 1 < rows) vals[r1 * d + col + k] = v1[k];
+                        }
                 }
                 if (new_quad && have) {
 #pragma unroll
@@ -1438,7 +1516,7 @@ template <int RP>
 __device__ __forceinline__ void gs_ahead_body(const GsAhead& g, int k)
 {
     if (g.parts[k]) {
-        gram_orthogonalise_body<RP, kGsRegThreads>(g.src[k], g.dst[k], g.rows[k], g.parts[k], g.nparts[k], g.eps);
+        gram_orthogonalise_body<RP, kGsRegThreads>(g.src[k], g.dst[k], g.rows[k], g.parts[k], g.nparts[k], g.r, g.eps);
         return;
     }
     // at most kGsAheadRowSlots rows a thread: the taller bodies hold over a hundred values in
@@ -1787,8 +1865,7 @@ int launch_mq(float* x, const float* err, const float* cs, const uint32_t* pktab
               hipStream_t s)
 {
     ConefMod mod = conef_make_mod(w > 0 ? w : 1);
-    if (rank_bound(r) >= 16 && m % 4 == 0 && aligned16(x) && (MODE != 1 || aligned16(err)) &&
-        (!pktab || aligned16(pktab))) {
+    if (rank_bound(r) >= 16 && m >= 4) {
         size_t lds = (size_t)kMfmaWaves * 16 * 64 * 4 + (MODE == 2 ? (size_t)32 * w * 4 : 0);
         if (MODE == 2 && (mfma_mq_shape(n, m).splits > 1 || lds > kMfmaMqLdsLimit)) {
             // Parking 32 sketch rows per workgroup costs more than the tile's share of M once the
@@ -1816,8 +1893,7 @@ int launch_mq(float* x, const float* err, const float* cs, const uint32_t* pktab
             return (int)hipGetLastError();
         }
     }
-    const bool fast = r == rank_bound(r) && m % 4 == 0 && aligned16(x) && aligned16(q) && (MODE != 1 || aligned16(err)) &&
-                      (!pktab || aligned16(pktab));
+    const bool fast = r == rank_bound(r) && m >= 4;
     const int rp = rank_bound(r);
     if (fast && rp < 16) {
         std::vector<MqsItem> one(1);
@@ -2092,6 +2168,9 @@ inline bool gsg_workspace_ok(const void* workspace, int64_t workspace_bytes)
     return workspace && workspace_bytes >= (int64_t)sizeof(GsgWs) && (reinterpret_cast<uintptr_t>(workspace) & 255u) == 0;
 }
 
+int pqt_batch(const ConefPsgdItem* items, int count, int mode, float beta, int32_t a, int32_t b, hipStream_t s,
+              const GsAhead* ahead = nullptr, bool* ahead_used = nullptr);
+
 inline bool psgd_args_ok(int64_t n, int64_t m, int32_t r)
 {
     return n >= 1 && m >= 1 && r >= 1 && r <= kMaxRank && m <= 0x7fffffffLL && n <= 0x7fffffffLL;
@@ -2171,8 +2250,7 @@ int conef_psgd_mtp_f32(const float* x, const float* p, float* q, int64_t n, int6
     if (!psgd_args_ok(n, m, r) || !x || !q || !p) return CONEF_ERR_INVALID;
     hipStream_t s = (hipStream_t)stream;
     if (rank_bound(r) >= 16) {
-        const uintptr_t xa = reinterpret_cast<uintptr_t>(x);
-        int vmax = (m % 4 == 0 && (xa & 15u) == 0) ? 4 : (m % 2 == 0 && (xa & 7u) == 0) ? 2 : 1;
+        const int vmax = m >= 4 ? 4 : m >= 2 ? 2 : 1;
         MfmaMtpShape t = mfma_mtp_shape(n, m, r, vmax);
         float* dst = q;
         if (t.slabs > 1) {
@@ -2196,7 +2274,7 @@ int conef_psgd_mtp_f32(const float* x, const float* p, float* q, int64_t n, int6
         if (!workspace || workspace_bytes < (int64_t)g.slabs * m * r * 4) return CONEF_ERR_INVALID;
         out = (float*)workspace;
     }
-    const bool fast = r == rank_bound(r) && m % 4 == 0 && aligned16(x) && aligned16(p) && aligned16(out);
+    const bool fast = r == rank_bound(r) && m >= 4;
     dim3 grid((unsigned)g.col_tiles, (unsigned)g.slabs);
 #define CONEF_MTP(RP)                                                                                            \
     do {                                                                                                         \
@@ -2218,7 +2296,7 @@ int conef_psgd_mtp_f32(const float* x, const float* p, float* q, int64_t n, int6
 static int launch_pqt(float* x, float* err, const float* p, const float* q, int64_t n, int64_t m, int32_t r,
                       hipStream_t s)
 {
-    if ((r == 16 || r == 32) && aligned16(p) && aligned16(q)) {
+    if (r == 16 || r == 32) {
         int64_t col_wgs = (m + 32 * kMfmaWaves - 1) / (32 * kMfmaWaves);
         int64_t slabs = (1024 + col_wgs - 1) / col_wgs;
         int64_t rps = ((n + slabs - 1) / slabs + 31) / 32 * 32;
@@ -2237,7 +2315,11 @@ static int launch_pqt(float* x, float* err, const float* p, const float* q, int6
         }
         return (int)hipGetLastError();
     }
-    const bool fast = r == rank_bound(r) && m % 4 == 0 && aligned16(x) && aligned16(q) && (!err || aligned16(err));
+    if (r <= 8 && r == rank_bound(r) && m >= 4) {
+        ConefPsgdItem it = {};
+        it.x = x; it.err = err; it.p = const_cast<float*>(p); it.q = const_cast<float*>(q); it.n = n; it.m = m; it.r = r;
+        return pqt_batch(&it, 1, err ? 1 : 0, 0.f, 0, 0, s);
+    }
     int64_t col_tiles = (m + 1023) / 1024;
     int64_t slabs = (1024 + col_tiles - 1) / col_tiles;       // about a thousand workgroups ...
     int64_t rps = (n + slabs - 1) / slabs;
@@ -2248,17 +2330,12 @@ static int launch_pqt(float* x, float* err, const float* p, const float* q, int6
         slabs = (n + rps - 1) / rps;
     }
     dim3 grid((unsigned)col_tiles, (unsigned)slabs);
-#define CONEF_PQT_GO(RP, MODE, F) \
-    hipLaunchKernelGGL((psgd_pqt_kernel<RP, MODE, F>), grid, dim3(256), 0, s, x, err, p, q, n, (int)m, r, (int)rps)
+#define CONEF_PQT_GO(RP, MODE) \
+    hipLaunchKernelGGL((psgd_pqt_kernel<RP, MODE>), grid, dim3(256), 0, s, x, err, p, q, n, (int)m, r, (int)rps)
 #define CONEF_PQT(RP)                                 \
     do {                                              \
-        if (err) {                                    \
-            if (fast) CONEF_PQT_GO(RP, 1, true);      \
-            else CONEF_PQT_GO(RP, 1, false);          \
-        } else {                                      \
-            if (fast) CONEF_PQT_GO(RP, 0, true);      \
-            else CONEF_PQT_GO(RP, 0, false);          \
-        }                                             \
+        if (err) CONEF_PQT_GO(RP, 1);                 \
+        else CONEF_PQT_GO(RP, 0);                     \
     } while (0)
     CONEF_RANK_SWITCH(r, CONEF_PQT)
 #undef CONEF_PQT
@@ -2298,7 +2375,7 @@ int conef_psgd_pqt_conef_planned_f32(float* x, const float* p, const float* q, c
     if (!psgd_args_ok(n, m, r) || !x || !q || !p || !cs_in || !cs_out || !plan_dev ||
         !conef_plan_matches(hp, n, m, w, a, b) || hp->kind != kConefPlanRowlist)
         return CONEF_ERR_INVALID;
-    const bool fast = r == rank_bound(r) && m % 4 == 0 && aligned16(x) && aligned16(q) && aligned16(p);
+    const bool fast = r == rank_bound(r) && m >= 4;
     ConefRowlistView view = conef_rowlist_view(hp, plan_dev);
     hipStream_t s = (hipStream_t)stream;
     int rc = CONEF_ERR_INVALID;
@@ -2672,20 +2749,18 @@ int mq_batch(const ConefPsgdItem* items, int count, float alpha, int32_t a, int3
         const ConefPsgdItem& lead = items[k];
         const int rp = rank_bound(lead.r);
         auto fast_of = [&](const ConefPsgdItem& it) {
-            return it.r == rank_bound(it.r) && it.m % 4 == 0 && aligned16(it.x) && aligned16(it.q) &&
-                   (MODE != 1 || aligned16(it.err)) && (MODE != 2 || !item_pktab(it) || aligned16(item_pktab(it)));
+            return it.r == rank_bound(it.r) && it.m >= 4;
         };
         const bool fast = fast_of(lead);
         // ranks on the matrix cores, and sketch rows too wide for LDS, go one by one
         auto alone = [&](const ConefPsgdItem& it) {
             return rank_bound(it.r) >= 16 || (MODE == 2 && (size_t)4 * it.w * 4 + 4 * 4 * 8 * 4 > 64 * 1024);
         };
-        // ranks on the matrix cores whose shapes allow the 16-byte paths share launches: the sketch
+        // ranks on the matrix cores share launches: the sketch
         // query first when there is one, then the plain (or error-adding) product, then the sums
         // of the column splits
         auto mfma_ok = [&](const ConefPsgdItem& it) {
-            return rank_bound(it.r) >= 16 && it.m % 4 == 0 && aligned16(it.x) && (MODE != 1 || aligned16(it.err)) &&
-                   (MODE != 2 || !item_pktab(it) || aligned16(item_pktab(it)));
+            return rank_bound(it.r) >= 16 && it.m >= 4;
         };
         if (mfma_ok(lead)) {
             std::vector<int64_t> offs;
@@ -2725,7 +2800,7 @@ int mq_batch(const ConefPsgdItem* items, int count, float alpha, int32_t a, int3
             int rc = CONEF_OK;
             if (MODE == 2)
                 rc = run_batches(queries, qblocks, [&](const PsgdBatch<QueryItem>& bt, int grid) {
-                    hipLaunchKernelGGL(psgd_cs_query_batch_kernel<true>, dim3((unsigned)grid), dim3(256), 0, s, bt, alpha, hs);
+                    hipLaunchKernelGGL(psgd_cs_query_batch_kernel, dim3((unsigned)grid), dim3(256), 0, s, bt, alpha, hs);
                 });
             if (rc != CONEF_OK) return rc;
             const size_t lds = (size_t)kMfmaWaves * 16 * 64 * 4;
@@ -2866,8 +2941,7 @@ int mtp_batch(const ConefPsgdItem* items, int count, void* workspace, int64_t wo
         for (int k = 0; k < count; ++k) {
             const ConefPsgdItem& it = items[k];
             if (done[(size_t)k] || rank_bound(it.r) < 16) continue;
-            const uintptr_t xa = reinterpret_cast<uintptr_t>(it.x);
-            const int vmax = (it.m % 4 == 0 && (xa & 15u) == 0) ? 4 : (it.m % 2 == 0 && (xa & 7u) == 0) ? 2 : 1;
+            const int vmax = it.m >= 4 ? 4 : it.m >= 2 ? 2 : 1;
             MfmaMtpShape t = mfma_mtp_shape(it.n, it.m, it.r, vmax, want_wgs < 512 ? want_wgs : 512);
             if (v != 0 && t.v != v) continue;
             float* out = t.slabs > 1 ? mfma_partials + mfma_offs[(size_t)k] : it.q;
@@ -2915,9 +2989,7 @@ int mtp_batch(const ConefPsgdItem* items, int count, void* workspace, int64_t wo
             continue;
         }
         auto fast_of = [&](int j) {
-            const ConefPsgdItem& it = items[j];
-            const float* out = plans[(size_t)j].partial_off >= 0 ? partial_base + plans[(size_t)j].partial_off : it.q;
-            return it.r == rank_bound(it.r) && it.m % 4 == 0 && aligned16(it.x) && aligned16(it.p) && aligned16(out);
+            return items[j].r == rank_bound(items[j].r) && items[j].m >= 4;
         };
         const bool fast = fast_of(k);
         std::vector<MtpItem> table;
@@ -2970,8 +3042,7 @@ int mtp_batch(const ConefPsgdItem* items, int count, void* workspace, int64_t wo
 // ---- deferred orthogonalisation of P: host side ----
 // The end of a batch workspace holds, per matrix, the shares of P^T P (ranks up to 8: one per
 // workgroup of the first product, at most one per four rows; ranks 16 and 32: one per 256 rows),
-// the solved system (b_ij and 1 / d_i) and, at ranks up to 8, the shares of Q^T Q (one per 256
-// rows of Q).
+// the solved system (b_ij and 1 / d_i) and the shares of Q^T Q (one per 256 rows of Q).
 inline int64_t defer_tmat_bytes(int rp) { return conef_align256((int64_t)(rp * rp + rp) * 4); }
 
 inline int64_t defer_gram_doubles(const ConefPsgdItem& it)
@@ -2985,7 +3056,7 @@ inline int64_t defer_gram_doubles(const ConefPsgdItem& it)
 inline int64_t defer_qgram_doubles(const ConefPsgdItem& it)
 {
     const int rp = rank_bound(it.r);
-    return rp <= 8 ? ((it.m + 255) / 256) * (int64_t)(rp * (rp + 1) / 2) : 0;
+    return ((it.m + 255) / 256) * (int64_t)(rp * (rp + 1) / 2);
 }
 
 inline int64_t defer_region_bytes(const ConefPsgdItem* items, int count)
@@ -3008,38 +3079,158 @@ inline int64_t defer_region_offset(const ConefPsgdItem* items, int count)
            conef_align256(4 * mfma_batch_layout(items, count, nullptr));
 }
 
+// The matrices of a round whose factors have rows of rank_bound(r) floats.  At ranks 1, 2, 4, 8, 16 and
+// 32 those are the caller's own factors; at a rank between two of them the round works on copies in
+// its workspace, zeros behind the first r of a row, and its fix launch writes both.  A row of zeros
+// more costs nothing a streaming pass notices (the matrix is what moves) and buys 16-byte accesses
+// and one contiguous run of Q per column quad; the general kernels, which take a rank as it comes and
+// go by single floats, were 3 to 6 times slower on whole rounds at ranks 3, 5, 6 and 20.
+struct PaddedRound {
+    std::vector<ConefPsgdItem> items;
+    std::vector<float*> pt, qt;      // the caller's factors where items holds copies, else null
+    int rp;
+    bool padded;
+};
+
+inline int64_t padded_factor_bytes(const ConefPsgdItem& it)
+{
+    const int rp = rank_bound(it.r);
+    return rp == it.r ? 0 : conef_align256(4 * it.n * rp) + conef_align256(4 * it.m * rp);
+}
+
+inline std::vector<ConefPsgdItem> at_rank_bound(const ConefPsgdItem* items, int count)
+{
+    std::vector<ConefPsgdItem> v(items, items + count);
+    for (ConefPsgdItem& it : v) it.r = rank_bound(it.r);
+    return v;
+}
+
+// Workspace of a deferred round: the products' regions, the Gram shares, the copies of the factors.
+inline int64_t padded_round_bytes(const ConefPsgdItem* items, int count)
+{
+    const std::vector<ConefPsgdItem> v = at_rank_bound(items, count);
+    int64_t bytes = defer_region_offset(v.data(), count) + defer_region_bytes(v.data(), count);
+    for (int k = 0; k < count; ++k) bytes += padded_factor_bytes(items[k]);
+    return bytes;
+}
+
+// Whether the round of these matrices runs with the orthogonalisation of P deferred: one launch's
+// worth of matrices of one rank, rows of at least four columns, a workspace of padded_round_bytes.
+inline bool padded_round(const ConefPsgdItem* items, int count, int mq_mode, void* workspace, int64_t workspace_bytes,
+                         PaddedRound* pr)
+{
+    if (count < 1 || count > kPsgdBatchMax || !workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) return false;
+    for (int k = 0; k < count; ++k)
+        if (items[k].r != items[0].r || items[k].m < 4 || items[k].n > 0x7fffffffLL || items[k].m > 0x7fffffffLL) return false;
+    if (workspace_bytes < padded_round_bytes(items, count)) return false;
+    pr->items = at_rank_bound(items, count);
+    pr->rp = rank_bound(items[0].r);
+    pr->padded = pr->rp != items[0].r;
+    char* at = (char*)workspace + defer_region_offset(pr->items.data(), count) + defer_region_bytes(pr->items.data(), count);
+    for (int k = 0; k < count; ++k) {
+        ConefPsgdItem& it = pr->items[(size_t)k];
+        pr->pt.push_back(pr->padded ? it.p : nullptr);
+        pr->qt.push_back(pr->padded ? it.q : nullptr);
+        if (pr->padded) {
+            it.p = (float*)at;
+            at += conef_align256(4 * it.n * pr->rp);
+            it.q = (float*)at;
+            at += conef_align256(4 * it.m * pr->rp);
+        }
+    }
+    if (pr->rp > 8) {
+        std::vector<int64_t> offs;
+        return mfma_partial_base(pr->items.data(), count, workspace, workspace_bytes, &offs) != nullptr;
+    }
+    // the streaming first product takes every shape whose sketch rows fit its LDS
+    std::vector<MqsItem> table;
+    for (const ConefPsgdItem& it : pr->items) {
+        MqsItem t = {};
+        t.n = it.n;
+        t.m = (int)it.m;
+        t.w = mq_mode == 2 ? it.w : 1;
+        table.push_back(t);
+    }
+    int T, S;
+    size_t lds;
+    return mqs_plan_launch(table.data(), count, pr->rp, mq_mode == 2, &T, &S, &lds, true);
+}
+
+// dst[row] = src[row] and zeros behind it, rows of r and RP floats
+struct PadRowsItem {
+    const float* src;
+    float* dst;
+    int64_t rows;
+};
+
+__global__ void __launch_bounds__(256)
+psgd_pad_rows_batch_kernel(PsgdBatch<PadRowsItem> b, int r, int rp)
+{
+    int local;
+    const PadRowsItem& it = b.item[psgd_batch_locate(b, &local)];
+    const int64_t e = (int64_t)local * 256 + threadIdx.x;
+    if (e >= it.rows * rp) return;
+    const int64_t row = e / rp;
+    const int c = (int)(e - row * rp);
+    it.dst[e] = c < r ? it.src[row * r + c] : 0.f;
+}
+
+int pad_rows(const std::vector<PadRowsItem>& table, int r, int rp, hipStream_t s)
+{
+    std::vector<int> blocks;
+    for (const PadRowsItem& t : table) blocks.push_back((int)((t.rows * rp + 255) / 256));
+    return run_batches(table, blocks, [&](const PsgdBatch<PadRowsItem>& bt, int grid) {
+        hipLaunchKernelGGL(psgd_pad_rows_batch_kernel, dim3((unsigned)grid), dim3(256), 0, s, bt, r, rp);
+    });
+}
+
+// The fix launch of a deferred round over `raw` (where the products left the raw Q).
+int defer_fix(const PaddedRound& pr, int r, const std::vector<MtpRaw>& raw, const std::vector<float*>& tmats,
+              const std::vector<double*>* qgrams, hipStream_t s)
+{
+    const int rp = pr.rp, count = (int)pr.items.size();
+    const int rows_per_wg = rp <= 8 ? 256 : 256 / (rp / 4);
+    std::vector<DeferFixItem> fix;
+    std::vector<int> blocks;
+    for (int k = 0; k < count; ++k) {
+        const ConefPsgdItem& it = pr.items[(size_t)k];
+        const int pb = (int)((it.n + rows_per_wg - 1) / rows_per_wg), qb = (int)((it.m + rows_per_wg - 1) / rows_per_wg);
+        fix.push_back(DeferFixItem{it.p, raw[(size_t)k].src, it.q, tmats[(size_t)k], qgrams ? (*qgrams)[(size_t)k] : nullptr,
+                                   it.n, it.m, raw[(size_t)k].slabs, pb, pr.pt[(size_t)k], pr.qt[(size_t)k], r});
+        blocks.push_back(pb + qb);
+    }
+    return run_batches(fix, blocks, [&](const PsgdBatch<DeferFixItem>& bt, int grid) {
+        const dim3 g((unsigned)grid), t(256);
+        switch (rp) {
+            case 1: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<1>, g, t, 0, s, bt); break;
+            case 2: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<2>, g, t, 0, s, bt); break;
+            case 4: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<4>, g, t, 0, s, bt); break;
+            case 8: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<8>, g, t, 0, s, bt); break;
+            case 16: hipLaunchKernelGGL(psgd_defer_fix_wide_batch_kernel<16>, g, t, 0, s, bt); break;
+            default: hipLaunchKernelGGL(psgd_defer_fix_wide_batch_kernel<32>, g, t, 0, s, bt); break;
+        }
+    });
+}
+
 // P = X Q (raw) with the Gram shares, Q = X^T P (raw) with the systems solved on the side, then T
-// applied to both.  `mq_items` differ from `items` in q only: the Q the first product reads.
+// applied to both.  q_in: the Q the first product reads, rows of pr.rp floats.
 // q_shares (optional): the fix launch also leaves the shares of Q^T Q of the new Q factors; their
 // places are recorded in q_shares->parts / nparts.
-// kMqsNoFit with nothing launched: the batch is not one this path takes (ranks
-// above 8 or mixed, shapes without 16-byte accesses, a workspace without the region above).
 template <int MODE>
-int round_products_deferred(const ConefPsgdItem* items, const ConefPsgdItem* mq_items, int count, float alpha, float eps,
-                            int32_t a, int32_t b, void* workspace, int64_t workspace_bytes, hipStream_t s,
-                            GsAhead* q_shares)
+int round_products_deferred(const PaddedRound& pr, int r, float* const* q_in, float alpha, float eps, int32_t a, int32_t b,
+                            void* workspace, int64_t workspace_bytes, hipStream_t s, GsAhead* q_shares)
 {
-    if (count < 1 || count > kPsgdBatchMax || !workspace) return kMqsNoFit;
-    const int rp = rank_bound(items[0].r);
-    if (rp > 8) return kMqsNoFit;
-    const int ng = rp * (rp + 1) / 2;
-    const int64_t region = defer_region_offset(items, count);
-    if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0 || workspace_bytes < region + defer_region_bytes(items, count))
-        return kMqsNoFit;
+    const ConefPsgdItem* items = pr.items.data();
+    const int count = (int)pr.items.size(), rp = pr.rp;
     ConefSeeds hs = {a, b, a + 2, b + 3};
     std::vector<MqsItem> table;
     std::vector<float*> tmats;
     std::vector<double*> qgrams;
-    char* at = (char*)workspace + region;
+    char* at = (char*)workspace + defer_region_offset(items, count);
     for (int k = 0; k < count; ++k) {
         const ConefPsgdItem& it = items[k];
-        const uint32_t* pk = MODE == 2 ? item_pktab(it) : nullptr;
-        const float* q_in = mq_items[k].q;       // the first product's Q (last round's, orthogonalised); it.q receives the new one
-        if (it.r != rp || it.m % 4 != 0 || it.n > 0x7fffffffLL || !aligned16(it.x) || !aligned16(it.q) || !aligned16(it.p) ||
-            !aligned16(q_in) || (MODE == 1 && !aligned16(it.err)) || (pk && !aligned16(pk)))
-            return kMqsNoFit;
-        MqsItem t = {it.x, it.err, it.cs, pk, q_in, it.p, it.n, (int)it.m, (int)(MODE == 2 ? it.w : 1), 0, 0,
-                     conef_make_mod(MODE == 2 ? it.w : 1), (double*)at};
+        MqsItem t = {it.x, it.err, it.cs, MODE == 2 ? item_pktab(it) : nullptr, q_in[k], it.p, it.n, (int)it.m,
+                     (int)(MODE == 2 ? it.w : 1), 0, 0, conef_make_mod(MODE == 2 ? it.w : 1), (double*)at};
         table.push_back(t);
         at += conef_align256(8 * defer_gram_doubles(it));
         tmats.push_back((float*)at);
@@ -3049,88 +3240,49 @@ int round_products_deferred(const ConefPsgdItem* items, const ConefPsgdItem* mq_
     }
     int T, S;
     size_t lds;
-    if (!mqs_plan_launch(table.data(), count, rp, MODE == 2, &T, &S, &lds, true)) return kMqsNoFit;
-    // the second product must be the 16-byte form of one launch, its partials inside the workspace
-    std::vector<MtpPlan> plans;
-    const int64_t mtp_floats = mtp_batch_layout(items, count, &plans);
-    if (workspace_bytes < 4 * mtp_floats) return kMqsNoFit;
-    for (int k = 0; k < count; ++k) {
-        const float* out = plans[(size_t)k].partial_off >= 0 ? (const float*)workspace + plans[(size_t)k].partial_off : items[k].q;
-        if (!aligned16(out)) return kMqsNoFit;
-    }
-
+    if (!mqs_plan_launch(table.data(), count, rp, MODE == 2, &T, &S, &lds, true)) return CONEF_ERR_INVALID;
     int rc = mqs_run<MODE>(table, rp, alpha, hs, s, true);
-    if (rc != CONEF_OK) return rc;         // mqs_plan_launch above is the same decision: not kMqsNoFit here
+    if (rc != CONEF_OK) return rc == kMqsNoFit ? CONEF_ERR_INVALID : rc;
     GramTask gram;
     gram.count = count;
+    gram.r = r;
     gram.eps = eps;
     for (int k = 0; k < count; ++k) {
         const int gw = mqs_group_width(items[k].m, T);
         gram.parts[k] = table[(size_t)k].gram;
         gram.nparts[k] = (int)mqs_workgroups(items[k].n, gw, S, T);
         gram.tmat[k] = tmats[(size_t)k];
+        if (q_shares) {
+            q_shares->parts[k] = qgrams[(size_t)k];
+            q_shares->nparts[k] = (int)((items[k].m + 255) / 256);
+        }
     }
     std::vector<MtpRaw> raw((size_t)count);
     rc = mtp_batch(items, count, workspace, workspace_bytes, s, &gram, &raw);
     if (rc != CONEF_OK) return rc;
-    std::vector<DeferFixItem> fix;
-    std::vector<int> blocks;
-    for (int k = 0; k < count; ++k) {
-        const ConefPsgdItem& it = items[k];
-        const int pb = (int)((it.n + 255) / 256), qb = (int)((it.m + 255) / 256);
-        fix.push_back(DeferFixItem{it.p, raw[(size_t)k].src, it.q, tmats[(size_t)k], q_shares ? qgrams[(size_t)k] : nullptr,
-                                   it.n, it.m, raw[(size_t)k].slabs, pb});
-        blocks.push_back(pb + qb);
-        if (q_shares) {
-            q_shares->parts[k] = qgrams[(size_t)k];
-            q_shares->nparts[k] = qb;
-        }
-    }
-    (void)ng;
-#define CONEF_DFX(RP)                                                                                               \
-    do {                                                                                                            \
-        if (RP >= 16) break;                                                                                        \
-        rc = run_batches(fix, blocks, [&](const PsgdBatch<DeferFixItem>& bt, int grid) {                            \
-            hipLaunchKernelGGL((psgd_defer_fix_batch_kernel<(RP < 16 ? RP : 8)>), dim3((unsigned)grid), dim3(256), 0, s, bt); \
-        });                                                                                                         \
-    } while (0)
-    CONEF_RANK_SWITCH(rp, CONEF_DFX)
-#undef CONEF_DFX
-    return rc;
+    return defer_fix(pr, r, raw, tmats, q_shares ? &qgrams : nullptr, s);
 }
 
-// The same for ranks 16 and 32, whose products run on the matrix cores: the shares of P^T P come
+// The same for ranks 9 to 32, whose products run on the matrix cores: the shares of P^T P come
 // from a short launch of their own over the finished P, the systems ride in the second product's
 // first launch, and the fix launch is the wide form.  `mq_mode` as in conef_psgd_mq_batch_f32.
-int round_products_deferred_mfma(const ConefPsgdItem* items, const ConefPsgdItem* mq_items, int count, int mq_mode,
-                                 float alpha, float eps, int32_t a, int32_t b, void* workspace, int64_t workspace_bytes,
-                                 hipStream_t s)
+int round_products_deferred_mfma(const PaddedRound& pr, int r, float* const* q_in, int mq_mode, float alpha, float eps,
+                                 int32_t a, int32_t b, void* workspace, int64_t workspace_bytes, hipStream_t s)
 {
-    if (count < 1 || count > kPsgdBatchMax || !workspace) return kMqsNoFit;
-    const int rp = items[0].r;
-    if (rp != 16 && rp != 32) return kMqsNoFit;
-    const int64_t region = defer_region_offset(items, count);
-    if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0 || workspace_bytes < region + defer_region_bytes(items, count))
-        return kMqsNoFit;
-    for (int k = 0; k < count; ++k) {
-        const ConefPsgdItem& it = items[k];
-        if (it.r != rp || it.m % 4 != 0 || it.n > 0x7fffffffLL || !aligned16(it.x) || !aligned16(it.q) || !aligned16(it.p) ||
-            !aligned16(mq_items[k].q) || (mq_mode == 1 && !aligned16(it.err)))
-            return kMqsNoFit;
-    }
-    // the second product must run as matrix-core launches (the systems ride in the first of them)
-    // with their slabs inside the workspace
-    std::vector<int64_t> offs;
-    if (!mfma_partial_base(items, count, workspace, workspace_bytes, &offs)) return kMqsNoFit;
-    int rc = conef_psgd_mq_batch_f32(mq_items, count, mq_mode, alpha, a, b, workspace, workspace_bytes, (void*)s);
+    const ConefPsgdItem* items = pr.items.data();
+    const int count = (int)pr.items.size(), rp = pr.rp;
+    std::vector<ConefPsgdItem> first(pr.items);
+    for (int k = 0; k < count; ++k) first[(size_t)k].q = q_in[k];
+    int rc = conef_psgd_mq_batch_f32(first.data(), count, mq_mode, alpha, a, b, workspace, workspace_bytes, (void*)s);
     if (rc != CONEF_OK) return rc;
     std::vector<GramShareItem> shares;
     std::vector<int> share_blocks;
     std::vector<float*> tmats;
     GramTask gram;
     gram.count = count;
+    gram.r = r;
     gram.eps = eps;
-    char* at = (char*)workspace + region;
+    char* at = (char*)workspace + defer_region_offset(items, count);
     for (int k = 0; k < count; ++k) {
         const ConefPsgdItem& it = items[k];
         const int nb = (int)((it.n + 255) / 256);
@@ -3151,16 +3303,64 @@ int round_products_deferred_mfma(const ConefPsgdItem* items, const ConefPsgdItem
     std::vector<MtpRaw> raw((size_t)count);
     rc = mtp_batch(items, count, workspace, workspace_bytes, s, &gram, &raw);
     if (rc != CONEF_OK) return rc;
+    return defer_fix(pr, r, raw, tmats, nullptr, s);
+}
+
+// Either of the two by rank.
+int deferred_products(const PaddedRound& pr, int r, float* const* q_in, int mq_mode, float alpha, float eps, int32_t a, int32_t b,
+                      void* workspace, int64_t workspace_bytes, hipStream_t s, GsAhead* q_shares)
+{
+    if (pr.rp > 8)
+        return round_products_deferred_mfma(pr, r, q_in, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, s);
+    if (mq_mode == 0)
+        return round_products_deferred<0>(pr, r, q_in, 0.f, eps, a, b, workspace, workspace_bytes, s, q_shares);
+    if (mq_mode == 1)
+        return round_products_deferred<1>(pr, r, q_in, 0.f, eps, a, b, workspace, workspace_bytes, s, q_shares);
+    return round_products_deferred<2>(pr, r, q_in, alpha, eps, a, b, workspace, workspace_bytes, s, q_shares);
+}
+
+// dst[k] <- the rows of src[k] ([m, RP], zeros behind column r) orthogonalised, at ranks 9 to 32: the
+// shares of Q^T Q, the system solved by one workgroup a matrix, T applied row by row.  Three short
+// launches whatever the height, where the kernels that go column by column or meet across
+// workgroups took 28 to 43 us a bucket.
+int orthogonalise_by_gram_wide(const PaddedRound& pr, int r, const std::vector<const float*>& src, float* const* dst, float eps,
+                               void* workspace, hipStream_t s)
+{
+    const int count = (int)pr.items.size(), rp = pr.rp;
+    // the Gram region of P is free by now (the fix launch was its last reader), and so is the front for T
+    std::vector<GramShareItem> shares;
+    std::vector<int> share_blocks, fix_blocks;
     std::vector<DeferFixItem> fix;
-    std::vector<int> blocks;
+    GramTask gram;
+    gram.count = count;
+    gram.r = r;
+    gram.eps = eps;
+    char* at = (char*)workspace + defer_region_offset(pr.items.data(), count);
     const int rows_per_wg = 256 / (rp / 4);
     for (int k = 0; k < count; ++k) {
-        const ConefPsgdItem& it = items[k];
-        const int pb = (int)((it.n + rows_per_wg - 1) / rows_per_wg), qb = (int)((it.m + rows_per_wg - 1) / rows_per_wg);
-        fix.push_back(DeferFixItem{it.p, raw[(size_t)k].src, it.q, tmats[(size_t)k], nullptr, it.n, it.m, raw[(size_t)k].slabs, pb});
-        blocks.push_back(pb + qb);
+        const ConefPsgdItem& it = pr.items[(size_t)k];
+        const int nb = (int)((it.m + 255) / 256);
+        at += conef_align256(8 * defer_gram_doubles(it));
+        float* tmat = (float*)at;
+        at += defer_tmat_bytes(rp);
+        double* parts = (double*)at;
+        at += conef_align256(8 * defer_qgram_doubles(it));
+        shares.push_back(GramShareItem{src[(size_t)k], it.m, parts});
+        share_blocks.push_back(nb);
+        gram.parts[k] = parts;
+        gram.nparts[k] = nb;
+        gram.tmat[k] = tmat;
+        fix.push_back(DeferFixItem{nullptr, src[(size_t)k], dst[k], tmat, nullptr, 0, it.m, 1, 0, nullptr, nullptr, r});
+        fix_blocks.push_back((int)((it.m + rows_per_wg - 1) / rows_per_wg));
     }
-    return run_batches(fix, blocks, [&](const PsgdBatch<DeferFixItem>& bt, int grid) {
+    int rc = run_batches(shares, share_blocks, [&](const PsgdBatch<GramShareItem>& bt, int grid) {
+        if (rp == 32) hipLaunchKernelGGL(psgd_gram_shares_batch_kernel<32>, dim3((unsigned)grid), dim3(kGsgThreads), 0, s, bt);
+        else hipLaunchKernelGGL(psgd_gram_shares_batch_kernel<16>, dim3((unsigned)grid), dim3(kGsgThreads), 0, s, bt);
+    });
+    if (rc != CONEF_OK) return rc;
+    if (rp == 32) hipLaunchKernelGGL(psgd_gram_solve_batch_kernel<32>, dim3((unsigned)count), dim3(kMfmaThreads), 0, s, gram);
+    else hipLaunchKernelGGL(psgd_gram_solve_batch_kernel<16>, dim3((unsigned)count), dim3(kMfmaThreads), 0, s, gram);
+    return run_batches(fix, fix_blocks, [&](const PsgdBatch<DeferFixItem>& bt, int grid) {
         if (rp == 32) hipLaunchKernelGGL(psgd_defer_fix_wide_batch_kernel<32>, dim3((unsigned)grid), dim3(256), 0, s, bt);
         else hipLaunchKernelGGL(psgd_defer_fix_wide_batch_kernel<16>, dim3((unsigned)grid), dim3(256), 0, s, bt);
     });
@@ -3222,8 +3422,33 @@ psgd_pqt_gs_batch_kernel(PsgdBatch<PqtItem> b, GsAhead g)
     while (i + 1 < b.count && bx >= b.first[i + 1]) ++i;
     const PqtItem& it = b.item[i];
     const int local = bx - b.first[i];
-    psgd_pqt_body<RP, MODE, FAST>(it.x, it.err, it.p, it.q, it.n, it.m, it.r, it.rows_per_slab, local % it.col_tiles,
-                                  local / it.col_tiles);
+    psgd_pqt_item<RP, MODE, FAST>(it, local);
+}
+
+// Rows a workgroup of the dense M = P Q^T takes: as many as leave the launch two thousand workgroups
+// (eight a CU: the walk has no prefetch of its own and lives off resident waves), at most sixteen a
+// thread (the thread's slice of Q, RP 16-byte loads, is then read once per sixteen rows of three
+// accesses each), at least four (one trip).
+inline void pqt_rows_table(const ConefPsgdItem* items, const std::vector<int>& members, int mode, std::vector<PqtItem>* table,
+                           std::vector<int>* blocks)
+{
+    int per_thread = 16;
+    for (; per_thread > 4; per_thread >>= 1) {
+        int64_t wgs = 0;
+        for (int j : members) {
+            const int64_t rows = (int64_t)(256 / pqt_lanes(items[j].m)) * per_thread;
+            wgs += (items[j].m + 1023) / 1024 * ((items[j].n + rows - 1) / rows);
+        }
+        if (wgs >= 2048) break;
+    }
+    for (int j : members) {
+        const ConefPsgdItem& it = items[j];
+        const int lanes = pqt_lanes(it.m);
+        const int64_t rows = (int64_t)(256 / lanes) * per_thread, col_tiles = (it.m + 1023) / 1024;
+        table->push_back(PqtItem{it.x, mode == 1 ? it.err : nullptr, it.p, it.q, it.n, (int)it.m, it.r, (int)rows,
+                                 (int)col_tiles, lanes});
+        blocks->push_back((int)(col_tiles * ((it.n + rows - 1) / rows)));
+    }
 }
 
 template <int RP, bool FAST>
@@ -3272,7 +3497,7 @@ int pqt_sketch_group(const ConefPsgdItem* items, const std::vector<int>& members
 // ahead: the Q factors to orthogonalise alongside (mode 2, one rank class over the whole bucket
 // only); *ahead_used says whether that was done.
 int pqt_batch(const ConefPsgdItem* items, int count, int mode, float beta, int32_t a, int32_t b, hipStream_t s,
-              const GsAhead* ahead = nullptr, bool* ahead_used = nullptr)
+              const GsAhead* ahead, bool* ahead_used)
 {
     if (ahead_used) *ahead_used = false;
     std::vector<char> done((size_t)count, 0);
@@ -3280,13 +3505,13 @@ int pqt_batch(const ConefPsgdItem* items, int count, int mode, float beta, int32
         if (done[(size_t)k]) continue;
         const ConefPsgdItem& lead = items[k];
         const int rp = rank_bound(lead.r);
-        if (mode != 2 && (lead.r == 16 || lead.r == 32) && aligned16(lead.p) && aligned16(lead.q)) {
+        if (mode != 2 && (lead.r == 16 || lead.r == 32)) {
             // matrix-core items of one rank share a launch
             std::vector<MfmaPqtItem> table;
             std::vector<int> blocks;
             for (int j = k; j < count; ++j) {
                 const ConefPsgdItem& it = items[j];
-                if (done[(size_t)j] || it.r != lead.r || !aligned16(it.p) || !aligned16(it.q)) continue;
+                if (done[(size_t)j] || it.r != lead.r) continue;
                 int64_t col_wgs = (it.m + 32 * kMfmaWaves - 1) / (32 * kMfmaWaves);
                 int64_t slabs = (1024 + col_wgs - 1) / col_wgs;
                 int64_t rps = ((it.n + slabs - 1) / slabs + 31) / 32 * 32;
@@ -3312,7 +3537,7 @@ int pqt_batch(const ConefPsgdItem* items, int count, int mode, float beta, int32
             if (mode == 2 && rp < 16) {
                 // residual sketch on row-list plans: items of one rank class share launches
                 auto fast_of = [&](const ConefPsgdItem& it) {
-                    return it.r == rank_bound(it.r) && it.m % 4 == 0 && aligned16(it.x) && aligned16(it.q) && aligned16(it.p);
+                    return it.r == rank_bound(it.r) && it.m >= 4;
                 };
                 const bool fast = fast_of(lead);
                 std::vector<int> members;
@@ -3351,25 +3576,31 @@ int pqt_batch(const ConefPsgdItem* items, int count, int mode, float beta, int32
             continue;
         }
         auto fast_of = [&](const ConefPsgdItem& it) {
-            return it.r == rank_bound(it.r) && it.m % 4 == 0 && aligned16(it.x) && aligned16(it.q) &&
-                   (mode != 1 || aligned16(it.err));
+            return it.r == rank_bound(it.r) && it.m >= 4;
         };
         const bool fast = fast_of(lead);
-        std::vector<PqtItem> table;
-        std::vector<int> blocks;
+        std::vector<int> members;
         for (int j = k; j < count; ++j) {
             if (done[(size_t)j] || rank_bound(items[j].r) != rp || fast_of(items[j]) != fast) continue;
-            const ConefPsgdItem& it = items[j];
-            // about a thousand workgroups for the batch as a whole, slabs of at least four rows
-            int64_t col_tiles = (it.m + 1023) / 1024;
-            int64_t slabs = (256 + col_tiles - 1) / col_tiles;
-            int64_t rps = (it.n + slabs - 1) / slabs;
-            if (rps < 4) rps = 4;
-            slabs = (it.n + rps - 1) / rps;
-            PqtItem t = {it.x, mode == 1 ? it.err : nullptr, it.p, it.q, it.n, (int)it.m, it.r, (int)rps, (int)col_tiles};
-            table.push_back(t);
-            blocks.push_back((int)(col_tiles * slabs));
+            members.push_back(j);
             done[(size_t)j] = 1;
+        }
+        std::vector<PqtItem> table;
+        std::vector<int> blocks;
+        if (fast) {
+            pqt_rows_table(items, members, mode, &table, &blocks);
+        } else {
+            for (int j : members) {
+                const ConefPsgdItem& it = items[j];
+                const int64_t col_tiles = (it.m + 1023) / 1024;
+                int64_t slabs = (256 + col_tiles - 1) / col_tiles;
+                int64_t rps = (it.n + slabs - 1) / slabs;
+                if (rps < 4) rps = 4;
+                slabs = (it.n + rps - 1) / rps;
+                table.push_back(PqtItem{it.x, mode == 1 ? it.err : nullptr, it.p, it.q, it.n, (int)it.m, it.r, (int)rps,
+                                        (int)col_tiles, 256});
+                blocks.push_back((int)(col_tiles * slabs));
+            }
         }
         int rc = CONEF_OK;
         const GsAhead* ride = (ahead && ahead->count > 0 && table.size() == (size_t)count && count <= kPsgdBatchMax &&
@@ -3405,6 +3636,39 @@ int pqt_batch(const ConefPsgdItem* items, int count, int mode, float beta, int32
     return CONEF_OK;
 }
 
+// P = X Q with the Q factors of `its`, P orthogonalised, Q = X^T P into items[k].q, on the caller's factors.
+int round_products(const ConefPsgdItem* items, const ConefPsgdItem* its, int count, int mq_mode, float alpha, float eps,
+                   int32_t a, int32_t b, void* workspace, int64_t workspace_bytes, hipStream_t s)
+{
+    const char* defer_env = getenv("CONEF_ROUND_DEFER");
+    PaddedRound pr;
+    if (!(defer_env && defer_env[0] == '0') && padded_round(items, count, mq_mode, workspace, workspace_bytes, &pr)) {
+        const int r = items[0].r;
+        std::vector<float*> q_in;
+        std::vector<PadRowsItem> pad;
+        for (int k = 0; k < count; ++k) {
+            q_in.push_back(pr.padded ? pr.items[(size_t)k].q : its[k].q);
+            if (pr.padded) pad.push_back(PadRowsItem{its[k].q, pr.items[(size_t)k].q, its[k].m});
+        }
+        if (pr.padded)
+            if (int rc = pad_rows(pad, r, pr.rp, s); rc != CONEF_OK) return rc;
+        return deferred_products(pr, r, q_in.data(), mq_mode, alpha, eps, a, b, workspace, workspace_bytes, s, nullptr);
+    }
+    int rc = conef_psgd_mq_batch_f32(its, count, mq_mode, alpha, a, b, workspace, workspace_bytes, (void*)s);
+    if (rc != CONEF_OK) return rc;
+    std::vector<float*> mats;
+    std::vector<int64_t> rows;
+    std::vector<int32_t> ranks;
+    for (int k = 0; k < count; ++k) {
+        mats.push_back(items[k].p);
+        rows.push_back(items[k].n);
+        ranks.push_back(items[k].r);
+    }
+    rc = conef_gram_schmidt_batch_f32(mats.data(), rows.data(), ranks.data(), count, eps, workspace, workspace_bytes, (void*)s);
+    if (rc != CONEF_OK) return rc;
+    return conef_psgd_mtp_batch_f32(items, count, workspace, workspace_bytes, (void*)s);
+}
+
 }  // namespace
 
 extern "C" {
@@ -3418,8 +3682,10 @@ int64_t conef_psgd_batch_workspace_bytes(const ConefPsgdItem* items, int32_t cou
         int64_t b = conef_psgd_workspace_bytes(items[k].n, items[k].m, items[k].r);
         if (b > single) single = b;
     }
-    const int64_t launches = conef_align256(single) + conef_align256(4 * mtp_batch_layout(items, count, nullptr)) +
-                             conef_align256(4 * mfma_batch_layout(items, count, nullptr)) + defer_region_bytes(items, count);
+    int64_t launches = conef_align256(single) + conef_align256(4 * mtp_batch_layout(items, count, nullptr)) +
+                       conef_align256(4 * mfma_batch_layout(items, count, nullptr));
+    const int64_t padded = padded_round_bytes(items, count);
+    if (padded > launches) launches = padded;
     const int64_t small = conef_psgd_round_small_workspace_bytes(items, count);      // the one-launch round's records
     return small > launches ? small : launches;
 }
@@ -3521,81 +3787,88 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
         rows[(size_t)k] = items[k].m;
         ranks[(size_t)k] = items[k].r;
     }
-    // P = X Q, P orthogonalised, Q = X^T P: with the orthogonalisation deferred where the batch
-    // allows (round_products_deferred; CONEF_ROUND_DEFER=0 keeps the reference's order of steps,
-    // for comparisons), else as three steps
-    const char* defer_env = getenv("CONEF_ROUND_DEFER");      // read on every call: a test switches it
-    const bool defer_on = !(defer_env && defer_env[0] == '0');
+    for (int k = 0; k < count; ++k)
+        if ((pqt_mode == 1 || pqt_mode == 3) && !items[k].err) return CONEF_ERR_INVALID;
+    if (mq_mode < 0 || mq_mode > 2) return CONEF_ERR_INVALID;
+    for (int k = 0; k < count; ++k) {
+        const ConefPsgdItem& it = items[k];
+        if ((mq_mode == 1 && !it.err) || (mq_mode == 2 && (!it.cs || it.w < 1 || it.w > (1 << 30)))) return CONEF_ERR_INVALID;
+        if (mq_mode == 2 && it.plan_host && !conef_plan_matches((const ConefPlanHeader*)it.plan_host, it.n, it.m, it.w, a, b))
+            return CONEF_ERR_INVALID;
+        if ((flags & CONEF_ROUND_Q_READY) && !q_next[k]) return CONEF_ERR_INVALID;
+    }
+    hipStream_t hs = (hipStream_t)stream;
     GsAhead ahead;
     ahead.count = 0;
     for (int k = 0; k < kPsgdBatchMax; ++k) {
         ahead.parts[k] = nullptr;
         ahead.nparts[k] = 0;
     }
-    // the next round's Q factors are wanted in q_next, by workgroups of this round's last launch
-    bool want_next = (flags & CONEF_ROUND_MAKE_NEXT) && pqt_mode <= 2 && count <= kPsgdBatchMax && rank_bound(items[0].r) <= 8;
-    for (int k = 0; k < count && want_next; ++k)
-        want_next = q_next[k] && items[k].r == items[0].r && aligned16(q_next[k]) && aligned16(items[k].q) &&
-                    items[k].m <= 0x7fffffffLL;
-    bool q_shares_made = false;
-    auto products = [&](const ConefPsgdItem* its) -> int {      // its: the items with the Q the first product reads
-        if (mq_mode < 0 || mq_mode > 2) return CONEF_ERR_INVALID;
-        for (int k = 0; k < count; ++k) {
-            const ConefPsgdItem& it = its[k];
-            if ((mq_mode == 1 && !it.err) || (mq_mode == 2 && (!it.cs || it.w < 1 || it.w > (1 << 30)))) return CONEF_ERR_INVALID;
-            if (mq_mode == 2 && it.plan_host && !conef_plan_matches((const ConefPlanHeader*)it.plan_host, it.n, it.m, it.w, a, b))
-                return CONEF_ERR_INVALID;
-        }
-        if (defer_on) {
-            hipStream_t hs = (hipStream_t)stream;
-            GsAhead* qs = want_next ? &ahead : nullptr;
-            const int rd = mq_mode == 0   ? round_products_deferred<0>(items, its, count, 0.f, eps, a, b, workspace, workspace_bytes, hs, qs)
-                           : mq_mode == 1 ? round_products_deferred<1>(items, its, count, 0.f, eps, a, b, workspace, workspace_bytes, hs, qs)
-                                          : round_products_deferred<2>(items, its, count, alpha, eps, a, b, workspace, workspace_bytes, hs, qs);
-            if (rd == CONEF_OK) q_shares_made = want_next;
-            if (rd != kMqsNoFit) return rd;
-            const int rm = round_products_deferred_mfma(items, its, count, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, hs);
-            if (rm != kMqsNoFit) return rm;
-        }
-        int rp = conef_psgd_mq_batch_f32(its, count, mq_mode, alpha, a, b, workspace, workspace_bytes, stream);
-        if (rp != CONEF_OK) return rp;
-        for (int k = 0; k < count; ++k) {
-            mats[(size_t)k] = items[k].p;
-            rows[(size_t)k] = items[k].n;
-        }
-        rp = conef_gram_schmidt_batch_f32(mats.data(), rows.data(), ranks.data(), count, eps, workspace, workspace_bytes, stream);
-        if (rp != CONEF_OK) return rp;
-        return conef_psgd_mtp_batch_f32(items, count, workspace, workspace_bytes, stream);
-    };
+    // the next round's Q factors are wanted in q_next
+    bool want_next = (flags & CONEF_ROUND_MAKE_NEXT) && count <= kPsgdBatchMax;
+    for (int k = 0; k < count && want_next; ++k) want_next = q_next[k] && items[k].r == items[0].r && items[k].m <= 0x7fffffffLL;
+    const int rp = rank_bound(items[0].r);
+    // P = X Q, P orthogonalised, Q = X^T P: with the orthogonalisation deferred where the batch
+    // allows (padded_round; CONEF_ROUND_DEFER=0 keeps the reference's order of steps, for
+    // comparisons), else as three steps
+    const char* defer_env = getenv("CONEF_ROUND_DEFER");      // read on every call: a test switches it
+    PaddedRound pr;
+    const bool deferred = !(defer_env && defer_env[0] == '0') &&
+                          padded_round(items, count, mq_mode, workspace, workspace_bytes, &pr);
+    const ConefPsgdItem* its = deferred ? pr.items.data() : items;       // whose factors the rest of the round reads
     int rc = CONEF_OK;
-    if (flags & CONEF_ROUND_Q_READY) {
-        // q_next holds this round's Q factors, orthogonalised at the end of the bucket's last round
-        std::vector<ConefPsgdItem> with_q(items, items + count);
-        for (int k = 0; k < count; ++k) {
-            if (!q_next[k]) return CONEF_ERR_INVALID;
-            with_q[(size_t)k].q = q_next[k];
+    if (deferred) {
+        // The Q the first product reads, rows of rp floats: q_next (orthogonalised at the end of the
+        // bucket's last round), else Q orthogonalised now
+        const int r = items[0].r;
+        std::vector<float*> q_in((size_t)count);
+        for (int k = 0; k < count; ++k) q_in[(size_t)k] = (flags & CONEF_ROUND_Q_READY) ? q_next[k] : pr.items[(size_t)k].q;
+        if (!(flags & CONEF_ROUND_Q_READY)) {
+            if (rp <= 8) {
+                rc = conef_gram_schmidt_batch_f32(mats.data(), rows.data(), ranks.data(), count, eps, workspace, workspace_bytes, stream);
+                if (rc != CONEF_OK) return rc;
+            }
+            if (pr.padded) {
+                std::vector<PadRowsItem> pad;
+                for (int k = 0; k < count; ++k) pad.push_back(PadRowsItem{items[k].q, pr.items[(size_t)k].q, items[k].m});
+                rc = pad_rows(pad, r, rp, hs);
+                if (rc != CONEF_OK) return rc;
+            }
+            if (rp > 8) {      // in place: a workgroup of the last launch reads its rows before it writes them
+                std::vector<const float*> src;
+                for (int k = 0; k < count; ++k) src.push_back(pr.items[(size_t)k].q);
+                rc = orthogonalise_by_gram_wide(pr, r, src, q_in.data(), eps, workspace, hs);
+                if (rc != CONEF_OK) return rc;
+            }
         }
-        rc = products(with_q.data());
-    } else {
-        rc = conef_gram_schmidt_batch_f32(mats.data(), rows.data(), ranks.data(), count, eps, workspace, workspace_bytes, stream);
+        GsAhead* qs = want_next && rp <= 8 ? &ahead : nullptr;
+        rc = deferred_products(pr, r, q_in.data(), mq_mode, alpha, eps, a, b, workspace, workspace_bytes, hs, qs);
         if (rc != CONEF_OK) return rc;
-        rc = products(items);
+    } else {
+        std::vector<ConefPsgdItem> first(items, items + count);
+        if (flags & CONEF_ROUND_Q_READY) {
+            for (int k = 0; k < count; ++k) first[(size_t)k].q = q_next[k];
+        } else {
+            rc = conef_gram_schmidt_batch_f32(mats.data(), rows.data(), ranks.data(), count, eps, workspace, workspace_bytes, stream);
+            if (rc != CONEF_OK) return rc;
+        }
+        rc = round_products(items, first.data(), count, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, hs);
+        if (rc != CONEF_OK) return rc;
     }
-    if (rc != CONEF_OK) return rc;
-    // The new Q factors orthogonalised into q_next by workgroups of the last launch, where that
-    // launch covers the whole bucket (one rank, at most 8): from the shares of Q^T Q when the
-    // products above left them, else by the column steps themselves, which takes a short Q factor.
-    if (want_next) {
+    // The new Q factors orthogonalised into q_next, ranks up to 8: by workgroups of the last launch,
+    // where that launch covers the whole bucket; from the shares of Q^T Q when the products above left
+    // them, else by the column steps themselves, which takes a short Q factor.
+    if (want_next && rp <= 8 && pqt_mode <= 2) {
         bool ok = true;
-        for (int k = 0; k < count && ok && !q_shares_made; ++k)
+        for (int k = 0; k < count && ok && !deferred; ++k)
             ok = gs_reg_class(items[k].q, items[k].m, items[k].r) >= 0 &&
                  items[k].m <= (int64_t)kGsAheadRowSlots * kGsRegThreads;
         if (ok) {
             for (int k = 0; k < count; ++k) {
-                ahead.src[k] = items[k].q;
+                ahead.src[k] = its[k].q;
                 ahead.dst[k] = q_next[k];
                 ahead.rows[k] = (int)items[k].m;
-                if (!q_shares_made) ahead.parts[k] = nullptr;
+                if (!deferred) ahead.parts[k] = nullptr;
             }
             ahead.count = count;
             ahead.r = items[0].r;
@@ -3603,13 +3876,44 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
         }
     }
     bool used = false;
-    for (int k = 0; k < count; ++k)
-        if ((pqt_mode == 1 || pqt_mode == 3) && !items[k].err) return CONEF_ERR_INVALID;
-    rc = pqt_batch(items, count, pqt_mode == 3 ? 1 : pqt_mode, pqt_mode == 2 ? beta : 0.f, a, b, (hipStream_t)stream,
+    rc = pqt_batch(its, count, pqt_mode == 3 ? 1 : pqt_mode, pqt_mode == 2 ? beta : 0.f, a, b, hs,
                    ahead.count ? &ahead : nullptr, &used);
     if (rc != CONEF_OK) return rc;
+    if (want_next && deferred && rp > 8) {
+        std::vector<const float*> src;
+        for (int k = 0; k < count; ++k) src.push_back(its[k].q);
+        rc = orthogonalise_by_gram_wide(pr, items[0].r, src, q_next, eps, workspace, hs);
+        if (rc != CONEF_OK) return rc;
+        used = true;
+    }
     if (made) *made = used ? 1 : 0;
     if (pqt_mode == 3) rc = conef_psgd_sketch_update_batch_f32(items, count, beta, a, b, stream);
+    return rc;
+}
+
+// The second half of CONEF_ROUND_MAKE_NEXT at ranks 9 to 32 as a call of its own (for another stream).
+int conef_psgd_q_next_f32(const ConefPsgdItem* items, int32_t count, float eps, float* const* q_next, int32_t* made,
+                          void* workspace, int64_t workspace_bytes, void* stream)
+{
+    if (!made || count < 0 || (count > 0 && (!items || !q_next))) return CONEF_ERR_INVALID;
+    *made = 0;
+    for (int k = 0; k < count; ++k)
+        if (!item_ok(items[k]) || !q_next[k]) return CONEF_ERR_INVALID;
+    const char* defer_env = getenv("CONEF_ROUND_DEFER");
+    PaddedRound pr;
+    if ((defer_env && defer_env[0] == '0') || !padded_round(items, count, 0, workspace, workspace_bytes, &pr) || pr.rp <= 8)
+        return CONEF_OK;
+    hipStream_t s = (hipStream_t)stream;
+    std::vector<const float*> src;
+    std::vector<PadRowsItem> pad;
+    for (int k = 0; k < count; ++k) {
+        src.push_back(pr.padded ? q_next[k] : items[k].q);
+        pad.push_back(PadRowsItem{items[k].q, q_next[k], items[k].m});
+    }
+    if (pr.padded)
+        if (int rc = pad_rows(pad, items[0].r, pr.rp, s); rc != CONEF_OK) return rc;
+    const int rc = orthogonalise_by_gram_wide(pr, items[0].r, src, q_next, eps, workspace, s);
+    if (rc == CONEF_OK) *made = 1;
     return rc;
 }
 
@@ -3770,10 +4074,9 @@ int conef_psgd_round_f32(const ConefPsgdItem* items, int32_t count, int32_t mq_m
                                       workspace, workspace_bytes, stream);
 }
 
-// The middle of a round as a call of its own, for a caller that splits the round (the hooks at
-// ranks above 8 do, to run the Gram-Schmidt of the new Q on a side stream): P = X Q with the Q of
-// `first` (items whose q may point elsewhere, or null for items' own), P orthogonalised,
-// Q = X^T P into items[k].q - deferred where the batch allows, as in conef_psgd_round_f32.
+// The middle of a round as a call of its own, for a caller that splits the round: P = X Q with the Q of
+// `first` (items whose q may point elsewhere, or null for items' own), P orthogonalised, Q = X^T P into
+// items[k].q - deferred where the batch allows, as in conef_psgd_round_f32.
 int conef_psgd_products_f32(const ConefPsgdItem* items, const ConefPsgdItem* first, int32_t count, int32_t mq_mode,
                             float alpha, float eps, int32_t a, int32_t b, void* workspace, int64_t workspace_bytes,
                             void* stream)
@@ -3790,29 +4093,7 @@ int conef_psgd_products_f32(const ConefPsgdItem* items, const ConefPsgdItem* fir
         if (mq_mode == 2 && it.plan_host && !conef_plan_matches((const ConefPlanHeader*)it.plan_host, it.n, it.m, it.w, a, b))
             return CONEF_ERR_INVALID;
     }
-    const char* defer_env = getenv("CONEF_ROUND_DEFER");
-    if (!(defer_env && defer_env[0] == '0')) {
-        hipStream_t hs = (hipStream_t)stream;
-        const int rd = mq_mode == 0   ? round_products_deferred<0>(items, its, count, 0.f, eps, a, b, workspace, workspace_bytes, hs, nullptr)
-                       : mq_mode == 1 ? round_products_deferred<1>(items, its, count, 0.f, eps, a, b, workspace, workspace_bytes, hs, nullptr)
-                                      : round_products_deferred<2>(items, its, count, alpha, eps, a, b, workspace, workspace_bytes, hs, nullptr);
-        if (rd != kMqsNoFit) return rd;
-        const int rm = round_products_deferred_mfma(items, its, count, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, hs);
-        if (rm != kMqsNoFit) return rm;
-    }
-    int rc = conef_psgd_mq_batch_f32(its, count, mq_mode, alpha, a, b, workspace, workspace_bytes, stream);
-    if (rc != CONEF_OK) return rc;
-    std::vector<float*> mats((size_t)count);
-    std::vector<int64_t> rows((size_t)count);
-    std::vector<int32_t> ranks((size_t)count);
-    for (int k = 0; k < count; ++k) {
-        mats[(size_t)k] = items[k].p;
-        rows[(size_t)k] = items[k].n;
-        ranks[(size_t)k] = items[k].r;
-    }
-    rc = conef_gram_schmidt_batch_f32(mats.data(), rows.data(), ranks.data(), count, eps, workspace, workspace_bytes, stream);
-    if (rc != CONEF_OK) return rc;
-    return conef_psgd_mtp_batch_f32(items, count, workspace, workspace_bytes, stream);
+    return round_products(items, its, count, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 // dense error feedback on the parts of a bucket that are not compressed: x += e; e = 0
@@ -3822,23 +4103,68 @@ int conef_ef_passthrough_f32(float* x, float* err, int64_t count, void* stream);
 }  // extern "C"
 
 namespace {
-__global__ void ef_passthrough_kernel(float* __restrict__ x, float* __restrict__ err, int64_t count)
+// x += e; e = 0 over up to kEfSpans stretches of a bucket in one launch: a model's bucket holds dozens of
+// biases and norms between its matrices, and a launch each was most of a small model's step (3 to 4 us
+// a tensor).  Workgroup b of a stretch takes elements b * 256 .. of it, striding by its workgroups.
+constexpr int kEfSpans = 96;
+struct EfSpans {
+    float* x[kEfSpans];
+    float* err[kEfSpans];
+    int count[kEfSpans];
+    int first[kEfSpans + 1];
+    int spans;
+};
+
+__global__ void __launch_bounds__(256)
+ef_passthrough_kernel(EfSpans b)
 {
-    int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (; i < count; i += stride) {
+    int lo = 0, hi = b.spans - 1;                          // the last stretch that starts at or before this workgroup
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (b.first[mid] <= (int)blockIdx.x) lo = mid;
+        else hi = mid - 1;
+    }
+    float* x = b.x[lo];
+    float* err = b.err[lo];
+    const int step = (b.first[lo + 1] - b.first[lo]) * 256;
+    for (int i = ((int)blockIdx.x - b.first[lo]) * 256 + threadIdx.x; i < b.count[lo]; i += step) {
         x[i] = __fadd_rn(x[i], err[i]);
         err[i] = 0.f;
     }
 }
 }  // namespace
 
+// The same over `spans` stretches: x[k][0 .. counts[k]) and err[k][0 .. counts[k]) (host arrays of device pointers).
+extern "C" int conef_ef_passthrough_batch_f32(float* const* x, float* const* err, const int64_t* counts, int32_t spans,
+                                              void* stream)
+{
+    if (spans < 0 || (spans > 0 && (!x || !err || !counts))) return CONEF_ERR_INVALID;
+    for (int k = 0; k < spans; ++k)
+        if (counts[k] < 0 || (counts[k] > 0 && (!x[k] || !err[k]))) return CONEF_ERR_INVALID;
+    constexpr int64_t kPiece = (int64_t)1 << 30;           // indices are 32 bits wide
+    EfSpans b;
+    b.spans = 0;
+    b.first[0] = 0;
+    auto flush = [&]() {
+        if (b.spans > 0)
+            hipLaunchKernelGGL(ef_passthrough_kernel, dim3((unsigned)b.first[b.spans]), dim3(256), 0, (hipStream_t)stream, b);
+        b.spans = 0;
+    };
+    for (int k = 0; k < spans; ++k)
+        for (int64_t at = 0; at < counts[k]; at += kPiece) {
+            const int64_t n = counts[k] - at < kPiece ? counts[k] - at : kPiece;
+            b.x[b.spans] = x[k] + at;
+            b.err[b.spans] = err[k] + at;
+            b.count[b.spans] = (int)n;
+            const int64_t wgs = (n + 255) / 256;
+            b.first[b.spans + 1] = b.first[b.spans] + (int)(wgs < 4096 ? wgs : 4096);
+            if (++b.spans == kEfSpans) flush();
+        }
+    flush();
+    return (int)hipGetLastError();
+}
+
 extern "C" int conef_ef_passthrough_f32(float* x, float* err, int64_t count, void* stream)
 {
-    if (count < 0 || (count > 0 && (!x || !err))) return CONEF_ERR_INVALID;
-    if (count == 0) return CONEF_OK;
-    int64_t g = (count + 255) / 256;
-    if (g > 4096) g = 4096;
-    hipLaunchKernelGGL(ef_passthrough_kernel, dim3((unsigned)g), dim3(256), 0, (hipStream_t)stream, x, err, count);
-    return (int)hipGetLastError();
+    return conef_ef_passthrough_batch_f32(&x, &err, &count, 1, stream);
 }

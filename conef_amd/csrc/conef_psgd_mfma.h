@@ -36,7 +36,9 @@ constexpr int kMfmaThreads = 64 * kMfmaWaves;
 // X[row][c .. c+3] with c = block + 8u + 4 * half for u = 0..3 and feeds step (u, j) with component j;
 // the matching B operand is Q[c + j][l % 32].  The waves' tiles meet in LDS in a fixed order; with
 // more than one column split the tile goes to a partial buffer [split][n][r] that a second kernel
-// adds up in split order.  Requires m % 4 == 0 and 16-byte aligned x (err, pktab).
+// adds up in split order.  Rows of any length from four up and any alignment: a row's last quad is
+// moved back to end with the row (conef_quad_col), its columns that are the quad's before it count
+// as zeros.
 template <int MODE>
 __device__ __forceinline__ void
 psgd_mfma_mq_body(float* __restrict__ x, const float* __restrict__ err, const float* __restrict__ cs,
@@ -76,17 +78,13 @@ psgd_mfma_mq_body(float* __restrict__ x, const float* __restrict__ err, const fl
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int c = cb + 8 * u + 4 * half;
-            const int cc = c < c_end ? c : c_begin;     // a valid quad, its products are zeroed
-            float4 t = *reinterpret_cast<const float4*>(xrow + cc);
-            st.xv[u][0] = t.x; st.xv[u][1] = t.y; st.xv[u][2] = t.z; st.xv[u][3] = t.w;
-            if (MODE == 1) {
-                float4 e = *reinterpret_cast<const float4*>(erow + cc);
-                st.ev[u][0] = e.x; st.ev[u][1] = e.y; st.ev[u][2] = e.z; st.ev[u][3] = e.w;
-            }
+            const int ce = c < c_end ? c : c_begin;     // past the end: a valid quad, its products are zeroed
+            const int cc = ce + 4 <= m ? ce : m - 4;
+            conef_ld4u(xrow + cc, st.xv[u]);
+            if (MODE == 1) conef_ld4u(erow + cc, st.ev[u]);
             if (MODE == 2) {
                 if (pktab) {
-                    uint4 p4 = *reinterpret_cast<const uint4*>(pktab + cc);
-                    st.pk[u][0] = p4.x; st.pk[u][1] = p4.y; st.pk[u][2] = p4.z; st.pk[u][3] = p4.w;
+                    conef_ld4u(pktab + cc, st.pk[u]);
                 } else {
 #pragma unroll
                     for (int j = 0; j < 4; ++j) st.pk[u][j] = conef_bucket_sign(cc + j, mod, hs.a, hs.b, hs.sa, hs.sb);
@@ -99,7 +97,9 @@ psgd_mfma_mq_body(float* __restrict__ x, const float* __restrict__ err, const fl
     auto compute = [&](Stage& st, int cb) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const bool ok = cb + 8 * u + 4 * half < c_end;
+            const int c = cb + 8 * u + 4 * half;
+            const bool ok = c < c_end;
+            const int dup = ok && c + 4 > m ? c - (m - 4) : 0;
             if (MODE == 1) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) st.xv[u][j] = __fadd_rn(st.xv[u][j], st.ev[u][j]);
@@ -110,12 +110,10 @@ psgd_mfma_mq_body(float* __restrict__ x, const float* __restrict__ err, const fl
                     st.xv[u][j] = __fadd_rn(st.xv[u][j], conef_query_term(cells[lrow * w + (st.pk[u][j] & 0x7fffffffu)],
                                                                           st.pk[u][j], alpha));
             }
-            if (MODE != 0 && ok && row_ok)
-                *reinterpret_cast<float4*>(xrow + cb + 8 * u + 4 * half) =
-                    make_float4(st.xv[u][0], st.xv[u][1], st.xv[u][2], st.xv[u][3]);
+            if (MODE != 0 && ok && row_ok) conef_st4_own(xrow + c - dup, st.xv[u], dup);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                float a = ok ? st.xv[u][j] : 0.f;
+                float a = ok && j >= dup ? st.xv[u][j] : 0.f;
                 float b = (ok && rank_ok) ? st.qv[u][j] : 0.f;
                 acc = conef_mfma32(a, b, acc);
             }
@@ -168,7 +166,8 @@ psgd_mfma_mq_kernel(float* __restrict__ x, const float* __restrict__ err, const 
 // (q = l % 32, half) reads X[i][c0 + V*q .. + V) of row i = pair + half) and keeps V tiles, tile t
 // for the columns c0 + V*q + t; a step consumes two rows.  The four waves of a workgroup split the
 // rows of the slab, meet in LDS, and the slab's tile is stored (one slab) or left as a partial.
-// Requires m % V == 0 and V*4-byte aligned x.
+// Any alignment, any m >= V: the last run of V columns is moved back to end with the row (columns
+// two lanes then hold come out of both the same).
 template <int V>
 __device__ __forceinline__ void
 psgd_mfma_mtp_body(const float* __restrict__ x, const float* __restrict__ p, float* __restrict__ out, int64_t n, int m,
@@ -180,7 +179,7 @@ psgd_mfma_mtp_body(const float* __restrict__ x, const float* __restrict__ p, flo
     const int c0 = bx * 32 * V;
     const int c = c0 + V * lq;
     const bool col_ok = c < m;
-    const int cc = col_ok ? c : 0;
+    const int cc = col_ok ? (c + V <= m ? c : m - V) : 0;
     const int64_t i0 = (int64_t)by * rows_per_slab;
     const int64_t i1 = i0 + rows_per_slab < n ? i0 + rows_per_slab : n;
     const bool rank_ok = lq < r;
@@ -200,10 +199,9 @@ psgd_mfma_mtp_body(const float* __restrict__ x, const float* __restrict__ p, flo
             const int64_t ii = i < i1 ? i : i0;         // past the slab: a valid row, its products are zeroed
             const float* src = x + ii * m + cc;
             if constexpr (V == 4) {
-                float4 t = *reinterpret_cast<const float4*>(src);
-                st.xv[u][0] = t.x; st.xv[u][1] = t.y; st.xv[u][2] = t.z; st.xv[u][3] = t.w;
+                conef_ld4u(src, st.xv[u]);
             } else if constexpr (V == 2) {
-                float2 t = *reinterpret_cast<const float2*>(src);
+                conef_f2u t = *reinterpret_cast<const conef_f2u*>(src);
                 st.xv[u][0] = t.x; st.xv[u][1] = t.y;
             } else {
                 st.xv[u][0] = *src;
@@ -249,9 +247,10 @@ psgd_mfma_mtp_body(const float* __restrict__ x, const float* __restrict__ p, flo
             const int v = e >> 6, l = e & 63;
             const float* rr = &red[0][0][0];
             float s = (rr[e] + rr[16 * 64 + e]) + (rr[2 * 16 * 64 + e] + rr[3 * 16 * 64 + e]);
-            const int col = c0 + V * conef_mfma_row(v, l) + t;
+            const int cq = c0 + V * conef_mfma_row(v, l);                // the lane's run of columns, as it was loaded
+            const int col = (cq + V <= m ? cq : m - V) + t;
             const int j = l & 31;
-            if (col < m && j < r) dst[(int64_t)col * r + j] = s;
+            if (cq < m && j < r) dst[(int64_t)col * r + j] = s;
         }
     }
 }
@@ -286,8 +285,7 @@ psgd_mfma_pqt_body(float* __restrict__ x, float* __restrict__ err, const float* 
         const float* src = q + (int64_t)(col_ok ? c : m - 1) * R + half * KS;
 #pragma unroll
         for (int s = 0; s < KS; s += 4) {
-            float4 t = *reinterpret_cast<const float4*>(src + s);
-            qb[s] = t.x; qb[s + 1] = t.y; qb[s + 2] = t.z; qb[s + 3] = t.w;
+            conef_ld4u(src + s, qb + s);
         }
     }
     const int64_t i0 = (int64_t)by * rows_per_slab;
@@ -299,8 +297,7 @@ psgd_mfma_pqt_body(float* __restrict__ x, float* __restrict__ err, const float* 
             const float* src = p + i * R + half * KS;
 #pragma unroll
             for (int s = 0; s < KS; s += 4) {
-                float4 t = *reinterpret_cast<const float4*>(src + s);
-                pa[s] = t.x; pa[s + 1] = t.y; pa[s + 2] = t.z; pa[s + 3] = t.w;
+                conef_ld4u(src + s, pa + s);
             }
         }
         if (MODE == 1) {

@@ -17,16 +17,6 @@
 #include <stdint.h>
 #include "conef_device.h"
 
-__device__ __forceinline__ void mqs_ld4(const float* p, float* v)
-{
-    const float4 t = *reinterpret_cast<const float4*>(p);
-    v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
-}
-__device__ __forceinline__ void mqs_st4(float* p, const float* v)
-{
-    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-}
-
 struct MqsItem {
     float* x;
     const float* err;
@@ -46,7 +36,7 @@ struct MqsItem {
 // threads of a group for a matrix of m columns in a workgroup of T threads
 inline int mqs_group_width(int64_t m, int T)
 {
-    const int64_t m4 = m >> 2;
+    const int64_t m4 = (m + 3) >> 2;
     const int64_t nslab = (m4 + T - 1) / T;
     int64_t gw = ((m4 + nslab - 1) / nslab + 63) / 64 * 64;
     if (gw < 64) gw = 64;
@@ -67,7 +57,7 @@ inline int64_t mqs_workgroups(int64_t n, int gw, int S, int T)
 
 inline size_t mqs_lds_bytes(int64_t m, int w, int gw, int S, int T, int rp, bool sketch, bool gram = false)
 {
-    const int64_t m4 = m >> 2;
+    const int64_t m4 = (m + 3) >> 2;
     const int64_t niter = (m4 + gw - 1) / gw * (S >> 2);
     return (size_t)niter * (T / 64) * 4 * rp * 4 + (sketch ? (size_t)(T / gw) * S * w * 4 : 0) +
            (gram ? (size_t)(T / gw) * S * rp * 4 : 0);
@@ -82,7 +72,7 @@ inline bool mqs_plan_launch(const MqsItem* items, int count, int rp, bool sketch
 {
     int T = 256;
     for (int k = 0; k < count; ++k)
-        if ((items[k].m >> 2) > 512) T = 1024;
+        if (((items[k].m + 3) >> 2) > 512) T = 1024;
     const int want = T == 256 ? 384 : 160;
     for (int S = T == 256 ? 16 : 8; S >= 4; S >>= 1) {
         int64_t wgs = 0;
@@ -96,7 +86,8 @@ inline bool mqs_plan_launch(const MqsItem* items, int count, int rp, bool sketch
         if (lds > 64 * 1024) continue;
         // a launch that cannot give every CU a workgroup's worth of threads is better served by the
         // row-block kernel, whose workgroups are a row or four each
-        if (S == 4 && wgs * T < 256 * 256) return false;
+        // (not where the caller wants the shares of P^T P: those save it more launches than that)
+        if (S == 4 && wgs * T < 256 * 256 && !gram) return false;
         if (wgs >= want || S == 4) {
             *T_out = T;
             *S_out = S;
@@ -142,7 +133,7 @@ psgd_mqs_body(const MqsItem& it, float alpha, ConefSeeds hs, int bx)
     constexpr int WAVES = T / 64;
     constexpr int kShift = NV >= 32 ? 1 : NV >= 16 ? 2 : NV >= 8 ? 3 : NV >= 4 ? 4 : 5;   // 6 - log2 NV
     extern __shared__ float mqs_lds[];
-    const int m = it.m, m4 = m >> 2, w = it.w, gw = it.gw, S = it.S;
+    const int m = it.m, m4 = (m + 3) >> 2, w = it.w, gw = it.gw, S = it.S;
     const int64_t n = it.n;
     const int groups = T / gw;
     const int nslab = (m4 + gw - 1) / gw;
@@ -172,9 +163,9 @@ psgd_mqs_body(const MqsItem& it, float alpha, ConefSeeds hs, int bx)
         const int j = quad_of(slab);
 #pragma unroll
         for (int a = 0; a < 4; ++a) {
-            const int64_t off = (wg_row0 + local_row(b, a)) * m + 4 * j;
-            mqs_ld4(it.x + off, xn[a]);
-            if (MODE == 1) mqs_ld4(it.err + off, en[a]);
+            const int64_t off = (wg_row0 + local_row(b, a)) * m + conef_quad_col(j, m);
+            conef_ld4u(it.x + off, xn[a]);
+            if (MODE == 1) conef_ld4u(it.err + off, en[a]);
         }
     };
     request(0);
@@ -186,25 +177,27 @@ psgd_mqs_body(const MqsItem& it, float alpha, ConefSeeds hs, int bx)
     float qreg[4 * RP];
     uint32_t pk[4] = {0u, 0u, 0u, 0u};
     bool valid = false;
-    int j = 0;
+    int col = 0, dup = 0;
     for (int iter = 0; iter < niter; ++iter) {
         const int slab = iter / nblk, b = iter - slab * nblk;
         if (b == 0) {
-            j = quad_of(slab);
+            const int j = quad_of(slab);
+            col = conef_quad_col(j, m);
+            dup = 4 * j - col;
             valid = !idle && slab * gw + gt < m4;
 #pragma unroll
-            for (int t = 0; t < RP; ++t) mqs_ld4(it.q + (int64_t)j * 4 * RP + 4 * t, qreg + 4 * t);
-            if (!valid) {                                  // a duplicate of the last quad: it adds nothing
+            for (int t = 0; t < RP; ++t) conef_ld4u(it.q + (int64_t)col * RP + 4 * t, qreg + 4 * t);
+            if (!valid || dup) {        // another thread's columns (the last quad a second time, a moved quad's first ones): they add nothing
 #pragma unroll
-                for (int t = 0; t < 4 * RP; ++t) qreg[t] = 0.f;
+                for (int t = 0; t < 4 * RP; ++t)
+                    if (!valid || t / RP < dup) qreg[t] = 0.f;
             }
             if (MODE == 2) {
                 if (it.pktab) {
-                    const uint4 t = reinterpret_cast<const uint4*>(it.pktab)[j];
-                    pk[0] = t.x; pk[1] = t.y; pk[2] = t.z; pk[3] = t.w;
+                    conef_ld4u(it.pktab + col, pk);
                 } else {
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) pk[k] = conef_bucket_sign(4 * j + k, it.mod, hs.a, hs.b, hs.sa, hs.sb);
+                    for (int k = 0; k < 4; ++k) pk[k] = conef_bucket_sign(col + k, it.mod, hs.a, hs.b, hs.sa, hs.sb);
                 }
             }
         }
@@ -226,7 +219,7 @@ psgd_mqs_body(const MqsItem& it, float alpha, ConefSeeds hs, int bx)
                 for (int k = 0; k < 4; ++k)
                     xv[a][k] = __fadd_rn(xv[a][k], conef_query_term(crow[pk[k] & 0x7fffffffu], pk[k], alpha));
             }
-            if (MODE != 0 && valid && lr < rows_here) mqs_st4(it.x + (wg_row0 + lr) * m + 4 * j, xv[a]);
+            if (MODE != 0 && valid && lr < rows_here) conef_st4_own(it.x + (wg_row0 + lr) * m + col, xv[a], dup);
         }
         float acc[NV];
 #pragma unroll

@@ -370,34 +370,41 @@ int conef_psgd_round_small_f32(const ConefPsgdItem* items, int32_t count, int32_
                                float beta, float eps, int32_t a, int32_t b, void* workspace, int64_t workspace_bytes,
                                void* stream);
 
-/* The middle of that round as a call of its own, for a caller that splits the round (the hooks above
- * rank 8 do, to orthogonalise the new Q on a side stream meanwhile): P = X Q with the Q factors of
- * `first` (a copy of `items` whose q may point elsewhere; null: items' own), P orthogonalised
- * (powerSGD_hook.py:516-531), Q = X^T P into items[k].q.  Deferred orthogonalisation of P where the
- * batch allows, as in conef_psgd_round_f32 (ranks 1, 2, 4, 8, 16, 32 of 16-byte shaped matrices). */
+/* The middle of that round as a call of its own, for a caller that splits the round: P = X Q with the Q
+ * factors of `first` (a copy of `items` whose q may point elsewhere; null: items' own), P orthogonalised
+ * (powerSGD_hook.py:516-531), Q = X^T P into items[k].q.  Deferred orthogonalisation of P where the batch
+ * allows, as in conef_psgd_round_f32. */
 int conef_psgd_products_f32(const ConefPsgdItem* items, const ConefPsgdItem* first, int32_t count, int32_t mq_mode,
                             float alpha, float eps, int32_t a, int32_t b, void* workspace, int64_t workspace_bytes,
                             void* stream);
 
-/* The same round for callers that keep a second buffer per Q factor (q_next[k], [m,r] like items[k].q).
- * The reference orthogonalises a bucket's Q factors at the start of the bucket's next round
- * (powerSGD_hook.py:496-497), a launch of a few workgroups with the machine idle around it.  Here
- * flags & CONEF_ROUND_MAKE_NEXT asks for that to be done at the end of this round instead, out of
- * place into q_next, by workgroups that ride along in the round's last launch; *made tells whether it
- * was (only for pqt_mode 0..2 over a bucket of at most 24 matrices of one rank <= 8 whose Q factors have
- * at most 1024 rows).  items[k].q keeps what the reference keeps there.  In the next round
- * flags & CONEF_ROUND_Q_READY says q_next holds the orthogonal Q factors: the first step is left out
- * and P = M Q reads them.  Same arithmetic on the same values either way.  No counterpart in the
- * reference's interface. */
+/* The same round for callers that keep a second buffer per Q factor.  The reference orthogonalises a
+ * bucket's Q factors at the start of the bucket's next round (powerSGD_hook.py:496-497), a few short
+ * launches with the machine idle around them.  Here flags & CONEF_ROUND_MAKE_NEXT asks for that to be
+ * done at the end of this round instead, out of place into q_next; *made tells whether it was (a bucket
+ * of at most 24 matrices of one rank).  items[k].q keeps what the reference keeps there.  In the next
+ * round flags & CONEF_ROUND_Q_READY says q_next holds the orthogonal Q factors: the first step is left
+ * out and P = M Q reads them.  q_next[k] belongs to the library between the two calls: m rows of as many
+ * floats as the next of 1, 2, 4, 8, 16 and 32 that is not below the rank.  No counterpart in the reference's
+ * interface. */
 #define CONEF_ROUND_Q_READY 1
 #define CONEF_ROUND_MAKE_NEXT 2
 int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_t mq_mode, int32_t pqt_mode, float alpha,
                                float beta, float eps, int32_t a, int32_t b, float* const* q_next, int32_t flags,
                                int32_t* made, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The second half of CONEF_ROUND_MAKE_NEXT as a call of its own, at ranks 9 to 32, for a caller that runs it
+ * on another stream (with a workspace of its own) once the round's Q factors are final: items[k].q into
+ * q_next[k].  *made is 0, and nothing is launched, for a bucket that call would not have done it for. */
+int conef_psgd_q_next_f32(const ConefPsgdItem* items, int32_t count, float eps, float* const* q_next, int32_t* made,
+                          void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Dense error feedback on a stretch of the bucket that is not compressed: x += err; err = 0
  * (the copy-minus-result of powerSGD_hook.py:558 is exactly zero there). */
 int conef_ef_passthrough_f32(float* x, float* err, int64_t count, void* stream);
+/* The same over `spans` stretches in one launch per 96 of them: x[k], err[k] (device pointers in host
+ * arrays), counts[k] elements each. */
+int conef_ef_passthrough_batch_f32(float* const* x, float* const* err, const int64_t* counts, int32_t spans, void* stream);
 
 /* ------------------------------------------------------------- magnitude top-k ---------- */
 

@@ -1071,6 +1071,41 @@ def test_high_rank_rounds_orthogonalise_q_on_a_side_stream(monkeypatch, rank, mo
         np.testing.assert_array_equal(x, y)
 
 
+# matrices whose rows are no whole number of quads and start anywhere in memory; widths at the edges of a
+# quad, a wave's and a workgroup's quads, and a column tile; heights at the edges of a row block
+RAGGED_BUCKETS = [
+    [(3,), (70, 65), (1,), (61, 254), (37, 257), (2,), (130, 126), (600, 5), (300, 7), (5, 300)],
+    [(1,), (64, 1023), (2,), (35, 2049), (3,), (33, 4097), (2050, 66)],
+]
+
+
+@pytest.mark.parametrize("rank", [1, 2, 3, 5, 8, 9, 17, 32])
+@pytest.mark.parametrize("mode", [None, "ef", "conef", "topk"])
+def test_rounds_at_any_rank_and_alignment(monkeypatch, oracle, mode, rank):
+    """Rounds of the separate launches at ranks between the kernels' sizes (copies of the factors with zero
+    columns) and on rows of any length and alignment (the last quad of a row moved back to end with it),
+    against the oracle with the state carried over three steps."""
+    monkeypatch.setenv("CONEF_ROUND_SMALL", "0")
+    for shapes in RAGGED_BUCKETS:
+        st, hook = _state_for(mode, rank, 0.3)
+        ost = oracle.PowerSGDOracle(matrix_approximation_rank=rank, error_mode=mode, sketch_size=0.3, beta=0.9, topk_ratio=0.4)
+        run_steps(hook, st, ost, shapes, 3, check=psgd_check_factory(st, ost, mode),
+                  resync=psgd_resync_factory(st, ost, mode, free_steps=1))
+        assert st.round_cache[0].q_next_ready == (st.round_cache[0].count > 0)
+
+
+@pytest.mark.parametrize("small", ["0", "1"])
+@pytest.mark.parametrize("mode,rank", [("ef", 3), ("conef", 4)])
+def test_round_of_more_matrices_than_a_launch_takes(monkeypatch, oracle, mode, rank, small):
+    monkeypatch.setenv("CONEF_ROUND_SMALL", small)
+    shapes = [(24 + k, 50 + 3 * k) for k in range(25)] + [(7,)]
+    st, hook = _state_for(mode, rank, 0.3)
+    ost = oracle.PowerSGDOracle(matrix_approximation_rank=rank, error_mode=mode, sketch_size=0.3, beta=0.9)
+    run_steps(hook, st, ost, shapes, 3, check=psgd_check_factory(st, ost, mode),
+              resync=psgd_resync_factory(st, ost, mode, free_steps=1))
+    assert len(st.round_cache[0].chunks) == 2
+
+
 def test_powersgd_state_errors_and_warmup():
     from conef_amd.powerSGD_hook import PowerSGDState, _should_compress, powerSGD_hook
     with pytest.raises(ValueError, match="Expect `start_powerSGD_iter` > 1"):
