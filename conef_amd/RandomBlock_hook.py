@@ -111,16 +111,17 @@ class _BucketTable:
     """What a bucket's step needs, worked out once: the >= 2-D gradients as matrices, their block
     sizes, payload slices and the item table the batch entry point reads.  Rebuilt when the
     bucket's buffer or layout changes."""
-    __slots__ = ("key", "shapes", "matrices", "uncompressed", "numels", "blocks", "offsets", "items", "count")
+    __slots__ = ("key", "sig", "matrices", "uncompressed", "numels", "blocks", "offsets", "items", "count", "starts",
+                 "errors", "sketches", "moving", "need")
 
 
-def _build_table(state, grads, shapes, key, device, bucket_index, errors):
+def _build_table(state, grads, key, device, bucket_index, errors):
     t = _BucketTable()
-    t.key, t.shapes = key, shapes
+    t.key, t.sig = key, _bucket.layout_signature(grads)
     t.matrices = [g.view(g.shape[0], -1) for g in grads if g.ndimension() > 1]
     t.uncompressed = [g for g in grads if g.ndimension() <= 1]
-    t.numels = [m.numel() for m in t.matrices]
-    t.blocks = [_block_size(state, n) for n in t.numels]
+    t.numels = np.array([m.numel() for m in t.matrices], dtype=np.int64)
+    t.blocks = [_block_size(state, n) for n in t.numels.tolist()]
     t.count = len(t.matrices)
     for cnt, matrix in enumerate(t.matrices):
         if len(errors) <= cnt:
@@ -132,6 +133,7 @@ def _build_table(state, grads, shapes, key, device, bucket_index, errors):
         state.compressed_tensor_memory[bucket_index] = torch.empty(sum(t.blocks), dtype=torch.float32, device=device)
     payload_all = state.compressed_tensor_memory[bucket_index]
     t.items = (_lib.RandBlockItem * max(t.count, 1))()
+    t.starts = _lib.randblock_starts(t.items, t.count)
     t.offsets, idx = [], 0
     for cnt, (matrix, block) in enumerate(zip(t.matrices, t.blocks)):
         it = t.items[cnt]
@@ -140,7 +142,50 @@ def _build_table(state, grads, shapes, key, device, bucket_index, errors):
         it.n, it.m, it.block = matrix.shape[0], matrix.shape[1], block
         t.offsets.append(idx)
         idx += block
+    t.errors, t.sketches = None, []
     return t
+
+
+def _point_at_errors(state, t, errors):
+    """The error memory's places in the item table.  ``t.moving``: the sketches that are not updated in
+    place and swap two buffers, whose places a step takes anew; the others stay where they are."""
+    t.errors = list(errors)
+    t.moving, t.need = [], 0
+    t.sketches = []
+    for cnt, error in enumerate(errors[:t.count]):
+        it = t.items[cnt]
+        if not state.use_error_compression:
+            it.err = error.data_ptr()
+            continue
+        plan = error.plan()
+        it.w = error.range
+        it.plan_host, it.plan_dev = (plan.host_ptr, plan.device.data_ptr()) if plan is not None else (None, None)
+        it.staging = None
+        if plan is not None and plan.in_place:
+            it.cs_in = it.cs_out = error.cs.data_ptr()
+        else:
+            t.moving.append((it, error, plan))
+            # One staging buffer serves every binned sketch of the bucket (the launches run one after the
+            # other on the stream): it is sized for the largest of them
+            if plan is not None:
+                t.need = max(t.need, plan.workspace_bytes)
+    if state.use_error_compression:
+        moving = {id(error) for _, error, _ in t.moving}
+        t.sketches = [(error, error._plan, None if id(error) in moving else error.cs) for error in errors[:t.count]]
+
+
+def _errors_moved(t, errors):
+    """Whether a bucket's error memory is no longer what the table points at: other objects, a sketch whose
+    cells or plan were replaced."""
+    if t.errors is None or len(errors) != len(t.errors):
+        return True
+    for error, known in zip(errors, t.errors):
+        if error is not known:
+            return True
+    for error, plan, cells in t.sketches:
+        if error._plan is not plan or (cells is not None and error.cs is not cells):
+            return True
+    return False
 
 
 def RandomBlock_hook(state: RandomBlockState, bucket) -> torch.futures.Future[torch.Tensor]:
@@ -164,59 +209,37 @@ def RandomBlock_hook(state: RandomBlockState, bucket) -> torch.futures.Future[to
     errors = state.error_dict.setdefault(bucket_index, [])
 
     grads = _bucket.gradients(bucket)
-    shapes = [g.shape for g in grads]
     payload_all = state.compressed_tensor_memory.get(bucket_index)
     key = (input_tensor.data_ptr(), input_tensor.numel(), bool(state.use_error_compression), state.compression_ratio,
            payload_all.data_ptr() if payload_all is not None else 0)
     table = state.round_cache.get(bucket_index)
-    if table is None or table.key != key or table.shapes != shapes or len(errors) < table.count:
-        table = _build_table(state, grads, shapes, key, device, bucket_index, errors)
+    if table is None or table.key != key or table.sig != _bucket.layout_signature(grads) or len(errors) < table.count:
+        table = _build_table(state, grads, key, device, bucket_index, errors)
         payload_all = state.compressed_tensor_memory[bucket_index]
         table.key = key[:4] + (payload_all.data_ptr(),)
         state.round_cache[bucket_index] = table
+    if _errors_moved(table, errors):
+        _point_at_errors(state, table, errors)
     items, count = table.items, table.count
 
     alpha = 1 - state.beta          # python double, rounded to fp32 at the boundary (reference :190)
-    starts = []
-    randint = state.rng.randint     # RandomState.choice(n) of an int n draws randint(0, n): same stream (:218)
     written = []
-    staging = None
-    if state.use_error_compression:
-        # One staging buffer serves every binned sketch of the bucket (the launches run one after the
-        # other on this stream): it is sized for the largest of them before any pointer is taken, since
-        # the pool replaces its buffer when it has to grow.
-        need = max((p.workspace_bytes for p in (errors[cnt].plan() for cnt in range(count))
-                    if p is not None and not p.in_place), default=0)
-        if need:
-            staging = _pools.staging(device, stream, need).data_ptr()
-    for cnt in range(count):
-        it = items[cnt]
-        start = int(randint(0, table.numels[cnt]))             # one draw per tensor, in bucket order (:218)
-        it.start = start
-        starts.append(start)
-        error = errors[cnt]
-        if state.use_error_compression:
-            plan = error.plan()
-            it.w = error.range
-            it.cs_in = error.cs.data_ptr()
-            if plan is not None:
-                # the binned step reads the old sketch while it writes the new one
-                out = error.cs if plan.in_place else error.spare_buffer()
-                it.plan_host, it.plan_dev = plan.host_ptr, plan.device.data_ptr()
-                it.staging = None if plan.in_place else staging
-            else:
-                out = error.next_buffer()
-                it.plan_host = it.plan_dev = it.staging = None
-            it.cs_out = out.data_ptr()
-            written.append(out)
-        else:
-            it.err = error.data_ptr()
     if count:
+        # one draw per tensor, in bucket order (:218)
+        _bucket.draw_starts(state.rng, table.numels, items, table.starts)
+        if table.moving:
+            staging = _pools.staging(device, stream, table.need).data_ptr() if table.need else None
+            for it, error, plan in table.moving:
+                # the binned step reads the old sketch while it writes the new one
+                out = error.spare_buffer() if plan is not None else error.next_buffer()
+                it.cs_in, it.cs_out = error.cs.data_ptr(), out.data_ptr()
+                it.staging = staging if plan is not None else None
+                written.append((error, out))
         rc = lib.conef_randblock_step_batch_f32(items, count, 2 if state.use_error_compression else 1, float(alpha),
                                                 float(state.beta), HASH_A, HASH_B, stream)
         _lib.check(rc, "conef_randblock_step_batch_f32")
-    for error, out in zip(errors, written):
-        error.commit(out)
+        for error, out in written:
+            error.commit(out)
 
     if world_size == 1:
         # every all-reduce is the identity: the fused kernels already left zeros + block in place
@@ -226,7 +249,7 @@ def RandomBlock_hook(state: RandomBlockState, bucket) -> torch.futures.Future[to
     # More than one rank (not exercised on the single-GPU boxes this was developed on): average the
     # small tensors and the payload, then put the averaged block back.
     uncompressed = table.uncompressed
-    spans = [(m, st, bl, off) for m, st, bl, off in zip(table.matrices, starts, table.blocks, table.offsets)]
+    spans = list(zip(table.matrices, table.starts.tolist(), table.blocks, table.offsets))
     flat_small = (torch.cat([t.view(-1) for t in uncompressed]) if uncompressed
                   else torch.tensor([], device=device, dtype=input_tensor.dtype))
     fut = dist.all_reduce(flat_small, group=group, async_op=True).get_future()

@@ -78,12 +78,12 @@ def UnbiasedRandomBlock_hook(state: UnbiasedRandomBlockState, bucket) -> torch.f
     bucket_index = _bucket.index(bucket)
 
     grads = _bucket.gradients(bucket)
-    shapes = [g.shape for g in grads]
+    sig = _bucket.layout_signature(grads)
     payload_all = state.compressed_tensor_memory.get(bucket_index)
     key = (input_tensor.data_ptr(), input_tensor.numel(), state.compression_ratio,
            payload_all.data_ptr() if payload_all is not None else 0)
     table = state.round_cache.get(bucket_index)
-    if table is None or table[0] != key or table[1] != shapes:
+    if table is None or table[0] != key or table[1] != sig:
         # worked out once per bucket: the >= 2-D gradients, their block sizes and the item table
         tensors = [g for g in grads if g.ndimension() > 1]
         uncompressed = [g for g in grads if g.ndimension() <= 1]
@@ -99,25 +99,21 @@ def UnbiasedRandomBlock_hook(state: UnbiasedRandomBlockState, bucket) -> torch.f
             it.n, it.m, it.block = tensor.shape[0], numel // tensor.shape[0], block     # prob = block / numel is formed in the library (:155)
             offsets.append(idx)
             idx += block
-        table = (key[:3] + (payload_all.data_ptr(),), shapes, tensors, uncompressed, numels, blocks, offsets, items)
+        table = (key[:3] + (payload_all.data_ptr(),), sig, tensors, uncompressed, np.array(numels, dtype=np.int64), blocks, offsets,
+                 items, _lib.randblock_starts(items, len(tensors)))
         state.round_cache[bucket_index] = table
-    _, _, tensors, uncompressed, numels, blocks, offsets, items = table
+    _, _, tensors, uncompressed, numels, blocks, offsets, items, starts = table
     payload_all = state.compressed_tensor_memory[bucket_index]
 
-    starts = []
-    randint = state.rng.randint     # RandomState.choice(n) of an int n draws randint(0, n): same stream (:157)
-    for it, numel in zip(items, numels):
-        start = int(randint(0, numel))                          # :157
-        it.start = start
-        starts.append(start)
     if tensors:
+        _bucket.draw_starts(state.rng, numels, items, starts)              # :157
         rc = lib.conef_randblock_step_batch_f32(items, len(tensors), 0, 0.0, 0.0, 0, 0, stream)
         _lib.check(rc, "conef_randblock_step_batch_f32")
 
     if world_size == 1:
         state.maybe_increase_iter(bucket)
         return _bucket.completed_future(input_tensor)
-    spans = list(zip(tensors, starts, blocks, offsets))
+    spans = list(zip(tensors, starts.tolist(), blocks, offsets))
 
     # More than one rank (not exercised on the single-GPU boxes this was developed on).
     flat_small = (torch.cat([t.view(-1) for t in uncompressed]) if uncompressed

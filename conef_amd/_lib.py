@@ -9,6 +9,7 @@ library is missing the import of any op fails loudly.
 import ctypes
 import os
 
+import numpy as np
 import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -101,6 +102,13 @@ class RandBlockItem(ctypes.Structure):
     _fields_ = [("x", _P), ("err", _P), ("cs_in", _P), ("cs_out", _P), ("payload", _P), ("plan_host", _P),
                 ("plan_dev", _P), ("staging", _P), ("n", _I64), ("m", _I64), ("start", _I64), ("block", _I64),
                 ("w", _I32), ("reserved", _I32)]
+
+
+def randblock_starts(items, count):
+    """The block starts of the first ``count`` items of a RandBlockItem array as a numpy view: a step
+    writes them all with one assignment."""
+    return np.ndarray((count,), dtype=np.int64, buffer=items, offset=RandBlockItem.start.offset,
+                      strides=(ctypes.sizeof(RandBlockItem),))
 
 
 _RETURNS_I64 = ("conef_topk_workspace_bytes", "conef_topk_batch_workspace_bytes", "conef_plan_bytes",

@@ -25,6 +25,7 @@ class SketchPlan:
         if nbytes <= 0:
             raise ValueError("no plan for shape n=%d d=%d w=%d" % (n, d, w))
         self.host = np.zeros(nbytes, dtype=np.uint8)
+        self.host_ptr = self.host.ctypes.data      # (numpy builds an object for every look at .ctypes)
         sa, sb = sign_seeds if sign_seeds is not None else (a + 2, b + 3)
         rc = lib.conef_plan_build_host_seeded(self.host.ctypes.data, nbytes, n, d, w, a, b, sa, sb, chunk_cols,
                                               bin_buckets)
@@ -53,10 +54,6 @@ class SketchPlan:
         stream = (_lib._raw_stream(dev.index if dev.index is not None else torch.cuda.current_device())
                   if _lib._raw_stream is not None else torch.cuda.current_stream(dev).cuda_stream)
         return _pools.staging(dev, stream, max(self.workspace_bytes, 16))
-
-    @property
-    def host_ptr(self):
-        return self.host.ctypes.data
 
     BINNED, ROWLIST, PANELS = 0, 1, 2
 

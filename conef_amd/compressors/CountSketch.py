@@ -63,6 +63,7 @@ class DenseCS:
         self.cs.copy_(torch.from_numpy(d["cs"]).to(self.cs.device))
         self.a = int(d.get("a", HASH_A))
         self.b = int(d.get("b", HASH_B))
+        self._plan = None          # a plan belongs to its hash seeds
 
     @classmethod
     def from_state_dict(cls, d, device=None):

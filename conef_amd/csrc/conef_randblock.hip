@@ -22,20 +22,18 @@ inline int grid_for(int64_t work_items, int threads, int64_t cap = 16384)
     return (int)g;
 }
 
-template <bool VEC>
 __global__ void __launch_bounds__(256)
 randblock_ef_kernel(float* __restrict__ x, float* __restrict__ err, float* __restrict__ payload, int64_t numel,
                     ConefBlock blk)
 {
-    conef_randblock_ef_body<VEC>(x, err, payload, numel, blk, (int)blockIdx.x, (int)gridDim.x);
+    conef_randblock_ef_body(x, err, payload, numel, blk, (int)blockIdx.x, (int)gridDim.x);
 }
 
-template <bool VEC>
 __global__ void __launch_bounds__(256)
 randblock_unbiased_kernel(float* __restrict__ x, float* __restrict__ payload, int64_t numel, ConefBlock blk,
                           float prob)
 {
-    conef_randblock_unbiased_body<VEC>(x, payload, numel, blk, prob, (int)blockIdx.x, (int)gridDim.x);
+    conef_randblock_unbiased_body(x, payload, numel, blk, prob, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // payload[p] = x[(start + p) mod numel] / scale   (scale = 1 for the biased compressor)
@@ -104,13 +102,8 @@ int conef_randblock_ef_step_f32(float* x, float* err, float* payload, int64_t nu
 {
     if (!block_args_ok(numel, start, block) || !x || !err || !payload) return CONEF_ERR_INVALID;
     ConefBlock blk = conef_make_block(numel, start, block);
-    int g = grid_for((numel + 3) / 4, 256);
-    if (aligned16(x) && aligned16(err))
-        hipLaunchKernelGGL(randblock_ef_kernel<true>, dim3(g), dim3(256), 0, (hipStream_t)stream, x, err, payload,
-                           numel, blk);
-    else
-        hipLaunchKernelGGL(randblock_ef_kernel<false>, dim3(g), dim3(256), 0, (hipStream_t)stream, x, err, payload,
-                           numel, blk);
+    hipLaunchKernelGGL(randblock_ef_kernel, dim3((unsigned)conef_rb_groups(numel)), dim3(256), 0, (hipStream_t)stream, x, err,
+                       payload, numel, blk);
     return (int)hipGetLastError();
 }
 
@@ -119,13 +112,8 @@ int conef_randblock_unbiased_step_f32(float* x, float* payload, int64_t numel, i
 {
     if (!block_args_ok(numel, start, block) || !x || !payload || !(prob > 0.f)) return CONEF_ERR_INVALID;
     ConefBlock blk = conef_make_block(numel, start, block);
-    int g = grid_for((numel + 3) / 4, 256);
-    if (aligned16(x))
-        hipLaunchKernelGGL(randblock_unbiased_kernel<true>, dim3(g), dim3(256), 0, (hipStream_t)stream, x, payload,
-                           numel, blk, prob);
-    else
-        hipLaunchKernelGGL(randblock_unbiased_kernel<false>, dim3(g), dim3(256), 0, (hipStream_t)stream, x, payload,
-                           numel, blk, prob);
+    hipLaunchKernelGGL(randblock_unbiased_kernel, dim3((unsigned)conef_rb_groups(numel)), dim3(256), 0, (hipStream_t)stream, x,
+                       payload, numel, blk, prob);
     return (int)hipGetLastError();
 }
 

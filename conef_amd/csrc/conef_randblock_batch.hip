@@ -16,22 +16,29 @@
 
 namespace {
 
-inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-
-constexpr int kRbBatchMax = 16;
-
+// Tensors a launch takes: as many as its arguments have room for (4 KB).  The arguments of a launch
+// are copied into memory the GPU reads whatever part of them is used, 3 us for 3 KB: buckets of up
+// to four tensors (a layer, an LSTM's) take a table of four.
 template <typename Item>
+constexpr int rb_batch_max() { return sizeof(Item) <= 64 ? 48 : 32; }
+constexpr int kRbFew = 4;
+
+template <typename Item, int CAP = rb_batch_max<Item>()>
 struct RbBatch {
-    Item item[kRbBatchMax];
-    int first[kRbBatchMax + 1];   // first workgroup of item i; first[count] = workgroups in all
+    Item item[CAP];
+    int first[CAP + 1];   // first workgroup of item i; first[count] = workgroups in all
     int count;
 };
 
-template <typename Item>
-__device__ __forceinline__ int rb_locate(const RbBatch<Item>& b, int* local, int* width)
+template <typename Item, int CAP>
+__device__ __forceinline__ int rb_locate(const RbBatch<Item, CAP>& b, int* local, int* width)
 {
-    int i = 0;
-    while (i + 1 < b.count && (int)blockIdx.x >= b.first[i + 1]) ++i;
+    int i = 0, last = b.count - 1;                // the last item that starts at or before this workgroup
+    while (i < last) {
+        const int mid = (i + last + 1) >> 1;
+        if (b.first[mid] <= (int)blockIdx.x) i = mid;
+        else last = mid - 1;
+    }
     *local = (int)blockIdx.x - b.first[i];
     *width = b.first[i + 1] - b.first[i];
     return i;
@@ -44,23 +51,22 @@ struct DenseItem {
     int64_t numel;
     ConefBlock blk;
     float prob;        // mode 0
-    int vec;
 };
 
-__global__ void __launch_bounds__(256) randblock_unbiased_batch_kernel(RbBatch<DenseItem> b)
+template <int CAP>
+__global__ void __launch_bounds__(256) randblock_unbiased_batch_kernel(RbBatch<DenseItem, CAP> b)
 {
     int local, width;
     const DenseItem& it = b.item[rb_locate(b, &local, &width)];
-    if (it.vec) conef_randblock_unbiased_body<true>(it.x, it.payload, it.numel, it.blk, it.prob, local, width);
-    else conef_randblock_unbiased_body<false>(it.x, it.payload, it.numel, it.blk, it.prob, local, width);
+    conef_randblock_unbiased_body(it.x, it.payload, it.numel, it.blk, it.prob, local, width);
 }
 
-__global__ void __launch_bounds__(256) randblock_ef_batch_kernel(RbBatch<DenseItem> b)
+template <int CAP>
+__global__ void __launch_bounds__(256) randblock_ef_batch_kernel(RbBatch<DenseItem, CAP> b)
 {
     int local, width;
     const DenseItem& it = b.item[rb_locate(b, &local, &width)];
-    if (it.vec) conef_randblock_ef_body<true>(it.x, it.err, it.payload, it.numel, it.blk, local, width);
-    else conef_randblock_ef_body<false>(it.x, it.err, it.payload, it.numel, it.blk, local, width);
+    conef_randblock_ef_body(it.x, it.err, it.payload, it.numel, it.blk, local, width);
 }
 
 struct ListItem {
@@ -73,8 +79,9 @@ struct ListItem {
     bool pk_lds;
 };
 
+template <int CAP>
 __global__ void __launch_bounds__(kConefRowlistThreads)
-randblock_rowlist_batch_kernel(RbBatch<ListItem> b, double one_minus_beta)
+randblock_rowlist_batch_kernel(RbBatch<ListItem, CAP> b, double one_minus_beta)
 {
     int local, width;
     const ListItem& it = b.item[rb_locate(b, &local, &width)];
@@ -82,14 +89,14 @@ randblock_rowlist_batch_kernel(RbBatch<ListItem> b, double one_minus_beta)
                                                   one_minus_beta, local, it.pk_lds);
 }
 
-template <typename Item, typename Go>
-int rb_run(const std::vector<Item>& table, const std::vector<int>& blocks, Go go)
+template <typename Item, int CAP, typename Go>
+int rb_run_cap(const std::vector<Item>& table, const std::vector<int>& blocks, Go go)
 {
     size_t k = 0;
     while (k < table.size()) {
-        RbBatch<Item> b;
+        RbBatch<Item, CAP> b;
         int nb = 0, total = 0;
-        while (k < table.size() && nb < kRbBatchMax) {
+        while (k < table.size() && nb < CAP) {
             b.item[nb] = table[k];
             b.first[nb] = total;
             total += blocks[k];
@@ -101,6 +108,14 @@ int rb_run(const std::vector<Item>& table, const std::vector<int>& blocks, Go go
         if (total > 0) go(b, total);
     }
     return (int)hipGetLastError();
+}
+
+// go(batch, workgroups) for the table in runs; `go` is generic over the batch's capacity
+template <typename Item, typename Go>
+int rb_run(const std::vector<Item>& table, const std::vector<int>& blocks, Go go)
+{
+    if (table.size() <= (size_t)kRbFew) return rb_run_cap<Item, kRbFew>(table, blocks, go);
+    return rb_run_cap<Item, rb_batch_max<Item>()>(table, blocks, go);
 }
 
 }  // namespace
@@ -143,16 +158,15 @@ int conef_randblock_step_batch_f32(const ConefRandBlockItem* items, int32_t coun
             d.blk = conef_make_block(numel, it.start, it.block);
             // the reference divides by the Python double block / numel, which reaches the tensor as fp32
             d.prob = (float)((double)it.block / (double)numel);
-            d.vec = aligned16(it.x) && (mode == 0 || aligned16(it.err));
             table.push_back(d);
-            blocks.push_back(conef_grid_for((numel + 3) / 4, 256));
+            blocks.push_back(conef_rb_groups(numel));
         }
         if (mode == 0)
-            return rb_run(table, blocks, [&](const RbBatch<DenseItem>& bt, int grid) {
-                hipLaunchKernelGGL(randblock_unbiased_batch_kernel, dim3((unsigned)grid), dim3(256), 0, s, bt);
+            return rb_run(table, blocks, [&](const auto& bt, int grid) {
+                hipLaunchKernelGGL((randblock_unbiased_batch_kernel<sizeof(bt.item) / sizeof(bt.item[0])>), dim3((unsigned)grid), dim3(256), 0, s, bt);
             });
-        return rb_run(table, blocks, [&](const RbBatch<DenseItem>& bt, int grid) {
-            hipLaunchKernelGGL(randblock_ef_batch_kernel, dim3((unsigned)grid), dim3(256), 0, s, bt);
+        return rb_run(table, blocks, [&](const auto& bt, int grid) {
+            hipLaunchKernelGGL((randblock_ef_batch_kernel<sizeof(bt.item) / sizeof(bt.item[0])>), dim3((unsigned)grid), dim3(256), 0, s, bt);
         });
     }
     // sketched error: row-list plans share launches, the rest go one by one
@@ -172,11 +186,13 @@ int conef_randblock_step_batch_f32(const ConefRandBlockItem* items, int32_t coun
         if (shape.lds > lds) lds = shape.lds;
     }
     if (!table.empty()) {
-        hipError_t e = conef_allow_lds((const void*)randblock_rowlist_batch_kernel, lds);
+        const void* kern = table.size() <= (size_t)kRbFew ? (const void*)randblock_rowlist_batch_kernel<kRbFew>
+                                                          : (const void*)randblock_rowlist_batch_kernel<rb_batch_max<ListItem>()>;
+        hipError_t e = conef_allow_lds(kern, lds);
         if (e != hipSuccess) return (int)e;
         const double omb = 1. - (double)beta;
-        int rc = rb_run(table, blocks, [&](const RbBatch<ListItem>& bt, int grid) {
-            hipLaunchKernelGGL(randblock_rowlist_batch_kernel, dim3((unsigned)grid), dim3(kConefRowlistThreads), lds, s,
+        int rc = rb_run(table, blocks, [&](const auto& bt, int grid) {
+            hipLaunchKernelGGL((randblock_rowlist_batch_kernel<sizeof(bt.item) / sizeof(bt.item[0])>), dim3((unsigned)grid), dim3(kConefRowlistThreads), lds, s,
                                bt, omb);
         });
         if (rc != CONEF_OK) return rc;

@@ -4,101 +4,152 @@
 #pragma once
 #include "conef_device.h"
 
+// The tensor goes by tiles of kRbTile consecutive elements, kRbQuads column quads a thread, all of
+// them requested before the first is used.  A tile that holds none of the block - at the ratios that
+// compress, nine in ten - takes no test per element; in the others the block is two ranges of the tile,
+// and a quad inside one of them moves as a quad.  Pure streaming (dense error: 16 bytes an element,
+// unbiased: 4), bounded by memory.
+constexpr int kRbQuads = 4;
+constexpr int kRbTile = 256 * 4 * kRbQuads;
+
+// The block's ranges [lo, hi) and [0, rest) relative to the tile at f0, and where in the payload the
+// tile's element 0 would sit as part of the one and of the other.
+struct RbTile {
+    int lo, hi, rest;
+    int64_t at, at_rest;
+    __device__ __forceinline__ RbTile(const ConefBlock& b, int64_t f0)
+    {
+        const int64_t l = b.start - f0, h = b.end - f0, r = b.rest - f0;
+        lo = l < 0 ? 0 : l > kRbTile ? kRbTile : (int)l;
+        hi = h < 0 ? 0 : h > kRbTile ? kRbTile : (int)h;
+        rest = r < 0 ? 0 : r > kRbTile ? kRbTile : (int)r;
+        at = f0 - b.start;
+        at_rest = b.end - b.start + f0;
+    }
+    __device__ __forceinline__ bool touched() const { return hi > lo || rest > 0; }
+    __device__ __forceinline__ bool inside(int e) const { return (e >= lo && e < hi) || e < rest; }
+    __device__ __forceinline__ int64_t pos(int e) const { return (e < rest ? at_rest : at) + e; }
+    // all four elements from e on in one of the ranges
+    __device__ __forceinline__ bool whole(int e) const { return (e >= lo && e + 4 <= hi) || e + 4 <= rest; }
+    __device__ __forceinline__ bool outside(int e) const { return (e + 4 <= lo || e >= hi) && e >= rest; }
+};
+
 // x = g + e;  selected: payload = x, out = x, e' = 0;  not selected: out = 0, e' = x.
 // (RandomBlock_hook.py:182-184,222,228,237,240,276-280)
-template <bool VEC>
 __device__ __forceinline__ void
 conef_randblock_ef_body(float* __restrict__ x, float* __restrict__ err, float* __restrict__ payload, int64_t numel,
                         ConefBlock blk, int bx, int gx)
 {
-    int64_t quads = (numel + 3) / 4;
-    int64_t stride = (int64_t)gx * blockDim.x;
-    for (int64_t q = bx * (int64_t)blockDim.x + threadIdx.x; q < quads; q += stride) {
-        int64_t f = q * 4;
-        int valid = numel - f < 4 ? (int)(numel - f) : 4;
-        float g[4], e[4], o[4], ne[4];
-        if (VEC && valid == 4) {
-            float4 tg = *reinterpret_cast<const float4*>(x + f);
-            float4 te = *reinterpret_cast<const float4*>(err + f);
-            g[0] = tg.x; g[1] = tg.y; g[2] = tg.z; g[3] = tg.w;
-            e[0] = te.x; e[1] = te.y; e[2] = te.z; e[3] = te.w;
-        } else {
+    const int64_t tiles = (numel + kRbTile - 1) / kRbTile;
+    const float zero[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int64_t t = bx; t < tiles; t += gx) {
+        const int64_t f0 = t * kRbTile;
+        float* xt = x + f0;
+        float* et = err + f0;
+        const RbTile in(blk, f0);
+        if (f0 + kRbTile <= numel) {
+            float g[kRbQuads][4], e[kRbQuads][4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                g[k] = k < valid ? x[f + k] : 0.f;
-                e[k] = k < valid ? err[f + k] : 0.f;
+            for (int u = 0; u < kRbQuads; ++u) {
+                const int i = 4 * (threadIdx.x + 256 * u);
+                conef_ld4u(xt + i, g[u]);
+                conef_ld4u(et + i, e[u]);
             }
-        }
+            const bool touched = in.touched();
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            float xq = __fadd_rn(g[k], e[k]);
-            int64_t pos = k < valid ? conef_payload_pos(f + k, blk) : -1;
-            if (pos >= 0) {
-                payload[pos] = xq;
-                o[k] = xq;
-                ne[k] = 0.f;
-            } else {
-                o[k] = 0.f;
-                ne[k] = xq;
-            }
-        }
-        if (VEC && valid == 4) {
-            *reinterpret_cast<float4*>(x + f) = make_float4(o[0], o[1], o[2], o[3]);
-            *reinterpret_cast<float4*>(err + f) = make_float4(ne[0], ne[1], ne[2], ne[3]);
-        } else {
+            for (int u = 0; u < kRbQuads; ++u) {
+                const int i = 4 * (threadIdx.x + 256 * u);
+                float xq[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (k < valid) {
-                    x[f + k] = o[k];
-                    err[f + k] = ne[k];
+                for (int k = 0; k < 4; ++k) xq[k] = __fadd_rn(g[u][k], e[u][k]);
+                if (!touched || in.outside(i)) {
+                    conef_st4u(xt + i, zero);
+                    conef_st4u(et + i, xq);
+                } else if (in.whole(i)) {
+                    conef_st4u(xt + i, xq);
+                    conef_st4u(et + i, zero);
+                    conef_st4u(payload + in.pos(i), xq);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const bool sel = in.inside(i + k);
+                        if (sel) payload[in.pos(i + k)] = xq[k];
+                        xt[i + k] = sel ? xq[k] : 0.f;
+                        et[i + k] = sel ? 0.f : xq[k];
+                    }
                 }
+            }
+        } else {
+            const int left = (int)(numel - f0);
+            for (int i = threadIdx.x; i < left; i += 256) {
+                const float xq = __fadd_rn(xt[i], et[i]);
+                const bool sel = in.inside(i);
+                if (sel) payload[in.pos(i)] = xq;
+                xt[i] = sel ? xq : 0.f;
+                et[i] = sel ? 0.f : xq;
+            }
         }
     }
 }
 
-// selected: payload = x / prob, out = payload;  not selected: out = 0
+// selected: payload = x / prob, out = payload;  not selected: out = 0 (written, never read)
 // (UnbiasedRandomBlock_hook.py:155,161-167,200-204)
-template <bool VEC>
 __device__ __forceinline__ void
 conef_randblock_unbiased_body(float* __restrict__ x, float* __restrict__ payload, int64_t numel, ConefBlock blk,
                               float prob, int bx, int gx)
 {
-    int64_t quads = (numel + 3) / 4;
-    int64_t stride = (int64_t)gx * blockDim.x;
-    for (int64_t q = bx * (int64_t)blockDim.x + threadIdx.x; q < quads; q += stride) {
-        int64_t f = q * 4;
-        int valid = numel - f < 4 ? (int)(numel - f) : 4;
-        // a quad with no selected element is only written, never read
-        bool any = false;
+    const int64_t tiles = (numel + kRbTile - 1) / kRbTile;
+    const float zero[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int64_t t = bx; t < tiles; t += gx) {
+        const int64_t f0 = t * kRbTile;
+        float* xt = x + f0;
+        const RbTile in(blk, f0);
+        if (f0 + kRbTile <= numel) {
+            if (!in.touched()) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) any |= (k < valid) && conef_payload_pos(f + k, blk) >= 0;
-        float o[4] = {0.f, 0.f, 0.f, 0.f};
-        if (any) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                int64_t pos = k < valid ? conef_payload_pos(f + k, blk) : -1;
-                if (pos >= 0) {
-                    float s = __fdiv_rn(x[f + k], prob);
-                    payload[pos] = s;
-                    o[k] = s;
-                }
+                for (int u = 0; u < kRbQuads; ++u) conef_st4u(xt + 4 * (threadIdx.x + 256 * u), zero);
+                continue;
             }
-        }
-        if (VEC && valid == 4) {
-            *reinterpret_cast<float4*>(x + f) = make_float4(o[0], o[1], o[2], o[3]);
-        } else {
+            float g[kRbQuads][4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (k < valid) x[f + k] = o[k];
+            for (int u = 0; u < kRbQuads; ++u) conef_ld4u(xt + 4 * (threadIdx.x + 256 * u), g[u]);
+#pragma unroll
+            for (int u = 0; u < kRbQuads; ++u) {
+                const int i = 4 * (threadIdx.x + 256 * u);
+                if (in.whole(i)) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) g[u][k] = __fdiv_rn(g[u][k], prob);
+                    conef_st4u(payload + in.pos(i), g[u]);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        if (in.inside(i + k)) {
+                            g[u][k] = __fdiv_rn(g[u][k], prob);
+                            payload[in.pos(i + k)] = g[u][k];
+                        } else {
+                            g[u][k] = 0.f;
+                        }
+                    }
+                }
+                conef_st4u(xt + i, g[u]);
+            }
+        } else {
+            const int left = (int)(numel - f0);
+            for (int i = threadIdx.x; i < left; i += 256) {
+                float o = 0.f;
+                if (in.inside(i)) {
+                    o = __fdiv_rn(xt[i], prob);
+                    payload[in.pos(i)] = o;
+                }
+                xt[i] = o;
+            }
         }
     }
 }
 
-// workgroups of 256 threads for `work_items` items, capped
-inline int conef_grid_for(int64_t work_items, int threads, int64_t cap = 16384)
+// workgroups of a tensor of `numel` elements
+inline int conef_rb_groups(int64_t numel)
 {
-    int64_t g = (work_items + threads - 1) / threads;
-    if (g < 1) g = 1;
-    if (g > cap) g = cap;
-    return (int)g;
+    const int64_t g = (numel + kRbTile - 1) / kRbTile;
+    return (int)(g < 1 ? 1 : g > 16384 ? 16384 : g);
 }
