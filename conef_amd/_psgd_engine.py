@@ -131,10 +131,7 @@ class _RoundPlan:
                  "topk_event", "ws_need", "handoff_event", "topk_number", "q_next_number", "is_wide", "wide", "chunks", "ef_spans")
 
 
-def _layout_signature(grads):
-    """What a step compares instead of every tensor's shape: a bucket keeps its buffer, its length
-    (both part of the plan's key) and its parameters for as long as DDP keeps the bucket."""
-    return (len(grads), grads[0].shape, grads[-1].shape) if grads else (0, None, None)
+_layout_signature = _bucket.layout_signature
 
 
 BATCH_ITEMS = 24        # matrices the batch entry points take into one launch
@@ -518,21 +515,24 @@ def _run_round(state, bucket, error_mode, streams=1):
         # comparisons).  Where the buckets do not run side by side (one stream), those launches go to a side
         # stream, which the bucket's next round waits for, and overlap the next bucket.
         if plan.q_next is None:
-            plan.q_next = torch.empty(sum(m * _rank_bound(rank) for _, _, m, rank in work), device=device, dtype=dtype)
-            at, ptrs = plan.q_next.data_ptr(), []
-            for _, n, m, rank in work:
-                ptrs.append(at)
-                at += 4 * m * _rank_bound(rank)
-            plan.q_next_ptrs = (ctypes.c_void_p * count)(*ptrs)
+            # row-major factors first, then the same in the order the kernels of ranks up to 8 load them
+            by_rows = [m * _rank_bound(rank) for _, _, m, rank in work]
+            by_quads = [-(-m // 4) * 4 * _rank_bound(rank) for _, _, m, rank in work]
+            plan.q_next = torch.empty(sum(by_rows) + sum(by_quads), device=device, dtype=dtype)
+            at = [plan.q_next.data_ptr()]
+            for numel in by_rows + by_quads:
+                at.append(at[-1] + 4 * numel)
+            plan.q_next_ptrs = [(ctypes.c_void_p * (2 * part))(*at[first: first + part], *at[count + first: count + first + part])
+                                for first, part in plan.chunks]
             plan.made = [ctypes.c_int32(0) for _ in plan.chunks]
             plan.q_next_ready = False
         aside = state.matrix_approximation_rank > 8 and streams <= 1
         if aside and plan.q_next_ready:
             _pools.side_wait(device, _lib.current_stream(device), plan.q_next_number)
-        flags = (1 if plan.q_next_ready else 0) | (0 if aside else 2)
-        for (first, part), made in zip(plan.chunks, plan.made):
+        flags = (1 if plan.q_next_ready else 0) | (0 if aside else 2) | 4
+        for (first, part), q_next, made in zip(plan.chunks, plan.q_next_ptrs, plan.made):
             rc = lib.conef_psgd_round_ahead_f32(_at(items, first), part, mode1, mode3, float(alpha), beta3, eps, HASH_A, HASH_B,
-                                                _at(plan.q_next_ptrs, first), flags, ctypes.byref(made), ws_ptr, ws_len, stream)
+                                                q_next, flags, ctypes.byref(made), ws_ptr, ws_len, stream)
             _lib.check(rc, "conef_psgd_round_ahead_f32")
         plan.q_next_ready = all(made.value for made in plan.made)
         if aside:
@@ -604,8 +604,8 @@ def _orthogonalise_q_aside(plan, lib, items, eps, ws_len, device):
         plan.q_next.record_stream(side)       # memory the side stream works on must not go back to the allocator under it
     with _lib.on_stream(side):
         ws = _workspace(device, side.cuda_stream, max(ws_len, 256))
-    for (first, part), made in zip(plan.chunks, plan.made):
-        rc = lib.conef_psgd_q_next_f32(_at(items, first), part, eps, _at(plan.q_next_ptrs, first), ctypes.byref(made),
+    for (first, part), q_next, made in zip(plan.chunks, plan.q_next_ptrs, plan.made):
+        rc = lib.conef_psgd_q_next_f32(_at(items, first), part, eps, q_next, ctypes.byref(made),
                                        ws.data_ptr(), ws.numel(), side.cuda_stream)
         _lib.check(rc, "conef_psgd_q_next_f32")
     plan.q_next_event.record(side)

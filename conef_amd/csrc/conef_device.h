@@ -61,6 +61,55 @@ __device__ __forceinline__ void conef_st4u(float* p, const float* v)
 // quad's.  Whoever owns it ignores them (they are never stored and never counted).
 __device__ __forceinline__ int conef_quad_col(int quad, int m) { return 4 * quad + 4 <= m ? 4 * quad : m - 4; }
 
+// The quads' slices of a factor Q [m, RP] laid out for them: 16-byte piece v (of RP) of every quad's
+// 4 x RP floats, one quad after the other, then piece v + 1.  Neighbouring lanes own neighbouring quads,
+// so a load of piece v is one run of memory; from the row-major factor the same load takes 16 bytes out
+// of a different cache line (RP = 8: every 128 bytes) for every lane, and RP such loads a quad are
+// what the products at rank 8 were waiting for.  The moved quad of a row's end has its own slice.
+__host__ __device__ __forceinline__ int64_t conef_quads(int64_t m) { return (m + 3) >> 2; }
+
+struct ConefQuadSlices {
+    const float* base;      // of this thread's quad
+    int step;               // floats from one 16-byte piece to the next
+};
+
+// qi: the layout above, or null: the row-major q
+template <int RP>
+__device__ __forceinline__ ConefQuadSlices conef_quad_slices(const float* q, const float* qi, int quad, int col, int m)
+{
+    if (qi) return {qi + 4 * (int64_t)quad, 4 * (int)conef_quads(m)};
+    return {q + (int64_t)col * RP, 4};
+}
+
+template <int RP>
+__device__ __forceinline__ void conef_load_slices(const ConefQuadSlices& s, float* out)
+{
+#pragma unroll
+    for (int v = 0; v < RP; ++v) conef_ld4u(s.base + (int64_t)v * s.step, out + 4 * v);
+}
+
+// Row i of Q (RP floats) into that layout.  own_only: the moved quad's first columns, which the quad
+// before it owns, are left zero in it, so that a product that reads them counts them once.
+template <int RP>
+__device__ __forceinline__ void conef_store_slice_row(float* qi, int64_t i, int64_t m, const float* x, bool own_only)
+{
+    const int64_t m4 = conef_quads(m);
+    auto put = [&](int64_t quad, int k, bool zero) {
+        constexpr int R = RP < 4 ? RP : 4;                 // floats of a row that sit in one piece
+#pragma unroll
+        for (int c = 0; c < RP; c += R) {
+            const int t = k * RP + c;
+            float* dst = qi + ((int64_t)(t >> 2) * m4 + quad) * 4 + (t & 3);
+#pragma unroll
+            for (int e = 0; e < R; ++e) dst[e] = zero ? 0.f : x[c + e];
+        }
+    };
+    const int64_t last = m4 - 1;
+    const bool moved = (m & 3) != 0;
+    if (!moved || i < 4 * last) put(i >> 2, (int)(i & 3), false);
+    if (moved && i >= m - 4) put(last, (int)(i - (m - 4)), own_only && i < 4 * last);
+}
+
 // Stores the columns of a quad that are its own.
 __device__ __forceinline__ void conef_st4_own(float* p, const float* v, int dup)
 {

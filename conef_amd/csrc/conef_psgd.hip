@@ -62,11 +62,23 @@ struct PsgdBatch {
     int count;
 };
 
+// item that workgroup bx of the table works for: the last one that starts at or before it
+template <typename Item>
+__device__ __forceinline__ int psgd_batch_item(const PsgdBatch<Item>& b, int bx)
+{
+    int i = 0, last = b.count - 1;
+    while (i < last) {
+        const int mid = (i + last + 1) >> 1;
+        if (b.first[mid] <= bx) i = mid;
+        else last = mid - 1;
+    }
+    return i;
+}
+
 template <typename Item>
 __device__ __forceinline__ int psgd_batch_locate(const PsgdBatch<Item>& b, int* local)
 {
-    int i = 0;
-    while (i + 1 < b.count && (int)blockIdx.x >= b.first[i + 1]) ++i;
+    const int i = psgd_batch_item(b, (int)blockIdx.x);
     *local = (int)blockIdx.x - b.first[i];
     return i;
 }
@@ -600,7 +612,7 @@ __device__ __forceinline__ void store_row(float* p, const float* x)
 template <int RP, int T>
 __device__ __forceinline__ void
 gram_orthogonalise_body(const float* __restrict__ src, float* __restrict__ dst, int rows, const double* parts, int nparts,
-                        int r, float eps)
+                        int r, float eps, float* __restrict__ quads)
 {
     __shared__ float t_l[RP * RP + RP];
     gram_solve_lds<RP, T>(parts, nparts, eps, t_l);
@@ -620,7 +632,10 @@ gram_orthogonalise_body(const float* __restrict__ src, float* __restrict__ dst, 
                 for (int c = 0; c < RP; ++c)
                     if (c >= r) x[u][c] = 0.f;
             }
-            if (row < rows) store_row<RP>(dst + (int64_t)row * RP, x[u]);
+            if (row < rows) {
+                store_row<RP>(dst + (int64_t)row * RP, x[u]);
+                if (quads) conef_store_slice_row<RP>(quads, row, rows, x[u], true);
+            }
         }
     }
 }
@@ -634,8 +649,7 @@ psgd_mtp_gram_batch_kernel(PsgdBatch<MtpItem> b, GramTask g)
         return;
     }
     const int bx = (int)blockIdx.x - g.count;
-    int i = 0;
-    while (i + 1 < b.count && bx >= b.first[i + 1]) ++i;
+    const int i = psgd_batch_item(b, bx);
     const MtpItem& it = b.item[i];
     const int local = bx - b.first[i];
     psgd_mtp_body<RP, FAST>(it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, local % it.col_tiles,
@@ -658,6 +672,7 @@ struct DeferFixItem {
     float* pt;
     float* qt;
     int r;
+    float* qi;               // not null: Q by quads for the launch that follows (conef_store_slice_row)
 };
 
 // A finished row (P or Q, zeros from column r on) into the caller's [rows, r] factor.
@@ -715,6 +730,7 @@ psgd_defer_fix_batch_kernel(PsgdBatch<DeferFixItem> b)
         if (row < rows) store_tight_row<RP>(is_p ? it.pt : it.qt, row, x, it.r);
     }
     if (row < rows) store_row<RP>((is_p ? it.p : it.q) + row * RP, x);
+    if (!is_p && it.qi && row < rows) conef_store_slice_row<RP>(it.qi, row, it.m, x, false);
     if (!is_p && it.qgram) {                                // uniform over the workgroup
 #pragma unroll
         for (int c = 0; c < RP; ++c) rows_l[threadIdx.x][c] = row < rows ? x[c] : 0.f;
@@ -894,8 +910,7 @@ psgd_mfma_mtp_gram_batch_kernel(PsgdBatch<MfmaMtpItem> b, GramTask g)
         return;
     }
     const int bx = (int)blockIdx.x - g.count;
-    int i = 0;
-    while (i + 1 < b.count && bx >= b.first[i + 1]) ++i;
+    const int i = psgd_batch_item(b, bx);
     const MfmaMtpItem& it = b.item[i];
     const int local = bx - b.first[i];
     const int ct = local % it.col_tiles, slab = local / it.col_tiles;
@@ -1009,6 +1024,7 @@ struct PqtItem {
     int64_t n;
     int m, r, rows_per_slab, col_tiles;
     int lanes;
+    const float* qi;         // not null: q laid out by quads (conef_load_slices)
 };
 
 inline int pqt_lanes(int64_t m)
@@ -1029,8 +1045,7 @@ __device__ __forceinline__ void psgd_pqt_rows(const PqtItem& it, int bx, int by)
     const int64_t i0 = (int64_t)by * it.rows_per_slab;
     const int64_t i1 = i0 + it.rows_per_slab < it.n ? i0 + it.rows_per_slab : it.n;
     float qf[4 * RP];
-#pragma unroll
-    for (int t = 0; t < RP; ++t) conef_ld4u(it.q + (int64_t)col * RP + 4 * t, qf + 4 * t);
+    conef_load_slices<RP>(conef_quad_slices<RP>(it.q, it.qi, quad, col, m), qf);
     for (int64_t ib = i0 + grp; ib < i1; ib += 4 * groups) {
         float xv[4][4];
         if (MODE == 1) {
@@ -1131,6 +1146,7 @@ struct ListPsgdResidual {
     const float* p;
     const float* q;
     int r;
+    const float* qi;         // not null: q laid out by quads (conef_load_slices), FAST
     static constexpr bool kNeedsCells = false;
     struct Regs {};
     __device__ __forceinline__ void stage(int64_t row0, int rows, int d, int, float* vals, const float*,
@@ -1161,8 +1177,7 @@ struct ListPsgdResidual {
                 conef_ld4u(base + (int64_t)r1 * d + col, x1n);
             };
             if (have) {
-#pragma unroll
-                for (int v = 0; v < RP; ++v) conef_ld4u(q + (int64_t)conef_quad_col(c4, d) * RP + 4 * v, flat + 4 * v);
+                conef_load_slices<RP>(conef_quad_slices<RP>(q, qi, c4, conef_quad_col(c4, d), d), flat);
                 request_rows(c4, rw);
             }
             __syncthreads();
@@ -1184,10 +1199,7 @@ struct ListPsgdResidual {
                 }
                 have = c4 < d4;
                 if (have) {
-                    if (new_quad) {
-#pragma unroll
-                        for (int v = 0; v < RP; ++v) conef_ld4u(q + (int64_t)conef_quad_col(c4, d) * RP + 4 * v, flatn + 4 * v);
-                    }
+                    if (new_quad) conef_load_slices<RP>(conef_quad_slices<RP>(q, qi, c4, conef_quad_col(c4, d), d), flatn);
                     request_rows(c4, rw);
                 }
                 const float* pa = ptile + cur_rw * RP;
@@ -1510,13 +1522,14 @@ struct GsAhead {
     // orthogonalised from its Gram matrix, whatever its height (gram_orthogonalise_body)
     const double* parts[kPsgdBatchMax];
     int nparts[kPsgdBatchMax];
+    float* quads[kPsgdBatchMax];      // with parts, not null: dst by quads as well (conef_store_slice_row)
 };
 
 template <int RP>
 __device__ __forceinline__ void gs_ahead_body(const GsAhead& g, int k)
 {
     if (g.parts[k]) {
-        gram_orthogonalise_body<RP, kGsRegThreads>(g.src[k], g.dst[k], g.rows[k], g.parts[k], g.nparts[k], g.r, g.eps);
+        gram_orthogonalise_body<RP, kGsRegThreads>(g.src[k], g.dst[k], g.rows[k], g.parts[k], g.nparts[k], g.r, g.eps, g.quads[k]);
         return;
     }
     // at most kGsAheadRowSlots rows a thread: the taller bodies hold over a hundred values in
@@ -2169,7 +2182,7 @@ inline bool gsg_workspace_ok(const void* workspace, int64_t workspace_bytes)
 }
 
 int pqt_batch(const ConefPsgdItem* items, int count, int mode, float beta, int32_t a, int32_t b, hipStream_t s,
-              const GsAhead* ahead = nullptr, bool* ahead_used = nullptr);
+              const GsAhead* ahead = nullptr, bool* ahead_used = nullptr, const std::vector<float*>* qi = nullptr);
 
 inline bool psgd_args_ok(int64_t n, int64_t m, int32_t r)
 {
@@ -2382,10 +2395,10 @@ int conef_psgd_pqt_conef_planned_f32(float* x, const float* p, const float* q, c
 #define CONEF_RES(RP)                                                                          \
     do {                                                                                       \
         if (fast) {                                                                            \
-            ListPsgdResidual<RP, true> front = {x, p, q, r};                                   \
+            ListPsgdResidual<RP, true> front = {x, p, q, r, nullptr};                                   \
             rc = conef_launch_rowlist(front, view, cs_in, cs_out, n, m, w, beta, s);           \
         } else {                                                                               \
-            ListPsgdResidual<RP, false> front = {x, p, q, r};                                  \
+            ListPsgdResidual<RP, false> front = {x, p, q, r, nullptr};                                  \
             rc = conef_launch_rowlist(front, view, cs_in, cs_out, n, m, w, beta, s);           \
         }                                                                                      \
     } while (0)
@@ -3088,6 +3101,7 @@ inline int64_t defer_region_offset(const ConefPsgdItem* items, int count)
 struct PaddedRound {
     std::vector<ConefPsgdItem> items;
     std::vector<float*> pt, qt;      // the caller's factors where items holds copies, else null
+    std::vector<float*> qi;          // ranks up to 8: the new Q by quads (conef_store_slice_row)
     int rp;
     bool padded;
 };
@@ -3095,7 +3109,8 @@ struct PaddedRound {
 inline int64_t padded_factor_bytes(const ConefPsgdItem& it)
 {
     const int rp = rank_bound(it.r);
-    return rp == it.r ? 0 : conef_align256(4 * it.n * rp) + conef_align256(4 * it.m * rp);
+    return (rp == it.r ? 0 : conef_align256(4 * it.n * rp) + conef_align256(4 * it.m * rp)) +
+           (rp <= 8 ? conef_align256(16 * conef_quads(it.m) * rp) : 0);
 }
 
 inline std::vector<ConefPsgdItem> at_rank_bound(const ConefPsgdItem* items, int count)
@@ -3136,6 +3151,10 @@ inline bool padded_round(const ConefPsgdItem* items, int count, int mq_mode, voi
             at += conef_align256(4 * it.n * pr->rp);
             it.q = (float*)at;
             at += conef_align256(4 * it.m * pr->rp);
+        }
+        if (pr->rp <= 8) {
+            pr->qi.push_back((float*)at);
+            at += conef_align256(16 * conef_quads(it.m) * pr->rp);
         }
     }
     if (pr->rp > 8) {
@@ -3196,7 +3215,8 @@ int defer_fix(const PaddedRound& pr, int r, const std::vector<MtpRaw>& raw, cons
         const ConefPsgdItem& it = pr.items[(size_t)k];
         const int pb = (int)((it.n + rows_per_wg - 1) / rows_per_wg), qb = (int)((it.m + rows_per_wg - 1) / rows_per_wg);
         fix.push_back(DeferFixItem{it.p, raw[(size_t)k].src, it.q, tmats[(size_t)k], qgrams ? (*qgrams)[(size_t)k] : nullptr,
-                                   it.n, it.m, raw[(size_t)k].slabs, pb, pr.pt[(size_t)k], pr.qt[(size_t)k], r});
+                                   it.n, it.m, raw[(size_t)k].slabs, pb, pr.pt[(size_t)k], pr.qt[(size_t)k], r,
+                                   rp <= 8 ? pr.qi[(size_t)k] : nullptr});
         blocks.push_back(pb + qb);
     }
     return run_batches(fix, blocks, [&](const PsgdBatch<DeferFixItem>& bt, int grid) {
@@ -3213,11 +3233,11 @@ int defer_fix(const PaddedRound& pr, int r, const std::vector<MtpRaw>& raw, cons
 }
 
 // P = X Q (raw) with the Gram shares, Q = X^T P (raw) with the systems solved on the side, then T
-// applied to both.  q_in: the Q the first product reads, rows of pr.rp floats.
+// applied to both.  q_in: the Q the first product reads, rows of pr.rp floats; qi_in: by quads, or null.
 // q_shares (optional): the fix launch also leaves the shares of Q^T Q of the new Q factors; their
 // places are recorded in q_shares->parts / nparts.
 template <int MODE>
-int round_products_deferred(const PaddedRound& pr, int r, float* const* q_in, float alpha, float eps, int32_t a, int32_t b,
+int round_products_deferred(const PaddedRound& pr, int r, float* const* q_in, float* const* qi_in, float alpha, float eps, int32_t a, int32_t b,
                             void* workspace, int64_t workspace_bytes, hipStream_t s, GsAhead* q_shares)
 {
     const ConefPsgdItem* items = pr.items.data();
@@ -3230,7 +3250,7 @@ int round_products_deferred(const PaddedRound& pr, int r, float* const* q_in, fl
     for (int k = 0; k < count; ++k) {
         const ConefPsgdItem& it = items[k];
         MqsItem t = {it.x, it.err, it.cs, MODE == 2 ? item_pktab(it) : nullptr, q_in[k], it.p, it.n, (int)it.m,
-                     (int)(MODE == 2 ? it.w : 1), 0, 0, conef_make_mod(MODE == 2 ? it.w : 1), (double*)at};
+                     (int)(MODE == 2 ? it.w : 1), 0, 0, conef_make_mod(MODE == 2 ? it.w : 1), (double*)at, qi_in ? qi_in[k] : nullptr};
         table.push_back(t);
         at += conef_align256(8 * defer_gram_doubles(it));
         tmats.push_back((float*)at);
@@ -3307,16 +3327,16 @@ int round_products_deferred_mfma(const PaddedRound& pr, int r, float* const* q_i
 }
 
 // Either of the two by rank.
-int deferred_products(const PaddedRound& pr, int r, float* const* q_in, int mq_mode, float alpha, float eps, int32_t a, int32_t b,
+int deferred_products(const PaddedRound& pr, int r, float* const* q_in, float* const* qi_in, int mq_mode, float alpha, float eps, int32_t a, int32_t b,
                       void* workspace, int64_t workspace_bytes, hipStream_t s, GsAhead* q_shares)
 {
     if (pr.rp > 8)
         return round_products_deferred_mfma(pr, r, q_in, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, s);
     if (mq_mode == 0)
-        return round_products_deferred<0>(pr, r, q_in, 0.f, eps, a, b, workspace, workspace_bytes, s, q_shares);
+        return round_products_deferred<0>(pr, r, q_in, qi_in, 0.f, eps, a, b, workspace, workspace_bytes, s, q_shares);
     if (mq_mode == 1)
-        return round_products_deferred<1>(pr, r, q_in, 0.f, eps, a, b, workspace, workspace_bytes, s, q_shares);
-    return round_products_deferred<2>(pr, r, q_in, alpha, eps, a, b, workspace, workspace_bytes, s, q_shares);
+        return round_products_deferred<1>(pr, r, q_in, qi_in, 0.f, eps, a, b, workspace, workspace_bytes, s, q_shares);
+    return round_products_deferred<2>(pr, r, q_in, qi_in, alpha, eps, a, b, workspace, workspace_bytes, s, q_shares);
 }
 
 // dst[k] <- the rows of src[k] ([m, RP], zeros behind column r) orthogonalised, at ranks 9 to 32: the
@@ -3350,7 +3370,7 @@ int orthogonalise_by_gram_wide(const PaddedRound& pr, int r, const std::vector<c
         gram.parts[k] = parts;
         gram.nparts[k] = nb;
         gram.tmat[k] = tmat;
-        fix.push_back(DeferFixItem{nullptr, src[(size_t)k], dst[k], tmat, nullptr, 0, it.m, 1, 0, nullptr, nullptr, r});
+        fix.push_back(DeferFixItem{nullptr, src[(size_t)k], dst[k], tmat, nullptr, 0, it.m, 1, 0, nullptr, nullptr, r, nullptr});
         fix_blocks.push_back((int)((it.m + rows_per_wg - 1) / rows_per_wg));
     }
     int rc = run_batches(shares, share_blocks, [&](const PsgdBatch<GramShareItem>& bt, int grid) {
@@ -3400,8 +3420,7 @@ psgd_residual_rowlist_gs_batch_kernel(PsgdBatch<RowlistResidualItem<RP, FAST>> b
         return;
     }
     const int bx = (int)blockIdx.x - g.count;
-    int i = 0;
-    while (i + 1 < b.count && bx >= b.first[i + 1]) ++i;
+    const int i = psgd_batch_item(b, bx);
     const RowlistResidualItem<RP, FAST>& it = b.item[i];
     conef_rowlist_body<float, ListPsgdResidual<RP, FAST>>(it.front, it.plan, it.cs_in, it.cs_out, it.n, it.d, it.w, it.rb,
                                                           one_minus_beta, bx - b.first[i]);
@@ -3418,8 +3437,7 @@ psgd_pqt_gs_batch_kernel(PsgdBatch<PqtItem> b, GsAhead g)
         return;
     }
     const int bx = (int)blockIdx.x - g.count;
-    int i = 0;
-    while (i + 1 < b.count && bx >= b.first[i + 1]) ++i;
+    const int i = psgd_batch_item(b, bx);
     const PqtItem& it = b.item[i];
     const int local = bx - b.first[i];
     psgd_pqt_item<RP, MODE, FAST>(it, local);
@@ -3430,7 +3448,7 @@ psgd_pqt_gs_batch_kernel(PsgdBatch<PqtItem> b, GsAhead g)
 // thread (the thread's slice of Q, RP 16-byte loads, is then read once per sixteen rows of three
 // accesses each), at least four (one trip).
 inline void pqt_rows_table(const ConefPsgdItem* items, const std::vector<int>& members, int mode, std::vector<PqtItem>* table,
-                           std::vector<int>* blocks)
+                           std::vector<int>* blocks, const std::vector<float*>* qi)
 {
     int per_thread = 16;
     for (; per_thread > 4; per_thread >>= 1) {
@@ -3446,14 +3464,14 @@ inline void pqt_rows_table(const ConefPsgdItem* items, const std::vector<int>& m
         const int lanes = pqt_lanes(it.m);
         const int64_t rows = (int64_t)(256 / lanes) * per_thread, col_tiles = (it.m + 1023) / 1024;
         table->push_back(PqtItem{it.x, mode == 1 ? it.err : nullptr, it.p, it.q, it.n, (int)it.m, it.r, (int)rows,
-                                 (int)col_tiles, lanes});
+                                 (int)col_tiles, lanes, qi ? (*qi)[(size_t)j] : nullptr});
         blocks->push_back((int)(col_tiles * ((it.n + rows - 1) / rows)));
     }
 }
 
 template <int RP, bool FAST>
 int pqt_sketch_group(const ConefPsgdItem* items, const std::vector<int>& members, float beta, hipStream_t s,
-                     const GsAhead* ahead = nullptr)
+                     const GsAhead* ahead, const std::vector<float*>* qi)
 {
     std::vector<RowlistResidualItem<RP, FAST>> table;
     std::vector<int> blocks;
@@ -3471,7 +3489,7 @@ int pqt_sketch_group(const ConefPsgdItem* items, const std::vector<int>& members
         const ConefPsgdItem& it = items[j];
         ConefRowlistShape shape;
         if (!conef_rowlist_shape(it.n, it.m, it.w, false, &shape, companions)) return CONEF_ERR_INVALID;
-        RowlistResidualItem<RP, FAST> t = {{it.x, it.p, it.q, it.r},
+        RowlistResidualItem<RP, FAST> t = {{it.x, it.p, it.q, it.r, qi ? (*qi)[(size_t)j] : nullptr},
                                            conef_rowlist_view((const ConefPlanHeader*)it.plan_host, it.plan_dev),
                                            it.cs, it.cs, it.n, (int)it.m, it.w, shape.rb};
         table.push_back(t);
@@ -3497,7 +3515,7 @@ int pqt_sketch_group(const ConefPsgdItem* items, const std::vector<int>& members
 // ahead: the Q factors to orthogonalise alongside (mode 2, one rank class over the whole bucket
 // only); *ahead_used says whether that was done.
 int pqt_batch(const ConefPsgdItem* items, int count, int mode, float beta, int32_t a, int32_t b, hipStream_t s,
-              const GsAhead* ahead, bool* ahead_used)
+              const GsAhead* ahead, bool* ahead_used, const std::vector<float*>* qi)
 {
     if (ahead_used) *ahead_used = false;
     std::vector<char> done((size_t)count, 0);
@@ -3556,8 +3574,8 @@ int pqt_batch(const ConefPsgdItem* items, int count, int mode, float beta, int32
 #define CONEF_PQS(RP)                                                                  \
     do {                                                                               \
         if (RP >= 16) break;                                                           \
-        if (fast) rc = pqt_sketch_group<(RP < 16 ? RP : 8), true>(items, members, beta, s, ride);  \
-        else rc = pqt_sketch_group<(RP < 16 ? RP : 8), false>(items, members, beta, s, ride);      \
+        if (fast) rc = pqt_sketch_group<(RP < 16 ? RP : 8), true>(items, members, beta, s, ride, qi);  \
+        else rc = pqt_sketch_group<(RP < 16 ? RP : 8), false>(items, members, beta, s, ride, qi);      \
     } while (0)
                 CONEF_RANK_SWITCH(lead.r, CONEF_PQS)
 #undef CONEF_PQS
@@ -3588,7 +3606,7 @@ int pqt_batch(const ConefPsgdItem* items, int count, int mode, float beta, int32
         std::vector<PqtItem> table;
         std::vector<int> blocks;
         if (fast) {
-            pqt_rows_table(items, members, mode, &table, &blocks);
+            pqt_rows_table(items, members, mode, &table, &blocks, qi);
         } else {
             for (int j : members) {
                 const ConefPsgdItem& it = items[j];
@@ -3598,7 +3616,7 @@ int pqt_batch(const ConefPsgdItem* items, int count, int mode, float beta, int32
                 if (rps < 4) rps = 4;
                 slabs = (it.n + rps - 1) / rps;
                 table.push_back(PqtItem{it.x, mode == 1 ? it.err : nullptr, it.p, it.q, it.n, (int)it.m, it.r, (int)rps,
-                                        (int)col_tiles, 256});
+                                        (int)col_tiles, 256, nullptr});
                 blocks.push_back((int)(col_tiles * slabs));
             }
         }
@@ -3652,7 +3670,7 @@ int round_products(const ConefPsgdItem* items, const ConefPsgdItem* its, int cou
         }
         if (pr.padded)
             if (int rc = pad_rows(pad, r, pr.rp, s); rc != CONEF_OK) return rc;
-        return deferred_products(pr, r, q_in.data(), mq_mode, alpha, eps, a, b, workspace, workspace_bytes, s, nullptr);
+        return deferred_products(pr, r, q_in.data(), nullptr, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, s, nullptr);
     }
     int rc = conef_psgd_mq_batch_f32(its, count, mq_mode, alpha, a, b, workspace, workspace_bytes, (void*)s);
     if (rc != CONEF_OK) return rc;
@@ -3805,6 +3823,7 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
         ahead.nparts[k] = 0;
     }
     // the next round's Q factors are wanted in q_next
+    const bool by_quads = (flags & CONEF_ROUND_NEXT_QUADS) != 0;      // q_next[count + k]: the same by quads
     bool want_next = (flags & CONEF_ROUND_MAKE_NEXT) && count <= kPsgdBatchMax;
     for (int k = 0; k < count && want_next; ++k) want_next = q_next[k] && items[k].r == items[0].r && items[k].m <= 0x7fffffffLL;
     const int rp = rank_bound(items[0].r);
@@ -3842,7 +3861,7 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
             }
         }
         GsAhead* qs = want_next && rp <= 8 ? &ahead : nullptr;
-        rc = deferred_products(pr, r, q_in.data(), mq_mode, alpha, eps, a, b, workspace, workspace_bytes, hs, qs);
+        rc = deferred_products(pr, r, q_in.data(), by_quads && (flags & CONEF_ROUND_Q_READY) ? q_next + count : nullptr, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, hs, qs);
         if (rc != CONEF_OK) return rc;
     } else {
         std::vector<ConefPsgdItem> first(items, items + count);
@@ -3868,6 +3887,7 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
                 ahead.src[k] = its[k].q;
                 ahead.dst[k] = q_next[k];
                 ahead.rows[k] = (int)items[k].m;
+                ahead.quads[k] = deferred && by_quads ? q_next[count + k] : nullptr;
                 if (!deferred) ahead.parts[k] = nullptr;
             }
             ahead.count = count;
@@ -3877,7 +3897,7 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
     }
     bool used = false;
     rc = pqt_batch(its, count, pqt_mode == 3 ? 1 : pqt_mode, pqt_mode == 2 ? beta : 0.f, a, b, hs,
-                   ahead.count ? &ahead : nullptr, &used);
+                   ahead.count ? &ahead : nullptr, &used, deferred && rp <= 8 ? &pr.qi : nullptr);
     if (rc != CONEF_OK) return rc;
     if (want_next && deferred && rp > 8) {
         std::vector<const float*> src;

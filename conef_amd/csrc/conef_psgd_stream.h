@@ -31,6 +31,7 @@ struct MqsItem {
     // not null: workgroup g of the matrix also leaves the upper triangle of (its rows of P)^T (its
     // rows of P), RP (RP + 1) / 2 doubles, at gram[g * RP (RP + 1) / 2]: the shares of P^T P
     double* gram;
+    const float* qi;         // not null: q laid out by quads (conef_load_slices)
 };
 
 // threads of a group for a matrix of m columns in a workgroup of T threads
@@ -185,8 +186,7 @@ psgd_mqs_body(const MqsItem& it, float alpha, ConefSeeds hs, int bx)
             col = conef_quad_col(j, m);
             dup = 4 * j - col;
             valid = !idle && slab * gw + gt < m4;
-#pragma unroll
-            for (int t = 0; t < RP; ++t) conef_ld4u(it.q + (int64_t)col * RP + 4 * t, qreg + 4 * t);
+            conef_load_slices<RP>(conef_quad_slices<RP>(it.q, it.qi, j, col, m), qreg);
             if (!valid || dup) {        // another thread's columns (the last quad a second time, a moved quad's first ones): they add nothing
 #pragma unroll
                 for (int t = 0; t < 4 * RP; ++t)

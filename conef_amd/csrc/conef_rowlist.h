@@ -61,8 +61,9 @@ inline bool conef_rowlist_shape(int64_t n, int64_t d, int32_t w, bool cells, Con
 {
     if (d < 1 || d > kConefRowlistMaxCols || n < 1 || w < 1 || w > 0xffff) return false;
     int64_t rb = 8192 / d;
-    // tiles to spare: half-height ones, twice as many resident per CU (a quarter was slower again)
-    if (rb >= 2 && n / rb >= 2048) rb = (rb + 1) / 2;
+    // tiles to spare, in a front that keeps the column table in LDS next to them: half-height ones, twice as
+    // many resident per CU (a quarter was slower again; the other fronts are 2 % faster at full height)
+    if (cells && rb >= 2 && n / rb >= 2048) rb = (rb + 1) / 2;
     if (companions > 0 && rb > n * companions / 1024) rb = n * companions / 1024;
     if (rb > 16) rb = 16;
     if (rb < 1) rb = 1;
@@ -341,14 +342,14 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
     uint32_t ent_pre[kPreE], csr_pre[kPreC];
     const uint32_t ord_pre = ord_src[(int)threadIdx.x < ord_words ? (int)threadIdx.x : ord_words - 1];
 #pragma unroll
-    for (int u = 0; u < kPreE; ++u) {
+    for (int u = 0; u < kPreE; ++u) {                  // (uniform: a request past the end is a request all the same)
         const int i = threadIdx.x + u * kConefRowlistThreads;
-        ent_pre[u] = ent_src[i < ent_words ? i : ent_words - 1];
+        if (u * kConefRowlistThreads < ent_words) ent_pre[u] = ent_src[i < ent_words ? i : ent_words - 1];
     }
 #pragma unroll
     for (int u = 0; u < kPreC; ++u) {
         const int i = threadIdx.x + u * kConefRowlistThreads;
-        csr_pre[u] = plan.csr[i < csr_words ? i : csr_words - 1];
+        if (u * kConefRowlistThreads < csr_words) csr_pre[u] = plan.csr[i < csr_words ? i : csr_words - 1];
     }
     typename Front::Regs regs;
     uint32_t* pk_l = reinterpret_cast<uint32_t*>(cells + rb * w);
@@ -364,8 +365,8 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
 #pragma unroll
         for (int u = 0; u < kPark; ++u) {
             const int i = threadIdx.x + u * kConefRowlistThreads;
-            ct[u] = conef_ld(src + (i < count ? i : count - 1));
-            pt[u] = plan.pk[i < d ? i : d - 1];
+            if (u * kConefRowlistThreads < count) ct[u] = conef_ld(src + (i < count ? i : count - 1));
+            if (pk_lds && u * kConefRowlistThreads < d) pt[u] = plan.pk[i < d ? i : d - 1];
         }
 #pragma unroll
         for (int u = 0; u < kPark; ++u) {
@@ -390,7 +391,7 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
 #pragma unroll
         for (int u = 0; u < kPre; ++u) {
             const int p = threadIdx.x + u * kConefRowlistThreads;
-            aux_pre[u] = conef_ld(cs_in + row0 * w + (p < total ? p : total - 1));
+            if (u * kConefRowlistThreads < total) aux_pre[u] = conef_ld(cs_in + row0 * w + (p < total ? p : total - 1));
         }
     }
     if constexpr (Front::kNeedsCells) {

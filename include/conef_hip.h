@@ -389,6 +389,9 @@ int conef_psgd_products_f32(const ConefPsgdItem* items, const ConefPsgdItem* fir
  * interface. */
 #define CONEF_ROUND_Q_READY 1
 #define CONEF_ROUND_MAKE_NEXT 2
+/* q_next has 2 * count entries: q_next[count + k] is a second buffer of 16 * ceil(m / 4) times that many
+ * bytes, in which the library keeps the same factor in the order its kernels load it (ranks up to 8). */
+#define CONEF_ROUND_NEXT_QUADS 4
 int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_t mq_mode, int32_t pqt_mode, float alpha,
                                float beta, float eps, int32_t a, int32_t b, float* const* q_next, int32_t flags,
                                int32_t* made, void* workspace, int64_t workspace_bytes, void* stream);
