@@ -55,6 +55,10 @@ struct TopkItem {
     int64_t numel;
     TopkState* st;
     uint32_t k;
+    uint32_t cap;               // candidates a workgroup's segment holds
+    uint32_t* counts;           // [workgroups] candidates found, or kTopkOverflow
+    uint2* list;                // [workgroups][cap] (index, magnitude key)
+    uint32_t* final_idx;        // [kTopkFinal] the keys that share two digits with the threshold, then their keys
 };
 
 struct TopkBatch {
@@ -86,26 +90,18 @@ __global__ void topk_init_kernel(TopkState* st, uint32_t k) { topk_init_body(st,
 
 __global__ void topk_init_batch_kernel(TopkBatch b) { topk_init_body(b.item[blockIdx.x].st, b.item[blockIdx.x].k); }
 
-// What pass `p` selected, from its finished histogram: the digit holding the k-th largest key
-// among those matching the earlier digits.  Every thread of a 256-thread workgroup returns the
-// same (prefix, remaining, ties); workgroup 0 (bx) of the tensor also leaves them in the state for
-// the next kernel.
-__device__ __forceinline__ void topk_resolve(TopkState* st, int p, uint32_t* prefix, uint32_t* remaining, uint32_t* ties,
-                                             int bx)
+// The bin that holds the want-th largest of the keys counted in 256 * per bins, thread t holding the counts
+// of bins t * per .. in cnt: (bin, how many are wanted of it, how many it holds), the same in every
+// thread of a 256-thread workgroup.
+__device__ __forceinline__ void topk_pick(const uint32_t (&cnt)[8], int per, uint32_t want, uint32_t* bin, uint32_t* wanted,
+                                          uint32_t* held)
 {
     __shared__ uint32_t wave_sum[4];
     __shared__ uint32_t picked[3];
-    const uint32_t before_prefix = p == 0 ? 0u : st->prefix[p - 1];
-    const uint32_t before_remaining = p == 0 ? st->k : st->remaining[p - 1];
-    const int bins = 1 << kDigitBits[p], per = bins / 256;          // 8, 8, 2 bins per thread
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    uint32_t cnt[8];
     uint32_t mine = 0;
-    for (int b = 0; b < per; ++b) {
-        cnt[b] = st->hist[p][threadIdx.x * per + b];
-        mine += cnt[b];
-    }
-    // suffix sums over threads: keys in digits above mine
+    for (int b = 0; b < per; ++b) mine += cnt[b];
+    // suffix sums over threads: keys in bins above mine
     uint32_t incl = mine;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -116,25 +112,42 @@ __device__ __forceinline__ void topk_resolve(TopkState* st, int p, uint32_t* pre
     __syncthreads();
     uint32_t above = incl - mine;
     for (int wv = wave + 1; wv < 4; ++wv) above += wave_sum[wv];
-    // exactly one (thread, bin) satisfies above < remaining <= above + count
+    // exactly one (thread, bin) satisfies above < want <= above + count
     for (int b = per - 1; b >= 0; --b) {
-        if (above < before_remaining && before_remaining <= above + cnt[b]) {
-            picked[0] = (before_prefix << kDigitBits[p]) | (uint32_t)(threadIdx.x * per + b);
-            picked[1] = before_remaining - above;
+        if (above < want && want <= above + cnt[b]) {
+            picked[0] = (uint32_t)(threadIdx.x * per + b);
+            picked[1] = want - above;
             picked[2] = cnt[b];
         }
         above += cnt[b];
     }
     __syncthreads();
-    *prefix = picked[0];
-    *remaining = picked[1];
-    *ties = picked[2];
-    if (bx == 0 && threadIdx.x == 0) {
-        st->prefix[p] = picked[0];
-        st->remaining[p] = picked[1];
-        st->ties[p] = picked[2];
-    }
+    *bin = picked[0];
+    *wanted = picked[1];
+    *held = picked[2];
     __syncthreads();
+}
+
+// What pass `p` selected, from its finished histogram: the digit holding the k-th largest key
+// among those matching the earlier digits.  Every thread of a 256-thread workgroup returns the
+// same (prefix, remaining, ties); workgroup 0 (bx) of the tensor also leaves them in the state for
+// the next kernel.
+__device__ __forceinline__ void topk_resolve(TopkState* st, int p, uint32_t* prefix, uint32_t* remaining, uint32_t* ties,
+                                             int bx)
+{
+    const uint32_t before_prefix = p == 0 ? 0u : st->prefix[p - 1];
+    const uint32_t before_remaining = p == 0 ? st->k : st->remaining[p - 1];
+    const int per = (1 << kDigitBits[p]) / 256;          // 8, 8, 2 bins per thread
+    uint32_t cnt[8];
+    for (int b = 0; b < per; ++b) cnt[b] = st->hist[p][threadIdx.x * per + b];
+    uint32_t digit;
+    topk_pick(cnt, per, before_remaining, &digit, remaining, ties);
+    *prefix = (before_prefix << kDigitBits[p]) | digit;
+    if (bx == 0 && threadIdx.x == 0) {
+        st->prefix[p] = *prefix;
+        st->remaining[p] = *remaining;
+        st->ties[p] = *ties;
+    }
 }
 
 // REP copies of every bin, copy = lane % REP, laid out [bin][copy]: the keys of a gradient crowd
@@ -142,7 +155,7 @@ __device__ __forceinline__ void topk_resolve(TopkState* st, int p, uint32_t* pre
 // wave that meet in a bin then add to different LDS banks instead of queueing on one address.
 // `kept` (a state that stays with its tensor from call to call, zero-filled before the first): no
 // launch clears the state; the first workgroup of pass 0 clears what the later passes count into,
-// and the filter's clears what pass 0 of the next call counts into (topk_filter_body).
+// and pass 2's clears what pass 0 of the next call counts into (topk_settle_body).
 template <int REP>
 __device__ __forceinline__ void
 topk_hist_body(const float* __restrict__ x, int64_t numel, TopkState* st, int pass, int bx, int gx, bool kept = false,
@@ -266,14 +279,12 @@ __device__ __forceinline__ void topk_order_ties(float* __restrict__ x, int64_t n
 
 // keep key >= threshold, zero the rest, settle surplus ties on the threshold by index
 __device__ __forceinline__ void
-topk_filter_body(float* __restrict__ x, int64_t numel, TopkState* st, int bx, int gx, bool kept = false)
+topk_filter_body(float* __restrict__ x, int64_t numel, TopkState* st, int bx, int gx)
 {
     __shared__ uint32_t ticket;
     __shared__ uint32_t idx_l[kTieMax];
     uint32_t thr, keep_ties, ties;
     topk_resolve(st, kPasses - 1, &thr, &keep_ties, &ties, bx);
-    if (kept && bx == 0)       // nobody reads the first digit's counters any more: ready for the next call
-        for (int i = threadIdx.x; i < kBins; i += 256) st->hist[0][i] = 0u;
     const bool surplus = ties != keep_ties && thr != 0u;      // a zero threshold has only zeros for ties
     const bool listed = surplus && ties <= (uint32_t)kTieMax;
     auto note = [&](int64_t i) {
@@ -349,13 +360,252 @@ topk_filter_kernel(float* __restrict__ x, int64_t numel, TopkState* st)
 }
 
 __global__ void __launch_bounds__(256)
-topk_filter_batch_kernel(TopkBatch b, bool kept)
+topk_filter_batch_kernel(TopkBatch b)
 {
     int local, width;
     const TopkItem& it = b.item[topk_locate(b.first, b.count, &local, &width)];
-    topk_filter_body(it.x, it.numel, it.st, local, width, kept);
+    topk_filter_body(it.x, it.numel, it.st, local, width);
 }
 
+
+// ---- selection through a candidate list ----
+// Three histogram passes and the filter read a tensor four times.  After the first digit, though, only
+// the keys that share it with the threshold are undecided - about one in twenty of a gradient's error,
+// 11 bits being an exponent and three mantissa bits.  So, for a workspace that stays with its tensors:
+//   pass 0     the first digit's histogram, as above;
+//   pass 1     zeroes what lies below the digit, counts the second digit of the keys that share it
+//              and notes them, (index, key), each workgroup in a segment of its own: no counter is shared;
+//   pass 2     goes over the notes alone: zeroes what lies below the first two digits and gathers the
+//              keys that share both (a few hundred); the workgroup that finishes last ranks those.
+// Two reads and one write of the tensor instead of four and one.  A workgroup whose segment runs over
+// (more than a quarter of its keys share the digit) goes over its elements again in pass 2; more than
+// kTopkFinal keys that share two digits (a tensor of repeated values) are settled by one workgroup
+// walking the tensor.
+constexpr uint32_t kTopkOverflow = 0xffffffffu;
+constexpr int kTopkFinal = 2048;
+constexpr int kTopkTrip = 8;             // quads a thread requests together
+
+// f(index, key) for every element of a workgroup's share, in trips: the elements of quads first, then the rest
+template <typename F>
+__device__ __forceinline__ void topk_for_each(const float* x, int64_t numel, int bx, int gx, F f)
+{
+    const int64_t quads = numel >> 2, stride = (int64_t)gx * 256;
+    for (int64_t q0 = bx * (int64_t)256 + threadIdx.x; q0 < quads; q0 += stride) {
+        float v[4];
+        conef_ld4u(x + 4 * q0, v);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f(4 * q0 + e, mag_key(v[e]));
+    }
+    for (int64_t i = quads * 4 + bx * (int64_t)256 + threadIdx.x; i < numel; i += stride) f(i, mag_key(x[i]));
+}
+
+__device__ __forceinline__ void topk_note_body(const TopkItem& it, int bx, int gx)
+{
+    __shared__ uint32_t bins[kBins];
+    __shared__ uint32_t found;
+    TopkState* st = it.st;
+    uint32_t digit, remaining, ties;
+    topk_resolve(st, 0, &digit, &remaining, &ties, bx);
+    for (int i = threadIdx.x; i < kBins; i += 256) bins[i] = 0u;
+    if (threadIdx.x == 0) found = 0u;
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    const int shift = kDigitShift[0];
+    uint2* seg = it.list + (size_t)bx * it.cap;
+    const int64_t quads = it.numel >> 2, stride = (int64_t)gx * 256;
+    const int64_t rest0 = quads * 4;
+    // A thread's quads of one trip; the elements behind the last quad are a trip of single ones at the end.
+    // Zeros are never noted: there is nothing to clear in them (they are counted where they share the digit).
+    uint32_t zeros = 0u;
+    auto note = [&](uint32_t mask, auto index_of, auto key_of) {
+        const uint32_t mine = (uint32_t)__popc(mask);
+        uint32_t incl = mine;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t t = __shfl_up(incl, off, 64);
+            if (lane >= off) incl += t;
+        }
+        const uint32_t total = __shfl(incl, 63, 64);
+        uint32_t base = 0;
+        if (total && lane == 63) base = atomicAdd(&found, total);
+        base = __shfl(base, 63, 64) + incl - mine;
+        while (mask) {
+            const int b = __ffs(mask) - 1;
+            mask &= mask - 1;
+            const uint32_t key = key_of(b);
+            atomicAdd(&bins[(key >> kDigitShift[1]) & (kBins - 1)], 1u);
+            if (base < it.cap) seg[base] = make_uint2(index_of(b), key);
+            ++base;
+        }
+    };
+    for (int64_t t0 = bx * (int64_t)256; t0 < quads; t0 += kTopkTrip * stride) {     // uniform: the waves scan together
+        const int64_t q0 = t0 + threadIdx.x;
+        float v[kTopkTrip][4];
+#pragma unroll
+        for (int u = 0; u < kTopkTrip; ++u) {
+            const int64_t q = q0 + u * stride;
+            conef_ld4u(it.x + 4 * (q < quads ? q : quads - 1), v[u]);
+        }
+        uint32_t mask = 0u;
+#pragma unroll
+        for (int u = 0; u < kTopkTrip; ++u) {
+            const int64_t q = q0 + u * stride;
+            if (q >= quads) continue;
+            float o[4];
+            bool any = false;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t key = mag_key(v[u][e]), d = key >> shift;
+                o[e] = d >= digit ? v[u][e] : 0.f;
+                any |= d < digit;
+                if (d == digit) {
+                    if (key) mask |= 1u << (4 * u + e);
+                    else ++zeros;
+                }
+            }
+            if (any) conef_st4u(it.x + 4 * q, o);
+        }
+        note(mask, [&](int b) { return (uint32_t)(4 * (q0 + (b >> 2) * stride) + (b & 3)); },
+             [&](int b) {
+                 float f = 0.f;
+#pragma unroll
+                 for (int u = 0; u < kTopkTrip; ++u)
+#pragma unroll
+                     for (int e = 0; e < 4; ++e) f = b == 4 * u + e ? v[u][e] : f;
+                 return mag_key(f);
+             });
+    }
+    for (int64_t t0 = rest0 + bx * (int64_t)256; t0 < it.numel; t0 += stride) {
+        const int64_t i = t0 + threadIdx.x;
+        uint32_t key = 0u;
+        if (i < it.numel) {
+            key = mag_key(it.x[i]);
+            if ((key >> shift) < digit) it.x[i] = 0.f;
+            if (digit == 0u && !key) ++zeros;
+        }
+        note(key && (key >> shift) == digit ? 1u : 0u, [&](int) { return (uint32_t)i; }, [&](int) { return key; });
+    }
+    if (zeros) atomicAdd(&bins[0], zeros);
+    __syncthreads();
+    if (threadIdx.x == 0) it.counts[bx] = found <= it.cap ? found : kTopkOverflow;
+    for (int i = threadIdx.x; i < kBins; i += 256)
+        if (bins[i]) atomicAdd(&st->hist[1][i], bins[i]);
+}
+
+// One workgroup: of the keys that share `prefix` (the first two digits) the `keep` largest stay, equal
+// ones in index order; the others are cleared.  each(f) calls f(index, key) for the keys.
+constexpr int kTopkLow = 1 << kDigitBits[2];
+
+template <typename Each>
+__device__ __forceinline__ void topk_last_digit(uint32_t (&bins)[kTopkLow], uint32_t prefix, uint32_t keep, Each each,
+                                                uint32_t* thr, uint32_t* ties, uint32_t* held)
+{
+    for (int i = threadIdx.x; i < kTopkLow; i += 256) bins[i] = 0u;
+    __syncthreads();
+    each([&](uint32_t, uint32_t key) { atomicAdd(&bins[key & (kTopkLow - 1)], 1u); });
+    __syncthreads();
+    uint32_t cnt[8], digit;
+    for (int b = 0; b < kTopkLow / 256; ++b) cnt[b] = bins[threadIdx.x * (kTopkLow / 256) + b];
+    topk_pick(cnt, kTopkLow / 256, keep, &digit, ties, held);
+    *thr = (prefix << kDigitBits[2]) | digit;
+}
+
+__device__ __forceinline__ void topk_settle_body(const TopkItem& it, int bx, int gx)
+{
+    __shared__ uint32_t ticket;
+    __shared__ uint32_t key_l[kTopkFinal], idx_l[kTopkFinal];
+    TopkState* st = it.st;
+    uint32_t prefix, keep, share;                        // `share` keys share both digits, `keep` of them stay
+    topk_resolve(st, 1, &prefix, &keep, &share, bx);
+    if (bx == 0)       // nobody reads the first digit's counters any more: ready for the next call
+        for (int i = threadIdx.x; i < kBins; i += 256) st->hist[0][i] = 0u;
+    const uint32_t digit = prefix >> kDigitBits[1];
+    auto one = [&](uint32_t i, uint32_t key) {
+        const uint32_t two = key >> kDigitBits[2];
+        if (two < prefix) {
+            it.x[i] = 0.f;
+        } else if (two == prefix && keep < share) {      // all of them stay otherwise
+            const uint32_t slot = atomicAdd(&st->tie_count, 1u);
+            if (slot < (uint32_t)kTopkFinal) {
+                __hip_atomic_store(it.final_idx + slot, i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(it.final_idx + kTopkFinal + slot, key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+    };
+    const uint32_t n = it.counts[bx];
+    if (n != kTopkOverflow) {
+        const uint2* seg = it.list + (size_t)bx * it.cap;
+        for (uint32_t j0 = threadIdx.x; j0 < n; j0 += 4 * 256) {
+            uint2 c[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) c[u] = seg[j0 + u * 256 < n ? j0 + u * 256 : j0];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (j0 + u * 256 < n) one(c[u].x, c[u].y);
+        }
+    } else {
+        topk_for_each(it.x, it.numel, bx, gx, [&](int64_t i, uint32_t key) {
+            if (key && (key >> kDigitShift[0]) == digit) one((uint32_t)i, key);
+        });
+    }
+    if (keep >= share) return;
+    // The gathered keys went out past the caches (agent-scope stores): once they have arrived a plain count
+    // tells the last workgroup that it can see them all.  Nobody reads what anybody else clears.  (A
+    // fence here writes back whatever the caches hold, 10 to 30 us behind the passes before.)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) ticket = atomicAdd(&st->done, 1u);
+    __syncthreads();
+    if (ticket != (uint32_t)gx - 1u) return;
+    const uint32_t m = __hip_atomic_load(&st->tie_count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (m <= keep) return;                               // the rest of the share are zeros
+    __shared__ uint32_t low[kTopkLow];
+    uint32_t thr, ties, held;
+    if (m > (uint32_t)kTopkFinal) {
+        topk_last_digit(low, prefix, keep, [&](auto f) {
+            topk_for_each(it.x, it.numel, 0, 1, [&](int64_t i, uint32_t key) {
+                if (key && (key >> kDigitBits[2]) == prefix) f((uint32_t)i, key);
+            });
+        }, &thr, &ties, &held);
+        topk_for_each(it.x, it.numel, 0, 1, [&](int64_t i, uint32_t key) {
+            if (key < thr && (key >> kDigitBits[2]) == prefix) it.x[i] = 0.f;
+        });
+        if (ties < held) topk_order_ties(it.x, it.numel, thr, ties);
+        return;
+    }
+    for (uint32_t j = threadIdx.x; j < m; j += 256) {
+        idx_l[j] = __hip_atomic_load(it.final_idx + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        key_l[j] = __hip_atomic_load(it.final_idx + kTopkFinal + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    topk_last_digit(low, prefix, keep, [&](auto f) {
+        for (uint32_t j = threadIdx.x; j < m; j += 256) f(idx_l[j], key_l[j]);
+    }, &thr, &ties, &held);
+    for (uint32_t j = threadIdx.x; j < m; j += 256) {
+        const uint32_t key = key_l[j], idx = idx_l[j];
+        if (key > thr || (key == thr && ties == held)) continue;
+        uint32_t rank = 0;
+        if (key == thr)
+            for (uint32_t t = 0; t < m; ++t) rank += key_l[t] == key && idx_l[t] < idx;
+        if (key < thr || rank >= ties) it.x[idx] = 0.f;
+    }
+}
+
+__global__ void __launch_bounds__(256)
+topk_note_batch_kernel(TopkBatch b)
+{
+    int local, width;
+    const TopkItem& it = b.item[topk_locate(b.first, b.count, &local, &width)];
+    topk_note_body(it, local, width);
+}
+
+__global__ void __launch_bounds__(256)
+topk_settle_batch_kernel(TopkBatch b)
+{
+    int local, width;
+    const TopkItem& it = b.item[topk_locate(b.first, b.count, &local, &width)];
+    topk_settle_body(it, local, width);
+}
 
 // Workgroups of a pass over a tensor.  A histogram workgroup ends with one global atomic per bin
 // it touched, all workgroups on the same few dozen counters, and a filter workgroup that has to
@@ -364,7 +614,7 @@ topk_filter_batch_kernel(TopkBatch b, bool kept)
 inline int64_t topk_hist_groups(int64_t numel)
 {
     int64_t g = (numel + 255) / 256 / 64;
-    return g < 1 ? 1 : g > 512 ? 512 : g;
+    return g < 1 ? 1 : g > 1024 ? 1024 : g;
 }
 
 
@@ -433,6 +683,22 @@ int conef_topk_sparsify_f32(float* x, int64_t numel, int64_t k, void* workspace,
     return (int)hipGetLastError();
 }
 
+namespace {
+// candidates a workgroup of the note pass has room for: a quarter of its elements
+inline int64_t topk_segment(int64_t numel)
+{
+    const int64_t g = topk_hist_groups(numel);
+    return ((numel + g - 1) / g / 4 + 63) / 64 * 64;
+}
+
+// a tensor's part of a batch workspace: the state, the workgroups' counts, their segments
+inline int64_t topk_batch_item_bytes(int64_t numel)
+{
+    const int64_t g = topk_hist_groups(numel);
+    return (int64_t)kScratchBytes + 8 * kTopkFinal + (4 * g + 255) / 256 * 256 + g * topk_segment(numel) * 8;
+}
+}  // namespace
+
 // The same for `count` tensors, every pass one launch over all of them (in runs of 24): tensor i
 // is xs[i] with numels[i] elements and keeps ks[i]; tensors with ks[i] >= numels[i] are left as
 // they are.  xs / numels / ks are host arrays, read before the call returns.
@@ -442,7 +708,7 @@ int64_t conef_topk_batch_workspace_bytes(const int64_t* numels, int32_t count)
     int64_t total = 0;
     for (int i = 0; i < count; ++i) {
         if (numels[i] < 0) return -1;
-        total += (conef_topk_workspace_bytes(numels[i]) + 255) / 256 * 256;
+        total += topk_batch_item_bytes(numels[i]);
     }
     return total > 256 ? total : 256;
 }
@@ -465,13 +731,17 @@ int topk_sparsify_batch(float* const* xs, const int64_t* numels, const int64_t* 
         int nb = 0, wgs = 0;
         for (; i < count && nb < kTopkBatchMax; ++i) {
             char* mine = ws;
-            ws += (conef_topk_workspace_bytes(numels[i]) + 255) / 256 * 256;
+            ws += topk_batch_item_bytes(numels[i]);
             if (ks[i] >= numels[i]) continue;
             TopkItem& it = b.item[nb];
             it.x = xs[i];
             it.numel = numels[i];
             it.st = (TopkState*)mine;
             it.k = (uint32_t)ks[i];
+            it.cap = (uint32_t)topk_segment(numels[i]);
+            it.final_idx = (uint32_t*)(mine + kScratchBytes);
+            it.counts = it.final_idx + 2 * kTopkFinal;
+            it.list = (uint2*)(mine + kScratchBytes + 8 * kTopkFinal + (4 * topk_hist_groups(numels[i]) + 255) / 256 * 256);
             b.first[nb] = wgs;
             wgs += (int)topk_hist_groups(numels[i]);
             ++nb;
@@ -479,10 +749,17 @@ int topk_sparsify_batch(float* const* xs, const int64_t* numels, const int64_t* 
         if (nb == 0) continue;
         b.first[nb] = wgs;
         b.count = nb;
-        if (!kept) hipLaunchKernelGGL(topk_init_batch_kernel, dim3((unsigned)nb), dim3(256), 0, s, b);
+        const dim3 grid((unsigned)wgs), threads(256);
+        if (kept) {
+            hipLaunchKernelGGL(topk_hist_batch_kernel, grid, threads, 0, s, b, 0, true);
+            hipLaunchKernelGGL(topk_note_batch_kernel, grid, threads, 0, s, b);
+            hipLaunchKernelGGL(topk_settle_batch_kernel, grid, threads, 0, s, b);
+            continue;
+        }
+        hipLaunchKernelGGL(topk_init_batch_kernel, dim3((unsigned)nb), threads, 0, s, b);
         for (int pass = 0; pass < kPasses; ++pass)
-            hipLaunchKernelGGL(topk_hist_batch_kernel, dim3((unsigned)wgs), dim3(256), 0, s, b, pass, kept);
-        hipLaunchKernelGGL(topk_filter_batch_kernel, dim3((unsigned)wgs), dim3(256), 0, s, b, kept);
+            hipLaunchKernelGGL(topk_hist_batch_kernel, grid, threads, 0, s, b, pass, false);
+        hipLaunchKernelGGL(topk_filter_batch_kernel, grid, threads, 0, s, b);
     }
     return (int)hipGetLastError();
 }
@@ -496,8 +773,8 @@ int conef_topk_sparsify_batch_f32(float* const* xs, const int64_t* numels, const
 
 // The same for a workspace that stays with its tensors: zero-filled by the caller before its first
 // use and passed to nothing but this entry point, with the same xs / numels / count, afterwards.
-// No launch clears the selection state then (the passes clear behind themselves): four launches a
-// call instead of five.
+// No launch clears the selection state then (the passes clear behind themselves), and the selection goes
+// through a candidate list: three launches a call instead of five, two reads of a tensor instead of four.
 int conef_topk_sparsify_batch_kept_f32(float* const* xs, const int64_t* numels, const int64_t* ks, int32_t count,
                                        void* workspace, int64_t workspace_bytes, void* stream)
 {

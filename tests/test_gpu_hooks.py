@@ -1106,6 +1106,63 @@ def test_round_of_more_matrices_than_a_launch_takes(monkeypatch, oracle, mode, r
     assert len(st.round_cache[0].chunks) == 2
 
 
+def _topk_inputs():
+    """(name, values, k): the branches of the selection through a candidate list."""
+    g = torch.Generator().manual_seed(7)
+    x = torch.randn(100_003, generator=g) * 1e-3
+    yield "one trip and a rest", x[:1025].clone(), 100
+    yield "gradient-like", x.clone(), 20_000
+    yield "k of one", x[:4099].clone(), 1
+    yield "all but one", x[:4099].clone(), 4098
+    narrow = 1.0 + 1e-3 * torch.rand(70_001, generator=g)
+    yield "more candidates than a segment holds", narrow * torch.sign(x[:70_001]), 30_000
+    steps = torch.randint(0, 3, (60_000,), generator=g).float() * torch.sign(x[:60_000])
+    yield "more equal keys than the final list holds", steps, 25_000
+    sparse = torch.where(torch.rand(50_001, generator=g) < 0.1, x[:50_001], torch.zeros(()))
+    yield "fewer values than k", sparse, 20_000
+    tiny = sparse.clone()
+    tiny[::7] = 1e-42
+    tiny[1::11] = -3e-43
+    yield "the threshold among denormal numbers", tiny, 10_000
+    few = x[:2000].clone()
+    few[500:540] = few.abs().kthvalue(1000).values
+    yield "ties at the threshold", few, 1010
+
+
+def test_topk_through_a_candidate_list():
+    """The entry point whose workspace stays with its tensors (the hooks' one), three calls on one
+    workspace, every tensor alone and all of them in one batch."""
+    import ctypes
+    from conef_amd import _lib
+    lib = _lib.load()
+
+    def batches():
+        cases = list(_topk_inputs())
+        for c in cases:
+            yield [c]
+        yield cases
+
+    for batch in batches():
+        n = len(batch)
+        tensors = [v.cuda() for _, v, _ in batch]
+        ptrs = (ctypes.c_void_p * n)(*[t.data_ptr() for t in tensors])
+        numels = (ctypes.c_int64 * n)(*[t.numel() for t in tensors])
+        ks = (ctypes.c_int64 * n)(*[k for _, _, k in batch])
+        ws = torch.zeros(lib.conef_topk_batch_workspace_bytes(numels, n), dtype=torch.uint8, device="cuda")
+        for call in range(3):
+            for t, (_, v, _) in zip(tensors, batch):
+                t.copy_(v.roll(call))
+            rc = lib.conef_topk_sparsify_batch_kept_f32(ptrs, numels, ks, n, ws.data_ptr(), ws.numel(),
+                                                        torch.cuda.current_stream().cuda_stream)
+            assert rc == 0
+            for t, (name, v, k) in zip(tensors, batch):
+                full = v.roll(call).numpy()
+                want = np.zeros_like(full)
+                order = np.argsort(-np.abs(full), kind="stable")[:k]
+                want[order] = full[order]
+                np.testing.assert_array_equal(to_np(t), want, err_msg="%s, call %d, batch of %d" % (name, call, n))
+
+
 def test_powersgd_state_errors_and_warmup():
     from conef_amd.powerSGD_hook import PowerSGDState, _should_compress, powerSGD_hook
     with pytest.raises(ValueError, match="Expect `start_powerSGD_iter` > 1"):
