@@ -169,14 +169,34 @@ psgd_mqs_body(const MqsItem& it, float alpha, ConefSeeds hs, int bx)
             if (MODE == 1) conef_ld4u(it.err + off, en[a]);
         }
     };
-    request(0);
-    if (MODE == 2) {
-        const float* src = it.cs + wg_row0 * w;
-        for (int i = tid; i < rows_here * w; i += T) cells[i] = src[i];
-        __syncthreads();
-    }
+    // a slab's slice of Q and its columns' buckets.  With sketch rows to wait for, the first slab's travel with them;
+    // without, the registers they would hold that long cost more than the wait (MODE 1 at rank 8: 926 against 915 us
+    // over BERT's buckets)
     float qreg[4 * RP];
     uint32_t pk[4] = {0u, 0u, 0u, 0u};
+    auto request_slab = [&](int slab) {
+        const int j = quad_of(slab), c = conef_quad_col(j, m);
+        conef_load_slices<RP>(conef_quad_slices<RP>(it.q, it.qi, j, c, m), qreg);
+        if (MODE == 2 && it.pktab) conef_ld4u(it.pktab + c, pk);
+    };
+    request(0);
+    if (MODE == 2) {
+        request_slab(0);
+        // the workgroup's sketch rows, eight requests a thread at a time: one by one, as a plain loop, each was
+        // a trip to memory, 7 of the 16 us of a [640, 5760] launch with 1152 cells a row
+        const float* src = it.cs + wg_row0 * w;
+        const int count = rows_here * w;
+        for (int i0 = tid; i0 < count; i0 += 8 * T) {
+            float t[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (i0 - tid + u * T < count) t[u] = src[i0 + u * T < count ? i0 + u * T : count - 1];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (i0 + u * T < count) cells[i0 + u * T] = t[u];
+        }
+        __syncthreads();
+    }
     bool valid = false;
     int col = 0, dup = 0;
     for (int iter = 0; iter < niter; ++iter) {
@@ -186,16 +206,14 @@ psgd_mqs_body(const MqsItem& it, float alpha, ConefSeeds hs, int bx)
             col = conef_quad_col(j, m);
             dup = 4 * j - col;
             valid = !idle && slab * gw + gt < m4;
-            conef_load_slices<RP>(conef_quad_slices<RP>(it.q, it.qi, j, col, m), qreg);
+            if (MODE != 2 || slab > 0) request_slab(slab);
             if (!valid || dup) {        // another thread's columns (the last quad a second time, a moved quad's first ones): they add nothing
 #pragma unroll
                 for (int t = 0; t < 4 * RP; ++t)
                     if (!valid || t / RP < dup) qreg[t] = 0.f;
             }
             if (MODE == 2) {
-                if (it.pktab) {
-                    conef_ld4u(it.pktab + col, pk);
-                } else {
+                if (!it.pktab) {
 #pragma unroll
                     for (int k = 0; k < 4; ++k) pk[k] = conef_bucket_sign(col + k, it.mod, hs.a, hs.b, hs.sa, hs.sb);
                 }
@@ -244,6 +262,7 @@ psgd_mqs_body(const MqsItem& it, float alpha, ConefSeeds hs, int bx)
         float s = 0.f;
         for (int slab = 0; slab < nslab; ++slab) {
             const float* base = red + ((size_t)(slab * nblk + b) * WAVES + gg * wpg) * NV + idx;
+#pragma unroll 4
             for (int v = 0; v < wpg; ++v) s += base[(size_t)v * NV];
         }
         it.p[(wg_row0 + lr) * RP + c] = s;
@@ -260,6 +279,7 @@ psgd_mqs_body(const MqsItem& it, float alpha, ConefSeeds hs, int bx)
             }
             const int j = i + (tid - e0);
             double s = 0.;
+#pragma unroll 8
             for (int lr = 0; lr < rows_here; ++lr) s = fma((double)prow[lr * RP + i], (double)prow[lr * RP + j], s);
             it.gram[(size_t)bx * NG + tid] = s;
         }
