@@ -127,7 +127,7 @@ class _RoundPlan:
     and layout, so that a step costs a handful of foreign calls however many tensors it has."""
     __slots__ = ("small", "sig", "errs_sig", "cs_static", "env_ahead", "env_topk_side", "env_small", "key", "shapes", "work", "passthrough", "before", "after", "total_ps", "total_qs", "arena_key", "ps",
                  "qs", "items", "count", "sketches", "fused_sketch", "batched_update", "residual_offsets",
-                 "topk_table", "q_next", "q_next_ptrs", "q_next_ready", "made", "q_next_event",
+                 "topk_table", "q_next", "q_next_ptrs", "q_next_ready", "made", "q_next_event", "aside_recorded",
                  "topk_event", "ws_need", "handoff_event", "topk_number", "q_next_number", "is_wide", "wide", "chunks", "ef_spans")
 
 
@@ -218,6 +218,7 @@ def _build_round(state, grads, shapes, key, error_mode):
     plan.q_next_ready = False
     plan.made = None
     plan.q_next_event = None
+    plan.aside_recorded = None      # the side stream (raw) that q_next and the Q arena are known to the allocator to be used on
     plan.chunks = _chunks(plan.count)
     plan.ef_spans = None            # dense error feedback: host arrays of the stretches that are not compressed
     plan.residual_offsets = []
@@ -227,6 +228,22 @@ def _build_round(state, grads, shapes, key, error_mode):
         off += n * m
     plan.residual_offsets.append(off)
     return plan
+
+
+def _take_arenas(plan, p_mem, q_mem):
+    """Points the table of matrices at the bucket's P and Q arenas.  What belonged to the arenas before -
+    the second buffer of the Q factors, what the allocator was told about either - goes with them."""
+    plan.ps, plan.qs, p_idx, q_idx = [], [], 0, 0
+    for it, (_, n, m, rank) in zip(plan.items, plan.work):
+        plan.ps.append(p_mem[p_idx: p_idx + n * rank].view(n, rank))
+        plan.qs.append(q_mem[q_idx: q_idx + m * rank].view(m, rank))
+        it.p, it.q = plan.ps[-1].data_ptr(), plan.qs[-1].data_ptr()
+        p_idx += n * rank
+        q_idx += m * rank
+    plan.arena_key = (p_mem.data_ptr(), q_mem.data_ptr())
+    plan.q_next = None
+    plan.q_next_ready = False
+    plan.aside_recorded = None
 
 
 _side_stream = _pools.side_stream
@@ -262,6 +279,15 @@ def wait_for_side_topk(plan, device, stream_now):
     if plan.topk_number is not None:
         _pools.side_wait(device, stream_now(), plan.topk_number)
         plan.topk_number = None
+
+
+def wait_for_side_q(plan, device, stream_now):
+    """Orders the stream a round is about to run on after the side stream's work on the bucket's Q factors
+    from its previous round: it reads the Q arena and writes ``plan.q_next``, whichever of the two the
+    round goes on to use and whichever stream it runs on now."""
+    if plan.q_next_number is not None:
+        _pools.side_wait(device, stream_now(), plan.q_next_number)
+        plan.q_next_number = None
 
 
 def settle(state):
@@ -369,16 +395,7 @@ def _run_round(state, bucket, error_mode, streams=1):
         state.q_memory_dict[bucket_index] = torch.empty(plan.total_qs, device=device, dtype=dtype)
     p_mem, q_mem = state.p_memory_dict[bucket_index], state.q_memory_dict[bucket_index]
     if plan.arena_key != (p_mem.data_ptr(), q_mem.data_ptr()):
-        plan.ps, plan.qs, p_idx, q_idx = [], [], 0, 0
-        for cnt, (matrix, n, m, rank) in enumerate(work):
-            plan.ps.append(p_mem[p_idx: p_idx + n * rank].view(n, rank))
-            plan.qs.append(q_mem[q_idx: q_idx + m * rank].view(m, rank))
-            items[cnt].p, items[cnt].q = plan.ps[-1].data_ptr(), plan.qs[-1].data_ptr()
-            p_idx += n * rank
-            q_idx += m * rank
-        plan.arena_key = (p_mem.data_ptr(), q_mem.data_ptr())
-        plan.q_next = None
-        plan.q_next_ready = False
+        _take_arenas(plan, p_mem, q_mem)
         if plan.is_wide and plan.wide is None:
             from ._psgd_wide import WideRound
             plan.wide = WideRound(work, plan.ps, plan.qs, device)
@@ -429,8 +446,10 @@ def _run_round(state, bucket, error_mode, streams=1):
             if cnt not in errs:
                 errs[cnt] = DenseCS(m, n, state.sketch_size, device=device)
 
-    # the errors this round adds to may still be being sparsified on the side stream
+    # the errors this round adds to may still be being sparsified on the side stream, and the Q factors
+    # it writes may still be being read there
     wait_for_side_topk(plan, device, lambda: _lib.current_stream(device))
+    wait_for_side_q(plan, device, lambda: _lib.current_stream(device))
     eps = float(state.orthogonalization_epsilon)
     if plan.ws_need is None:
         plan.ws_need = plan.wide.ws_need if plan.is_wide else max(
@@ -527,8 +546,6 @@ def _run_round(state, bucket, error_mode, streams=1):
             plan.made = [ctypes.c_int32(0) for _ in plan.chunks]
             plan.q_next_ready = False
         aside = state.matrix_approximation_rank > 8 and streams <= 1
-        if aside and plan.q_next_ready:
-            _pools.side_wait(device, _lib.current_stream(device), plan.q_next_number)
         flags = (1 if plan.q_next_ready else 0) | (0 if aside else 2) | 4
         for (first, part), q_next, made in zip(plan.chunks, plan.q_next_ptrs, plan.made):
             rc = lib.conef_psgd_round_ahead_f32(_at(items, first), part, mode1, mode3, float(alpha), beta3, eps, HASH_A, HASH_B,
@@ -601,7 +618,12 @@ def _orthogonalise_q_aside(plan, lib, items, eps, ws_len, device):
     side.wait_event(plan.handoff_event)
     if plan.q_next_event is None:
         plan.q_next_event = torch.cuda.Event()
-        plan.q_next.record_stream(side)       # memory the side stream works on must not go back to the allocator under it
+    if plan.aside_recorded != side.cuda_stream:
+        # memory the side stream works on must not go back to the allocator under it: the second buffer it
+        # writes and the arena it reads, each time either is a new one (all of plan.qs is one allocation)
+        plan.q_next.record_stream(side)
+        plan.qs[0].record_stream(side)
+        plan.aside_recorded = side.cuda_stream
     with _lib.on_stream(side):
         ws = _workspace(device, side.cuda_stream, max(ws_len, 256))
     for (first, part), q_next, made in zip(plan.chunks, plan.q_next_ptrs, plan.made):

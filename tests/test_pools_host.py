@@ -111,3 +111,57 @@ def test_a_stale_topk_table_is_told_from_a_current_one():
     assert not engine.topk_table_is_stale(table, tensors, 0.4)
     assert engine.topk_table_is_stale(table, tensors, 0.3)                         # another ratio
     assert engine.topk_table_is_stale(table, [tensors[0], torch.zeros(9)], 0.4)    # an error tensor was replaced
+
+
+class FakeBuffer:
+    def __init__(self):
+        self.recorded_on = []
+
+    def record_stream(self, stream):
+        self.recorded_on.append(stream)
+
+
+class FakeEvent:
+    def record(self, stream):
+        pass
+
+
+def test_every_buffer_the_side_stream_works_on_is_known_to_the_allocator(monkeypatch):
+    """The Gram-Schmidt of a bucket's next Q factors reads the Q arena and writes a second buffer on the
+    side stream.  Both are replaced when a caller drops the P / Q memory of a bucket, and the new ones
+    have to be recorded on the side stream like the first ones were."""
+    from contextlib import nullcontext
+    from types import SimpleNamespace
+
+    from conef_amd import _lib, _psgd_engine as engine
+
+    device, main, side = torch.device("cpu"), FakeStream(31), FakeStream(32)
+    monkeypatch.setattr(torch.cuda, "Event", FakeEvent)
+    monkeypatch.setattr(_lib, "current_stream", lambda dev: main)
+    monkeypatch.setattr(_lib, "on_stream", lambda stream: nullcontext())
+    monkeypatch.setattr(_pools, "side_stream", lambda dev, index, count: side)
+    monkeypatch.setattr(engine, "_workspace", lambda dev, stream, nbytes: torch.zeros(8))
+    lib = SimpleNamespace(conef_psgd_q_next_f32=lambda *a: 0)
+    _pools._SIDE_ORDER.pop(device, None)
+    try:
+        state = SimpleNamespace(round_cache={}, matrix_approximation_rank=12, min_compression_rate=2)
+        plan = engine._build_round(state, [torch.zeros(64, 96)], [(64, 96)], ("key",), None)
+        plan.q_next_ptrs, plan.made = [None], [SimpleNamespace(value=1)]
+        monkeypatch.setattr(engine.ctypes, "byref", lambda *a: None)
+
+        def hand_over():
+            engine._orthogonalise_q_aside(plan, lib, plan.items, 0.0, 256, device)
+
+        for _ in range(2):           # the second time: a caller dropped the bucket's arenas, a round took new ones
+            engine._take_arenas(plan, torch.zeros(64 * 12), torch.zeros(96 * 12))
+            assert plan.q_next is None and not plan.q_next_ready
+            plan.q_next, plan.qs = FakeBuffer(), [FakeBuffer()]
+            hand_over()
+            hand_over()
+            assert plan.q_next.recorded_on == [side] and plan.qs[0].recorded_on == [side]       # once is enough
+        # and the round that follows waits for that work whether or not its result is used
+        plan.q_next_ready = False
+        engine.wait_for_side_q(plan, device, lambda: main)
+        assert len(main.waited_for) == 1 and plan.q_next_number is None
+    finally:
+        _pools._SIDE_ORDER.pop(device, None)
