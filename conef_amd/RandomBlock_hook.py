@@ -15,6 +15,7 @@ import torch
 import torch.distributed as dist
 
 from . import _bucket
+from . import _host
 from . import _lib
 from . import _pools
 from ._checkpoint import Checkpointable
@@ -111,13 +112,13 @@ class _BucketTable:
     """What a bucket's step needs, worked out once: the >= 2-D gradients as matrices, their block
     sizes, payload slices and the item table the batch entry point reads.  Rebuilt when the
     bucket's buffer or layout changes."""
-    __slots__ = ("key", "sig", "matrices", "uncompressed", "numels", "blocks", "offsets", "items", "count", "starts",
-                 "errors", "sketches", "moving", "need")
+    __slots__ = ("key", "layout", "matrices", "uncompressed", "numels", "blocks", "offsets", "items", "count", "starts",
+                 "places", "staying", "plans", "moving", "need")
 
 
 def _build_table(state, grads, key, device, bucket_index, errors):
     t = _BucketTable()
-    t.key, t.sig = key, _bucket.layout_signature(grads)
+    t.key, t.layout = key, _bucket.layout(grads)
     t.matrices = [g.view(g.shape[0], -1) for g in grads if g.ndimension() > 1]
     t.uncompressed = [g for g in grads if g.ndimension() <= 1]
     t.numels = np.array([m.numel() for m in t.matrices], dtype=np.int64)
@@ -142,50 +143,48 @@ def _build_table(state, grads, key, device, bucket_index, errors):
         it.n, it.m, it.block = matrix.shape[0], matrix.shape[1], block
         t.offsets.append(idx)
         idx += block
-    t.errors, t.sketches = None, []
+    t.places = None
     return t
 
 
 def _point_at_errors(state, t, errors):
     """The error memory's places in the item table.  ``t.moving``: the sketches that are not updated in
     place and swap two buffers, whose places a step takes anew; the others stay where they are."""
-    t.errors = list(errors)
-    t.moving, t.need = [], 0
-    t.sketches = []
-    for cnt, error in enumerate(errors[:t.count]):
-        it = t.items[cnt]
+    t.moving, t.need, t.plans, staying = [], 0, [], []
+    for it, error in zip(t.items, errors[:t.count]):
         if not state.use_error_compression:
             it.err = error.data_ptr()
+            staying.append(error)
             continue
         plan = error.plan()
+        t.plans.append((error, plan))
         it.w = error.range
         it.plan_host, it.plan_dev = (plan.host_ptr, plan.device.data_ptr()) if plan is not None else (None, None)
         it.staging = None
         if plan is not None and plan.in_place:
             it.cs_in = it.cs_out = error.cs.data_ptr()
+            staying.append(error)
         else:
             t.moving.append((it, error, plan))
             # One staging buffer serves every binned sketch of the bucket (the launches run one after the
             # other on the stream): it is sized for the largest of them
             if plan is not None:
                 t.need = max(t.need, plan.workspace_bytes)
-    if state.use_error_compression:
-        moving = {id(error) for _, error, _ in t.moving}
-        t.sketches = [(error, error._plan, None if id(error) in moving else error.cs) for error in errors[:t.count]]
+    t.staying = staying if state.use_error_compression else None
+    t.places = _host.Places(staying)
 
 
 def _errors_moved(t, errors):
-    """Whether a bucket's error memory is no longer what the table points at: other objects, a sketch whose
-    cells or plan were replaced."""
-    if t.errors is None or len(errors) != len(t.errors):
+    """Whether a bucket's error memory is no longer where the table points: another tensor, the same one
+    over other storage, another sketch, a sketch whose cells or plan were replaced."""
+    if t.places is None:
         return True
-    for error, known in zip(errors, t.errors):
-        if error is not known:
+    if t.staying is None:                    # dense errors
+        return not t.places.same(errors if len(errors) == t.count else errors[:t.count])
+    for error, (known, plan) in zip(errors, t.plans):
+        if error is not known or error.plan() is not plan:
             return True
-    for error, plan, cells in t.sketches:
-        if error._plan is not plan or (cells is not None and error.cs is not cells):
-            return True
-    return False
+    return not t.places.same(t.staying)
 
 
 def RandomBlock_hook(state: RandomBlockState, bucket) -> torch.futures.Future[torch.Tensor]:
@@ -213,7 +212,7 @@ def RandomBlock_hook(state: RandomBlockState, bucket) -> torch.futures.Future[to
     key = (input_tensor.data_ptr(), input_tensor.numel(), bool(state.use_error_compression), state.compression_ratio,
            payload_all.data_ptr() if payload_all is not None else 0)
     table = state.round_cache.get(bucket_index)
-    if table is None or table.key != key or table.sig != _bucket.layout_signature(grads) or len(errors) < table.count:
+    if table is None or table.key != key or not table.layout.same(grads) or len(errors) < table.count:
         table = _build_table(state, grads, key, device, bucket_index, errors)
         payload_all = state.compressed_tensor_memory[bucket_index]
         table.key = key[:4] + (payload_all.data_ptr(),)

@@ -78,12 +78,11 @@ def UnbiasedRandomBlock_hook(state: UnbiasedRandomBlockState, bucket) -> torch.f
     bucket_index = _bucket.index(bucket)
 
     grads = _bucket.gradients(bucket)
-    sig = _bucket.layout_signature(grads)
     payload_all = state.compressed_tensor_memory.get(bucket_index)
     key = (input_tensor.data_ptr(), input_tensor.numel(), state.compression_ratio,
            payload_all.data_ptr() if payload_all is not None else 0)
     table = state.round_cache.get(bucket_index)
-    if table is None or table[0] != key or table[1] != sig:
+    if table is None or table[0] != key or not table[1].same(grads):
         # worked out once per bucket: the >= 2-D gradients, their block sizes and the item table
         tensors = [g for g in grads if g.ndimension() > 1]
         uncompressed = [g for g in grads if g.ndimension() <= 1]
@@ -99,7 +98,7 @@ def UnbiasedRandomBlock_hook(state: UnbiasedRandomBlockState, bucket) -> torch.f
             it.n, it.m, it.block = tensor.shape[0], numel // tensor.shape[0], block     # prob = block / numel is formed in the library (:155)
             offsets.append(idx)
             idx += block
-        table = (key[:3] + (payload_all.data_ptr(),), sig, tensors, uncompressed, np.array(numels, dtype=np.int64), blocks, offsets,
+        table = (key[:3] + (payload_all.data_ptr(),), _bucket.layout(grads), tensors, uncompressed, np.array(numels, dtype=np.int64), blocks, offsets,
                  items, _lib.randblock_starts(items, len(tensors)))
         state.round_cache[bucket_index] = table
     _, _, tensors, uncompressed, numels, blocks, offsets, items, starts = table

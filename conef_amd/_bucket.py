@@ -5,34 +5,30 @@ communication/powerSGD_hook.py:343,386,355,244), and a completed Future."""
 import torch
 import torch.distributed as dist
 
-
-def _call(bucket, new, old):
-    fn = getattr(bucket, new, None)
-    if fn is None:
-        fn = getattr(bucket, old)
-    return fn()
+from . import _host
 
 
 def buffer(bucket):
-    return _call(bucket, "buffer", "get_tensor")
+    return (getattr(bucket, "buffer", None) or bucket.get_tensor)()
 
 
 def gradients(bucket):
-    return _call(bucket, "gradients", "get_per_parameter_tensors")
+    return (getattr(bucket, "gradients", None) or bucket.get_per_parameter_tensors)()
 
 
 def index(bucket):
-    return _call(bucket, "index", "get_index")
+    return (getattr(bucket, "index", None) or bucket.get_index)()
 
 
 def is_last(bucket):
-    return _call(bucket, "is_last", "is_the_last_bucket_to_allreduce")
+    return (getattr(bucket, "is_last", None) or bucket.is_the_last_bucket_to_allreduce)()
 
 
-def layout_signature(grads):
-    """What a step compares instead of every tensor's shape: a bucket keeps its buffer, its length
-    (both part of what is cached for it) and its parameters for as long as DDP keeps the bucket."""
-    return (len(grads), grads[0].shape, grads[-1].shape) if grads else (0, None, None)
+def layout(grads):
+    """What a step compares (``.same(grads)``) to see that a bucket still has the tensors its cached tables
+    were made for: the shape of every one, in order.  The buffer's place and length go into the cache keys
+    beside it."""
+    return _host.Shapes(grads)
 
 
 def draw_starts(rng, numels, items, starts):

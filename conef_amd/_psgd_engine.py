@@ -14,7 +14,7 @@ import os
 import torch
 import torch.distributed as dist
 
-from . import _bucket, _lib, _pools
+from . import _bucket, _host, _lib, _pools
 from .compressors.CountSketch import HASH_A, HASH_B, DenseCS
 
 
@@ -125,13 +125,10 @@ class _RoundPlan:
     compressed, the table of matrices the batch entry points read, the views into the P / Q
     arenas.  Built on the first step of a bucket and reused while the bucket keeps its buffer
     and layout, so that a step costs a handful of foreign calls however many tensors it has."""
-    __slots__ = ("small", "sig", "errs_sig", "cs_static", "env_ahead", "env_topk_side", "env_small", "key", "shapes", "work", "passthrough", "before", "after", "total_ps", "total_qs", "arena_key", "ps",
+    __slots__ = ("small", "layout", "errs_known", "cells", "cs_static", "env_ahead", "env_topk_side", "env_small", "key", "shapes", "work", "passthrough", "before", "after", "total_ps", "total_qs", "arena_key", "ps",
                  "qs", "items", "count", "sketches", "fused_sketch", "batched_update", "residual_offsets",
                  "topk_table", "q_next", "q_next_ptrs", "q_next_ready", "made", "q_next_event", "aside_recorded",
                  "topk_event", "ws_need", "handoff_event", "topk_number", "q_next_number", "is_wide", "wide", "chunks", "ef_spans")
-
-
-_layout_signature = _bucket.layout_signature
 
 
 BATCH_ITEMS = 24        # matrices the batch entry points take into one launch
@@ -169,8 +166,9 @@ def _rank_bound(rank):
 def _build_round(state, grads, shapes, key, error_mode):
     plan = _RoundPlan()
     plan.key, plan.shapes = key, shapes
-    plan.sig = _layout_signature(grads)
-    plan.errs_sig = None
+    plan.layout = _bucket.layout(grads)
+    plan.errs_known = None          # the bucket's sketches, and where their cells were, when the table was pointed at them
+    plan.cells = None
     plan.cs_static = False
     # switches read when the plan is built (a bucket's plan lives as long as its buffer does)
     plan.env_ahead = os.environ.get("CONEF_ROUND_AHEAD", "1") != "0"
@@ -230,6 +228,18 @@ def _build_round(state, grads, shapes, key, error_mode):
     return plan
 
 
+def _sketches_moved(plan, errs):
+    """Whether the bucket's sketches are others than the table points at, or the same ones with their cells
+    elsewhere (sketches that swap two buffers are pointed at anew every step anyway)."""
+    known = plan.errs_known
+    if known is None or len(known) != len(errs):
+        return True
+    for cs, now in zip(known, errs.values()):
+        if cs is not now:
+            return True
+    return plan.cs_static and not plan.cells.same(known)
+
+
 def _take_arenas(plan, p_mem, q_mem):
     """Points the table of matrices at the bucket's P and Q arenas.  What belonged to the arenas before -
     the second buffer of the Q factors, what the allocator was told about either - goes with them."""
@@ -262,7 +272,7 @@ def plan_for(state, bucket_index, grads, key, error_mode, device, stream_now):
     round is about to run on (``stream_now()``) is ordered after a pending copy of the Q arena
     here, since the new plan no longer knows of it."""
     plan = state.round_cache.get(bucket_index)
-    if plan is None or plan.key != key or plan.sig != _layout_signature(grads):
+    if plan is None or plan.key != key or not plan.layout.same(grads):
         old = plan
         plan = _build_round(state, grads, [t.shape for t in grads], key, error_mode)
         if old is not None:
@@ -380,7 +390,9 @@ def _run_round(state, bucket, error_mode, streams=1):
     grads = _bucket.gradients(bucket)
     key = (base_ptr, total_length, error_mode, state.matrix_approximation_rank, state.min_compression_rate,
            getattr(state, "sketch_size", None), dense_err.data_ptr() if dense_err is not None else 0)
-    plan = plan_for(state, bucket_index, grads, key, error_mode, device, lambda: _lib.current_stream(device))
+    plan = state.round_cache.get(bucket_index)
+    if plan is None or plan.key != key or not plan.layout.same(grads):
+        plan = plan_for(state, bucket_index, grads, key, error_mode, device, lambda: _lib.current_stream(device))
     work, items, count = plan.work, plan.items, plan.count
     state.total_numel_before_compression += plan.before
     state.total_numel_after_compression += plan.after
@@ -416,9 +428,7 @@ def _run_round(state, bucket, error_mode, streams=1):
                 errs[cnt] = torch.zeros_like(matrix)
             items[cnt].err = errs[cnt].data_ptr()
     elif error_mode == "conef":
-        # (the dict of a bucket's sketches is only ever replaced as a whole, with the round cache cleared:
-        # load_state_dict; its identity and size stand for its entries)
-        if plan.errs_sig != (id(errs), len(errs)) or len(plan.sketches) != count:
+        if _sketches_moved(plan, errs):
             plan.sketches = []
             for cnt, (matrix, n, m, rank) in enumerate(work):
                 if cnt not in errs:
@@ -432,10 +442,11 @@ def _run_round(state, bucket, error_mode, streams=1):
             plan.batched_update = all(p is not None and p.batchable for _, p in plan.sketches)
             plan.fused_sketch = state.matrix_approximation_rank <= 8 and plan.batched_update
             plan.small = None
-            plan.errs_sig = (id(errs), len(errs))
-            # sketches on row lists are updated in place: their cells never move.  The others swap
-            # two buffers, so their pointers are refreshed every step.
+            # sketches on row lists are updated in place.  The others swap two buffers, so their pointers
+            # are refreshed every step.
             plan.cs_static = all(p is not None and p.in_place for _, p in plan.sketches)
+            plan.errs_known = list(errs.values())
+            plan.cells = _host.Places(plan.errs_known)
             for cnt, (cs, _) in enumerate(plan.sketches):
                 items[cnt].cs = cs.cs.data_ptr()
         if not plan.cs_static:
@@ -448,8 +459,10 @@ def _run_round(state, bucket, error_mode, streams=1):
 
     # the errors this round adds to may still be being sparsified on the side stream, and the Q factors
     # it writes may still be being read there
-    wait_for_side_topk(plan, device, lambda: _lib.current_stream(device))
-    wait_for_side_q(plan, device, lambda: _lib.current_stream(device))
+    if plan.topk_number is not None:
+        wait_for_side_topk(plan, device, lambda: _lib.current_stream(device))
+    if plan.q_next_number is not None:
+        wait_for_side_q(plan, device, lambda: _lib.current_stream(device))
     eps = float(state.orthogonalization_epsilon)
     if plan.ws_need is None:
         plan.ws_need = plan.wide.ws_need if plan.is_wide else max(

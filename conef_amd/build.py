@@ -1,4 +1,5 @@
-"""Compiles the HIP kernels into conef_amd/lib/libconef_hip.so (gfx950 only).
+"""Compiles the HIP kernels into conef_amd/lib/libconef_hip.so (gfx950 only), and the host helpers
+into conef_amd/lib/libconef_host.so.
 
 hipcc cross-compiles without a GPU, so this runs anywhere the ROCm toolchain is installed.
 The library is built in-tree; nothing is JIT-compiled at run time.
@@ -33,6 +34,26 @@ HIPCC_FLAGS = [
 ]
 
 
+# checks on Python lists of tensors (host only, against torch's own libraries)
+HOST_SOURCE, HOST_LIBPATH = "conef_host.cpp", os.path.join(LIBDIR, "libconef_host.so")
+
+
+def _build_host(verbose):
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    cxx = os.environ.get("CXX") or shutil.which("g++") or "c++"
+    includes = [f for path in cpp_extension.include_paths() + [sysconfig.get_paths()["include"]] for f in ("-isystem", path)]
+    cmd = [cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI]
+    cmd += includes + [os.path.join(CSRC, HOST_SOURCE), "-o", HOST_LIBPATH, "-L" + cpp_extension.TORCH_LIB_PATH, "-ltorch_python", "-lc10"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("%s failed on %s:\n%s\n%s" % (cxx, HOST_SOURCE, res.stdout, res.stderr))
+
+
 def _hipcc():
     for cand in (os.environ.get("HIPCC"), shutil.which("hipcc"), "/opt/rocm/bin/hipcc"):
         if cand and os.path.exists(cand):
@@ -61,8 +82,11 @@ def build(verbose=False, trace=False):
             print(res.stderr, file=sys.stderr)
         return obj
 
-    with ThreadPoolExecutor(max_workers=min(6, len(sources))) as pool:
+    with ThreadPoolExecutor(max_workers=min(6, len(sources)) + 1) as pool:
+        host = pool.submit(_build_host, verbose) if not trace else None
         objs = list(pool.map(compile_one, sources))
+        if host is not None:
+            host.result()
     cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", libpath] + objs
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:

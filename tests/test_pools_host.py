@@ -165,3 +165,94 @@ def test_every_buffer_the_side_stream_works_on_is_known_to_the_allocator(monkeyp
         assert len(main.waited_for) == 1 and plan.q_next_number is None
     finally:
         _pools._SIDE_ORDER.pop(device, None)
+
+
+def _views(flat, shapes):
+    out, off = [], 0
+    for shape in shapes:
+        n = int(torch.Size(shape).numel())
+        out.append(flat[off: off + n].view(shape))
+        off += n
+    return out
+
+
+def test_a_bucket_of_other_tensors_over_the_same_buffer_is_another_bucket():
+    """Same buffer, same count, same first and last tensor, another order in between: the tables a hook
+    keeps for the bucket point at other spans."""
+    from types import SimpleNamespace
+
+    from conef_amd import _bucket, _psgd_engine as engine
+
+    flat = torch.zeros(4 * 8 + 6 * 4 + 3 + 2 * 2)
+    one = _views(flat, [(4, 8), (6, 4), (3,), (2, 2)])
+    other = _views(flat, [(4, 8), (3,), (6, 4), (2, 2)])
+    layout = _bucket.layout(one)
+    assert layout.same(_views(flat, [(4, 8), (6, 4), (3,), (2, 2)])) and layout.same(tuple(one))
+    for shapes in ([(4, 8), (4, 6), (3,), (2, 2)], [(4, 8), (24,), (3,), (2, 2)], [(4, 8), (6, 4), (3,)],
+                   [(4, 8), (6, 4), (3,), (2, 2), ()], [(4, 8), (6, 4), (3, 1), (2, 2)], []):
+        assert not layout.same(_views(torch.zeros(100), shapes)), shapes
+    assert not layout.same(other) and not layout.same([1, 2, 3, 4]) and not layout.same(None)
+    assert _bucket.layout([]).same([]) and _bucket.layout([torch.zeros(())]).same([torch.ones(())])
+    state = SimpleNamespace(round_cache={}, matrix_approximation_rank=1, min_compression_rate=0.1)
+    main, device = FakeStream(41), torch.device("cpu")
+    plan = engine.plan_for(state, 0, one, ("buffer",), None, device, lambda: main)
+    assert engine.plan_for(state, 0, _views(flat, [(4, 8), (6, 4), (3,), (2, 2)]), ("buffer",), None, device, lambda: main) is plan
+    assert engine.plan_for(state, 0, other, ("buffer",), None, device, lambda: main) is not plan
+
+
+def test_random_block_errors_are_found_where_they_are_now():
+    """A dense error tensor that a caller gave other storage (``.data =``, ``set_``), a sketch whose cells
+    were replaced in the object: the step has to follow, whatever the objects' identity says."""
+    from types import SimpleNamespace
+
+    from conef_amd import RandomBlock_hook as rb, _lib
+
+    def table(count):
+        return SimpleNamespace(items=(_lib.RandBlockItem * count)(), count=count, places=None)
+
+    state = SimpleNamespace(use_error_compression=False)
+    errors = [torch.zeros(3, 4), torch.zeros(5, 2)]
+    t = table(2)
+    assert rb._errors_moved(t, errors)
+    rb._point_at_errors(state, t, errors)
+    assert not rb._errors_moved(t, errors)
+    errors[1].data = torch.ones(5, 2)
+    assert rb._errors_moved(t, errors)
+    rb._point_at_errors(state, t, errors)
+    assert not rb._errors_moved(t, errors) and t.items[1].err == errors[1].data_ptr()
+    errors[0].set_(torch.ones(3, 4))
+    assert rb._errors_moved(t, errors)
+
+    state.use_error_compression = True
+    plan = SimpleNamespace(in_place=True, host_ptr=16, device=torch.zeros(4), workspace_bytes=0)
+    sketches = [SimpleNamespace(cs=torch.zeros(3, 4), range=4, plan=lambda: plan) for _ in range(2)]
+    t = table(2)
+    rb._point_at_errors(state, t, sketches)
+    assert not rb._errors_moved(t, sketches)
+    sketches[1].cs.data = torch.ones(3, 4)
+    assert rb._errors_moved(t, sketches)
+    rb._point_at_errors(state, t, sketches)
+    assert not rb._errors_moved(t, sketches) and t.items[1].cs_in == sketches[1].cs.data_ptr()
+    sketches[0].plan = lambda: None              # other hash seeds, say: the plan is another one
+    assert rb._errors_moved(t, sketches)
+
+
+def test_powersgd_sketches_are_found_where_they_are_now():
+    from types import SimpleNamespace
+
+    from conef_amd import _host, _psgd_engine as engine
+
+    sketches = [SimpleNamespace(cs=torch.zeros(3, 4)) for _ in range(2)]
+    plan = SimpleNamespace(cells=None, errs_known=None, cs_static=True)
+    errs = dict(enumerate(sketches))
+    assert engine._sketches_moved(plan, errs)
+    plan.errs_known, plan.cells = sketches, _host.Places(sketches)
+    assert not engine._sketches_moved(plan, errs) and not engine._sketches_moved(plan, dict(errs))
+    assert engine._sketches_moved(plan, {})                                   # dropped by the caller
+    assert engine._sketches_moved(plan, {0: sketches[0], 1: SimpleNamespace(cs=sketches[1].cs)})
+    sketches[1].cs.data = torch.ones(3, 4)
+    assert engine._sketches_moved(plan, errs)
+    sketches[1].cs = None                        # whatever is found there: the table is built anew, and says so
+    assert engine._sketches_moved(plan, errs)
+    plan.cs_static = False                       # pointed at anew every step
+    assert not engine._sketches_moved(plan, errs)
