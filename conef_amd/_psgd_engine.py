@@ -127,9 +127,12 @@ class _RoundPlan:
     and layout, so that a step costs a handful of foreign calls however many tensors it has."""
     __slots__ = ("small", "layout", "errs_known", "cells", "cs_static", "env_ahead", "env_topk_side", "env_small", "key", "shapes", "work", "passthrough", "before", "after", "total_ps", "total_qs", "arena_key", "ps",
                  "qs", "items", "count", "sketches", "fused_sketch", "batched_update", "residual_offsets",
-                 "topk_table", "q_next", "q_next_ptrs", "q_next_ready", "made", "q_next_event", "aside_recorded",
+                 "topk_table", "q_next", "q_next_ptrs", "q_next_ready", "q_next_quads", "made", "q_next_event", "aside_recorded",
                  "topk_event", "ws_need", "handoff_event", "topk_number", "q_next_number", "is_wide", "wide", "chunks", "ef_spans")
 
+
+# flags of conef_psgd_round_ahead_f32 (include/conef_hip.h)
+_ROUND_Q_READY, _ROUND_MAKE_NEXT, _ROUND_NEXT_QUADS, _ROUND_NEXT_WIDE, _ROUND_QUADS_READY = 1, 2, 4, 8, 16
 
 BATCH_ITEMS = 24        # matrices the batch entry points take into one launch
 
@@ -213,7 +216,7 @@ def _build_round(state, grads, shapes, key, error_mode):
     # round (conef_psgd_round_ahead_f32).  Derived data: q_memory_dict keeps what the reference
     # keeps, and the flag falls with the plan whenever the state is replaced.
     plan.q_next = plan.q_next_ptrs = None
-    plan.q_next_ready = False
+    plan.q_next_ready = plan.q_next_quads = False
     plan.made = None
     plan.q_next_event = None
     plan.aside_recorded = None      # the side stream (raw) that q_next and the Q arena are known to the allocator to be used on
@@ -559,12 +562,15 @@ def _run_round(state, bucket, error_mode, streams=1):
             plan.made = [ctypes.c_int32(0) for _ in plan.chunks]
             plan.q_next_ready = False
         aside = state.matrix_approximation_rank > 8 and streams <= 1
-        flags = (1 if plan.q_next_ready else 0) | (0 if aside else 2) | 4
+        flags = _ROUND_NEXT_QUADS | _ROUND_NEXT_WIDE | (0 if aside else _ROUND_MAKE_NEXT)
+        if plan.q_next_ready:
+            flags |= _ROUND_Q_READY | (_ROUND_QUADS_READY if plan.q_next_quads else 0)
         for (first, part), q_next, made in zip(plan.chunks, plan.q_next_ptrs, plan.made):
             rc = lib.conef_psgd_round_ahead_f32(_at(items, first), part, mode1, mode3, float(alpha), beta3, eps, HASH_A, HASH_B,
                                                 q_next, flags, ctypes.byref(made), ws_ptr, ws_len, stream)
             _lib.check(rc, "conef_psgd_round_ahead_f32")
         plan.q_next_ready = all(made.value for made in plan.made)
+        plan.q_next_quads = all(made.value & 2 for made in plan.made)
         if aside:
             _orthogonalise_q_aside(plan, lib, items, eps, ws_len, device)
     else:
@@ -646,6 +652,7 @@ def _orthogonalise_q_aside(plan, lib, items, eps, ws_len, device):
     plan.q_next_event.record(side)
     plan.q_next_number = _pools.side_recorded(device, plan.q_next_event)
     plan.q_next_ready = all(made.value for made in plan.made)
+    plan.q_next_quads = False
 
 
 def run_batched_round(state, bucket):

@@ -3175,31 +3175,34 @@ inline bool padded_round(const ConefPsgdItem* items, int count, int mq_mode, voi
     return mqs_plan_launch(table.data(), count, pr->rp, mq_mode == 2, &T, &S, &lds, true);
 }
 
-// dst[row] = src[row] and zeros behind it, rows of r and RP floats
-struct PadRowsItem {
+// dst[row] = src[row], cut or with zeros behind it: factors between rows of r floats (a caller's) and of
+// rank_bound(r) (the library's own)
+struct RowsItem {
     const float* src;
     float* dst;
     int64_t rows;
+    int from, to;            // floats in a row of src, of dst
 };
 
 __global__ void __launch_bounds__(256)
-psgd_pad_rows_batch_kernel(PsgdBatch<PadRowsItem> b, int r, int rp)
+psgd_rows_batch_kernel(PsgdBatch<RowsItem> b)
 {
     int local;
-    const PadRowsItem& it = b.item[psgd_batch_locate(b, &local)];
+    const RowsItem& it = b.item[psgd_batch_locate(b, &local)];
     const int64_t e = (int64_t)local * 256 + threadIdx.x;
-    if (e >= it.rows * rp) return;
-    const int64_t row = e / rp;
-    const int c = (int)(e - row * rp);
-    it.dst[e] = c < r ? it.src[row * r + c] : 0.f;
+    if (e >= it.rows * it.to) return;
+    const int64_t row = e / it.to;
+    const int c = (int)(e - row * it.to);
+    it.dst[e] = c < it.from ? it.src[row * it.from + c] : 0.f;
 }
 
-int pad_rows(const std::vector<PadRowsItem>& table, int r, int rp, hipStream_t s)
+int copy_rows(const std::vector<RowsItem>& table, hipStream_t s)
 {
+    if (table.empty()) return CONEF_OK;
     std::vector<int> blocks;
-    for (const PadRowsItem& t : table) blocks.push_back((int)((t.rows * rp + 255) / 256));
-    return run_batches(table, blocks, [&](const PsgdBatch<PadRowsItem>& bt, int grid) {
-        hipLaunchKernelGGL(psgd_pad_rows_batch_kernel, dim3((unsigned)grid), dim3(256), 0, s, bt, r, rp);
+    for (const RowsItem& t : table) blocks.push_back((int)((t.rows * t.to + 255) / 256));
+    return run_batches(table, blocks, [&](const PsgdBatch<RowsItem>& bt, int grid) {
+        hipLaunchKernelGGL(psgd_rows_batch_kernel, dim3((unsigned)grid), dim3(256), 0, s, bt);
     });
 }
 
@@ -3663,13 +3666,12 @@ int round_products(const ConefPsgdItem* items, const ConefPsgdItem* its, int cou
     if (!(defer_env && defer_env[0] == '0') && padded_round(items, count, mq_mode, workspace, workspace_bytes, &pr)) {
         const int r = items[0].r;
         std::vector<float*> q_in;
-        std::vector<PadRowsItem> pad;
+        std::vector<RowsItem> pad;
         for (int k = 0; k < count; ++k) {
             q_in.push_back(pr.padded ? pr.items[(size_t)k].q : its[k].q);
-            if (pr.padded) pad.push_back(PadRowsItem{its[k].q, pr.items[(size_t)k].q, its[k].m});
+            if (pr.padded) pad.push_back(RowsItem{its[k].q, pr.items[(size_t)k].q, its[k].m, r, pr.rp});
         }
-        if (pr.padded)
-            if (int rc = pad_rows(pad, r, pr.rp, s); rc != CONEF_OK) return rc;
+        if (int rc = copy_rows(pad, s); rc != CONEF_OK) return rc;
         return deferred_products(pr, r, q_in.data(), nullptr, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, s, nullptr);
     }
     int rc = conef_psgd_mq_batch_f32(its, count, mq_mode, alpha, a, b, workspace, workspace_bytes, (void*)s);
@@ -3794,7 +3796,7 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
 {
     if (made) *made = 0;
     if (count < 0 || (count > 0 && !items) || pqt_mode < 0 || pqt_mode > 3) return CONEF_ERR_INVALID;
-    if ((flags & (CONEF_ROUND_Q_READY | CONEF_ROUND_MAKE_NEXT)) && (!q_next || !made)) return CONEF_ERR_INVALID;
+    if ((flags & (CONEF_ROUND_Q_READY | CONEF_ROUND_MAKE_NEXT | CONEF_ROUND_QUADS_READY)) && (!q_next || !made)) return CONEF_ERR_INVALID;
     if (count == 0) return CONEF_OK;
     std::vector<float*> mats((size_t)count);
     std::vector<int64_t> rows((size_t)count);
@@ -3814,6 +3816,7 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
         if (mq_mode == 2 && it.plan_host && !conef_plan_matches((const ConefPlanHeader*)it.plan_host, it.n, it.m, it.w, a, b))
             return CONEF_ERR_INVALID;
         if ((flags & CONEF_ROUND_Q_READY) && !q_next[k]) return CONEF_ERR_INVALID;
+        if ((flags & CONEF_ROUND_QUADS_READY) && !q_next[count + k]) return CONEF_ERR_INVALID;
     }
     hipStream_t hs = (hipStream_t)stream;
     GsAhead ahead;
@@ -3822,9 +3825,14 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
         ahead.parts[k] = nullptr;
         ahead.nparts[k] = 0;
     }
-    // the next round's Q factors are wanted in q_next
-    const bool by_quads = (flags & CONEF_ROUND_NEXT_QUADS) != 0;      // q_next[count + k]: the same by quads
-    bool want_next = (flags & CONEF_ROUND_MAKE_NEXT) && count <= kPsgdBatchMax;
+    // The next round's Q factors are wanted in q_next.  What lies there is a matter of the flags alone, never of
+    // the way a round happens to run (deferred or not can change between two rounds, with the mode, the
+    // workspace or the environment): rows of rank_bound(r) floats under NEXT_WIDE, of r floats without.
+    const bool ready = (flags & CONEF_ROUND_Q_READY) != 0;
+    const bool wide = (flags & CONEF_ROUND_NEXT_WIDE) != 0;
+    const bool by_quads = (flags & CONEF_ROUND_NEXT_QUADS) != 0;      // q_next[count + k]: room for the same by quads
+    const bool quads_ready = ready && (flags & CONEF_ROUND_QUADS_READY) != 0;
+    bool want_next = (flags & CONEF_ROUND_MAKE_NEXT) && count <= kPsgdBatchMax && (wide || items[0].r <= 8);
     for (int k = 0; k < count && want_next; ++k) want_next = q_next[k] && items[k].r == items[0].r && items[k].m <= 0x7fffffffLL;
     const int rp = rank_bound(items[0].r);
     // P = X Q, P orthogonalised, Q = X^T P: with the orthogonalisation deferred where the batch
@@ -3841,18 +3849,19 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
         // bucket's last round), else Q orthogonalised now
         const int r = items[0].r;
         std::vector<float*> q_in((size_t)count);
-        for (int k = 0; k < count; ++k) q_in[(size_t)k] = (flags & CONEF_ROUND_Q_READY) ? q_next[k] : pr.items[(size_t)k].q;
-        if (!(flags & CONEF_ROUND_Q_READY)) {
-            if (rp <= 8) {
-                rc = conef_gram_schmidt_batch_f32(mats.data(), rows.data(), ranks.data(), count, eps, workspace, workspace_bytes, stream);
-                if (rc != CONEF_OK) return rc;
-            }
-            if (pr.padded) {
-                std::vector<PadRowsItem> pad;
-                for (int k = 0; k < count; ++k) pad.push_back(PadRowsItem{items[k].q, pr.items[(size_t)k].q, items[k].m});
-                rc = pad_rows(pad, r, rp, hs);
-                if (rc != CONEF_OK) return rc;
-            }
+        std::vector<RowsItem> pad;
+        for (int k = 0; k < count; ++k) {
+            float* own = pr.items[(size_t)k].q;      // a copy of the library's own where pr.padded
+            q_in[(size_t)k] = ready && (wide || !pr.padded) ? q_next[k] : own;
+            if (pr.padded && !(ready && wide)) pad.push_back(RowsItem{ready ? q_next[k] : items[k].q, own, items[k].m, r, rp});
+        }
+        if (!ready && rp <= 8) {
+            rc = conef_gram_schmidt_batch_f32(mats.data(), rows.data(), ranks.data(), count, eps, workspace, workspace_bytes, stream);
+            if (rc != CONEF_OK) return rc;
+        }
+        rc = copy_rows(pad, hs);
+        if (rc != CONEF_OK) return rc;
+        if (!ready) {
             if (rp > 8) {      // in place: a workgroup of the last launch reads its rows before it writes them
                 std::vector<const float*> src;
                 for (int k = 0; k < count; ++k) src.push_back(pr.items[(size_t)k].q);
@@ -3861,12 +3870,21 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
             }
         }
         GsAhead* qs = want_next && rp <= 8 ? &ahead : nullptr;
-        rc = deferred_products(pr, r, q_in.data(), by_quads && (flags & CONEF_ROUND_Q_READY) ? q_next + count : nullptr, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, hs, qs);
+        rc = deferred_products(pr, r, q_in.data(), quads_ready ? q_next + count : nullptr, mq_mode, alpha, eps, a, b, workspace,
+                               workspace_bytes, hs, qs);
         if (rc != CONEF_OK) return rc;
     } else {
         std::vector<ConefPsgdItem> first(items, items + count);
-        if (flags & CONEF_ROUND_Q_READY) {
-            for (int k = 0; k < count; ++k) first[(size_t)k].q = q_next[k];
+        if (ready) {
+            // (a factor of wide rows into Q itself, which the next product overwrites)
+            std::vector<RowsItem> cut;
+            for (int k = 0; k < count; ++k) {
+                const int bound = rank_bound(items[k].r);
+                if (wide && bound != items[k].r) cut.push_back(RowsItem{q_next[k], items[k].q, items[k].m, bound, items[k].r});
+                else first[(size_t)k].q = q_next[k];
+            }
+            rc = copy_rows(cut, hs);
+            if (rc != CONEF_OK) return rc;
         } else {
             rc = conef_gram_schmidt_batch_f32(mats.data(), rows.data(), ranks.data(), count, eps, workspace, workspace_bytes, stream);
             if (rc != CONEF_OK) return rc;
@@ -3877,18 +3895,19 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
     // The new Q factors orthogonalised into q_next, ranks up to 8: by workgroups of the last launch,
     // where that launch covers the whole bucket; from the shares of Q^T Q when the products above left
     // them, else by the column steps themselves, which takes a short Q factor.
+    const bool by_shares = deferred && (wide || !pr.padded);
     if (want_next && rp <= 8 && pqt_mode <= 2) {
-        bool ok = true;
-        for (int k = 0; k < count && ok && !deferred; ++k)
+        bool ok = by_shares || !wide || items[0].r == rp;           // the column steps leave rows of r floats
+        for (int k = 0; k < count && ok && !by_shares; ++k)
             ok = gs_reg_class(items[k].q, items[k].m, items[k].r) >= 0 &&
                  items[k].m <= (int64_t)kGsAheadRowSlots * kGsRegThreads;
         if (ok) {
             for (int k = 0; k < count; ++k) {
-                ahead.src[k] = its[k].q;
+                ahead.src[k] = by_shares ? its[k].q : items[k].q;
                 ahead.dst[k] = q_next[k];
                 ahead.rows[k] = (int)items[k].m;
-                ahead.quads[k] = deferred && by_quads ? q_next[count + k] : nullptr;
-                if (!deferred) ahead.parts[k] = nullptr;
+                ahead.quads[k] = by_shares && by_quads ? q_next[count + k] : nullptr;
+                if (!by_shares) ahead.parts[k] = nullptr;
             }
             ahead.count = count;
             ahead.r = items[0].r;
@@ -3906,7 +3925,7 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
         if (rc != CONEF_OK) return rc;
         used = true;
     }
-    if (made) *made = used ? 1 : 0;
+    if (made) *made = !used ? 0 : by_shares && by_quads && rp <= 8 ? 3 : 1;
     if (pqt_mode == 3) rc = conef_psgd_sketch_update_batch_f32(items, count, beta, a, b, stream);
     return rc;
 }
@@ -3925,13 +3944,12 @@ int conef_psgd_q_next_f32(const ConefPsgdItem* items, int32_t count, float eps, 
         return CONEF_OK;
     hipStream_t s = (hipStream_t)stream;
     std::vector<const float*> src;
-    std::vector<PadRowsItem> pad;
+    std::vector<RowsItem> pad;
     for (int k = 0; k < count; ++k) {
         src.push_back(pr.padded ? q_next[k] : items[k].q);
-        pad.push_back(PadRowsItem{items[k].q, q_next[k], items[k].m});
+        if (pr.padded) pad.push_back(RowsItem{items[k].q, q_next[k], items[k].m, items[0].r, pr.rp});
     }
-    if (pr.padded)
-        if (int rc = pad_rows(pad, items[0].r, pr.rp, s); rc != CONEF_OK) return rc;
+    if (int rc = copy_rows(pad, s); rc != CONEF_OK) return rc;
     const int rc = orthogonalise_by_gram_wide(pr, items[0].r, src, q_next, eps, workspace, s);
     if (rc == CONEF_OK) *made = 1;
     return rc;

@@ -381,17 +381,25 @@ int conef_psgd_products_f32(const ConefPsgdItem* items, const ConefPsgdItem* fir
 /* The same round for callers that keep a second buffer per Q factor.  The reference orthogonalises a
  * bucket's Q factors at the start of the bucket's next round (powerSGD_hook.py:496-497), a few short
  * launches with the machine idle around them.  Here flags & CONEF_ROUND_MAKE_NEXT asks for that to be
- * done at the end of this round instead, out of place into q_next; *made tells whether it was (a bucket
- * of at most 24 matrices of one rank).  items[k].q keeps what the reference keeps there.  In the next
- * round flags & CONEF_ROUND_Q_READY says q_next holds the orthogonal Q factors: the first step is left
- * out and P = M Q reads them.  q_next[k] belongs to the library between the two calls: m rows of as many
- * floats as the next of 1, 2, 4, 8, 16 and 32 that is not below the rank.  No counterpart in the reference's
- * interface. */
+ * done at the end of this round instead, out of place into q_next; *made tells whether it was (0: no, and
+ * q_next is untouched; not 0: yes).  items[k].q keeps what the reference keeps there.  In the next round
+ * flags & CONEF_ROUND_Q_READY says q_next holds the orthogonal Q factors: the first step is left out and
+ * P = M Q reads them.  No counterpart in the reference's interface.
+ *
+ * q_next[k] is [m, r] like items[k].q, and CONEF_ROUND_MAKE_NEXT serves buckets of at most 24 matrices of
+ * one rank up to 8, at ranks 3, 5, 6 and 7 with Q factors of at most 1024 rows.
+ * CONEF_ROUND_NEXT_WIDE, in both rounds, changes that: a row of q_next[k] takes as many floats as the
+ * next of 1, 2, 4, 8, 16 and 32 that is not below the rank, the library's own layout, and ranks up to 32
+ * and Q factors of any height are served.  The flags alone decide the layout, in whichever way
+ * either round runs. */
 #define CONEF_ROUND_Q_READY 1
 #define CONEF_ROUND_MAKE_NEXT 2
-/* q_next has 2 * count entries: q_next[count + k] is a second buffer of 16 * ceil(m / 4) times that many
- * bytes, in which the library keeps the same factor in the order its kernels load it (ranks up to 8). */
+/* q_next has 2 * count entries: q_next[count + k] is a further buffer of 16 * ceil(m / 4) times that many
+ * bytes, for the same factor in the order the library's kernels load it (ranks up to 8).  Whether that
+ * was filled as well is in *made & 2; the next round is told so by CONEF_ROUND_QUADS_READY. */
 #define CONEF_ROUND_NEXT_QUADS 4
+#define CONEF_ROUND_NEXT_WIDE 8
+#define CONEF_ROUND_QUADS_READY 16
 int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_t mq_mode, int32_t pqt_mode, float alpha,
                                float beta, float eps, int32_t a, int32_t b, float* const* q_next, int32_t flags,
                                int32_t* made, void* workspace, int64_t workspace_bytes, void* stream);

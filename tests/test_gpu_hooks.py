@@ -1019,6 +1019,92 @@ def test_q_factors_orthogonalised_by_the_last_launch(monkeypatch, oracle, rank, 
             same(x, z)
 
 
+def _two_rounds(oracle, monkeypatch, rank, flags, defer, quads=False):
+    """Two rounds over the same two matrices through conef_psgd_round_ahead_f32, the second starting from
+    what the first left in q_next where it says so.  Each q_next[k] is followed by a stretch of sentinels.
+    Returns (*made of the first round, [q_next buffer, rows asked for, orthogonal Q the oracle makes], results)."""
+    from conef_amd import _lib
+    lib = _lib.load()
+    specs = [(512, 300, rank), (96, 1000, rank)]
+    bound = 1 << (rank - 1).bit_length()
+    row = bound if flags & 8 else rank
+    rs = np.random.RandomState(21)
+    items, keep, nexts = (_lib.PsgdItem * 2)(), [], []
+    for it, (n, m, r) in zip(items, specs):
+        M = torch.from_numpy(rs.randn(n, m).astype(np.float32)).cuda()
+        Q = torch.from_numpy(rs.randn(m, r).astype(np.float32)).cuda()
+        P = torch.empty(n, r, device="cuda")
+        it.x, it.p, it.q, it.n, it.m, it.r, it.w = M.data_ptr(), P.data_ptr(), Q.data_ptr(), n, m, r, 1
+        keep.append((M, P, Q, M.clone()))
+        nexts.append(torch.full((m * bound + 64,), 7.0, device="cuda"))
+    quad_bufs = [torch.full((4 * (-(-m // 4)) * bound,), 7.0, device="cuda") for _, m, _ in specs]
+    ptrs = (ctypes.c_void_p * 4)(*[t.data_ptr() for t in nexts + quad_bufs])
+    ws = torch.empty(lib.conef_psgd_batch_workspace_bytes(items, 2), dtype=torch.uint8, device="cuda")
+    stream, made = torch.cuda.current_stream().cuda_stream, ctypes.c_int32(-1)
+
+    def go(f):
+        rc = lib.conef_psgd_round_ahead_f32(items, 2, 0, 0, 0.0, 0.0, 0.0, 1, 1, ptrs, f, ctypes.byref(made), ws.data_ptr(),
+                                            ws.numel(), stream)
+        assert rc == 0
+        return made.value
+
+    monkeypatch.setenv("CONEF_ROUND_DEFER", defer[0])
+    first = go(flags | 2)
+    torch.cuda.synchronize()
+    want = []
+    for (M, P, Q, M0), (n, m, r) in zip(keep, specs):
+        q = to_np(Q).copy()
+        oracle.gram_schmidt(q, 0.0)
+        want.append(q)
+        M.copy_(M0)
+        M.mul_(1.5)                                    # another gradient
+    made_rows = [(to_np(t).copy(), row) for t in nexts]
+    monkeypatch.setenv("CONEF_ROUND_DEFER", defer[1])
+    go(flags | (1 if first else 0) | (16 if first & 2 and quads else 0))
+    torch.cuda.synchronize()
+    return first, made_rows, want, keep, specs
+
+
+@pytest.mark.parametrize("rank", [1, 3, 5, 6, 7, 8, 12, 16])
+@pytest.mark.parametrize("defer", ["11", "00"])
+def test_a_second_buffer_of_tight_rows_stays_within_them(monkeypatch, oracle, rank, defer):
+    """Without CONEF_ROUND_NEXT_WIDE a second buffer is [m, rank]: nothing behind it is written, whatever
+    the rank, and above rank 8 nothing at all."""
+    made, rows, want, keep, specs = _two_rounds(oracle, monkeypatch, rank, 0, defer)
+    assert (made & 1) == (rank <= 8)
+    for (buf, row), q, (n, m, r) in zip(rows, want, specs):
+        assert row == rank
+        used = m * rank if made else 0
+        assert (buf[used:] == 7.0).all()
+        if made:
+            assert_close(buf[:used].reshape(m, r), q, what="orthogonal Q, rank %d" % rank)
+
+
+@pytest.mark.parametrize("rank", [3, 4, 6, 8, 12, 16])
+@pytest.mark.parametrize("defer", ["11", "10", "01", "00"])
+@pytest.mark.parametrize("wide", [0, 8, 12])
+def test_what_a_round_leaves_for_the_next_does_not_depend_on_how_either_runs(monkeypatch, oracle, rank, defer, wide):
+    """The order of steps inside a round (deferred or the reference's) can change between the round that
+    makes the next Q factors and the one that reads them: the layout of q_next is what the flags say, and
+    the second round agrees with the oracle's either way.  1e-4: the second round's input has been through
+    one fp32 orthogonalisation here and one in the oracle, whose roundings its products carry on."""
+    made, rows, want, keep, specs = _two_rounds(oracle, monkeypatch, rank, wide, defer, quads=wide == 12)
+    if wide and made:
+        bound = 1 << (rank - 1).bit_length()
+        for (buf, row), q, (n, m, r) in zip(rows, want, specs):
+            got = buf[:m * bound].reshape(m, bound)
+            assert_close(got[:, :r], q, what="orthogonal Q, rank %d" % rank)
+            assert (got[:, r:] == 0).all() and (buf[m * bound:] == 7.0).all()
+    for (M, P, Q, M0), q0, (n, m, r) in zip(keep, want, specs):
+        X = 1.5 * to_np(M0)
+        p = oracle.mq(X, q0)
+        oracle.gram_schmidt(p, 0.0)
+        q = oracle.mtp(X, p)
+        assert_close(P, p, rel=1e-4, what="P of the second round")
+        assert_close(Q, q, rel=1e-4, what="Q of the second round")
+        assert_close(M, oracle.pqt(p, q), rel=1e-4, what="M of the second round")
+
+
 @pytest.mark.parametrize("rank,mode", [(32, "conef"), (16, "ef"), (12, "plain")])
 def test_high_rank_rounds_orthogonalise_q_on_a_side_stream(monkeypatch, rank, mode):
     """Above rank 8 the new Q factors of a bucket are orthogonalised for its next round on a side stream
