@@ -85,6 +85,8 @@ SIGNATURES = {
     "conef_topk_workspace_bytes": [_I64],
     "conef_topk_sparsify_f32": [_P, _I64, _I64, _P, _I64, _P],
     "conef_topk_batch_workspace_bytes": [_P, _I32],
+    "conef_topk_batch_list_bytes": [_P, _I32],
+    "conef_topk_sparsify_batch_listed_f32": [_P, _P, _P, _I32, _P, _I64, _P, _I64, _P],
     "conef_topk_sparsify_batch_f32": [_P, _P, _P, _I32, _P, _I64, _P],
     "conef_topk_sparsify_batch_kept_f32": [_P, _P, _P, _I32, _P, _I64, _P],
     "conef_topk_sparsify_noalloc_f32": [_P, _I64, _I64, _P],
@@ -111,7 +113,7 @@ def randblock_starts(items, count):
                       strides=(ctypes.sizeof(RandBlockItem),))
 
 
-_RETURNS_I64 = ("conef_topk_workspace_bytes", "conef_topk_batch_workspace_bytes", "conef_plan_bytes",
+_RETURNS_I64 = ("conef_topk_workspace_bytes", "conef_topk_batch_workspace_bytes", "conef_topk_batch_list_bytes", "conef_plan_bytes",
                 "conef_plan_workspace_bytes", "conef_psgd_workspace_bytes", "conef_psgd_batch_workspace_bytes",
                 "conef_psgd_round_small_workspace_bytes")
 

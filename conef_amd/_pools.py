@@ -15,6 +15,7 @@ runtime later in the process's life registers its own exit handlers (handlers ru
 first-out), so device memory held here is returned while the runtime is still intact.
 """
 import atexit
+import contextlib
 import threading
 
 import torch
@@ -44,10 +45,11 @@ def plan(key, build):
     return hit
 
 
-def _grown(pool, key, numel, dtype, device):
+def _grown(pool, key, numel, dtype, device, on=None):
     buf = pool.get(key)
     if buf is None or buf.numel() < numel:
-        buf = torch.empty(max(int(numel), 64), dtype=dtype, device=device)
+        with contextlib.nullcontext() if on is None else torch.cuda.stream(on):
+            buf = torch.empty(max(int(numel), 64), dtype=dtype, device=device)
         pool[key] = buf
     return buf
 
@@ -57,10 +59,12 @@ def staging(device, stream, nbytes):
     return _grown(_STAGING, (device, stream), nbytes, torch.uint8, device)
 
 
-def workspace(device, stream, nbytes):
-    """Device scratch for sums that cross workgroups: one buffer per (device, stream), grown on
-    demand.  Kernels that use it are ordered by that stream."""
-    return _grown(_WORKSPACES, (device, stream), max(nbytes, 256), torch.uint8, device)
+def workspace(device, stream, nbytes, on=None):
+    """Device scratch that is live inside one call (sums that cross workgroups, lists of candidates): one
+    buffer per (device, stream), grown on demand.  Kernels that use it are ordered by that stream.
+    ``on``: that stream as a torch Stream where it is not the current one, so that the allocator knows
+    whose memory it is."""
+    return _grown(_WORKSPACES, (device, stream), max(nbytes, 256), torch.uint8, device, on)
 
 
 def scratch_f32(device, stream, numel):

@@ -7,6 +7,7 @@ those stages in the reference are the identity at world size 1.  Here each matri
 streaming passes over its memory: the error add is fused into the first product, the residual
 (dense, or count-sketched) into the last.
 """
+import contextlib
 import ctypes
 import logging
 import os
@@ -91,32 +92,42 @@ def topk_sparsify(err, topk_ratio, workspace=None):
     return workspace
 
 
-def topk_sparsify_all(tensors, topk_ratio, table=None, stream=None):
+class _TopkTable(tuple):
+    """(tensors' places, pointers, element counts, how many stay, selection state, ratio)"""
+    list_bytes = 0
+
+
+def topk_sparsify_all(tensors, topk_ratio, table=None, side=None):
     """``topk_sparsify`` of every tensor of a list (one stream, one device) with each pass a
     single launch over all of them.  ``table`` is what an earlier call over the same tensors
-    returned: the host arrays and the workspace are reused while the tensors stay where they are.
-    ``stream``: the raw stream to launch on (torch's current one if None)."""
+    returned: the host arrays and the selection state are reused while the tensors stay where they are.
+    ``side``: the torch Stream to launch on (the current one if None)."""
     count = len(tensors)
     if count == 0:
         return table
     key = tuple(t.data_ptr() for t in tensors)
     lib = _lib.load()
+    device = tensors[0].device
     if table is None or table[0] != key:
         for t in tensors:
             _lib.require_device_f32(t, "err")
         ptrs = (ctypes.c_void_p * count)(*key)
         numels = (ctypes.c_int64 * count)(*[t.numel() for t in tensors])
         ks = (ctypes.c_int64 * count)(*[max(1, int(0.5 * topk_ratio * t.numel())) for t in tensors])
-        # zero-filled once: the table keeps this workspace with these tensors, and the passes clear the
-        # selection state behind themselves (conef_topk_sparsify_batch_kept_f32)
-        ws = torch.zeros(lib.conef_topk_batch_workspace_bytes(numels, count), dtype=torch.uint8, device=tensors[0].device)
-        table = (key, ptrs, numels, ks, ws, topk_ratio)
+        # zero-filled once, on the stream whose kernels rely on the zeros: the table keeps this state with
+        # these tensors, and the passes clear it behind themselves (conef_topk_sparsify_batch_listed_f32)
+        with contextlib.nullcontext() if side is None else _lib.on_stream(side):
+            ws = torch.zeros(lib.conef_topk_batch_workspace_bytes(numels, count), dtype=torch.uint8, device=device)
+        table = _TopkTable((key, ptrs, numels, ks, ws, topk_ratio))
+        table.list_bytes = lib.conef_topk_batch_list_bytes(numels, count)
     elif table[5] != topk_ratio:
-        return topk_sparsify_all(tensors, topk_ratio, None, stream)
+        return topk_sparsify_all(tensors, topk_ratio, None, side)
     _, ptrs, numels, ks, ws, _ = table
-    rc = lib.conef_topk_sparsify_batch_kept_f32(ptrs, numels, ks, count, ws.data_ptr(), ws.numel(),
-                                                _lib.stream_ptr(tensors[0]) if stream is None else stream)
-    _lib.check(rc, "conef_topk_sparsify_batch_kept_f32")
+    stream = _lib.stream_ptr(tensors[0]) if side is None else side.cuda_stream
+    lists = _workspace(device, stream, table.list_bytes, side)
+    rc = lib.conef_topk_sparsify_batch_listed_f32(ptrs, numels, ks, count, ws.data_ptr(), ws.numel(), lists.data_ptr(),
+                                                  lists.numel(), stream)
+    _lib.check(rc, "conef_topk_sparsify_batch_listed_f32")
     return table
 
 
@@ -128,7 +139,7 @@ class _RoundPlan:
     __slots__ = ("small", "layout", "errs_known", "cells", "cs_static", "env_ahead", "env_topk_side", "env_small", "key", "shapes", "work", "passthrough", "before", "after", "total_ps", "total_qs", "arena_key", "ps",
                  "qs", "items", "count", "sketches", "fused_sketch", "batched_update", "residual_offsets",
                  "topk_table", "q_next", "q_next_ptrs", "q_next_ready", "q_next_quads", "made", "q_next_event", "aside_recorded",
-                 "topk_event", "ws_need", "handoff_event", "topk_number", "q_next_number", "is_wide", "wide", "chunks", "ef_spans")
+                 "topk_event", "topk_recorded", "ws_need", "handoff_event", "topk_number", "q_next_number", "is_wide", "wide", "chunks", "ef_spans")
 
 
 # flags of conef_psgd_round_ahead_f32 (include/conef_hip.h)
@@ -208,6 +219,7 @@ def _build_round(state, grads, shapes, key, error_mode):
     plan.batched_update = False
     plan.topk_table = None
     plan.topk_event = None          # the side stream's top-k of this bucket's errors, to be waited for by its next round
+    plan.topk_recorded = None       # the side stream (raw) that the errors are known to the allocator to be used on
     plan.topk_number = None         # the side stream's running number of that top-k (None: nothing to wait for)
     plan.q_next_number = None       # likewise for the Gram-Schmidt of the next round's Q factors
     plan.ws_need = None             # bytes of workspace the batch entry points ask for (a function of the table's shapes)
@@ -582,25 +594,23 @@ def _run_round(state, bucket, error_mode, streams=1):
     if error_mode == "topk":
         if count and streams <= 1 and plan.env_ahead and plan.env_topk_side:
             # The sparsification only touches the error tensors, which nobody reads before this bucket's
-            # next round: it runs on a side stream while this stream goes on with the next bucket (five
-            # streaming passes next to launches that are mostly latency).  Same kernels, same values.
+            # next round: it runs on a side stream while this stream goes on with the next bucket
+            # (streaming passes next to launches that are mostly latency).  Same kernels, same values.
             if plan.handoff_event is None:
                 plan.handoff_event = torch.cuda.Event()
             plan.handoff_event.record(_lib.current_stream(device))
             side = _pools.side_stream(device, 0, 1)
             side.wait_event(plan.handoff_event)
             tensors = [errs[cnt] for cnt in range(count)]
-            # a table that no longer fits (an error tensor was replaced, another ratio) is a new one: its
-            # workspace has to be allocated and zero-filled on the stream whose kernels rely on the zeros
-            if topk_table_is_stale(plan.topk_table, tensors, state.topk_ratio):
-                with _lib.on_stream(side):
-                    plan.topk_table = topk_sparsify_all(tensors, state.topk_ratio, None)
-                # memory the side stream works on must not go back to the allocator under it
+            if topk_table_is_stale(plan.topk_table, tensors, state.topk_ratio) or plan.topk_recorded != side.cuda_stream:
+                # a new table (an error tensor was replaced, another ratio), another stream: memory the side
+                # stream works on must not go back to the allocator under it
+                plan.topk_table = topk_sparsify_all(tensors, state.topk_ratio, None, side)
                 for t in tensors:
                     t.record_stream(side)
-                plan.topk_table[4].record_stream(side)
+                plan.topk_recorded = side.cuda_stream
             else:
-                plan.topk_table = topk_sparsify_all(tensors, state.topk_ratio, plan.topk_table, side.cuda_stream)
+                plan.topk_table = topk_sparsify_all(tensors, state.topk_ratio, plan.topk_table, side)
             if plan.topk_event is None:
                 plan.topk_event = torch.cuda.Event()
             plan.topk_event.record(side)

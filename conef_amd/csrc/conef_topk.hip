@@ -37,7 +37,8 @@ struct TopkState {
     uint32_t ties[kPasses];         // keys that match prefix[p] exactly in their high digits
     uint32_t done;                  // workgroups of the filter that have finished (surplus ties only)
     uint32_t tie_count;             // indices recorded in tie_idx so far
-    uint32_t pad[4];
+    uint32_t final_count;           // keys gathered in final_idx so far (selection through a candidate list)
+    uint32_t pad[3];
     uint32_t hist[kPasses][kBins];
     uint32_t tie_idx[kTieMax];      // where the keys equal to the threshold sit, in no order
 };
@@ -83,6 +84,7 @@ __device__ __forceinline__ void topk_init_body(TopkState* st, uint32_t k)
         st->k = k;
         st->done = 0u;
         st->tie_count = 0u;
+        st->final_count = 0u;
     }
 }
 
@@ -155,7 +157,7 @@ __device__ __forceinline__ void topk_resolve(TopkState* st, int p, uint32_t* pre
 // wave that meet in a bin then add to different LDS banks instead of queueing on one address.
 // `kept` (a state that stays with its tensor from call to call, zero-filled before the first): no
 // launch clears the state; the first workgroup of pass 0 clears what the later passes count into,
-// and pass 2's clears what pass 0 of the next call counts into (topk_settle_body).
+// and the filter's, or the settling pass's, clears what pass 0 of the next call counts into.
 template <int REP>
 __device__ __forceinline__ void
 topk_hist_body(const float* __restrict__ x, int64_t numel, TopkState* st, int pass, int bx, int gx, bool kept = false,
@@ -170,6 +172,7 @@ topk_hist_body(const float* __restrict__ x, int64_t numel, TopkState* st, int pa
             st->k = k;
             st->done = 0u;
             st->tie_count = 0u;
+            st->final_count = 0u;
         }
     }
     const int nb = 1 << kDigitBits[pass];
@@ -277,14 +280,42 @@ __device__ __forceinline__ void topk_order_ties(float* __restrict__ x, int64_t n
     }
 }
 
-// keep key >= threshold, zero the rest, settle surplus ties on the threshold by index
-__device__ __forceinline__ void
-topk_filter_body(float* __restrict__ x, int64_t numel, TopkState* st, int bx, int gx)
+// Surplus ties on the threshold (`held` keys equal it, `keep_ties` of them stay): every workgroup comes here
+// when it is through with its own share, up to kTieMax ties noted in tie_idx; the last one settles them.
+__device__ __forceinline__ void topk_settle_ties(float* __restrict__ x, int64_t numel, TopkState* st, uint32_t thr,
+                                                 uint32_t keep_ties, uint32_t held, int gx)
 {
     __shared__ uint32_t ticket;
-    __shared__ uint32_t idx_l[kTieMax];
+    __shared__ uint32_t tie_l[kTieMax];
+    __syncthreads();
+    if (threadIdx.x == 0) ticket = atomicAdd(&st->done, 1u);
+    __syncthreads();
+    if (ticket != (uint32_t)gx - 1u) return;
+    __threadfence();
+    if (held > (uint32_t)kTieMax) {
+        topk_order_ties(x, numel, thr, keep_ties);
+        return;
+    }
+    const int n = (int)held;
+    for (int j = threadIdx.x; j < n; j += blockDim.x)
+        tie_l[j] = __hip_atomic_load(&st->tie_idx[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    for (int j = threadIdx.x; j < n; j += blockDim.x) {
+        const uint32_t mine = tie_l[j];
+        uint32_t rank = 0;
+        for (int t = 0; t < n; ++t) rank += tie_l[t] < mine;
+        if (rank >= keep_ties) x[mine] = 0.f;
+    }
+}
+
+// keep key >= threshold, zero the rest, settle surplus ties on the threshold by index
+__device__ __forceinline__ void
+topk_filter_body(float* __restrict__ x, int64_t numel, TopkState* st, int bx, int gx, bool kept = false)
+{
     uint32_t thr, keep_ties, ties;
     topk_resolve(st, kPasses - 1, &thr, &keep_ties, &ties, bx);
+    if (kept && bx == 0)       // nobody reads the first digit's counters any more: ready for the next call
+        for (int i = threadIdx.x; i < kBins; i += 256) st->hist[0][i] = 0u;
     const bool surplus = ties != keep_ties && thr != 0u;      // a zero threshold has only zeros for ties
     const bool listed = surplus && ties <= (uint32_t)kTieMax;
     auto note = [&](int64_t i) {
@@ -332,25 +363,7 @@ topk_filter_body(float* __restrict__ x, int64_t numel, TopkState* st, int bx, in
     // (which rewrite a tie with its own value when a neighbour in the quad goes) can land after
     // the zeros it writes.
     __threadfence();
-    __syncthreads();
-    if (threadIdx.x == 0) ticket = atomicAdd(&st->done, 1u);
-    __syncthreads();
-    if (ticket != (uint32_t)gx - 1u) return;
-    __threadfence();
-    if (!listed) {
-        topk_order_ties(x, numel, thr, keep_ties);
-        return;
-    }
-    const int n = (int)ties;
-    for (int j = threadIdx.x; j < n; j += blockDim.x)
-        idx_l[j] = __hip_atomic_load(&st->tie_idx[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    for (int j = threadIdx.x; j < n; j += blockDim.x) {
-        const uint32_t mine = idx_l[j];
-        uint32_t rank = 0;
-        for (int t = 0; t < n; ++t) rank += idx_l[t] < mine;
-        if (rank >= keep_ties) x[mine] = 0.f;
-    }
+    topk_settle_ties(x, numel, st, thr, keep_ties, ties, gx);
 }
 
 __global__ void __launch_bounds__(256)
@@ -360,27 +373,31 @@ topk_filter_kernel(float* __restrict__ x, int64_t numel, TopkState* st)
 }
 
 __global__ void __launch_bounds__(256)
-topk_filter_batch_kernel(TopkBatch b)
+topk_filter_batch_kernel(TopkBatch b, bool kept)
 {
     int local, width;
     const TopkItem& it = b.item[topk_locate(b.first, b.count, &local, &width)];
-    topk_filter_body(it.x, it.numel, it.st, local, width);
+    topk_filter_body(it.x, it.numel, it.st, local, width, kept);
 }
 
 
 // ---- selection through a candidate list ----
 // Three histogram passes and the filter read a tensor four times.  After the first digit, though, only
 // the keys that share it with the threshold are undecided - about one in twenty of a gradient's error,
-// 11 bits being an exponent and three mantissa bits.  So, for a workspace that stays with its tensors:
+// 11 bits being an exponent and three mantissa bits.  So, for a caller that lends room for lists:
 //   pass 0     the first digit's histogram, as above;
 //   pass 1     zeroes what lies below the digit, counts the second digit of the keys that share it
 //              and notes them, (index, key), each workgroup in a segment of its own: no counter is shared;
-//   pass 2     goes over the notes alone: zeroes what lies below the first two digits and gathers the
-//              keys that share both (a few hundred); the workgroup that finishes last ranks those.
+//   pass 2     goes over the notes alone: zeroes what lies below the first two digits, counts the third of
+//              the keys that share both and, if they are no more than kTopkFinal, gathers them;
+//   pass 3     resolves the threshold and clears what lies below it: one workgroup over the gathered keys
+//              (a few hundred of a gradient's), else every workgroup over its own notes once more.
 // Two reads and one write of the tensor instead of four and one.  A workgroup whose segment runs over
-// (more than a quarter of its keys share the digit) goes over its elements again in pass 2; more than
-// kTopkFinal keys that share two digits (a tensor of repeated values) are settled by one workgroup
-// walking the tensor.
+// (more than a quarter of its keys share the digit) goes over its elements again instead of its notes.
+// Every step is spread over all workgroups however the magnitudes are distributed, but for more than
+// kTieMax keys equal to the threshold (as in the filter).  The keys that share two digits grow with the
+// tensor - 2e-5 of a Gaussian's, more than kTopkFinal from 100 M elements on - and are all of a tensor
+// whose magnitudes lie within 512 floats of each other.
 constexpr uint32_t kTopkOverflow = 0xffffffffu;
 constexpr int kTopkFinal = 2048;
 constexpr int kTopkTrip = 8;             // quads a thread requests together
@@ -492,103 +509,117 @@ __device__ __forceinline__ void topk_note_body(const TopkItem& it, int bx, int g
         if (bins[i]) atomicAdd(&st->hist[1][i], bins[i]);
 }
 
-// One workgroup: of the keys that share `prefix` (the first two digits) the `keep` largest stay, equal
-// ones in index order; the others are cleared.  each(f) calls f(index, key) for the keys.
 constexpr int kTopkLow = 1 << kDigitBits[2];
 
-template <typename Each>
-__device__ __forceinline__ void topk_last_digit(uint32_t (&bins)[kTopkLow], uint32_t prefix, uint32_t keep, Each each,
-                                                uint32_t* thr, uint32_t* ties, uint32_t* held)
+// f(index, key) for a workgroup's notes, or for its elements that share the digit where it has none
+template <typename F>
+__device__ __forceinline__ void topk_for_notes(const TopkItem& it, uint32_t digit, int bx, int gx, F f)
 {
-    for (int i = threadIdx.x; i < kTopkLow; i += 256) bins[i] = 0u;
-    __syncthreads();
-    each([&](uint32_t, uint32_t key) { atomicAdd(&bins[key & (kTopkLow - 1)], 1u); });
-    __syncthreads();
-    uint32_t cnt[8], digit;
-    for (int b = 0; b < kTopkLow / 256; ++b) cnt[b] = bins[threadIdx.x * (kTopkLow / 256) + b];
-    topk_pick(cnt, kTopkLow / 256, keep, &digit, ties, held);
-    *thr = (prefix << kDigitBits[2]) | digit;
+    const uint32_t n = it.counts[bx];
+    if (n == kTopkOverflow) {
+        topk_for_each(it.x, it.numel, bx, gx, [&](int64_t i, uint32_t key) {
+            if (key && (key >> kDigitShift[0]) == digit) f((uint32_t)i, key);
+        });
+        return;
+    }
+    const uint2* seg = it.list + (size_t)bx * it.cap;
+    for (uint32_t j0 = threadIdx.x; j0 < n; j0 += 4 * 256) {
+        uint2 c[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) c[u] = seg[j0 + u * 256 < n ? j0 + u * 256 : j0];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (j0 + u * 256 < n) f(c[u].x, c[u].y);
+    }
 }
 
-__device__ __forceinline__ void topk_settle_body(const TopkItem& it, int bx, int gx)
+// pass 2
+__device__ __forceinline__ void topk_gather_body(const TopkItem& it, int bx, int gx)
 {
-    __shared__ uint32_t ticket;
-    __shared__ uint32_t key_l[kTopkFinal], idx_l[kTopkFinal];
+    __shared__ uint32_t low[kTopkLow];
     TopkState* st = it.st;
     uint32_t prefix, keep, share;                        // `share` keys share both digits, `keep` of them stay
     topk_resolve(st, 1, &prefix, &keep, &share, bx);
     if (bx == 0)       // nobody reads the first digit's counters any more: ready for the next call
         for (int i = threadIdx.x; i < kBins; i += 256) st->hist[0][i] = 0u;
-    const uint32_t digit = prefix >> kDigitBits[1];
-    auto one = [&](uint32_t i, uint32_t key) {
+    for (int i = threadIdx.x; i < kTopkLow; i += 256) low[i] = 0u;
+    __syncthreads();
+    const bool undecided = keep < share, gathered = share <= (uint32_t)kTopkFinal;      // all of them stay otherwise
+    topk_for_notes(it, prefix >> kDigitBits[1], bx, gx, [&](uint32_t i, uint32_t key) {
         const uint32_t two = key >> kDigitBits[2];
         if (two < prefix) {
             it.x[i] = 0.f;
-        } else if (two == prefix && keep < share) {      // all of them stay otherwise
-            const uint32_t slot = atomicAdd(&st->tie_count, 1u);
-            if (slot < (uint32_t)kTopkFinal) {
-                __hip_atomic_store(it.final_idx + slot, i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(it.final_idx + kTopkFinal + slot, key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else if (two == prefix && undecided) {
+            atomicAdd(&low[key & (kTopkLow - 1)], 1u);
+            if (gathered) {
+                const uint32_t slot = atomicAdd(&st->final_count, 1u);      // below `share`
+                it.final_idx[slot] = i;
+                it.final_idx[kTopkFinal + slot] = key;
             }
         }
-    };
-    const uint32_t n = it.counts[bx];
-    if (n != kTopkOverflow) {
-        const uint2* seg = it.list + (size_t)bx * it.cap;
-        for (uint32_t j0 = threadIdx.x; j0 < n; j0 += 4 * 256) {
-            uint2 c[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) c[u] = seg[j0 + u * 256 < n ? j0 + u * 256 : j0];
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (j0 + u * 256 < n) one(c[u].x, c[u].y);
-        }
-    } else {
-        topk_for_each(it.x, it.numel, bx, gx, [&](int64_t i, uint32_t key) {
-            if (key && (key >> kDigitShift[0]) == digit) one((uint32_t)i, key);
-        });
+    });
+    if (!undecided) return;
+    __syncthreads();
+    for (int i = threadIdx.x; i < kTopkLow; i += 256)
+        if (low[i]) atomicAdd(&st->hist[2][i], low[i]);
+}
+
+// pass 3
+__device__ __forceinline__ void topk_settle_body(const TopkItem& it, int bx, int gx)
+{
+    __shared__ uint32_t key_l[kTopkFinal], idx_l[kTopkFinal];
+    __shared__ uint32_t total;
+    TopkState* st = it.st;
+    const uint32_t prefix = st->prefix[1], keep = st->remaining[1], share = st->ties[1];
+    const bool gathered = share <= (uint32_t)kTopkFinal;
+    if (keep >= share || (gathered && bx != 0)) return;
+    // the third digit's counts: of the keys but not of the zeros that may share both digits with them
+    uint32_t cnt[8], m = 0;
+    if (threadIdx.x == 0) total = 0u;
+    __syncthreads();
+    for (int b = 0; b < kTopkLow / 256; ++b) {
+        cnt[b] = st->hist[2][threadIdx.x * (kTopkLow / 256) + b];
+        m += cnt[b];
     }
-    if (keep >= share) return;
-    // The gathered keys went out past the caches (agent-scope stores): once they have arrived a plain count
-    // tells the last workgroup that it can see them all.  Nobody reads what anybody else clears.  (A
-    // fence here writes back whatever the caches hold, 10 to 30 us behind the passes before.)
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (m) atomicAdd(&total, m);
     __syncthreads();
-    if (threadIdx.x == 0) ticket = atomicAdd(&st->done, 1u);
-    __syncthreads();
-    if (ticket != (uint32_t)gx - 1u) return;
-    const uint32_t m = __hip_atomic_load(&st->tie_count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    m = total;
     if (m <= keep) return;                               // the rest of the share are zeros
-    __shared__ uint32_t low[kTopkLow];
-    uint32_t thr, ties, held;
-    if (m > (uint32_t)kTopkFinal) {
-        topk_last_digit(low, prefix, keep, [&](auto f) {
-            topk_for_each(it.x, it.numel, 0, 1, [&](int64_t i, uint32_t key) {
-                if (key && (key >> kDigitBits[2]) == prefix) f((uint32_t)i, key);
-            });
-        }, &thr, &ties, &held);
-        topk_for_each(it.x, it.numel, 0, 1, [&](int64_t i, uint32_t key) {
-            if (key < thr && (key >> kDigitBits[2]) == prefix) it.x[i] = 0.f;
-        });
-        if (ties < held) topk_order_ties(it.x, it.numel, thr, ties);
+    uint32_t low, ties, held;                            // `held` keys equal the threshold, `ties` of them stay
+    topk_pick(cnt, kTopkLow / 256, keep, &low, &ties, &held);
+    const uint32_t thr = (prefix << kDigitBits[2]) | low;
+    if (gathered) {
+        for (uint32_t j = threadIdx.x; j < m; j += 256) {
+            idx_l[j] = it.final_idx[j];
+            key_l[j] = it.final_idx[kTopkFinal + j];
+        }
+        __syncthreads();
+        for (uint32_t j = threadIdx.x; j < m; j += 256) {
+            const uint32_t key = key_l[j], idx = idx_l[j];
+            if (key > thr || (key == thr && ties == held)) continue;
+            uint32_t rank = 0;
+            if (key == thr)
+                for (uint32_t t = 0; t < m; ++t) rank += key_l[t] == key && idx_l[t] < idx;
+            if (key < thr || rank >= ties) it.x[idx] = 0.f;
+        }
         return;
     }
-    for (uint32_t j = threadIdx.x; j < m; j += 256) {
-        idx_l[j] = __hip_atomic_load(it.final_idx + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        key_l[j] = __hip_atomic_load(it.final_idx + kTopkFinal + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();
-    topk_last_digit(low, prefix, keep, [&](auto f) {
-        for (uint32_t j = threadIdx.x; j < m; j += 256) f(idx_l[j], key_l[j]);
-    }, &thr, &ties, &held);
-    for (uint32_t j = threadIdx.x; j < m; j += 256) {
-        const uint32_t key = key_l[j], idx = idx_l[j];
-        if (key > thr || (key == thr && ties == held)) continue;
-        uint32_t rank = 0;
-        if (key == thr)
-            for (uint32_t t = 0; t < m; ++t) rank += key_l[t] == key && idx_l[t] < idx;
-        if (key < thr || rank >= ties) it.x[idx] = 0.f;
-    }
+    const bool surplus = ties != held, listed = held <= (uint32_t)kTieMax;
+    topk_for_notes(it, prefix >> kDigitBits[1], bx, gx, [&](uint32_t i, uint32_t key) {
+        if ((key >> kDigitBits[2]) != prefix || key > thr) return;
+        if (key < thr) {
+            it.x[i] = 0.f;
+        } else if (surplus && listed) {
+            const uint32_t slot = atomicAdd(&st->tie_count, 1u);      // below `held`
+            __hip_atomic_store(&st->tie_idx[slot], i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    });
+    if (!surplus) return;
+    // The noted indices went out past the caches (agent-scope stores): once they have arrived a plain count
+    // tells the last workgroup that it can see them all.  A walk of its own reads only keys equal to the
+    // threshold, which nobody else writes.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    topk_settle_ties(it.x, it.numel, st, thr, ties, held, gx);
 }
 
 __global__ void __launch_bounds__(256)
@@ -597,6 +628,14 @@ topk_note_batch_kernel(TopkBatch b)
     int local, width;
     const TopkItem& it = b.item[topk_locate(b.first, b.count, &local, &width)];
     topk_note_body(it, local, width);
+}
+
+__global__ void __launch_bounds__(256)
+topk_gather_batch_kernel(TopkBatch b)
+{
+    int local, width;
+    const TopkItem& it = b.item[topk_locate(b.first, b.count, &local, &width)];
+    topk_gather_body(it, local, width);
 }
 
 __global__ void __launch_bounds__(256)
@@ -691,11 +730,11 @@ inline int64_t topk_segment(int64_t numel)
     return ((numel + g - 1) / g / 4 + 63) / 64 * 64;
 }
 
-// a tensor's part of a batch workspace: the state, the workgroups' counts, their segments
-inline int64_t topk_batch_item_bytes(int64_t numel)
+// a tensor's part of the lists: the gathered keys, the workgroups' counts, their segments
+inline int64_t topk_list_bytes(int64_t numel)
 {
     const int64_t g = topk_hist_groups(numel);
-    return (int64_t)kScratchBytes + 8 * kTopkFinal + (4 * g + 255) / 256 * 256 + g * topk_segment(numel) * 8;
+    return 8 * kTopkFinal + (4 * g + 255) / 256 * 256 + g * topk_segment(numel) * 8;
 }
 }  // namespace
 
@@ -708,14 +747,27 @@ int64_t conef_topk_batch_workspace_bytes(const int64_t* numels, int32_t count)
     int64_t total = 0;
     for (int i = 0; i < count; ++i) {
         if (numels[i] < 0) return -1;
-        total += topk_batch_item_bytes(numels[i]);
+        total += (int64_t)kScratchBytes;
+    }
+    return total > 256 ? total : 256;
+}
+
+int64_t conef_topk_batch_list_bytes(const int64_t* numels, int32_t count)
+{
+    if (count < 0 || (count > 0 && !numels)) return -1;
+    int64_t total = 0;
+    for (int i = 0; i < count; ++i) {
+        if (numels[i] < 0) return -1;
+        total += topk_list_bytes(numels[i]);
     }
     return total > 256 ? total : 256;
 }
 
 namespace {
+enum class TopkRun { kFresh, kKept, kListed };
+
 int topk_sparsify_batch(float* const* xs, const int64_t* numels, const int64_t* ks, int32_t count, void* workspace,
-                        int64_t workspace_bytes, void* stream, bool kept)
+                        int64_t workspace_bytes, void* lists, void* stream, TopkRun run)
 {
     if (count < 0 || (count > 0 && (!xs || !numels || !ks))) return CONEF_ERR_INVALID;
     for (int i = 0; i < count; ++i)
@@ -725,23 +777,27 @@ int topk_sparsify_batch(float* const* xs, const int64_t* numels, const int64_t* 
         return CONEF_ERR_INVALID;
     hipStream_t s = (hipStream_t)stream;
     char* ws = (char*)workspace;
+    char* room = (char*)lists;
     int i = 0;
     while (i < count) {
         TopkBatch b;
         int nb = 0, wgs = 0;
         for (; i < count && nb < kTopkBatchMax; ++i) {
             char* mine = ws;
-            ws += topk_batch_item_bytes(numels[i]);
+            ws += kScratchBytes;
             if (ks[i] >= numels[i]) continue;
             TopkItem& it = b.item[nb];
             it.x = xs[i];
             it.numel = numels[i];
             it.st = (TopkState*)mine;
             it.k = (uint32_t)ks[i];
-            it.cap = (uint32_t)topk_segment(numels[i]);
-            it.final_idx = (uint32_t*)(mine + kScratchBytes);
-            it.counts = it.final_idx + 2 * kTopkFinal;
-            it.list = (uint2*)(mine + kScratchBytes + 8 * kTopkFinal + (4 * topk_hist_groups(numels[i]) + 255) / 256 * 256);
+            if (run == TopkRun::kListed) {
+                it.cap = (uint32_t)topk_segment(numels[i]);
+                it.final_idx = (uint32_t*)room;
+                it.counts = it.final_idx + 2 * kTopkFinal;
+                it.list = (uint2*)(room + 8 * kTopkFinal + (4 * topk_hist_groups(numels[i]) + 255) / 256 * 256);
+                room += topk_list_bytes(numels[i]);
+            }
             b.first[nb] = wgs;
             wgs += (int)topk_hist_groups(numels[i]);
             ++nb;
@@ -750,16 +806,18 @@ int topk_sparsify_batch(float* const* xs, const int64_t* numels, const int64_t* 
         b.first[nb] = wgs;
         b.count = nb;
         const dim3 grid((unsigned)wgs), threads(256);
-        if (kept) {
+        if (run == TopkRun::kListed) {
             hipLaunchKernelGGL(topk_hist_batch_kernel, grid, threads, 0, s, b, 0, true);
             hipLaunchKernelGGL(topk_note_batch_kernel, grid, threads, 0, s, b);
+            hipLaunchKernelGGL(topk_gather_batch_kernel, grid, threads, 0, s, b);
             hipLaunchKernelGGL(topk_settle_batch_kernel, grid, threads, 0, s, b);
             continue;
         }
-        hipLaunchKernelGGL(topk_init_batch_kernel, dim3((unsigned)nb), threads, 0, s, b);
+        const bool kept = run == TopkRun::kKept;
+        if (!kept) hipLaunchKernelGGL(topk_init_batch_kernel, dim3((unsigned)nb), threads, 0, s, b);
         for (int pass = 0; pass < kPasses; ++pass)
-            hipLaunchKernelGGL(topk_hist_batch_kernel, grid, threads, 0, s, b, pass, false);
-        hipLaunchKernelGGL(topk_filter_batch_kernel, grid, threads, 0, s, b);
+            hipLaunchKernelGGL(topk_hist_batch_kernel, grid, threads, 0, s, b, pass, kept);
+        hipLaunchKernelGGL(topk_filter_batch_kernel, grid, threads, 0, s, b, kept);
     }
     return (int)hipGetLastError();
 }
@@ -768,17 +826,28 @@ int topk_sparsify_batch(float* const* xs, const int64_t* numels, const int64_t* 
 int conef_topk_sparsify_batch_f32(float* const* xs, const int64_t* numels, const int64_t* ks, int32_t count,
                                   void* workspace, int64_t workspace_bytes, void* stream)
 {
-    return topk_sparsify_batch(xs, numels, ks, count, workspace, workspace_bytes, stream, false);
+    return topk_sparsify_batch(xs, numels, ks, count, workspace, workspace_bytes, nullptr, stream, TopkRun::kFresh);
 }
 
 // The same for a workspace that stays with its tensors: zero-filled by the caller before its first
-// use and passed to nothing but this entry point, with the same xs / numels / count, afterwards.
-// No launch clears the selection state then (the passes clear behind themselves), and the selection goes
-// through a candidate list: three launches a call instead of five, two reads of a tensor instead of four.
+// use and passed to nothing but this entry point and the next, with the same xs / numels / count, afterwards.
+// No launch clears the selection state then (the passes clear behind themselves): four launches a
+// call instead of five.
 int conef_topk_sparsify_batch_kept_f32(float* const* xs, const int64_t* numels, const int64_t* ks, int32_t count,
                                        void* workspace, int64_t workspace_bytes, void* stream)
 {
-    return topk_sparsify_batch(xs, numels, ks, count, workspace, workspace_bytes, stream, true);
+    return topk_sparsify_batch(xs, numels, ks, count, workspace, workspace_bytes, nullptr, stream, TopkRun::kKept);
+}
+
+// The same again with room for candidate lists, which live inside the call only: two reads of a tensor
+// instead of four.
+int conef_topk_sparsify_batch_listed_f32(float* const* xs, const int64_t* numels, const int64_t* ks, int32_t count,
+                                         void* workspace, int64_t workspace_bytes, void* lists, int64_t list_bytes, void* stream)
+{
+    if (count > 0 && numels && (!lists || list_bytes < conef_topk_batch_list_bytes(numels, count) ||
+                                (reinterpret_cast<uintptr_t>(lists) & 15u) != 0))
+        return CONEF_ERR_INVALID;
+    return topk_sparsify_batch(xs, numels, ks, count, workspace, workspace_bytes, lists, stream, TopkRun::kListed);
 }
 
 

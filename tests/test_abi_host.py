@@ -272,3 +272,24 @@ def test_one_launch_round_qualification_and_workspace(lib):
     arr = items_for(sliced, 2)
     assert lib.conef_psgd_round_small_f32(arr, len(sliced), 1, 1, 0.0, 0.0, 0.0, 994443, 609478, None, 0, None) != 0
     assert lib.conef_psgd_round_small_f32(items_for([(128, 577)], 2), 1, 0, 0, 0.0, 0.0, 0.0, 994443, 609478, None, 0, None) != 0
+
+
+def test_topk_workspaces_are_what_they_were():
+    """The batch entry points take a selection state a tensor, as long as the single-tensor one's, whatever
+    the tensors' sizes: callers that sized their buffers before candidate lists came along still fit.
+    The lists are a buffer of their own, with a call of its own for the size."""
+    from conef_amd import _lib
+    lib = _lib.load()
+    sizes = [1, 1000, 1 << 20, 25 << 20]
+    numels = (ctypes.c_int64 * 4)(*sizes)
+    one = -(-lib.conef_topk_workspace_bytes(1) // 256) * 256
+    assert lib.conef_topk_batch_workspace_bytes(numels, 4) == 4 * one
+    assert lib.conef_topk_batch_workspace_bytes(numels, 0) == 256
+    lists = lib.conef_topk_batch_list_bytes(numels, 4)
+    assert 2 * sum(sizes) <= lists <= 2 * sum(sizes) + (1 << 20)            # eight bytes for a quarter of the elements
+    assert lib.conef_topk_batch_list_bytes(None, 1) == -1
+    # a list buffer that is missing, short or misaligned is refused before anything is launched
+    ks = (ctypes.c_int64 * 4)(1, 10, 10, 10)
+    xs = (ctypes.c_void_p * 4)(*[4096] * 4)
+    for at, n in ((None, lists), (4096, lists - 1), (4104, lists)):
+        assert lib.conef_topk_sparsify_batch_listed_f32(xs, numels, ks, 4, 4096, 4 * one, at, n, 0) == -1

@@ -1249,6 +1249,82 @@ def test_topk_through_a_candidate_list():
                 np.testing.assert_array_equal(to_np(t), want, err_msg="%s, call %d, batch of %d" % (name, call, n))
 
 
+def _listed(lib, tensors, ks, ws=None, lists=None):
+    """conef_topk_sparsify_batch_listed_f32 of some device tensors; returns the selection state it keeps."""
+    n = len(tensors)
+    ptrs = (ctypes.c_void_p * n)(*[t.data_ptr() for t in tensors])
+    numels = (ctypes.c_int64 * n)(*[t.numel() for t in tensors])
+    if ws is None:
+        ws = torch.zeros(lib.conef_topk_batch_workspace_bytes(numels, n), dtype=torch.uint8, device="cuda")
+    if lists is None:
+        lists = torch.full((lib.conef_topk_batch_list_bytes(numels, n),), 0xA5, dtype=torch.uint8, device="cuda")
+    rc = lib.conef_topk_sparsify_batch_listed_f32(ptrs, numels, (ctypes.c_int64 * n)(*ks), n, ws.data_ptr(), ws.numel(),
+                                                  lists.data_ptr(), lists.numel(), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    return ws, lists
+
+
+def test_topk_with_lists_lent_by_the_caller():
+    """The hooks' entry point: the state stays with the tensors, the lists are scratch that anything may have
+    written in between; tensors whose undecided keys fit the short list and tensors where they do not."""
+    from conef_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(8)
+    near = 1.0 + torch.rand(70_001, generator=gen) * 2.0 ** -14          # 512 floats: all keys share two digits
+    repeated = near.clone()
+    repeated[torch.rand(70_001, generator=gen) < 0.01] = float(near[77])     # some 800 ties, as many as are noted
+    crowd = near.clone()
+    crowd[torch.rand(70_001, generator=gen) < 0.05] = float(near[77])        # some 3500, more than are noted
+    rank_of = int((near > near[77]).sum())
+    inf = near.clone()
+    inf[5], inf[9] = float("inf"), -float("inf")
+    zeros = torch.where(torch.rand(70_001, generator=gen) < 0.9, torch.zeros(()), torch.full((), 1e-44))
+    cases = list(_topk_inputs()) + [("narrow", near, 30_000), ("narrow, one stays", near, 1), ("narrow, one goes", near, 70_000),
+                                    ("ties", repeated, rank_of + 300), ("many ties", crowd, rank_of + 500),
+                                    ("infinities", inf, 20), ("denormals and zeros", zeros, 5000), ("only zeros go", zeros, 60_000)]
+    for batch in [[c] for c in cases] + [cases]:
+        tensors, ks = [v.cuda() for _, v, _ in batch], [k for _, _, k in batch]
+        ws = lists = None
+        for call in range(3):
+            for t, (_, v, _) in zip(tensors, batch):
+                t.copy_(v.roll(call))
+            ws, lists = _listed(lib, tensors, ks, ws, lists)
+            for t, (name, v, k) in zip(tensors, batch):
+                full = v.roll(call).numpy()
+                want = np.zeros_like(full)
+                order = np.argsort(-np.abs(full), kind="stable")[:k]
+                want[order] = full[order]
+                np.testing.assert_array_equal(to_np(t), want, err_msg="%s, call %d, batch of %d" % (name, call, len(batch)))
+            lists.fill_(0x5A + call)
+
+
+def test_topk_time_does_not_hang_on_the_spread_of_the_magnitudes():
+    """8 M elements, one in 25 of them within 512 floats of each other and of the threshold (335 000 keys
+    that share two digits with it, some 650 that equal it): a few times what a Gaussian's selection costs.
+    One workgroup walking the tensor takes a hundred times as long."""
+    from conef_amd import _lib
+    lib = _lib.load()
+    n = 8 << 20
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    gauss = torch.randn(n, device="cuda", generator=gen)
+    crowd = torch.rand(n, device="cuda", generator=gen) < 0.04
+    near = torch.where(crowd, 1.0 + torch.rand(n, device="cuda", generator=gen) * 2.0 ** -14, gauss)
+    k = int(((near.abs() > 1.0) & ~crowd).sum()) + int(crowd.sum()) // 2
+    x = torch.empty_like(gauss)
+    ws = lists = None
+    best = {}
+    for name, v in (("gauss", gauss), ("near", near)) * 4:
+        x.copy_(v)
+        ends = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        ends[0].record()
+        ws, lists = _listed(lib, [x], [k], ws, lists)
+        ends[1].record()
+        torch.cuda.synchronize()
+        best[name] = min(best.get(name, 1e9), ends[0].elapsed_time(ends[1]))
+        assert int((x != 0).sum()) == k
+    assert best["near"] < 10 * best["gauss"], best
+
+
 def test_powersgd_state_errors_and_warmup():
     from conef_amd.powerSGD_hook import PowerSGDState, _should_compress, powerSGD_hook
     with pytest.raises(ValueError, match="Expect `start_powerSGD_iter` > 1"):
