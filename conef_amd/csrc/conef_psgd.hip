@@ -669,6 +669,7 @@ struct DeferFixItem {
     int pblocks;             // workgroups that take rows of P; the others take rows of Q
     // A rank r below RP: p, qsrc and q hold rows of RP floats with zeros behind the first r, and the
     // factors the caller keeps, rows of r floats, are written here (null: r is RP, p and q are those).
+    // At ranks 16 and 32 qt can be a second copy of the new Q instead.
     float* pt;
     float* qt;
     int r;
@@ -845,8 +846,8 @@ psgd_defer_fix_wide_batch_kernel(PsgdBatch<DeferFixItem> b)
 #pragma unroll
         for (int c = 0; c < 4; ++c) o[c] = rows_l[lrow][4 * piece + c];
         st4((is_p ? it.p : it.q) + row * RP + 4 * piece, o);
-        if (it.pt) {
-            float* dst = (is_p ? it.pt : it.qt) + row * it.r + 4 * piece;
+        if (float* copy = is_p ? it.pt : it.qt) {
+            float* dst = copy + row * it.r + 4 * piece;
 #pragma unroll
             for (int c = 0; c < 4; ++c)
                 if (4 * piece + c < it.r) dst[c] = o[c];
@@ -867,7 +868,7 @@ struct MfmaMqItem {
     ConefMod mod;       // of width 1: the batched kernel never unsketches
 };
 
-template <int MODE>
+template <int MODE, bool EXACT>
 __global__ void __launch_bounds__(kMfmaThreads)
 psgd_mfma_mq_batch_kernel(PsgdBatch<MfmaMqItem> b)
 {
@@ -875,7 +876,7 @@ psgd_mfma_mq_batch_kernel(PsgdBatch<MfmaMqItem> b)
     int local;
     const MfmaMqItem& it = b.item[psgd_batch_locate(b, &local)];
     const ConefSeeds hs = {0, 0, 0, 0};
-    psgd_mfma_mq_body<MODE>(it.x, it.err, nullptr, nullptr, it.q, it.out, it.n, it.m, it.r, it.cols_per_split, it.mod, 0.f,
+    psgd_mfma_mq_body<MODE, EXACT>(it.x, it.err, nullptr, nullptr, it.q, it.out, it.n, it.m, it.r, it.cols_per_split, it.mod, 0.f,
                             hs, local % it.row_tiles, local / it.row_tiles);
 }
 
@@ -977,15 +978,20 @@ psgd_cs_query_batch_kernel(PsgdBatch<QueryItem> b, float alpha, ConefSeeds hs)
     const int64_t r0 = (int64_t)by * it.rows_per_block;
     const int64_t r1 = r0 + it.rows_per_block < it.n ? r0 + it.rows_per_block : it.n;
     const int w = (int)it.mod.w;
-    for (int64_t r = r0; r < r1; ++r) {
-        const float* row = it.cs + r * w;
-        float* xr = it.x + r * it.m + col;
-        float v[4];
-        conef_ld4u(xr, v);
+    // (the moved quad has a loop of its own: its test inside cost 3.3 of 20.1 us on BERT's buckets)
+    auto walk = [&](auto store) {
+        for (int64_t r = r0; r < r1; ++r) {
+            const float* row = it.cs + r * w;
+            float* xr = it.x + r * it.m + col;
+            float v[4];
+            conef_ld4u(xr, v);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = __fadd_rn(v[k], conef_query_term(row[pk[k] & 0x7fffffffu], pk[k], alpha));
-        conef_st4_own(xr, v, dup);
-    }
+            for (int k = 0; k < 4; ++k) v[k] = __fadd_rn(v[k], conef_query_term(row[pk[k] & 0x7fffffffu], pk[k], alpha));
+            store(xr, v);
+        }
+    };
+    if (dup == 0) walk([](float* xr, const float* v) { conef_st4u(xr, v); });
+    else walk([&](float* xr, const float* v) { conef_st4_own(xr, v, dup); });
 }
 
 // DenseCS.update(vec, beta) (CountSketch.py:27-48) of the sketches of a bucket's matrices on
@@ -2817,9 +2823,12 @@ int mq_batch(const ConefPsgdItem* items, int count, float alpha, int32_t a, int3
                 });
             if (rc != CONEF_OK) return rc;
             const size_t lds = (size_t)kMfmaWaves * 16 * 64 * 4;
+            bool exact = true;
+            for (const MfmaMqItem& t : table) exact = exact && t.m % 4 == 0;
             rc = run_batches(table, blocks, [&](const PsgdBatch<MfmaMqItem>& bt, int grid) {
-                hipLaunchKernelGGL((psgd_mfma_mq_batch_kernel<(MODE == 1 ? 1 : 0)>), dim3((unsigned)grid), dim3(kMfmaThreads),
-                                   lds, s, bt);
+                const dim3 g((unsigned)grid), t(kMfmaThreads);
+                if (exact) hipLaunchKernelGGL((psgd_mfma_mq_batch_kernel<(MODE == 1 ? 1 : 0), true>), g, t, lds, s, bt);
+                else hipLaunchKernelGGL((psgd_mfma_mq_batch_kernel<(MODE == 1 ? 1 : 0), false>), g, t, lds, s, bt);
             });
             if (rc != CONEF_OK) return rc;
             if (!sums.empty()) {
@@ -3342,10 +3351,32 @@ int deferred_products(const PaddedRound& pr, int r, float* const* q_in, float* c
     return round_products_deferred<2>(pr, r, q_in, qi_in, alpha, eps, a, b, workspace, workspace_bytes, s, q_shares);
 }
 
+// Whether the Q factors of a bucket at ranks 9 to 32 go through the kernels that take column after column
+// (one launch, in place) instead of their Gram matrix (three launches).  Rank 16 and rank 32 have such
+// kernels of their own, a matrix a workgroup up to some 2000 rows and a few workgroups that meet above: six
+// factors [1024,32] take 26.4 us against 30.6, [4096,32] 29.7 against 33.4, [1024,16] 12.1 against 16.7,
+// [4096,16] 18.1 against 17.6 - and [8192,32] 69.6 against 38.4.  Between those ranks rows are padded and
+// the column kernels go by single floats: [1024,20] 59.9 us against 35.9.
+inline bool gs_wide_by_columns(const PaddedRound& pr)
+{
+    bool ok = pr.rp > 8 && !pr.padded;
+    for (const ConefPsgdItem& it : pr.items) ok = ok && it.m <= 4096;
+    return ok;
+}
+
+// mats[k], [items[k].m, r], in place
+int orthogonalise_by_columns(const PaddedRound& pr, int r, float* const* mats, float eps, void* workspace, int64_t workspace_bytes,
+                             hipStream_t s)
+{
+    std::vector<int64_t> rows;
+    for (const ConefPsgdItem& it : pr.items) rows.push_back(it.m);
+    const std::vector<int32_t> ranks(pr.items.size(), r);
+    return conef_gram_schmidt_batch_f32(mats, rows.data(), ranks.data(), (int32_t)rows.size(), eps, workspace, workspace_bytes, (void*)s);
+}
+
 // dst[k] <- the rows of src[k] ([m, RP], zeros behind column r) orthogonalised, at ranks 9 to 32: the
 // shares of Q^T Q, the system solved by one workgroup a matrix, T applied row by row.  Three short
-// launches whatever the height, where the kernels that go column by column or meet across
-// workgroups took 28 to 43 us a bucket.
+// launches whatever the height.
 int orthogonalise_by_gram_wide(const PaddedRound& pr, int r, const std::vector<const float*>& src, float* const* dst, float eps,
                                void* workspace, hipStream_t s)
 {
@@ -3855,20 +3886,22 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
             q_in[(size_t)k] = ready && (wide || !pr.padded) ? q_next[k] : own;
             if (pr.padded && !(ready && wide)) pad.push_back(RowsItem{ready ? q_next[k] : items[k].q, own, items[k].m, r, rp});
         }
-        if (!ready && rp <= 8) {
+        const bool columns = rp <= 8 || gs_wide_by_columns(pr);
+        if (!ready && columns) {
             rc = conef_gram_schmidt_batch_f32(mats.data(), rows.data(), ranks.data(), count, eps, workspace, workspace_bytes, stream);
             if (rc != CONEF_OK) return rc;
         }
         rc = copy_rows(pad, hs);
         if (rc != CONEF_OK) return rc;
-        if (!ready) {
-            if (rp > 8) {      // in place: a workgroup of the last launch reads its rows before it writes them
-                std::vector<const float*> src;
-                for (int k = 0; k < count; ++k) src.push_back(pr.items[(size_t)k].q);
-                rc = orthogonalise_by_gram_wide(pr, r, src, q_in.data(), eps, workspace, hs);
-                if (rc != CONEF_OK) return rc;
-            }
+        if (!ready && !columns) {      // in place: a workgroup of the last launch reads its rows before it writes them
+            std::vector<const float*> src;
+            for (int k = 0; k < count; ++k) src.push_back(pr.items[(size_t)k].q);
+            rc = orthogonalise_by_gram_wide(pr, r, src, q_in.data(), eps, workspace, hs);
+            if (rc != CONEF_OK) return rc;
         }
+        // the column kernels work in place: the fix launch leaves the new Q in q_next as well
+        if (want_next && rp > 8 && columns)
+            for (int k = 0; k < count; ++k) pr.qt[(size_t)k] = q_next[k];
         GsAhead* qs = want_next && rp <= 8 ? &ahead : nullptr;
         rc = deferred_products(pr, r, q_in.data(), quads_ready ? q_next + count : nullptr, mq_mode, alpha, eps, a, b, workspace,
                                workspace_bytes, hs, qs);
@@ -3919,9 +3952,13 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
                    ahead.count ? &ahead : nullptr, &used, deferred && rp <= 8 ? &pr.qi : nullptr);
     if (rc != CONEF_OK) return rc;
     if (want_next && deferred && rp > 8) {
-        std::vector<const float*> src;
-        for (int k = 0; k < count; ++k) src.push_back(its[k].q);
-        rc = orthogonalise_by_gram_wide(pr, items[0].r, src, q_next, eps, workspace, hs);
+        if (gs_wide_by_columns(pr)) {
+            rc = orthogonalise_by_columns(pr, items[0].r, q_next, eps, workspace, workspace_bytes, hs);
+        } else {
+            std::vector<const float*> src;
+            for (int k = 0; k < count; ++k) src.push_back(its[k].q);
+            rc = orthogonalise_by_gram_wide(pr, items[0].r, src, q_next, eps, workspace, hs);
+        }
         if (rc != CONEF_OK) return rc;
         used = true;
     }
@@ -3943,14 +3980,17 @@ int conef_psgd_q_next_f32(const ConefPsgdItem* items, int32_t count, float eps, 
     if ((defer_env && defer_env[0] == '0') || !padded_round(items, count, 0, workspace, workspace_bytes, &pr) || pr.rp <= 8)
         return CONEF_OK;
     hipStream_t s = (hipStream_t)stream;
+    const bool columns = gs_wide_by_columns(pr);
     std::vector<const float*> src;
-    std::vector<RowsItem> pad;
+    std::vector<RowsItem> copies;
     for (int k = 0; k < count; ++k) {
         src.push_back(pr.padded ? q_next[k] : items[k].q);
-        if (pr.padded) pad.push_back(RowsItem{items[k].q, q_next[k], items[k].m, items[0].r, pr.rp});
+        if (pr.padded || columns) copies.push_back(RowsItem{items[k].q, q_next[k], items[k].m, items[0].r, pr.rp});
     }
-    if (int rc = copy_rows(pad, s); rc != CONEF_OK) return rc;
-    const int rc = orthogonalise_by_gram_wide(pr, items[0].r, src, q_next, eps, workspace, s);
+    int rc = copy_rows(copies, s);
+    if (rc != CONEF_OK) return rc;
+    rc = columns ? orthogonalise_by_columns(pr, items[0].r, q_next, eps, workspace, workspace_bytes, s)
+                 : orthogonalise_by_gram_wide(pr, items[0].r, src, q_next, eps, workspace, s);
     if (rc == CONEF_OK) *made = 1;
     return rc;
 }

@@ -38,8 +38,9 @@ constexpr int kMfmaThreads = 64 * kMfmaWaves;
 // more than one column split the tile goes to a partial buffer [split][n][r] that a second kernel
 // adds up in split order.  Rows of any length from four up and any alignment: a row's last quad is
 // moved back to end with the row (conef_quad_col), its columns that are the quad's before it count
-// as zeros.
-template <int MODE>
+// as zeros.  EXACT: m % 4 == 0, no quad is moved (the tests for one cost 0.5 of 13.1 us on BERT's buckets
+// at rank 32).
+template <int MODE, bool EXACT>
 __device__ __forceinline__ void
 psgd_mfma_mq_body(float* __restrict__ x, const float* __restrict__ err, const float* __restrict__ cs,
                   const uint32_t* __restrict__ pktab, const float* __restrict__ q, float* __restrict__ out, int64_t n,
@@ -79,7 +80,7 @@ psgd_mfma_mq_body(float* __restrict__ x, const float* __restrict__ err, const fl
         for (int u = 0; u < 4; ++u) {
             const int c = cb + 8 * u + 4 * half;
             const int ce = c < c_end ? c : c_begin;     // past the end: a valid quad, its products are zeroed
-            const int cc = ce + 4 <= m ? ce : m - 4;
+            const int cc = EXACT || ce + 4 <= m ? ce : m - 4;
             conef_ld4u(xrow + cc, st.xv[u]);
             if (MODE == 1) conef_ld4u(erow + cc, st.ev[u]);
             if (MODE == 2) {
@@ -99,7 +100,7 @@ psgd_mfma_mq_body(float* __restrict__ x, const float* __restrict__ err, const fl
         for (int u = 0; u < 4; ++u) {
             const int c = cb + 8 * u + 4 * half;
             const bool ok = c < c_end;
-            const int dup = ok && c + 4 > m ? c - (m - 4) : 0;
+            const int dup = !EXACT && ok && c + 4 > m ? c - (m - 4) : 0;
             if (MODE == 1) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) st.xv[u][j] = __fadd_rn(st.xv[u][j], st.ev[u][j]);
@@ -113,7 +114,7 @@ psgd_mfma_mq_body(float* __restrict__ x, const float* __restrict__ err, const fl
             if (MODE != 0 && ok && row_ok) conef_st4_own(xrow + c - dup, st.xv[u], dup);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                float a = ok && j >= dup ? st.xv[u][j] : 0.f;
+                float a = ok && (EXACT || j >= dup) ? st.xv[u][j] : 0.f;
                 float b = (ok && rank_ok) ? st.qv[u][j] : 0.f;
                 acc = conef_mfma32(a, b, acc);
             }
@@ -156,7 +157,7 @@ psgd_mfma_mq_kernel(float* __restrict__ x, const float* __restrict__ err, const 
                     const uint32_t* __restrict__ pktab, const float* __restrict__ q, float* __restrict__ out, int64_t n,
                     int m, int r, int cols_per_split, ConefMod mod, float alpha, ConefSeeds hs)
 {
-    psgd_mfma_mq_body<MODE>(x, err, cs, pktab, q, out, n, m, r, cols_per_split, mod, alpha, hs, (int)blockIdx.x,
+    psgd_mfma_mq_body<MODE, false>(x, err, cs, pktab, q, out, n, m, r, cols_per_split, mod, alpha, hs, (int)blockIdx.x,
                             (int)blockIdx.y);
 }
 

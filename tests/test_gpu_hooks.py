@@ -1019,13 +1019,13 @@ def test_q_factors_orthogonalised_by_the_last_launch(monkeypatch, oracle, rank, 
             same(x, z)
 
 
-def _two_rounds(oracle, monkeypatch, rank, flags, defer, quads=False):
+def _two_rounds(oracle, monkeypatch, rank, flags, defer, quads=False, cols=(300, 1000)):
     """Two rounds over the same two matrices through conef_psgd_round_ahead_f32, the second starting from
     what the first left in q_next where it says so.  Each q_next[k] is followed by a stretch of sentinels.
     Returns (*made of the first round, [q_next buffer, rows asked for, orthogonal Q the oracle makes], results)."""
     from conef_amd import _lib
     lib = _lib.load()
-    specs = [(512, 300, rank), (96, 1000, rank)]
+    specs = [(512, cols[0], rank), (96, cols[1], rank)]
     bound = 1 << (rank - 1).bit_length()
     row = bound if flags & 8 else rank
     rs = np.random.RandomState(21)
@@ -1083,12 +1083,13 @@ def test_a_second_buffer_of_tight_rows_stays_within_them(monkeypatch, oracle, ra
 @pytest.mark.parametrize("rank", [3, 4, 6, 8, 12, 16])
 @pytest.mark.parametrize("defer", ["11", "10", "01", "00"])
 @pytest.mark.parametrize("wide", [0, 8, 12])
-def test_what_a_round_leaves_for_the_next_does_not_depend_on_how_either_runs(monkeypatch, oracle, rank, defer, wide):
+def test_what_a_round_leaves_for_the_next_does_not_depend_on_how_either_runs(monkeypatch, oracle, rank, defer, wide,
+                                                                             cols=(300, 1000)):
     """The order of steps inside a round (deferred or the reference's) can change between the round that
     makes the next Q factors and the one that reads them: the layout of q_next is what the flags say, and
     the second round agrees with the oracle's either way.  1e-4: the second round's input has been through
     one fp32 orthogonalisation here and one in the oracle, whose roundings its products carry on."""
-    made, rows, want, keep, specs = _two_rounds(oracle, monkeypatch, rank, wide, defer, quads=wide == 12)
+    made, rows, want, keep, specs = _two_rounds(oracle, monkeypatch, rank, wide, defer, quads=wide == 12, cols=cols)
     if wide and made:
         bound = 1 << (rank - 1).bit_length()
         for (buf, row), q, (n, m, r) in zip(rows, want, specs):
@@ -1103,6 +1104,14 @@ def test_what_a_round_leaves_for_the_next_does_not_depend_on_how_either_runs(mon
         assert_close(P, p, rel=1e-4, what="P of the second round")
         assert_close(Q, q, rel=1e-4, what="Q of the second round")
         assert_close(M, oracle.pqt(p, q), rel=1e-4, what="M of the second round")
+
+
+@pytest.mark.parametrize("rank", [16, 32])
+@pytest.mark.parametrize("cols", [(300, 4096), (4100, 40), (4097, 4096)])
+@pytest.mark.parametrize("defer", ["11", "10"])
+def test_q_factors_around_the_height_where_the_column_kernels_end(monkeypatch, oracle, rank, cols, defer):
+    """Ranks 16 and 32 orthogonalise Q column by column up to 4096 rows, from its Gram matrix above."""
+    test_what_a_round_leaves_for_the_next_does_not_depend_on_how_either_runs(monkeypatch, oracle, rank, defer, 8, cols=cols)
 
 
 @pytest.mark.parametrize("rank,mode", [(32, "conef"), (16, "ef"), (12, "plain")])
