@@ -323,6 +323,11 @@ __device__ __forceinline__ void
 conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, CsT* cs_out, int64_t n, int d, int w,
                    int rb, double one_minus_beta, int bx, bool pk_lds = false)
 {
+    // Requests past the end of a table are left out where the cells are floats (a uniform test each; rows there
+    // are often short, and a request past the end is a request all the same: [33278,650] 25.6 us against 26.0,
+    // [30522,1024] 34.8 against 36.2, a pair [4096,1024] + [1024,4096] 16.9 against 16.7) and made where they are
+    // halves ([640,5760] 10.3 us without the tests, 11.2 with them; [33278,650] 25.5 and 27.8).
+    constexpr bool sparing = sizeof(CsT) == sizeof(float);
     extern __shared__ float conef_rl[];
     float* vals = conef_rl;
     uint16_t* ent_l = reinterpret_cast<uint16_t*>(vals + ((rb * d + 3) & ~3));
@@ -342,14 +347,14 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
     uint32_t ent_pre[kPreE], csr_pre[kPreC];
     const uint32_t ord_pre = ord_src[(int)threadIdx.x < ord_words ? (int)threadIdx.x : ord_words - 1];
 #pragma unroll
-    for (int u = 0; u < kPreE; ++u) {                  // (uniform: a request past the end is a request all the same)
+    for (int u = 0; u < kPreE; ++u) {
         const int i = threadIdx.x + u * kConefRowlistThreads;
-        if (u * kConefRowlistThreads < ent_words) ent_pre[u] = ent_src[i < ent_words ? i : ent_words - 1];
+        if (!sparing || u * kConefRowlistThreads < ent_words) ent_pre[u] = ent_src[i < ent_words ? i : ent_words - 1];
     }
 #pragma unroll
     for (int u = 0; u < kPreC; ++u) {
         const int i = threadIdx.x + u * kConefRowlistThreads;
-        if (u * kConefRowlistThreads < csr_words) csr_pre[u] = plan.csr[i < csr_words ? i : csr_words - 1];
+        if (!sparing || u * kConefRowlistThreads < csr_words) csr_pre[u] = plan.csr[i < csr_words ? i : csr_words - 1];
     }
     typename Front::Regs regs;
     uint32_t* pk_l = reinterpret_cast<uint32_t*>(cells + rb * w);
@@ -365,8 +370,8 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
 #pragma unroll
         for (int u = 0; u < kPark; ++u) {
             const int i = threadIdx.x + u * kConefRowlistThreads;
-            if (u * kConefRowlistThreads < count) ct[u] = conef_ld(src + (i < count ? i : count - 1));
-            if (pk_lds && u * kConefRowlistThreads < d) pt[u] = plan.pk[i < d ? i : d - 1];
+            if (!sparing || u * kConefRowlistThreads < count) ct[u] = conef_ld(src + (i < count ? i : count - 1));
+            if (!sparing || (pk_lds && u * kConefRowlistThreads < d)) pt[u] = plan.pk[i < d ? i : d - 1];
         }
 #pragma unroll
         for (int u = 0; u < kPark; ++u) {
@@ -391,7 +396,7 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
 #pragma unroll
         for (int u = 0; u < kPre; ++u) {
             const int p = threadIdx.x + u * kConefRowlistThreads;
-            if (u * kConefRowlistThreads < total) aux_pre[u] = conef_ld(cs_in + row0 * w + (p < total ? p : total - 1));
+            if (!sparing || u * kConefRowlistThreads < total) aux_pre[u] = conef_ld(cs_in + row0 * w + (p < total ? p : total - 1));
         }
     }
     if constexpr (Front::kNeedsCells) {
