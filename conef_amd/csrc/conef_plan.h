@@ -75,7 +75,7 @@ inline bool conef_plan_shape(int64_t n, int64_t d, int32_t w, int32_t hint_chunk
 {
     if (n < 1 || d < 1 || d > 0x7fffffffLL || w < 1 || w > (1 << 30)) return false;
     ConefRowlistShape rl;
-    if (hint_chunk <= 0 && hint_bin <= 0 && conef_rowlist_shape(n, d, w, true, &rl)) {
+    if (hint_chunk <= 0 && hint_bin <= 0 && conef_rowlist_shape(n, d, w, true, true, &rl)) {
         memset(h, 0, sizeof(*h));
         h->magic = kConefPlanMagic;
         h->version = 1;

@@ -1154,6 +1154,11 @@ struct ListPsgdResidual {
     int r;
     const float* qi;         // not null: q laid out by quads (conef_load_slices), FAST
     static constexpr bool kNeedsCells = false;
+    // Half-height tiles where there are tiles to spare (conef_rowlist_shape) up to rank 4 and from 512 columns
+    // on: full against half height [30522,1024] 69.2 and 62.5 us at rank 4 (79.0 and 93.0 at rank 8, whose slices
+    // of Q a tile loads whatever its height), [50000,512] 64.0 and 52.7 (72.0 and 73.1), [20000,2048] 89.3 and
+    // 74.9 at rank 1; [60000,300] at rank 4 40.5 and 43.1.
+    static bool halves(int64_t m) { return RP <= 4 && m >= 512; }
     struct Regs {};
     __device__ __forceinline__ void stage(int64_t row0, int rows, int d, int, float* vals, const float*,
                                           const uint32_t*) const
@@ -3515,14 +3520,14 @@ int pqt_sketch_group(const ConefPsgdItem* items, const std::vector<int>& members
     int64_t full_tiles = 0;
     for (int j : members) {
         ConefRowlistShape shape;
-        if (!conef_rowlist_shape(items[j].n, items[j].m, items[j].w, false, &shape, 0)) return CONEF_ERR_INVALID;
+        if (!conef_rowlist_shape(items[j].n, items[j].m, items[j].w, false, ListPsgdResidual<RP, FAST>::halves(items[j].m), &shape, 0)) return CONEF_ERR_INVALID;
         full_tiles += shape.tiles;
     }
     const int companions = full_tiles >= 600 ? 0 : (int)members.size();
     for (int j : members) {
         const ConefPsgdItem& it = items[j];
         ConefRowlistShape shape;
-        if (!conef_rowlist_shape(it.n, it.m, it.w, false, &shape, companions)) return CONEF_ERR_INVALID;
+        if (!conef_rowlist_shape(it.n, it.m, it.w, false, ListPsgdResidual<RP, FAST>::halves(it.m), &shape, companions)) return CONEF_ERR_INVALID;
         RowlistResidualItem<RP, FAST> t = {{it.x, it.p, it.q, it.r, qi ? (*qi)[(size_t)j] : nullptr},
                                            conef_rowlist_view((const ConefPlanHeader*)it.plan_host, it.plan_dev),
                                            it.cs, it.cs, it.n, (int)it.m, it.w, shape.rb};
@@ -3789,7 +3794,7 @@ int conef_psgd_sketch_update_batch_f32(const ConefPsgdItem* items, int32_t count
     int64_t full_tiles = 0;     // as in pqt_sketch_group: full-height tiles when there are 600 of them
     for (int k = 0; k < count; ++k) {
         ConefRowlistShape shape;
-        if (conef_rowlist_shape(items[k].n, items[k].m, items[k].w, ConefListVec::kNeedsCells, &shape, 0))
+        if (conef_rowlist_shape(items[k].n, items[k].m, items[k].w, ConefListVec::kNeedsCells, ConefListVec::halves(items[k].m), &shape, 0))
             full_tiles += shape.tiles;
     }
     const int companions = full_tiles >= 600 ? 0 : count;
@@ -3800,7 +3805,7 @@ int conef_psgd_sketch_update_batch_f32(const ConefPsgdItem* items, int32_t count
             !conef_plan_matches(hp, it.n, it.m, it.w, a, b) || hp->kind != kConefPlanRowlist)
             return CONEF_ERR_INVALID;
         ConefRowlistShape shape;
-        if (!conef_rowlist_shape(it.n, it.m, it.w, ConefListVec::kNeedsCells, &shape, companions)) return CONEF_ERR_INVALID;
+        if (!conef_rowlist_shape(it.n, it.m, it.w, ConefListVec::kNeedsCells, ConefListVec::halves(it.m), &shape, companions)) return CONEF_ERR_INVALID;
         RowlistVecItem t = {{it.err, aligned16(it.err) && it.m % 4 == 0}, conef_rowlist_view(hp, it.plan_dev), it.cs, it.cs,
                             it.n, (int)it.m, it.w, shape.rb};
         table.push_back(t);

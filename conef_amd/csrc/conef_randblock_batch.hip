@@ -178,7 +178,7 @@ int conef_randblock_step_batch_f32(const ConefRandBlockItem* items, int32_t coun
         const ConefPlanHeader* hp = (const ConefPlanHeader*)it.plan_host;
         if (!hp || hp->kind != kConefPlanRowlist) continue;
         ConefRowlistShape shape;
-        if (!conef_rowlist_shape(it.n, it.m, it.w, ConefListRandBlock::kNeedsCells, &shape)) return CONEF_ERR_INVALID;
+        if (!conef_rowlist_shape(it.n, it.m, it.w, ConefListRandBlock::kNeedsCells, ConefListRandBlock::halves(it.m), &shape)) return CONEF_ERR_INVALID;
         ListItem t = {{it.x, it.payload, conef_make_block(it.n * it.m, it.start, it.block), alpha},
                       conef_rowlist_view(hp, it.plan_dev), it.cs_in, it.cs_out, it.n, (int)it.m, it.w, shape.rb, shape.pk_lds};
         table.push_back(t);

@@ -57,13 +57,14 @@ inline size_t conef_rowlist_lds(int rb, int64_t d, int32_t w, bool cells)
 // `companions`: matrices of about this size that share the launch (a batch leaves enough tiles
 // for the machine with taller tiles per matrix); 0: full-height tiles whatever the count (for a
 // batch whose caller has checked that it has tiles enough that way).
-inline bool conef_rowlist_shape(int64_t n, int64_t d, int32_t w, bool cells, ConefRowlistShape* s, int companions = 1)
+inline bool conef_rowlist_shape(int64_t n, int64_t d, int32_t w, bool cells, bool halves, ConefRowlistShape* s,
+                                int companions = 1)
 {
     if (d < 1 || d > kConefRowlistMaxCols || n < 1 || w < 1 || w > 0xffff) return false;
     int64_t rb = 8192 / d;
-    // tiles to spare, in a front that keeps the column table in LDS next to them: half-height ones, twice as
-    // many resident per CU (a quarter was slower again; the other fronts are 2 % faster at full height)
-    if (cells && rb >= 2 && n / rb >= 2048) rb = (rb + 1) / 2;
+    // tiles to spare, in a front that asks for it (Front::halves): half-height ones, twice as many resident per
+    // CU (a quarter was slower again)
+    if (halves && rb >= 2 && n / rb >= 2048) rb = (rb + 1) / 2;
     if (companions > 0 && rb > n * companions / 1024) rb = n * companions / 1024;
     if (rb > 16) rb = 16;
     if (rb < 1) rb = 1;
@@ -94,6 +95,10 @@ struct ConefListVec {
     const float* vec;
     bool vec_ok;           // base 16-byte aligned and d % 4 == 0 (the tile copy works either way)
     static constexpr bool kNeedsCells = false;
+    // whether a tensor with tiles to spare goes by half-height ones.  Full against half height: [50000,512] 40.2
+    // and 29.9 us, [20000,2048] 49.0 and 45.9, [30522,1024] 37.0 and 36.2, [33278,650] 26.2 and 26.0, [60000,300]
+    // and [33278,200] within 1 % either way.
+    static bool halves(int64_t) { return true; }
     struct Regs {};
     __device__ __forceinline__ void stage(int64_t row0, int rows, int d, int, float* vals, const float*,
                                           const uint32_t*) const
@@ -151,6 +156,7 @@ struct ConefListRandBlock {
     ConefBlock blk;
     float alpha;
     static constexpr bool kNeedsCells = true;
+    static bool halves(int64_t) { return true; }      // (the column table sits in LDS next to the tiles)
     static constexpr int kQuads = 4;
     struct Regs {          // a thread's first kQuads quads, by name: no array for the compiler to keep in memory
         float4 g0, g1, g2, g3;
@@ -494,7 +500,7 @@ int conef_launch_rowlist(Front front, ConefRowlistView plan, const CsT* cs_in, C
                          int32_t w, float beta, hipStream_t s)
 {
     ConefRowlistShape shape;
-    if (!conef_rowlist_shape(n, d, w, Front::kNeedsCells, &shape)) return CONEF_ERR_INVALID;
+    if (!conef_rowlist_shape(n, d, w, Front::kNeedsCells, Front::halves(d), &shape)) return CONEF_ERR_INVALID;
     auto k = conef_rowlist_kernel<CsT, Front>;
     hipError_t e = conef_allow_lds((const void*)k, shape.lds);
     if (e != hipSuccess) return (int)e;

@@ -488,6 +488,36 @@ def test_batch_sketched_products_on_matrix_cores(oracle):
     assert lib.conef_psgd_sketch_update_batch_f32(items, count, 0.9, a, b, 0) == -1      # every item needs its plan
 
 
+@pytest.mark.parametrize("n,m", [(32767, 512), (32773, 512), (32800, 511), (4099, 4096)])
+@pytest.mark.parametrize("rank", [0, 4, 8])
+def test_row_list_tiles_on_either_side_of_half_height(oracle, n, m, rank):
+    """Tensors with 2048 full-height tiles or more go by half-height ones: the plain update (rank 0) and the
+    residual of a round up to rank 4 on rows of at least 512 columns."""
+    from conef_amd import _lib
+    from conef_amd.compressors.CountSketch import DenseCS
+    lib = _lib.load()
+    gen = torch.Generator(device="cuda").manual_seed(n + m + rank)
+    X = torch.randn(n, m, device="cuda", generator=gen)
+    cs, ocs = DenseCS(n, m, 0.05), oracle.DenseCS(n, m, 0.05)
+    cs.cs.normal_(generator=gen)
+    ocs.cs[:] = to_np(cs.cs)
+    if rank == 0:
+        cs.update(X, 0.9)
+        ocs.update(to_np(X), 0.9)
+        np.testing.assert_array_equal(to_np(cs.cs), ocs.cs)
+        return
+    P, Q = torch.randn(n, rank, device="cuda", generator=gen) * 0.1, torch.randn(m, rank, device="cuda", generator=gen)
+    x, plan, items = to_np(X).copy(), cs.plan(), (_lib.PsgdItem * 1)()
+    it = items[0]
+    it.x, it.cs, it.p, it.q, it.n, it.m, it.r, it.w = X.data_ptr(), cs.cs.data_ptr(), P.data_ptr(), Q.data_ptr(), n, m, rank, cs.range
+    it.plan_host, it.plan_dev = plan.host_ptr, plan.device.data_ptr()
+    assert lib.conef_psgd_pqt_batch_f32(items, 1, 2, 0.9, cs.a, cs.b, torch.cuda.current_stream().cuda_stream) == 0
+    low = to_np(X)
+    assert_close(low, oracle.pqt(to_np(P), to_np(Q)), what="M = P Q^T")
+    ocs.update(x - low, 0.9)
+    np.testing.assert_array_equal(to_np(cs.cs), ocs.cs)
+
+
 def psgd_check_factory(st, ost, mode):
     def check(step, gd, og):
         assert_close(gd, og, what="%s: decompressed bucket, step %d" % (mode, step))
