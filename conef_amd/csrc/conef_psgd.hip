@@ -3693,23 +3693,19 @@ int pqt_batch(const ConefPsgdItem* items, int count, int mode, float beta, int32
     return CONEF_OK;
 }
 
-// P = X Q with the Q factors of `its`, P orthogonalised, Q = X^T P into items[k].q, on the caller's factors.
-int round_products(const ConefPsgdItem* items, const ConefPsgdItem* its, int count, int mq_mode, float alpha, float eps,
-                   int32_t a, int32_t b, void* workspace, int64_t workspace_bytes, hipStream_t s)
+// Whether a round of these matrices runs with the orthogonalisation of P deferred: where the batch allows
+// (padded_round), unless CONEF_ROUND_DEFER=0 asks for the reference's order of steps (read on every call: a
+// test switches it).
+bool round_defers(const ConefPsgdItem* items, int count, int mq_mode, void* workspace, int64_t workspace_bytes, PaddedRound* pr)
 {
     const char* defer_env = getenv("CONEF_ROUND_DEFER");
-    PaddedRound pr;
-    if (!(defer_env && defer_env[0] == '0') && padded_round(items, count, mq_mode, workspace, workspace_bytes, &pr)) {
-        const int r = items[0].r;
-        std::vector<float*> q_in;
-        std::vector<RowsItem> pad;
-        for (int k = 0; k < count; ++k) {
-            q_in.push_back(pr.padded ? pr.items[(size_t)k].q : its[k].q);
-            if (pr.padded) pad.push_back(RowsItem{its[k].q, pr.items[(size_t)k].q, its[k].m, r, pr.rp});
-        }
-        if (int rc = copy_rows(pad, s); rc != CONEF_OK) return rc;
-        return deferred_products(pr, r, q_in.data(), nullptr, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, s, nullptr);
-    }
+    return !(defer_env && defer_env[0] == '0') && padded_round(items, count, mq_mode, workspace, workspace_bytes, pr);
+}
+
+// P = X Q with the Q factors of `its`, P orthogonalised, Q = X^T P into items[k].q, as the three steps they are.
+int products_in_order(const ConefPsgdItem* items, const ConefPsgdItem* its, int count, int mq_mode, float alpha, float eps,
+                      int32_t a, int32_t b, void* workspace, int64_t workspace_bytes, hipStream_t s)
+{
     int rc = conef_psgd_mq_batch_f32(its, count, mq_mode, alpha, a, b, workspace, workspace_bytes, (void*)s);
     if (rc != CONEF_OK) return rc;
     std::vector<float*> mats;
@@ -3872,12 +3868,9 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
     for (int k = 0; k < count && want_next; ++k) want_next = q_next[k] && items[k].r == items[0].r && items[k].m <= 0x7fffffffLL;
     const int rp = rank_bound(items[0].r);
     // P = X Q, P orthogonalised, Q = X^T P: with the orthogonalisation deferred where the batch
-    // allows (padded_round; CONEF_ROUND_DEFER=0 keeps the reference's order of steps, for
-    // comparisons), else as three steps
-    const char* defer_env = getenv("CONEF_ROUND_DEFER");      // read on every call: a test switches it
+    // allows, else as three steps
     PaddedRound pr;
-    const bool deferred = !(defer_env && defer_env[0] == '0') &&
-                          padded_round(items, count, mq_mode, workspace, workspace_bytes, &pr);
+    const bool deferred = round_defers(items, count, mq_mode, workspace, workspace_bytes, &pr);
     const ConefPsgdItem* its = deferred ? pr.items.data() : items;       // whose factors the rest of the round reads
     int rc = CONEF_OK;
     if (deferred) {
@@ -3927,7 +3920,7 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
             rc = conef_gram_schmidt_batch_f32(mats.data(), rows.data(), ranks.data(), count, eps, workspace, workspace_bytes, stream);
             if (rc != CONEF_OK) return rc;
         }
-        rc = round_products(items, first.data(), count, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, hs);
+        rc = products_in_order(items, first.data(), count, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, hs);
         if (rc != CONEF_OK) return rc;
     }
     // The new Q factors orthogonalised into q_next, ranks up to 8: by workgroups of the last launch,
@@ -3980,10 +3973,8 @@ int conef_psgd_q_next_f32(const ConefPsgdItem* items, int32_t count, float eps, 
     *made = 0;
     for (int k = 0; k < count; ++k)
         if (!item_ok(items[k]) || !q_next[k]) return CONEF_ERR_INVALID;
-    const char* defer_env = getenv("CONEF_ROUND_DEFER");
     PaddedRound pr;
-    if ((defer_env && defer_env[0] == '0') || !padded_round(items, count, 0, workspace, workspace_bytes, &pr) || pr.rp <= 8)
-        return CONEF_OK;
+    if (!round_defers(items, count, 0, workspace, workspace_bytes, &pr) || pr.rp <= 8) return CONEF_OK;
     hipStream_t s = (hipStream_t)stream;
     const bool columns = gs_wide_by_columns(pr);
     std::vector<const float*> src;
@@ -4176,7 +4167,19 @@ int conef_psgd_products_f32(const ConefPsgdItem* items, const ConefPsgdItem* fir
         if (mq_mode == 2 && it.plan_host && !conef_plan_matches((const ConefPlanHeader*)it.plan_host, it.n, it.m, it.w, a, b))
             return CONEF_ERR_INVALID;
     }
-    return round_products(items, its, count, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, (hipStream_t)stream);
+    hipStream_t s = (hipStream_t)stream;
+    PaddedRound pr;
+    if (!round_defers(items, count, mq_mode, workspace, workspace_bytes, &pr))
+        return products_in_order(items, its, count, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, s);
+    const int r = items[0].r;
+    std::vector<float*> q_in;
+    std::vector<RowsItem> pad;
+    for (int k = 0; k < count; ++k) {
+        q_in.push_back(pr.padded ? pr.items[(size_t)k].q : its[k].q);
+        if (pr.padded) pad.push_back(RowsItem{its[k].q, pr.items[(size_t)k].q, its[k].m, r, pr.rp});
+    }
+    if (int rc = copy_rows(pad, s); rc != CONEF_OK) return rc;
+    return deferred_products(pr, r, q_in.data(), nullptr, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, s, nullptr);
 }
 
 // dense error feedback on the parts of a bucket that are not compressed: x += e; e = 0

@@ -392,6 +392,39 @@ def test_round_defers_the_orthogonalisation_of_p(monkeypatch, oracle, mq_mode, e
         assert not identical, "the round took the step-by-step path on %s" % (specs,)
 
 
+@pytest.mark.parametrize("defer", ["0", "1"])
+@pytest.mark.parametrize("rank", [3, 4, 12, 32])
+@pytest.mark.parametrize("elsewhere", [False, True])
+def test_middle_of_a_round_as_a_call_of_its_own(monkeypatch, oracle, rank, defer, elsewhere):
+    """conef_psgd_products_f32: P = X Q with the Q of `first`, P orthogonalised, Q = X^T P into items' q."""
+    from conef_amd import _lib
+    monkeypatch.setenv("CONEF_ROUND_DEFER", defer)
+    lib = _lib.load()
+    rs = np.random.RandomState(31)
+    specs = [(512, 300), (96, 1000)]
+    items, first, keep = (_lib.PsgdItem * 2)(), (_lib.PsgdItem * 2)(), []
+    for it, other, (n, m) in zip(items, first, specs):
+        M, E = rs.randn(n, m).astype(np.float32), (0.1 * rs.randn(n, m)).astype(np.float32)
+        Q = rs.randn(m, rank).astype(np.float32)
+        Md, Ed, Qd = torch.from_numpy(M).cuda(), torch.from_numpy(E).cuda(), torch.from_numpy(Q).cuda()
+        Pd, Qout = torch.empty(n, rank, device="cuda"), torch.full((m, rank), 7.0, device="cuda")
+        for t, q in ((it, Qout if elsewhere else Qd), (other, Qd)):
+            t.x, t.err, t.p, t.q, t.n, t.m, t.r, t.w = Md.data_ptr(), Ed.data_ptr(), Pd.data_ptr(), q.data_ptr(), n, m, rank, 1
+        keep.append((Md, Ed, Qd, Pd, Qout, M, E, Q))
+    ws = torch.empty(lib.conef_psgd_batch_workspace_bytes(items, 2), dtype=torch.uint8, device="cuda")
+    assert lib.conef_psgd_products_f32(items, first if elsewhere else None, 2, 1, 0.0, 0.0, 1, 1, ws.data_ptr(), ws.numel(),
+                                       torch.cuda.current_stream().cuda_stream) == 0
+    for Md, Ed, Qd, Pd, Qout, M, E, Q in keep:
+        X = M + E
+        p = oracle.mq(X, Q)
+        oracle.gram_schmidt(p, 0.0)
+        np.testing.assert_array_equal(to_np(Md), X)
+        assert_close(Pd, p, what="P")
+        assert_close(Qout if elsewhere else Qd, oracle.mtp(X, p), what="Q")
+        if elsewhere:
+            np.testing.assert_array_equal(to_np(Qd), Q)
+
+
 def test_products_with_sketch_on_a_plan(oracle):
     """P = (M + alpha unsketch) Q and the residual sketch after M = P Q^T, on row-list plans: the
     sketch must come out bit for bit (same terms, same order as the serial definition)."""
