@@ -834,7 +834,11 @@ psgd_defer_fix_wide_batch_kernel(PsgdBatch<DeferFixItem> b)
         const int lr = wave * RPW + u * 4 * RPW + sub;
         float acc = 0.f;
 #pragma unroll 8
-        for (int i = 0; i < RP; ++i) acc = fmaf(rows_l[lr][i], t_l[i * RP + col], acc);      // T is zero below the diagonal
+        for (int i = 0; i < RP; ++i) {
+            // T is zero below the diagonal; a NaN in a later column is not to reach this one through it
+            const float v = rows_l[lr][i];
+            acc = fmaf(i <= col ? v : 0.f, t_l[i * RP + col], acc);
+        }
         out[u] = col < it.r ? acc : 0.f;
     }
     __syncthreads();

@@ -1639,6 +1639,46 @@ def test_hook_step_with_an_all_zero_gradient_matrix(monkeypatch, oracle, rank, m
                     assert np.isfinite(got_e).all() and np.count_nonzero(got_e) == np.count_nonzero(want_e)
 
 
+@pytest.mark.parametrize("eps", [0.0, 1e-8])
+@pytest.mark.parametrize("rank,mode", [(3, "conef"), (5, "ef"), (7, "topk"), (12, "conef"), (20, "ef")])
+def test_all_zero_gradient_matrix_at_ranks_with_padded_factors(monkeypatch, oracle, rank, mode, eps):
+    """The same where the factors have zero columns behind the rank, which are not to be taken for its own."""
+    test_hook_step_with_an_all_zero_gradient_matrix(monkeypatch, oracle, rank, mode, eps, "1")
+
+
+@pytest.mark.parametrize("eps", [0.0, 1e-8])
+@pytest.mark.parametrize("rank", [3, 4, 6, 12, 20, 32])
+@pytest.mark.parametrize("defer", ["0", "1"])
+def test_round_from_a_q_with_a_zero_column(monkeypatch, oracle, rank, eps, defer):
+    """What the reference makes of a column it cannot normalise, through a whole round: NaN from that column on
+    at epsilon 0, a column of zeros at epsilon != 0, at ranks with and without padded factors."""
+    from conef_amd import _lib
+    monkeypatch.setenv("CONEF_ROUND_DEFER", defer)
+    lib = _lib.load()
+    rs = np.random.RandomState(41)
+    items, keep = (_lib.PsgdItem * 2)(), []
+    for it, (n, m) in zip(items, [(512, 300), (96, 1000)]):
+        M, Q = rs.randn(n, m).astype(np.float32), rs.randn(m, rank).astype(np.float32)
+        Q[:, rank // 2] = 0
+        Md, Qd, Pd = torch.from_numpy(M).cuda(), torch.from_numpy(Q).cuda(), torch.empty(n, rank, device="cuda")
+        it.x, it.p, it.q, it.n, it.m, it.r, it.w = Md.data_ptr(), Pd.data_ptr(), Qd.data_ptr(), n, m, rank, 1
+        keep.append((Md, Qd, Pd, M, Q))
+    ws = torch.empty(lib.conef_psgd_batch_workspace_bytes(items, 2), dtype=torch.uint8, device="cuda")
+    assert lib.conef_psgd_round_f32(items, 2, 0, 0, 0.0, 0.0, eps, 1, 1, ws.data_ptr(), ws.numel(),
+                                    torch.cuda.current_stream().cuda_stream) == 0
+    for Md, Qd, Pd, M, Q in keep:
+        q = Q.copy()
+        oracle.gram_schmidt(q, eps)
+        p = oracle.mq(M, q)
+        oracle.gram_schmidt(p, eps)
+        q = oracle.mtp(M, p)
+        assert np.isfinite(p).all() == (eps != 0)
+        what = "rank %d eps %g defer %s" % (rank, eps, defer)
+        _nan_aware_close(Pd, p, what + ", P")
+        _nan_aware_close(Qd, q, what + ", Q")
+        _nan_aware_close(Md, oracle.pqt(p, q), what + ", M")
+
+
 # ------------------------------------------------------- unbiased random matrix --
 
 @pytest.mark.parametrize("shapes,rank", [([(64, 576), (64,), (300, 40), (2, 1024)], 4),
