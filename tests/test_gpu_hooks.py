@@ -1679,6 +1679,95 @@ def test_round_from_a_q_with_a_zero_column(monkeypatch, oracle, rank, eps, defer
         _nan_aware_close(Md, oracle.pqt(p, q), what + ", M")
 
 
+def test_dropped_factors_are_drawn_anew_with_work_left_on_the_side_stream(oracle):
+    """Rank 12 on one hook stream: the round leaves the next Q factors to a side stream.  A caller drops the
+    bucket's P / Q memory after every step; each round then draws new factors into new buffers and must not be
+    touched by what the side stream still had to do."""
+    shapes, rank = [(300, 400), (37,), (257, 128)], 12
+    outs = []
+    for ahead_buffers in (1, 40):                 # few and many allocations between the steps
+        st, hook = _state_for("ef", rank, 0.1, hook_streams=1)
+        st.iter = 2
+        got = []
+        for step in range(6):
+            gd = grads(numel_of(shapes), 900 + step).cuda()
+            hook(st, FakeGradBucket(gd, shapes)).wait()
+            assert st.round_cache[0].q_next is not None
+            st.p_memory_dict.clear()
+            st.q_memory_dict.clear()
+            junk = [torch.full((400 * rank + 16 * k,), float("nan"), device="cuda") for k in range(ahead_buffers)]
+            got.append(to_np(gd))
+            del junk
+        outs.append(got)
+    for a, b in zip(*outs):
+        assert np.isfinite(a).all()
+        np.testing.assert_array_equal(a, b)
+
+
+# block (start, length) as functions of the number of elements: nothing but the head, the tail, a whole tile,
+# across a tile's edges, wrapping round the end with both parts inside full tiles, wrapping with one element,
+# everything from the start and everything from the middle (ratio 1)
+TILE_BLOCKS = [lambda n: (0, 1), lambda n: (n - 1, 1), lambda n: (4096 % n, 4096), lambda n: (4093, 4102), lambda n: (4099, 3),
+               lambda n: (n - 2050, 2050 + 2049), lambda n: (n - 4100, 4100 + 4097), lambda n: (n - 1, 2), lambda n: (n - 3, 8191),
+               lambda n: (0, n), lambda n: (n // 2, n), lambda n: (5000, n - 1)]
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("shift", [0, 1, 2, 3])
+@pytest.mark.parametrize("n", [3 * 4096, 2 * 4096 + 4095, 5 * 4096 + 1])
+def test_random_block_tiles(mode, shift, n):
+    """The kernels without a sketch go by tiles of 4096 elements: full tiles that start 0, 4, 8 and 12 bytes off
+    a 16-byte boundary, the rest, and blocks at every place in them.  Bit for bit, in batches of 1, 5, and
+    more tensors than a launch takes, and through the single-tensor entry points."""
+    from conef_amd import _lib
+    lib = _lib.load()
+    stream = torch.cuda.current_stream().cuda_stream
+    rs = np.random.RandomState(n + shift)
+
+    def check(blocks, batched):
+        count, items, keep = len(blocks), (_lib.RandBlockItem * len(blocks))(), []
+        for it, (start, block) in zip(items, blocks):
+            x, e = rs.randn(n + 8).astype(np.float32), rs.randn(n + 8).astype(np.float32)
+            xd, ed = torch.from_numpy(x).cuda(), torch.from_numpy(e).cuda()
+            pay = torch.full((block + 8,), 7.0, device="cuda")
+            it.x, it.err, it.payload = xd.data_ptr() + 4 * shift, ed.data_ptr() + 4 * shift, pay.data_ptr() + 4 * (3 - shift)
+            it.n, it.m, it.start, it.block = 1, n, start, block
+            keep.append((xd, ed, pay, x, e, start, block))
+        if batched:
+            assert lib.conef_randblock_step_batch_f32(items, count, mode, 0.0, 0.0, 0, 0, stream) == 0
+        else:
+            for it in items:
+                if mode == 0:
+                    rc = lib.conef_randblock_unbiased_step_f32(it.x, it.payload, n, it.start, it.block,
+                                                               float(np.float32(it.block / n)), stream)
+                else:
+                    rc = lib.conef_randblock_ef_step_f32(it.x, it.err, it.payload, n, it.start, it.block, stream)
+                assert rc == 0
+        for xd, ed, pay, x, e, start, block in keep:
+            inner = slice(shift, shift + n)
+            where = (start + np.arange(block)) % n
+            value = x[inner] / np.float32(block / n) if mode == 0 else x[inner] + e[inner]
+            ox, oe = x.copy(), e.copy()
+            ox[inner] = 0
+            ox[inner][where] = value[where]
+            if mode == 1:
+                oe[inner] = value
+                oe[inner][where] = 0
+            opay = np.full(block + 8, 7.0, np.float32)
+            opay[3 - shift: 3 - shift + block] = value[where]
+            what = "mode %d n %d shift %d block (%d, %d)" % (mode, n, shift, start, block)
+            np.testing.assert_array_equal(to_np(xd), ox, err_msg=what)
+            np.testing.assert_array_equal(to_np(ed), oe, err_msg=what + ", error")
+            np.testing.assert_array_equal(to_np(pay), opay, err_msg=what + ", payload")
+
+    blocks = [b(n) for b in TILE_BLOCKS]
+    for b in blocks:
+        check([b], True)
+    check(blocks[:5], True)
+    check((blocks * 5)[:50], True)
+    check(blocks, False)
+
+
 # ------------------------------------------------------- unbiased random matrix --
 
 @pytest.mark.parametrize("shapes,rank", [([(64, 576), (64,), (300, 40), (2, 1024)], 4),
