@@ -10,6 +10,7 @@ streaming passes over its memory: the error add is fused into the first product,
 import contextlib
 import ctypes
 import logging
+import operator
 import os
 
 import torch
@@ -139,7 +140,7 @@ class _RoundPlan:
     __slots__ = ("small", "layout", "errs_known", "cells", "cs_static", "env_ahead", "env_topk_side", "env_small", "key", "shapes", "work", "passthrough", "before", "after", "total_ps", "total_qs", "arena_key", "ps",
                  "qs", "items", "count", "sketches", "fused_sketch", "batched_update", "residual_offsets",
                  "topk_table", "q_next", "q_next_ptrs", "q_next_ready", "q_next_quads", "made", "q_next_event", "aside_recorded",
-                 "topk_event", "topk_recorded", "ws_need", "handoff_event", "topk_number", "q_next_number", "is_wide", "wide", "chunks", "ef_spans")
+                 "topk_event", "topk_recorded", "ws_need", "handoff_event", "topk_number", "q_next_number", "is_wide", "wide", "chunks", "runs", "ef_spans")
 
 
 # flags of conef_psgd_round_ahead_f32 (include/conef_hip.h)
@@ -233,6 +234,7 @@ def _build_round(state, grads, shapes, key, error_mode):
     plan.q_next_event = None
     plan.aside_recorded = None      # the side stream (raw) that q_next and the Q arena are known to the allocator to be used on
     plan.chunks = _chunks(plan.count)
+    plan.runs = [(_at(plan.items, first), part) for first, part in plan.chunks]      # the same as arguments
     plan.ef_spans = None            # dense error feedback: host arrays of the stretches that are not compressed
     plan.residual_offsets = []
     off = 0
@@ -247,11 +249,8 @@ def _sketches_moved(plan, errs):
     """Whether the bucket's sketches are others than the table points at, or the same ones with their cells
     elsewhere (sketches that swap two buffers are pointed at anew every step anyway)."""
     known = plan.errs_known
-    if known is None or len(known) != len(errs):
+    if known is None or len(known) != len(errs) or not all(map(operator.is_, known, errs.values())):
         return True
-    for cs, now in zip(known, errs.values()):
-        if cs is not now:
-            return True
     return plan.cs_static and not plan.cells.same(known)
 
 
@@ -339,12 +338,12 @@ def run_round(state, bucket, error_mode):
     input_tensor = _bucket.buffer(bucket)
     streams = streams_for(state, input_tensor)
     if streams <= 1 or not input_tensor.is_cuda or state.iter < state.start_powerSGD_iter:
-        return _run_round(state, bucket, error_mode, 1)
+        return _run_round(state, bucket, input_tensor, error_mode, 1)
     device = input_tensor.device
     index = _bucket.index(bucket)
     lane = index % streams
     if lane == 0:
-        return _run_round(state, bucket, error_mode, streams)
+        return _run_round(state, bucket, input_tensor, error_mode, streams)
     side = _side_stream(device, lane - 1, streams - 1)
     # the side stream starts where the hook's stream is now (one event per side stream, recorded again
     # for every bucket: a wait takes the event as it is when the wait is enqueued)
@@ -353,7 +352,7 @@ def run_round(state, bucket, error_mode):
     side.wait_event(event)
     input_tensor.record_stream(side)
     with _lib.on_stream(side):
-        return _run_round(state, bucket, error_mode, streams)
+        return _run_round(state, bucket, input_tensor, error_mode, streams)
 
 
 AUTO_STREAMS_MIN_NUMEL = 1 << 20
@@ -371,9 +370,8 @@ def streams_for(state, input_tensor):
     return streams
 
 
-def _run_round(state, bucket, error_mode, streams=1):
+def _run_round(state, bucket, input_tensor, error_mode, streams):
     group, world_size = _bucket.group_and_size(state.process_group)
-    input_tensor = _bucket.buffer(bucket)
 
     if state.iter < state.start_powerSGD_iter:
         state.maybe_increase_iter(bucket)
@@ -481,8 +479,7 @@ def _run_round(state, bucket, error_mode, streams=1):
     eps = float(state.orthogonalization_epsilon)
     if plan.ws_need is None:
         plan.ws_need = plan.wide.ws_need if plan.is_wide else max(
-            [lib.conef_psgd_batch_workspace_bytes(_at(items, first), part)
-             for first, part in plan.chunks] + [256])
+            [lib.conef_psgd_batch_workspace_bytes(run, part) for run, part in plan.runs] + [256])
     ws = _workspace(device, stream, plan.ws_need)
     ws_ptr, ws_len = ws.data_ptr(), ws.numel()
     if need_randomize_qs:
@@ -542,16 +539,16 @@ def _run_round(state, bucket, error_mode, streams=1):
     elif plan.small is None or plan.small[0] != (mode1, mode3):
         # a bucket of small matrices (every one fits a workgroup's LDS with its factors): the whole round in one launch
         fits = bool(count and mode3 in (0, 1, 2) and plan.env_small
-                    and all(lib.conef_psgd_round_small_fits(_at(items, first), part, mode1, mode3, HASH_A, HASH_B)
-                            for first, part in plan.chunks))
+                    and all(lib.conef_psgd_round_small_fits(run, part, mode1, mode3, HASH_A, HASH_B)
+                            for run, part in plan.runs))
         plan.small = ((mode1, mode3), fits)
     beta3 = float(state.beta) if mode3 in (2, 3) else 0.0
     if plan.is_wide:
         pass
     elif plan.small[1]:
         plan.q_next_ready = False
-        for first, part in plan.chunks:
-            rc = lib.conef_psgd_round_small_f32(_at(items, first), part, mode1, mode3, float(alpha), beta3, eps, HASH_A, HASH_B,
+        for run, part in plan.runs:
+            rc = lib.conef_psgd_round_small_f32(run, part, mode1, mode3, float(alpha), beta3, eps, HASH_A, HASH_B,
                                                 ws_ptr, ws_len, stream)
             _lib.check(rc, "conef_psgd_round_small_f32")
     elif count and state.warm_start and plan.env_ahead and (state.matrix_approximation_rank > 8 or mode3 in (0, 1, 2)):
@@ -577,18 +574,19 @@ def _run_round(state, bucket, error_mode, streams=1):
         flags = _ROUND_NEXT_QUADS | _ROUND_NEXT_WIDE | (0 if aside else _ROUND_MAKE_NEXT)
         if plan.q_next_ready:
             flags |= _ROUND_Q_READY | (_ROUND_QUADS_READY if plan.q_next_quads else 0)
-        for (first, part), q_next, made in zip(plan.chunks, plan.q_next_ptrs, plan.made):
-            rc = lib.conef_psgd_round_ahead_f32(_at(items, first), part, mode1, mode3, float(alpha), beta3, eps, HASH_A, HASH_B,
+        all_made = 3
+        for (run, part), q_next, made in zip(plan.runs, plan.q_next_ptrs, plan.made):
+            rc = lib.conef_psgd_round_ahead_f32(run, part, mode1, mode3, float(alpha), beta3, eps, HASH_A, HASH_B,
                                                 q_next, flags, ctypes.byref(made), ws_ptr, ws_len, stream)
             _lib.check(rc, "conef_psgd_round_ahead_f32")
-        plan.q_next_ready = all(made.value for made in plan.made)
-        plan.q_next_quads = all(made.value & 2 for made in plan.made)
+            all_made &= made.value
+        plan.q_next_ready, plan.q_next_quads = bool(all_made & 1), bool(all_made & 2)
         if aside:
-            _orthogonalise_q_aside(plan, lib, items, eps, ws_len, device)
+            _orthogonalise_q_aside(plan, lib, eps, ws_len, device)
     else:
         plan.q_next_ready = False
-        for first, part in plan.chunks:
-            rc = lib.conef_psgd_round_f32(_at(items, first), part, mode1, mode3, float(alpha), beta3, eps, HASH_A, HASH_B,
+        for run, part in plan.runs:
+            rc = lib.conef_psgd_round_f32(run, part, mode1, mode3, float(alpha), beta3, eps, HASH_A, HASH_B,
                                           ws_ptr, ws_len, stream)
             _lib.check(rc, "conef_psgd_round_f32")
     if error_mode == "topk":
@@ -638,7 +636,7 @@ def _at(array, index):
     return ctypes.byref(array, index * ctypes.sizeof(array._type_))
 
 
-def _orthogonalise_q_aside(plan, lib, items, eps, ws_len, device):
+def _orthogonalise_q_aside(plan, lib, eps, ws_len, device):
     """The new Q factors of a bucket orthogonalised for its next round on the side stream."""
     if plan.handoff_event is None:
         plan.handoff_event = torch.cuda.Event()
@@ -655,8 +653,8 @@ def _orthogonalise_q_aside(plan, lib, items, eps, ws_len, device):
         plan.aside_recorded = side.cuda_stream
     with _lib.on_stream(side):
         ws = _workspace(device, side.cuda_stream, max(ws_len, 256))
-    for (first, part), q_next, made in zip(plan.chunks, plan.q_next_ptrs, plan.made):
-        rc = lib.conef_psgd_q_next_f32(_at(items, first), part, eps, q_next, ctypes.byref(made),
+    for (run, part), q_next, made in zip(plan.runs, plan.q_next_ptrs, plan.made):
+        rc = lib.conef_psgd_q_next_f32(run, part, eps, q_next, ctypes.byref(made),
                                        ws.data_ptr(), ws.numel(), side.cuda_stream)
         _lib.check(rc, "conef_psgd_q_next_f32")
     plan.q_next_event.record(side)

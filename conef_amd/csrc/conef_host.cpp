@@ -56,19 +56,21 @@ int conef_host_same_places(PyObject* holders, const int64_t* places, int64_t n)
     }
     int same = cells && PySequence_Fast_GET_SIZE(seq) == (Py_ssize_t)n;
     for (int64_t i = 0; i < n && same; ++i) {
+        // (the exact type first: asking a sketch whether it is a tensor goes through Python)
         PyObject* o = PySequence_Fast_GET_ITEM(seq, i);
-        Py_INCREF(o);
-        if (!THPVariable_Check(o)) {
-            PyObject* inner = PyObject_GetAttr(o, cells);
-            Py_DECREF(o);
+        PyObject* inner = THPVariable_CheckExact(o) ? nullptr : PyObject_GetAttr(o, cells);
+        if (inner) {
             o = inner;
+        } else {
+            PyErr_Clear();
+            Py_INCREF(o);
         }
         try {
-            same = o && THPVariable_Check(o) && (int64_t)(intptr_t)THPVariable_Unpack(o).data_ptr() == places[i];
+            same = THPVariable_Check(o) && (int64_t)(intptr_t)THPVariable_Unpack(o).data_ptr() == places[i];
         } catch (...) {
             same = 0;
         }
-        Py_XDECREF(o);
+        Py_DECREF(o);
     }
     Py_DECREF(seq);
     if (!same) PyErr_Clear();

@@ -150,7 +150,7 @@ def test_every_buffer_the_side_stream_works_on_is_known_to_the_allocator(monkeyp
         monkeypatch.setattr(engine.ctypes, "byref", lambda *a: None)
 
         def hand_over():
-            engine._orthogonalise_q_aside(plan, lib, plan.items, 0.0, 256, device)
+            engine._orthogonalise_q_aside(plan, lib, 0.0, 256, device)
 
         for _ in range(2):           # the second time: a caller dropped the bucket's arenas, a round took new ones
             engine._take_arenas(plan, torch.zeros(64 * 12), torch.zeros(96 * 12))
