@@ -48,8 +48,10 @@ __device__ __forceinline__ uint32_t mag_key(float v) { return __float_as_uint(v)
 // Several tensors per launch (the dense errors of a bucket's matrices, each with its own k and its
 // own state): the table travels by value, a workgroup finds its tensor from the running workgroup
 // count (`first`, the same for every pass) and then
-// does what it would do in a launch of its own.
-constexpr int kTopkBatchMax = 24;
+// does what it would do in a launch of its own.  The arguments of a launch are copied into memory the GPU
+// reads whatever part of them is used (3 us for 3 KB): up to eight tensors, most buckets of a large model,
+// take a table of eight, more of them one of 48 (2.9 KB).
+constexpr int kTopkBatchFew = 8, kTopkBatchMax = 48;
 
 struct TopkItem {
     float* x;
@@ -62,9 +64,10 @@ struct TopkItem {
     uint32_t* final_idx;        // [kTopkFinal] the keys that share two digits with the threshold, then their keys
 };
 
+template <int CAP>
 struct TopkBatch {
-    TopkItem item[kTopkBatchMax];
-    int first[kTopkBatchMax + 1];
+    TopkItem item[CAP];
+    int first[CAP + 1];
     int count;
 };
 
@@ -90,7 +93,8 @@ __device__ __forceinline__ void topk_init_body(TopkState* st, uint32_t k)
 
 __global__ void topk_init_kernel(TopkState* st, uint32_t k) { topk_init_body(st, k); }
 
-__global__ void topk_init_batch_kernel(TopkBatch b) { topk_init_body(b.item[blockIdx.x].st, b.item[blockIdx.x].k); }
+template <int CAP>
+__global__ void topk_init_batch_kernel(TopkBatch<CAP> b) { topk_init_body(b.item[blockIdx.x].st, b.item[blockIdx.x].k); }
 
 // The bin that holds the want-th largest of the keys counted in 256 * per bins, thread t holding the counts
 // of bins t * per .. in cnt: (bin, how many are wanted of it, how many it holds), the same in every
@@ -226,8 +230,9 @@ topk_hist_kernel(const float* __restrict__ x, int64_t numel, TopkState* st, int 
     else topk_hist_body<1>(x, numel, st, pass, (int)blockIdx.x, (int)gridDim.x);
 }
 
+template <int CAP>
 __global__ void __launch_bounds__(256)
-topk_hist_batch_kernel(TopkBatch b, int pass, bool kept)
+topk_hist_batch_kernel(TopkBatch<CAP> b, int pass, bool kept)
 {
     int local, width;
     const TopkItem& it = b.item[topk_locate(b.first, b.count, &local, &width)];
@@ -372,8 +377,9 @@ topk_filter_kernel(float* __restrict__ x, int64_t numel, TopkState* st)
     topk_filter_body(x, numel, st, (int)blockIdx.x, (int)gridDim.x);
 }
 
+template <int CAP>
 __global__ void __launch_bounds__(256)
-topk_filter_batch_kernel(TopkBatch b, bool kept)
+topk_filter_batch_kernel(TopkBatch<CAP> b, bool kept)
 {
     int local, width;
     const TopkItem& it = b.item[topk_locate(b.first, b.count, &local, &width)];
@@ -622,24 +628,27 @@ __device__ __forceinline__ void topk_settle_body(const TopkItem& it, int bx, int
     topk_settle_ties(it.x, it.numel, st, thr, ties, held, gx);
 }
 
+template <int CAP>
 __global__ void __launch_bounds__(256)
-topk_note_batch_kernel(TopkBatch b)
+topk_note_batch_kernel(TopkBatch<CAP> b)
 {
     int local, width;
     const TopkItem& it = b.item[topk_locate(b.first, b.count, &local, &width)];
     topk_note_body(it, local, width);
 }
 
+template <int CAP>
 __global__ void __launch_bounds__(256)
-topk_gather_batch_kernel(TopkBatch b)
+topk_gather_batch_kernel(TopkBatch<CAP> b)
 {
     int local, width;
     const TopkItem& it = b.item[topk_locate(b.first, b.count, &local, &width)];
     topk_gather_body(it, local, width);
 }
 
+template <int CAP>
 __global__ void __launch_bounds__(256)
-topk_settle_batch_kernel(TopkBatch b)
+topk_settle_batch_kernel(TopkBatch<CAP> b)
 {
     int local, width;
     const TopkItem& it = b.item[topk_locate(b.first, b.count, &local, &width)];
@@ -738,7 +747,7 @@ inline int64_t topk_list_bytes(int64_t numel)
 }
 }  // namespace
 
-// The same for `count` tensors, every pass one launch over all of them (in runs of 24): tensor i
+// The same for `count` tensors, every pass one launch over all of them (in runs of 48): tensor i
 // is xs[i] with numels[i] elements and keeps ks[i]; tensors with ks[i] >= numels[i] are left as
 // they are.  xs / numels / ks are host arrays, read before the call returns.
 int64_t conef_topk_batch_workspace_bytes(const int64_t* numels, int32_t count)
@@ -763,8 +772,37 @@ int64_t conef_topk_batch_list_bytes(const int64_t* numels, int32_t count)
     return total > 256 ? total : 256;
 }
 
+}  // extern "C"
+
 namespace {
 enum class TopkRun { kFresh, kKept, kListed };
+
+template <int CAP>
+void topk_launch(const TopkItem* items, int nb, TopkRun run, hipStream_t s)
+{
+    TopkBatch<CAP> b;
+    int wgs = 0;
+    for (int k = 0; k < nb; ++k) {
+        b.item[k] = items[k];
+        b.first[k] = wgs;
+        wgs += (int)topk_hist_groups(items[k].numel);
+    }
+    b.first[nb] = wgs;
+    b.count = nb;
+    const dim3 grid((unsigned)wgs), threads(256);
+    if (run == TopkRun::kListed) {
+        hipLaunchKernelGGL(topk_hist_batch_kernel<CAP>, grid, threads, 0, s, b, 0, true);
+        hipLaunchKernelGGL(topk_note_batch_kernel<CAP>, grid, threads, 0, s, b);
+        hipLaunchKernelGGL(topk_gather_batch_kernel<CAP>, grid, threads, 0, s, b);
+        hipLaunchKernelGGL(topk_settle_batch_kernel<CAP>, grid, threads, 0, s, b);
+        return;
+    }
+    const bool kept = run == TopkRun::kKept;
+    if (!kept) hipLaunchKernelGGL(topk_init_batch_kernel<CAP>, dim3((unsigned)nb), threads, 0, s, b);
+    for (int pass = 0; pass < kPasses; ++pass)
+        hipLaunchKernelGGL(topk_hist_batch_kernel<CAP>, grid, threads, 0, s, b, pass, kept);
+    hipLaunchKernelGGL(topk_filter_batch_kernel<CAP>, grid, threads, 0, s, b, kept);
+}
 
 int topk_sparsify_batch(float* const* xs, const int64_t* numels, const int64_t* ks, int32_t count, void* workspace,
                         int64_t workspace_bytes, void* lists, void* stream, TopkRun run)
@@ -776,20 +814,16 @@ int topk_sparsify_batch(float* const* xs, const int64_t* numels, const int64_t* 
                       (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0))
         return CONEF_ERR_INVALID;
     hipStream_t s = (hipStream_t)stream;
-    char* ws = (char*)workspace;
     char* room = (char*)lists;
-    int i = 0;
-    while (i < count) {
-        TopkBatch b;
-        int nb = 0, wgs = 0;
-        for (; i < count && nb < kTopkBatchMax; ++i) {
-            char* mine = ws;
-            ws += kScratchBytes;
-            if (ks[i] >= numels[i]) continue;
-            TopkItem& it = b.item[nb];
+    TopkItem table[kTopkBatchMax];
+    int nb = 0;
+    for (int i = 0; i < count; ++i) {
+        if (ks[i] < numels[i]) {
+            TopkItem& it = table[nb++];
+            it = {};
             it.x = xs[i];
             it.numel = numels[i];
-            it.st = (TopkState*)mine;
+            it.st = (TopkState*)((char*)workspace + i * (int64_t)kScratchBytes);
             it.k = (uint32_t)ks[i];
             if (run == TopkRun::kListed) {
                 it.cap = (uint32_t)topk_segment(numels[i]);
@@ -798,30 +832,18 @@ int topk_sparsify_batch(float* const* xs, const int64_t* numels, const int64_t* 
                 it.list = (uint2*)(room + 8 * kTopkFinal + (4 * topk_hist_groups(numels[i]) + 255) / 256 * 256);
                 room += topk_list_bytes(numels[i]);
             }
-            b.first[nb] = wgs;
-            wgs += (int)topk_hist_groups(numels[i]);
-            ++nb;
         }
-        if (nb == 0) continue;
-        b.first[nb] = wgs;
-        b.count = nb;
-        const dim3 grid((unsigned)wgs), threads(256);
-        if (run == TopkRun::kListed) {
-            hipLaunchKernelGGL(topk_hist_batch_kernel, grid, threads, 0, s, b, 0, true);
-            hipLaunchKernelGGL(topk_note_batch_kernel, grid, threads, 0, s, b);
-            hipLaunchKernelGGL(topk_gather_batch_kernel, grid, threads, 0, s, b);
-            hipLaunchKernelGGL(topk_settle_batch_kernel, grid, threads, 0, s, b);
-            continue;
+        if (nb == kTopkBatchMax || (i + 1 == count && nb > 0)) {
+            if (nb <= kTopkBatchFew) topk_launch<kTopkBatchFew>(table, nb, run, s);
+            else topk_launch<kTopkBatchMax>(table, nb, run, s);
+            nb = 0;
         }
-        const bool kept = run == TopkRun::kKept;
-        if (!kept) hipLaunchKernelGGL(topk_init_batch_kernel, dim3((unsigned)nb), threads, 0, s, b);
-        for (int pass = 0; pass < kPasses; ++pass)
-            hipLaunchKernelGGL(topk_hist_batch_kernel, grid, threads, 0, s, b, pass, kept);
-        hipLaunchKernelGGL(topk_filter_batch_kernel, grid, threads, 0, s, b, kept);
     }
     return (int)hipGetLastError();
 }
 }  // namespace
+
+extern "C" {
 
 int conef_topk_sparsify_batch_f32(float* const* xs, const int64_t* numels, const int64_t* ks, int32_t count,
                                   void* workspace, int64_t workspace_bytes, void* stream)

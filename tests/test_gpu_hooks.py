@@ -1354,7 +1354,8 @@ def test_topk_with_lists_lent_by_the_caller():
     cases = list(_topk_inputs()) + [("narrow", near, 30_000), ("narrow, one stays", near, 1), ("narrow, one goes", near, 70_000),
                                     ("ties", repeated, rank_of + 300), ("many ties", crowd, rank_of + 500),
                                     ("infinities", inf, 20), ("denormals and zeros", zeros, 5000), ("only zeros go", zeros, 60_000)]
-    for batch in [[c] for c in cases] + [cases]:
+    # alone, as many as the small table of a launch holds and one more, and more than the large one holds
+    for batch in [[c] for c in cases] + [cases[:8], cases[:9], cases, (cases * 4)[:49]]:
         tensors, ks = [v.cuda() for _, v, _ in batch], [k for _, _, k in batch]
         ws = lists = None
         for call in range(3):
