@@ -113,7 +113,7 @@ class _BucketTable:
     sizes, payload slices and the item table the batch entry point reads.  Rebuilt when the
     bucket's buffer or layout changes."""
     __slots__ = ("key", "layout", "matrices", "uncompressed", "numels", "blocks", "offsets", "items", "count", "starts",
-                 "places", "staying", "plans", "moving", "need")
+                 "places", "moving", "need")
 
 
 def _build_table(state, grads, key, device, bucket_index, errors):
@@ -150,41 +150,32 @@ def _build_table(state, grads, key, device, bucket_index, errors):
 def _point_at_errors(state, t, errors):
     """The error memory's places in the item table.  ``t.moving``: the sketches that are not updated in
     place and swap two buffers, whose places a step takes anew; the others stay where they are."""
-    t.moving, t.need, t.plans, staying = [], 0, [], []
-    for it, error in zip(t.items, errors[:t.count]):
+    t.moving, t.need, moves = [], 0, []
+    errors = errors[:t.count]
+    for it, error in zip(t.items, errors):
         if not state.use_error_compression:
             it.err = error.data_ptr()
-            staying.append(error)
             continue
         plan = error.plan()
-        t.plans.append((error, plan))
         it.w = error.range
         it.plan_host, it.plan_dev = (plan.host_ptr, plan.device.data_ptr()) if plan is not None else (None, None)
         it.staging = None
-        if plan is not None and plan.in_place:
+        moves.append(plan is None or not plan.in_place)
+        if not moves[-1]:
             it.cs_in = it.cs_out = error.cs.data_ptr()
-            staying.append(error)
         else:
             t.moving.append((it, error, plan))
             # One staging buffer serves every binned sketch of the bucket (the launches run one after the
             # other on the stream): it is sized for the largest of them
             if plan is not None:
                 t.need = max(t.need, plan.workspace_bytes)
-    t.staying = staying if state.use_error_compression else None
-    t.places = _host.Places(staying)
+    t.places = _host.Sketches(errors, moves) if state.use_error_compression else _host.Places(errors)
 
 
 def _errors_moved(t, errors):
     """Whether a bucket's error memory is no longer where the table points: another tensor, the same one
     over other storage, another sketch, a sketch whose cells or plan were replaced."""
-    if t.places is None:
-        return True
-    if t.staying is None:                    # dense errors
-        return not t.places.same(errors if len(errors) == t.count else errors[:t.count])
-    for error, (known, plan) in zip(errors, t.plans):
-        if error is not known or error.plan() is not plan:
-            return True
-    return not t.places.same(t.staying)
+    return t.places is None or not t.places.same(errors if len(errors) == t.count else errors[:t.count])
 
 
 def RandomBlock_hook(state: RandomBlockState, bucket) -> torch.futures.Future[torch.Tensor]:

@@ -10,7 +10,6 @@ streaming passes over its memory: the error add is fused into the first product,
 import contextlib
 import ctypes
 import logging
-import operator
 import os
 
 import torch
@@ -137,7 +136,7 @@ class _RoundPlan:
     compressed, the table of matrices the batch entry points read, the views into the P / Q
     arenas.  Built on the first step of a bucket and reused while the bucket keeps its buffer
     and layout, so that a step costs a handful of foreign calls however many tensors it has."""
-    __slots__ = ("small", "layout", "errs_known", "cells", "cs_static", "env_ahead", "env_topk_side", "env_small", "key", "shapes", "work", "passthrough", "before", "after", "total_ps", "total_qs", "arena_key", "ps",
+    __slots__ = ("small", "layout", "cells", "cs_static", "env_ahead", "env_topk_side", "env_small", "key", "shapes", "work", "passthrough", "before", "after", "total_ps", "total_qs", "arena_key", "ps",
                  "qs", "items", "count", "sketches", "fused_sketch", "batched_update", "residual_offsets",
                  "topk_table", "q_next", "q_next_ptrs", "q_next_ready", "q_next_quads", "made", "q_next_event", "aside_recorded",
                  "topk_event", "topk_recorded", "ws_need", "handoff_event", "topk_number", "q_next_number", "is_wide", "wide", "chunks", "runs", "ef_spans")
@@ -182,8 +181,7 @@ def _build_round(state, grads, shapes, key, error_mode):
     plan = _RoundPlan()
     plan.key, plan.shapes = key, shapes
     plan.layout = _bucket.layout(grads)
-    plan.errs_known = None          # the bucket's sketches, and where their cells were, when the table was pointed at them
-    plan.cells = None
+    plan.cells = None               # the bucket's sketches as they were when the table was pointed at them
     plan.cs_static = False
     # switches read when the plan is built (a bucket's plan lives as long as its buffer does)
     plan.env_ahead = os.environ.get("CONEF_ROUND_AHEAD", "1") != "0"
@@ -243,15 +241,6 @@ def _build_round(state, grads, shapes, key, error_mode):
         off += n * m
     plan.residual_offsets.append(off)
     return plan
-
-
-def _sketches_moved(plan, errs):
-    """Whether the bucket's sketches are others than the table points at, or the same ones with their cells
-    elsewhere (sketches that swap two buffers are pointed at anew every step anyway)."""
-    known = plan.errs_known
-    if known is None or len(known) != len(errs) or not all(map(operator.is_, known, errs.values())):
-        return True
-    return plan.cs_static and not plan.cells.same(known)
 
 
 def _take_arenas(plan, p_mem, q_mem):
@@ -441,7 +430,8 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
                 errs[cnt] = torch.zeros_like(matrix)
             items[cnt].err = errs[cnt].data_ptr()
     elif error_mode == "conef":
-        if _sketches_moved(plan, errs):
+        # (the bucket's sketches, their plans, and the cells of those that are updated in place)
+        if plan.cells is None or not plan.cells.same(errs.values()):
             plan.sketches = []
             for cnt, (matrix, n, m, rank) in enumerate(work):
                 if cnt not in errs:
@@ -458,8 +448,7 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
             # sketches on row lists are updated in place.  The others swap two buffers, so their pointers
             # are refreshed every step.
             plan.cs_static = all(p is not None and p.in_place for _, p in plan.sketches)
-            plan.errs_known = list(errs.values())
-            plan.cells = _host.Places(plan.errs_known)
+            plan.cells = _host.Sketches(list(errs.values()), [p is None or not p.in_place for _, p in plan.sketches])
             for cnt, (cs, _) in enumerate(plan.sketches):
                 items[cnt].cs = cs.cs.data_ptr()
         if not plan.cs_static:

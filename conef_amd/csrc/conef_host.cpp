@@ -8,6 +8,20 @@
 // tables anew, which raises whatever there is to raise.
 #include <torch/csrc/autograd/python_variable.h>
 
+namespace {
+
+bool starts_at(PyObject* tensor, int64_t place)
+{
+    if (!THPVariable_Check(tensor)) return false;
+    try {
+        return (int64_t)(intptr_t)THPVariable_Unpack(tensor).data_ptr() == place;
+    } catch (...) {
+        return false;
+    }
+}
+
+}  // namespace
+
 extern "C" {
 
 // 1 if `tensors` (a list or tuple) holds tensors of the shapes in want[0 .. n): per tensor the number of
@@ -44,33 +58,44 @@ int conef_host_same_shapes(PyObject* tensors, const int64_t* want, int64_t n)
     return same;
 }
 
-// 1 if the memory of holders[i] - a tensor, or an object whose attribute `cs` is one - starts at places[i]
-// for every i below n, and there are n of them.
-int conef_host_same_places(PyObject* holders, const int64_t* places, int64_t n)
+// 1 if the memory of tensors[i] starts at places[i] for every i below n, and there are n of them.
+int conef_host_same_places(PyObject* tensors, const int64_t* places, int64_t n)
 {
-    static PyObject* const cells = PyUnicode_InternFromString("cs");
-    PyObject* seq = PySequence_Fast(holders, "");
+    PyObject* seq = PySequence_Fast(tensors, "");
     if (!seq) {
         PyErr_Clear();
         return 0;
     }
-    int same = cells && PySequence_Fast_GET_SIZE(seq) == (Py_ssize_t)n;
+    int same = PySequence_Fast_GET_SIZE(seq) == (Py_ssize_t)n;
+    for (int64_t i = 0; i < n && same; ++i) same = starts_at(PySequence_Fast_GET_ITEM(seq, i), places[i]);
+    Py_DECREF(seq);
+    return same;
+}
+
+// 1 if `sketches` holds the very objects of the list `known`, each with the object of the list `plans` as its
+// attribute _plan and its cells (attribute cs, a tensor) at places[i], where places[i] is not 0.
+int conef_host_same_sketches(PyObject* sketches, PyObject* known, PyObject* plans, const int64_t* places, int64_t n)
+{
+    static PyObject* const cells = PyUnicode_InternFromString("cs");
+    static PyObject* const plan = PyUnicode_InternFromString("_plan");
+    PyObject* seq = PySequence_Fast(sketches, "");
+    if (!seq) {
+        PyErr_Clear();
+        return 0;
+    }
+    int same = cells && plan && PyList_Check(known) && PyList_Check(plans) && PySequence_Fast_GET_SIZE(seq) == (Py_ssize_t)n &&
+               PyList_GET_SIZE(known) == (Py_ssize_t)n && PyList_GET_SIZE(plans) == (Py_ssize_t)n;
     for (int64_t i = 0; i < n && same; ++i) {
-        // (the exact type first: asking a sketch whether it is a tensor goes through Python)
         PyObject* o = PySequence_Fast_GET_ITEM(seq, i);
-        PyObject* inner = THPVariable_CheckExact(o) ? nullptr : PyObject_GetAttr(o, cells);
-        if (inner) {
-            o = inner;
-        } else {
-            PyErr_Clear();
-            Py_INCREF(o);
-        }
-        try {
-            same = THPVariable_Check(o) && (int64_t)(intptr_t)THPVariable_Unpack(o).data_ptr() == places[i];
-        } catch (...) {
-            same = 0;
-        }
-        Py_DECREF(o);
+        same = o == PyList_GET_ITEM(known, i);
+        if (!same) break;
+        PyObject* p = PyObject_GetAttr(o, plan);
+        same = p == PyList_GET_ITEM(plans, i);
+        Py_XDECREF(p);
+        if (!same || places[i] == 0) continue;
+        PyObject* t = PyObject_GetAttr(o, cells);
+        same = t && starts_at(t, places[i]);
+        Py_XDECREF(t);
     }
     Py_DECREF(seq);
     if (!same) PyErr_Clear();

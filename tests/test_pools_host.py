@@ -225,7 +225,7 @@ def test_random_block_errors_are_found_where_they_are_now():
 
     state.use_error_compression = True
     plan = SimpleNamespace(in_place=True, host_ptr=16, device=torch.zeros(4), workspace_bytes=0)
-    sketches = [SimpleNamespace(cs=torch.zeros(3, 4), range=4, plan=lambda: plan) for _ in range(2)]
+    sketches = [SimpleNamespace(cs=torch.zeros(3, 4), range=4, _plan=plan, plan=lambda: plan) for _ in range(2)]
     t = table(2)
     rb._point_at_errors(state, t, sketches)
     assert not rb._errors_moved(t, sketches)
@@ -233,26 +233,32 @@ def test_random_block_errors_are_found_where_they_are_now():
     assert rb._errors_moved(t, sketches)
     rb._point_at_errors(state, t, sketches)
     assert not rb._errors_moved(t, sketches) and t.items[1].cs_in == sketches[1].cs.data_ptr()
-    sketches[0].plan = lambda: None              # other hash seeds, say: the plan is another one
+    sketches[0]._plan = None                     # a sketch loaded from a checkpoint: the plan may be another one
     assert rb._errors_moved(t, sketches)
 
 
-def test_powersgd_sketches_are_found_where_they_are_now():
+def test_sketches_are_found_where_they_are_now():
     from types import SimpleNamespace
 
-    from conef_amd import _host, _psgd_engine as engine
+    from conef_amd import _host
 
-    sketches = [SimpleNamespace(cs=torch.zeros(3, 4)) for _ in range(2)]
-    plan = SimpleNamespace(cells=None, errs_known=None, cs_static=True)
+    plan = object()
+    sketches = [SimpleNamespace(cs=torch.zeros(3, 4), _plan=plan) for _ in range(3)]
     errs = dict(enumerate(sketches))
-    assert engine._sketches_moved(plan, errs)
-    plan.errs_known, plan.cells = sketches, _host.Places(sketches)
-    assert not engine._sketches_moved(plan, errs) and not engine._sketches_moved(plan, dict(errs))
-    assert engine._sketches_moved(plan, {})                                   # dropped by the caller
-    assert engine._sketches_moved(plan, {0: sketches[0], 1: SimpleNamespace(cs=sketches[1].cs)})
+    cells = _host.Sketches(sketches, [False, False, True])
+    assert cells.same(errs.values()) and cells.same(sketches) and cells.same(tuple(sketches))
+    assert not cells.same({}.values()) and not cells.same(sketches[:2]) and not cells.same(None)      # dropped by the caller
+    twin = SimpleNamespace(cs=sketches[1].cs, _plan=plan)
+    assert not cells.same([sketches[0], twin, sketches[2]])
+    sketches[2].cs = torch.ones(3, 4)            # the one that swaps two buffers
+    assert cells.same(sketches)
+    sketches[0]._plan = None
+    assert not cells.same(sketches)
+    sketches[0]._plan = plan
+    assert cells.same(sketches)
     sketches[1].cs.data = torch.ones(3, 4)
-    assert engine._sketches_moved(plan, errs)
+    assert not cells.same(sketches)
     sketches[1].cs = None                        # whatever is found there: the table is built anew, and says so
-    assert engine._sketches_moved(plan, errs)
-    plan.cs_static = False                       # pointed at anew every step
-    assert not engine._sketches_moved(plan, errs)
+    assert not cells.same(sketches)
+    del sketches[1].cs
+    assert not cells.same(sketches)
