@@ -169,13 +169,13 @@ def _point_at_errors(state, t, errors):
             # other on the stream): it is sized for the largest of them
             if plan is not None:
                 t.need = max(t.need, plan.workspace_bytes)
-    t.places = _host.Sketches(errors, moves) if state.use_error_compression else _host.Places(errors)
+    t.places = _host.same_sketches(errors, moves) if state.use_error_compression else _host.same_places(errors)
 
 
 def _errors_moved(t, errors):
     """Whether a bucket's error memory is no longer where the table points: another tensor, the same one
     over other storage, another sketch, a sketch whose cells or plan were replaced."""
-    return t.places is None or not t.places.same(errors if len(errors) == t.count else errors[:t.count])
+    return t.places is None or not t.places(errors if len(errors) == t.count else errors[:t.count])
 
 
 def RandomBlock_hook(state: RandomBlockState, bucket) -> torch.futures.Future[torch.Tensor]:
@@ -203,7 +203,7 @@ def RandomBlock_hook(state: RandomBlockState, bucket) -> torch.futures.Future[to
     key = (input_tensor.data_ptr(), input_tensor.numel(), bool(state.use_error_compression), state.compression_ratio,
            payload_all.data_ptr() if payload_all is not None else 0)
     table = state.round_cache.get(bucket_index)
-    if table is None or table.key != key or not table.layout.same(grads) or len(errors) < table.count:
+    if table is None or table.key != key or not table.layout(grads) or len(errors) < table.count:
         table = _build_table(state, grads, key, device, bucket_index, errors)
         payload_all = state.compressed_tensor_memory[bucket_index]
         table.key = key[:4] + (payload_all.data_ptr(),)

@@ -82,7 +82,7 @@ def UnbiasedRandomBlock_hook(state: UnbiasedRandomBlockState, bucket) -> torch.f
     key = (input_tensor.data_ptr(), input_tensor.numel(), state.compression_ratio,
            payload_all.data_ptr() if payload_all is not None else 0)
     table = state.round_cache.get(bucket_index)
-    if table is None or table[0] != key or not table[1].same(grads):
+    if table is None or table[0] != key or not table[1](grads):
         # worked out once per bucket: the >= 2-D gradients, their block sizes and the item table
         tensors = [g for g in grads if g.ndimension() > 1]
         uncompressed = [g for g in grads if g.ndimension() <= 1]

@@ -25,10 +25,10 @@ def is_last(bucket):
 
 
 def layout(grads):
-    """What a step compares (``.same(grads)``) to see that a bucket still has the tensors its cached tables
-    were made for: the shape of every one, in order.  The buffer's place and length go into the cache keys
-    beside it."""
-    return _host.Shapes(grads)
+    """What a step asks (``layout(grads)(grads_now)``) to see that a bucket still has the tensors its cached
+    tables were made for: the shape of every one, in order.  The buffer's place and length go into the cache
+    keys beside it."""
+    return _host.same_shapes(grads)
 
 
 def draw_starts(rng, numels, items, starts):

@@ -275,7 +275,7 @@ def plan_for(state, bucket_index, grads, key, error_mode, device, stream_now):
     round is about to run on (``stream_now()``) is ordered after a pending copy of the Q arena
     here, since the new plan no longer knows of it."""
     plan = state.round_cache.get(bucket_index)
-    if plan is None or plan.key != key or not plan.layout.same(grads):
+    if plan is None or plan.key != key or not plan.layout(grads):
         old = plan
         plan = _build_round(state, grads, [t.shape for t in grads], key, error_mode)
         if old is not None:
@@ -393,7 +393,7 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
     key = (base_ptr, total_length, error_mode, state.matrix_approximation_rank, state.min_compression_rate,
            getattr(state, "sketch_size", None), dense_err.data_ptr() if dense_err is not None else 0)
     plan = state.round_cache.get(bucket_index)
-    if plan is None or plan.key != key or not plan.layout.same(grads):
+    if plan is None or plan.key != key or not plan.layout(grads):
         plan = plan_for(state, bucket_index, grads, key, error_mode, device, lambda: _lib.current_stream(device))
     work, items, count = plan.work, plan.items, plan.count
     state.total_numel_before_compression += plan.before
@@ -431,7 +431,7 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
             items[cnt].err = errs[cnt].data_ptr()
     elif error_mode == "conef":
         # (the bucket's sketches, their plans, and the cells of those that are updated in place)
-        if plan.cells is None or not plan.cells.same(errs.values()):
+        if plan.cells is None or not plan.cells(errs.values()):
             plan.sketches = []
             for cnt, (matrix, n, m, rank) in enumerate(work):
                 if cnt not in errs:
@@ -448,7 +448,8 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
             # sketches on row lists are updated in place.  The others swap two buffers, so their pointers
             # are refreshed every step.
             plan.cs_static = all(p is not None and p.in_place for _, p in plan.sketches)
-            plan.cells = _host.Sketches(list(errs.values()), [p is None or not p.in_place for _, p in plan.sketches])
+            moves = [p is None or not p.in_place for _, p in plan.sketches]
+            plan.cells = _host.same_sketches(errs.values(), moves + [True] * (len(errs) - count))
             for cnt, (cs, _) in enumerate(plan.sketches):
                 items[cnt].cs = cs.cs.data_ptr()
         if not plan.cs_static:

@@ -34,7 +34,7 @@ HIPCC_FLAGS = [
 ]
 
 
-# checks on Python lists of tensors (host only, against torch's own libraries)
+# checks on Python lists of tensors (a CPython module, host only, against torch's own libraries)
 HOST_SOURCE, HOST_LIBPATH = "conef_host.cpp", os.path.join(LIBDIR, "libconef_host.so")
 
 

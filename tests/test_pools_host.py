@@ -187,12 +187,12 @@ def test_a_bucket_of_other_tensors_over_the_same_buffer_is_another_bucket():
     one = _views(flat, [(4, 8), (6, 4), (3,), (2, 2)])
     other = _views(flat, [(4, 8), (3,), (6, 4), (2, 2)])
     layout = _bucket.layout(one)
-    assert layout.same(_views(flat, [(4, 8), (6, 4), (3,), (2, 2)])) and layout.same(tuple(one))
+    assert layout(_views(flat, [(4, 8), (6, 4), (3,), (2, 2)])) and layout(tuple(one))
     for shapes in ([(4, 8), (4, 6), (3,), (2, 2)], [(4, 8), (24,), (3,), (2, 2)], [(4, 8), (6, 4), (3,)],
                    [(4, 8), (6, 4), (3,), (2, 2), ()], [(4, 8), (6, 4), (3, 1), (2, 2)], []):
-        assert not layout.same(_views(torch.zeros(100), shapes)), shapes
-    assert not layout.same(other) and not layout.same([1, 2, 3, 4]) and not layout.same(None)
-    assert _bucket.layout([]).same([]) and _bucket.layout([torch.zeros(())]).same([torch.ones(())])
+        assert not layout(_views(torch.zeros(100), shapes)), shapes
+    assert not layout(other) and not layout([1, 2, 3, 4]) and not layout(None)
+    assert _bucket.layout([])([]) and _bucket.layout([torch.zeros(())])([torch.ones(())])
     state = SimpleNamespace(round_cache={}, matrix_approximation_rank=1, min_compression_rate=0.1)
     main, device = FakeStream(41), torch.device("cpu")
     plan = engine.plan_for(state, 0, one, ("buffer",), None, device, lambda: main)
@@ -245,20 +245,20 @@ def test_sketches_are_found_where_they_are_now():
     plan = object()
     sketches = [SimpleNamespace(cs=torch.zeros(3, 4), _plan=plan) for _ in range(3)]
     errs = dict(enumerate(sketches))
-    cells = _host.Sketches(sketches, [False, False, True])
-    assert cells.same(errs.values()) and cells.same(sketches) and cells.same(tuple(sketches))
-    assert not cells.same({}.values()) and not cells.same(sketches[:2]) and not cells.same(None)      # dropped by the caller
+    cells = _host.same_sketches(sketches, [False, False, True])
+    assert cells(errs.values()) and cells(sketches) and cells(tuple(sketches))
+    assert not cells({}.values()) and not cells(sketches[:2]) and not cells(None)      # dropped by the caller
     twin = SimpleNamespace(cs=sketches[1].cs, _plan=plan)
-    assert not cells.same([sketches[0], twin, sketches[2]])
+    assert not cells([sketches[0], twin, sketches[2]])
     sketches[2].cs = torch.ones(3, 4)            # the one that swaps two buffers
-    assert cells.same(sketches)
+    assert cells(sketches)
     sketches[0]._plan = None
-    assert not cells.same(sketches)
+    assert not cells(sketches)
     sketches[0]._plan = plan
-    assert cells.same(sketches)
+    assert cells(sketches)
     sketches[1].cs.data = torch.ones(3, 4)
-    assert not cells.same(sketches)
+    assert not cells(sketches)
     sketches[1].cs = None                        # whatever is found there: the table is built anew, and says so
-    assert not cells.same(sketches)
+    assert not cells(sketches)
     del sketches[1].cs
-    assert not cells.same(sketches)
+    assert not cells(sketches)
