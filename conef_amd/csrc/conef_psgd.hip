@@ -3372,17 +3372,32 @@ int deferred_products(const PaddedRound& pr, int r, float* const* q_in, float* c
     return round_products_deferred<2>(pr, r, q_in, qi_in, alpha, eps, a, b, workspace, workspace_bytes, s, q_shares);
 }
 
-// Whether the Q factors of a bucket at ranks 9 to 32 go through the kernels that take column after column
-// (one launch, in place) instead of their Gram matrix (three launches).  Rank 16 and rank 32 have such
-// kernels of their own, a matrix a workgroup up to some 2000 rows and a few workgroups that meet above: six
-// factors [1024,32] take 26.4 us against 30.6, [4096,32] 29.7 against 33.4, [1024,16] 12.1 against 16.7,
-// [4096,16] 18.1 against 17.6 - and [8192,32] 69.6 against 38.4.  Between those ranks rows are padded and
-// the column kernels go by single floats: [1024,20] 59.9 us against 35.9.
+// Whether the Q factors of a bucket at ranks 9 to 32 go through the kernels that take column after column, in
+// place, instead of their Gram matrix (three launches).  Rank 16 and rank 32 have such kernels of their own, a
+// matrix a workgroup up to some 1024 rows and a few workgroups that meet above: six factors [1024,32] take
+// 26.4 us against 30.6, [4096,32] 29.7 against 33.4, [1024,16] 12.1 against 16.7, [4096,16] 18.1 against 17.6 -
+// and [8192,32] 69.6 against 38.4.  Where the factors' heights need several of those launches, one after the
+// other, the three are the shorter chain ([261,32] and [1000,32] in one bucket 20.2 and 26.1 us against 30).
+// Between those ranks rows are padded and the column kernels go by single floats: [1024,20] 59.9 us against 35.9.
 inline bool gs_wide_by_columns(const PaddedRound& pr)
 {
-    bool ok = pr.rp > 8 && !pr.padded;
-    for (const ConefPsgdItem& it : pr.items) ok = ok && it.m <= 4096;
-    return ok;
+    if (pr.rp <= 8 || pr.padded) return false;
+    bool tall = false;
+    int wgs = 0;
+    for (const ConefPsgdItem& it : pr.items) {
+        if (it.m > 4096 || !gsg_can(it.q, it.m, it.r)) return false;
+        tall = tall || gsg_wants(it.q, it.m, it.r);
+        int slab, w;
+        gsg_split(it.m, it.r, &slab, &w);
+        wgs += w;
+    }
+    if (tall) return wgs <= kGsgMaxWgs && (int)pr.items.size() <= kGsgMaxItems;      // the shorter ones come along
+    const GslChoice first = gsl_choose(pr.items[0].m, pr.rp);
+    for (const ConefPsgdItem& it : pr.items) {
+        const GslChoice c = gsl_choose(it.m, pr.rp);
+        if (c.kind != 1 || c.rpt != first.rpt) return false;
+    }
+    return true;
 }
 
 // mats[k], [items[k].m, r], in place
