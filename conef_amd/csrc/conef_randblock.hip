@@ -102,7 +102,7 @@ int conef_randblock_ef_step_f32(float* x, float* err, float* payload, int64_t nu
 {
     if (!block_args_ok(numel, start, block) || !x || !err || !payload) return CONEF_ERR_INVALID;
     ConefBlock blk = conef_make_block(numel, start, block);
-    hipLaunchKernelGGL(randblock_ef_kernel, dim3((unsigned)conef_rb_groups(numel)), dim3(256), 0, (hipStream_t)stream, x, err,
+    hipLaunchKernelGGL(randblock_ef_kernel, dim3((unsigned)conef_rb_groups(numel, kRbEfQuads)), dim3(256), 0, (hipStream_t)stream, x, err,
                        payload, numel, blk);
     return (int)hipGetLastError();
 }
@@ -112,7 +112,7 @@ int conef_randblock_unbiased_step_f32(float* x, float* payload, int64_t numel, i
 {
     if (!block_args_ok(numel, start, block) || !x || !payload || !(prob > 0.f)) return CONEF_ERR_INVALID;
     ConefBlock blk = conef_make_block(numel, start, block);
-    hipLaunchKernelGGL(randblock_unbiased_kernel, dim3((unsigned)conef_rb_groups(numel)), dim3(256), 0, (hipStream_t)stream, x,
+    hipLaunchKernelGGL(randblock_unbiased_kernel, dim3((unsigned)conef_rb_groups(numel, kRbUnbiasedQuads)), dim3(256), 0, (hipStream_t)stream, x,
                        payload, numel, blk, prob);
     return (int)hipGetLastError();
 }

@@ -159,7 +159,7 @@ int conef_randblock_step_batch_f32(const ConefRandBlockItem* items, int32_t coun
             // the reference divides by the Python double block / numel, which reaches the tensor as fp32
             d.prob = (float)((double)it.block / (double)numel);
             table.push_back(d);
-            blocks.push_back(conef_rb_groups(numel));
+            blocks.push_back(conef_rb_groups(numel, mode == 0 ? kRbUnbiasedQuads : kRbEfQuads));
         }
         if (mode == 0)
             return rb_run(table, blocks, [&](const auto& bt, int grid) {

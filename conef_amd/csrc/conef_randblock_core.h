@@ -4,25 +4,29 @@
 #pragma once
 #include "conef_device.h"
 
-// The tensor goes by tiles of kRbTile consecutive elements, kRbQuads column quads a thread, all of
-// them requested before the first is used.  A tile that holds none of the block - at the ratios that
-// compress, nine in ten - takes no test per element; in the others the block is two ranges of the tile,
-// and a quad inside one of them moves as a quad.  Pure streaming (dense error: 16 bytes an element,
-// unbiased: 4), bounded by memory.
-constexpr int kRbQuads = 4;
-constexpr int kRbTile = 256 * 4 * kRbQuads;
+// The tensor goes by tiles of 1024 consecutive elements a quad of every thread, all of a tile's quads
+// requested before the first is used.  A tile that holds none of the block - at the ratios that compress, nine
+// in ten - takes no test per element; in the others the block is two ranges of the tile, and a quad inside one
+// of them moves as a quad.  Pure streaming (dense error: 16 bytes an element, unbiased: 4), bounded by memory.
+// The dense step reads and writes, and workgroups that do one after the other overlap best when they are many and
+// short: with 1, 2 and 4 quads a thread 23.6, 24.8 and 28.1 us for 6.5 M elements, 171, 173 and 185 us for the
+// step of an LSTM (33278 x 650), 159, 157 and 163 us for WRN-28-10's.  The unbiased step only writes.
+constexpr int kRbEfQuads = 1, kRbUnbiasedQuads = 4;
+constexpr int conef_rb_tile(int quads) { return 256 * 4 * quads; }
 
 // The block's ranges [lo, hi) and [0, rest) relative to the tile at f0, and where in the payload the
 // tile's element 0 would sit as part of the one and of the other.
+template <int QUADS>
 struct RbTile {
+    static constexpr int kTile = conef_rb_tile(QUADS);
     int lo, hi, rest;
     int64_t at, at_rest;
     __device__ __forceinline__ RbTile(const ConefBlock& b, int64_t f0)
     {
         const int64_t l = b.start - f0, h = b.end - f0, r = b.rest - f0;
-        lo = l < 0 ? 0 : l > kRbTile ? kRbTile : (int)l;
-        hi = h < 0 ? 0 : h > kRbTile ? kRbTile : (int)h;
-        rest = r < 0 ? 0 : r > kRbTile ? kRbTile : (int)r;
+        lo = l < 0 ? 0 : l > kTile ? kTile : (int)l;
+        hi = h < 0 ? 0 : h > kTile ? kTile : (int)h;
+        rest = r < 0 ? 0 : r > kTile ? kTile : (int)r;
         at = f0 - b.start;
         at_rest = b.end - b.start + f0;
     }
@@ -40,24 +44,25 @@ __device__ __forceinline__ void
 conef_randblock_ef_body(float* __restrict__ x, float* __restrict__ err, float* __restrict__ payload, int64_t numel,
                         ConefBlock blk, int bx, int gx)
 {
-    const int64_t tiles = (numel + kRbTile - 1) / kRbTile;
+    constexpr int kTile = conef_rb_tile(kRbEfQuads);
+    const int64_t tiles = (numel + kTile - 1) / kTile;
     const float zero[4] = {0.f, 0.f, 0.f, 0.f};
     for (int64_t t = bx; t < tiles; t += gx) {
-        const int64_t f0 = t * kRbTile;
+        const int64_t f0 = t * kTile;
         float* xt = x + f0;
         float* et = err + f0;
-        const RbTile in(blk, f0);
-        if (f0 + kRbTile <= numel) {
-            float g[kRbQuads][4], e[kRbQuads][4];
+        const RbTile<kRbEfQuads> in(blk, f0);
+        if (f0 + kTile <= numel) {
+            float g[kRbEfQuads][4], e[kRbEfQuads][4];
 #pragma unroll
-            for (int u = 0; u < kRbQuads; ++u) {
+            for (int u = 0; u < kRbEfQuads; ++u) {
                 const int i = 4 * (threadIdx.x + 256 * u);
                 conef_ld4u(xt + i, g[u]);
                 conef_ld4u(et + i, e[u]);
             }
             const bool touched = in.touched();
 #pragma unroll
-            for (int u = 0; u < kRbQuads; ++u) {
+            for (int u = 0; u < kRbEfQuads; ++u) {
                 const int i = 4 * (threadIdx.x + 256 * u);
                 float xq[4];
 #pragma unroll
@@ -98,23 +103,24 @@ __device__ __forceinline__ void
 conef_randblock_unbiased_body(float* __restrict__ x, float* __restrict__ payload, int64_t numel, ConefBlock blk,
                               float prob, int bx, int gx)
 {
-    const int64_t tiles = (numel + kRbTile - 1) / kRbTile;
+    constexpr int kTile = conef_rb_tile(kRbUnbiasedQuads);
+    const int64_t tiles = (numel + kTile - 1) / kTile;
     const float zero[4] = {0.f, 0.f, 0.f, 0.f};
     for (int64_t t = bx; t < tiles; t += gx) {
-        const int64_t f0 = t * kRbTile;
+        const int64_t f0 = t * kTile;
         float* xt = x + f0;
-        const RbTile in(blk, f0);
-        if (f0 + kRbTile <= numel) {
+        const RbTile<kRbUnbiasedQuads> in(blk, f0);
+        if (f0 + kTile <= numel) {
             if (!in.touched()) {
 #pragma unroll
-                for (int u = 0; u < kRbQuads; ++u) conef_st4u(xt + 4 * (threadIdx.x + 256 * u), zero);
+                for (int u = 0; u < kRbUnbiasedQuads; ++u) conef_st4u(xt + 4 * (threadIdx.x + 256 * u), zero);
                 continue;
             }
-            float g[kRbQuads][4];
+            float g[kRbUnbiasedQuads][4];
 #pragma unroll
-            for (int u = 0; u < kRbQuads; ++u) conef_ld4u(xt + 4 * (threadIdx.x + 256 * u), g[u]);
+            for (int u = 0; u < kRbUnbiasedQuads; ++u) conef_ld4u(xt + 4 * (threadIdx.x + 256 * u), g[u]);
 #pragma unroll
-            for (int u = 0; u < kRbQuads; ++u) {
+            for (int u = 0; u < kRbUnbiasedQuads; ++u) {
                 const int i = 4 * (threadIdx.x + 256 * u);
                 if (in.whole(i)) {
 #pragma unroll
@@ -148,8 +154,8 @@ conef_randblock_unbiased_body(float* __restrict__ x, float* __restrict__ payload
 }
 
 // workgroups of a tensor of `numel` elements
-inline int conef_rb_groups(int64_t numel)
+inline int conef_rb_groups(int64_t numel, int quads)
 {
-    const int64_t g = (numel + kRbTile - 1) / kRbTile;
+    const int64_t g = (numel + conef_rb_tile(quads) - 1) / conef_rb_tile(quads);
     return (int)(g < 1 ? 1 : g > 16384 ? 16384 : g);
 }
