@@ -658,12 +658,16 @@ topk_settle_batch_kernel(TopkBatch<CAP> b)
 // Workgroups of a pass over a tensor.  A histogram workgroup ends with one global atomic per bin
 // it touched, all workgroups on the same few dozen counters, and a filter workgroup that has to
 // settle ties ends with one on a single counter: fewer workgroups with longer loops (16 quads a
-// thread) beat many short ones.
-inline int64_t topk_hist_groups(int64_t numel)
+// thread) beat many short ones.  At most 512 where three such passes read the tensor (31 M elements 141 us,
+// 164 with 1024), 1024 where there is one and the note pass, which ends with no shared counter but the
+// second digit's, gains from them.
+inline int64_t topk_groups(int64_t numel, int64_t most)
 {
-    int64_t g = (numel + 255) / 256 / 64;
-    return g < 1 ? 1 : g > 1024 ? 1024 : g;
+    const int64_t g = (numel + 255) / 256 / 64;
+    return g < 1 ? 1 : g > most ? most : g;
 }
+inline int64_t topk_hist_groups(int64_t numel) { return topk_groups(numel, 512); }
+inline int64_t topk_listed_groups(int64_t numel) { return topk_groups(numel, 1024); }
 
 
 // ---- selection state of the entry point that allocates nothing ------------------------------
@@ -735,14 +739,14 @@ namespace {
 // candidates a workgroup of the note pass has room for: a quarter of its elements
 inline int64_t topk_segment(int64_t numel)
 {
-    const int64_t g = topk_hist_groups(numel);
+    const int64_t g = topk_listed_groups(numel);
     return ((numel + g - 1) / g / 4 + 63) / 64 * 64;
 }
 
 // a tensor's part of the lists: the gathered keys, the workgroups' counts, their segments
 inline int64_t topk_list_bytes(int64_t numel)
 {
-    const int64_t g = topk_hist_groups(numel);
+    const int64_t g = topk_listed_groups(numel);
     return 8 * kTopkFinal + (4 * g + 255) / 256 * 256 + g * topk_segment(numel) * 8;
 }
 }  // namespace
@@ -785,7 +789,7 @@ void topk_launch(const TopkItem* items, int nb, TopkRun run, hipStream_t s)
     for (int k = 0; k < nb; ++k) {
         b.item[k] = items[k];
         b.first[k] = wgs;
-        wgs += (int)topk_hist_groups(items[k].numel);
+        wgs += (int)(run == TopkRun::kListed ? topk_listed_groups(items[k].numel) : topk_hist_groups(items[k].numel));
     }
     b.first[nb] = wgs;
     b.count = nb;
@@ -829,7 +833,7 @@ int topk_sparsify_batch(float* const* xs, const int64_t* numels, const int64_t* 
                 it.cap = (uint32_t)topk_segment(numels[i]);
                 it.final_idx = (uint32_t*)room;
                 it.counts = it.final_idx + 2 * kTopkFinal;
-                it.list = (uint2*)(room + 8 * kTopkFinal + (4 * topk_hist_groups(numels[i]) + 255) / 256 * 256);
+                it.list = (uint2*)(room + 8 * kTopkFinal + (4 * topk_listed_groups(numels[i]) + 255) / 256 * 256);
                 room += topk_list_bytes(numels[i]);
             }
         }
