@@ -1049,6 +1049,8 @@ struct PqtItem {
     const float* qi;         // not null: q laid out by quads (conef_load_slices)
 };
 
+typedef __attribute__((address_space(4))) float conef_cfloat;      // constant memory: uniform loads are scalar
+
 inline int pqt_lanes(int64_t m)
 {
     const int64_t m4 = (m + 3) / 4;
@@ -1056,7 +1058,9 @@ inline int pqt_lanes(int64_t m)
 }
 
 template <int RP, int MODE, bool UNIFORM>
-__device__ __forceinline__ void psgd_pqt_rows(const PqtItem& it, int bx, int by)
+__device__ __forceinline__ void
+psgd_pqt_rows(float* __restrict__ x, float* __restrict__ err, const float* __restrict__ p, const float* __restrict__ q,
+              const float* __restrict__ qi, const PqtItem& it, int bx, int by)
 {
     const int m = it.m, groups = 256 / it.lanes;
     int grp = (int)threadIdx.x / it.lanes;
@@ -1067,37 +1071,57 @@ __device__ __forceinline__ void psgd_pqt_rows(const PqtItem& it, int bx, int by)
     const int64_t i0 = (int64_t)by * it.rows_per_slab;
     const int64_t i1 = i0 + it.rows_per_slab < it.n ? i0 + it.rows_per_slab : it.n;
     float qf[4 * RP];
-    conef_load_slices<RP>(conef_quad_slices<RP>(it.q, it.qi, quad, col, m), qf);
-    for (int64_t ib = i0 + grp; ib < i1; ib += 4 * groups) {
-        float xv[4][4];
-        if (MODE == 1) {
+    conef_load_slices<RP>(conef_quad_slices<RP>(q, qi, quad, col, m), qf);
+    auto walk = [&](auto store) {
+        for (int64_t ib = i0 + grp; ib < i1; ib += 4 * groups) {
+            float xv[4][4];
+            if (MODE == 1) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int64_t i = ib + u * groups < i1 ? ib + u * groups : ib;
+                    conef_ld4u(x + i * m + col, xv[u]);
+                }
+            }
+            // The four rows of P: through constant memory where they are uniform.  (The pointers come out of a table:
+            // nothing else tells the compiler that the stores leave P alone, and the rows became vector loads
+            // behind them.)
+            float pv[4][RP];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const int64_t i = ib + u * groups < i1 ? ib + u * groups : ib;
-                conef_ld4u(it.x + i * m + col, xv[u]);
+                if (UNIFORM) {
+                    const conef_cfloat* ps = (const conef_cfloat*)(uintptr_t)(p + i * RP);
+#pragma unroll
+                    for (int c = 0; c < RP; ++c) pv[u][c] = ps[c];
+                } else {
+#pragma unroll
+                    for (int c = 0; c < RP; ++c) pv[u][c] = p[i * RP + c];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int64_t i = ib + u * groups;
+                if (i >= i1) break;
+                float mh[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int c = 0; c < RP; ++c) {
+                    const float pc = pv[u][c];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) mh[k] = fmaf(pc, qf[k * RP + c], mh[k]);
+                }
+                if (MODE == 1) {
+                    float ev[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) ev[k] = __fsub_rn(xv[u][k], mh[k]);
+                    store(err + i * m + col, ev);
+                }
+                store(x + i * m + col, mh);
             }
         }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int64_t i = ib + u * groups;
-            if (i >= i1) break;
-            const float* pi = it.p + i * RP;
-            float mh[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int c = 0; c < RP; ++c) {
-                const float pc = pi[c];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) mh[k] = fmaf(pc, qf[k * RP + c], mh[k]);
-            }
-            if (MODE == 1) {
-                float ev[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) ev[k] = __fsub_rn(xv[u][k], mh[k]);
-                conef_st4_own(it.err + i * m + col, ev, dup);
-            }
-            conef_st4_own(it.x + i * m + col, mh, dup);
-        }
-    }
+    };
+    // (rows of whole quads have a loop without the moved quad's test; uniform)
+    if (m % 4 == 0) walk([](float* at, const float* v) { conef_st4u(at, v); });
+    else walk([&](float* at, const float* v) { conef_st4_own(at, v, dup); });
 }
 
 // The general form: any rank up to RP, element by element.
@@ -1147,8 +1171,8 @@ __device__ __forceinline__ void psgd_pqt_item(const PqtItem& it, int local)
 {
     const int bx = local % it.col_tiles, by = local / it.col_tiles;
     if (!FAST) psgd_pqt_body<RP, MODE>(it.x, it.err, it.p, it.q, it.n, it.m, it.r, it.rows_per_slab, bx, by);
-    else if (it.lanes % 64 == 0) psgd_pqt_rows<RP, MODE, true>(it, bx, by);
-    else psgd_pqt_rows<RP, MODE, false>(it, bx, by);
+    else if (it.lanes % 64 == 0) psgd_pqt_rows<RP, MODE, true>(it.x, it.err, it.p, it.q, it.qi, it, bx, by);
+    else psgd_pqt_rows<RP, MODE, false>(it.x, it.err, it.p, it.q, it.qi, it, bx, by);
 }
 
 template <int RP, int MODE, bool FAST>
@@ -1158,6 +1182,14 @@ psgd_pqt_batch_kernel(PsgdBatch<PqtItem> b)
     int local;
     const PqtItem& it = b.item[psgd_batch_locate(b, &local)];
     psgd_pqt_item<RP, MODE, FAST>(it, local);
+}
+
+// one matrix of rank RP, rows of at least four columns
+template <int RP, int MODE>
+__global__ void __launch_bounds__(256)
+psgd_pqt_one_kernel(PqtItem it)
+{
+    psgd_pqt_item<RP, MODE, true>(it, (int)blockIdx.x);
 }
 
 // Front of the row-list sketch kernel: the value to sketch is the residual X - P Q^T, and M is
@@ -2355,12 +2387,27 @@ static int launch_pqt(float* x, float* err, const float* p, const float* q, int6
         }
         return (int)hipGetLastError();
     }
-    if (r <= 8 && r == rank_bound(r) && m >= 4) {
-        ConefPsgdItem it = {};
-        it.x = x; it.err = err; it.p = const_cast<float*>(p); it.q = const_cast<float*>(q); it.n = n; it.m = m; it.r = r;
-        return pqt_batch(&it, 1, err ? 1 : 0, 0.f, 0, 0, s);
-    }
     int64_t col_tiles = (m + 1023) / 1024;
+    if (r <= 8 && r == rank_bound(r) && m >= 4) {
+        // One matrix is a kernel's arguments, not a table of 24 (1.7 KB, 2 us a launch), and Q comes row-major: about
+        // a thousand workgroups, so that one reads its slice of Q for as many rows as that leaves it
+        // ([30522,1024] at rank 8 33 us; with the eight rows a batch gives it, whose Q lies by quads, 45).
+        const int lanes = pqt_lanes(m), per_trip = 4 * (256 / lanes);
+        const int64_t slabs = (1024 + col_tiles - 1) / col_tiles;
+        int64_t rows = (n + slabs - 1) / slabs;
+        if (rows < per_trip) rows = per_trip;
+        const PqtItem it = {x, err, p, q, n, (int)m, r, (int)rows, (int)col_tiles, lanes, nullptr};
+        const dim3 grid((unsigned)(col_tiles * ((n + rows - 1) / rows)));
+#define CONEF_PQ1(RP)                                                                                       \
+    do {                                                                                                    \
+        if (RP >= 16) break;                                                                                \
+        if (err) hipLaunchKernelGGL((psgd_pqt_one_kernel<(RP < 16 ? RP : 8), 1>), grid, dim3(256), 0, s, it); \
+        else hipLaunchKernelGGL((psgd_pqt_one_kernel<(RP < 16 ? RP : 8), 0>), grid, dim3(256), 0, s, it);     \
+    } while (0)
+        CONEF_RANK_SWITCH(r, CONEF_PQ1)
+#undef CONEF_PQ1
+        return (int)hipGetLastError();
+    }
     int64_t slabs = (1024 + col_tiles - 1) / col_tiles;       // about a thousand workgroups ...
     int64_t rps = (n + slabs - 1) / slabs;
     if (rps < 4) rps = 4;                                     // ... of at least four rows
