@@ -95,20 +95,23 @@ def topk_sparsify(err, topk_ratio, workspace=None):
 class _TopkTable(tuple):
     """(tensors' places, pointers, element counts, how many stay, selection state, ratio)"""
     list_bytes = 0
+    stream = None       # the raw stream the selection state was allocated and cleared on, the only one it is used on
 
 
 def topk_sparsify_all(tensors, topk_ratio, table=None, side=None):
     """``topk_sparsify`` of every tensor of a list (one stream, one device) with each pass a
     single launch over all of them.  ``table`` is what an earlier call over the same tensors
-    returned: the host arrays and the selection state are reused while the tensors stay where they are.
+    returned: the host arrays and the selection state are reused while the tensors stay where they are
+    and the calls on one stream.
     ``side``: the torch Stream to launch on (the current one if None)."""
     count = len(tensors)
     if count == 0:
         return table
-    key = tuple(t.data_ptr() for t in tensors)
     lib = _lib.load()
     device = tensors[0].device
-    if table is None or table[0] != key:
+    stream = _lib.stream_ptr(tensors[0]) if side is None else side.cuda_stream
+    if topk_table_is_stale(table, tensors, topk_ratio) or table.stream != stream:
+        key = tuple(t.data_ptr() for t in tensors)
         for t in tensors:
             _lib.require_device_f32(t, "err")
         ptrs = (ctypes.c_void_p * count)(*key)
@@ -120,10 +123,8 @@ def topk_sparsify_all(tensors, topk_ratio, table=None, side=None):
             ws = torch.zeros(lib.conef_topk_batch_workspace_bytes(numels, count), dtype=torch.uint8, device=device)
         table = _TopkTable((key, ptrs, numels, ks, ws, topk_ratio))
         table.list_bytes = lib.conef_topk_batch_list_bytes(numels, count)
-    elif table[5] != topk_ratio:
-        return topk_sparsify_all(tensors, topk_ratio, None, side)
+        table.stream = stream
     _, ptrs, numels, ks, ws, _ = table
-    stream = _lib.stream_ptr(tensors[0]) if side is None else side.cuda_stream
     lists = _workspace(device, stream, table.list_bytes, side)
     rc = lib.conef_topk_sparsify_batch_listed_f32(ptrs, numels, ks, count, ws.data_ptr(), ws.numel(), lists.data_ptr(),
                                                   lists.numel(), stream)
@@ -139,7 +140,7 @@ class _RoundPlan:
     __slots__ = ("small", "layout", "cells", "cs_static", "env_ahead", "env_topk_side", "env_small", "key", "shapes", "work", "passthrough", "before", "after", "total_ps", "total_qs", "arena_key", "ps",
                  "qs", "items", "count", "sketches", "fused_sketch", "batched_update", "residual_offsets",
                  "topk_table", "q_next", "q_next_ptrs", "q_next_ready", "q_next_quads", "made", "q_next_event", "aside_recorded",
-                 "topk_event", "topk_recorded", "ws_need", "handoff_event", "topk_number", "q_next_number", "is_wide", "wide", "chunks", "runs", "ef_spans")
+                 "topk_event", "ws_need", "handoff_event", "topk_number", "q_next_number", "is_wide", "wide", "chunks", "runs", "ef_spans")
 
 
 # flags of conef_psgd_round_ahead_f32 (include/conef_hip.h)
@@ -218,7 +219,6 @@ def _build_round(state, grads, shapes, key, error_mode):
     plan.batched_update = False
     plan.topk_table = None
     plan.topk_event = None          # the side stream's top-k of this bucket's errors, to be waited for by its next round
-    plan.topk_recorded = None       # the side stream (raw) that the errors are known to the allocator to be used on
     plan.topk_number = None         # the side stream's running number of that top-k (None: nothing to wait for)
     plan.q_next_number = None       # likewise for the Gram-Schmidt of the next round's Q factors
     plan.ws_need = None             # bytes of workspace the batch entry points ask for (a function of the table's shapes)
@@ -428,6 +428,7 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
         for cnt, (matrix, n, m, rank) in enumerate(work):
             if cnt not in errs:
                 errs[cnt] = torch.zeros_like(matrix)
+                plan.topk_table = None       # perhaps at the address of a dropped one, and yet another allocation
             items[cnt].err = errs[cnt].data_ptr()
     elif error_mode == "conef":
         # (the bucket's sketches, their plans, and the cells of those that are updated in place)
@@ -584,25 +585,7 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
             # The sparsification only touches the error tensors, which nobody reads before this bucket's
             # next round: it runs on a side stream while this stream goes on with the next bucket
             # (streaming passes next to launches that are mostly latency).  Same kernels, same values.
-            if plan.handoff_event is None:
-                plan.handoff_event = torch.cuda.Event()
-            plan.handoff_event.record(_lib.current_stream(device))
-            side = _pools.side_stream(device, 0, 1)
-            side.wait_event(plan.handoff_event)
-            tensors = [errs[cnt] for cnt in range(count)]
-            if topk_table_is_stale(plan.topk_table, tensors, state.topk_ratio) or plan.topk_recorded != side.cuda_stream:
-                # a new table (an error tensor was replaced, another ratio), another stream: memory the side
-                # stream works on must not go back to the allocator under it
-                plan.topk_table = topk_sparsify_all(tensors, state.topk_ratio, None, side)
-                for t in tensors:
-                    t.record_stream(side)
-                plan.topk_recorded = side.cuda_stream
-            else:
-                plan.topk_table = topk_sparsify_all(tensors, state.topk_ratio, plan.topk_table, side)
-            if plan.topk_event is None:
-                plan.topk_event = torch.cuda.Event()
-            plan.topk_event.record(side)
-            plan.topk_number = _pools.side_recorded(device, plan.topk_event)
+            _sparsify_aside(plan, [errs[cnt] for cnt in range(count)], state.topk_ratio, device)
         else:
             plan.topk_table = topk_sparsify_all([errs[cnt] for cnt in range(count)], state.topk_ratio, plan.topk_table)
     elif residual is not None and mode3 != 3:
@@ -624,6 +607,26 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
 def _at(array, index):
     """The ctypes array from entry ``index`` on, as an argument."""
     return ctypes.byref(array, index * ctypes.sizeof(array._type_))
+
+
+def _sparsify_aside(plan, tensors, topk_ratio, device):
+    """The top-k of a bucket's error tensors on the side stream, which the bucket's next round waits for."""
+    if plan.handoff_event is None:
+        plan.handoff_event = torch.cuda.Event()
+    plan.handoff_event.record(_lib.current_stream(device))
+    side = _pools.side_stream(device, 0, 1)
+    side.wait_event(plan.handoff_event)
+    table = topk_sparsify_all(tensors, topk_ratio, plan.topk_table, side)
+    if table is not plan.topk_table:
+        # a new table (an error tensor was replaced, another ratio, a round on another stream before): memory
+        # the side stream works on must not go back to the allocator under it
+        plan.topk_table = table
+        for t in tensors:
+            t.record_stream(side)
+    if plan.topk_event is None:
+        plan.topk_event = torch.cuda.Event()
+    plan.topk_event.record(side)
+    plan.topk_number = _pools.side_recorded(device, plan.topk_event)
 
 
 def _orthogonalise_q_aside(plan, lib, eps, ws_len, device):

@@ -167,6 +167,67 @@ def test_every_buffer_the_side_stream_works_on_is_known_to_the_allocator(monkeyp
         _pools._SIDE_ORDER.pop(device, None)
 
 
+def test_errors_the_side_stream_sparsifies_are_known_to_the_allocator(monkeypatch):
+    """hPowerSGD's top-k works on a bucket's error tensors on the side stream or, with several hook streams,
+    on the round's own.  New tensors have to be recorded on the side stream whenever they get there, also
+    when a round of the other kind saw them first, and the selection state (zeroed by one stream's
+    kernels for the next call) stays with one stream."""
+    from contextlib import nullcontext
+    from types import SimpleNamespace
+
+    from conef_amd import _lib, _psgd_engine as engine
+
+    class Err:
+        def __init__(self, place):
+            self.place, self.recorded_on, self.device = place, [], device
+
+        def data_ptr(self):
+            return self.place
+
+        def numel(self):
+            return 100
+
+        def record_stream(self, stream):
+            self.recorded_on.append(stream)
+
+    device, main, side = torch.device("cpu"), FakeStream(51), FakeStream(52)
+    launches = []
+    lib = SimpleNamespace(conef_topk_batch_workspace_bytes=lambda *a: 64, conef_topk_batch_list_bytes=lambda *a: 32,
+                          conef_topk_sparsify_batch_listed_f32=lambda *a: launches.append((a[-1], a[4])) or 0)
+    monkeypatch.setattr(torch.cuda, "Event", FakeEvent)
+    monkeypatch.setattr(_lib, "load", lambda: lib)
+    monkeypatch.setattr(_lib, "require_device_f32", lambda t, name: None)
+    monkeypatch.setattr(_lib, "current_stream", lambda dev: main)
+    monkeypatch.setattr(_lib, "stream_ptr", lambda t: main.cuda_stream)
+    monkeypatch.setattr(_lib, "on_stream", lambda stream: nullcontext())
+    monkeypatch.setattr(_pools, "side_stream", lambda dev, index, count: side)
+    monkeypatch.setattr(engine, "_workspace", lambda dev, stream, nbytes, on=None: torch.zeros(8))
+    _pools._SIDE_ORDER.pop(device, None)
+    try:
+        state = SimpleNamespace(round_cache={}, matrix_approximation_rank=1, min_compression_rate=2)
+        plan = engine._build_round(state, [torch.zeros(64, 96)], [(64, 96)], ("key",), "topk")
+        first, second = [Err(1000), Err(2000)], [Err(3000), Err(4000)]
+
+        def aside(errs):
+            engine._sparsify_aside(plan, errs, 0.4, device)
+
+        aside(first)
+        aside(first)
+        assert [e.recorded_on for e in first] == [[side]] * 2           # once is enough
+        assert launches[0] == launches[1] and launches[0][0] == side.cuda_stream
+        # a caller replaced the errors and went to several hook streams for a round, then back
+        plan.topk_table = engine.topk_sparsify_all(second, 0.4, plan.topk_table)
+        assert [e.recorded_on for e in second] == [[]] * 2
+        aside(second)
+        assert [e.recorded_on for e in second] == [[side]] * 2
+        # the same tensors on another stream: a selection state of that stream's own
+        kept = plan.topk_table
+        plan.topk_table = engine.topk_sparsify_all(second, 0.4, plan.topk_table)
+        assert plan.topk_table is not kept and launches[-1][0] == main.cuda_stream and launches[-1][1] != launches[-2][1]
+    finally:
+        _pools._SIDE_ORDER.pop(device, None)
+
+
 def _views(flat, shapes):
     out, off = [], 0
     for shape in shapes:
