@@ -9,7 +9,7 @@
 //   stage   the values to be sketched are produced in column order with 16-byte accesses and
 //           parked in LDS; whatever the fused step has to do in column order (payload, writing
 //           the decompressed gradient, the low-rank product) happens here;
-//   gather  one thread per (row, bucket) walks the bucket's list, picks its values out of LDS
+//   gather  a thread walks a bucket's list for a row or two, picks its values out of LDS
 //           and adds the terms in ascending column order, several entries a trip; buckets are
 //           handed out in the order of falling list length (a table of the plan), so that the
 //           lanes of a wave have lists of about the same length to walk.
@@ -449,6 +449,52 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
     // bucket on neighbouring lanes: the lanes of a wave walk lists of about the same length (a wave
     // takes as many trips as its longest list).
     constexpr int kWalk = 4;
+    // A tile with more (bucket, row) pairs than threads: a thread walks a bucket's list for two rows, an entry
+    // is taken apart once for both.  Update and random-block step, one row and two rows a thread: [33278,650]
+    // 24.0 and 22.5, 38.5 and 37.3 us; [30522,1024] 33.1 and 31.9, 54.0 and 52.6; [6144,1024] 10.9 and 10.2, 17.5 and
+    // 16.8; [9000,333] with 166 buckets 9.9 and 8.7, 13.3 and 12.2.  Four rows were slower than two everywhere
+    // ([33278,650] 25.4), and two lose where they leave threads without work ([20000,300] with 15 buckets 9.0
+    // and 9.7).
+    if (sizeof(CsT) == sizeof(float) && rows >= 2 && total > kConefRowlistThreads) {
+        constexpr int kTrip = 2;
+        const int per = (rows + 1) >> 1, items = per * w;
+        int jj = threadIdx.x / per, rg = threadIdx.x - jj * per;
+        const int sjj = kConefRowlistThreads / per, srg = kConefRowlistThreads - sjj * per;
+        for (int p = threadIdx.x; p < items; p += kConefRowlistThreads) {
+            const int j = ord_l[jj], ra = 2 * rg, rb2 = ra + 1 < rows ? ra + 1 : ra;
+            const uint32_t e0 = csr_l[j], e1 = csr_l[j + 1];
+            const float *va = vals + ra * d, *vb = vals + rb2 * d;
+            float acc_a = cells[ra * w + j], acc_b = cells[rb2 * w + j];
+            const double decay_a = __dmul_rn(one_minus_beta, (double)acc_a), decay_b = __dmul_rn(one_minus_beta, (double)acc_b);
+            for (uint32_t e = e0; e < e1; e += kTrip) {
+                uint32_t en[kTrip];
+                float ta[kTrip], tb[kTrip];
+#pragma unroll
+                for (int u = 0; u < kTrip; ++u) en[u] = ent_l[e + u < e1 ? e + u : e1 - 1];
+#pragma unroll
+                for (int u = 0; u < kTrip; ++u) {
+                    const uint32_t at = en[u] & 0x7fffu, flip = ((~en[u]) & 0x8000u) << 16;      // sign bit clear (-1): flip the float's sign
+                    ta[u] = (float)__dsub_rn((double)__uint_as_float(__float_as_uint(va[at]) ^ flip), decay_a);
+                    tb[u] = (float)__dsub_rn((double)__uint_as_float(__float_as_uint(vb[at]) ^ flip), decay_b);
+                }
+#pragma unroll
+                for (int u = 0; u < kTrip; ++u)
+                    if (e + u < e1) {
+                        acc_a = __fadd_rn(acc_a, ta[u]);
+                        acc_b = __fadd_rn(acc_b, tb[u]);
+                    }
+            }
+            conef_st(cs_out + (row0 + ra) * w + j, acc_a);
+            if (rb2 != ra) conef_st(cs_out + (row0 + rb2) * w + j, acc_b);
+            jj += sjj;
+            rg += srg;
+            if (rg >= per) {
+                rg -= per;
+                ++jj;
+            }
+        }
+        return;
+    }
     int jj = threadIdx.x / rows, row = threadIdx.x - jj * rows;
     const int sjj = kConefRowlistThreads / rows, srow = kConefRowlistThreads - sjj * rows;
     for (int p = threadIdx.x; p < total; p += kConefRowlistThreads) {
