@@ -139,12 +139,13 @@ class _RoundPlan:
     and layout, so that a step costs a handful of foreign calls however many tensors it has."""
     __slots__ = ("small", "layout", "cells", "cs_static", "env_ahead", "env_topk_side", "env_small", "key", "shapes", "work", "passthrough", "before", "after", "total_ps", "total_qs", "arena_key", "ps",
                  "qs", "items", "count", "sketches", "fused_sketch", "batched_update", "residual_offsets",
-                 "topk_table", "q_next", "q_next_ptrs", "q_next_ready", "q_next_quads", "made", "q_next_event", "aside_recorded",
+                 "topk_table", "q_next", "q_next_ptrs", "q_next_ready", "q_next_quads", "q_next_fold", "made", "q_next_event", "aside_recorded",
                  "topk_event", "ws_need", "handoff_event", "topk_number", "q_next_number", "is_wide", "wide", "chunks", "runs", "ef_spans")
 
 
 # flags of conef_psgd_round_ahead_f32 (include/conef_hip.h)
 _ROUND_Q_READY, _ROUND_MAKE_NEXT, _ROUND_NEXT_QUADS, _ROUND_NEXT_WIDE, _ROUND_QUADS_READY = 1, 2, 4, 8, 16
+_ROUND_NEXT_FOLD, _ROUND_FOLD_READY = 32, 64
 
 BATCH_ITEMS = 24        # matrices the batch entry points take into one launch
 
@@ -227,7 +228,7 @@ def _build_round(state, grads, shapes, key, error_mode):
     # round (conef_psgd_round_ahead_f32).  Derived data: q_memory_dict keeps what the reference
     # keeps, and the flag falls with the plan whenever the state is replaced.
     plan.q_next = plan.q_next_ptrs = None
-    plan.q_next_ready = plan.q_next_quads = False
+    plan.q_next_ready = plan.q_next_quads = plan.q_next_fold = False
     plan.made = None
     plan.q_next_event = None
     plan.aside_recorded = None      # the side stream (raw) that q_next and the Q arena are known to the allocator to be used on
@@ -446,6 +447,10 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
             plan.batched_update = all(p is not None and p.batchable for _, p in plan.sketches)
             plan.fused_sketch = state.matrix_approximation_rank <= 8 and plan.batched_update
             plan.small = None
+            plan.ws_need = None
+            plan.q_next = None               # sized for the sketches, and holds sums over their buckets
+            plan.q_next_ready = False
+            plan.aside_recorded = None
             # sketches on row lists are updated in place.  The others swap two buffers, so their pointers
             # are refreshed every step.
             plan.cs_static = all(p is not None and p.in_place for _, p in plan.sketches)
@@ -550,9 +555,11 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
         # comparisons).  Where the buckets do not run side by side (one stream), those launches go to a side
         # stream, which the bucket's next round waits for, and overlap the next bucket.
         if plan.q_next is None:
-            # row-major factors first, then the same in the order the kernels of ranks up to 8 load them
+            # row-major factors first, then the same in the order the kernels of ranks up to 8 load them, and behind
+            # that what a round with a sketched error keeps (CONEF_ROUND_NEXT_FOLD)
             by_rows = [m * _rank_bound(rank) for _, _, m, rank in work]
-            by_quads = [-(-m // 4) * 4 * _rank_bound(rank) for _, _, m, rank in work]
+            by_quads = [(-(-m // 4) * 4 + (items[cnt].w + _rank_bound(rank) + 1 if mode1 == 2 else 0)) * _rank_bound(rank)
+                        for cnt, (_, _, m, rank) in enumerate(work)]
             plan.q_next = torch.empty(sum(by_rows) + sum(by_quads), device=device, dtype=dtype)
             at = [plan.q_next.data_ptr()]
             for numel in by_rows + by_quads:
@@ -562,16 +569,16 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
             plan.made = [ctypes.c_int32(0) for _ in plan.chunks]
             plan.q_next_ready = False
         aside = state.matrix_approximation_rank > 8 and streams <= 1
-        flags = _ROUND_NEXT_QUADS | _ROUND_NEXT_WIDE | (0 if aside else _ROUND_MAKE_NEXT)
+        flags = _ROUND_NEXT_QUADS | _ROUND_NEXT_WIDE | (_ROUND_NEXT_FOLD if mode1 == 2 else 0) | (0 if aside else _ROUND_MAKE_NEXT)
         if plan.q_next_ready:
-            flags |= _ROUND_Q_READY | (_ROUND_QUADS_READY if plan.q_next_quads else 0)
-        all_made = 3
+            flags |= _ROUND_Q_READY | (_ROUND_QUADS_READY if plan.q_next_quads else 0) | (_ROUND_FOLD_READY if plan.q_next_fold else 0)
+        all_made = 7
         for (run, part), q_next, made in zip(plan.runs, plan.q_next_ptrs, plan.made):
             rc = lib.conef_psgd_round_ahead_f32(run, part, mode1, mode3, float(alpha), beta3, eps, HASH_A, HASH_B,
                                                 q_next, flags, ctypes.byref(made), ws_ptr, ws_len, stream)
             _lib.check(rc, "conef_psgd_round_ahead_f32")
             all_made &= made.value
-        plan.q_next_ready, plan.q_next_quads = bool(all_made & 1), bool(all_made & 2)
+        plan.q_next_ready, plan.q_next_quads, plan.q_next_fold = bool(all_made & 1), bool(all_made & 2), bool(all_made & 4)
         if aside:
             _orthogonalise_q_aside(plan, lib, eps, ws_len, device)
     else:
@@ -653,7 +660,7 @@ def _orthogonalise_q_aside(plan, lib, eps, ws_len, device):
     plan.q_next_event.record(side)
     plan.q_next_number = _pools.side_recorded(device, plan.q_next_event)
     plan.q_next_ready = all(made.value for made in plan.made)
-    plan.q_next_quads = False
+    plan.q_next_quads = plan.q_next_fold = False
 
 
 def run_batched_round(state, bucket):

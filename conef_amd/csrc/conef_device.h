@@ -56,6 +56,22 @@ __device__ __forceinline__ void conef_st4u(float* p, const float* v)
     *reinterpret_cast<conef_f4u*>(p) = t;
 }
 
+// 16 (4) bytes a lane from global memory to LDS without a register in between: lane l's land at lds + 16 l
+// (4 l), lds uniform over the wave, 16-byte (4-byte) aligned.  Not there before conef_wait_lds(), for other waves
+// not before a barrier behind it.
+__device__ __forceinline__ void conef_to_lds16(const void* src, void* lds)
+{
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+}
+__device__ __forceinline__ void conef_to_lds4(const void* src, void* lds)
+{
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)lds, 4, 0, 0);
+}
+
+__device__ __forceinline__ void conef_wait_lds() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // Rows cut into column quads when their length is not a multiple of four: the last quad is moved
 // back to end with the row, so that it stays inside, and its first `dup` columns are the previous
 // quad's.  Whoever owns it ignores them (they are never stored and never counted).
@@ -100,8 +116,15 @@ __device__ __forceinline__ void conef_store_slice_row(float* qi, int64_t i, int6
         for (int c = 0; c < RP; c += R) {
             const int t = k * RP + c;
             float* dst = qi + ((int64_t)(t >> 2) * m4 + quad) * 4 + (t & 3);
+            float v[R];
 #pragma unroll
-            for (int e = 0; e < R; ++e) dst[e] = zero ? 0.f : x[c + e];
+            for (int e = 0; e < R; ++e) v[e] = zero ? 0.f : x[c + e];
+            if constexpr (R == 4) {
+                conef_st4u(dst, v);
+            } else {
+#pragma unroll
+                for (int e = 0; e < R; ++e) dst[e] = v[e];
+            }
         }
     };
     const int64_t last = m4 - 1;

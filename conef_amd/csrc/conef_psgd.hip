@@ -24,6 +24,7 @@
 #include "conef_gs_gram.h"
 #include "conef_psgd_stream.h"
 #include "conef_psgd_small.h"
+#include "conef_psgd_linear.h"
 #include "conef_hip.h"      // ConefPsgdItem, and a check of this file's definitions against the public header
 
 extern "C" int conef_cs_query_f32(float* x, const float* cs, int64_t n, int64_t d, int32_t w, float alpha, int32_t a,
@@ -382,6 +383,10 @@ struct MtpItem {
     float* out;
     int64_t n;
     int m, r, rows_per_slab, col_tiles;
+    // not null: out2 = cs^T P of the cells [n, w] as well, by cs_wgs workgroups in front, a row slab of cs_rows each
+    const float* cs;
+    float* out2;
+    int w, cs_tiles, cs_rows, cs_wgs;
 };
 
 template <int RP, bool FAST>
@@ -524,19 +529,6 @@ gram_solve_lds(const double* __restrict__ parts, int nparts, float eps, float* t
     __syncthreads();
 }
 
-// x_k -= b_ik x_i (k > i), x_i *= 1 / d_i for i = 0 .. r - 1: the reference's column steps
-// (powerSGD_hook.py:21-43) on one row, coefficients from t_l as gram_solve_lds leaves them
-template <int RP>
-__device__ __forceinline__ void gram_apply_row(float* x, const float* t_l)
-{
-#pragma unroll
-    for (int i = 0; i < RP; ++i) {
-#pragma unroll
-        for (int k = i + 1; k < RP; ++k) x[k] = fmaf(-t_l[i * RP + k], x[i], x[k]);
-        x[i] = __fmul_rn(x[i], t_l[RP * RP + i]);
-    }
-}
-
 // tmat receives the steps themselves (b_ij, 1 / d_i) or, EXPLICIT, their product: the upper
 // triangular matrix T with orth(A) = A T, row-major [RP][RP] (row i is what the steps make of the
 // unit vector e_i).  A row times T is RP independent multiply-adds a column where the steps are a
@@ -580,30 +572,6 @@ gram_solve_body(const double* __restrict__ parts, int nparts, float* __restrict_
         gram_apply_row<RP>(x, t_l);
 #pragma unroll
         for (int k = 0; k < RP; ++k) tmat[threadIdx.x * RP + k] = x[k];
-    }
-}
-
-template <int RP>
-__device__ __forceinline__ void load_row(const float* p, float* x)
-{
-    if (RP >= 4) {
-#pragma unroll
-        for (int c = 0; c < RP; c += 4) ld4(p + c, x + c);
-    } else {
-#pragma unroll
-        for (int c = 0; c < RP; ++c) x[c] = p[c];
-    }
-}
-
-template <int RP>
-__device__ __forceinline__ void store_row(float* p, const float* x)
-{
-    if (RP >= 4) {
-#pragma unroll
-        for (int c = 0; c < RP; c += 4) st4(p + c, x + c);
-    } else {
-#pragma unroll
-        for (int c = 0; c < RP; ++c) p[c] = x[c];
     }
 }
 
@@ -652,18 +620,20 @@ psgd_mtp_gram_batch_kernel(PsgdBatch<MtpItem> b, GramTask g)
     const int i = psgd_batch_item(b, bx);
     const MtpItem& it = b.item[i];
     const int local = bx - b.first[i];
-    psgd_mtp_body<RP, FAST>(it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, local % it.col_tiles,
-                            local / it.col_tiles);
+    const bool cells = local < it.cs_wgs;
+    const int at = cells ? local : local - it.cs_wgs, tiles = cells ? it.cs_tiles : it.col_tiles, slab = at / tiles;
+    psgd_mtp_body<RP, FAST>(cells ? it.cs : it.x, it.p, cells ? it.out2 : it.out, it.n, cells ? it.w : it.m, it.r,
+                            cells ? it.cs_rows : it.rows_per_slab, at - slab * tiles, slab);
 }
 
-// rows of P and of the raw Q times T, a row a thread: x_k -= b_ik x_i (k > i), x_i *= 1 / d_i for
-// i = 0 .. r - 1, the reference's column steps (powerSGD_hook.py:21-43) with the coefficients known
+// rows of P and of the raw Q times T: x_k -= b_ik x_i (k > i), x_i *= 1 / d_i for i = 0 .. r - 1, the
+// reference's column steps (powerSGD_hook.py:21-43) with the coefficients known
 struct DeferFixItem {
     float* p;
     const float* qsrc;       // [slabs][m][RP] partials of Q = M^T P, or q itself with one slab
     float* q;
     const float* tmat;
-    double* qgram;           // not null: the workgroups of Q also leave their rows' share of Q^T Q, [m / 256][RP (RP + 1) / 2]
+    double* qgram;           // not null: the workgroups of Q also leave their rows' share of Q^T Q, [m / kFixQRows][RP (RP + 1) / 2]
     int64_t n, m;
     int slabs;
     int pblocks;             // workgroups that take rows of P; the others take rows of Q
@@ -674,6 +644,11 @@ struct DeferFixItem {
     float* qt;
     int r;
     float* qi;               // not null: Q by quads for the launch that follows (conef_store_slice_row)
+    // not null: partials of cs^T P, [slabs][w][RP]; row j of Q gets alpha times the row of its bucket
+    // (conef_psgd_linear.h)
+    const float* cs_src;
+    const uint32_t* pk;      // bucket and sign of every column
+    int w;
 };
 
 // A finished row (P or Q, zeros from column r on) into the caller's [rows, r] factor.
@@ -685,69 +660,131 @@ __device__ __forceinline__ void store_tight_row(float* dst, int64_t row, const f
         if (c < r) dst[row * r + c] = x[c];
 }
 
+// Ranks up to 8.  A row of P a thread.  A row of Q, a sum over as many slabs as there are (64 for a
+// [4096, 1024] matrix), four threads in different waves: they take a quarter of the slabs each.
+constexpr int kFixQRows = 64;
+
 template <int RP>
-__global__ void __launch_bounds__(256)
-psgd_defer_fix_batch_kernel(PsgdBatch<DeferFixItem> b)
+__device__ __forceinline__ void fix_p_rows(const DeferFixItem& it, int block, const float* t_l)
 {
-    constexpr int NG = RP * (RP + 1) / 2;
-    __shared__ float t_l[RP * RP + RP];
-    __shared__ float rows_l[256][RP + 1];
-    __shared__ double part_l[4][NG];
-    int local;
-    const DeferFixItem& it = b.item[psgd_batch_locate(b, &local)];
-    const bool is_p = local < it.pblocks;
-    const int64_t rows = is_p ? it.n : it.m;
-    const int64_t row = (int64_t)(is_p ? local : local - it.pblocks) * 256 + threadIdx.x;
-    const int64_t rc = row < rows ? row : rows - 1;
-    const float* src = is_p ? it.p : it.qsrc;
-    const int slabs = is_p ? 1 : it.slabs;
-    const int64_t stride = it.m * RP;
-    if (threadIdx.x < RP * RP + RP) t_l[threadIdx.x] = it.tmat[threadIdx.x];      // requested first: it travels with the rows
+    const int64_t row = (int64_t)block * 256 + threadIdx.x;
     float x[RP];
-#pragma unroll
-    for (int c = 0; c < RP; ++c) x[c] = 0.f;
-    int sl = 0;
-    for (; sl + 4 <= slabs; sl += 4) {                      // slabs in ascending order, four requested together
-        float v[4][RP];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) load_row<RP>(src + (int64_t)(sl + u) * stride + rc * RP, v[u]);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int c = 0; c < RP; ++c) x[c] += v[u][c];
-    }
-    for (; sl < slabs; ++sl) {
-        float v[RP];
-        load_row<RP>(src + (int64_t)sl * stride + rc * RP, v);
-#pragma unroll
-        for (int c = 0; c < RP; ++c) x[c] += v[c];
-    }
+    load_row<RP>(it.p + (row < it.n ? row : it.n - 1) * RP, x);
     __syncthreads();
     gram_apply_row<RP>(x, t_l);
     if (it.pt) {                     // the steps of columns that are not there divide by zero
 #pragma unroll
         for (int c = 0; c < RP; ++c)
             if (c >= it.r) x[c] = 0.f;
-        if (row < rows) store_tight_row<RP>(is_p ? it.pt : it.qt, row, x, it.r);
+        if (row < it.n) store_tight_row<RP>(it.pt, row, x, it.r);
     }
-    if (row < rows) store_row<RP>((is_p ? it.p : it.q) + row * RP, x);
-    if (!is_p && it.qi && row < rows) conef_store_slice_row<RP>(it.qi, row, it.m, x, false);
-    if (!is_p && it.qgram) {                                // uniform over the workgroup
+    if (row < it.n) store_row<RP>(it.p + row * RP, x);
+}
+
+// sums slabs [s0, s1) of a row in ascending order, eight requested together
+template <int RP>
+__device__ __forceinline__ void fix_sum_slabs(const float* src, int64_t stride, int s0, int s1, float* out)
+{
 #pragma unroll
-        for (int c = 0; c < RP; ++c) rows_l[threadIdx.x][c] = row < rows ? x[c] : 0.f;
-        __syncthreads();
-        const int e = threadIdx.x >> 2, quarter = threadIdx.x & 3;      // four threads an entry, 64 rows each
-        if (e < NG) {
-            int i, j;
-            gsg_entry(e, RP, &i, &j);
-            double s = 0.;
-            for (int t = quarter * 64; t < quarter * 64 + 64; ++t) s = fma((double)rows_l[t][i], (double)rows_l[t][j], s);
-            part_l[quarter][e] = s;
+    for (int c = 0; c < RP; ++c) out[c] = 0.f;
+    for (int sl = s0; sl < s1; sl += 8) {
+        float v[8][RP];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (sl + u < s1) load_row<RP>(src + (int64_t)(sl + u) * stride, v[u]);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (sl + u < s1) {
+#pragma unroll
+                for (int c = 0; c < RP; ++c) out[c] += v[u][c];
+            }
+    }
+}
+
+// a finished row of Q
+template <int RP>
+__device__ __forceinline__ void fix_store_q(const DeferFixItem& it, int64_t row, float* x)
+{
+    if (it.qt) {
+#pragma unroll
+        for (int c = 0; c < RP; ++c)
+            if (c >= it.r) x[c] = 0.f;
+        if (row < it.m) store_tight_row<RP>(it.qt, row, x, it.r);
+    }
+    if (row < it.m) {
+        store_row<RP>(it.q + row * RP, x);
+        if (it.qi) conef_store_slice_row<RP>(it.qi, row, it.m, x, false);
+    }
+}
+
+// one thread's sixteen rows of an entry of Q^T Q: entry e = thread / 4, its quarter of the rows in LDS
+template <int RP>
+__device__ __forceinline__ double fix_gram_quarter(const float (*rows_l)[RP + 1])
+{
+    constexpr int NG = RP * (RP + 1) / 2;
+    const int e = threadIdx.x >> 2, quarter = threadIdx.x & 3;
+    double s = 0.;
+    if (e < NG) {
+        int i, j;
+        gsg_entry(e, RP, &i, &j);
+#pragma unroll 4
+        for (int t = quarter * 16; t < quarter * 16 + 16; ++t) s = fma((double)rows_l[t][i], (double)rows_l[t][j], s);
+    }
+    return s;
+}
+
+template <int RP>
+__global__ void __launch_bounds__(256)
+psgd_defer_fix_batch_kernel(PsgdBatch<DeferFixItem> b, float alpha)
+{
+    constexpr int NG = RP * (RP + 1) / 2;
+    __shared__ float t_l[RP * RP + RP];
+    __shared__ float rows_l[256][RP + 1];
+    __shared__ double part_l[NG][4];
+    int local;
+    const DeferFixItem& it = b.item[psgd_batch_locate(b, &local)];
+    if (threadIdx.x < RP * RP + RP) t_l[threadIdx.x] = it.tmat[threadIdx.x];      // requested first: it travels with the rows
+    if (local < it.pblocks) {
+        fix_p_rows<RP>(it, local, t_l);
+        return;
+    }
+    const int lrow = threadIdx.x & (kFixQRows - 1), part = __builtin_amdgcn_readfirstlane(threadIdx.x / kFixQRows);
+    const int64_t row = (int64_t)(local - it.pblocks) * kFixQRows + lrow;
+    const int64_t rc = row < it.m ? row : it.m - 1;
+    const int s0 = it.slabs * part / 4, s1 = it.slabs * (part + 1) / 4;
+    const uint32_t pk = it.cs_src ? it.pk[rc] : 0u;
+    float x[RP];
+    fix_sum_slabs<RP>(it.qsrc + rc * RP, it.m * RP, s0, s1, x);
+    if (it.cs_src) {
+        float y[RP];
+        fix_sum_slabs<RP>(it.cs_src + (int64_t)(pk & 0x7fffffffu) * RP, (int64_t)it.w * RP, s0, s1, y);
+        const float f = conef_apply_sign(alpha, pk);
+#pragma unroll
+        for (int c = 0; c < RP; ++c) x[c] = fmaf(f, y[c], x[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < RP; ++c) rows_l[threadIdx.x][c] = x[c];
+    __syncthreads();
+    if (part == 0) {
+#pragma unroll
+        for (int u = 1; u < 4; ++u)
+#pragma unroll
+            for (int c = 0; c < RP; ++c) x[c] += rows_l[u * kFixQRows + lrow][c];
+        gram_apply_row<RP>(x, t_l);
+        fix_store_q<RP>(it, row, x);
+    }
+    if (it.qgram) {                                         // uniform over the workgroup
+        if (part == 0) {
+#pragma unroll
+            for (int c = 0; c < RP; ++c) rows_l[lrow][c] = row < it.m ? x[c] : 0.f;
         }
+        __syncthreads();
+        const double s = fix_gram_quarter<RP>(rows_l);
+        if ((int)(threadIdx.x >> 2) < NG) part_l[threadIdx.x >> 2][threadIdx.x & 3] = s;
         __syncthreads();
         if (threadIdx.x < NG)
             it.qgram[(size_t)(local - it.pblocks) * NG + threadIdx.x] =
-                (part_l[0][threadIdx.x] + part_l[1][threadIdx.x]) + (part_l[2][threadIdx.x] + part_l[3][threadIdx.x]);
+                (part_l[threadIdx.x][0] + part_l[threadIdx.x][1]) + (part_l[threadIdx.x][2] + part_l[threadIdx.x][3]);
     }
 }
 
@@ -1030,100 +1067,6 @@ psgd_rowlist_vec_batch_kernel(PsgdBatch<RowlistVecItem> b, double one_minus_beta
                                             local);
 }
 
-// ------------------------------------------------------------ M = P Q^T ----
-// MODE 0: write M.  MODE 1: also write the dense residual E = X - M (X = what M held on entry).
-// Factors of rank RP exactly (rows of RP floats, 16-byte aligned), rows of at least four columns of
-// any alignment.  A thread owns a column quad, whose 4 x RP slice of Q stays in registers, and walks
-// rows four at a time with their loads in flight together.  A workgroup is cut into groups of
-// `lanes` threads that cover a row (or 1024 columns of it) and take rows in turn; lanes is a multiple
-// of 64 wherever a row has more than 64 quads, so that a wave's row of P is uniform and comes through
-// the scalar cache.
-struct PqtItem {
-    float* x;
-    float* err;
-    const float* p;
-    const float* q;
-    int64_t n;
-    int m, r, rows_per_slab, col_tiles;
-    int lanes;
-    const float* qi;         // not null: q laid out by quads (conef_load_slices)
-};
-
-typedef __attribute__((address_space(4))) float conef_cfloat;      // constant memory: uniform loads are scalar
-
-inline int pqt_lanes(int64_t m)
-{
-    const int64_t m4 = (m + 3) / 4;
-    return (int)(m4 >= 256 ? 256 : m4 > 64 ? (m4 + 63) / 64 * 64 : m4);
-}
-
-template <int RP, int MODE, bool UNIFORM>
-__device__ __forceinline__ void
-psgd_pqt_rows(float* __restrict__ x, float* __restrict__ err, const float* __restrict__ p, const float* __restrict__ q,
-              const float* __restrict__ qi, const PqtItem& it, int bx, int by)
-{
-    const int m = it.m, groups = 256 / it.lanes;
-    int grp = (int)threadIdx.x / it.lanes;
-    const int quad = bx * 256 + (int)threadIdx.x - grp * it.lanes;
-    if (UNIFORM) grp = __builtin_amdgcn_readfirstlane(grp);
-    if (grp >= groups || 4 * quad >= m) return;
-    const int col = conef_quad_col(quad, m), dup = 4 * quad - col;
-    const int64_t i0 = (int64_t)by * it.rows_per_slab;
-    const int64_t i1 = i0 + it.rows_per_slab < it.n ? i0 + it.rows_per_slab : it.n;
-    float qf[4 * RP];
-    conef_load_slices<RP>(conef_quad_slices<RP>(q, qi, quad, col, m), qf);
-    auto walk = [&](auto store) {
-        for (int64_t ib = i0 + grp; ib < i1; ib += 4 * groups) {
-            float xv[4][4];
-            if (MODE == 1) {
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int64_t i = ib + u * groups < i1 ? ib + u * groups : ib;
-                    conef_ld4u(x + i * m + col, xv[u]);
-                }
-            }
-            // The four rows of P: through constant memory where they are uniform.  (The pointers come out of a table:
-            // nothing else tells the compiler that the stores leave P alone, and the rows became vector loads
-            // behind them.)
-            float pv[4][RP];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int64_t i = ib + u * groups < i1 ? ib + u * groups : ib;
-                if (UNIFORM) {
-                    const conef_cfloat* ps = (const conef_cfloat*)(uintptr_t)(p + i * RP);
-#pragma unroll
-                    for (int c = 0; c < RP; ++c) pv[u][c] = ps[c];
-                } else {
-#pragma unroll
-                    for (int c = 0; c < RP; ++c) pv[u][c] = p[i * RP + c];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int64_t i = ib + u * groups;
-                if (i >= i1) break;
-                float mh[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int c = 0; c < RP; ++c) {
-                    const float pc = pv[u][c];
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) mh[k] = fmaf(pc, qf[k * RP + c], mh[k]);
-                }
-                if (MODE == 1) {
-                    float ev[4];
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) ev[k] = __fsub_rn(xv[u][k], mh[k]);
-                    store(err + i * m + col, ev);
-                }
-                store(x + i * m + col, mh);
-            }
-        }
-    };
-    // (rows of whole quads have a loop without the moved quad's test; uniform)
-    if (m % 4 == 0) walk([](float* at, const float* v) { conef_st4u(at, v); });
-    else walk([&](float* at, const float* v) { conef_st4_own(at, v, dup); });
-}
-
 // The general form: any rank up to RP, element by element.
 template <int RP, int MODE>
 __device__ __forceinline__ void
@@ -1194,22 +1137,26 @@ psgd_pqt_one_kernel(PqtItem it)
 
 // Front of the row-list sketch kernel: the value to sketch is the residual X - P Q^T, and M is
 // overwritten with P Q^T on the way (powerSGD_hook.py:551,563-564).
-template <int RP, bool FAST>
+// LIN (with FAST): M lies as the gradient came, and X = M + alpha * unsketch(cs) is formed here (conef_psgd_linear.h);
+// the tile's old cells go to their place in LDS first.
+template <int RP, bool FAST, bool LIN = false>
 struct ListPsgdResidual {
     float* x;
     const float* p;
     const float* q;
     int r;
     const float* qi;         // not null: q laid out by quads (conef_load_slices), FAST
-    static constexpr bool kNeedsCells = false;
+    const float* cs;         // LIN: the old cells
+    float alpha;             // LIN
+    static constexpr bool kNeedsCells = false, kParksCells = LIN;
     // Half-height tiles where there are tiles to spare (conef_rowlist_shape) up to rank 4 and from 512 columns
     // on: full against half height [30522,1024] 69.2 and 62.5 us at rank 4 (79.0 and 93.0 at rank 8, whose slices
     // of Q a tile loads whatever its height), [50000,512] 64.0 and 52.7 (72.0 and 73.1), [20000,2048] 89.3 and
     // 74.9 at rank 1; [60000,300] at rank 4 40.5 and 43.1.
     static bool halves(int64_t m) { return RP <= 4 && m >= 512; }
     struct Regs {};
-    __device__ __forceinline__ void stage(int64_t row0, int rows, int d, int, float* vals, const float*,
-                                          const uint32_t*) const
+    __device__ __forceinline__ void stage(int64_t row0, int rows, int d, int w, float* vals, float* cells,
+                                          const uint32_t* pktab) const
     {
         float* base = x + row0 * d;
         if (FAST) {
@@ -1229,15 +1176,49 @@ struct ListPsgdResidual {
             int c4 = threadIdx.x - grp * lanes, rw = 2 * grp;
             bool have = grp < groups && c4 < d4 && rw < rows;
             float flat[4 * RP], flatn[4 * RP], x0n[4], x1n[4];
+            uint32_t pk[4], pkn[4];                        // LIN: bucket and sign of the quad's columns
             auto request_rows = [&](int quad, int row) {
                 const int r1 = row + 1 < rows ? row + 1 : row;
                 const int col = conef_quad_col(quad, d);
                 conef_ld4u(base + (int64_t)row * d + col, x0n);
                 conef_ld4u(base + (int64_t)r1 * d + col, x1n);
             };
+            constexpr int kCells = 4;
+            float ct[kCells];
+            if constexpr (LIN) {
+#pragma unroll
+                for (int u = 0; u < kCells; ++u) {
+                    ct[u] = 0.f;
+                    if (u * kConefRowlistThreads < rows * w) {
+                        const int i = (int)threadIdx.x + u * kConefRowlistThreads;
+                        ct[u] = cs[row0 * w + (i < rows * w ? i : rows * w - 1)];
+                    }
+                }
+            }
             if (have) {
+                if constexpr (LIN) conef_ld4u(pktab + conef_quad_col(c4, d), pk);
                 conef_load_slices<RP>(conef_quad_slices<RP>(q, qi, c4, conef_quad_col(c4, d), d), flat);
                 request_rows(c4, rw);
+            }
+            if constexpr (LIN) {
+#pragma unroll
+                for (int u = 0; u < kCells; ++u) {
+                    const int i = (int)threadIdx.x + u * kConefRowlistThreads;
+                    if (i < rows * w) cells[i] = ct[u];
+                }
+                for (int i0 = (int)threadIdx.x + kCells * kConefRowlistThreads; i0 < rows * w; i0 += 4 * kConefRowlistThreads) {
+                    float t[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const int i = i0 + u * kConefRowlistThreads;
+                        t[u] = cs[row0 * w + (i < rows * w ? i : rows * w - 1)];
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const int i = i0 + u * kConefRowlistThreads;
+                        if (i < rows * w) cells[i] = t[u];
+                    }
+                }
             }
             __syncthreads();
             while (have) {
@@ -1257,8 +1238,20 @@ struct ListPsgdResidual {
                     new_quad = true;
                 }
                 have = c4 < d4;
+                if constexpr (LIN) {
+                    const float *ca = cells + cur_rw * w, *cb = cells + r1 * w;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const uint32_t at = pk[k] & 0x7fffffffu;
+                        x0[k] = __fadd_rn(x0[k], conef_query_term(ca[at], pk[k], alpha));
+                        x1[k] = __fadd_rn(x1[k], conef_query_term(cb[at], pk[k], alpha));
+                    }
+                }
                 if (have) {
-                    if (new_quad) conef_load_slices<RP>(conef_quad_slices<RP>(q, qi, c4, conef_quad_col(c4, d), d), flatn);
+                    if (new_quad) {
+                        if constexpr (LIN) conef_ld4u(pktab + conef_quad_col(c4, d), pkn);
+                        conef_load_slices<RP>(conef_quad_slices<RP>(q, qi, c4, conef_quad_col(c4, d), d), flatn);
+                    }
                     request_rows(c4, rw);
                 }
                 const float* pa = ptile + cur_rw * RP;
@@ -1295,6 +1288,10 @@ struct ListPsgdResidual {
                 if (new_quad && have) {
 #pragma unroll
                     for (int t = 0; t < 4 * RP; ++t) flat[t] = flatn[t];
+                    if constexpr (LIN) {
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) pk[k] = pkn[k];
+                    }
                 }
             }
         } else {
@@ -3089,7 +3086,7 @@ int mtp_batch(const ConefPsgdItem* items, int count, void* workspace, int64_t wo
             const ConefPsgdItem& it = items[j];
             const MtpPlan& pl = plans[(size_t)j];
             float* out = pl.partial_off >= 0 ? partial_base + pl.partial_off : it.q;
-            MtpItem t = {it.x, it.p, out, it.n, (int)it.m, it.r, pl.g.rows_per_slab, pl.g.col_tiles};
+            MtpItem t = {it.x, it.p, out, it.n, (int)it.m, it.r, pl.g.rows_per_slab, pl.g.col_tiles, nullptr, nullptr, 0, 0, 0, 0};
             table.push_back(t);
             blocks.push_back(pl.g.col_tiles * pl.g.slabs);
             if (outs) (*outs)[(size_t)j] = MtpRaw{out, pl.partial_off >= 0 ? pl.g.slabs : 1};
@@ -3141,12 +3138,18 @@ inline int64_t defer_gram_doubles(const ConefPsgdItem& it)
     return (rp <= 8 ? (it.n + 3) / 4 : (it.n + 255) / 256) * (int64_t)(rp * (rp + 1) / 2);
 }
 
-// shares of Q^T Q, one per 256 rows of Q (the fix launch leaves them for the workgroups that
-// orthogonalise Q for the bucket's next round)
+// shares of Q^T Q, one per workgroup of the fix launch up to rank 8, one per 256 rows above (left for the
+// workgroups that orthogonalise Q for the bucket's next round)
+inline int64_t defer_qgram_shares(const ConefPsgdItem& it)
+{
+    const int rows = rank_bound(it.r) <= 8 ? kFixQRows : 256;
+    return (it.m + rows - 1) / rows;
+}
+
 inline int64_t defer_qgram_doubles(const ConefPsgdItem& it)
 {
     const int rp = rank_bound(it.r);
-    return ((it.m + 255) / 256) * (int64_t)(rp * (rp + 1) / 2);
+    return defer_qgram_shares(it) * (int64_t)(rp * (rp + 1) / 2);
 }
 
 inline int64_t defer_region_bytes(const ConefPsgdItem* items, int count)
@@ -3181,6 +3184,8 @@ struct PaddedRound {
     std::vector<float*> qi;          // ranks up to 8: the new Q by quads (conef_store_slice_row)
     int rp;
     bool padded;
+    int64_t offset;                  // defer_region_offset of the items
+    int64_t bytes;                   // padded_round_bytes of the caller's items
 };
 
 inline int64_t padded_factor_bytes(const ConefPsgdItem& it)
@@ -3214,11 +3219,15 @@ inline bool padded_round(const ConefPsgdItem* items, int count, int mq_mode, voi
     if (count < 1 || count > kPsgdBatchMax || !workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) return false;
     for (int k = 0; k < count; ++k)
         if (items[k].r != items[0].r || items[k].m < 4 || items[k].n > 0x7fffffffLL || items[k].m > 0x7fffffffLL) return false;
-    if (workspace_bytes < padded_round_bytes(items, count)) return false;
     pr->items = at_rank_bound(items, count);
     pr->rp = rank_bound(items[0].r);
     pr->padded = pr->rp != items[0].r;
-    char* at = (char*)workspace + defer_region_offset(pr->items.data(), count) + defer_region_bytes(pr->items.data(), count);
+    pr->offset = defer_region_offset(pr->items.data(), count);
+    const int64_t factors = pr->offset + defer_region_bytes(pr->items.data(), count);
+    pr->bytes = factors;
+    for (int k = 0; k < count; ++k) pr->bytes += padded_factor_bytes(items[k]);
+    if (workspace_bytes < pr->bytes) return false;
+    char* at = (char*)workspace + factors;
     for (int k = 0; k < count; ++k) {
         ConefPsgdItem& it = pr->items[(size_t)k];
         pr->pt.push_back(pr->padded ? it.p : nullptr);
@@ -3283,29 +3292,37 @@ int copy_rows(const std::vector<RowsItem>& table, hipStream_t s)
     });
 }
 
-// The fix launch of a deferred round over `raw` (where the products left the raw Q).
+// The cells' part of the second product (conef_psgd_linear.h): partials of cs^T P, [slabs][w][RP]
+struct CellRaw {
+    const float* src;
+    const uint32_t* pk;
+    int w;
+};
+
+// The fix launch of a deferred round over `raw` (where the products left the raw Q) and `cells` (or null).
 int defer_fix(const PaddedRound& pr, int r, const std::vector<MtpRaw>& raw, const std::vector<float*>& tmats,
-              const std::vector<double*>* qgrams, hipStream_t s)
+              const std::vector<double*>* qgrams, hipStream_t s, const std::vector<CellRaw>* cells = nullptr, float alpha = 0.f)
 {
     const int rp = pr.rp, count = (int)pr.items.size();
-    const int rows_per_wg = rp <= 8 ? 256 : 256 / (rp / 4);
+    const int rows_per_wg = rp <= 8 ? 256 : 256 / (rp / 4), qrows_per_wg = rp <= 8 ? kFixQRows : rows_per_wg;
     std::vector<DeferFixItem> fix;
     std::vector<int> blocks;
     for (int k = 0; k < count; ++k) {
         const ConefPsgdItem& it = pr.items[(size_t)k];
-        const int pb = (int)((it.n + rows_per_wg - 1) / rows_per_wg), qb = (int)((it.m + rows_per_wg - 1) / rows_per_wg);
+        const int pb = (int)((it.n + rows_per_wg - 1) / rows_per_wg), qb = (int)((it.m + qrows_per_wg - 1) / qrows_per_wg);
+        const CellRaw c = cells ? (*cells)[(size_t)k] : CellRaw{nullptr, nullptr, 0};
         fix.push_back(DeferFixItem{it.p, raw[(size_t)k].src, it.q, tmats[(size_t)k], qgrams ? (*qgrams)[(size_t)k] : nullptr,
                                    it.n, it.m, raw[(size_t)k].slabs, pb, pr.pt[(size_t)k], pr.qt[(size_t)k], r,
-                                   rp <= 8 ? pr.qi[(size_t)k] : nullptr});
+                                   rp <= 8 ? pr.qi[(size_t)k] : nullptr, c.src, c.pk, c.w});
         blocks.push_back(pb + qb);
     }
     return run_batches(fix, blocks, [&](const PsgdBatch<DeferFixItem>& bt, int grid) {
         const dim3 g((unsigned)grid), t(256);
         switch (rp) {
-            case 1: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<1>, g, t, 0, s, bt); break;
-            case 2: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<2>, g, t, 0, s, bt); break;
-            case 4: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<4>, g, t, 0, s, bt); break;
-            case 8: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<8>, g, t, 0, s, bt); break;
+            case 1: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<1>, g, t, 0, s, bt, alpha); break;
+            case 2: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<2>, g, t, 0, s, bt, alpha); break;
+            case 4: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<4>, g, t, 0, s, bt, alpha); break;
+            case 8: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<8>, g, t, 0, s, bt, alpha); break;
             case 16: hipLaunchKernelGGL(psgd_defer_fix_wide_batch_kernel<16>, g, t, 0, s, bt); break;
             default: hipLaunchKernelGGL(psgd_defer_fix_wide_batch_kernel<32>, g, t, 0, s, bt); break;
         }
@@ -3326,7 +3343,7 @@ int round_products_deferred(const PaddedRound& pr, int r, float* const* q_in, fl
     std::vector<MqsItem> table;
     std::vector<float*> tmats;
     std::vector<double*> qgrams;
-    char* at = (char*)workspace + defer_region_offset(items, count);
+    char* at = (char*)workspace + pr.offset;
     for (int k = 0; k < count; ++k) {
         const ConefPsgdItem& it = items[k];
         MqsItem t = {it.x, it.err, it.cs, MODE == 2 ? item_pktab(it) : nullptr, q_in[k], it.p, it.n, (int)it.m,
@@ -3354,7 +3371,7 @@ int round_products_deferred(const PaddedRound& pr, int r, float* const* q_in, fl
         gram.tmat[k] = tmats[(size_t)k];
         if (q_shares) {
             q_shares->parts[k] = qgrams[(size_t)k];
-            q_shares->nparts[k] = (int)((items[k].m + 255) / 256);
+            q_shares->nparts[k] = (int)defer_qgram_shares(items[k]);
         }
     }
     std::vector<MtpRaw> raw((size_t)count);
@@ -3382,7 +3399,7 @@ int round_products_deferred_mfma(const PaddedRound& pr, int r, float* const* q_i
     gram.count = count;
     gram.r = r;
     gram.eps = eps;
-    char* at = (char*)workspace + defer_region_offset(items, count);
+    char* at = (char*)workspace + pr.offset;
     for (int k = 0; k < count; ++k) {
         const ConefPsgdItem& it = items[k];
         const int nb = (int)((it.n + 255) / 256);
@@ -3472,7 +3489,7 @@ int orthogonalise_by_gram_wide(const PaddedRound& pr, int r, const std::vector<c
     gram.count = count;
     gram.r = r;
     gram.eps = eps;
-    char* at = (char*)workspace + defer_region_offset(pr.items.data(), count);
+    char* at = (char*)workspace + pr.offset;
     const int rows_per_wg = 256 / (rp / 4);
     for (int k = 0; k < count; ++k) {
         const ConefPsgdItem& it = pr.items[(size_t)k];
@@ -3487,7 +3504,8 @@ int orthogonalise_by_gram_wide(const PaddedRound& pr, int r, const std::vector<c
         gram.parts[k] = parts;
         gram.nparts[k] = nb;
         gram.tmat[k] = tmat;
-        fix.push_back(DeferFixItem{nullptr, src[(size_t)k], dst[k], tmat, nullptr, 0, it.m, 1, 0, nullptr, nullptr, r, nullptr});
+        fix.push_back(DeferFixItem{nullptr, src[(size_t)k], dst[k], tmat, nullptr, 0, it.m, 1, 0, nullptr, nullptr, r, nullptr,
+                                   nullptr, nullptr, 0});
         fix_blocks.push_back((int)((it.m + rows_per_wg - 1) / rows_per_wg));
     }
     int rc = run_batches(shares, share_blocks, [&](const PsgdBatch<GramShareItem>& bt, int grid) {
@@ -3503,9 +3521,9 @@ int orthogonalise_by_gram_wide(const PaddedRound& pr, int r, const std::vector<c
     });
 }
 
-template <int RP, bool FAST>
+template <int RP, bool FAST, bool LIN = false>
 struct RowlistResidualItem {
-    ListPsgdResidual<RP, FAST> front;
+    ListPsgdResidual<RP, FAST, LIN> front;
     ConefRowlistView plan;
     const float* cs_in;
     float* cs_out;
@@ -3560,6 +3578,102 @@ psgd_pqt_gs_batch_kernel(PsgdBatch<PqtItem> b, GsAhead g)
     psgd_pqt_item<RP, MODE, FAST>(it, local);
 }
 
+// ------------------------------------------------------ sketched error, linear form ----
+// Kernels of conef_psgd_linear.h over the matrices of a bucket.
+template <int RP>
+__global__ void __launch_bounds__(256)
+psgd_fold_batch_kernel(PsgdBatch<FoldItem> b)
+{
+    int local;
+    const FoldItem& it = b.item[psgd_batch_locate(b, &local)];
+    const int j = local * 256 + (int)threadIdx.x;
+    if (j >= it.w) return;
+    float f[RP];
+    conef_fold_row<RP, 4>(it.q, RP, it.ent, it.csr[j], it.csr[j + 1], f);
+    store_row<RP>(it.f + (int64_t)j * RP, f);
+}
+
+template <int RP, int T>
+__global__ void __launch_bounds__(T)
+psgd_lin_mq_batch_kernel(PsgdBatch<LinMqItem> b, float alpha)
+{
+    int local;
+    const LinMqItem& it = b.item[psgd_batch_locate(b, &local)];
+    psgd_lin_mq_body<RP, T>(it, alpha, local);
+}
+
+// For the bucket's next round, in front of the launch: `split` workgroups a matrix solve the system of Q^T Q, each
+// for itself, and write their rows of Q orthogonalised; the first also leaves the steps.  `fold_split` more add up
+// F(Q), 256 buckets each.
+struct LinNext {
+    float* dst[kPsgdBatchMax];
+    float* tmat[kPsgdBatchMax];       // or null
+    float* fold[kPsgdBatchMax];       // or null
+    const double* parts[kPsgdBatchMax];
+    int nparts[kPsgdBatchMax];
+    int count, split, fold_split, r;
+    float eps;
+};
+
+constexpr int kLinNextRows = 512;     // rows a workgroup takes at once
+
+template <int RP>
+__device__ __forceinline__ void psgd_lin_next_body(const LinNext& g, const float* q, int m, int k, int part)
+{
+    constexpr int U = kLinNextRows / 256;
+    __shared__ float t_l[RP * RP + RP];
+    float x[U][RP];
+    auto request = [&](int row) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) load_row<RP>(q + (int64_t)(row + u * 256 < m ? row + u * 256 : m - 1) * RP, x[u]);
+    };
+    int row = part * kLinNextRows + (int)threadIdx.x;
+    request(row);                                                      // travels while the system is solved
+    gram_solve_lds<RP, 256>(g.parts[k], g.nparts[k], g.eps, t_l);
+    if (part == 0 && g.tmat[k] && (int)threadIdx.x < RP * RP + RP) g.tmat[k][threadIdx.x] = t_l[threadIdx.x];
+    for (;;) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            gram_apply_row<RP>(x[u], t_l);
+            if (g.r < RP) {
+#pragma unroll
+                for (int c = 0; c < RP; ++c)
+                    if (c >= g.r) x[u][c] = 0.f;
+            }
+            if (row + u * 256 < m) store_row<RP>(g.dst[k] + (int64_t)(row + u * 256) * RP, x[u]);
+        }
+        row += g.split * kLinNextRows;
+        if (row >= m) break;
+        request(row);
+    }
+}
+
+// The residual kernel over M as the gradient came, with those workgroups in front.
+template <int RP>
+__global__ void __launch_bounds__(kConefRowlistThreads)
+psgd_lin_residual_batch_kernel(PsgdBatch<RowlistResidualItem<RP, true, true>> b, double one_minus_beta, LinNext g)
+{
+    static_assert(kConefRowlistThreads == 256, "one block size for both kinds of workgroup");
+    const int riders = g.count * (g.split + g.fold_split);
+    if ((int)blockIdx.x < riders) {
+        const int k = (int)blockIdx.x / (g.split + g.fold_split), part = (int)blockIdx.x - k * (g.split + g.fold_split);
+        const RowlistResidualItem<RP, true, true>& it = b.item[k];
+        if (part < g.split) {
+            psgd_lin_next_body<RP>(g, it.front.q, it.d, k, part);
+        } else if (const int j = (part - g.split) * 256 + (int)threadIdx.x; j < it.w) {
+            float f[RP];
+            conef_fold_row<RP, 4>(it.front.q, RP, it.plan.ent, it.plan.csr[j], it.plan.csr[j + 1], f);
+            store_row<RP>(g.fold[k] + (int64_t)j * RP, f);
+        }
+        return;
+    }
+    const int bx = (int)blockIdx.x - riders;
+    const int i = psgd_batch_item(b, bx);
+    const RowlistResidualItem<RP, true, true>& it = b.item[i];
+    conef_rowlist_body<float, ListPsgdResidual<RP, true, true>>(it.front, it.plan, it.cs_in, it.cs_out, it.n, it.d, it.w, it.rb,
+                                                                one_minus_beta, bx - b.first[i]);
+}
+
 // Rows a workgroup of the dense M = P Q^T takes: as many as leave the launch two thousand workgroups
 // (eight a CU: the walk has no prefetch of its own and lives off resident waves), at most sixteen a
 // thread (the thread's slice of Q, RP 16-byte loads, is then read once per sixteen rows of three
@@ -3586,6 +3700,27 @@ inline void pqt_rows_table(const ConefPsgdItem* items, const std::vector<int>& m
     }
 }
 
+// Tiles of the residual launch.  Full-height ones when the bucket has 600 of them that way (over two a CU); shorter
+// ones otherwise.  (Resident workgroups are bounded by LDS, so fewer, fuller tiles mean fewer rounds of them.)
+template <int RP, bool FAST>
+bool residual_tiles(const ConefPsgdItem* items, const std::vector<int>& members, std::vector<ConefRowlistShape>* shapes)
+{
+    int companions = 0;
+    for (int pass = 0; pass < 2; ++pass) {
+        int64_t tiles = 0;
+        shapes->clear();
+        for (int j : members) {
+            ConefRowlistShape shape;
+            if (!conef_rowlist_shape(items[j].n, items[j].m, items[j].w, false, ListPsgdResidual<RP, FAST>::halves(items[j].m), &shape, companions)) return false;
+            shapes->push_back(shape);
+            tiles += shape.tiles;
+        }
+        if (tiles >= 600) break;
+        companions = (int)members.size();
+    }
+    return true;
+}
+
 template <int RP, bool FAST>
 int pqt_sketch_group(const ConefPsgdItem* items, const std::vector<int>& members, float beta, hipStream_t s,
                      const GsAhead* ahead, const std::vector<float*>* qi)
@@ -3593,20 +3728,13 @@ int pqt_sketch_group(const ConefPsgdItem* items, const std::vector<int>& members
     std::vector<RowlistResidualItem<RP, FAST>> table;
     std::vector<int> blocks;
     size_t lds = 0;
-    // Full-height tiles when the bucket has 600 of them that way (over two a CU); shorter ones otherwise.
-    // (Resident workgroups are bounded by LDS, so fewer, fuller tiles mean fewer rounds of them.)
-    int64_t full_tiles = 0;
-    for (int j : members) {
-        ConefRowlistShape shape;
-        if (!conef_rowlist_shape(items[j].n, items[j].m, items[j].w, false, ListPsgdResidual<RP, FAST>::halves(items[j].m), &shape, 0)) return CONEF_ERR_INVALID;
-        full_tiles += shape.tiles;
-    }
-    const int companions = full_tiles >= 600 ? 0 : (int)members.size();
-    for (int j : members) {
+    std::vector<ConefRowlistShape> shapes;
+    if (!residual_tiles<RP, FAST>(items, members, &shapes)) return CONEF_ERR_INVALID;
+    for (size_t k = 0; k < members.size(); ++k) {
+        const int j = members[k];
         const ConefPsgdItem& it = items[j];
-        ConefRowlistShape shape;
-        if (!conef_rowlist_shape(it.n, it.m, it.w, false, ListPsgdResidual<RP, FAST>::halves(it.m), &shape, companions)) return CONEF_ERR_INVALID;
-        RowlistResidualItem<RP, FAST> t = {{it.x, it.p, it.q, it.r, qi ? (*qi)[(size_t)j] : nullptr},
+        const ConefRowlistShape& shape = shapes[k];
+        RowlistResidualItem<RP, FAST> t = {{it.x, it.p, it.q, it.r, qi ? (*qi)[(size_t)j] : nullptr, nullptr, 0.f},
                                            conef_rowlist_view((const ConefPlanHeader*)it.plan_host, it.plan_dev),
                                            it.cs, it.cs, it.n, (int)it.m, it.w, shape.rb};
         table.push_back(t);
@@ -3771,6 +3899,230 @@ int pqt_batch(const ConefPsgdItem* items, int count, int mode, float beta, int32
     return CONEF_OK;
 }
 
+// ---- rounds with a sketched error in linear form (conef_psgd_linear.h): host side ----
+// Behind the deferred round's part of the workspace, per matrix: the shares of P^T P, the partials of cs^T P, F(Q)
+// of the Q the first product reads.
+struct LinearRound {
+    std::vector<LinMqItem> mq;
+    LinMqShape shape;
+    std::vector<MtpPlan> mtp;
+    std::vector<float*> cs_part, fold;
+    std::vector<ConefRowlistView> view;
+};
+
+inline bool linear_shapes(const ConefPsgdItem* items, int count, std::vector<LinMqItem>* mq, LinMqShape* shape)
+{
+    if (count < 1 || count > kPsgdBatchMax || rank_bound(items[0].r) > 8) return false;
+    for (int k = 0; k < count; ++k) {
+        const ConefPsgdItem& it = items[k];
+        if (!it.plan_host || it.r != items[0].r || it.m < 4 || it.m > kConefRowlistMaxCols || it.n > 0x7fffffffLL || it.w < 4 ||
+            it.w > 0xffff)
+            return false;
+        LinMqItem t = {};
+        t.n = (int)it.n;
+        t.m = (int)it.m;
+        t.w = it.w;
+        mq->push_back(t);
+    }
+    return lin_mq_plan(mq->data(), count, rank_bound(items[0].r), shape);
+}
+
+// Slabs of the second product: those of a matrix in a launch of its own (mtp_shape), but twice as tall where a
+// matrix has more than 32 and the launch 256 workgroups either way: the fix launch adds their partials ([4096, 1024]
+// next to two of [1024, 1024] at rank 8: 13.0 -> 9.9 us there, the product 10.4 us as before).  Never more
+// partials than mtp_batch_layout makes room for.
+inline void linear_mtp(const ConefPsgdItem* items, int count, std::vector<MtpPlan>* plans)
+{
+    mtp_batch_layout(items, count, plans);
+    int64_t wgs = 0;
+    for (const MtpPlan& pl : *plans) wgs += (int64_t)pl.g.col_tiles * (pl.g.slabs > 32 ? (pl.g.slabs + 1) / 2 : pl.g.slabs);
+    if (wgs < 256) return;
+    for (int k = 0; k < count; ++k) {
+        MtpShape& g = (*plans)[(size_t)k].g;
+        if (g.slabs <= 32) continue;
+        g.rows_per_slab *= 2;
+        g.slabs = (int)((items[k].n + g.rows_per_slab - 1) / g.rows_per_slab);
+    }
+}
+
+inline int64_t linear_item_bytes(const ConefPsgdItem& it, const LinMqItem& t, const MtpPlan& pl, int64_t* gram, int64_t* cs_part)
+{
+    const int64_t rp = rank_bound(it.r);
+    *gram = conef_align256(8 * ((it.n + t.rows - 1) / t.rows) * (rp * (rp + 1) / 2));
+    *cs_part = conef_align256(4 * (int64_t)pl.g.slabs * it.w * rp);
+    return *gram + *cs_part + conef_align256(4 * (int64_t)it.w * rp);
+}
+
+inline int64_t linear_round_bytes(const ConefPsgdItem* items, int count)
+{
+    LinearRound lr;
+    if (!linear_shapes(items, count, &lr.mq, &lr.shape)) return 0;
+    linear_mtp(items, count, &lr.mtp);
+    int64_t bytes = 0, gram, cs_part;
+    for (int k = 0; k < count; ++k) bytes += linear_item_bytes(items[k], lr.mq[(size_t)k], lr.mtp[(size_t)k], &gram, &cs_part);
+    return bytes;
+}
+
+// Whether the round of pr's matrices runs in linear form: row-list plans of at least four buckets and the room.
+bool linear_round(const ConefPsgdItem* items, int count, int32_t a, int32_t b, void* workspace, int64_t workspace_bytes,
+                  const PaddedRound& pr, LinearRound* lr)
+{
+    for (int k = 0; k < count; ++k) {
+        const ConefPlanHeader* hp = (const ConefPlanHeader*)items[k].plan_host;
+        if (!items[k].cs || !items[k].plan_dev || !conef_plan_matches(hp, items[k].n, items[k].m, items[k].w, a, b) ||
+            hp->kind != kConefPlanRowlist)
+            return false;
+    }
+    if (!linear_shapes(items, count, &lr->mq, &lr->shape)) return false;
+    linear_mtp(pr.items.data(), count, &lr->mtp);
+    const int64_t front = pr.bytes;
+    char* at = (char*)workspace + front;
+    int64_t bytes = 0;
+    for (int k = 0; k < count; ++k) {
+        const ConefPsgdItem& it = pr.items[(size_t)k];
+        const ConefRowlistView view = conef_rowlist_view((const ConefPlanHeader*)it.plan_host, it.plan_dev);
+        LinMqItem& t = lr->mq[(size_t)k];
+        int64_t gram, cs_part;
+        const int64_t need = linear_item_bytes(it, t, lr->mtp[(size_t)k], &gram, &cs_part);
+        t.x = it.x;
+        t.cs = it.cs;
+        t.gram = (double*)at;
+        t.p = it.p;
+        lr->cs_part.push_back((float*)(at + gram));
+        lr->fold.push_back((float*)(at + gram + cs_part));
+        lr->view.push_back(view);
+        at += need;
+        bytes += need;
+    }
+    return workspace_bytes >= front + bytes;
+}
+
+// What a round in linear form leaves for the bucket's next one, in the buffer behind q_next (CONEF_ROUND_NEXT_FOLD):
+// its Q by quads as the products left it, F of that, and the column steps that orthogonalise it.  The next
+// round's P = X Q' is then (X Q) T, T applied to the rows of P where they are made (as the deferred
+// orthogonalisation of P does with Q), and nobody waits for Q' to be written.
+struct LinKept {
+    float *quads, *fold, *tmat;
+};
+
+inline LinKept linear_kept(float* at, int64_t m, int w, int rp)
+{
+    LinKept k = {at, at + 4 * conef_quads(m) * rp, nullptr};
+    k.tmat = k.fold + (int64_t)w * rp;
+    return k;
+}
+
+// The round after Q: q_in (orthogonal, rows of rp floats), or, with `kept_ready`, what the last round kept; kept
+// (or empty): where to leave that for the next; next: where the next round's Q factors go, count 0 for none.
+template <int RP>
+int round_linear(PaddedRound& pr, LinearRound& lr, int r, float* const* q_in, const std::vector<LinKept>& kept, bool kept_ready,
+                 LinNext next, float alpha, float beta, float eps, void* workspace, hipStream_t s)
+{
+    const ConefPsgdItem* items = pr.items.data();
+    const int count = (int)pr.items.size();
+    int rc = CONEF_OK;
+    if (!kept_ready) {
+        std::vector<FoldItem> folds;
+        std::vector<int> blocks;
+        for (int k = 0; k < count; ++k) {
+            folds.push_back(FoldItem{q_in[k], lr.view[(size_t)k].csr, lr.view[(size_t)k].ent, lr.fold[(size_t)k], items[k].w});
+            blocks.push_back((items[k].w + 255) / 256);
+        }
+        rc = run_batches(folds, blocks, [&](const PsgdBatch<FoldItem>& bt, int grid) {
+            hipLaunchKernelGGL(psgd_fold_batch_kernel<RP>, dim3((unsigned)grid), dim3(256), 0, s, bt);
+        });
+        if (rc != CONEF_OK) return rc;
+    }
+    std::vector<int> blocks;
+    std::vector<float*> tmats;
+    std::vector<double*> qgrams;
+    GramTask gram;
+    gram.count = count;
+    gram.r = r;
+    gram.eps = eps;
+    char* at = (char*)workspace + pr.offset;
+    for (int k = 0; k < count; ++k) {
+        LinMqItem& t = lr.mq[(size_t)k];
+        t.q = q_in[k];
+        t.qi = kept_ready ? kept[(size_t)k].quads : nullptr;
+        t.fold = kept_ready ? kept[(size_t)k].fold : lr.fold[(size_t)k];
+        t.tmat = kept_ready ? kept[(size_t)k].tmat : nullptr;
+        t.r = r;
+        blocks.push_back((t.n + t.rows - 1) / t.rows);
+        at += conef_align256(8 * defer_gram_doubles(items[k]));
+        tmats.push_back((float*)at);
+        at += defer_tmat_bytes(RP);
+        qgrams.push_back((double*)at);
+        at += conef_align256(8 * defer_qgram_doubles(items[k]));
+        gram.parts[k] = t.gram;
+        gram.nparts[k] = blocks.back();
+        gram.tmat[k] = tmats.back();
+    }
+    const LinMqShape& sh = lr.shape;
+    auto kern = sh.T == 256 ? psgd_lin_mq_batch_kernel<RP, 256> : psgd_lin_mq_batch_kernel<RP, 512>;
+    if (hipError_t e = conef_allow_lds((const void*)kern, sh.lds); e != hipSuccess) return (int)e;
+    rc = run_batches(lr.mq, blocks, [&](const PsgdBatch<LinMqItem>& bt, int grid) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3((unsigned)sh.T), sh.lds, s, bt, alpha);
+    });
+    if (rc != CONEF_OK) return rc;
+
+    std::vector<MtpItem> mtp;
+    std::vector<MtpRaw> raw;
+    std::vector<CellRaw> cells;
+    float* partials = (float*)workspace;         // batch_single_bytes is 0 below rank 16
+    blocks.clear();
+    for (int k = 0; k < count; ++k) {
+        const ConefPsgdItem& it = items[k];
+        const MtpPlan& pl = lr.mtp[(size_t)k];
+        float* out = pl.partial_off >= 0 ? partials + pl.partial_off : it.q;
+        const int cs_tiles = (it.w + 255) / 256, cs_wgs = cs_tiles * pl.g.slabs;
+        mtp.push_back(MtpItem{it.x, it.p, out, it.n, (int)it.m, it.r, pl.g.rows_per_slab, pl.g.col_tiles, it.cs, lr.cs_part[(size_t)k],
+                              it.w, cs_tiles, pl.g.rows_per_slab, cs_wgs});
+        blocks.push_back(pl.g.col_tiles * pl.g.slabs + cs_wgs);
+        if (!kept.empty()) pr.qi[(size_t)k] = kept[(size_t)k].quads;
+        raw.push_back(MtpRaw{out, pl.g.slabs});
+        cells.push_back(CellRaw{lr.cs_part[(size_t)k], lr.view[(size_t)k].pk, it.w});
+    }
+    rc = run_batches(mtp, blocks, [&](const PsgdBatch<MtpItem>& bt, int grid) {
+        hipLaunchKernelGGL((psgd_mtp_gram_batch_kernel<RP, true>), dim3((unsigned)(grid + count)), dim3(kMtpThreads), 0, s, bt, gram);
+    });
+    if (rc != CONEF_OK) return rc;
+    rc = defer_fix(pr, r, raw, tmats, next.count ? &qgrams : nullptr, s, &cells, alpha);
+    if (rc != CONEF_OK) return rc;
+
+    std::vector<int> members;
+    for (int k = 0; k < count; ++k) members.push_back(k);
+    std::vector<ConefRowlistShape> shapes;
+    if (!residual_tiles<RP, true>(items, members, &shapes)) return CONEF_ERR_INVALID;
+    std::vector<RowlistResidualItem<RP, true, true>> last;
+    size_t lds = 0;
+    blocks.clear();
+    next.split = 1;
+    next.fold_split = 0;
+    for (int k = 0; k < count; ++k) {
+        const ConefPsgdItem& it = items[k];
+        const ConefRowlistShape& shape = shapes[(size_t)k];
+        last.push_back(RowlistResidualItem<RP, true, true>{{it.x, it.p, it.q, it.r, pr.qi[(size_t)k], it.cs, alpha}, lr.view[(size_t)k],
+                                                           it.cs, it.cs, it.n, (int)it.m, it.w, shape.rb});
+        blocks.push_back((int)shape.tiles);
+        if (shape.lds > lds) lds = shape.lds;
+        next.split = std::max(next.split, (int)std::min((it.m + kLinNextRows - 1) / kLinNextRows, (int64_t)16));
+        next.tmat[k] = kept.empty() ? nullptr : kept[(size_t)k].tmat;
+        next.parts[k] = qgrams[(size_t)k];
+        next.nparts[k] = (int)defer_qgram_shares(it);
+        next.fold[k] = kept.empty() ? nullptr : kept[(size_t)k].fold;
+        next.fold_split = std::max(next.fold_split, kept.empty() ? 0 : (it.w + 255) / 256);
+    }
+    next.r = r;
+    next.eps = eps;
+    auto residual = psgd_lin_residual_batch_kernel<RP>;
+    if (hipError_t e = conef_allow_lds((const void*)residual, lds); e != hipSuccess) return (int)e;
+    const double omb = 1. - (double)beta;
+    return run_batches(last, blocks, [&](const PsgdBatch<RowlistResidualItem<RP, true, true>>& bt, int grid) {
+        hipLaunchKernelGGL(residual, dim3((unsigned)(grid + next.count * (next.split + next.fold_split))), dim3(kConefRowlistThreads), lds, s, bt, omb, next);
+    });
+}
+
 // Whether a round of these matrices runs with the orthogonalisation of P deferred: where the batch allows
 // (padded_round), unless CONEF_ROUND_DEFER=0 asks for the reference's order of steps (read on every call: a
 // test switches it).
@@ -3814,7 +4166,7 @@ int64_t conef_psgd_batch_workspace_bytes(const ConefPsgdItem* items, int32_t cou
     }
     int64_t launches = conef_align256(single) + conef_align256(4 * mtp_batch_layout(items, count, nullptr)) +
                        conef_align256(4 * mfma_batch_layout(items, count, nullptr));
-    const int64_t padded = padded_round_bytes(items, count);
+    const int64_t padded = padded_round_bytes(items, count) + linear_round_bytes(items, count);
     if (padded > launches) launches = padded;
     const int64_t small = conef_psgd_round_small_workspace_bytes(items, count);      // the one-launch round's records
     return small > launches ? small : launches;
@@ -3906,7 +4258,7 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
 {
     if (made) *made = 0;
     if (count < 0 || (count > 0 && !items) || pqt_mode < 0 || pqt_mode > 3) return CONEF_ERR_INVALID;
-    if ((flags & (CONEF_ROUND_Q_READY | CONEF_ROUND_MAKE_NEXT | CONEF_ROUND_QUADS_READY)) && (!q_next || !made)) return CONEF_ERR_INVALID;
+    if ((flags & (CONEF_ROUND_Q_READY | CONEF_ROUND_MAKE_NEXT | CONEF_ROUND_QUADS_READY | CONEF_ROUND_FOLD_READY)) && (!q_next || !made)) return CONEF_ERR_INVALID;
     if (count == 0) return CONEF_OK;
     std::vector<float*> mats((size_t)count);
     std::vector<int64_t> rows((size_t)count);
@@ -3926,7 +4278,7 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
         if (mq_mode == 2 && it.plan_host && !conef_plan_matches((const ConefPlanHeader*)it.plan_host, it.n, it.m, it.w, a, b))
             return CONEF_ERR_INVALID;
         if ((flags & CONEF_ROUND_Q_READY) && !q_next[k]) return CONEF_ERR_INVALID;
-        if ((flags & CONEF_ROUND_QUADS_READY) && !q_next[count + k]) return CONEF_ERR_INVALID;
+        if ((flags & (CONEF_ROUND_QUADS_READY | CONEF_ROUND_FOLD_READY)) && !q_next[count + k]) return CONEF_ERR_INVALID;
     }
     hipStream_t hs = (hipStream_t)stream;
     GsAhead ahead;
@@ -3942,13 +4294,22 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
     const bool wide = (flags & CONEF_ROUND_NEXT_WIDE) != 0;
     const bool by_quads = (flags & CONEF_ROUND_NEXT_QUADS) != 0;      // q_next[count + k]: room for the same by quads
     const bool quads_ready = ready && (flags & CONEF_ROUND_QUADS_READY) != 0;
+    const bool by_fold = (flags & CONEF_ROUND_NEXT_FOLD) != 0;        // with room for F(Q) behind the quads
+    const bool fold_ready = ready && (flags & CONEF_ROUND_FOLD_READY) != 0;
     bool want_next = (flags & CONEF_ROUND_MAKE_NEXT) && count <= kPsgdBatchMax && (wide || items[0].r <= 8);
     for (int k = 0; k < count && want_next; ++k) want_next = q_next[k] && items[k].r == items[0].r && items[k].m <= 0x7fffffffLL;
     const int rp = rank_bound(items[0].r);
     // P = X Q, P orthogonalised, Q = X^T P: with the orthogonalisation deferred where the batch
     // allows, else as three steps
     PaddedRound pr;
-    const bool deferred = round_defers(items, count, mq_mode, workspace, workspace_bytes, &pr);
+    LinearRound lr;
+    // A sketched error in linear form, where the error is added and the residual sketched in one round.  (The rows of
+    // r floats that a caller without NEXT_WIDE wants next, at a rank that is padded, come out of the other way only.)
+    const bool linear = mq_mode == 2 && pqt_mode == 2 && rp <= 8 && (wide || rp == items[0].r) &&
+                        round_defers(items, count, 0, workspace, workspace_bytes, &pr) &&
+                        linear_round(items, count, a, b, workspace, workspace_bytes, pr, &lr);
+    if (!linear) pr = PaddedRound();
+    const bool deferred = linear || round_defers(items, count, mq_mode, workspace, workspace_bytes, &pr);
     const ConefPsgdItem* its = deferred ? pr.items.data() : items;       // whose factors the rest of the round reads
     int rc = CONEF_OK;
     if (deferred) {
@@ -3974,6 +4335,23 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
             for (int k = 0; k < count; ++k) src.push_back(pr.items[(size_t)k].q);
             rc = orthogonalise_by_gram_wide(pr, r, src, q_in.data(), eps, workspace, hs);
             if (rc != CONEF_OK) return rc;
+        }
+        if (linear) {
+            LinNext next;
+            next.count = want_next ? count : 0;
+            std::vector<LinKept> kept;
+            for (int k = 0; k < count; ++k) {
+                next.dst[k] = want_next ? q_next[k] : nullptr;
+                if ((want_next && by_quads && by_fold) || fold_ready) kept.push_back(linear_kept(q_next[count + k], items[k].m, items[k].w, rp));
+            }
+            switch (rp) {
+                case 1: rc = round_linear<1>(pr, lr, r, q_in.data(), kept, fold_ready, next, alpha, beta, eps, workspace, hs); break;
+                case 2: rc = round_linear<2>(pr, lr, r, q_in.data(), kept, fold_ready, next, alpha, beta, eps, workspace, hs); break;
+                case 4: rc = round_linear<4>(pr, lr, r, q_in.data(), kept, fold_ready, next, alpha, beta, eps, workspace, hs); break;
+                default: rc = round_linear<8>(pr, lr, r, q_in.data(), kept, fold_ready, next, alpha, beta, eps, workspace, hs); break;
+            }
+            if (rc == CONEF_OK && made && want_next) *made = by_quads && by_fold ? 5 : 1;
+            return rc;
         }
         // the column kernels work in place: the fix launch leaves the new Q in q_next as well
         if (want_next && rp > 8 && columns)

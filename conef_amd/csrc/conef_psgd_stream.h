@@ -99,15 +99,75 @@ inline bool mqs_plan_launch(const MqsItem* items, int count, int rp, bool sketch
     return false;
 }
 
-template <int N>
-__device__ __forceinline__ void mqs_halve(float* v, int lane, int mask)
+// x_k -= b_ik x_i (k > i), x_i *= 1 / d_i for i = 0 .. r - 1: the reference's column steps
+// (powerSGD_hook.py:21-43) on one row, coefficients from t_l as gram_solve_lds leaves them
+template <int RP>
+__device__ __forceinline__ void gram_apply_row(float* x, const float* t_l)
 {
-    const bool hi = (lane & mask) != 0;
+#pragma unroll
+    for (int i = 0; i < RP; ++i) {
+#pragma unroll
+        for (int k = i + 1; k < RP; ++k) x[k] = fmaf(-t_l[i * RP + k], x[i], x[k]);
+        x[i] = __fmul_rn(x[i], t_l[RP * RP + i]);
+    }
+}
+
+template <int RP>
+__device__ __forceinline__ void load_row(const float* p, float* x)
+{
+    if (RP >= 4) {
+#pragma unroll
+        for (int c = 0; c < RP; c += 4) conef_ld4u(p + c, x + c);
+    } else {
+#pragma unroll
+        for (int c = 0; c < RP; ++c) x[c] = p[c];
+    }
+}
+
+template <int RP>
+__device__ __forceinline__ void store_row(float* p, const float* x)
+{
+    if (RP >= 4) {
+#pragma unroll
+        for (int c = 0; c < RP; c += 4) conef_st4u(p + c, x + c);
+    } else {
+#pragma unroll
+        for (int c = 0; c < RP; ++c) p[c] = x[c];
+    }
+}
+
+// The value of lane l ^ mask, by the crossing that mask has of its own (no index to form, and LDS for mask 4
+// alone).
+template <int MASK>
+__device__ __forceinline__ float mqs_xor(float v)
+{
+    const int x = __float_as_int(v);
+    if constexpr (MASK == 1) return __int_as_float(__builtin_amdgcn_mov_dpp(x, 0xb1, 0xf, 0xf, true));         // quad_perm [1, 0, 3, 2]
+    else if constexpr (MASK == 2) return __int_as_float(__builtin_amdgcn_mov_dpp(x, 0x4e, 0xf, 0xf, true));    // quad_perm [2, 3, 0, 1]
+    else if constexpr (MASK == 4) return __int_as_float(__builtin_amdgcn_ds_swizzle(x, (4 << 10) | 0x1f));
+    else if constexpr (MASK == 8) return __int_as_float(__builtin_amdgcn_mov_dpp(x, 0x128, 0xf, 0xf, true));   // row_ror 8
+    else return __shfl_xor(v, MASK, 64);
+}
+
+// One exchange of the butterfly: lanes with the mask's bit keep the upper N / 2 values, the others the lower,
+// each with its partner's added.  Across half waves and rows of 16 lanes an instruction swaps the two
+// values' halves, and the sum of what comes out is both lanes' result.
+template <int N, int MASK>
+__device__ __forceinline__ void mqs_halve(float* v, int lane)
+{
 #pragma unroll
     for (int i = 0; i < N / 2; ++i) {
-        const float keep = hi ? v[N / 2 + i] : v[i];
-        const float send = hi ? v[i] : v[N / 2 + i];
-        v[i] = keep + __shfl_xor(send, mask, 64);
+        if constexpr (MASK >= 16) {
+            const unsigned lo = __float_as_uint(v[i]), hi = __float_as_uint(v[N / 2 + i]);
+            const auto t = MASK == 32 ? __builtin_amdgcn_permlane32_swap(lo, hi, false, false)
+                                      : __builtin_amdgcn_permlane16_swap(lo, hi, false, false);
+            v[i] = __uint_as_float(t[0]) + __uint_as_float(t[1]);
+        } else {
+            const bool up = (lane & MASK) != 0;
+            const float keep = up ? v[N / 2 + i] : v[i];
+            const float send = up ? v[i] : v[N / 2 + i];
+            v[i] = keep + mqs_xor<MASK>(send);
+        }
     }
 }
 
@@ -116,14 +176,18 @@ __device__ __forceinline__ void mqs_halve(float* v, int lane, int mask)
 template <int NV>
 __device__ __forceinline__ void mqs_wave_reduce(float* v, int lane)
 {
-    if (NV >= 32) mqs_halve<(NV >= 32 ? 32 : 2)>(v, lane, 32);
-    if (NV >= 16) mqs_halve<(NV >= 16 ? 16 : 2)>(v, lane, NV >= 32 ? 16 : 32);
-    if (NV >= 8) mqs_halve<(NV >= 8 ? 8 : 2)>(v, lane, NV >= 32 ? 8 : NV >= 16 ? 16 : 32);
-    if (NV >= 4) mqs_halve<4>(v, lane, NV >= 32 ? 4 : NV >= 16 ? 8 : NV >= 8 ? 16 : 32);
-    mqs_halve<2>(v, lane, NV >= 32 ? 2 : NV >= 16 ? 4 : NV >= 8 ? 8 : NV >= 4 ? 16 : 32);
-    constexpr int kLeft = NV >= 32 ? 1 : NV >= 16 ? 2 : NV >= 8 ? 4 : NV >= 4 ? 8 : 16;   // lanes that still differ
-#pragma unroll
-    for (int mask = kLeft; mask >= 1; mask >>= 1) v[0] += __shfl_xor(v[0], mask, 64);
+    constexpr int kTop = NV >= 32 ? 32 : NV >= 16 ? 16 : NV >= 8 ? 8 : NV >= 4 ? 4 : 2;
+    mqs_halve<kTop, 32>(v, lane);
+    if constexpr (kTop >= 4) mqs_halve<kTop / 2, 16>(v, lane);
+    if constexpr (kTop >= 8) mqs_halve<kTop / 4, 8>(v, lane);
+    if constexpr (kTop >= 16) mqs_halve<kTop / 8, 4>(v, lane);
+    if constexpr (kTop >= 32) mqs_halve<kTop / 16, 2>(v, lane);
+    // the lanes that still differ
+    if constexpr (kTop < 4) v[0] += mqs_xor<16>(v[0]);
+    if constexpr (kTop < 8) v[0] += mqs_xor<8>(v[0]);
+    if constexpr (kTop < 16) v[0] += mqs_xor<4>(v[0]);
+    if constexpr (kTop < 32) v[0] += mqs_xor<2>(v[0]);
+    v[0] += mqs_xor<1>(v[0]);
 }
 
 template <int RP, int MODE, int T>
@@ -284,4 +348,98 @@ psgd_mqs_body(const MqsItem& it, float alpha, ConefSeeds hs, int bx)
             it.gram[(size_t)bx * NG + tid] = s;
         }
     }
+}
+
+// ------------------------------------------------------------ M = P Q^T ----
+// MODE 0: write M.  MODE 1: also write the dense residual E = X - M (X = what M held on entry).
+// Factors of rank RP exactly (rows of RP floats, 16-byte aligned), rows of at least four columns of
+// any alignment.  A thread owns a column quad, whose 4 x RP slice of Q stays in registers, and walks
+// rows four at a time with their loads in flight together.  A workgroup is cut into groups of
+// `lanes` threads that cover a row (or 1024 columns of it) and take rows in turn; lanes is a multiple
+// of 64 wherever a row has more than 64 quads, so that a wave's row of P is uniform and comes through
+// the scalar cache.
+struct PqtItem {
+    float* x;
+    float* err;
+    const float* p;
+    const float* q;
+    int64_t n;
+    int m, r, rows_per_slab, col_tiles;
+    int lanes;
+    const float* qi;         // not null: q laid out by quads (conef_load_slices)
+};
+
+typedef __attribute__((address_space(4))) float conef_cfloat;      // constant memory: uniform loads are scalar
+
+inline int pqt_lanes(int64_t m)
+{
+    const int64_t m4 = (m + 3) / 4;
+    return (int)(m4 >= 256 ? 256 : m4 > 64 ? (m4 + 63) / 64 * 64 : m4);
+}
+
+template <int RP, int MODE, bool UNIFORM>
+__device__ __forceinline__ void
+psgd_pqt_rows(float* __restrict__ x, float* __restrict__ err, const float* __restrict__ p, const float* __restrict__ q,
+              const float* __restrict__ qi, const PqtItem& it, int bx, int by)
+{
+    const int m = it.m, groups = 256 / it.lanes;
+    int grp = (int)threadIdx.x / it.lanes;
+    const int quad = bx * 256 + (int)threadIdx.x - grp * it.lanes;
+    if (UNIFORM) grp = __builtin_amdgcn_readfirstlane(grp);
+    if (grp >= groups || 4 * quad >= m) return;
+    const int col = conef_quad_col(quad, m), dup = 4 * quad - col;
+    const int64_t i0 = (int64_t)by * it.rows_per_slab;
+    const int64_t i1 = i0 + it.rows_per_slab < it.n ? i0 + it.rows_per_slab : it.n;
+    float qf[4 * RP];
+    conef_load_slices<RP>(conef_quad_slices<RP>(q, qi, quad, col, m), qf);
+    auto walk = [&](auto store) {
+        for (int64_t ib = i0 + grp; ib < i1; ib += 4 * groups) {
+            float xv[4][4];
+            if (MODE == 1) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int64_t i = ib + u * groups < i1 ? ib + u * groups : ib;
+                    conef_ld4u(x + i * m + col, xv[u]);
+                }
+            }
+            // The four rows of P: through constant memory where they are uniform.  (The pointers come out of a table:
+            // nothing else tells the compiler that the stores leave P alone, and the rows became vector loads
+            // behind them.)
+            float pv[4][RP];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int64_t i = ib + u * groups < i1 ? ib + u * groups : ib;
+                if (UNIFORM) {
+                    const conef_cfloat* ps = (const conef_cfloat*)(uintptr_t)(p + i * RP);
+#pragma unroll
+                    for (int c = 0; c < RP; ++c) pv[u][c] = ps[c];
+                } else {
+#pragma unroll
+                    for (int c = 0; c < RP; ++c) pv[u][c] = p[i * RP + c];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int64_t i = ib + u * groups;
+                if (i >= i1) break;
+                float mh[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int c = 0; c < RP; ++c) {
+                    const float pc = pv[u][c];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) mh[k] = fmaf(pc, qf[k * RP + c], mh[k]);
+                }
+                if (MODE == 1) {
+                    float ev[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) ev[k] = __fsub_rn(xv[u][k], mh[k]);
+                    store(err + i * m + col, ev);
+                }
+                store(x + i * m + col, mh);
+            }
+        }
+    };
+    // (rows of whole quads have a loop without the moved quad's test; uniform)
+    if (m % 4 == 0) walk([](float* at, const float* v) { conef_st4u(at, v); });
+    else walk([&](float* at, const float* v) { conef_st4_own(at, v, dup); });
 }

@@ -88,13 +88,14 @@ inline bool conef_rowlist_shape(int64_t n, int64_t d, int32_t w, bool cells, boo
 
 // ------------------------------------------------------------------ fronts ----
 // A front fills vals[row_in_tile * d + col] for the tile's rows.  `cells` (only when
-// kNeedsCells) holds the tile's old sketch rows, [rows][w].
+// kNeedsCells) holds the tile's old sketch rows, [rows][w]; a front with kParksCells puts them there itself
+// while it stages.
 
 // DenseCS.update: the value is the dense tensor itself.
 struct ConefListVec {
     const float* vec;
     bool vec_ok;           // base 16-byte aligned and d % 4 == 0 (the tile copy works either way)
-    static constexpr bool kNeedsCells = false;
+    static constexpr bool kNeedsCells = false, kParksCells = false;
     // whether a tensor with tiles to spare goes by half-height ones.  Full against half height: [50000,512] 40.2
     // and 29.9 us, [20000,2048] 49.0 and 45.9, [30522,1024] 37.0 and 36.2, [33278,650] 26.2 and 26.0, [60000,300]
     // and [33278,200] within 1 % either way.
@@ -155,7 +156,7 @@ struct ConefListRandBlock {
     float* payload;
     ConefBlock blk;
     float alpha;
-    static constexpr bool kNeedsCells = true;
+    static constexpr bool kNeedsCells = true, kParksCells = false;
     static bool halves(int64_t) { return true; }      // (the column table sits in LDS next to the tiles)
     static constexpr int kQuads = 4;
     struct Regs {          // a thread's first kQuads quads, by name: no array for the compiler to keep in memory
@@ -398,7 +399,7 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
     const int total = rows * w;
     constexpr int kPre = 8;
     float aux_pre[kPre];
-    if (!Front::kNeedsCells) {
+    if constexpr (!Front::kNeedsCells && !Front::kParksCells) {
 #pragma unroll
         for (int u = 0; u < kPre; ++u) {
             const int p = threadIdx.x + u * kConefRowlistThreads;
@@ -434,7 +435,7 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
             conef_copy_words_to_lds(csr_l + kPreC * kConefRowlistThreads, plan.csr + kPreC * kConefRowlistThreads,
                                     csr_words - kPreC * kConefRowlistThreads);
     }
-    if (!Front::kNeedsCells) {
+    if constexpr (!Front::kNeedsCells && !Front::kParksCells) {
 #pragma unroll
         for (int u = 0; u < kPre; ++u) {
             const int p = threadIdx.x + u * kConefRowlistThreads;

@@ -400,6 +400,13 @@ int conef_psgd_products_f32(const ConefPsgdItem* items, const ConefPsgdItem* fir
 #define CONEF_ROUND_NEXT_QUADS 4
 #define CONEF_ROUND_NEXT_WIDE 8
 #define CONEF_ROUND_QUADS_READY 16
+/* The further buffer is longer, by that many floats (R) times w, the item's sketch width, and R * (R + 1): a round with a
+ * sketched error (mq_mode 2, pqt_mode 2) at ranks up to 8 leaves there what its next round starts from - the factor
+ * as the products left it, its rows summed over the columns of each of the sketch's buckets with their signs, and
+ * the steps that orthogonalise it.  *made & 4 tells whether it did; CONEF_ROUND_FOLD_READY tells the next round,
+ * whose sketches must hash as this one's do. */
+#define CONEF_ROUND_NEXT_FOLD 32
+#define CONEF_ROUND_FOLD_READY 64
 int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_t mq_mode, int32_t pqt_mode, float alpha,
                                float beta, float eps, int32_t a, int32_t b, float* const* q_next, int32_t flags,
                                int32_t* made, void* workspace, int64_t workspace_bytes, void* stream);

@@ -1252,6 +1252,35 @@ def test_rounds_at_any_rank_and_alignment(monkeypatch, oracle, mode, rank):
         assert st.round_cache[0].q_next_ready == (st.round_cache[0].count > 0)
 
 
+# (shapes, sketch size, whether the round runs in linear form): widths around a quad, a wave's quads and the two workgroup
+# sizes, one and several slabs of columns, rows of one tile and a remainder; sketches of four buckets and (the general
+# path) three, wider than a slab of the matrix, as wide as the matrix
+LINEAR_ROUNDS = [
+    ([(300, 40), (9, 44), (130, 257)], 0.1, True),
+    ([(64, 33), (40, 32)], 0.1, False),
+    ([(1, 4000), (65, 2048), (33, 2051), (3,), (66, 1026)], 0.02, True),
+    ([(1030, 96), (70, 120)], 1.0, True),
+    ([(37, 5760), (640, 650)], 0.5, True),
+    ([(25, 9001), (12, 100)], 0.13, True),
+    ([(2100, 1024), (5000, 64)], 0.1, True),
+]
+
+
+@pytest.mark.parametrize("rank", [1, 2, 3, 4, 8])
+@pytest.mark.parametrize("case", range(len(LINEAR_ROUNDS)))
+def test_sketched_rounds_in_linear_form(monkeypatch, oracle, case, rank):
+    """A round whose products take a sketched error without it being laid out, over steps that start from what the last
+    one kept, against the oracle (sums of fp32 terms in another order: 1e-5, as for every round)."""
+    monkeypatch.setenv("CONEF_ROUND_SMALL", "0")
+    shapes, ss, linear = LINEAR_ROUNDS[case]
+    st, hook = _state_for("conef", rank, ss)
+    ost = oracle.PowerSGDOracle(matrix_approximation_rank=rank, error_mode="conef", sketch_size=ss, beta=0.9, topk_ratio=0.4)
+    run_steps(hook, st, ost, shapes, 3, check=psgd_check_factory(st, ost, "conef"),
+              resync=psgd_resync_factory(st, ost, "conef", free_steps=1))
+    plan = st.round_cache[0]
+    assert plan.count > 0 and plan.q_next_ready and plan.q_next_fold == linear
+
+
 @pytest.mark.parametrize("small", ["0", "1"])
 @pytest.mark.parametrize("mode,rank", [("ef", 3), ("conef", 4)])
 def test_round_of_more_matrices_than_a_launch_takes(monkeypatch, oracle, mode, rank, small):
