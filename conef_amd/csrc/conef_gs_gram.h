@@ -284,8 +284,10 @@ __device__ __forceinline__ void gsg_recurrence(double (*gram)[RP + 1], float (*c
         }
 #pragma unroll
         for (int u = 0; u < EPT; ++u) {
-            if (na[u] > 0) gram[ej[u]][ek[u]] = g[u];
             const int dj = ej[u] - i0;
+            // only below the panel: its own rows are not read again, but a wave that has yet to start this panel
+            // still reads them as they are
+            if (dj >= B) gram[ej[u]][ek[u]] = g[u];
             if (dj >= 0 && dj < B && ek[u] > ej[u]) {       // an entry of pivot row j is final after dj steps
                 double r = inv2[0];
 #pragma unroll
