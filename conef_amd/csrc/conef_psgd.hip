@@ -660,14 +660,19 @@ __device__ __forceinline__ void store_tight_row(float* dst, int64_t row, const f
         if (c < r) dst[row * r + c] = x[c];
 }
 
-// Ranks up to 8.  A row of P a thread.  A row of Q, a sum over as many slabs as there are (64 for a
-// [4096, 1024] matrix), four threads in different waves: they take a quarter of the slabs each.
+// Ranks up to 8.  A row of P a thread.  A row of Q is a sum over as many slabs as there are (64 for a [4096, 1024]
+// matrix, 256 for a narrow one), in ascending order: a thread per entry, with up to 64 of its slabs requested
+// together, then a thread per row for T.  The launch is one chain of trips to memory (the slabs lie in other XCDs' caches):
+// with a thread per row of Q and four slabs in flight a launch of the LSTM's [33278, 650] at rank 4 took 10.9 us
+// and of four [4096, 1024] at rank 8 8.4, now 5.7 and 6.4; with four threads per row that add a quarter of
+// the slabs each it took as long, but added them in another order.
 constexpr int kFixQRows = 64;
+constexpr int fix_threads(int rp) { return rp == 8 ? 8 * kFixQRows : 4 * kFixQRows; }
 
 template <int RP>
 __device__ __forceinline__ void fix_p_rows(const DeferFixItem& it, int block, const float* t_l)
 {
-    const int64_t row = (int64_t)block * 256 + threadIdx.x;
+    const int64_t row = (int64_t)block * fix_threads(RP) + threadIdx.x;
     float x[RP];
     load_row<RP>(it.p + (row < it.n ? row : it.n - 1) * RP, x);
     __syncthreads();
@@ -681,24 +686,31 @@ __device__ __forceinline__ void fix_p_rows(const DeferFixItem& it, int block, co
     if (row < it.n) store_row<RP>(it.p + row * RP, x);
 }
 
-// sums slabs [s0, s1) of a row in ascending order, eight requested together
-template <int RP>
-__device__ __forceinline__ void fix_sum_slabs(const float* src, int64_t stride, int s0, int s1, float* out)
+// adds U slabs of an entry, `left` of which are there
+template <int U>
+__device__ __forceinline__ float fix_add_slabs(const float* src, int64_t stride, int left, float sum)
 {
+    float v[U];
 #pragma unroll
-    for (int c = 0; c < RP; ++c) out[c] = 0.f;
-    for (int sl = s0; sl < s1; sl += 8) {
-        float v[8][RP];
+    for (int u = 0; u < U; ++u) v[u] = src[(int64_t)(u < left ? u : left - 1) * stride];
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-            if (sl + u < s1) load_row<RP>(src + (int64_t)(sl + u) * stride, v[u]);
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            if (sl + u < s1) {
-#pragma unroll
-                for (int c = 0; c < RP; ++c) out[c] += v[u][c];
-            }
+    for (int u = 0; u < U; ++u)
+        if (u < left) sum += v[u];                          // uniform
+    return sum;
+}
+
+__device__ __forceinline__ float fix_sum_slabs(const float* src, int64_t stride, int slabs)
+{
+    float sum = 0.f;
+    for (int at = 0; at < slabs; at += 64) {
+        const float* from = src + (int64_t)at * stride;
+        const int left = slabs - at;
+        if (left > 32) sum = fix_add_slabs<64>(from, stride, left, sum);
+        else if (left > 16) sum = fix_add_slabs<32>(from, stride, left, sum);
+        else if (left > 8) sum = fix_add_slabs<16>(from, stride, left, sum);
+        else sum = fix_add_slabs<8>(from, stride, left, sum);
     }
+    return sum;
 }
 
 // a finished row of Q
@@ -734,12 +746,12 @@ __device__ __forceinline__ double fix_gram_quarter(const float (*rows_l)[RP + 1]
 }
 
 template <int RP>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(fix_threads(RP))
 psgd_defer_fix_batch_kernel(PsgdBatch<DeferFixItem> b, float alpha)
 {
     constexpr int NG = RP * (RP + 1) / 2;
     __shared__ float t_l[RP * RP + RP];
-    __shared__ float rows_l[256][RP + 1];
+    __shared__ float rows_l[kFixQRows][RP + 1];
     __shared__ double part_l[NG][4];
     int local;
     const DeferFixItem& it = b.item[psgd_batch_locate(b, &local)];
@@ -748,36 +760,32 @@ psgd_defer_fix_batch_kernel(PsgdBatch<DeferFixItem> b, float alpha)
         fix_p_rows<RP>(it, local, t_l);
         return;
     }
-    const int lrow = threadIdx.x & (kFixQRows - 1), part = __builtin_amdgcn_readfirstlane(threadIdx.x / kFixQRows);
-    const int64_t row = (int64_t)(local - it.pblocks) * kFixQRows + lrow;
-    const int64_t rc = row < it.m ? row : it.m - 1;
-    const int s0 = it.slabs * part / 4, s1 = it.slabs * (part + 1) / 4;
-    const uint32_t pk = it.cs_src ? it.pk[rc] : 0u;
-    float x[RP];
-    fix_sum_slabs<RP>(it.qsrc + rc * RP, it.m * RP, s0, s1, x);
-    if (it.cs_src) {
-        float y[RP];
-        fix_sum_slabs<RP>(it.cs_src + (int64_t)(pk & 0x7fffffffu) * RP, (int64_t)it.w * RP, s0, s1, y);
-        const float f = conef_apply_sign(alpha, pk);
-#pragma unroll
-        for (int c = 0; c < RP; ++c) x[c] = fmaf(f, y[c], x[c]);
+    const int64_t row0 = (int64_t)(local - it.pblocks) * kFixQRows;
+    if ((int)threadIdx.x < kFixQRows * RP) {
+        const int lrow = threadIdx.x / RP, c = threadIdx.x % RP;
+        const int64_t rc = row0 + lrow < it.m ? row0 + lrow : it.m - 1;
+        const uint32_t pk = it.cs_src ? it.pk[rc] : 0u;
+        float x = fix_sum_slabs(it.qsrc + rc * RP + c, it.m * RP, it.slabs);
+        if (it.cs_src) {
+            const float y = fix_sum_slabs(it.cs_src + (int64_t)(pk & 0x7fffffffu) * RP + c, (int64_t)it.w * RP, it.slabs);
+            x = fmaf(conef_apply_sign(alpha, pk), y, x);
+        }
+        rows_l[lrow][c] = x;
     }
-#pragma unroll
-    for (int c = 0; c < RP; ++c) rows_l[threadIdx.x][c] = x[c];
     __syncthreads();
-    if (part == 0) {
+    if (threadIdx.x < kFixQRows) {
+        const int64_t row = row0 + threadIdx.x;
+        float x[RP];
 #pragma unroll
-        for (int u = 1; u < 4; ++u)
-#pragma unroll
-            for (int c = 0; c < RP; ++c) x[c] += rows_l[u * kFixQRows + lrow][c];
+        for (int c = 0; c < RP; ++c) x[c] = rows_l[threadIdx.x][c];
         gram_apply_row<RP>(x, t_l);
         fix_store_q<RP>(it, row, x);
+        if (it.qgram) {
+#pragma unroll
+            for (int c = 0; c < RP; ++c) rows_l[threadIdx.x][c] = row < it.m ? x[c] : 0.f;
+        }
     }
     if (it.qgram) {                                         // uniform over the workgroup
-        if (part == 0) {
-#pragma unroll
-            for (int c = 0; c < RP; ++c) rows_l[lrow][c] = row < it.m ? x[c] : 0.f;
-        }
         __syncthreads();
         const double s = fix_gram_quarter<RP>(rows_l);
         if ((int)(threadIdx.x >> 2) < NG) part_l[threadIdx.x >> 2][threadIdx.x & 3] = s;
@@ -3304,7 +3312,7 @@ int defer_fix(const PaddedRound& pr, int r, const std::vector<MtpRaw>& raw, cons
               const std::vector<double*>* qgrams, hipStream_t s, const std::vector<CellRaw>* cells = nullptr, float alpha = 0.f)
 {
     const int rp = pr.rp, count = (int)pr.items.size();
-    const int rows_per_wg = rp <= 8 ? 256 : 256 / (rp / 4), qrows_per_wg = rp <= 8 ? kFixQRows : rows_per_wg;
+    const int rows_per_wg = rp <= 8 ? fix_threads(rp) : 256 / (rp / 4), qrows_per_wg = rp <= 8 ? kFixQRows : rows_per_wg;
     std::vector<DeferFixItem> fix;
     std::vector<int> blocks;
     for (int k = 0; k < count; ++k) {
@@ -3317,7 +3325,7 @@ int defer_fix(const PaddedRound& pr, int r, const std::vector<MtpRaw>& raw, cons
         blocks.push_back(pb + qb);
     }
     return run_batches(fix, blocks, [&](const PsgdBatch<DeferFixItem>& bt, int grid) {
-        const dim3 g((unsigned)grid), t(256);
+        const dim3 g((unsigned)grid), t((unsigned)(rp <= 8 ? fix_threads(rp) : 256));
         switch (rp) {
             case 1: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<1>, g, t, 0, s, bt, alpha); break;
             case 2: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<2>, g, t, 0, s, bt, alpha); break;
