@@ -8,6 +8,7 @@ library is missing the import of any op fails loudly.
 """
 import ctypes
 import os
+import weakref
 
 import numpy as np
 import torch
@@ -21,7 +22,7 @@ _I32 = ctypes.c_int32
 _F32 = ctypes.c_float
 
 # name -> argtypes; every function returns int (0 = ok, >0 hipError_t, -1 invalid argument, -2 too large),
-# except the *_bytes functions, which return a byte count as int64
+# except the *_bytes functions, which return a byte count as int64, and conef_tape_create, which returns a handle
 SIGNATURES = {
     "conef_version": [],
     "conef_hash_table_i32": [_P, _P, _I64, _I32, _I32, _I32, _I32, _I32, _P],
@@ -72,6 +73,11 @@ SIGNATURES = {
     "conef_ef_passthrough_batch_f32": [_P, _P, _P, _I32, _P],
     "conef_psgd_q_next_f32": [_P, _I32, _F32, _P, _P, _P, _I64, _P],
     "conef_ef_passthrough_f32": [_P, _P, _I64, _P],
+    "conef_tape_create": [],
+    "conef_tape_destroy": [_I64],
+    "conef_tape_record": [_I64],
+    "conef_tape_stop": [_I64, _P, _I32, _I32],
+    "conef_tape_replay": [_I64, _P, _I32, _P],
     "conef_plan_bytes": [_I64, _I64, _I32, _I32, _I32],
     "conef_plan_build_host": [_P, _I64, _I64, _I64, _I32, _I32, _I32, _I32, _I32],
     "conef_plan_build_host_seeded": [_P, _I64, _I64, _I64, _I32, _I32, _I32, _I32, _I32, _I32, _I32],
@@ -99,6 +105,24 @@ class PsgdItem(ctypes.Structure):
                 ("n", _I64), ("m", _I64), ("r", _I32), ("w", _I32)]
 
 
+TAPE_STALE = -3
+
+
+class Tape:
+    """A round's launches kept by the library (conef_tape_record of include/conef_hip.h)."""
+    __slots__ = ("handle", "signature", "seen", "__weakref__")
+
+    def __init__(self):
+        self.handle = 0
+        self.signature = self.seen = None        # what the kept launches were formed for; what the last round was
+
+    def record(self, lib):
+        if not self.handle:
+            self.handle = lib.conef_tape_create()
+            weakref.finalize(self, lib.conef_tape_destroy, self.handle)
+        check(lib.conef_tape_record(self.handle), "conef_tape_record")
+
+
 class RandBlockItem(ctypes.Structure):
     """ConefRandBlockItem of include/conef_hip.h: one tensor of a bucket for conef_randblock_step_batch_f32."""
     _fields_ = [("x", _P), ("err", _P), ("cs_in", _P), ("cs_out", _P), ("payload", _P), ("plan_host", _P),
@@ -115,7 +139,7 @@ def randblock_starts(items, count):
 
 _RETURNS_I64 = ("conef_topk_workspace_bytes", "conef_topk_batch_workspace_bytes", "conef_topk_batch_list_bytes", "conef_plan_bytes",
                 "conef_plan_workspace_bytes", "conef_psgd_workspace_bytes", "conef_psgd_batch_workspace_bytes",
-                "conef_psgd_round_small_workspace_bytes")
+                "conef_psgd_round_small_workspace_bytes", "conef_tape_create")
 
 _handle = None
 

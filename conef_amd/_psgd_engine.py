@@ -137,7 +137,7 @@ class _RoundPlan:
     compressed, the table of matrices the batch entry points read, the views into the P / Q
     arenas.  Built on the first step of a bucket and reused while the bucket keeps its buffer
     and layout, so that a step costs a handful of foreign calls however many tensors it has."""
-    __slots__ = ("small", "layout", "cells", "cs_static", "env_ahead", "env_topk_side", "env_small", "key", "shapes", "work", "passthrough", "before", "after", "total_ps", "total_qs", "arena_key", "ps",
+    __slots__ = ("small", "layout", "cells", "cs_static", "env_ahead", "env_topk_side", "env_small", "env_check_gs", "tape", "key", "shapes", "work", "passthrough", "before", "after", "total_ps", "total_qs", "arena_key", "ps",
                  "qs", "items", "count", "sketches", "fused_sketch", "batched_update", "residual_offsets",
                  "topk_table", "q_next", "q_next_ptrs", "q_next_ready", "q_next_quads", "q_next_fold", "made", "q_next_event", "aside_recorded",
                  "topk_event", "ws_need", "handoff_event", "topk_number", "q_next_number", "is_wide", "wide", "chunks", "runs", "ef_spans")
@@ -189,6 +189,8 @@ def _build_round(state, grads, shapes, key, error_mode):
     plan.env_ahead = os.environ.get("CONEF_ROUND_AHEAD", "1") != "0"
     plan.env_topk_side = os.environ.get("CONEF_TOPK_SIDE", "1") != "0"
     plan.env_small = os.environ.get("CONEF_ROUND_SMALL", "1") != "0"
+    plan.env_check_gs = os.environ.get("CONEF_CHECK_GS", "0") == "1"
+    plan.tape = _lib.Tape() if os.environ.get("CONEF_ROUND_TAPE", "1") != "0" else None      # the round's launches, kept (_lib.Tape)
     plan.work, plan.passthrough = [], []
     plan.before = plan.after = plan.total_ps = plan.total_qs = 0
     for tensor in grads:                                            # Step I (:394-418)
@@ -429,6 +431,8 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
         for cnt, (matrix, n, m, rank) in enumerate(work):
             if cnt not in errs:
                 errs[cnt] = torch.zeros_like(matrix)
+                if plan.tape is not None:
+                    plan.tape.signature = None
                 plan.topk_table = None       # perhaps at the address of a dropped one, and yet another allocation
             items[cnt].err = errs[cnt].data_ptr()
     elif error_mode == "conef":
@@ -490,13 +494,8 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
         # rows: query as a pass of its own (P = M Q then runs without a fused error add)
         for cnt, (matrix, n, m, rank) in enumerate(work):
             errs[cnt].query(matrix.view(m, n), alpha)
-    if error_mode == "ef":
-        # tensors that are not compressed: g += e, and their new error is exactly zero (:361,:558)
-        if plan.ef_spans is None:
-            plan.ef_spans = _ef_spans(plan, base_ptr, dense_err.data_ptr())
-        if plan.ef_spans[3]:
-            rc = lib.conef_ef_passthrough_batch_f32(*plan.ef_spans, stream)
-            _lib.check(rc, "conef_ef_passthrough_batch_f32")
+    if error_mode == "ef" and plan.ef_spans is None:
+        plan.ef_spans = _ef_spans(plan, base_ptr, dense_err.data_ptr())
 
     # The round itself, one foreign call: orthogonalise all Q side by side; pass 1, the error add
     # fused into P = M Q; orthogonalise all P; pass 2, Q = M^T P; pass 3, M = P Q^T with the
@@ -518,6 +517,76 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
         mode3 = 3 if error_mode == "conef" and plan.batched_update else 1
     else:
         mode3 = 0
+    beta3 = float(state.beta) if mode3 in (2, 3) else 0.0
+    topk_aside = error_mode == "topk" and count and streams <= 1 and plan.env_ahead and plan.env_topk_side
+
+    # A step like the last one - the same tables, scalars and buffers - makes the launches the last one made
+    # (_lib.Tape; the tables are compared natively).  What a round starts on other streams is not kept.
+    tape = plan.tape
+    if tape is not None and (need_randomize_qs or plan.is_wide or not count or error_mode == "conef_v2" or not state.warm_start
+                             or mode1 == 2 and not plan.cs_static
+                             or residual is not None and (mode3 != 3 or streams <= 1)
+                             or state.matrix_approximation_rank > 8 and streams <= 1):
+        tape = None
+    if tape is not None:
+        signature = (plan.q_next_ready, plan.q_next_quads, plan.q_next_fold, mode1, mode3, alpha, beta3, eps, ws_ptr, ws_len,
+                     stream, topk_aside, getattr(state, "topk_ratio", None) if error_mode == "topk" else None)
+        if signature == tape.signature:
+            rc = lib.conef_tape_replay(tape.handle, items, count, stream)
+            if rc == 0:
+                if topk_aside:
+                    _sparsify_aside(plan, [errs[cnt] for cnt in range(count)], state.topk_ratio, device)
+                return _end_round(state, plan, bucket, bucket_index, input_tensor)
+            if rc != _lib.TAPE_STALE:
+                _lib.check(rc, "conef_tape_replay")
+    if plan.tape is not None:
+        plan.tape.signature = None       # a round that makes its launches anew may replace what the kept ones point to
+    if tape is not None and signature != tape.seen:
+        tape.seen, tape = signature, None        # kept from the second such round on: a single one costs nothing more
+    if tape is not None:
+        tape.record(lib)
+        done = False
+        try:
+            _issue_round(state, plan, lib, errs, error_mode, mode1, mode3, alpha, beta3, eps, ws_ptr, ws_len, stream, streams, residual,
+                         topk_aside, device, dtype)
+            # (a round that leaves the second buffer in another state than it found it in is not the next one's;
+            # nor is one whose top-k lists lie elsewhere than in this workspace)
+            done = (signature[:3] == (plan.q_next_ready, plan.q_next_quads, plan.q_next_fold)
+                    and (error_mode != "topk" or topk_aside or plan.topk_table.list_bytes <= ws_len))
+        finally:
+            lib.conef_tape_stop(tape.handle, items, count, done)
+        tape.signature = signature if done else None
+    else:
+        _issue_round(state, plan, lib, errs, error_mode, mode1, mode3, alpha, beta3, eps, ws_ptr, ws_len, stream, streams, residual,
+                     topk_aside, device, dtype)
+    if topk_aside:
+        # The sparsification only touches the error tensors, which nobody reads before this bucket's
+        # next round: it runs on a side stream while this stream goes on with the next bucket
+        # (streaming passes next to launches that are mostly latency).  Same kernels, same values.
+        _sparsify_aside(plan, [errs[cnt] for cnt in range(count)], state.topk_ratio, device)
+    return _end_round(state, plan, bucket, bucket_index, input_tensor)
+
+
+def _end_round(state, plan, bucket, bucket_index, input_tensor):
+    if not state.warm_start:
+        state.p_memory_dict.clear()
+        state.q_memory_dict.clear()
+
+    if plan.env_check_gs and gram_schmidt_give_ups():
+        raise RuntimeError("a Gram-Schmidt workgroup gave up waiting for its neighbours: the factors of bucket %d hold NaN"
+                           % bucket_index)
+    state.maybe_increase_iter(bucket)
+    return _bucket.completed_future(input_tensor)
+
+
+def _issue_round(state, plan, lib, errs, error_mode, mode1, mode3, alpha, beta3, eps, ws_ptr, ws_len, stream, streams, residual,
+                 topk_aside, device, dtype):
+    """The launches of a round."""
+    work, items, count = plan.work, plan.items, plan.count
+    if error_mode == "ef" and plan.ef_spans[3]:
+        # tensors that are not compressed: g += e, and their new error is exactly zero (:361,:558)
+        rc = lib.conef_ef_passthrough_batch_f32(*plan.ef_spans, stream)
+        _lib.check(rc, "conef_ef_passthrough_batch_f32")
     if plan.is_wide:
         # A rank above 32: the error is added in passes of its own, the round runs on column chunks of
         # the factors, and the residual leaves the round dense (a sketch is updated from it below).
@@ -538,7 +607,6 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
                     and all(lib.conef_psgd_round_small_fits(run, part, mode1, mode3, HASH_A, HASH_B)
                             for run, part in plan.runs))
         plan.small = ((mode1, mode3), fits)
-    beta3 = float(state.beta) if mode3 in (2, 3) else 0.0
     if plan.is_wide:
         pass
     elif plan.small[1]:
@@ -588,27 +656,12 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
                                           ws_ptr, ws_len, stream)
             _lib.check(rc, "conef_psgd_round_f32")
     if error_mode == "topk":
-        if count and streams <= 1 and plan.env_ahead and plan.env_topk_side:
-            # The sparsification only touches the error tensors, which nobody reads before this bucket's
-            # next round: it runs on a side stream while this stream goes on with the next bucket
-            # (streaming passes next to launches that are mostly latency).  Same kernels, same values.
-            _sparsify_aside(plan, [errs[cnt] for cnt in range(count)], state.topk_ratio, device)
-        else:
+        if not topk_aside:
             plan.topk_table = topk_sparsify_all([errs[cnt] for cnt in range(count)], state.topk_ratio, plan.topk_table)
     elif residual is not None and mode3 != 3:
         for cnt, (matrix, n, m, rank) in enumerate(work):
             res = residual[plan.residual_offsets[cnt]: plan.residual_offsets[cnt + 1]]
             errs[cnt].update(res.view(n, m) if error_mode == "conef" else res.view(m, n), state.beta)
-
-    if not state.warm_start:
-        state.p_memory_dict.clear()
-        state.q_memory_dict.clear()
-
-    if os.environ.get("CONEF_CHECK_GS", "0") == "1" and gram_schmidt_give_ups():
-        raise RuntimeError("a Gram-Schmidt workgroup gave up waiting for its neighbours: the factors of bucket %d hold NaN"
-                           % bucket_index)
-    state.maybe_increase_iter(bucket)
-    return _bucket.completed_future(input_tensor)
 
 
 def _at(array, index):

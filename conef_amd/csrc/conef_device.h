@@ -1,5 +1,6 @@
 // Device-side building blocks shared by the ConEF kernels (gfx950 only).
 #pragma once
+#include "conef_tape.h"
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 #include <stdint.h>

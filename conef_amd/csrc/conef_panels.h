@@ -301,7 +301,7 @@ int conef_launch_panels(Front front, ConefPanelView plan, const CsT* cs_in, CsT*
     hipError_t e = conef_allow_lds((const void*)k, shape.lds);
     if (e != hipSuccess) return (int)e;
     const double omb = 1. - (double)beta;   // (1. - beta) with beta an fp32 value, CountSketch.py:38,63
-    hipLaunchKernelGGL(k, dim3((unsigned)shape.tiles), dim3(kConefPanelThreads), shape.lds, s, front, plan, cs_in, cs_out,
+    conef_launch(k, dim3((unsigned)shape.tiles), dim3(kConefPanelThreads), shape.lds, s, front, plan, cs_in, cs_out,
                        n, (int)d, (int)w, shape.rb, omb);
     return (int)hipGetLastError();
 }

@@ -730,12 +730,12 @@ int conef_launch_stage_rows(Stage stage, const ConefPlanHeader* hp, const void* 
         auto ka = conef_binned_stage_kernel<NROWS, Stage, true>;
         e = conef_allow_lds((const void*)ka, lds_a);
         if (e != hipSuccess) return (int)e;
-        hipLaunchKernelGGL(ka, dim3(ga, groups), dim3(threads_a), lds_a, s, stage, view, staging, hp->d, ga, row_first);
+        conef_launch(ka, dim3(ga, groups), dim3(threads_a), lds_a, s, stage, view, staging, hp->d, ga, row_first);
     } else {
         auto ka = conef_binned_stage_kernel<NROWS, Stage, false>;
         e = conef_allow_lds((const void*)ka, lds_a);
         if (e != hipSuccess) return (int)e;
-        hipLaunchKernelGGL(ka, dim3(ga, groups), dim3(threads_a), lds_a, s, stage, view, staging, hp->d, ga, row_first);
+        conef_launch(ka, dim3(ga, groups), dim3(threads_a), lds_a, s, stage, view, staging, hp->d, ga, row_first);
     }
     return (int)hipGetLastError();
 }
@@ -765,7 +765,7 @@ int conef_launch_accumulate_rows(const ConefPlanHeader* hp, const void* plan_dev
     double mean_seg = (double)hp->chunk_cols * hp->bin_buckets / (double)hp->w * 1.3;
     int glog = 3;
     while (glog < 6 && (1 << glog) < mean_seg) ++glog;
-    hipLaunchKernelGGL(kb, dim3(gb, groups), dim3(threads_b), lds_b, s, staging, view, cs_in, cs_out, hp->w, alpha, omb, gb,
+    conef_launch(kb, dim3(gb, groups), dim3(threads_b), lds_b, s, staging, view, cs_in, cs_out, hp->w, alpha, omb, gb,
                        hp->max_bin_records, glog, col_threads, bw, row_first, hp->d);
     return (int)hipGetLastError();
 }

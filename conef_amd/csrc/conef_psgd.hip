@@ -11,6 +11,8 @@
 // the passes that touch M anyway.  Sums that cross workgroups meet through a caller-provided
 // workspace in a fixed order: no atomics, results do not change from run to run.
 #include <cstdlib>
+#include <cstring>
+#include <new>
 #include <type_traits>
 #include <algorithm>
 #include <atomic>
@@ -1924,10 +1926,10 @@ int mqs_run(const std::vector<MqsItem>& table, int rp, float alpha, ConefSeeds h
     do {                                                                                                            \
         if (RP >= 16) break;                                                                                        \
         if (c.T == 256)                                                                                             \
-            hipLaunchKernelGGL((psgd_mqs_batch_kernel<(RP < 16 ? RP : 8), MODE, 256>), dim3((unsigned)total), dim3(256),  \
+            conef_launch((psgd_mqs_batch_kernel<(RP < 16 ? RP : 8), MODE, 256>), dim3((unsigned)total), dim3(256),  \
                                c.lds, s, b, alpha, hs);                                                             \
         else                                                                                                        \
-            hipLaunchKernelGGL((psgd_mqs_batch_kernel<(RP < 16 ? RP : 8), MODE, 1024>), dim3((unsigned)total), dim3(1024), \
+            conef_launch((psgd_mqs_batch_kernel<(RP < 16 ? RP : 8), MODE, 1024>), dim3((unsigned)total), dim3(1024), \
                                c.lds, s, b, alpha, hs);                                                             \
     } while (0)
         CONEF_RANK_SWITCH(rp, CONEF_MQS)
@@ -1960,11 +1962,11 @@ int launch_mq(float* x, const float* err, const float* cs, const uint32_t* pktab
             float* out = g.splits > 1 ? (float*)workspace : p;
             auto k = psgd_mfma_mq_kernel<MODE>;
             if (hipError_t e = conef_allow_lds((const void*)k, lds); e != hipSuccess) return (int)e;
-            hipLaunchKernelGGL(k, dim3((unsigned)g.row_tiles, (unsigned)g.splits), dim3(kMfmaThreads), lds, s, x, err, cs,
+            conef_launch(k, dim3((unsigned)g.row_tiles, (unsigned)g.splits), dim3(kMfmaThreads), lds, s, x, err, cs,
                                pktab, q, out, n, (int)m, r, g.cols_per_split, mod, alpha, hs);
             if (g.splits > 1) {
                 int64_t count = n * r;
-                hipLaunchKernelGGL(psgd_sum_partials_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, out,
+                conef_launch(psgd_sum_partials_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, out,
                                    p, count, g.splits);
             }
             return (int)hipGetLastError();
@@ -1985,7 +1987,7 @@ int launch_mq(float* x, const float* err, const float* cs, const uint32_t* pktab
     if (lds > 64 * 1024) return CONEF_ERR_INVALID;   // sketch rows wider than 16K cells per matrix row group
     dim3 grid((unsigned)((n + rb - 1) / rb));
 #define CONEF_MQ_GO(RB, RP, F)                                                                                    \
-    hipLaunchKernelGGL((psgd_mq_kernel<RB, RP, MODE, F>), grid, dim3(256), lds, s, x, err, cs, pktab, q, p, n, (int)m, \
+    conef_launch((psgd_mq_kernel<RB, RP, MODE, F>), grid, dim3(256), lds, s, x, err, cs, pktab, q, p, n, (int)m, \
                        r, mod, alpha, hs)
 #define CONEF_MQ(RP)                                     \
     do {                                                 \
@@ -2090,7 +2092,7 @@ inline int gs_launch_reg_batch(const GsBatch& batch, int count, int r, int slots
 {
     if (slots == 0) {
 #define CONEF_GSM(RP) \
-    hipLaunchKernelGGL((gram_schmidt_reg_mixed_kernel<RP>), dim3((unsigned)count), dim3(kGsRegThreads), 0, s, batch, r, eps)
+    conef_launch((gram_schmidt_reg_mixed_kernel<RP>), dim3((unsigned)count), dim3(kGsRegThreads), 0, s, batch, r, eps)
         switch (rank_bound(r)) {
             case 1: CONEF_GSM(1); break;
             case 2: CONEF_GSM(2); break;
@@ -2102,7 +2104,7 @@ inline int gs_launch_reg_batch(const GsBatch& batch, int count, int r, int slots
         return (int)hipGetLastError();
     }
 #define CONEF_GSR_GO(RP, RPT) \
-    hipLaunchKernelGGL((gram_schmidt_reg_kernel<RP, (RPT)>), dim3((unsigned)count), dim3(kGsRegThreads), 0, s, batch, r, eps)
+    conef_launch((gram_schmidt_reg_kernel<RP, (RPT)>), dim3((unsigned)count), dim3(kGsRegThreads), 0, s, batch, r, eps)
 #define CONEF_GSR(RP)                                                       \
     do {                                                                    \
         constexpr int kAll = kGsRegFloats / RP;                             \
@@ -2162,7 +2164,7 @@ inline hipError_t gsw_go(const GswBatch& batch, int count, float eps, hipStream_
                                                hipFuncAttributeMaxDynamicSharedMemorySize, kLds)
                          : hipSuccess;
     if (attr != hipSuccess) return attr;
-    hipLaunchKernelGGL((gsw_kernel<RP, RPT, CW>), dim3((unsigned)count), dim3(64 * RP / CW), kLds, s, batch, eps);
+    conef_launch((gsw_kernel<RP, RPT, CW>), dim3((unsigned)count), dim3(64 * RP / CW), kLds, s, batch, eps);
     return hipGetLastError();
 }
 
@@ -2196,8 +2198,9 @@ inline int gsl_launch(const GslBatch& batch, int count, int r, int rpt, int wgs,
                                                                                             : (const void*)gsl_kernel<8, 16>;
 #undef CONEF_GSL
     if (!fn) return CONEF_ERR_INVALID;
-    hipLaunchKernelGGL(gsl_reset_kernel, dim3(8), dim3(1024), 0, s, ws, wgs);
+    conef_launch(gsl_reset_kernel, dim3(8), dim3(1024), 0, s, ws, wgs);
     void* args[] = {(void*)&batch, (void*)&count, (void*)&eps, (void*)&ws};
+    conef_launch_unkept();
     hipError_t e = hipLaunchCooperativeKernel(fn, dim3((unsigned)wgs), dim3(kGslThreads), args, 0, s);
     if (e != hipSuccess) (void)hipGetLastError();
     return (int)e;
@@ -2230,12 +2233,11 @@ std::atomic<unsigned> g_small_launches{0};
 // side by side; the waits inside are bounded either way.
 inline int gsg_launch(const GsgBatch& batch, int count, int r, int wgs, float eps, void* workspace, hipStream_t s)
 {
-    unsigned tag = (g_gsg_launches.fetch_add(1u) + 1u) * 0x9E3779B9u;
-    if (tag == 0u) tag = 1u;
+    const unsigned tag = 0u;      // drawn by conef_launch_tagged
     GsgWs* ws = (GsgWs*)workspace;
-    if (r == 32) hipLaunchKernelGGL(gsg_kernel<32>, dim3((unsigned)wgs), dim3(kGsgThreads), 0, s, batch, count, eps, ws, tag);
-    else if (r == 16) hipLaunchKernelGGL(gsg_kernel<16>, dim3((unsigned)wgs), dim3(kGsgThreads), 0, s, batch, count, eps, ws, tag);
-    else if (r == 8) hipLaunchKernelGGL(gsg_kernel<8>, dim3((unsigned)wgs), dim3(kGsgThreads), 0, s, batch, count, eps, ws, tag);
+    if (r == 32) conef_launch_tagged<4>(g_gsg_launches, gsg_kernel<32>, dim3((unsigned)wgs), dim3(kGsgThreads), 0, s, batch, count, eps, ws, tag);
+    else if (r == 16) conef_launch_tagged<4>(g_gsg_launches, gsg_kernel<16>, dim3((unsigned)wgs), dim3(kGsgThreads), 0, s, batch, count, eps, ws, tag);
+    else if (r == 8) conef_launch_tagged<4>(g_gsg_launches, gsg_kernel<8>, dim3((unsigned)wgs), dim3(kGsgThreads), 0, s, batch, count, eps, ws, tag);
     else return CONEF_ERR_INVALID;
     return (int)hipGetLastError();
 }
@@ -2335,12 +2337,12 @@ int conef_psgd_mtp_f32(const float* x, const float* p, float* q, int64_t n, int6
             dst = (float*)workspace;
         }
         dim3 grid((unsigned)t.col_tiles, (unsigned)t.slabs);
-        if (t.v == 4) hipLaunchKernelGGL(psgd_mfma_mtp_kernel<4>, grid, dim3(kMfmaThreads), 0, s, x, p, dst, n, (int)m, r, t.rows_per_slab);
-        else if (t.v == 2) hipLaunchKernelGGL(psgd_mfma_mtp_kernel<2>, grid, dim3(kMfmaThreads), 0, s, x, p, dst, n, (int)m, r, t.rows_per_slab);
-        else hipLaunchKernelGGL(psgd_mfma_mtp_kernel<1>, grid, dim3(kMfmaThreads), 0, s, x, p, dst, n, (int)m, r, t.rows_per_slab);
+        if (t.v == 4) conef_launch(psgd_mfma_mtp_kernel<4>, grid, dim3(kMfmaThreads), 0, s, x, p, dst, n, (int)m, r, t.rows_per_slab);
+        else if (t.v == 2) conef_launch(psgd_mfma_mtp_kernel<2>, grid, dim3(kMfmaThreads), 0, s, x, p, dst, n, (int)m, r, t.rows_per_slab);
+        else conef_launch(psgd_mfma_mtp_kernel<1>, grid, dim3(kMfmaThreads), 0, s, x, p, dst, n, (int)m, r, t.rows_per_slab);
         if (t.slabs > 1) {
             int64_t count = m * r;
-            hipLaunchKernelGGL(psgd_sum_partials_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, dst, q,
+            conef_launch(psgd_sum_partials_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, dst, q,
                                count, t.slabs);
         }
         return (int)hipGetLastError();
@@ -2355,16 +2357,16 @@ int conef_psgd_mtp_f32(const float* x, const float* p, float* q, int64_t n, int6
     dim3 grid((unsigned)g.col_tiles, (unsigned)g.slabs);
 #define CONEF_MTP(RP)                                                                                            \
     do {                                                                                                         \
-        if (fast) hipLaunchKernelGGL((psgd_mtp_kernel<RP, true>), grid, dim3(kMtpThreads), 0, s, x, p, out, n, (int)m, r, \
+        if (fast) conef_launch((psgd_mtp_kernel<RP, true>), grid, dim3(kMtpThreads), 0, s, x, p, out, n, (int)m, r, \
                                      g.rows_per_slab);                                                           \
-        else hipLaunchKernelGGL((psgd_mtp_kernel<RP, false>), grid, dim3(kMtpThreads), 0, s, x, p, out, n, (int)m, r,     \
+        else conef_launch((psgd_mtp_kernel<RP, false>), grid, dim3(kMtpThreads), 0, s, x, p, out, n, (int)m, r,     \
                                 g.rows_per_slab);                                                                \
     } while (0)
     CONEF_RANK_SWITCH(r, CONEF_MTP)
 #undef CONEF_MTP
     if (g.slabs > 1) {
         int64_t count = m * r;
-        hipLaunchKernelGGL(psgd_sum_partials_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, out, q,
+        conef_launch(psgd_sum_partials_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, out, q,
                            count, g.slabs);
     }
     return (int)hipGetLastError();
@@ -2384,11 +2386,11 @@ static int launch_pqt(float* x, float* err, const float* p, const float* q, int6
         }
         dim3 grid((unsigned)col_wgs, (unsigned)slabs);
         if (r == 32) {
-            if (err) hipLaunchKernelGGL((psgd_mfma_pqt_kernel<32, 1>), grid, dim3(kMfmaThreads), 0, s, x, err, p, q, n, (int)m, (int)rps);
-            else hipLaunchKernelGGL((psgd_mfma_pqt_kernel<32, 0>), grid, dim3(kMfmaThreads), 0, s, x, err, p, q, n, (int)m, (int)rps);
+            if (err) conef_launch((psgd_mfma_pqt_kernel<32, 1>), grid, dim3(kMfmaThreads), 0, s, x, err, p, q, n, (int)m, (int)rps);
+            else conef_launch((psgd_mfma_pqt_kernel<32, 0>), grid, dim3(kMfmaThreads), 0, s, x, err, p, q, n, (int)m, (int)rps);
         } else {
-            if (err) hipLaunchKernelGGL((psgd_mfma_pqt_kernel<16, 1>), grid, dim3(kMfmaThreads), 0, s, x, err, p, q, n, (int)m, (int)rps);
-            else hipLaunchKernelGGL((psgd_mfma_pqt_kernel<16, 0>), grid, dim3(kMfmaThreads), 0, s, x, err, p, q, n, (int)m, (int)rps);
+            if (err) conef_launch((psgd_mfma_pqt_kernel<16, 1>), grid, dim3(kMfmaThreads), 0, s, x, err, p, q, n, (int)m, (int)rps);
+            else conef_launch((psgd_mfma_pqt_kernel<16, 0>), grid, dim3(kMfmaThreads), 0, s, x, err, p, q, n, (int)m, (int)rps);
         }
         return (int)hipGetLastError();
     }
@@ -2406,8 +2408,8 @@ static int launch_pqt(float* x, float* err, const float* p, const float* q, int6
 #define CONEF_PQ1(RP)                                                                                       \
     do {                                                                                                    \
         if (RP >= 16) break;                                                                                \
-        if (err) hipLaunchKernelGGL((psgd_pqt_one_kernel<(RP < 16 ? RP : 8), 1>), grid, dim3(256), 0, s, it); \
-        else hipLaunchKernelGGL((psgd_pqt_one_kernel<(RP < 16 ? RP : 8), 0>), grid, dim3(256), 0, s, it);     \
+        if (err) conef_launch((psgd_pqt_one_kernel<(RP < 16 ? RP : 8), 1>), grid, dim3(256), 0, s, it); \
+        else conef_launch((psgd_pqt_one_kernel<(RP < 16 ? RP : 8), 0>), grid, dim3(256), 0, s, it);     \
     } while (0)
         CONEF_RANK_SWITCH(r, CONEF_PQ1)
 #undef CONEF_PQ1
@@ -2423,7 +2425,7 @@ static int launch_pqt(float* x, float* err, const float* p, const float* q, int6
     }
     dim3 grid((unsigned)col_tiles, (unsigned)slabs);
 #define CONEF_PQT_GO(RP, MODE) \
-    hipLaunchKernelGGL((psgd_pqt_kernel<RP, MODE>), grid, dim3(256), 0, s, x, err, p, q, n, (int)m, r, (int)rps)
+    conef_launch((psgd_pqt_kernel<RP, MODE>), grid, dim3(256), 0, s, x, err, p, q, n, (int)m, r, (int)rps)
 #define CONEF_PQT(RP)                                 \
     do {                                              \
         if (err) CONEF_PQT_GO(RP, 1);                 \
@@ -2536,7 +2538,7 @@ int conef_gram_schmidt_f32(float* a, int64_t rows, int32_t r, float eps, void* w
     do {                                                                                                          \
         auto k = gram_schmidt_lds_kernel<RP>;                                                                     \
         if (hipError_t e = conef_allow_lds((const void*)k, lds); e != hipSuccess) return (int)e; \
-        hipLaunchKernelGGL(k, dim3(1), dim3(threads), lds, s, a, (int)rows, r, eps);                              \
+        conef_launch(k, dim3(1), dim3(threads), lds, s, a, (int)rows, r, eps);                              \
     } while (0)
         CONEF_RANK_SWITCH(r, CONEF_GS)
 #undef CONEF_GS
@@ -2556,13 +2558,13 @@ int conef_gram_schmidt_f32(float* a, int64_t rows, int32_t r, float eps, void* w
             // fewer, fuller workgroups do not help: the step is bound by the barrier, not by arithmetic
             int rows_per_wg = (int)((rows + wgs - 1) / wgs);
             GsGridWs* gws = (GsGridWs*)workspace;
-            hipLaunchKernelGGL(gs_grid_reset_kernel, dim3(1), dim3(1), 0, s, gws);
+            conef_launch(gs_grid_reset_kernel, dim3(1), dim3(1), 0, s, gws);
             void* args[] = {(void*)&a, (void*)&rows, (void*)&r, (void*)&eps, (void*)&rows_per_wg, (void*)&gws};
             hipError_t e = hipErrorInvalidValue;
 #define CONEF_GSG(RP)                                                                                                 \
     do {                                                                                                              \
         constexpr int kSlots = RP >= 16 ? 4 : 16;                                                                     \
-        e = hipLaunchCooperativeKernel((const void*)gram_schmidt_grid_kernel<RP, kSlots>, dim3((unsigned)wgs),        \
+        conef_launch_unkept(); e = hipLaunchCooperativeKernel((const void*)gram_schmidt_grid_kernel<RP, kSlots>, dim3((unsigned)wgs),        \
                                        dim3(kGsRegThreads), args, 0, s);                                              \
     } while (0)
             CONEF_RANK_SWITCH(r, CONEF_GSG)
@@ -2582,7 +2584,7 @@ int conef_gram_schmidt_f32(float* a, int64_t rows, int32_t r, float eps, void* w
         const float* in = sums + ((i + 1) & 1) * (int64_t)kGsMaxWorkgroups * rp;
         float* out = sums + (i & 1) * (int64_t)kGsMaxWorkgroups * rp;
 #define CONEF_GSS(RP) \
-    hipLaunchKernelGGL(gram_schmidt_step_kernel<RP>, dim3((unsigned)wgs), dim3(256), 0, s, a, rows, r, eps, i, in, out, rows_per_wg)
+    conef_launch(gram_schmidt_step_kernel<RP>, dim3((unsigned)wgs), dim3(256), 0, s, a, rows, r, eps, i, in, out, rows_per_wg)
         CONEF_RANK_SWITCH(r, CONEF_GSS)
 #undef CONEF_GSS
     }
@@ -2892,7 +2894,7 @@ int mq_batch(const ConefPsgdItem* items, int count, float alpha, int32_t a, int3
             int rc = CONEF_OK;
             if (MODE == 2)
                 rc = run_batches(queries, qblocks, [&](const PsgdBatch<QueryItem>& bt, int grid) {
-                    hipLaunchKernelGGL(psgd_cs_query_batch_kernel, dim3((unsigned)grid), dim3(256), 0, s, bt, alpha, hs);
+                    conef_launch(psgd_cs_query_batch_kernel, dim3((unsigned)grid), dim3(256), 0, s, bt, alpha, hs);
                 });
             if (rc != CONEF_OK) return rc;
             const size_t lds = (size_t)kMfmaWaves * 16 * 64 * 4;
@@ -2900,13 +2902,13 @@ int mq_batch(const ConefPsgdItem* items, int count, float alpha, int32_t a, int3
             for (const MfmaMqItem& t : table) exact = exact && t.m % 4 == 0;
             rc = run_batches(table, blocks, [&](const PsgdBatch<MfmaMqItem>& bt, int grid) {
                 const dim3 g((unsigned)grid), t(kMfmaThreads);
-                if (exact) hipLaunchKernelGGL((psgd_mfma_mq_batch_kernel<(MODE == 1 ? 1 : 0), true>), g, t, lds, s, bt);
-                else hipLaunchKernelGGL((psgd_mfma_mq_batch_kernel<(MODE == 1 ? 1 : 0), false>), g, t, lds, s, bt);
+                if (exact) conef_launch((psgd_mfma_mq_batch_kernel<(MODE == 1 ? 1 : 0), true>), g, t, lds, s, bt);
+                else conef_launch((psgd_mfma_mq_batch_kernel<(MODE == 1 ? 1 : 0), false>), g, t, lds, s, bt);
             });
             if (rc != CONEF_OK) return rc;
             if (!sums.empty()) {
                 rc = run_batches(sums, sum_blocks, [&](const PsgdBatch<SumItem>& bt, int grid) {
-                    hipLaunchKernelGGL(psgd_sum_partials_batch_kernel, dim3((unsigned)grid), dim3(256), 0, s, bt);
+                    conef_launch(psgd_sum_partials_batch_kernel, dim3((unsigned)grid), dim3(256), 0, s, bt);
                 });
                 if (rc != CONEF_OK) return rc;
             }
@@ -2955,7 +2957,7 @@ int mq_batch(const ConefPsgdItem* items, int count, float alpha, int32_t a, int3
         }
 #define CONEF_MQB_GO(RB, RP, F)                                                                                    \
     run_batches(table, blocks, [&](const PsgdBatch<MqItem>& bt, int grid) {                                        \
-        hipLaunchKernelGGL((psgd_mq_batch_kernel<RB, RP, MODE, F>), dim3((unsigned)grid), dim3(256), lds, s, bt, alpha, hs); \
+        conef_launch((psgd_mq_batch_kernel<RB, RP, MODE, F>), dim3((unsigned)grid), dim3(256), lds, s, bt, alpha, hs); \
     })
 #define CONEF_MQB(RP)                                                  \
     do {                                                               \
@@ -3060,16 +3062,16 @@ int mtp_batch(const ConefPsgdItem* items, int count, void* workspace, int64_t wo
             const int rp = rank_bound(items[0].r);
             int rc = run_batches(table, blocks, [&](const PsgdBatch<MfmaMtpItem>& bt, int grid) {
                 const dim3 g3((unsigned)(grid + gram->count)), b3(kMfmaThreads);
-                if (rp == 32) hipLaunchKernelGGL(psgd_mfma_mtp_gram_batch_kernel<32>, g3, b3, 0, s, bt, *gram);
-                else hipLaunchKernelGGL(psgd_mfma_mtp_gram_batch_kernel<16>, g3, b3, 0, s, bt, *gram);
+                if (rp == 32) conef_launch(psgd_mfma_mtp_gram_batch_kernel<32>, g3, b3, 0, s, bt, *gram);
+                else conef_launch(psgd_mfma_mtp_gram_batch_kernel<16>, g3, b3, 0, s, bt, *gram);
             });
             if (rc != CONEF_OK) return rc;
             continue;
         }
         int rc = run_batches(table, blocks, [&](const PsgdBatch<MfmaMtpItem>& bt, int grid) {
-            if (v == 4) hipLaunchKernelGGL(psgd_mfma_mtp_batch_kernel<4>, dim3((unsigned)grid), dim3(kMfmaThreads), 0, s, bt);
-            else if (v == 2) hipLaunchKernelGGL(psgd_mfma_mtp_batch_kernel<2>, dim3((unsigned)grid), dim3(kMfmaThreads), 0, s, bt);
-            else hipLaunchKernelGGL(psgd_mfma_mtp_batch_kernel<1>, dim3((unsigned)grid), dim3(kMfmaThreads), 0, s, bt);
+            if (v == 4) conef_launch(psgd_mfma_mtp_batch_kernel<4>, dim3((unsigned)grid), dim3(kMfmaThreads), 0, s, bt);
+            else if (v == 2) conef_launch(psgd_mfma_mtp_batch_kernel<2>, dim3((unsigned)grid), dim3(kMfmaThreads), 0, s, bt);
+            else conef_launch(psgd_mfma_mtp_batch_kernel<1>, dim3((unsigned)grid), dim3(kMfmaThreads), 0, s, bt);
         });
         if (rc != CONEF_OK) return rc;
     }
@@ -3111,14 +3113,14 @@ int mtp_batch(const ConefPsgdItem* items, int count, void* workspace, int64_t wo
     do {                                                                                                            \
         if (RP >= 16) break;                                                                                        \
         if (gram) rc = run_batches(table, blocks, [&](const PsgdBatch<MtpItem>& bt, int grid) {                     \
-            if (fast) hipLaunchKernelGGL((psgd_mtp_gram_batch_kernel<(RP < 16 ? RP : 8), true>), dim3((unsigned)(grid + gram->count)), dim3(kMtpThreads), 0, s, bt, *gram); \
-            else hipLaunchKernelGGL((psgd_mtp_gram_batch_kernel<(RP < 16 ? RP : 8), false>), dim3((unsigned)(grid + gram->count)), dim3(kMtpThreads), 0, s, bt, *gram); \
+            if (fast) conef_launch((psgd_mtp_gram_batch_kernel<(RP < 16 ? RP : 8), true>), dim3((unsigned)(grid + gram->count)), dim3(kMtpThreads), 0, s, bt, *gram); \
+            else conef_launch((psgd_mtp_gram_batch_kernel<(RP < 16 ? RP : 8), false>), dim3((unsigned)(grid + gram->count)), dim3(kMtpThreads), 0, s, bt, *gram); \
         });                                                                                                         \
         else if (fast) rc = run_batches(table, blocks, [&](const PsgdBatch<MtpItem>& bt, int grid) {                \
-            hipLaunchKernelGGL((psgd_mtp_batch_kernel<(RP < 16 ? RP : 8), true>), dim3((unsigned)grid), dim3(kMtpThreads), 0, s, bt); \
+            conef_launch((psgd_mtp_batch_kernel<(RP < 16 ? RP : 8), true>), dim3((unsigned)grid), dim3(kMtpThreads), 0, s, bt); \
         });                                                                                                         \
         else rc = run_batches(table, blocks, [&](const PsgdBatch<MtpItem>& bt, int grid) {                          \
-            hipLaunchKernelGGL((psgd_mtp_batch_kernel<(RP < 16 ? RP : 8), false>), dim3((unsigned)grid), dim3(kMtpThreads), 0, s, bt); \
+            conef_launch((psgd_mtp_batch_kernel<(RP < 16 ? RP : 8), false>), dim3((unsigned)grid), dim3(kMtpThreads), 0, s, bt); \
         });                                                                                                         \
     } while (0)
         CONEF_RANK_SWITCH(lead.r, CONEF_MTPB)
@@ -3127,7 +3129,7 @@ int mtp_batch(const ConefPsgdItem* items, int count, void* workspace, int64_t wo
     }
     if (!sums.empty()) {
         int rc = run_batches(sums, sum_blocks, [&](const PsgdBatch<SumItem>& bt, int grid) {
-            hipLaunchKernelGGL(psgd_sum_partials_batch_kernel, dim3((unsigned)grid), dim3(256), 0, s, bt);
+            conef_launch(psgd_sum_partials_batch_kernel, dim3((unsigned)grid), dim3(256), 0, s, bt);
         });
         if (rc != CONEF_OK) return rc;
     }
@@ -3296,7 +3298,7 @@ int copy_rows(const std::vector<RowsItem>& table, hipStream_t s)
     std::vector<int> blocks;
     for (const RowsItem& t : table) blocks.push_back((int)((t.rows * t.to + 255) / 256));
     return run_batches(table, blocks, [&](const PsgdBatch<RowsItem>& bt, int grid) {
-        hipLaunchKernelGGL(psgd_rows_batch_kernel, dim3((unsigned)grid), dim3(256), 0, s, bt);
+        conef_launch(psgd_rows_batch_kernel, dim3((unsigned)grid), dim3(256), 0, s, bt);
     });
 }
 
@@ -3327,12 +3329,12 @@ int defer_fix(const PaddedRound& pr, int r, const std::vector<MtpRaw>& raw, cons
     return run_batches(fix, blocks, [&](const PsgdBatch<DeferFixItem>& bt, int grid) {
         const dim3 g((unsigned)grid), t((unsigned)(rp <= 8 ? fix_threads(rp) : 256));
         switch (rp) {
-            case 1: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<1>, g, t, 0, s, bt, alpha); break;
-            case 2: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<2>, g, t, 0, s, bt, alpha); break;
-            case 4: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<4>, g, t, 0, s, bt, alpha); break;
-            case 8: hipLaunchKernelGGL(psgd_defer_fix_batch_kernel<8>, g, t, 0, s, bt, alpha); break;
-            case 16: hipLaunchKernelGGL(psgd_defer_fix_wide_batch_kernel<16>, g, t, 0, s, bt); break;
-            default: hipLaunchKernelGGL(psgd_defer_fix_wide_batch_kernel<32>, g, t, 0, s, bt); break;
+            case 1: conef_launch(psgd_defer_fix_batch_kernel<1>, g, t, 0, s, bt, alpha); break;
+            case 2: conef_launch(psgd_defer_fix_batch_kernel<2>, g, t, 0, s, bt, alpha); break;
+            case 4: conef_launch(psgd_defer_fix_batch_kernel<4>, g, t, 0, s, bt, alpha); break;
+            case 8: conef_launch(psgd_defer_fix_batch_kernel<8>, g, t, 0, s, bt, alpha); break;
+            case 16: conef_launch(psgd_defer_fix_wide_batch_kernel<16>, g, t, 0, s, bt); break;
+            default: conef_launch(psgd_defer_fix_wide_batch_kernel<32>, g, t, 0, s, bt); break;
         }
     });
 }
@@ -3421,8 +3423,8 @@ int round_products_deferred_mfma(const PaddedRound& pr, int r, float* const* q_i
         at += defer_tmat_bytes(rp) + conef_align256(8 * defer_qgram_doubles(it));
     }
     rc = run_batches(shares, share_blocks, [&](const PsgdBatch<GramShareItem>& bt, int grid) {
-        if (rp == 32) hipLaunchKernelGGL(psgd_gram_shares_batch_kernel<32>, dim3((unsigned)grid), dim3(kGsgThreads), 0, s, bt);
-        else hipLaunchKernelGGL(psgd_gram_shares_batch_kernel<16>, dim3((unsigned)grid), dim3(kGsgThreads), 0, s, bt);
+        if (rp == 32) conef_launch(psgd_gram_shares_batch_kernel<32>, dim3((unsigned)grid), dim3(kGsgThreads), 0, s, bt);
+        else conef_launch(psgd_gram_shares_batch_kernel<16>, dim3((unsigned)grid), dim3(kGsgThreads), 0, s, bt);
     });
     if (rc != CONEF_OK) return rc;
     std::vector<MtpRaw> raw((size_t)count);
@@ -3517,15 +3519,15 @@ int orthogonalise_by_gram_wide(const PaddedRound& pr, int r, const std::vector<c
         fix_blocks.push_back((int)((it.m + rows_per_wg - 1) / rows_per_wg));
     }
     int rc = run_batches(shares, share_blocks, [&](const PsgdBatch<GramShareItem>& bt, int grid) {
-        if (rp == 32) hipLaunchKernelGGL(psgd_gram_shares_batch_kernel<32>, dim3((unsigned)grid), dim3(kGsgThreads), 0, s, bt);
-        else hipLaunchKernelGGL(psgd_gram_shares_batch_kernel<16>, dim3((unsigned)grid), dim3(kGsgThreads), 0, s, bt);
+        if (rp == 32) conef_launch(psgd_gram_shares_batch_kernel<32>, dim3((unsigned)grid), dim3(kGsgThreads), 0, s, bt);
+        else conef_launch(psgd_gram_shares_batch_kernel<16>, dim3((unsigned)grid), dim3(kGsgThreads), 0, s, bt);
     });
     if (rc != CONEF_OK) return rc;
-    if (rp == 32) hipLaunchKernelGGL(psgd_gram_solve_batch_kernel<32>, dim3((unsigned)count), dim3(kMfmaThreads), 0, s, gram);
-    else hipLaunchKernelGGL(psgd_gram_solve_batch_kernel<16>, dim3((unsigned)count), dim3(kMfmaThreads), 0, s, gram);
+    if (rp == 32) conef_launch(psgd_gram_solve_batch_kernel<32>, dim3((unsigned)count), dim3(kMfmaThreads), 0, s, gram);
+    else conef_launch(psgd_gram_solve_batch_kernel<16>, dim3((unsigned)count), dim3(kMfmaThreads), 0, s, gram);
     return run_batches(fix, fix_blocks, [&](const PsgdBatch<DeferFixItem>& bt, int grid) {
-        if (rp == 32) hipLaunchKernelGGL(psgd_defer_fix_wide_batch_kernel<32>, dim3((unsigned)grid), dim3(256), 0, s, bt);
-        else hipLaunchKernelGGL(psgd_defer_fix_wide_batch_kernel<16>, dim3((unsigned)grid), dim3(256), 0, s, bt);
+        if (rp == 32) conef_launch(psgd_defer_fix_wide_batch_kernel<32>, dim3((unsigned)grid), dim3(256), 0, s, bt);
+        else conef_launch(psgd_defer_fix_wide_batch_kernel<16>, dim3((unsigned)grid), dim3(256), 0, s, bt);
     });
 }
 
@@ -3757,11 +3759,11 @@ int pqt_sketch_group(const ConefPsgdItem* items, const std::vector<int>& members
         if (hipError_t e = conef_allow_lds((const void*)fused, lds); e != hipSuccess) return (int)e;
         const GsAhead g = *ahead;
         return run_batches(table, blocks, [&](const PsgdBatch<RowlistResidualItem<RP, FAST>>& bt, int grid) {
-            hipLaunchKernelGGL(fused, dim3((unsigned)(grid + g.count)), dim3(kConefRowlistThreads), lds, s, bt, omb, g);
+            conef_launch(fused, dim3((unsigned)(grid + g.count)), dim3(kConefRowlistThreads), lds, s, bt, omb, g);
         });
     }
     return run_batches(table, blocks, [&](const PsgdBatch<RowlistResidualItem<RP, FAST>>& bt, int grid) {
-        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kConefRowlistThreads), lds, s, bt, omb);
+        conef_launch(kern, dim3((unsigned)grid), dim3(kConefRowlistThreads), lds, s, bt, omb);
     });
 }
 
@@ -3794,11 +3796,11 @@ int pqt_batch(const ConefPsgdItem* items, int count, int mode, float beta, int32
             }
             int rc = run_batches(table, blocks, [&](const PsgdBatch<MfmaPqtItem>& bt, int grid) {
                 if (lead.r == 32) {
-                    if (mode == 1) hipLaunchKernelGGL((psgd_mfma_pqt_batch_kernel<32, 1>), dim3((unsigned)grid), dim3(kMfmaThreads), 0, s, bt);
-                    else hipLaunchKernelGGL((psgd_mfma_pqt_batch_kernel<32, 0>), dim3((unsigned)grid), dim3(kMfmaThreads), 0, s, bt);
+                    if (mode == 1) conef_launch((psgd_mfma_pqt_batch_kernel<32, 1>), dim3((unsigned)grid), dim3(kMfmaThreads), 0, s, bt);
+                    else conef_launch((psgd_mfma_pqt_batch_kernel<32, 0>), dim3((unsigned)grid), dim3(kMfmaThreads), 0, s, bt);
                 } else {
-                    if (mode == 1) hipLaunchKernelGGL((psgd_mfma_pqt_batch_kernel<16, 1>), dim3((unsigned)grid), dim3(kMfmaThreads), 0, s, bt);
-                    else hipLaunchKernelGGL((psgd_mfma_pqt_batch_kernel<16, 0>), dim3((unsigned)grid), dim3(kMfmaThreads), 0, s, bt);
+                    if (mode == 1) conef_launch((psgd_mfma_pqt_batch_kernel<16, 1>), dim3((unsigned)grid), dim3(kMfmaThreads), 0, s, bt);
+                    else conef_launch((psgd_mfma_pqt_batch_kernel<16, 0>), dim3((unsigned)grid), dim3(kMfmaThreads), 0, s, bt);
                 }
             });
             if (rc != CONEF_OK) return rc;
@@ -3882,10 +3884,10 @@ int pqt_batch(const ConefPsgdItem* items, int count, int mode, float beta, int32
 #define CONEF_PQB_GO(RP, MODE, F)                                                                                  \
     run_batches(table, blocks, [&](const PsgdBatch<PqtItem>& bt, int grid) {                                       \
         if (ride)                                                                                                  \
-            hipLaunchKernelGGL((psgd_pqt_gs_batch_kernel<RP, MODE, F>), dim3((unsigned)(grid + g.count)), dim3(256), 0, s, \
+            conef_launch((psgd_pqt_gs_batch_kernel<RP, MODE, F>), dim3((unsigned)(grid + g.count)), dim3(256), 0, s, \
                                bt, g);                                                                             \
         else                                                                                                       \
-            hipLaunchKernelGGL((psgd_pqt_batch_kernel<RP, MODE, F>), dim3((unsigned)grid), dim3(256), 0, s, bt);   \
+            conef_launch((psgd_pqt_batch_kernel<RP, MODE, F>), dim3((unsigned)grid), dim3(256), 0, s, bt);   \
     })
 #define CONEF_PQB(RP)                                                          \
     do {                                                                       \
@@ -4037,7 +4039,7 @@ int round_linear(PaddedRound& pr, LinearRound& lr, int r, float* const* q_in, co
             blocks.push_back((items[k].w + 255) / 256);
         }
         rc = run_batches(folds, blocks, [&](const PsgdBatch<FoldItem>& bt, int grid) {
-            hipLaunchKernelGGL(psgd_fold_batch_kernel<RP>, dim3((unsigned)grid), dim3(256), 0, s, bt);
+            conef_launch(psgd_fold_batch_kernel<RP>, dim3((unsigned)grid), dim3(256), 0, s, bt);
         });
         if (rc != CONEF_OK) return rc;
     }
@@ -4070,7 +4072,7 @@ int round_linear(PaddedRound& pr, LinearRound& lr, int r, float* const* q_in, co
     auto kern = sh.T == 256 ? psgd_lin_mq_batch_kernel<RP, 256> : psgd_lin_mq_batch_kernel<RP, 512>;
     if (hipError_t e = conef_allow_lds((const void*)kern, sh.lds); e != hipSuccess) return (int)e;
     rc = run_batches(lr.mq, blocks, [&](const PsgdBatch<LinMqItem>& bt, int grid) {
-        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3((unsigned)sh.T), sh.lds, s, bt, alpha);
+        conef_launch(kern, dim3((unsigned)grid), dim3((unsigned)sh.T), sh.lds, s, bt, alpha);
     });
     if (rc != CONEF_OK) return rc;
 
@@ -4092,7 +4094,7 @@ int round_linear(PaddedRound& pr, LinearRound& lr, int r, float* const* q_in, co
         cells.push_back(CellRaw{lr.cs_part[(size_t)k], lr.view[(size_t)k].pk, it.w});
     }
     rc = run_batches(mtp, blocks, [&](const PsgdBatch<MtpItem>& bt, int grid) {
-        hipLaunchKernelGGL((psgd_mtp_gram_batch_kernel<RP, true>), dim3((unsigned)(grid + count)), dim3(kMtpThreads), 0, s, bt, gram);
+        conef_launch((psgd_mtp_gram_batch_kernel<RP, true>), dim3((unsigned)(grid + count)), dim3(kMtpThreads), 0, s, bt, gram);
     });
     if (rc != CONEF_OK) return rc;
     rc = defer_fix(pr, r, raw, tmats, next.count ? &qgrams : nullptr, s, &cells, alpha);
@@ -4127,7 +4129,7 @@ int round_linear(PaddedRound& pr, LinearRound& lr, int r, float* const* q_in, co
     if (hipError_t e = conef_allow_lds((const void*)residual, lds); e != hipSuccess) return (int)e;
     const double omb = 1. - (double)beta;
     return run_batches(last, blocks, [&](const PsgdBatch<RowlistResidualItem<RP, true, true>>& bt, int grid) {
-        hipLaunchKernelGGL(residual, dim3((unsigned)(grid + next.count * (next.split + next.fold_split))), dim3(kConefRowlistThreads), lds, s, bt, omb, next);
+        conef_launch(residual, dim3((unsigned)(grid + next.count * (next.split + next.fold_split))), dim3(kConefRowlistThreads), lds, s, bt, omb, next);
     });
 }
 
@@ -4250,7 +4252,7 @@ int conef_psgd_sketch_update_batch_f32(const ConefPsgdItem* items, int32_t count
     const double omb = 1. - (double)beta;
     hipStream_t s = (hipStream_t)stream;
     return run_batches(table, blocks, [&](const PsgdBatch<RowlistVecItem>& bt, int grid) {
-        hipLaunchKernelGGL(psgd_rowlist_vec_batch_kernel, dim3((unsigned)grid), dim3(kConefRowlistThreads), lds, s, bt, omb);
+        conef_launch(psgd_rowlist_vec_batch_kernel, dim3((unsigned)grid), dim3(kConefRowlistThreads), lds, s, bt, omb);
     });
 }
 
@@ -4511,8 +4513,7 @@ int conef_psgd_round_small_f32(const ConefPsgdItem* items, int32_t count, int32_
     if (ws_need > 0 && (!workspace || workspace_bytes < ws_need || ((uintptr_t)workspace & 7))) return CONEF_ERR_INVALID;
     hipStream_t s = (hipStream_t)stream;
     const double omb = 1. - (double)beta;
-    unsigned tag = (g_small_launches.fetch_add(1u) + 1u) * 0x9E3779B9u;      // never the tag of the records' last use
-    if (tag == 0u) tag = 1u;
+    const unsigned tag = 0u;      // drawn by conef_launch_tagged: never the tag of the records' last use
     {
         const int k0 = 0, nb = count;
         SmallBatch batch;
@@ -4589,7 +4590,7 @@ int conef_psgd_round_small_f32(const ConefPsgdItem* items, int32_t count, int32_
     do {                                                                                                        \
         auto kern = psgd_small_round_kernel<RP>;                                                                \
         if (hipError_t e = conef_allow_lds((const void*)kern, lds); e != hipSuccess) return (int)e;             \
-        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kSmallThreads), lds, s, batch, tag, mq_mode, pqt_mode, alpha, omb, eps); \
+        conef_launch_tagged<1>(g_small_launches, kern, dim3((unsigned)grid), dim3(kSmallThreads), lds, s, batch, tag, mq_mode, pqt_mode, alpha, omb, eps); \
     } while (0)
         switch (rp) {
             case 1: CONEF_SMALL(1); break;
@@ -4697,7 +4698,7 @@ extern "C" int conef_ef_passthrough_batch_f32(float* const* x, float* const* err
     b.first[0] = 0;
     auto flush = [&]() {
         if (b.spans > 0)
-            hipLaunchKernelGGL(ef_passthrough_kernel, dim3((unsigned)b.first[b.spans]), dim3(256), 0, (hipStream_t)stream, b);
+            conef_launch(ef_passthrough_kernel, dim3((unsigned)b.first[b.spans]), dim3(256), 0, (hipStream_t)stream, b);
         b.spans = 0;
     };
     for (int k = 0; k < spans; ++k)
@@ -4717,4 +4718,52 @@ extern "C" int conef_ef_passthrough_batch_f32(float* const* x, float* const* err
 extern "C" int conef_ef_passthrough_f32(float* x, float* err, int64_t count, void* stream)
 {
     return conef_ef_passthrough_batch_f32(&x, &err, &count, 1, stream);
+}
+
+// ------------------------------------------------------------------- tapes ----
+extern "C" int64_t conef_tape_create(void)
+{
+    return (int64_t)(intptr_t) new (std::nothrow) ConefTape;
+}
+
+extern "C" int conef_tape_destroy(int64_t tape)
+{
+    delete (ConefTape*)(intptr_t)tape;
+    return CONEF_OK;
+}
+
+extern "C" int conef_tape_record(int64_t tape)
+{
+    ConefTape* t = (ConefTape*)(intptr_t)tape;
+    if (!t || conef_recording) return CONEF_ERR_INVALID;
+    t->launches.clear();
+    t->whole = true;
+    t->items.clear();
+    conef_recording = t;
+    return CONEF_OK;
+}
+
+extern "C" int conef_tape_stop(int64_t tape, const ConefPsgdItem* items, int32_t count, int32_t keep)
+{
+    ConefTape* t = (ConefTape*)(intptr_t)tape;
+    if (!t || conef_recording != t || count < 0 || (count > 0 && !items)) return CONEF_ERR_INVALID;
+    conef_recording = nullptr;
+    t->whole = t->whole && keep && !t->launches.empty();
+    if (!t->whole) {
+        t->launches.clear();
+        return CONEF_OK;
+    }
+    t->items.assign((const char*)items, (const char*)(items + count));
+    return CONEF_OK;
+}
+
+extern "C" int conef_tape_replay(int64_t tape, const ConefPsgdItem* items, int32_t count, void* stream)
+{
+    ConefTape* t = (ConefTape*)(intptr_t)tape;
+    if (!t || conef_recording || count < 0 || (count > 0 && !items)) return CONEF_ERR_INVALID;
+    if (!t->whole || t->launches.empty() || t->items.size() != sizeof(*items) * (size_t)count ||
+        memcmp(t->items.data(), items, t->items.size()) != 0)
+        return CONEF_TAPE_STALE;
+    for (const std::unique_ptr<ConefTape::Launch>& l : t->launches) l->go((hipStream_t)stream);
+    return (int)hipGetLastError();
 }

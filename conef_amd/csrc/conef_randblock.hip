@@ -102,7 +102,7 @@ int conef_randblock_ef_step_f32(float* x, float* err, float* payload, int64_t nu
 {
     if (!block_args_ok(numel, start, block) || !x || !err || !payload) return CONEF_ERR_INVALID;
     ConefBlock blk = conef_make_block(numel, start, block);
-    hipLaunchKernelGGL(randblock_ef_kernel, dim3((unsigned)conef_rb_groups(numel, kRbEfQuads)), dim3(256), 0, (hipStream_t)stream, x, err,
+    conef_launch(randblock_ef_kernel, dim3((unsigned)conef_rb_groups(numel, kRbEfQuads)), dim3(256), 0, (hipStream_t)stream, x, err,
                        payload, numel, blk);
     return (int)hipGetLastError();
 }
@@ -112,7 +112,7 @@ int conef_randblock_unbiased_step_f32(float* x, float* payload, int64_t numel, i
 {
     if (!block_args_ok(numel, start, block) || !x || !payload || !(prob > 0.f)) return CONEF_ERR_INVALID;
     ConefBlock blk = conef_make_block(numel, start, block);
-    hipLaunchKernelGGL(randblock_unbiased_kernel, dim3((unsigned)conef_rb_groups(numel, kRbUnbiasedQuads)), dim3(256), 0, (hipStream_t)stream, x,
+    conef_launch(randblock_unbiased_kernel, dim3((unsigned)conef_rb_groups(numel, kRbUnbiasedQuads)), dim3(256), 0, (hipStream_t)stream, x,
                        payload, numel, blk, prob);
     return (int)hipGetLastError();
 }
@@ -121,7 +121,7 @@ int conef_randblock_gather_f32(const float* x, float* payload, int64_t numel, in
                                float scale, void* stream)
 {
     if (!block_args_ok(numel, start, block) || !x || !payload || !(scale > 0.f)) return CONEF_ERR_INVALID;
-    hipLaunchKernelGGL(randblock_gather_kernel, dim3(grid_for(block, 256)), dim3(256), 0, (hipStream_t)stream, x,
+    conef_launch(randblock_gather_kernel, dim3(grid_for(block, 256)), dim3(256), 0, (hipStream_t)stream, x,
                        payload, numel, start, block, scale);
     return (int)hipGetLastError();
 }
@@ -133,10 +133,10 @@ int conef_randblock_scatter_f32(float* x, const float* payload, int64_t numel, i
     ConefBlock blk = conef_make_block(numel, start, block);
     int g = grid_for((numel + 3) / 4, 256);
     if (aligned16(x))
-        hipLaunchKernelGGL(randblock_scatter_kernel<true>, dim3(g), dim3(256), 0, (hipStream_t)stream, x, payload,
+        conef_launch(randblock_scatter_kernel<true>, dim3(g), dim3(256), 0, (hipStream_t)stream, x, payload,
                            numel, blk);
     else
-        hipLaunchKernelGGL(randblock_scatter_kernel<false>, dim3(g), dim3(256), 0, (hipStream_t)stream, x, payload,
+        conef_launch(randblock_scatter_kernel<false>, dim3(g), dim3(256), 0, (hipStream_t)stream, x, payload,
                            numel, blk);
     return (int)hipGetLastError();
 }

@@ -163,10 +163,10 @@ int conef_randblock_step_batch_f32(const ConefRandBlockItem* items, int32_t coun
         }
         if (mode == 0)
             return rb_run(table, blocks, [&](const auto& bt, int grid) {
-                hipLaunchKernelGGL((randblock_unbiased_batch_kernel<sizeof(bt.item) / sizeof(bt.item[0])>), dim3((unsigned)grid), dim3(256), 0, s, bt);
+                conef_launch((randblock_unbiased_batch_kernel<sizeof(bt.item) / sizeof(bt.item[0])>), dim3((unsigned)grid), dim3(256), 0, s, bt);
             });
         return rb_run(table, blocks, [&](const auto& bt, int grid) {
-            hipLaunchKernelGGL((randblock_ef_batch_kernel<sizeof(bt.item) / sizeof(bt.item[0])>), dim3((unsigned)grid), dim3(256), 0, s, bt);
+            conef_launch((randblock_ef_batch_kernel<sizeof(bt.item) / sizeof(bt.item[0])>), dim3((unsigned)grid), dim3(256), 0, s, bt);
         });
     }
     // sketched error: row-list plans share launches, the rest go one by one
@@ -192,7 +192,7 @@ int conef_randblock_step_batch_f32(const ConefRandBlockItem* items, int32_t coun
         if (e != hipSuccess) return (int)e;
         const double omb = 1. - (double)beta;
         int rc = rb_run(table, blocks, [&](const auto& bt, int grid) {
-            hipLaunchKernelGGL((randblock_rowlist_batch_kernel<sizeof(bt.item) / sizeof(bt.item[0])>), dim3((unsigned)grid), dim3(kConefRowlistThreads), lds, s,
+            conef_launch((randblock_rowlist_batch_kernel<sizeof(bt.item) / sizeof(bt.item[0])>), dim3((unsigned)grid), dim3(kConefRowlistThreads), lds, s,
                                bt, omb);
         });
         if (rc != CONEF_OK) return rc;

@@ -345,7 +345,7 @@ int launch_query(float* x, const CsT* cs, int64_t n, int64_t d, int32_t w, float
     const int vw = (d % 4 == 0 && aligned16(x)) ? 4 : (d % 2 == 0 && (reinterpret_cast<uintptr_t>(x) & 7u) == 0) ? 2 : 1;
     ConefMod mod = conef_make_mod(w);
     if (vw == 1) {
-        hipLaunchKernelGGL((cs_query_kernel<CsT, 1, 1>), grid, dim3(256), 0, stream, x, cs, n, d, mod, alpha, hs, rpb, pktab);
+        conef_launch((cs_query_kernel<CsT, 1, 1>), grid, dim3(256), 0, stream, x, cs, n, d, mod, alpha, hs, rpb, pktab);
         return (int)hipGetLastError();
     }
     // Rows in flight per thread: the whole row group when it is small; four at a time when the
@@ -356,10 +356,10 @@ int launch_query(float* x, const CsT* cs, int64_t n, int64_t d, int32_t w, float
 #define CONEF_QUERY_CASE(RB)                                                                                          \
     case RB:                                                                                                          \
         if (vw == 4)                                                                                                  \
-            hipLaunchKernelGGL((cs_query_kernel<CsT, 4, RB>), grid, dim3(256), 0, stream, x, cs, n, d, mod, alpha, hs, \
+            conef_launch((cs_query_kernel<CsT, 4, RB>), grid, dim3(256), 0, stream, x, cs, n, d, mod, alpha, hs, \
                                rpb, pktab);                                                                           \
         else                                                                                                          \
-            hipLaunchKernelGGL((cs_query_kernel<CsT, 2, RB>), grid, dim3(256), 0, stream, x, cs, n, d, mod, alpha, hs, \
+            conef_launch((cs_query_kernel<CsT, 2, RB>), grid, dim3(256), 0, stream, x, cs, n, d, mod, alpha, hs, \
                                rpb, pktab);                                                                           \
         break
         CONEF_QUERY_CASE(1);
@@ -450,11 +450,11 @@ int conef_launch_query_rows8_f32(float* x, const float* cs, int64_t n, int64_t d
                                  const uint32_t* pktab, float* scratch, hipStream_t stream)
 {
     if (n < 1 || n > 8 || d < 4 || d % 4 != 0 || !aligned16(x) || !aligned16(pktab) || !aligned16(scratch)) return CONEF_ERR_INVALID;
-    hipLaunchKernelGGL(cs_interleave8_kernel, dim3((unsigned)((w + 255) / 256)), dim3(256), 0, stream, cs, scratch, (int)n, (int)w);
+    conef_launch(cs_interleave8_kernel, dim3((unsigned)((w + 255) / 256)), dim3(256), 0, stream, cs, scratch, (int)n, (int)w);
     const dim3 grid((unsigned)((d / 4 + 255) / 256));
     switch ((int)n) {
 #define CONEF_ROWS8(NR) \
-    case NR: hipLaunchKernelGGL(cs_query_rows8_kernel<NR>, grid, dim3(256), 0, stream, x, scratch, d, alpha, pktab); break
+    case NR: conef_launch(cs_query_rows8_kernel<NR>, grid, dim3(256), 0, stream, x, scratch, d, alpha, pktab); break
         CONEF_ROWS8(1); CONEF_ROWS8(2); CONEF_ROWS8(3); CONEF_ROWS8(4);
         CONEF_ROWS8(5); CONEF_ROWS8(6); CONEF_ROWS8(7); CONEF_ROWS8(8);
 #undef CONEF_ROWS8
@@ -488,7 +488,7 @@ int conef_hash_table_i32(int32_t* bucket, int32_t* sign, int64_t d, int32_t w, i
     if (d == 0) return CONEF_OK;
     if (!bucket || !sign) return CONEF_ERR_INVALID;
     ConefSeeds hs = {a, b, sa, sb};
-    hipLaunchKernelGGL(hash_table_kernel, dim3((unsigned)((d + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+    conef_launch(hash_table_kernel, dim3((unsigned)((d + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
                        bucket, sign, d, conef_make_mod(w), hs);
     return (int)hipGetLastError();
 }
@@ -554,17 +554,17 @@ int conef_cs3_query_f32(float* x, const float* cs0, const float* cs1, const floa
         const int rows = rows_per_block_for(n, cb);
         dim3 g4((unsigned)cb, (unsigned)((n + rows - 1) / rows));
         if (rows == 1)
-            hipLaunchKernelGGL(cs3_query_vec_kernel<1>, g4, dim3(256), 0, (hipStream_t)stream, x, cs0, cs1, cs2, n, d,
+            conef_launch(cs3_query_vec_kernel<1>, g4, dim3(256), 0, (hipStream_t)stream, x, cs0, cs1, cs2, n, d,
                                conef_make_mod(w), alpha, rows);
         else
-            hipLaunchKernelGGL(cs3_query_vec_kernel<4>, g4, dim3(256), 0, (hipStream_t)stream, x, cs0, cs1, cs2, n, d,
+            conef_launch(cs3_query_vec_kernel<4>, g4, dim3(256), 0, (hipStream_t)stream, x, cs0, cs1, cs2, n, d,
                                conef_make_mod(w), alpha, rows);
         return (int)hipGetLastError();
     }
     int64_t col_blocks = (d + 255) / 256;
     int rpb = rows_per_block_for(n, col_blocks);
     dim3 grid((unsigned)col_blocks, (unsigned)((n + rpb - 1) / rpb));
-    hipLaunchKernelGGL(cs3_query_kernel, grid, dim3(256), 0, (hipStream_t)stream, x, cs0, cs1, cs2, n, d,
+    conef_launch(cs3_query_kernel, grid, dim3(256), 0, (hipStream_t)stream, x, cs0, cs1, cs2, n, d,
                        conef_make_mod(w), alpha, rpb);
     return (int)hipGetLastError();
 }
@@ -579,14 +579,14 @@ int conef_cs3_update_f32(const float* vec, const float* in0, const float* in1, c
     hipStream_t s = (hipStream_t)stream;
     int64_t cells = n * (int64_t)w;
     int g = grid_for(cells, 256);
-    hipLaunchKernelGGL(conef_copy_f32_kernel, dim3(g), dim3(256), 0, s, out0, in0, cells);
-    hipLaunchKernelGGL(conef_copy_f32_kernel, dim3(g), dim3(256), 0, s, out1, in1, cells);
-    hipLaunchKernelGGL(conef_copy_f32_kernel, dim3(g), dim3(256), 0, s, out2, in2, cells);
+    conef_launch(conef_copy_f32_kernel, dim3(g), dim3(256), 0, s, out0, in0, cells);
+    conef_launch(conef_copy_f32_kernel, dim3(g), dim3(256), 0, s, out1, in1, cells);
+    conef_launch(conef_copy_f32_kernel, dim3(g), dim3(256), 0, s, out2, in2, cells);
     if (d == 0) return (int)hipGetLastError();
     int64_t col_blocks = (d + 255) / 256;
     int rpb = rows_per_block_for(n, col_blocks);
     dim3 grid((unsigned)col_blocks, (unsigned)((n + rpb - 1) / rpb));
-    hipLaunchKernelGGL(cs3_update_kernel, grid, dim3(256), 0, s, vec, in0, in1, in2, out0, out1, out2, n, d,
+    conef_launch(cs3_update_kernel, grid, dim3(256), 0, s, vec, in0, in1, in2, out0, out1, out2, n, d,
                        conef_make_mod(w), beta, rpb);
     return (int)hipGetLastError();
 }
@@ -602,17 +602,17 @@ int conef_cs3_value_f32(const float* vec, const float* in0, const float* in1, co
         const int rows = rows_per_block_for(n, cb);
         dim3 g4((unsigned)cb, (unsigned)((n + rows - 1) / rows));
         if (rows == 1)
-            hipLaunchKernelGGL(cs3_value_vec_kernel<1>, g4, dim3(256), 0, (hipStream_t)stream, vec, in0, in1, in2, out_t,
+            conef_launch(cs3_value_vec_kernel<1>, g4, dim3(256), 0, (hipStream_t)stream, vec, in0, in1, in2, out_t,
                                n, d, conef_make_mod(w), beta, rows);
         else
-            hipLaunchKernelGGL(cs3_value_vec_kernel<4>, g4, dim3(256), 0, (hipStream_t)stream, vec, in0, in1, in2, out_t,
+            conef_launch(cs3_value_vec_kernel<4>, g4, dim3(256), 0, (hipStream_t)stream, vec, in0, in1, in2, out_t,
                                n, d, conef_make_mod(w), beta, rows);
         return (int)hipGetLastError();
     }
     int64_t col_blocks = (d + 255) / 256;
     int rpb = rows_per_block_for(n, col_blocks);
     dim3 grid((unsigned)col_blocks, (unsigned)((n + rpb - 1) / rpb));
-    hipLaunchKernelGGL(cs3_value_kernel, grid, dim3(256), 0, (hipStream_t)stream, vec, in0, in1, in2, out_t, n, d,
+    conef_launch(cs3_value_kernel, grid, dim3(256), 0, (hipStream_t)stream, vec, in0, in1, in2, out_t, n, d,
                        conef_make_mod(w), beta, rpb);
     return (int)hipGetLastError();
 }
@@ -621,7 +621,7 @@ int conef_scale_f32(float* x, int64_t count, float alpha, void* stream)
 {
     if (count < 0 || (count > 0 && !x)) return CONEF_ERR_INVALID;
     if (count == 0) return CONEF_OK;
-    hipLaunchKernelGGL(scale_kernel<float>, dim3(grid_for(count, 256)), dim3(256), 0, (hipStream_t)stream, x, count,
+    conef_launch(scale_kernel<float>, dim3(grid_for(count, 256)), dim3(256), 0, (hipStream_t)stream, x, count,
                        alpha);
     return (int)hipGetLastError();
 }
@@ -630,7 +630,7 @@ int conef_scale_f16(void* x_half, int64_t count, float alpha, void* stream)
 {
     if (count < 0 || (count > 0 && !x_half)) return CONEF_ERR_INVALID;
     if (count == 0) return CONEF_OK;
-    hipLaunchKernelGGL(scale_kernel<__half>, dim3(grid_for(count, 256)), dim3(256), 0, (hipStream_t)stream,
+    conef_launch(scale_kernel<__half>, dim3(grid_for(count, 256)), dim3(256), 0, (hipStream_t)stream,
                        (__half*)x_half, count, alpha);
     return (int)hipGetLastError();
 }
@@ -639,7 +639,7 @@ int conef_convert_f16_to_f32(float* dst, const void* src_half, int64_t count, vo
 {
     if (count < 0 || (count > 0 && (!dst || !src_half))) return CONEF_ERR_INVALID;
     if (count == 0) return CONEF_OK;
-    hipLaunchKernelGGL((convert_kernel<float, __half>), dim3(grid_for(count, 256)), dim3(256), 0,
+    conef_launch((convert_kernel<float, __half>), dim3(grid_for(count, 256)), dim3(256), 0,
                        (hipStream_t)stream, dst, (const __half*)src_half, count);
     return (int)hipGetLastError();
 }
@@ -648,7 +648,7 @@ int conef_convert_f32_to_f16(void* dst_half, const float* src, int64_t count, vo
 {
     if (count < 0 || (count > 0 && (!dst_half || !src))) return CONEF_ERR_INVALID;
     if (count == 0) return CONEF_OK;
-    hipLaunchKernelGGL((convert_kernel<__half, float>), dim3(grid_for(count, 256)), dim3(256), 0,
+    conef_launch((convert_kernel<__half, float>), dim3(grid_for(count, 256)), dim3(256), 0,
                        (hipStream_t)stream, (__half*)dst_half, src, count);
     return (int)hipGetLastError();
 }

@@ -228,7 +228,7 @@ int conef_launch_sketch_step(Front front, const CsT* cs_in, CsT* cs_out, int64_t
         int64_t blocks = (n + kConefRowWaves - 1) / kConefRowWaves;
         if (blocks > 4096) blocks = 4096;
         size_t lds = conef_row_shape_lds(d, w);
-        hipLaunchKernelGGL((conef_sketch_row_kernel<CsT, Front>), dim3((unsigned)blocks), dim3(kConefRowThreads), lds,
+        conef_launch((conef_sketch_row_kernel<CsT, Front>), dim3((unsigned)blocks), dim3(kConefRowThreads), lds,
                            stream, front, cs_in, cs_out, n, d, mod, omb, hs);
         return (int)hipGetLastError();
     }
@@ -239,7 +239,7 @@ int conef_launch_sketch_step(Front front, const CsT* cs_in, CsT* cs_out, int64_t
     int64_t cells = n * (int64_t)w;
     int64_t cg = (cells + 1023) / 1024;
     if (cg > 2048) cg = 2048;
-    hipLaunchKernelGGL(conef_copy_f32_kernel, dim3((unsigned)cg), dim3(256), 0, stream, out, in, cells);
+    conef_launch(conef_copy_f32_kernel, dim3((unsigned)cg), dim3(256), 0, stream, out, in, cells);
     if (d == 0) return (int)hipGetLastError();
     int64_t col_blocks = (d + 1023) / 1024;
     int64_t rpb = (n * col_blocks + 4095) / 4096;
@@ -248,10 +248,10 @@ int conef_launch_sketch_step(Front front, const CsT* cs_in, CsT* cs_out, int64_t
     while ((n + rpb - 1) / rpb > 65535) rpb *= 2;
     dim3 grid((unsigned)col_blocks, (unsigned)((n + rpb - 1) / rpb));
     if (vec_ok && d % 4 == 0)
-        hipLaunchKernelGGL((conef_sketch_tile_kernel<Front, true>), grid, dim3(256), 0, stream, front, in, out, n, d,
+        conef_launch((conef_sketch_tile_kernel<Front, true>), grid, dim3(256), 0, stream, front, in, out, n, d,
                            mod, omb, hs, (int)rpb);
     else
-        hipLaunchKernelGGL((conef_sketch_tile_kernel<Front, false>), grid, dim3(256), 0, stream, front, in, out, n,
+        conef_launch((conef_sketch_tile_kernel<Front, false>), grid, dim3(256), 0, stream, front, in, out, n,
                            d, mod, omb, hs, (int)rpb);
     return (int)hipGetLastError();
 }

@@ -728,10 +728,10 @@ int conef_topk_sparsify_f32(float* x, int64_t numel, int64_t k, void* workspace,
     hipStream_t s = (hipStream_t)stream;
     TopkState* st = (TopkState*)workspace;
     const int64_t g = topk_hist_groups(numel);
-    hipLaunchKernelGGL(topk_init_kernel, dim3(1), dim3(256), 0, s, st, (uint32_t)k);
+    conef_launch(topk_init_kernel, dim3(1), dim3(256), 0, s, st, (uint32_t)k);
     for (int pass = 0; pass < kPasses; ++pass)
-        hipLaunchKernelGGL(topk_hist_kernel, dim3((unsigned)g), dim3(256), 0, s, x, numel, st, pass);
-    hipLaunchKernelGGL(topk_filter_kernel, dim3((unsigned)g), dim3(256), 0, s, x, numel, st);
+        conef_launch(topk_hist_kernel, dim3((unsigned)g), dim3(256), 0, s, x, numel, st, pass);
+    conef_launch(topk_filter_kernel, dim3((unsigned)g), dim3(256), 0, s, x, numel, st);
     return (int)hipGetLastError();
 }
 
@@ -795,17 +795,17 @@ void topk_launch(const TopkItem* items, int nb, TopkRun run, hipStream_t s)
     b.count = nb;
     const dim3 grid((unsigned)wgs), threads(256);
     if (run == TopkRun::kListed) {
-        hipLaunchKernelGGL(topk_hist_batch_kernel<CAP>, grid, threads, 0, s, b, 0, true);
-        hipLaunchKernelGGL(topk_note_batch_kernel<CAP>, grid, threads, 0, s, b);
-        hipLaunchKernelGGL(topk_gather_batch_kernel<CAP>, grid, threads, 0, s, b);
-        hipLaunchKernelGGL(topk_settle_batch_kernel<CAP>, grid, threads, 0, s, b);
+        conef_launch(topk_hist_batch_kernel<CAP>, grid, threads, 0, s, b, 0, true);
+        conef_launch(topk_note_batch_kernel<CAP>, grid, threads, 0, s, b);
+        conef_launch(topk_gather_batch_kernel<CAP>, grid, threads, 0, s, b);
+        conef_launch(topk_settle_batch_kernel<CAP>, grid, threads, 0, s, b);
         return;
     }
     const bool kept = run == TopkRun::kKept;
-    if (!kept) hipLaunchKernelGGL(topk_init_batch_kernel<CAP>, dim3((unsigned)nb), threads, 0, s, b);
+    if (!kept) conef_launch(topk_init_batch_kernel<CAP>, dim3((unsigned)nb), threads, 0, s, b);
     for (int pass = 0; pass < kPasses; ++pass)
-        hipLaunchKernelGGL(topk_hist_batch_kernel<CAP>, grid, threads, 0, s, b, pass, kept);
-    hipLaunchKernelGGL(topk_filter_batch_kernel<CAP>, grid, threads, 0, s, b, kept);
+        conef_launch(topk_hist_batch_kernel<CAP>, grid, threads, 0, s, b, pass, kept);
+    conef_launch(topk_filter_batch_kernel<CAP>, grid, threads, 0, s, b, kept);
 }
 
 int topk_sparsify_batch(float* const* xs, const int64_t* numels, const int64_t* ks, int32_t count, void* workspace,
@@ -893,10 +893,10 @@ int conef_topk_sparsify_noalloc_f32(float* x, int64_t numel, int64_t k, void* st
     hipStream_t s = (hipStream_t)stream;
     TopkState* st = (TopkState*)ptr;
     const int64_t g = topk_hist_groups(numel);
-    hipLaunchKernelGGL(topk_init_kernel, dim3(1), dim3(256), 0, s, st, (uint32_t)k);      // clears what the last call left
+    conef_launch(topk_init_kernel, dim3(1), dim3(256), 0, s, st, (uint32_t)k);      // clears what the last call left
     for (int pass = 0; pass < kPasses; ++pass)
-        hipLaunchKernelGGL(topk_hist_kernel, dim3((unsigned)g), dim3(256), 0, s, x, numel, st, pass);
-    hipLaunchKernelGGL(topk_filter_kernel, dim3((unsigned)g), dim3(256), 0, s, x, numel, st);
+        conef_launch(topk_hist_kernel, dim3((unsigned)g), dim3(256), 0, s, x, numel, st, pass);
+    conef_launch(topk_filter_kernel, dim3((unsigned)g), dim3(256), 0, s, x, numel, st);
     return (int)hipGetLastError();
 }
 

@@ -417,6 +417,21 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
 int conef_psgd_q_next_f32(const ConefPsgdItem* items, int32_t count, float eps, float* const* q_next, int32_t* made,
                           void* workspace, int64_t workspace_bytes, void* stream);
 
+/* Tapes: a round's launches kept by the host and made again, for a caller whose tables and scalars stay as they
+ * are from step to step (no counterpart in the reference's interface).  Between conef_tape_record and
+ * conef_tape_stop, on one thread, the library's calls are made as always and their launches kept as well;
+ * conef_tape_stop names the table they were formed from (keep 0: forget them).  conef_tape_replay makes the launches
+ * again on `stream`: results are those of the calls.  It compares the table with what it held: CONEF_TAPE_STALE, and
+ * nothing is launched, where they differ or nothing is kept (a cooperative launch is not).  Whatever else the calls
+ * were given (scalars, flags, workspace, q_next) is the caller's to compare, and its memory the caller's to keep.  A
+ * tape is one thread's at a time; the handle is 0 where there is no memory. */
+#define CONEF_TAPE_STALE (-3)
+int64_t conef_tape_create(void);
+int conef_tape_destroy(int64_t tape);
+int conef_tape_record(int64_t tape);
+int conef_tape_stop(int64_t tape, const ConefPsgdItem* items, int32_t count, int32_t keep);
+int conef_tape_replay(int64_t tape, const ConefPsgdItem* items, int32_t count, void* stream);
+
 /* Dense error feedback on a stretch of the bucket that is not compressed: x += err; err = 0
  * (the copy-minus-result of powerSGD_hook.py:558 is exactly zero there). */
 int conef_ef_passthrough_f32(float* x, float* err, int64_t count, void* stream);

@@ -1255,6 +1255,69 @@ def test_high_rank_rounds_orthogonalise_q_on_a_side_stream(monkeypatch, rank, mo
         np.testing.assert_array_equal(x, y)
 
 
+@pytest.mark.parametrize("streams", [1, 2])
+@pytest.mark.parametrize("mode,rank", [("conef", 4), ("conef", 32), ("ef", 4), ("topk", 8), ("plain", 2)])
+def test_kept_launches_are_those_of_a_new_round(monkeypatch, mode, rank, streams):
+    """A step that repeats the last one's launches leaves the bits of one that forms them anew: over steps between
+    which nothing changes, a scalar changes, the state's buffers and sketches move, and the streams change."""
+    from conef_amd.hPowerSGD_hook import hPowerSGDState, hpowerSGD_hook
+    from conef_amd.powerSGD_hook import PowerSGDState, powerSGD_hook
+    buckets = [[(640, 576), (64,), (1100, 300), (1200, 130)], [(27, 40), (16, 27), (3,)], [(2100, 260), (100, 128)]]
+
+    def run(tape):
+        monkeypatch.setenv("CONEF_ROUND_TAPE", tape)
+        if mode == "topk":
+            hook, st = hpowerSGD_hook, hPowerSGDState(None, matrix_approximation_rank=rank, start_powerSGD_iter=2,
+                                                      use_error_compression=True, topk_ratio=0.4, hook_streams=streams)
+        else:
+            hook, st = powerSGD_hook, PowerSGDState(None, matrix_approximation_rank=rank, start_powerSGD_iter=2,
+                                                    use_error_feedback=mode != "plain", use_error_compression=mode == "conef",
+                                                    sketch_size=0.2, beta=0.9, hook_streams=streams)
+        st.iter = 2
+        flats = [torch.empty(numel_of(b), device="cuda") for b in buckets]
+        outs, kept = [], 0
+        for step in range(18):
+            if step == 6:
+                st.orthogonalization_epsilon = 1e-8
+                if mode == "conef":
+                    st.beta = 0.5
+                if mode == "topk":
+                    st.topk_ratio = 0.3
+            if step == 10:                       # the error state moves, as a loaded checkpoint's does
+                for i, e in st.error_dict.items():
+                    if isinstance(e, torch.Tensor):
+                        st.error_dict[i] = e.clone()
+                    else:
+                        for k in e:
+                            if isinstance(e[k], torch.Tensor):
+                                e[k] = e[k].clone()
+                            else:
+                                e[k].cs = e[k].cs.clone()
+            if step == 14:
+                st.hook_streams = 3 - streams
+            gen = torch.Generator().manual_seed(900 + step)
+            for f in flats:
+                f.copy_(torch.randn(f.numel(), generator=gen) * 1e-3)
+            futs = [hook(st, FakeGradBucket(f, b, index=i, is_last=i == len(buckets) - 1))
+                    for i, (f, b) in enumerate(zip(flats, buckets))]
+            outs += [to_np(f.wait()) for f in futs]
+            plan = st.round_cache[0]
+            kept += plan.tape is not None and plan.tape.signature is not None
+        for i in st.p_memory_dict:
+            outs += [to_np(st.p_memory_dict[i]), to_np(st.q_memory_dict[i])]
+            err = st.error_dict.get(i)
+            outs += [to_np(getattr(e, "cs", e)) for e in (err.values() if isinstance(err, dict) else [] if err is None else [err])]
+        return outs, kept
+
+    want, none = run("0")
+    got, kept = run("1")
+    # above rank 8 a single stream hands work to another one every step, which is not kept
+    assert none == 0 and (kept > 4 or rank > 8 and kept > 1), kept
+    assert len(want) == len(got)
+    for a, b in zip(want, got):
+        np.testing.assert_array_equal(a, b)
+
+
 # matrices whose rows are no whole number of quads and start anywhere in memory; widths at the edges of a
 # quad, a wave's and a workgroup's quads, and a column tile; heights at the edges of a row block
 RAGGED_BUCKETS = [
