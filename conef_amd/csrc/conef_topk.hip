@@ -162,7 +162,7 @@ __device__ __forceinline__ void topk_resolve(TopkState* st, int p, uint32_t* pre
 // `kept` (a state that stays with its tensor from call to call, zero-filled before the first): no
 // launch clears the state; the first workgroup of pass 0 clears what the later passes count into,
 // and the filter's, or the settling pass's, clears what pass 0 of the next call counts into.
-template <int REP>
+template <int REP, int T = 256>
 __device__ __forceinline__ void
 topk_hist_body(const float* __restrict__ x, int64_t numel, TopkState* st, int pass, int bx, int gx, bool kept = false,
                uint32_t k = 0)
@@ -171,7 +171,7 @@ topk_hist_body(const float* __restrict__ x, int64_t numel, TopkState* st, int pa
     uint32_t prefix = 0, remaining = 0, ties = 0;
     if (pass > 0) topk_resolve(st, pass - 1, &prefix, &remaining, &ties, bx);
     if (kept && pass == 0 && bx == 0) {
-        for (int i = threadIdx.x; i < (kPasses - 1) * kBins; i += 256) (&st->hist[1][0])[i] = 0u;
+        for (int i = threadIdx.x; i < (kPasses - 1) * kBins; i += T) (&st->hist[1][0])[i] = 0u;
         if (threadIdx.x == 0) {
             st->k = k;
             st->done = 0u;
@@ -180,41 +180,55 @@ topk_hist_body(const float* __restrict__ x, int64_t numel, TopkState* st, int pa
         }
     }
     const int nb = 1 << kDigitBits[pass];
-    for (int i = threadIdx.x; i < nb * REP; i += 256) bins[i] = 0u;
+    for (int i = threadIdx.x; i < nb * REP; i += T) bins[i] = 0u;
     __syncthreads();
     const int shift = kDigitShift[pass], hi = shift + kDigitBits[pass];
     const uint32_t mask = (uint32_t)nb - 1u;
     const int copy = (int)(threadIdx.x & (REP - 1));
     const int64_t quads = numel >> 2;
     const bool vec = (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
-    const int64_t stride = (int64_t)gx * blockDim.x;
+    const int64_t stride = (int64_t)gx * T;
     if (vec) {
         // eight 16-byte loads in flight per thread: a thread's share is sixteen quads or so, and every
         // round of loads is a trip to memory
         constexpr int U = 8;
-        for (int64_t q0 = bx * (int64_t)blockDim.x + threadIdx.x; q0 < quads; q0 += U * stride) {
+        auto count = [&](float4 v) {
+            const uint32_t key[4] = {mag_key(v.x), mag_key(v.y), mag_key(v.z), mag_key(v.w)};
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (pass == 0 || (key[e] >> hi) == prefix) atomicAdd(&bins[((key[e] >> shift) & mask) * REP + copy], 1u);
+        };
+        // Runs of 256 quads, run c to a workgroup whose number leaves the remainder of c by eight where there are
+        // that many: a pass with more threads in a workgroup then reads a run on the XCD whose L2 the next pass
+        // finds it in.
+        const int run = T == 256 || (gx & 7) ? bx * (T / 256) + ((int)threadIdx.x >> 8)
+                                             : (bx >> 3) * (T / 32) + ((int)threadIdx.x >> 8) * 8 + (bx & 7);
+        int64_t q0 = (int64_t)run * 256 + (threadIdx.x & 255);
+        for (; q0 + (U - 1) * stride < quads; q0 += U * stride) {
             float4 v[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
+            for (int u = 0; u < U; ++u) v[u] = reinterpret_cast<const float4*>(x)[q0 + u * stride];
+#pragma unroll
+            for (int u = 0; u < U; ++u) count(v[u]);
+        }
+        if (q0 < quads) {
+            float4 v[U - 1];
+#pragma unroll
+            for (int u = 0; u < U - 1; ++u) {
                 const int64_t q = q0 + u * stride;
                 v[u] = reinterpret_cast<const float4*>(x)[q < quads ? q : q0];
             }
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if (q0 + u * stride >= quads) break;
-                const uint32_t key[4] = {mag_key(v[u].x), mag_key(v[u].y), mag_key(v[u].z), mag_key(v[u].w)};
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (pass == 0 || (key[e] >> hi) == prefix) atomicAdd(&bins[((key[e] >> shift) & mask) * REP + copy], 1u);
-            }
+            for (int u = 0; u < U - 1; ++u)
+                if (q0 + u * stride < quads) count(v[u]);
         }
     }
-    for (int64_t i = (vec ? quads * 4 : 0) + bx * (int64_t)blockDim.x + threadIdx.x; i < numel; i += stride) {
+    for (int64_t i = (vec ? quads * 4 : 0) + bx * (int64_t)T + threadIdx.x; i < numel; i += stride) {
         uint32_t key = mag_key(x[i]);
         if (pass == 0 || (key >> hi) == prefix) atomicAdd(&bins[((key >> shift) & mask) * REP + copy], 1u);
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < nb; i += 256) {
+    for (int i = threadIdx.x; i < nb; i += T) {
         uint32_t c = 0;
 #pragma unroll
         for (int k = 0; k < REP; ++k) c += bins[i * REP + k];
@@ -628,6 +642,22 @@ __device__ __forceinline__ void topk_settle_body(const TopkItem& it, int bx, int
     topk_settle_ties(it.x, it.numel, st, thr, ties, held, gx);
 }
 
+// The first digit where the lists follow.  A histogram's workgroups end with an atomic addition for every bin they
+// have counted in, all on the same few dozen counters, and those queue: 8.4 M elements take 26 us with 1024 workgroups of
+// 256 threads, 19 with 512, 7.8 without the additions, and 11 with 256 workgroups of four times the threads (8 if they
+// take turns on eight copies of the counters, which the next pass then has to add up: not worth a larger state).
+// A bucket of BERT's errors, several tensors with counters of their own: 15.0 to 10.9 us.
+constexpr int kTopkFirst = 1024;
+
+template <int CAP>
+__global__ void __launch_bounds__(kTopkFirst)
+topk_first_batch_kernel(TopkBatch<CAP> b)
+{
+    int local, width;
+    const TopkItem& it = b.item[topk_locate(b.first, b.count, &local, &width)];
+    topk_hist_body<4, kTopkFirst>(it.x, it.numel, it.st, 0, local, width, true, it.k);
+}
+
 template <int CAP>
 __global__ void __launch_bounds__(256)
 topk_note_batch_kernel(TopkBatch<CAP> b)
@@ -659,15 +689,22 @@ topk_settle_batch_kernel(TopkBatch<CAP> b)
 // it touched, all workgroups on the same few dozen counters, and a filter workgroup that has to
 // settle ties ends with one on a single counter: fewer workgroups with longer loops (16 quads a
 // thread) beat many short ones.  At most 512 where three such passes read the tensor (31 M elements 141 us,
-// 164 with 1024), 1024 where there is one and the note pass, which ends with no shared counter but the
-// second digit's, gains from them.
+// 164 with 1024), 1024 for the note pass, which ends with no shared counter but the second digit's, and the passes
+// over its notes.  From eight on a multiple of eight, the XCDs (topk_hist_body).  (The note pass with workgroups of 1024 threads was slower, 18.0 against 16.5 us a BERT bucket.)
 inline int64_t topk_groups(int64_t numel, int64_t most)
 {
     const int64_t g = (numel + 255) / 256 / 64;
-    return g < 1 ? 1 : g > most ? most : g;
+    return g < 1 ? 1 : g > most ? most : g < 8 ? g : g & ~(int64_t)7;
 }
 inline int64_t topk_hist_groups(int64_t numel) { return topk_groups(numel, 512); }
 inline int64_t topk_listed_groups(int64_t numel) { return topk_groups(numel, 1024); }
+
+// of the first pass where the lists follow: four quads a thread or more
+inline int64_t topk_first_groups(int64_t numel)
+{
+    const int64_t g = topk_listed_groups(numel);
+    return g > 256 ? 256 : g;
+}
 
 
 // ---- selection state of the entry point that allocates nothing ------------------------------
@@ -795,7 +832,14 @@ void topk_launch(const TopkItem* items, int nb, TopkRun run, hipStream_t s)
     b.count = nb;
     const dim3 grid((unsigned)wgs), threads(256);
     if (run == TopkRun::kListed) {
-        conef_launch(topk_hist_batch_kernel<CAP>, grid, threads, 0, s, b, 0, true);
+        TopkBatch<CAP> fb = b;
+        int fw = 0;
+        for (int k = 0; k < nb; ++k) {
+            fb.first[k] = fw;
+            fw += (int)topk_first_groups(items[k].numel);
+        }
+        fb.first[nb] = fw;
+        conef_launch(topk_first_batch_kernel<CAP>, dim3((unsigned)fw), dim3(kTopkFirst), 0, s, fb);
         conef_launch(topk_note_batch_kernel<CAP>, grid, threads, 0, s, b);
         conef_launch(topk_gather_batch_kernel<CAP>, grid, threads, 0, s, b);
         conef_launch(topk_settle_batch_kernel<CAP>, grid, threads, 0, s, b);

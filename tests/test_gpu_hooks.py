@@ -1405,6 +1405,29 @@ def _topk_inputs():
     yield "ties at the threshold", few, 1010
 
 
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("numels", [(16_384,), (131_071,), (131_072, 5, 147_459), (1_000_003, 262_144), (4_300_001,)])
+def test_topk_first_digit_by_wide_workgroups(numels, off):
+    """The first digit's counts where a workgroup has 1024 threads: tensors of less than a trip, of several and a
+    rest, with workgroups in eights and not, on and off 16 bytes; every kept entry and no other."""
+    from conef_amd._psgd_engine import topk_sparsify_all
+    gen = torch.Generator().manual_seed(sum(numels))
+    host = [torch.randn(n, generator=gen) * 1e-3 for n in numels]
+    tensors = [torch.zeros(n + off, device="cuda")[off:] for n in numels]
+    table = None
+    for call in range(2):
+        for t, h in zip(tensors, host):
+            t.copy_(h.roll(call))
+        table = topk_sparsify_all(tensors, 0.4, table)
+        for t, h in zip(tensors, host):
+            full = h.roll(call).numpy()
+            k = max(1, int(0.5 * 0.4 * full.size))
+            want = np.zeros_like(full)
+            order = np.argsort(-np.abs(full), kind="stable")[:k]
+            want[order] = full[order]
+            np.testing.assert_array_equal(to_np(t), want)
+
+
 def test_topk_through_a_candidate_list():
     """The entry point whose workspace stays with its tensors (the hooks' one), three calls on one
     workspace, every tensor alone and all of them in one batch."""
