@@ -1149,7 +1149,7 @@ psgd_pqt_one_kernel(PqtItem it)
 // overwritten with P Q^T on the way (powerSGD_hook.py:551,563-564).
 // LIN (with FAST): M lies as the gradient came, and X = M + alpha * unsketch(cs) is formed here (conef_psgd_linear.h);
 // the tile's old cells go to their place in LDS first.
-template <int RP, bool FAST, bool LIN = false>
+template <int RP, bool FAST, bool LIN = false, int T = kConefRowlistThreads>
 struct ListPsgdResidual {
     float* x;
     const float* p;
@@ -1159,6 +1159,7 @@ struct ListPsgdResidual {
     const float* cs;         // LIN: the old cells
     float alpha;             // LIN
     static constexpr bool kNeedsCells = false, kParksCells = LIN;
+    static constexpr int kThreads = T;
     // Half-height tiles where there are tiles to spare (conef_rowlist_shape) up to rank 4 and from 512 columns
     // on: full against half height [30522,1024] 69.2 and 62.5 us at rank 4 (79.0 and 93.0 at rank 8, whose slices
     // of Q a tile loads whatever its height), [50000,512] 64.0 and 52.7 (72.0 and 73.1), [20000,2048] 89.3 and
@@ -1177,11 +1178,11 @@ struct ListPsgdResidual {
             // quad - or the next quad's slice of Q and its first two rows - are requested before the
             // current two are used, so that a thread has one round trip per tile, not one per step.
             __shared__ float ptile[16 * RP];              // at most 16 rows a tile
-            for (int i = threadIdx.x; i < rows * RP; i += kConefRowlistThreads) ptile[i] = p[row0 * RP + i];
+            for (int i = threadIdx.x; i < rows * RP; i += T) ptile[i] = p[row0 * RP + i];
             const int d4 = (d + 3) >> 2;
             const bool quad_rows = (d & 3) == 0;           // rows of LDS values start on 16 bytes
-            const int lanes = d4 < kConefRowlistThreads ? d4 : kConefRowlistThreads;
-            const int groups = kConefRowlistThreads / lanes, grp = threadIdx.x / lanes;
+            const int lanes = d4 < T ? d4 : T;
+            const int groups = T / lanes, grp = threadIdx.x / lanes;
             const int step = 2 * groups;
             int c4 = threadIdx.x - grp * lanes, rw = 2 * grp;
             bool have = grp < groups && c4 < d4 && rw < rows;
@@ -1199,8 +1200,8 @@ struct ListPsgdResidual {
 #pragma unroll
                 for (int u = 0; u < kCells; ++u) {
                     ct[u] = 0.f;
-                    if (u * kConefRowlistThreads < rows * w) {
-                        const int i = (int)threadIdx.x + u * kConefRowlistThreads;
+                    if (u * T < rows * w) {
+                        const int i = (int)threadIdx.x + u * T;
                         ct[u] = cs[row0 * w + (i < rows * w ? i : rows * w - 1)];
                     }
                 }
@@ -1213,19 +1214,19 @@ struct ListPsgdResidual {
             if constexpr (LIN) {
 #pragma unroll
                 for (int u = 0; u < kCells; ++u) {
-                    const int i = (int)threadIdx.x + u * kConefRowlistThreads;
+                    const int i = (int)threadIdx.x + u * T;
                     if (i < rows * w) cells[i] = ct[u];
                 }
-                for (int i0 = (int)threadIdx.x + kCells * kConefRowlistThreads; i0 < rows * w; i0 += 4 * kConefRowlistThreads) {
+                for (int i0 = (int)threadIdx.x + kCells * T; i0 < rows * w; i0 += 4 * T) {
                     float t[4];
 #pragma unroll
                     for (int u = 0; u < 4; ++u) {
-                        const int i = i0 + u * kConefRowlistThreads;
+                        const int i = i0 + u * T;
                         t[u] = cs[row0 * w + (i < rows * w ? i : rows * w - 1)];
                     }
 #pragma unroll
                     for (int u = 0; u < 4; ++u) {
-                        const int i = i0 + u * kConefRowlistThreads;
+                        const int i = i0 + u * T;
                         if (i < rows * w) cells[i] = t[u];
                     }
                 }
@@ -1307,8 +1308,8 @@ struct ListPsgdResidual {
         } else {
             const int total = rows * d;
             int row = threadIdx.x / d, col = threadIdx.x - row * d;
-            const int srow = kConefRowlistThreads / d, sc = kConefRowlistThreads - srow * d;
-            for (int e = threadIdx.x; e < total; e += kConefRowlistThreads) {
+            const int srow = T / d, sc = T - srow * d;
+            for (int e = threadIdx.x; e < total; e += T) {
                 const float* pi = p + (row0 + row) * r;
                 const float* qk = q + (int64_t)col * r;
                 float mh = 0.f;
@@ -3531,9 +3532,9 @@ int orthogonalise_by_gram_wide(const PaddedRound& pr, int r, const std::vector<c
     });
 }
 
-template <int RP, bool FAST, bool LIN = false>
+template <int RP, bool FAST, bool LIN = false, int T = kConefRowlistThreads>
 struct RowlistResidualItem {
-    ListPsgdResidual<RP, FAST, LIN> front;
+    ListPsgdResidual<RP, FAST, LIN, T> front;
     ConefRowlistView plan;
     const float* cs_in;
     float* cs_out;
@@ -3627,19 +3628,19 @@ struct LinNext {
 
 constexpr int kLinNextRows = 512;     // rows a workgroup takes at once
 
-template <int RP>
+template <int RP, int T>
 __device__ __forceinline__ void psgd_lin_next_body(const LinNext& g, const float* q, int m, int k, int part)
 {
-    constexpr int U = kLinNextRows / 256;
+    constexpr int U = kLinNextRows / T;
     __shared__ float t_l[RP * RP + RP];
     float x[U][RP];
     auto request = [&](int row) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) load_row<RP>(q + (int64_t)(row + u * 256 < m ? row + u * 256 : m - 1) * RP, x[u]);
+        for (int u = 0; u < U; ++u) load_row<RP>(q + (int64_t)(row + u * T < m ? row + u * T : m - 1) * RP, x[u]);
     };
     int row = part * kLinNextRows + (int)threadIdx.x;
     request(row);                                                      // travels while the system is solved
-    gram_solve_lds<RP, 256>(g.parts[k], g.nparts[k], g.eps, t_l);
+    gram_solve_lds<RP, T>(g.parts[k], g.nparts[k], g.eps, t_l);
     if (part == 0 && g.tmat[k] && (int)threadIdx.x < RP * RP + RP) g.tmat[k][threadIdx.x] = t_l[threadIdx.x];
     for (;;) {
 #pragma unroll
@@ -3650,7 +3651,7 @@ __device__ __forceinline__ void psgd_lin_next_body(const LinNext& g, const float
                 for (int c = 0; c < RP; ++c)
                     if (c >= g.r) x[u][c] = 0.f;
             }
-            if (row + u * 256 < m) store_row<RP>(g.dst[k] + (int64_t)(row + u * 256) * RP, x[u]);
+            if (row + u * T < m) store_row<RP>(g.dst[k] + (int64_t)(row + u * T) * RP, x[u]);
         }
         row += g.split * kLinNextRows;
         if (row >= m) break;
@@ -3659,18 +3660,17 @@ __device__ __forceinline__ void psgd_lin_next_body(const LinNext& g, const float
 }
 
 // The residual kernel over M as the gradient came, with those workgroups in front.
-template <int RP>
-__global__ void __launch_bounds__(kConefRowlistThreads)
-psgd_lin_residual_batch_kernel(PsgdBatch<RowlistResidualItem<RP, true, true>> b, double one_minus_beta, LinNext g)
+template <int RP, int T>
+__global__ void __launch_bounds__(T)
+psgd_lin_residual_batch_kernel(PsgdBatch<RowlistResidualItem<RP, true, true, T>> b, double one_minus_beta, LinNext g)
 {
-    static_assert(kConefRowlistThreads == 256, "one block size for both kinds of workgroup");
     const int riders = g.count * (g.split + g.fold_split);
     if ((int)blockIdx.x < riders) {
         const int k = (int)blockIdx.x / (g.split + g.fold_split), part = (int)blockIdx.x - k * (g.split + g.fold_split);
-        const RowlistResidualItem<RP, true, true>& it = b.item[k];
+        const RowlistResidualItem<RP, true, true, T>& it = b.item[k];
         if (part < g.split) {
-            psgd_lin_next_body<RP>(g, it.front.q, it.d, k, part);
-        } else if (const int j = (part - g.split) * 256 + (int)threadIdx.x; j < it.w) {
+            psgd_lin_next_body<RP, T>(g, it.front.q, it.d, k, part);
+        } else if (const int j = (part - g.split) * T + (int)threadIdx.x; j < it.w) {
             float f[RP];
             conef_fold_row<RP, 4>(it.front.q, RP, it.plan.ent, it.plan.csr[j], it.plan.csr[j + 1], f);
             store_row<RP>(g.fold[k] + (int64_t)j * RP, f);
@@ -3679,8 +3679,8 @@ psgd_lin_residual_batch_kernel(PsgdBatch<RowlistResidualItem<RP, true, true>> b,
     }
     const int bx = (int)blockIdx.x - riders;
     const int i = psgd_batch_item(b, bx);
-    const RowlistResidualItem<RP, true, true>& it = b.item[i];
-    conef_rowlist_body<float, ListPsgdResidual<RP, true, true>>(it.front, it.plan, it.cs_in, it.cs_out, it.n, it.d, it.w, it.rb,
+    const RowlistResidualItem<RP, true, true, T>& it = b.item[i];
+    conef_rowlist_body<float, ListPsgdResidual<RP, true, true, T>>(it.front, it.plan, it.cs_in, it.cs_out, it.n, it.d, it.w, it.rb,
                                                                 one_minus_beta, bx - b.first[i]);
 }
 
@@ -4104,16 +4104,25 @@ int round_linear(PaddedRound& pr, LinearRound& lr, int r, float* const* q_in, co
     for (int k = 0; k < count; ++k) members.push_back(k);
     std::vector<ConefRowlistShape> shapes;
     if (!residual_tiles<RP, true>(items, members, &shapes)) return CONEF_ERR_INVALID;
-    std::vector<RowlistResidualItem<RP, true, true>> last;
     size_t lds = 0;
+    bool wide_rows = false;
     blocks.clear();
     next.split = 1;
-    next.fold_split = 0;
     for (int k = 0; k < count; ++k) {
         const ConefPsgdItem& it = items[k];
-        const ConefRowlistShape& shape = shapes[(size_t)k];
-        last.push_back(RowlistResidualItem<RP, true, true>{{it.x, it.p, it.q, it.r, pr.qi[(size_t)k], it.cs, alpha}, lr.view[(size_t)k],
-                                                           it.cs, it.cs, it.n, (int)it.m, it.w, shape.rb});
+        ConefRowlistShape& shape = shapes[(size_t)k];
+        // Rows so wide that a tile would be one: two of them, and twice the threads for the launch.  A tile's chain of
+        // trips (column quads with their slices of Q, then the buckets) is what such a launch lasts, and half of what the
+        // stage forms for a pair of rows is thrown away with one: [640,5760] at rank 4 19.9 us, with two rows or with
+        // twice the threads alone 20.0 and 20.8, with both 16.4.  (Rows of several to a tile lose by more threads:
+        // BERT's buckets at rank 8 18.6 and 25.0.)
+        if (const size_t two = conef_rowlist_lds(2, it.m, it.w, false);
+            shape.rb == 1 && it.m > 4096 && it.n > 1 && two <= kConefRowlistLdsLimit / 2) {
+            shape.rb = 2;
+            shape.lds = two;
+            shape.tiles = (it.n + 1) / 2;
+            wide_rows = true;
+        }
         blocks.push_back((int)shape.tiles);
         if (shape.lds > lds) lds = shape.lds;
         next.split = std::max(next.split, (int)std::min((it.m + kLinNextRows - 1) / kLinNextRows, (int64_t)16));
@@ -4121,16 +4130,29 @@ int round_linear(PaddedRound& pr, LinearRound& lr, int r, float* const* q_in, co
         next.parts[k] = qgrams[(size_t)k];
         next.nparts[k] = (int)defer_qgram_shares(it);
         next.fold[k] = kept.empty() ? nullptr : kept[(size_t)k].fold;
-        next.fold_split = std::max(next.fold_split, kept.empty() ? 0 : (it.w + 255) / 256);
     }
     next.r = r;
     next.eps = eps;
-    auto residual = psgd_lin_residual_batch_kernel<RP>;
-    if (hipError_t e = conef_allow_lds((const void*)residual, lds); e != hipSuccess) return (int)e;
     const double omb = 1. - (double)beta;
-    return run_batches(last, blocks, [&](const PsgdBatch<RowlistResidualItem<RP, true, true>>& bt, int grid) {
-        conef_launch(residual, dim3((unsigned)(grid + next.count * (next.split + next.fold_split))), dim3(kConefRowlistThreads), lds, s, bt, omb, next);
-    });
+    auto residual = [&](auto threads) {
+        constexpr int T = decltype(threads)::value;
+        std::vector<RowlistResidualItem<RP, true, true, T>> last;
+        next.fold_split = 0;
+        for (int k = 0; k < count; ++k) {
+            const ConefPsgdItem& it = items[k];
+            last.push_back(RowlistResidualItem<RP, true, true, T>{{it.x, it.p, it.q, it.r, pr.qi[(size_t)k], it.cs, alpha},
+                                                                  lr.view[(size_t)k], it.cs, it.cs, it.n, (int)it.m, it.w,
+                                                                  shapes[(size_t)k].rb});
+            next.fold_split = std::max(next.fold_split, kept.empty() ? 0 : (it.w + T - 1) / T);
+        }
+        auto kern = psgd_lin_residual_batch_kernel<RP, T>;
+        if (hipError_t e = conef_allow_lds((const void*)kern, lds); e != hipSuccess) return (int)e;
+        return run_batches(last, blocks, [&](const PsgdBatch<RowlistResidualItem<RP, true, true, T>>& bt, int grid) {
+            conef_launch(kern, dim3((unsigned)(grid + next.count * (next.split + next.fold_split))), dim3(T), lds, s, bt, omb, next);
+        });
+    };
+    if (wide_rows) return residual(std::integral_constant<int, 2 * kConefRowlistThreads>());
+    return residual(std::integral_constant<int, kConefRowlistThreads>());
 }
 
 // Whether a round of these matrices runs with the orthogonalisation of P deferred: where the batch allows

@@ -96,6 +96,7 @@ struct ConefListVec {
     const float* vec;
     bool vec_ok;           // base 16-byte aligned and d % 4 == 0 (the tile copy works either way)
     static constexpr bool kNeedsCells = false, kParksCells = false;
+    static constexpr int kThreads = kConefRowlistThreads;
     // whether a tensor with tiles to spare goes by half-height ones.  Full against half height: [50000,512] 40.2
     // and 29.9 us, [20000,2048] 49.0 and 45.9, [30522,1024] 37.0 and 36.2, [33278,650] 26.2 and 26.0, [60000,300]
     // and [33278,200] within 1 % either way.
@@ -157,6 +158,7 @@ struct ConefListRandBlock {
     ConefBlock blk;
     float alpha;
     static constexpr bool kNeedsCells = true, kParksCells = false;
+    static constexpr int kThreads = kConefRowlistThreads;
     static bool halves(int64_t) { return true; }      // (the column table sits in LDS next to the tiles)
     static constexpr int kQuads = 4;
     struct Regs {          // a thread's first kQuads quads, by name: no array for the compiler to keep in memory
@@ -308,18 +310,19 @@ struct ConefListRandBlock {
 
 // ------------------------------------------------------------------ kernel ----
 // count >= 1 words from global memory to LDS, eight loads in flight per thread
+template <int T>
 __device__ __forceinline__ void conef_copy_words_to_lds(uint32_t* dst, const uint32_t* __restrict__ src, int count)
 {
-    for (int i0 = threadIdx.x; i0 < count; i0 += 8 * kConefRowlistThreads) {
+    for (int i0 = threadIdx.x; i0 < count; i0 += 8 * T) {
         uint32_t t[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            int i = i0 + u * kConefRowlistThreads;
+            int i = i0 + u * T;
             t[u] = src[i < count ? i : count - 1];
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            int i = i0 + u * kConefRowlistThreads;
+            int i = i0 + u * T;
             if (i < count) dst[i] = t[u];
         }
     }
@@ -334,6 +337,7 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
     // are often short, and a request past the end is a request all the same: [33278,650] 25.6 us against 26.0,
     // [30522,1024] 34.8 against 36.2, a pair [4096,1024] + [1024,4096] 16.9 against 16.7) and made where they are
     // halves ([640,5760] 10.3 us without the tests, 11.2 with them; [33278,650] 25.5 and 27.8).
+    constexpr int T = Front::kThreads;
     constexpr bool sparing = sizeof(CsT) == sizeof(float);
     extern __shared__ float conef_rl[];
     float* vals = conef_rl;
@@ -355,13 +359,13 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
     const uint32_t ord_pre = ord_src[(int)threadIdx.x < ord_words ? (int)threadIdx.x : ord_words - 1];
 #pragma unroll
     for (int u = 0; u < kPreE; ++u) {
-        const int i = threadIdx.x + u * kConefRowlistThreads;
-        if (!sparing || u * kConefRowlistThreads < ent_words) ent_pre[u] = ent_src[i < ent_words ? i : ent_words - 1];
+        const int i = threadIdx.x + u * T;
+        if (!sparing || u * T < ent_words) ent_pre[u] = ent_src[i < ent_words ? i : ent_words - 1];
     }
 #pragma unroll
     for (int u = 0; u < kPreC; ++u) {
-        const int i = threadIdx.x + u * kConefRowlistThreads;
-        if (!sparing || u * kConefRowlistThreads < csr_words) csr_pre[u] = plan.csr[i < csr_words ? i : csr_words - 1];
+        const int i = threadIdx.x + u * T;
+        if (!sparing || u * T < csr_words) csr_pre[u] = plan.csr[i < csr_words ? i : csr_words - 1];
     }
     typename Front::Regs regs;
     uint32_t* pk_l = reinterpret_cast<uint32_t*>(cells + rb * w);
@@ -376,20 +380,20 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
         uint32_t pt[kPark];
 #pragma unroll
         for (int u = 0; u < kPark; ++u) {
-            const int i = threadIdx.x + u * kConefRowlistThreads;
-            if (!sparing || u * kConefRowlistThreads < count) ct[u] = conef_ld(src + (i < count ? i : count - 1));
-            if (!sparing || (pk_lds && u * kConefRowlistThreads < d)) pt[u] = plan.pk[i < d ? i : d - 1];
+            const int i = threadIdx.x + u * T;
+            if (!sparing || u * T < count) ct[u] = conef_ld(src + (i < count ? i : count - 1));
+            if (!sparing || (pk_lds && u * T < d)) pt[u] = plan.pk[i < d ? i : d - 1];
         }
 #pragma unroll
         for (int u = 0; u < kPark; ++u) {
-            const int i = threadIdx.x + u * kConefRowlistThreads;
+            const int i = threadIdx.x + u * T;
             if (i < count) cells[i] = ct[u];
             if (pk_lds && i < d) pk_l[i] = pt[u];
         }
-        for (int i = threadIdx.x + kPark * kConefRowlistThreads; i < count; i += kConefRowlistThreads)
+        for (int i = threadIdx.x + kPark * T; i < count; i += T)
             cells[i] = conef_ld(src + i);
         if (pk_lds)
-            for (int i = threadIdx.x + kPark * kConefRowlistThreads; i < d; i += kConefRowlistThreads)
+            for (int i = threadIdx.x + kPark * T; i < d; i += T)
                 pk_l[i] = plan.pk[i];
         __syncthreads();
     }
@@ -402,8 +406,8 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
     if constexpr (!Front::kNeedsCells && !Front::kParksCells) {
 #pragma unroll
         for (int u = 0; u < kPre; ++u) {
-            const int p = threadIdx.x + u * kConefRowlistThreads;
-            if (!sparing || u * kConefRowlistThreads < total) aux_pre[u] = conef_ld(cs_in + row0 * w + (p < total ? p : total - 1));
+            const int p = threadIdx.x + u * T;
+            if (!sparing || u * T < total) aux_pre[u] = conef_ld(cs_in + row0 * w + (p < total ? p : total - 1));
         }
     }
     if constexpr (Front::kNeedsCells) {
@@ -415,33 +419,33 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
         uint32_t* ent_w = reinterpret_cast<uint32_t*>(ent_l);
 #pragma unroll
         for (int u = 0; u < kPreE; ++u) {
-            const int i = threadIdx.x + u * kConefRowlistThreads;
+            const int i = threadIdx.x + u * T;
             if (i < ent_words) ent_w[i] = ent_pre[u];
         }
 #pragma unroll
         for (int u = 0; u < kPreC; ++u) {
-            const int i = threadIdx.x + u * kConefRowlistThreads;
+            const int i = threadIdx.x + u * T;
             if (i < csr_words) csr_l[i] = csr_pre[u];
         }
         uint32_t* ord_w = reinterpret_cast<uint32_t*>(ord_l);
         if ((int)threadIdx.x < ord_words) ord_w[threadIdx.x] = ord_pre;
-        if (ord_words > kConefRowlistThreads)
-            conef_copy_words_to_lds(ord_w + kConefRowlistThreads, ord_src + kConefRowlistThreads,
-                                    ord_words - kConefRowlistThreads);
-        if (ent_words > kPreE * kConefRowlistThreads)
-            conef_copy_words_to_lds(ent_w + kPreE * kConefRowlistThreads, ent_src + kPreE * kConefRowlistThreads,
-                                    ent_words - kPreE * kConefRowlistThreads);
-        if (csr_words > kPreC * kConefRowlistThreads)
-            conef_copy_words_to_lds(csr_l + kPreC * kConefRowlistThreads, plan.csr + kPreC * kConefRowlistThreads,
-                                    csr_words - kPreC * kConefRowlistThreads);
+        if (ord_words > T)
+            conef_copy_words_to_lds<T>(ord_w + T, ord_src + T,
+                                    ord_words - T);
+        if (ent_words > kPreE * T)
+            conef_copy_words_to_lds<T>(ent_w + kPreE * T, ent_src + kPreE * T,
+                                    ent_words - kPreE * T);
+        if (csr_words > kPreC * T)
+            conef_copy_words_to_lds<T>(csr_l + kPreC * T, plan.csr + kPreC * T,
+                                    csr_words - kPreC * T);
     }
     if constexpr (!Front::kNeedsCells && !Front::kParksCells) {
 #pragma unroll
         for (int u = 0; u < kPre; ++u) {
-            const int p = threadIdx.x + u * kConefRowlistThreads;
+            const int p = threadIdx.x + u * T;
             if (p < total) cells[p] = aux_pre[u];
         }
-        for (int p = threadIdx.x + kPre * kConefRowlistThreads; p < total; p += kConefRowlistThreads)
+        for (int p = threadIdx.x + kPre * T; p < total; p += T)
             cells[p] = conef_ld(cs_in + row0 * w + p);
     }
     __syncthreads();
@@ -456,12 +460,12 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
     // 16.8; [9000,333] with 166 buckets 9.9 and 8.7, 13.3 and 12.2.  Four rows were slower than two everywhere
     // ([33278,650] 25.4), and two lose where they leave threads without work ([20000,300] with 15 buckets 9.0
     // and 9.7).
-    if (sizeof(CsT) == sizeof(float) && rows >= 2 && total > kConefRowlistThreads) {
+    if (sizeof(CsT) == sizeof(float) && rows >= 2 && total > T) {
         constexpr int kTrip = 2;
         const int per = (rows + 1) >> 1, items = per * w;
         int jj = threadIdx.x / per, rg = threadIdx.x - jj * per;
-        const int sjj = kConefRowlistThreads / per, srg = kConefRowlistThreads - sjj * per;
-        for (int p = threadIdx.x; p < items; p += kConefRowlistThreads) {
+        const int sjj = T / per, srg = T - sjj * per;
+        for (int p = threadIdx.x; p < items; p += T) {
             const int j = ord_l[jj], ra = 2 * rg, rb2 = ra + 1 < rows ? ra + 1 : ra;
             const uint32_t e0 = csr_l[j], e1 = csr_l[j + 1];
             const float *va = vals + ra * d, *vb = vals + rb2 * d;
@@ -497,8 +501,8 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
         return;
     }
     int jj = threadIdx.x / rows, row = threadIdx.x - jj * rows;
-    const int sjj = kConefRowlistThreads / rows, srow = kConefRowlistThreads - sjj * rows;
-    for (int p = threadIdx.x; p < total; p += kConefRowlistThreads) {
+    const int sjj = T / rows, srow = T - sjj * rows;
+    for (int p = threadIdx.x; p < total; p += T) {
         const int j = ord_l[jj];
         const int cell = row * w + j;
         const uint32_t e0 = csr_l[j], e1 = csr_l[j + 1];
