@@ -43,8 +43,9 @@ struct ConefKeptLaunch : ConefTape::Launch {
     unsigned* tag = nullptr;                       // the argument that is a launch tag, if one is
     std::atomic<unsigned>* counter = nullptr;
 
-    ConefKeptLaunch(void (*k)(P...), dim3 g, dim3 b, size_t l, std::tuple<P...>&& a)
-        : kernel(k), grid(g), block(b), lds((unsigned)l), args(std::move(a)) {}
+    template <typename... A>
+    ConefKeptLaunch(void (*k)(P...), dim3 g, dim3 b, size_t l, const A&... a)
+        : kernel(k), grid(g), block(b), lds((unsigned)l), args(a...) {}
 
     template <size_t... I>
     void make(hipStream_t s, std::index_sequence<I...>)
@@ -63,9 +64,8 @@ struct ConefKeptLaunch : ConefTape::Launch {
 template <typename... P, typename... A>
 void conef_launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t s, const A&... args)
 {
-    ConefKeptLaunch<P...> now(kernel, grid, block, lds, std::tuple<P...>(args...));
-    now.make(s, std::index_sequence_for<P...>());
-    if (conef_recording) conef_recording->launches.emplace_back(new ConefKeptLaunch<P...>(std::move(now)));
+    hipLaunchKernelGGL(kernel, grid, block, (unsigned)lds, s, P(args)...);
+    if (conef_recording) conef_recording->launches.emplace_back(new ConefKeptLaunch<P...>(kernel, grid, block, lds, args...));
 }
 
 // The same with argument I a launch tag drawn from `counter`.
@@ -73,7 +73,7 @@ template <size_t I, typename... P, typename... A>
 void conef_launch_tagged(std::atomic<unsigned>& counter, void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t s,
                          const A&... args)
 {
-    ConefKeptLaunch<P...> now(kernel, grid, block, lds, std::tuple<P...>(args...));
+    ConefKeptLaunch<P...> now(kernel, grid, block, lds, args...);
     std::get<I>(now.args) = conef_next_tag(counter);
     now.make(s, std::index_sequence_for<P...>());
     if (!conef_recording) return;
