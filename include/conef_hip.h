@@ -341,7 +341,9 @@ int conef_psgd_sketch_update_batch_f32(const ConefPsgdItem* items, int32_t count
  * conef_psgd_mq_batch_f32 (mq_mode), Gram-Schmidt of every P, conef_psgd_mtp_batch_f32,
  * conef_psgd_pqt_batch_f32 (pqt_mode 0..2; 3 = mode 1, then conef_psgd_sketch_update_batch_f32 on the
  * residuals it wrote to err).  Replaces powerSGD_hook.py:473-564 at world size 1 (the all-reduces in
- * between are the identity there).  Same launches as the separate calls, in the same order. */
+ * between are the identity there).  The launches are those of the separate calls, in the same order, only with
+ * CONEF_ROUND_DEFER=0 in the environment: the orthogonalisation of P is deferred else where the batch allows, and a
+ * sketched error (mq_mode 2, pqt_mode 2) up to rank 8 is added to the products instead of to the matrices. */
 int conef_psgd_round_f32(const ConefPsgdItem* items, int32_t count, int32_t mq_mode, int32_t pqt_mode, float alpha,
                          float beta, float eps, int32_t a, int32_t b, void* workspace, int64_t workspace_bytes,
                          void* stream);
