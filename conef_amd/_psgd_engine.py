@@ -464,7 +464,6 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
                 it.plan_host, it.plan_dev = (sk_plan.host_ptr, sk_plan.device.data_ptr()) if sk_plan is not None else (None, None)
                 plan.sketches.append((cs, sk_plan))
             plan.batched_update = all(p is not None and p.batchable for _, p in plan.sketches)
-            plan.fused_sketch = state.matrix_approximation_rank <= 8 and plan.batched_update
             plan.small = None
             plan.ws_need = None
             _drop_q_next(plan, lambda: _lib.current_stream(device))      # sized for the sketches, and holds sums over their buckets
@@ -475,6 +474,8 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
             plan.cells = _host.same_sketches(errs.values(), moves + [True] * (len(errs) - count))
             for cnt, (cs, _) in enumerate(plan.sketches):
                 items[cnt].cs = cs.cs.data_ptr()
+            plan.fused_sketch = plan.batched_update and (state.matrix_approximation_rank <= 8 or not plan.is_wide and all(
+                lib.conef_psgd_round_wide_sketch_fits(run, part, HASH_A, HASH_B) for run, part in plan.runs))
         if not plan.cs_static:
             for cnt, (cs, _) in enumerate(plan.sketches):
                 items[cnt].cs = cs.cs.data_ptr()
@@ -520,8 +521,8 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
     elif error_mode == "conef" and plan.fused_sketch:
         mode3 = 2
     elif error_mode in ("conef", "conef_v2"):
-        # The residual goes out dense and the sketches are updated from it afterwards: ranks above
-        # 8 (the low-rank product belongs on the matrix cores), sketches whose plan is not a row
+        # The residual goes out dense and the sketches are updated from it afterwards: buckets that
+        # conef_psgd_round_wide_sketch_fits does not take above rank 8, sketches whose plan is not a row
         # list, and the re-viewed sketches of C2CS_hook_v2.
         residual = _scratch_f32(device, stream, max(plan.residual_offsets[-1], 1))
         for cnt in range(count):

@@ -27,6 +27,7 @@
 #include "conef_psgd_stream.h"
 #include "conef_psgd_small.h"
 #include "conef_psgd_linear.h"
+#include "conef_psgd_mfma_residual.h"
 #include "conef_hip.h"      // ConefPsgdItem, and a check of this file's definitions against the public header
 
 extern "C" int conef_cs_query_f32(float* x, const float* cs, int64_t n, int64_t d, int32_t w, float alpha, int32_t a,
@@ -661,7 +662,7 @@ struct DeferFixItem {
     float* pt;
     float* qt;
     int r;
-    float* qi;               // not null: Q by quads for the launch that follows (conef_store_slice_row)
+    float* qi;               // not null: Q in the order the launch that follows loads it (conef_store_slice_row, conef_piece_at)
     // not null: partials of cs^T P, [slabs][w][RP]; row j of Q gets alpha times the row of its bucket
     // (conef_psgd_linear.h)
     const float* cs_src;
@@ -924,6 +925,7 @@ psgd_defer_fix_wide_batch_kernel(PsgdBatch<DeferFixItem> b)
 #pragma unroll
         for (int c = 0; c < 4; ++c) o[c] = rows_l[lrow][4 * piece + c];
         st4((is_p ? it.p : it.q) + row * RP + 4 * piece, o);
+        if (!is_p && it.qi) st4(it.qi + conef_piece_at(it.m, piece, row), o);
         if (float* copy = is_p ? it.pt : it.qt) {
             float* dst = copy + row * it.r + 4 * piece;
 #pragma unroll
@@ -1176,7 +1178,7 @@ struct ListPsgdResidual {
     const float* qi;         // not null: q laid out by quads (conef_load_slices), FAST
     const float* cs;         // LIN: the old cells
     float alpha;             // LIN
-    static constexpr bool kNeedsCells = false, kParksCells = LIN;
+    static constexpr bool kNeedsCells = false, kParksCells = LIN, kCompact = false;
     static constexpr int kThreads = T;
     static constexpr size_t kDeclaredLds = FAST ? 4 * 16 * RP : 0;      // ptile
     // Half-height tiles where there are tiles to spare (conef_rowlist_shape) up to rank 4 and from 512 columns
@@ -3219,7 +3221,7 @@ inline int64_t defer_region_offset(const ConefPsgdItem* items, int count)
 struct PaddedRound {
     std::vector<ConefPsgdItem> items;
     std::vector<float*> pt, qt;      // the caller's factors where items holds copies, else null
-    std::vector<float*> qi;          // ranks up to 8: the new Q by quads (conef_store_slice_row)
+    std::vector<float*> qi;          // the new Q by quads (ranks up to 8, conef_store_slice_row) or by pieces (wide_sketch_round)
     int rp;
     bool padded;
     int64_t offset;                  // defer_region_offset of the items
@@ -3357,7 +3359,7 @@ int defer_fix(const PaddedRound& pr, int r, const std::vector<MtpRaw>& raw, cons
         const CellRaw c = cells ? (*cells)[(size_t)k] : CellRaw{nullptr, nullptr, 0};
         fix.push_back(DeferFixItem{it.p, raw[(size_t)k].src, it.q, tmats[(size_t)k], qgrams ? (*qgrams)[(size_t)k] : nullptr,
                                    it.n, it.m, raw[(size_t)k].slabs, pb, pr.pt[(size_t)k], pr.qt[(size_t)k], r,
-                                   rp <= 8 ? pr.qi[(size_t)k] : nullptr, c.src, c.pk, c.w});
+                                   pr.qi.empty() ? nullptr : pr.qi[(size_t)k], c.src, c.pk, c.w});
         blocks.push_back(pb + qb);
     }
     return run_batches(fix, blocks, [&](const PsgdBatch<DeferFixItem>& bt, int grid) {
@@ -3717,6 +3719,17 @@ psgd_lin_residual_batch_kernel(PsgdBatch<RowlistResidualItem<RP, true, true, T>>
     const RowlistResidualItem<RP, true, true, T>& it = b.item[i];
     conef_rowlist_body<float, ListPsgdResidual<RP, true, true, T>>(it.front, it.plan, it.cs_in, it.cs_out, it.n, it.d, it.w, it.rb,
                                                                 one_minus_beta, bx - b.first[i]);
+}
+
+// M = P Q^T at ranks 9 to 32 with the residuals sketched (conef_psgd_mfma_residual.h).
+template <int RP, int T>
+__global__ void __launch_bounds__(T, 4)
+psgd_mfma_residual_batch_kernel(PsgdBatch<MfmaResidualItem<RP, T>> b, double one_minus_beta)
+{
+    int local;
+    const MfmaResidualItem<RP, T>& it = b.item[psgd_batch_locate(b, &local)];
+    conef_rowlist_body<float, ListMfmaResidual<RP, T>>(it.front, it.plan, it.cs_in, it.cs_out, it.n, it.d, it.w, it.rb,
+                                                       one_minus_beta, local);
 }
 
 // Rows a workgroup of the dense M = P Q^T takes: as many as leave the launch two thousand workgroups
@@ -4262,6 +4275,146 @@ int round_linear(PaddedRound& pr, LinearRound& lr, int r, float* const* q_in, co
     return residual(std::integral_constant<int, kConefRowlistThreads>());
 }
 
+// ---- rounds with a sketched error at ranks 9 to 32: host side ----
+// The last launch's tiles and workgroups (conef_psgd_mfma_residual.h).  Tiles of four rows at least where they fit: four
+// are what a step of the matrix cores forms, and every tile reads all of Q, RP / rows floats an element of M.  As many
+// threads as leave sixteen waves a CU (128 registers) with as many tiles as its LDS holds or the launch has.  Rank 32,
+// sketches of a tenth, us:
+//   rows of a tile, threads        (as the row lists of the lower ranks)    (as taken)
+//   [1024,4096] 2 x [1024,1024]    2, 8   256   29.1                       4, 8   512   21.4
+//   2 x [2048,2048]                4      256   31.8                       8      512   22.9
+//   [640,5760] [640,2880]          1, 2   256   53.7                       4, 8  1024   20.4
+//   [300,9000]                     1      256   48.5                       2     1024   23.5
+//   [4096,5000]                    1      256  147                         4     1024   63.1
+//   [4096,1024] 2 x [1024,1024]    8      256   19.3  (4 rows 24.6)        the same
+//   [30522,1024]                   8      256   64.9  (16 rows 73.4)       the same
+//   2 x [1024,1024]                8      256   12.1                       8      512   10.3
+// Shorter tiles only where a launch has hardly any: 2 x [256,1024] + [1024,256] 8, 16 rows 9.3, 4, 8 rows 8.1.  Not where
+// most of a bucket would go by one or two rows: rounds of [1000,20000] at rank 32 with dense residuals 257, without 317,
+// [400,8000] 115 and 118, [100,20000] 126 and 141 (three rows: [640,9000] 197 and 171).
+struct WideTiles {
+    std::vector<ConefRowlistShape> shapes;
+    size_t lds;
+    int threads;
+};
+
+inline bool wide_sketch_tiles(const ConefPsgdItem* items, int count, WideTiles* wt)
+{
+    if (count < 1 || count > kPsgdBatchMax || rank_bound(items[0].r) < 16) return false;
+    std::vector<int64_t> rows;
+    for (int k = 0; k < count; ++k) {
+        const ConefPsgdItem& it = items[k];
+        if (!it.plan_host || it.r != items[0].r || it.m < 4 || it.m > kConefRowlistMaxCols || it.n > 0x7fffffffLL || it.w < 1 ||
+            it.w > 0xffff)
+            return false;
+        int64_t rb = it.m <= 1024 ? std::min<int64_t>(16, 8192 / it.m) : it.m <= 2048 ? 8 : 4;
+        while (rb > 1 && conef_rowlist_lds_compact((int)rb, it.m, it.w) > kConefRowlistLdsLimit) --rb;
+        if (conef_rowlist_lds_compact((int)rb, it.m, it.w) > kConefRowlistLdsLimit) return false;
+        rows.push_back(std::min<int64_t>(rb, it.n));
+    }
+    auto measure = [&] {
+        int64_t tiles = 0;
+        wt->lds = 0;
+        for (int k = 0; k < count; ++k) {
+            const int64_t rb = rows[(size_t)k];
+            tiles += (items[k].n + rb - 1) / rb;
+            wt->lds = std::max(wt->lds, conef_rowlist_lds_compact((int)rb, items[k].m, items[k].w));
+        }
+        return tiles;
+    };
+    int64_t tiles = measure();
+    for (int64_t least = 4; least >= 1; least -= 3) {
+        bool shorter = true;
+        while (shorter && tiles < (least > 1 ? 192 : 128)) {
+            shorter = false;
+            for (int64_t& rb : rows)
+                if (rb > least) {
+                    rb = std::max(least, (rb + 1) / 2);
+                    shorter = true;
+                }
+            tiles = measure();
+        }
+    }
+    if (wt->lds > kConefRowlistLdsLimit / 2) wt->threads = 1024;
+    else if (wt->lds > kConefRowlistLdsLimit / 4) wt->threads = tiles <= 256 ? 1024 : 512;
+    else wt->threads = tiles <= 512 ? 512 : 256;
+    double values = 0., low = 0.;
+    for (int k = 0; k < count; ++k) {
+        ConefRowlistShape s = {};
+        s.rb = (int)rows[(size_t)k];
+        s.tiles = (items[k].n + s.rb - 1) / s.rb;
+        wt->shapes.push_back(s);
+        values += (double)items[k].n * (double)items[k].m;
+        if (s.rb < 3) low += (double)items[k].n * (double)items[k].m;
+    }
+    return tiles <= 0x7fffffffLL && 2. * low <= values;
+}
+
+inline bool wide_sketch_plans(const ConefPsgdItem* items, int count, int32_t a, int32_t b)
+{
+    for (int k = 0; k < count; ++k) {
+        const ConefPlanHeader* hp = (const ConefPlanHeader*)items[k].plan_host;
+        if (!items[k].cs || !items[k].plan_dev || !conef_plan_matches(hp, items[k].n, items[k].m, items[k].w, a, b) ||
+            hp->kind != kConefPlanRowlist)
+            return false;
+    }
+    return true;
+}
+
+// Behind the deferred round's part of the workspace: the new Q factors by pieces.
+inline int64_t wide_sketch_bytes(const ConefPsgdItem* items, int count)
+{
+    WideTiles tiles;
+    if (!wide_sketch_tiles(items, count, &tiles)) return 0;
+    int64_t bytes = 0;
+    for (int k = 0; k < count; ++k) bytes += conef_align256(4 * items[k].m * rank_bound(items[k].r));
+    return bytes;
+}
+
+bool wide_sketch_round(const ConefPsgdItem* items, int count, int32_t a, int32_t b, void* workspace, int64_t workspace_bytes,
+                       PaddedRound* pr, WideTiles* tiles)
+{
+    if (!wide_sketch_tiles(items, count, tiles) || !wide_sketch_plans(items, count, a, b) ||
+        workspace_bytes < pr->bytes + wide_sketch_bytes(items, count))
+        return false;
+    char* at = (char*)workspace + pr->bytes;
+    for (int k = 0; k < count; ++k) {
+        pr->qi.push_back((float*)at);
+        at += conef_align256(4 * items[k].m * pr->rp);
+    }
+    return true;
+}
+
+template <int RP, int T>
+int wide_sketch_residual(const PaddedRound& pr, const WideTiles& tiles, float beta, hipStream_t s)
+{
+    std::vector<MfmaResidualItem<RP, T>> table;
+    std::vector<int> blocks;
+    for (size_t k = 0; k < pr.items.size(); ++k) {
+        const ConefPsgdItem& it = pr.items[k];
+        table.push_back(MfmaResidualItem<RP, T>{{it.x, it.p, pr.qi[k]},
+                                                conef_rowlist_view((const ConefPlanHeader*)it.plan_host, it.plan_dev),
+                                                it.cs, it.cs, it.n, (int)it.m, it.w, tiles.shapes[k].rb});
+        blocks.push_back((int)tiles.shapes[k].tiles);
+    }
+    auto kern = psgd_mfma_residual_batch_kernel<RP, T>;
+    if (hipError_t e = conef_allow_lds((const void*)kern, tiles.lds); e != hipSuccess) return (int)e;
+    const double omb = 1. - (double)beta;
+    return run_batches(table, blocks, [&](const PsgdBatch<MfmaResidualItem<RP, T>>& bt, int grid) {
+        conef_launch(kern, dim3((unsigned)grid), dim3(T), tiles.lds, s, bt, omb);
+    });
+}
+
+template <int RP>
+int wide_sketch_residual(const PaddedRound& pr, const WideTiles& tiles, float beta, hipStream_t s)
+{
+    switch (tiles.threads) {
+        case 256: return wide_sketch_residual<RP, 256>(pr, tiles, beta, s);
+        case 512: return wide_sketch_residual<RP, 512>(pr, tiles, beta, s);
+        default: return wide_sketch_residual<RP, 1024>(pr, tiles, beta, s);
+    }
+}
+
 // CONEF_ROUND_DEFER=0 asks for the reference's order of steps (read on every call and every replay: it may be switched
 // while a program runs).
 bool order_asked()
@@ -4311,7 +4464,7 @@ int64_t conef_psgd_batch_workspace_bytes(const ConefPsgdItem* items, int32_t cou
     }
     int64_t launches = conef_align256(single) + conef_align256(4 * mtp_batch_layout(items, count, nullptr)) +
                        conef_align256(4 * mfma_batch_layout(items, count, nullptr));
-    const int64_t padded = padded_round_bytes(items, count) + linear_round_bytes(items, count);
+    const int64_t padded = padded_round_bytes(items, count) + linear_round_bytes(items, count) + wide_sketch_bytes(items, count);
     if (padded > launches) launches = padded;
     const int64_t small = conef_psgd_round_small_workspace_bytes(items, count);      // the one-launch round's records
     return small > launches ? small : launches;
@@ -4455,6 +4608,9 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
                         linear_round(items, count, a, b, workspace, workspace_bytes, pr, &lr);
     if (!linear) pr = PaddedRound();
     const bool deferred = linear || round_defers(items, count, mq_mode, workspace, workspace_bytes, &pr);
+    // Above rank 8 the residual is sketched by the last launch of a deferred round
+    WideTiles tiles;
+    const bool wide_sketch = deferred && rp > 8 && pqt_mode == 2 && wide_sketch_round(items, count, a, b, workspace, workspace_bytes, &pr, &tiles);
     const ConefPsgdItem* its = deferred ? pr.items.data() : items;       // whose factors the rest of the round reads
     int rc = CONEF_OK;
     if (deferred) {
@@ -4547,8 +4703,11 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
         }
     }
     bool used = false;
-    rc = pqt_batch(its, count, pqt_mode == 3 ? 1 : pqt_mode, pqt_mode == 2 ? beta : 0.f, a, b, hs,
-                   ahead.count ? &ahead : nullptr, &used, deferred && rp <= 8 ? &pr.qi : nullptr);
+    if (wide_sketch)
+        rc = rp == 16 ? wide_sketch_residual<16>(pr, tiles, beta, hs) : wide_sketch_residual<32>(pr, tiles, beta, hs);
+    else
+        rc = pqt_batch(its, count, pqt_mode == 3 ? 1 : pqt_mode, pqt_mode == 2 ? beta : 0.f, a, b, hs,
+                       ahead.count ? &ahead : nullptr, &used, deferred && rp <= 8 ? &pr.qi : nullptr);
     if (rc != CONEF_OK) return rc;
     if (want_next && deferred && rp > 8) {
         if (gs_wide_by_columns(pr)) {
@@ -4590,6 +4749,16 @@ int conef_psgd_q_next_f32(const ConefPsgdItem* items, int32_t count, float eps, 
                  : orthogonalise_by_gram_wide(pr, items[0].r, src, q_next, eps, workspace, s);
     if (rc == CONEF_OK) *made = 1;
     return rc;
+}
+
+// Whether a round with a sketched error at ranks 9 to 32 sketches the residuals in its last launch (pqt_mode 2).
+int conef_psgd_round_wide_sketch_fits(const ConefPsgdItem* items, int32_t count, int32_t a, int32_t b)
+{
+    if (count < 1 || !items || order_asked()) return 0;
+    for (int k = 0; k < count; ++k)
+        if (!item_ok(items[k])) return 0;
+    WideTiles tiles;
+    return wide_sketch_tiles(items, count, &tiles) && wide_sketch_plans(items, count, a, b) ? 1 : 0;
 }
 
 // Whether conef_psgd_round_small_f32 takes this bucket: at most 24 matrices of at most 73728 elements

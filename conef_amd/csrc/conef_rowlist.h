@@ -20,6 +20,7 @@
 #pragma once
 #include "conef_device.h"
 #include "conef_sketch_core.h"
+#include <type_traits>
 
 constexpr int kConefRowlistThreads = 256;
 constexpr int64_t kConefRowlistMaxCols = 24576;       // 4 B value + 2 B list entry per column in LDS
@@ -50,6 +51,13 @@ inline size_t conef_rowlist_lds(int rb, int64_t d, int32_t w, bool cells)
     size_t ord = (((size_t)w + 7) & ~(size_t)7) * 2;
     (void)cells;      // every front parks the tile's old sketch rows in LDS
     return vals + ent + csr + ord + (size_t)rb * w * 4;
+}
+
+// A front with kCompact has the offsets in 16 bits and nothing between the tables.
+inline size_t conef_rowlist_lds_compact(int rb, int64_t d, int32_t w)
+{
+    const size_t vals = (((size_t)rb * d + 3) & ~(size_t)3) * 4, ent = (((size_t)d + 7) & ~(size_t)7) * 2;
+    return vals + ent + (((size_t)2 * w + 1 + 1) & ~(size_t)1) * 2 + (size_t)rb * w * 4;
 }
 
 // Rows per tile: about 32 KB of values (several tiles per CU), but no more than leaves a
@@ -95,7 +103,7 @@ inline bool conef_rowlist_shape(int64_t n, int64_t d, int32_t w, bool cells, boo
 struct ConefListVec {
     const float* vec;
     bool vec_ok;           // base 16-byte aligned and d % 4 == 0 (the tile copy works either way)
-    static constexpr bool kNeedsCells = false, kParksCells = false;
+    static constexpr bool kNeedsCells = false, kParksCells = false, kCompact = false;
     static constexpr int kThreads = kConefRowlistThreads;
     // whether a tensor with tiles to spare goes by half-height ones.  Full against half height: [50000,512] 40.2
     // and 29.9 us, [20000,2048] 49.0 and 45.9, [30522,1024] 37.0 and 36.2, [33278,650] 26.2 and 26.0, [60000,300]
@@ -157,7 +165,7 @@ struct ConefListRandBlock {
     float* payload;
     ConefBlock blk;
     float alpha;
-    static constexpr bool kNeedsCells = true, kParksCells = false;
+    static constexpr bool kNeedsCells = true, kParksCells = false, kCompact = false;
     static constexpr int kThreads = kConefRowlistThreads;
     static bool halves(int64_t) { return true; }      // (the column table sits in LDS next to the tiles)
     static constexpr int kQuads = 4;
@@ -342,9 +350,11 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
     extern __shared__ float conef_rl[];
     float* vals = conef_rl;
     uint16_t* ent_l = reinterpret_cast<uint16_t*>(vals + ((rb * d + 3) & ~3));
-    uint32_t* csr_l = reinterpret_cast<uint32_t*>(ent_l + ((d + 7) & ~7));
-    uint16_t* ord_l = reinterpret_cast<uint16_t*>(csr_l + ((w + 1 + 3) & ~3));
-    float* cells = reinterpret_cast<float*>(ord_l + ((w + 7) & ~7));
+    constexpr bool compact = Front::kCompact;
+    using Offset = std::conditional_t<compact, uint16_t, uint32_t>;
+    Offset* csr_l = reinterpret_cast<Offset*>(ent_l + ((d + 7) & ~7));
+    uint16_t* ord_l = reinterpret_cast<uint16_t*>(csr_l + (compact ? w + 1 : (w + 1 + 3) & ~3));
+    float* cells = reinterpret_cast<float*>(compact ? ent_l + ((d + 7) & ~7) + ((2 * w + 1 + 1) & ~1) : ord_l + ((w + 7) & ~7));
     const int64_t row0 = (int64_t)bx * rb;
     const int rows = n - row0 < rb ? (int)(n - row0) : rb;
 
@@ -425,19 +435,28 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
 #pragma unroll
         for (int u = 0; u < kPreC; ++u) {
             const int i = threadIdx.x + u * T;
-            if (i < csr_words) csr_l[i] = csr_pre[u];
+            if (i < csr_words) csr_l[i] = (Offset)csr_pre[u];
         }
-        uint32_t* ord_w = reinterpret_cast<uint32_t*>(ord_l);
-        if ((int)threadIdx.x < ord_words) ord_w[threadIdx.x] = ord_pre;
-        if (ord_words > T)
-            conef_copy_words_to_lds<T>(ord_w + T, ord_src + T,
-                                    ord_words - T);
+        if constexpr (compact) {
+            for (int i = threadIdx.x; i < ord_words; i += T) {
+                const uint32_t two = i == (int)threadIdx.x ? ord_pre : ord_src[i];
+                ord_l[2 * i] = (uint16_t)two;
+                if (2 * i + 1 < w) ord_l[2 * i + 1] = (uint16_t)(two >> 16);
+            }
+            for (int i = threadIdx.x + kPreC * T; i < csr_words; i += T) csr_l[i] = (Offset)plan.csr[i];
+        } else {
+            uint32_t* ord_w = reinterpret_cast<uint32_t*>(ord_l);
+            if ((int)threadIdx.x < ord_words) ord_w[threadIdx.x] = ord_pre;
+            if (ord_words > T)
+                conef_copy_words_to_lds<T>(ord_w + T, ord_src + T,
+                                        ord_words - T);
+            if (csr_words > kPreC * T)
+                conef_copy_words_to_lds<T>(csr_l + kPreC * T, plan.csr + kPreC * T,
+                                        csr_words - kPreC * T);
+        }
         if (ent_words > kPreE * T)
             conef_copy_words_to_lds<T>(ent_w + kPreE * T, ent_src + kPreE * T,
                                     ent_words - kPreE * T);
-        if (csr_words > kPreC * T)
-            conef_copy_words_to_lds<T>(csr_l + kPreC * T, plan.csr + kPreC * T,
-                                    csr_words - kPreC * T);
     }
     if constexpr (!Front::kNeedsCells && !Front::kParksCells) {
 #pragma unroll

@@ -372,6 +372,12 @@ int conef_psgd_round_small_f32(const ConefPsgdItem* items, int32_t count, int32_
                                float beta, float eps, int32_t a, int32_t b, void* workspace, int64_t workspace_bytes,
                                void* stream);
 
+/* Whether a round with a sketched error (mq_mode 2) at ranks 9 to 32 is to be asked for with pqt_mode 2: 1 where the
+ * residuals of these matrices are sketched by the launch that forms them (at most 24 matrices of one rank, rows of four
+ * columns or more, a row-list plan per sketch for the seeds a and b, no CONEF_ROUND_DEFER=0), 0 where pqt_mode 3 with room for dense residuals is the
+ * faster call.  conef_psgd_batch_workspace_bytes covers what it needs. */
+int conef_psgd_round_wide_sketch_fits(const ConefPsgdItem* items, int32_t count, int32_t a, int32_t b);
+
 /* The middle of that round as a call of its own, for a caller that splits the round: P = X Q with the Q
  * factors of `first` (a copy of `items` whose q may point elsewhere; null: items' own), P orthogonalised
  * (powerSGD_hook.py:516-531), Q = X^T P into items[k].q.  Deferred orthogonalisation of P where the batch
