@@ -73,6 +73,14 @@ __device__ __forceinline__ void conef_to_lds4(const void* src, void* lds)
 
 __device__ __forceinline__ void conef_wait_lds() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// Workgroup `id` of `total` in an order that gives an XCD neighbours: consecutive workgroups of a launch go round the
+// eight XCDs, the ones that land on one XCD here are a run of the order.
+__device__ __forceinline__ int conef_xcd_order(int id, int total)
+{
+    const int x = id & 7, per = total >> 3, more = total & 7;
+    return x * per + (x < more ? x : more) + (id >> 3);
+}
+
 // Rows cut into column quads when their length is not a multiple of four: the last quad is moved
 // back to end with the row, so that it stays inside, and its first `dup` columns are the previous
 // quad's.  Whoever owns it ignores them (they are never stored and never counted).

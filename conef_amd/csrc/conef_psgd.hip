@@ -27,6 +27,7 @@
 #include "conef_psgd_stream.h"
 #include "conef_psgd_small.h"
 #include "conef_psgd_linear.h"
+#include "conef_psgd_look.h"
 #include "conef_psgd_mfma_residual.h"
 #include "conef_hip.h"      // ConefPsgdItem, and a check of this file's definitions against the public header
 
@@ -84,6 +85,27 @@ __device__ __forceinline__ int psgd_batch_locate(const PsgdBatch<Item>& b, int* 
 {
     const int i = psgd_batch_item(b, (int)blockIdx.x);
     *local = (int)blockIdx.x - b.first[i];
+    return i;
+}
+
+// The same with an item's workgroups in an order that gives an XCD neighbouring tiles (column splits of one row tile,
+// column tiles of one slab), in launches of two workgroups a CU or more: rows of Q, of P or of a sketch's cells that
+// neighbours share come out of the XCD's L2.  For the products on the matrix cores, us in grid order and so, rank 32:
+// P = X Q of [4096,1024] + 2 x [1024,1024] 10.8 and 9.2, of [30522,1024] 37.3 and 31.9; Q = X^T P 12.1 and 11.1, 36.0 and
+// 34.0, with X formed from the cells 17.9 and 13.3, 50.2 and 44.8.  (The streaming products of the lower ranks, the dense and the
+// row-list residuals measured the same either way or up to 5 % slower.)
+template <typename Item>
+__device__ __forceinline__ int psgd_batch_near(const PsgdBatch<Item>& b, int i, int bx)
+{
+    const int local = bx - b.first[i];
+    return b.first[b.count] >= 512 ? conef_xcd_order(local, b.first[i + 1] - b.first[i]) : local;
+}
+
+template <typename Item>
+__device__ __forceinline__ int psgd_batch_locate_near(const PsgdBatch<Item>& b, int* local)
+{
+    const int i = psgd_batch_item(b, (int)blockIdx.x);
+    *local = psgd_batch_near(b, i, (int)blockIdx.x);
     return i;
 }
 
@@ -944,7 +966,7 @@ struct MfmaMqItem {
     const float* q;
     float* out;
     int64_t n;
-    int m, r, cols_per_split, row_tiles;
+    int m, r, cols_per_split, splits;
     ConefMod mod;       // of width 1: the batched kernel never unsketches
 };
 
@@ -954,10 +976,31 @@ psgd_mfma_mq_batch_kernel(PsgdBatch<MfmaMqItem> b)
 {
     static_assert(MODE == 0 || MODE == 1, "the sketch query of a batch runs as a launch of its own");
     int local;
-    const MfmaMqItem& it = b.item[psgd_batch_locate(b, &local)];
+    const MfmaMqItem& it = b.item[psgd_batch_locate_near(b, &local)];
     const ConefSeeds hs = {0, 0, 0, 0};
     psgd_mfma_mq_body<MODE, EXACT>(it.x, it.err, nullptr, nullptr, it.q, it.out, it.n, it.m, it.r, it.cols_per_split, it.mod, 0.f,
-                            hs, local % it.row_tiles, local / it.row_tiles);
+                            hs, local / it.splits, local % it.splits);
+}
+
+struct LookMqItem {
+    const float* x;
+    const float* cs;
+    const uint32_t* pk;
+    const float* q;
+    float* out;
+    int64_t n;
+    int m, r, w, cols_per_split, splits;
+};
+
+template <bool EXACT, int G>
+__global__ void __launch_bounds__(G * kMfmaThreads)
+psgd_mfma_look_mq_batch_kernel(PsgdBatch<LookMqItem> b, float alpha)
+{
+    int local;
+    const LookMqItem& it = b.item[psgd_batch_locate_near(b, &local)];
+    const int wgs = (it.splits + G - 1) / G;            // to a row tile
+    psgd_mfma_look_mq_body<EXACT, G>(it.x, it.cs, it.pk, it.q, it.out, it.n, it.m, it.r, it.w, it.cols_per_split, it.splits, alpha,
+                                     local / wgs, local % wgs);
 }
 
 struct MfmaMtpItem {
@@ -969,12 +1012,16 @@ struct MfmaMtpItem {
     int v;              // floats a lane loads at a time (4, 2, 1): read by the launch that takes every width
 };
 
+struct MfmaLookMtpItem : MfmaMtpItem {
+    MfmaLook look;
+};
+
 template <int V>
 __global__ void __launch_bounds__(kMfmaThreads)
 psgd_mfma_mtp_batch_kernel(PsgdBatch<MfmaMtpItem> b)
 {
     int local;
-    const MfmaMtpItem& it = b.item[psgd_batch_locate(b, &local)];
+    const MfmaMtpItem& it = b.item[psgd_batch_locate_near(b, &local)];
     psgd_mfma_mtp_body<V>(it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, local % it.col_tiles, local / it.col_tiles);
 }
 
@@ -982,9 +1029,9 @@ psgd_mfma_mtp_batch_kernel(PsgdBatch<MfmaMtpItem> b)
 // orthogonalisation of P at ranks 16 and 32), and one launch for the matrices of every vector
 // width: the solving workgroups outlast the products of one width, and a launch per width would
 // each wait for its slowest workgroup
-template <int RP>
+template <int RP, typename Item>
 __global__ void __launch_bounds__(kMfmaThreads)
-psgd_mfma_mtp_gram_batch_kernel(PsgdBatch<MfmaMtpItem> b, GramTask g)
+psgd_mfma_mtp_gram_batch_kernel(PsgdBatch<Item> b, GramTask g)
 {
     if ((int)blockIdx.x < g.count) {
         gram_solve_body<RP, kMfmaThreads, true>(g.parts[blockIdx.x], g.nparts[blockIdx.x], g.tmat[blockIdx.x], g.eps);
@@ -992,12 +1039,15 @@ psgd_mfma_mtp_gram_batch_kernel(PsgdBatch<MfmaMtpItem> b, GramTask g)
     }
     const int bx = (int)blockIdx.x - g.count;
     const int i = psgd_batch_item(b, bx);
-    const MfmaMtpItem& it = b.item[i];
-    const int local = bx - b.first[i];
+    const Item& it = b.item[i];
+    const int local = psgd_batch_near(b, i, bx);
     const int ct = local % it.col_tiles, slab = local / it.col_tiles;
-    if (it.v == 4) psgd_mfma_mtp_body<4>(it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, ct, slab);
-    else if (it.v == 2) psgd_mfma_mtp_body<2>(it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, ct, slab);
-    else psgd_mfma_mtp_body<1>(it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, ct, slab);
+    constexpr bool LOOK = std::is_same<Item, MfmaLookMtpItem>::value;
+    MfmaLook look = {};
+    if constexpr (LOOK) look = it.look;
+    if (it.v == 4) psgd_mfma_mtp_body<4, LOOK>(it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, ct, slab, look);
+    else if (it.v == 2) psgd_mfma_mtp_body<2, LOOK>(it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, ct, slab, look);
+    else psgd_mfma_mtp_body<1, LOOK>(it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, ct, slab, look);
 }
 
 // the Gram systems alone (ranks 9 to 32): a workgroup a matrix
@@ -2910,7 +2960,7 @@ int mq_batch(const ConefPsgdItem* items, int count, float alpha, int32_t a, int3
                     qblocks.push_back((int)(col_blocks * ((it.n + rpb - 1) / rpb)));
                 }
                 MfmaMqItem t = {it.x, MODE == 1 ? it.err : nullptr, it.q, out, it.n, (int)it.m, it.r, g.cols_per_split,
-                                g.row_tiles, conef_make_mod(1)};
+                                g.splits, conef_make_mod(1)};
                 table.push_back(t);
                 blocks.push_back(g.row_tiles * g.splits);
                 if (g.splits > 1) {
@@ -3041,7 +3091,7 @@ struct MtpRaw {
 };
 
 int mtp_batch(const ConefPsgdItem* items, int count, void* workspace, int64_t workspace_bytes, hipStream_t s,
-              const GramTask* gram = nullptr, std::vector<MtpRaw>* outs = nullptr)
+              const GramTask* gram = nullptr, std::vector<MtpRaw>* outs = nullptr, const std::vector<MfmaLook>* look = nullptr)
 {
     std::vector<MtpPlan> plans;
     const int64_t floats = mtp_batch_layout(items, count, &plans);
@@ -3064,6 +3114,7 @@ int mtp_batch(const ConefPsgdItem* items, int count, void* workspace, int64_t wo
     for (int pass = 0; pass < (gram ? 1 : 3) && mfma_partials; ++pass) {
         const int v = gram ? 0 : 4 >> pass;
         std::vector<MfmaMtpItem> table;
+        std::vector<MfmaLookMtpItem> look_table;
         std::vector<int> blocks;
         for (int k = 0; k < count; ++k) {
             const ConefPsgdItem& it = items[k];
@@ -3074,6 +3125,7 @@ int mtp_batch(const ConefPsgdItem* items, int count, void* workspace, int64_t wo
             float* out = t.slabs > 1 ? mfma_partials + mfma_offs[(size_t)k] : it.q;
             MfmaMtpItem mi = {it.x, it.p, out, it.n, (int)it.m, it.r, t.rows_per_slab, t.col_tiles, t.v};
             table.push_back(mi);
+            if (look) look_table.push_back(MfmaLookMtpItem{mi, (*look)[(size_t)k]});
             blocks.push_back(t.col_tiles * t.slabs);
             if (outs) (*outs)[(size_t)k] = MtpRaw{out, t.slabs > 1 ? t.slabs : 1};
             if (t.slabs > 1 && !gram) {
@@ -3090,11 +3142,13 @@ int mtp_batch(const ConefPsgdItem* items, int count, void* workspace, int64_t wo
             if (riders_done) return CONEF_ERR_INVALID;
             riders_done = true;
             const int rp = rank_bound(items[0].r);
-            int rc = run_batches(table, blocks, [&](const PsgdBatch<MfmaMtpItem>& bt, int grid) {
+            auto go = [&](const auto& bt, int grid) {
+                using Item = std::decay_t<decltype(bt.item[0])>;
                 const dim3 g3((unsigned)(grid + gram->count)), b3(kMfmaThreads);
-                if (rp == 32) conef_launch(psgd_mfma_mtp_gram_batch_kernel<32>, g3, b3, 0, s, bt, *gram);
-                else conef_launch(psgd_mfma_mtp_gram_batch_kernel<16>, g3, b3, 0, s, bt, *gram);
-            });
+                if (rp == 32) conef_launch(psgd_mfma_mtp_gram_batch_kernel<32, Item>, g3, b3, 0, s, bt, *gram);
+                else conef_launch(psgd_mfma_mtp_gram_batch_kernel<16, Item>, g3, b3, 0, s, bt, *gram);
+            };
+            const int rc = look ? run_batches(look_table, blocks, go) : run_batches(table, blocks, go);
             if (rc != CONEF_OK) return rc;
             continue;
         }
@@ -3429,14 +3483,19 @@ int round_products_deferred(const PaddedRound& pr, int r, float* const* q_in, fl
 // The same for ranks 9 to 32, whose products run on the matrix cores: the shares of P^T P come
 // from a short launch of their own over the finished P, the systems ride in the second product's
 // first launch, and the fix launch is the wide form.  `mq_mode` as in conef_psgd_mq_batch_f32.
+// look: X = M + alpha * unsketch(cs) is formed where it is read, and M stays as it is.
+int look_mq(const std::vector<ConefPsgdItem>& items, float alpha, void* workspace, int64_t workspace_bytes, hipStream_t s);
+
 int round_products_deferred_mfma(const PaddedRound& pr, int r, float* const* q_in, int mq_mode, float alpha, float eps,
-                                 int32_t a, int32_t b, void* workspace, int64_t workspace_bytes, hipStream_t s)
+                                 int32_t a, int32_t b, void* workspace, int64_t workspace_bytes, hipStream_t s,
+                                 const std::vector<MfmaLook>* look = nullptr)
 {
     const ConefPsgdItem* items = pr.items.data();
     const int count = (int)pr.items.size(), rp = pr.rp;
     std::vector<ConefPsgdItem> first(pr.items);
     for (int k = 0; k < count; ++k) first[(size_t)k].q = q_in[k];
-    int rc = conef_psgd_mq_batch_f32(first.data(), count, mq_mode, alpha, a, b, workspace, workspace_bytes, (void*)s);
+    int rc = look ? look_mq(first, alpha, workspace, workspace_bytes, s)
+                  : conef_psgd_mq_batch_f32(first.data(), count, mq_mode, alpha, a, b, workspace, workspace_bytes, (void*)s);
     if (rc != CONEF_OK) return rc;
     std::vector<GramShareItem> shares;
     std::vector<int> share_blocks;
@@ -3464,17 +3523,17 @@ int round_products_deferred_mfma(const PaddedRound& pr, int r, float* const* q_i
     });
     if (rc != CONEF_OK) return rc;
     std::vector<MtpRaw> raw((size_t)count);
-    rc = mtp_batch(items, count, workspace, workspace_bytes, s, &gram, &raw);
+    rc = mtp_batch(items, count, workspace, workspace_bytes, s, &gram, &raw, look);
     if (rc != CONEF_OK) return rc;
     return defer_fix(pr, r, raw, tmats, nullptr, s);
 }
 
 // Either of the two by rank.
 int deferred_products(const PaddedRound& pr, int r, float* const* q_in, float* const* qi_in, int mq_mode, float alpha, float eps, int32_t a, int32_t b,
-                      void* workspace, int64_t workspace_bytes, hipStream_t s, GsAhead* q_shares)
+                      void* workspace, int64_t workspace_bytes, hipStream_t s, GsAhead* q_shares, const std::vector<MfmaLook>* look = nullptr)
 {
     if (pr.rp > 8)
-        return round_products_deferred_mfma(pr, r, q_in, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, s);
+        return round_products_deferred_mfma(pr, r, q_in, mq_mode, alpha, eps, a, b, workspace, workspace_bytes, s, look);
     if (mq_mode == 0)
         return round_products_deferred<0>(pr, r, q_in, qi_in, 0.f, eps, a, b, workspace, workspace_bytes, s, q_shares);
     if (mq_mode == 1)
@@ -3722,14 +3781,14 @@ psgd_lin_residual_batch_kernel(PsgdBatch<RowlistResidualItem<RP, true, true, T>>
 }
 
 // M = P Q^T at ranks 9 to 32 with the residuals sketched (conef_psgd_mfma_residual.h).
-template <int RP, int T>
+template <int RP, bool LOOK, int T>
 __global__ void __launch_bounds__(T, 4)
-psgd_mfma_residual_batch_kernel(PsgdBatch<MfmaResidualItem<RP, T>> b, double one_minus_beta)
+psgd_mfma_residual_batch_kernel(PsgdBatch<MfmaResidualItem<RP, LOOK, T>> b, double one_minus_beta)
 {
     int local;
-    const MfmaResidualItem<RP, T>& it = b.item[psgd_batch_locate(b, &local)];
-    conef_rowlist_body<float, ListMfmaResidual<RP, T>>(it.front, it.plan, it.cs_in, it.cs_out, it.n, it.d, it.w, it.rb,
-                                                       one_minus_beta, local);
+    const MfmaResidualItem<RP, LOOK, T>& it = b.item[psgd_batch_locate(b, &local)];
+    conef_rowlist_body<float, ListMfmaResidual<RP, LOOK, T>>(it.front, it.plan, it.cs_in, it.cs_out, it.n, it.d, it.w, it.rb,
+                                                             one_minus_beta, local);
 }
 
 // Rows a workgroup of the dense M = P Q^T takes: as many as leave the launch two thousand workgroups
@@ -4385,34 +4444,130 @@ bool wide_sketch_round(const ConefPsgdItem* items, int count, int32_t a, int32_t
     return true;
 }
 
-template <int RP, int T>
-int wide_sketch_residual(const PaddedRound& pr, const WideTiles& tiles, float beta, hipStream_t s)
+template <int RP, bool LOOK, int T>
+int wide_sketch_launch(const PaddedRound& pr, const WideTiles& tiles, const std::vector<MfmaLook>& look, float beta, hipStream_t s)
 {
-    std::vector<MfmaResidualItem<RP, T>> table;
+    using Item = MfmaResidualItem<RP, LOOK, T>;
+    std::vector<Item> table;
     std::vector<int> blocks;
     for (size_t k = 0; k < pr.items.size(); ++k) {
         const ConefPsgdItem& it = pr.items[k];
-        table.push_back(MfmaResidualItem<RP, T>{{it.x, it.p, pr.qi[k]},
-                                                conef_rowlist_view((const ConefPlanHeader*)it.plan_host, it.plan_dev),
-                                                it.cs, it.cs, it.n, (int)it.m, it.w, tiles.shapes[k].rb});
+        table.push_back(Item{{it.x, it.p, pr.qi[k], LOOK ? look[k] : MfmaLook{}},
+                             conef_rowlist_view((const ConefPlanHeader*)it.plan_host, it.plan_dev), it.cs, it.cs, it.n, (int)it.m, it.w,
+                             tiles.shapes[k].rb});
         blocks.push_back((int)tiles.shapes[k].tiles);
     }
-    auto kern = psgd_mfma_residual_batch_kernel<RP, T>;
+    auto kern = psgd_mfma_residual_batch_kernel<RP, LOOK, T>;
     if (hipError_t e = conef_allow_lds((const void*)kern, tiles.lds); e != hipSuccess) return (int)e;
     const double omb = 1. - (double)beta;
-    return run_batches(table, blocks, [&](const PsgdBatch<MfmaResidualItem<RP, T>>& bt, int grid) {
+    return run_batches(table, blocks, [&](const PsgdBatch<Item>& bt, int grid) {
         conef_launch(kern, dim3((unsigned)grid), dim3(T), tiles.lds, s, bt, omb);
     });
 }
 
 template <int RP>
-int wide_sketch_residual(const PaddedRound& pr, const WideTiles& tiles, float beta, hipStream_t s)
+int wide_sketch_residual(const PaddedRound& pr, const WideTiles& tiles, const std::vector<MfmaLook>& look, float beta, hipStream_t s)
 {
-    switch (tiles.threads) {
-        case 256: return wide_sketch_residual<RP, 256>(pr, tiles, beta, s);
-        case 512: return wide_sketch_residual<RP, 512>(pr, tiles, beta, s);
-        default: return wide_sketch_residual<RP, 1024>(pr, tiles, beta, s);
+    auto go = [&](auto looked) {
+        constexpr bool LOOK = decltype(looked)::value;
+        switch (tiles.threads) {
+            case 256: return wide_sketch_launch<RP, LOOK, 256>(pr, tiles, look, beta, s);
+            case 512: return wide_sketch_launch<RP, LOOK, 512>(pr, tiles, look, beta, s);
+            default: return wide_sketch_launch<RP, LOOK, 1024>(pr, tiles, look, beta, s);
+        }
+    };
+    return look.empty() ? go(std::false_type()) : go(std::true_type());
+}
+
+// The first product with X formed from the cells: two column splits of a row tile to a workgroup share its cells in LDS, four
+// where those are more than half a CU's.
+struct LookMqShape {
+    int groups;
+    size_t lds;
+};
+
+inline bool look_mq_shape(const ConefPsgdItem* items, int count, LookMqShape* g)
+{
+    int w = 1, splits = 1;
+    for (int k = 0; k < count; ++k) {
+        w = std::max(w, (int)items[k].w);
+        splits = std::max(splits, mfma_mq_shape(items[k].n, items[k].m).splits);
     }
+    const size_t cells = 32 * (size_t)look_cells_stride(w) * 4;
+    g->groups = cells > kConefRowlistLdsLimit / 2 ? 4 : splits > 1 ? 2 : 1;
+    g->lds = std::max(cells, (size_t)g->groups * kMfmaWaves * 16 * 64 * 4);
+    return g->lds <= kConefRowlistLdsLimit;
+}
+
+// Whether the products form X themselves.  It saves the query's launch, a read of M and a write of X; it costs the
+// cells: the second product reads a row of them for every 128 columns, so what counts is how wide they are, and the first and the
+// last read what the query read once more.  Steps with the query (an error laid out in M) and without, us:
+//   share of cells                 0.05           0.1            0.2            0.3            0.5
+//   a BERT encoder       rank 16   536  499       550  514       593  556       609  599       643  674
+//                        rank 32   630  603       640  616       676  656       696  694       729  762
+//   LSTM, 650 wide       rank 16   418  399       422  406       454  427       501  487       536  549
+//   [20000,512]          rank 16   104  100       105  101       106  105       109  109       112  115
+//   [1000,2000]          rank 16    76   74        77   76        77   78        77   82        77   86
+//   [4000,4096]          rank 16   147  144       149  148       161  170       169  184       182  181
+//   [640,9000]           rank 16    99  100        99  109
+//   WRN-16-2             rank 16    68   63        69   64        69   65        69   66        70   69
+// Up to 320 cells a row on average then, and a share of 0.35 where launches are more than latency.
+inline bool look_pays(const ConefPsgdItem* items, int count)
+{
+    double values = 0., cells = 0., widths = 0.;
+    for (int k = 0; k < count; ++k) {
+        const double n = (double)items[k].n, m = (double)items[k].m;
+        values += n * m;
+        cells += n * items[k].w;
+        widths += n * m * items[k].w;
+    }
+    LookMqShape g;
+    return widths <= 320. * values && (cells <= 0.35 * values || values <= 4e6) && look_mq_shape(items, count, &g);
+}
+
+int look_mq(const std::vector<ConefPsgdItem>& items, float alpha, void* workspace, int64_t workspace_bytes, hipStream_t s)
+{
+    const int count = (int)items.size();
+    std::vector<int64_t> offs;
+    float* partials = mfma_partial_base(items.data(), count, workspace, workspace_bytes, &offs);
+    LookMqShape shape;
+    if (!look_mq_shape(items.data(), count, &shape) || !partials) return CONEF_ERR_INVALID;
+    std::vector<LookMqItem> table;
+    std::vector<SumItem> sums;
+    std::vector<int> blocks, sum_blocks;
+    bool exact = true;
+    for (int k = 0; k < count; ++k) {
+        const ConefPsgdItem& it = items[(size_t)k];
+        const MfmaMqShape g = mfma_mq_shape(it.n, it.m);
+        float* out = g.splits > 1 ? partials + offs[(size_t)k] : it.p;
+        table.push_back(LookMqItem{it.x, it.cs, item_pktab(it), it.q, out, it.n, (int)it.m, it.r, it.w, g.cols_per_split, g.splits});
+        blocks.push_back(g.row_tiles * ((g.splits + shape.groups - 1) / shape.groups));
+        if (g.splits > 1) {
+            sums.push_back(SumItem{out, it.p, it.n * it.r, g.splits});
+            sum_blocks.push_back((int)((it.n * it.r + 255) / 256));
+        }
+        exact = exact && it.m % 4 == 0;
+    }
+    auto go = [&](auto exactly, auto groups) {
+        constexpr int G = decltype(groups)::value;
+        auto kern = psgd_mfma_look_mq_batch_kernel<decltype(exactly)::value, G>;
+        if (hipError_t e = conef_allow_lds((const void*)kern, shape.lds); e != hipSuccess) return (int)e;
+        return run_batches(table, blocks, [&](const PsgdBatch<LookMqItem>& bt, int grid) {
+            conef_launch(kern, dim3((unsigned)grid), dim3(G * kMfmaThreads), shape.lds, s, bt, alpha);
+        });
+    };
+    auto with = [&](auto exactly) {
+        switch (shape.groups) {
+            case 1: return go(exactly, std::integral_constant<int, 1>());
+            case 2: return go(exactly, std::integral_constant<int, 2>());
+            default: return go(exactly, std::integral_constant<int, 4>());
+        }
+    };
+    const int rc = exact ? with(std::true_type()) : with(std::false_type());
+    if (rc != CONEF_OK || sums.empty()) return rc;
+    return run_batches(sums, sum_blocks, [&](const PsgdBatch<SumItem>& bt, int grid) {
+        conef_launch(psgd_sum_partials_batch_kernel, dim3((unsigned)grid), dim3(256), 0, s, bt);
+    });
 }
 
 // CONEF_ROUND_DEFER=0 asks for the reference's order of steps (read on every call and every replay: it may be switched
@@ -4611,6 +4766,9 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
     // Above rank 8 the residual is sketched by the last launch of a deferred round
     WideTiles tiles;
     const bool wide_sketch = deferred && rp > 8 && pqt_mode == 2 && wide_sketch_round(items, count, a, b, workspace, workspace_bytes, &pr, &tiles);
+    std::vector<MfmaLook> look;
+    if (wide_sketch && mq_mode == 2 && look_pays(items, count))
+        for (int k = 0; k < count; ++k) look.push_back(MfmaLook{items[k].cs, item_pktab(items[k]), items[k].w, alpha});
     const ConefPsgdItem* its = deferred ? pr.items.data() : items;       // whose factors the rest of the round reads
     int rc = CONEF_OK;
     if (deferred) {
@@ -4659,7 +4817,7 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
             for (int k = 0; k < count; ++k) pr.qt[(size_t)k] = q_next[k];
         GsAhead* qs = want_next && rp <= 8 ? &ahead : nullptr;
         rc = deferred_products(pr, r, q_in.data(), quads_ready ? q_next + count : nullptr, mq_mode, alpha, eps, a, b, workspace,
-                               workspace_bytes, hs, qs);
+                               workspace_bytes, hs, qs, look.empty() ? nullptr : &look);
         if (rc != CONEF_OK) return rc;
     } else {
         std::vector<ConefPsgdItem> first(items, items + count);
@@ -4704,7 +4862,7 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
     }
     bool used = false;
     if (wide_sketch)
-        rc = rp == 16 ? wide_sketch_residual<16>(pr, tiles, beta, hs) : wide_sketch_residual<32>(pr, tiles, beta, hs);
+        rc = rp == 16 ? wide_sketch_residual<16>(pr, tiles, look, beta, hs) : wide_sketch_residual<32>(pr, tiles, look, beta, hs);
     else
         rc = pqt_batch(its, count, pqt_mode == 3 ? 1 : pqt_mode, pqt_mode == 2 ? beta : 0.f, a, b, hs,
                        ahead.count ? &ahead : nullptr, &used, deferred && rp <= 8 ? &pr.qi : nullptr);

@@ -169,10 +169,18 @@ psgd_mfma_mq_kernel(float* __restrict__ x, const float* __restrict__ err, const 
 // rows of the slab, meet in LDS, and the slab's tile is stored (one slab) or left as a partial.
 // Any alignment, any m >= V: the last run of V columns is moved back to end with the row (columns
 // two lanes then hold come out of both the same).
-template <int V>
+// LOOK: X = M + alpha * unsketch(cs), formed here (conef_psgd_look.h).
+struct MfmaLook {
+    const float* cs;         // [n, w]
+    const uint32_t* pk;      // bucket and sign of every column
+    int w;
+    float alpha;
+};
+
+template <int V, bool LOOK = false>
 __device__ __forceinline__ void
 psgd_mfma_mtp_body(const float* __restrict__ x, const float* __restrict__ p, float* __restrict__ out, int64_t n, int m,
-                   int r, int rows_per_slab, int bx, int by)
+                   int r, int rows_per_slab, int bx, int by, MfmaLook look = {})
 {
     __shared__ float red[kMfmaWaves][16][64];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -191,8 +199,13 @@ psgd_mfma_mtp_body(const float* __restrict__ x, const float* __restrict__ p, flo
         for (int v = 0; v < 16; ++v) acc[t][v] = 0.f;
     constexpr int U = V == 4 ? 4 : 8;                  // row pairs per stage
     struct Stage {
-        float xv[U][V], pv[U];
+        float xv[U][V], pv[U], cv[U][LOOK ? V : 1];
     };
+    uint32_t pk[V];
+    if constexpr (LOOK) {
+#pragma unroll
+        for (int t = 0; t < V; ++t) pk[t] = look.pk[cc + t];
+    }
     auto load = [&](Stage& st, int64_t ib) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -208,12 +221,20 @@ psgd_mfma_mtp_body(const float* __restrict__ x, const float* __restrict__ p, flo
                 st.xv[u][0] = *src;
             }
             st.pv[u] = p[ii * r + (rank_ok ? lq : 0)];
+            if constexpr (LOOK) {
+#pragma unroll
+                for (int t = 0; t < V; ++t) st.cv[u][t] = look.cs[ii * look.w + (pk[t] & 0x7fffffffu)];
+            }
         }
     };
     auto compute = [&](Stage& st, int64_t ib) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const bool ok = ib + 2 * u + half < i1;
+            if constexpr (LOOK) {
+#pragma unroll
+                for (int t = 0; t < V; ++t) st.xv[u][t] = __fadd_rn(st.xv[u][t], conef_query_term(st.cv[u][t], pk[t], look.alpha));
+            }
             const float b = (ok && rank_ok) ? st.pv[u] : 0.f;
 #pragma unroll
             for (int t = 0; t < V; ++t) acc[t] = conef_mfma32((ok && col_ok) ? st.xv[u][t] : 0.f, b, acc[t]);

@@ -43,16 +43,18 @@ __device__ __forceinline__ void conef_mfma_rows4(const float (*a)[RP / 16], cons
 // piece is one run of 1 KB (from the row-major factor 64 lines of 128 bytes).
 __host__ __device__ __forceinline__ int64_t conef_piece_at(int64_t m, int piece, int64_t col) { return (piece * m + col) * 4; }
 
-// Front of the row-list kernel (conef_rowlist.h).
-template <int RP, int T>
+// Front of the row-list kernel (conef_rowlist.h).  LOOK: M lies as the gradient came, and X is formed here
+// (conef_psgd_look.h); the tile's old cells go to their place in LDS first.
+template <int RP, bool LOOK, int T>
 struct ListMfmaResidual {
     float* x;
     const float* p;          // [n, RP]
     const float* qp;         // Q by pieces
-    static constexpr bool kNeedsCells = false, kParksCells = false, kCompact = true;
+    MfmaLook look;
+    static constexpr bool kNeedsCells = false, kParksCells = LOOK, kCompact = true;
     static constexpr int kThreads = T;
     struct Regs {};
-    __device__ __forceinline__ void stage(int64_t row0, int rows, int d, int, float* vals, float*, const uint32_t*) const
+    __device__ __forceinline__ void stage(int64_t row0, int rows, int d, int w, float* vals, float* cells, const uint32_t*) const
     {
         constexpr int H = RP / 16, W = T / 64;
         constexpr int kRows = 8, G = kRows / 4;            // rows of a column that are requested together
@@ -66,10 +68,12 @@ struct ListMfmaResidual {
         const int block0 = wave - part * bstep;
         int r = part < split ? kRows * part : rows, block = block0;
         float q[RP], qn[RP], xn[kRows], a[G][H], an[G][H];
+        uint32_t pkn = 0;
         auto request = [&](bool rows_too, float* qd) {     // what the unit (r, block) reads
             const int c = block * 64 + lane < d ? block * 64 + lane : d - 1;
 #pragma unroll
             for (int v = 0; v < RP / 4; ++v) conef_ld4u(qp + conef_piece_at(d, v, c), qd + 4 * v);
+            if constexpr (LOOK) pkn = look.pk[c];
             const float* src = base + (int64_t)r * d + c;
 #pragma unroll
             for (int u = 0; u < kRows; ++u)
@@ -86,11 +90,30 @@ struct ListMfmaResidual {
         };
         bool have = r < rows && block < blocks, fresh = true;
         if (have) request(true, qn);
+        if constexpr (LOOK) {                              // they travel together
+            const float* src = look.cs + row0 * w;
+            const int count = rows * w;
+            constexpr int kPark = 4;
+            for (int i0 = threadIdx.x; i0 < count; i0 += kPark * T) {
+                float t[kPark];
+#pragma unroll
+                for (int u = 0; u < kPark; ++u) t[u] = src[i0 + u * T < count ? i0 + u * T : count - 1];
+#pragma unroll
+                for (int u = 0; u < kPark; ++u)
+                    if (i0 + u * T < count) cells[i0 + u * T] = t[u];
+            }
+            __syncthreads();
+        }
         while (have) {
             const int cur = block, first = r;
             float xv[kRows];
 #pragma unroll
-            for (int u = 0; u < kRows; ++u) xv[u] = xn[u];
+            for (int u = 0; u < kRows; ++u) {
+                xv[u] = xn[u];
+                if constexpr (LOOK)
+                    if (first + u < rows)
+                        xv[u] = __fadd_rn(xv[u], conef_query_term(cells[(first + u) * w + (int)(pkn & 0x7fffffffu)], pkn, look.alpha));
+            }
 #pragma unroll
             for (int t = 0; t < RP; ++t) q[t] = qn[t];
             if (fresh) {
@@ -124,9 +147,9 @@ struct ListMfmaResidual {
     }
 };
 
-template <int RP, int T>
+template <int RP, bool LOOK, int T>
 struct MfmaResidualItem {
-    ListMfmaResidual<RP, T> front;
+    ListMfmaResidual<RP, LOOK, T> front;
     ConefRowlistView plan;
     const float* cs_in;
     float* cs_out;
