@@ -302,38 +302,41 @@ __device__ __forceinline__ void gsg_recurrence(double (*gram)[RP + 1], float (*c
 
 }
 
+// What a workgroup of the kernel keeps in LDS.
 template <int RP>
-__global__ void __launch_bounds__(kGsgThreads)
-gsg_kernel(GsgBatch batch, int count, float eps, GsgWs* ws, unsigned tag)
-{
-    constexpr int T = kGsgThreads, NW = T / 64;
-    constexpr int NC = RP >= 16 ? RP / 16 : 1;             // column groups of 16
-    constexpr int NT = NC * (NC + 1) / 2;                  // tiles of the upper triangle: 1 or 3
-    constexpr int NG = RP * (RP + 1) / 2;
-    __shared__ double tiles[NW][NT][256];                   // per-wave partial tiles, [i][j] row-major inside a tile
-    __shared__ double gram[RP][RP + 1];                     // upper triangle of the current Gram matrix
-    __shared__ __attribute__((aligned(16))) float coef[RP][RP];       // b_ij for i < j, rounded once for step 4
-    __shared__ double dinv[RP];                             // the pivots G_ii, then 1 / d_i
-    __shared__ double diag0[RP];                            // the least pivot each column may end up with
-    __shared__ float dinvf[RP];
-    __shared__ int failed;
+struct GsgLds {
+    static constexpr int NC = RP >= 16 ? RP / 16 : 1;      // column groups of 16
+    static constexpr int NT = NC * (NC + 1) / 2;           // tiles of the upper triangle: 1 or 3
+    double tiles[kGsgThreads / 64][NT][256];               // per-wave partial tiles, [i][j] row-major inside a tile
+    double gram[RP][RP + 1];                               // upper triangle of the current Gram matrix
+    double dinv[RP];                                       // the pivots G_ii, then 1 / d_i
+    double diag0[RP];                                      // the least pivot each column may end up with
+    alignas(16) float coef[RP][RP];                        // b_ij for i < j, rounded once for step 4
+    float dinvf[RP];
+    int failed;
+};
 
-    int it = 0;
-    while (it + 1 < count && (int)blockIdx.x >= batch.first[it + 1]) ++it;
-    const int wg0 = batch.first[it];
-    const int nwg = batch.first[it + 1] - wg0;
-    const int local = (int)blockIdx.x - wg0;
-    const int rows = batch.rows[it], slab = batch.slab[it];
+// Workgroup `local` of the nwg that take the [rows, RP] matrix src, slab rows each, into dst (which may be src).  Its records
+// are slots wg0 + local of ws.  T >= kGsgThreads threads, the first kGsgThreads of which form the share of G.
+// LEAN: in 128 registers (fewer requests in flight), for a kernel that also does something else.
+template <int RP, int T, bool LEAN = false>
+__device__ __forceinline__ void gsg_body(GsgLds<RP>& l, const float* src, float* dst, int rows, int slab, int wg0, int nwg, int local,
+                                         float eps, GsgWs* ws, unsigned tag)
+{
+    constexpr int NG = RP * (RP + 1) / 2;
+    auto& tiles = l.tiles;
+    auto& gram = l.gram;
+    auto& coef = l.coef;
+    float* dinvf = l.dinvf;
     const int r0 = local * slab;
     const int r1 = r0 + slab < rows ? r0 + slab : rows;
-    float* __restrict__ a = batch.a[it];
 
     const int tid = threadIdx.x;
-    if (tid == 0) failed = 0;
+    if (tid == 0) l.failed = 0;
     GSG_STAMP(0);
 
     // ---- 1. this workgroup's share of G on the matrix cores
-    gsg_gram_tiles<RP>(a, r0, r1, tiles);
+    if (T == kGsgThreads || tid < kGsgThreads) gsg_gram_tiles<RP>(src, r0, r1, tiles);
     __syncthreads();
     GSG_STAMP(1);
 
@@ -346,14 +349,14 @@ gsg_kernel(GsgBatch batch, int count, float eps, GsgWs* ws, unsigned tag)
             const unsigned long long bits = (unsigned long long)__double_as_longlong(s);
             const unsigned long long hi = ((unsigned long long)tag << 32) | (bits >> 32);
             const unsigned long long lo = ((unsigned long long)tag << 32) | (bits & 0xffffffffull);
-            __hip_atomic_store(&ws->slot[blockIdx.x][2 * e], hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&ws->slot[blockIdx.x][2 * e + 1], lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&ws->slot[wg0 + local][2 * e], hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&ws->slot[wg0 + local][2 * e + 1], lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {
             gram[i][j] = s;
         }
     }
     if (nwg > 1) {
-        constexpr int CH = 16;                              // workgroups whose records are requested together
+        constexpr int CH = LEAN ? 8 : 16;                   // workgroups whose records are requested together
         for (int e = tid; e < NG; e += T) {
             int i, j;
             gsg_entry(e, RP, &i, &j);
@@ -375,7 +378,7 @@ gsg_kernel(GsgBatch batch, int count, float eps, GsgWs* ws, unsigned tag)
                         if (spins > kGsgSpinLimit ||
                             ((spins & 255u) == 0 && __hip_atomic_load(&ws->gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == tag)) {
                             __hip_atomic_store(&ws->gave_up, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            failed = 1;
+                            l.failed = 1;
                             rec[u] = (unsigned long long)tag << 32;
                             break;
                         }
@@ -395,22 +398,23 @@ gsg_kernel(GsgBatch batch, int count, float eps, GsgWs* ws, unsigned tag)
     }
     __syncthreads();
     GSG_STAMP(2);
-    if (failed) {
+    if (l.failed) {
         if (tid == 0) gs_count_give_up();
         // a half-orthogonalised matrix would pass for a result: leave one that cannot
-        for (int e = tid; e < (r1 - r0) * RP; e += T) a[(int64_t)r0 * RP + e] = __builtin_nanf("");
+        for (int e = tid; e < (r1 - r0) * RP; e += T) dst[(int64_t)r0 * RP + e] = __builtin_nanf("");
         return;
     }
 
     // ---- 3. the r column steps on the r x r matrix
-    gsg_recurrence<RP, T>(gram, coef, dinv, dinvf, diag0, eps, tid);
+    gsg_recurrence<RP, T>(gram, coef, l.dinv, dinvf, l.diag0, eps, tid);
     GSG_STAMP(4);
 
     // ---- 4. the same steps on this workgroup's rows, a row per thread: the reference's column
     // operations in its own precision (fp32, one fused multiply-add per element and step), with
     // coefficients that were computed in double and rounded once
     for (int row = r0 + tid; row < r1; row += T) {
-        float* p = a + (int64_t)row * RP;
+        const float* p = src + (int64_t)row * RP;
+        float* to = dst + (int64_t)row * RP;
         float x[RP];
 #pragma unroll
         for (int c = 0; c < RP; c += 4) {
@@ -423,25 +427,37 @@ gsg_kernel(GsgBatch batch, int count, float eps, GsgWs* ws, unsigned tag)
         // One row of coefficients at a time, the next row requested before this row's multiply-adds
         // (without the fences the compiler requests all r (r - 1) / 2 up front and runs out of
         // registers at rank 32).
-        float cur[RP], nxt[RP];
+        float cur[RP], nxt[LEAN ? 1 : RP];
 #pragma unroll
         for (int k = 0; k < RP; ++k) cur[k] = coef[0][k];
 #pragma unroll
         for (int i = 0; i < RP; ++i) {
             asm volatile("" ::: "memory");
-            if (i + 1 < RP) {
+            if (!LEAN && i + 1 < RP) {
 #pragma unroll
-                for (int k = (i + 2) & ~3; k < RP; ++k) nxt[k] = coef[i + 1][k];      // whole 16-byte groups
+                for (int k = (i + 2) & ~3; k < RP; ++k) nxt[LEAN ? 0 : k] = coef[i + 1][k];      // whole 16-byte groups
             }
             asm volatile("" ::: "memory");
 #pragma unroll
             for (int k = i + 1; k < RP; ++k) x[k] = fmaf(-cur[k], x[i], x[k]);
             x[i] = __fmul_rn(x[i], dinvf[i]);
 #pragma unroll
-            for (int k = (i + 2) & ~3; k < RP; ++k) cur[k] = nxt[k];
+            for (int k = (i + 2) & ~3; k < RP; ++k) cur[k] = LEAN ? coef[i + 1 < RP ? i + 1 : i][k] : nxt[LEAN ? 0 : k];
         }
 #pragma unroll
-        for (int c = 0; c < RP; c += 4) *reinterpret_cast<float4*>(p + c) = make_float4(x[c], x[c + 1], x[c + 2], x[c + 3]);
+        for (int c = 0; c < RP; c += 4) *reinterpret_cast<float4*>(to + c) = make_float4(x[c], x[c + 1], x[c + 2], x[c + 3]);
     }
     GSG_STAMP(5);
+}
+
+template <int RP>
+__global__ void __launch_bounds__(kGsgThreads)
+gsg_kernel(GsgBatch batch, int count, float eps, GsgWs* ws, unsigned tag)
+{
+    __shared__ GsgLds<RP> l;
+    int it = 0;
+    while (it + 1 < count && (int)blockIdx.x >= batch.first[it + 1]) ++it;
+    const int wg0 = batch.first[it];
+    gsg_body<RP, kGsgThreads>(l, batch.a[it], batch.a[it], batch.rows[it], batch.slab[it], wg0, batch.first[it + 1] - wg0,
+                              (int)blockIdx.x - wg0, eps, ws, tag);
 }

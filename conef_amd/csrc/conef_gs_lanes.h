@@ -21,6 +21,7 @@
 // One exchange across workgroups per step (about 2 us) is what bounds this kernel, so the matrix
 // is spread thin: few rows a thread, many workgroups.
 #pragma once
+#include "conef_device.h"
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -342,34 +343,20 @@ __device__ __forceinline__ void gsw_store_columns(float* __restrict__ a, int row
     }
 }
 
-// Matrix batch.a[blockIdx.x]: [rows, RP] row-major, rows <= 64 RPT, in place.
-template <int RP, int RPT, int CW>
-__global__ void __launch_bounds__(64 * RP / CW)
-gsw_kernel(GswBatch batch, float eps)
+// The r column steps on columns in registers (v[cc][t]: row lane + 64 t of column w * CW + cc); piv: two pivot columns in LDS.
+// PRIO: the waves' priority when they come and go.
+template <int RP, int RPT, int CW, int PRIO = 0>
+__device__ __forceinline__ void gsw_steps(float (&v)[CW][RPT], float* piv, int lane, int w, float eps)
 {
     constexpr int PS = RPT + 4;      // a lane's slice of the pivot column: 16-byte accesses of 16 lanes then cover all banks once
-    extern __shared__ __attribute__((aligned(16))) float gsw_lds[];
-    float* piv = gsw_lds;                       // [2][64][PS]: the normalised pivot column, lane-major
-    float* tile = gsw_lds + 2 * 64 * PS;        // [TR][RP + 1]
-    float* __restrict__ a = batch.a[blockIdx.x];
-    const int rows = batch.rows[blockIdx.x];
-    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col0 = w * CW;
-
-    float v[CW][RPT];
-    gsw_load_columns<RP, RPT, CW>(a, rows, tile, v, tid, lane, col0);
-
     // Normalises this wave's column i and publishes it: a lane's slice of the column is RPT words,
     // written and read 16 bytes at a time.
     auto publish = [&](int i) __attribute__((always_inline)) {
         float* pb = piv + (i & 1) * (64 * PS) + lane * PS;
-        if constexpr (CW == 1) {
-            gsw_publish_column<RPT>(v[0], pb, eps);
-        } else {
-            static_assert(CW == 2, "columns per wave");
-            if (i % 2 == 0) gsw_publish_column<RPT>(v[0], pb, eps);
-            else gsw_publish_column<RPT>(v[1], pb, eps);
-        }
+#pragma unroll
+        for (int cc = 0; cc < CW; ++cc)
+            if (i % CW == cc) gsw_publish_column<RPT>(v[cc], pb, eps);
     };
 
     if (w == 0) publish(0);
@@ -419,9 +406,77 @@ gsw_kernel(GswBatch batch, float eps)
         }
         if (next_owner) {
             publish(i + 1);
-            __builtin_amdgcn_s_setprio(0);
+            __builtin_amdgcn_s_setprio(PRIO);
         }
         __syncthreads();
     }
+}
+
+// The same steps on a workgroup of T threads among others: the [rows, RP] matrix by pieces of four columns (qp:
+// conef_piece_at) into row-major dst.  A wave owns the columns that T threads leave it, loaded as they lie.  Needs
+// gsw_pieces_lds_floats<RPT>() floats.
+template <int RPT>
+constexpr int gsw_pieces_lds_floats() { return 2 * 64 * (RPT + 4); }
+
+template <int RP, int RPT, int T>
+__device__ __forceinline__ void gsw_pieces_body(const float* __restrict__ qp, float* __restrict__ dst, int rows, float* piv, float eps)
+{
+    constexpr int CW = 64 * RP / T;
+    static_assert(CW == 1 || CW == 2 || CW % 4 == 0, "columns of a wave lie in whole pieces or in one");
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), col0 = w * CW;
+    float v[CW][RPT];
+#pragma unroll
+    for (int t = 0; t < RPT; ++t) {
+        const int row = lane + 64 * t;
+        const float* src = qp + ((int64_t)(col0 >> 2) * rows + (row < rows ? row : rows - 1)) * 4 + (col0 & 3);
+        float x[CW];
+        if constexpr (CW % 4 == 0) {
+#pragma unroll
+            for (int c = 0; c < CW; c += 4) conef_ld4u(src + (int64_t)c * rows, x + c);
+        } else {
+#pragma unroll
+            for (int c = 0; c < CW; ++c) x[c] = src[c];
+        }
+#pragma unroll
+        for (int c = 0; c < CW; ++c) v[c][t] = row < rows ? x[c] : 0.f;
+    }
+    gsw_steps<RP, RPT, CW, 2>(v, piv, lane, w, eps);
+#pragma unroll
+    for (int t = 0; t < RPT; ++t) {
+        const int row = lane + 64 * t;
+        if (row < rows) {
+            float* to = dst + (int64_t)row * RP + col0;
+            if constexpr (CW % 4 == 0) {
+#pragma unroll
+                for (int c = 0; c < CW; c += 4) {
+                    const float x[4] = {v[c][t], v[c + 1][t], v[c + 2][t], v[c + 3][t]};
+                    conef_st4u(to + c, x);
+                }
+            } else {
+#pragma unroll
+                for (int c = 0; c < CW; ++c) to[c] = v[c][t];
+            }
+        }
+    }
+}
+
+// Matrix batch.a[blockIdx.x]: [rows, RP] row-major, rows <= 64 RPT, in place.
+template <int RP, int RPT, int CW>
+__global__ void __launch_bounds__(64 * RP / CW)
+gsw_kernel(GswBatch batch, float eps)
+{
+    constexpr int PS = RPT + 4;
+    extern __shared__ __attribute__((aligned(16))) float gsw_lds[];
+    float* piv = gsw_lds;                       // [2][64][PS]: the normalised pivot column, lane-major
+    float* tile = gsw_lds + 2 * 64 * PS;        // [TR][RP + 1]
+    float* __restrict__ a = batch.a[blockIdx.x];
+    const int rows = batch.rows[blockIdx.x];
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col0 = w * CW;
+
+    float v[CW][RPT];
+    gsw_load_columns<RP, RPT, CW>(a, rows, tile, v, tid, lane, col0);
+
+    gsw_steps<RP, RPT, CW>(v, piv, lane, w, eps);
     gsw_store_columns<RP, RPT, CW>(a, rows, tile, v, tid, lane, col0);
 }

@@ -3780,15 +3780,59 @@ psgd_lin_residual_batch_kernel(PsgdBatch<RowlistResidualItem<RP, true, true, T>>
                                                                 one_minus_beta, bx - b.first[i]);
 }
 
+// The Q factors of ranks 16 and 32 orthogonalised for the bucket's next round by workgroups in front of the last launch:
+// the kernels that take column after column (gs_wide_by_columns), from the new Q into q_next.  A launch of their own at the
+// end of a bucket's round was 27 us (six factors [1024,32]) or 34 (with a [4096,32]) behind a residual launch of 20 to 25; the
+// two together take 37 and 35.5, and 89 where [30522,1024] took 76 + 27 with narrower workgroups.  (Without the raised
+// priority the second kind took 52; its chain of short steps otherwise waits its turn between streaming waves.)
+struct WideNext {
+    const float* q[kPsgdBatchMax];       // row-major
+    const float* qp[kPsgdBatchMax];      // by pieces
+    float* dst[kPsgdBatchMax];
+    int rows[kPsgdBatchMax], slab[kPsgdBatchMax], first[kPsgdBatchMax + 1];
+    int count, wgs;
+    bool gram;                           // by their Gram matrices, several workgroups a matrix (conef_gs_gram.h)
+    float eps;
+};
+
+// at most this many rows of the others: a wave's share of the columns is in registers
+constexpr int wide_next_rows(int rp, int threads) { return rp == 32 && threads == 256 ? 512 : 1024; }
+
+template <int RP>
+constexpr size_t wide_next_lds_bytes(bool gram) { return gram ? sizeof(GsgLds<RP>) : sizeof(float) * gsw_pieces_lds_floats<16>(); }
+
+template <int RP, int T>
+__device__ __forceinline__ void wide_next_body(const WideNext& g, int bx, GsgWs* ws, unsigned tag)
+{
+    extern __shared__ __attribute__((aligned(16))) float wide_next_lds[];
+    __builtin_amdgcn_s_setprio(2);       // a chain of short steps that the launch waits for, next to waves that stream
+    int it = 0;
+    while (it + 1 < g.count && bx >= g.first[it + 1]) ++it;
+    if (g.gram) {
+        const int wg0 = g.first[it];
+        gsg_body<RP, T, true>(*reinterpret_cast<GsgLds<RP>*>(wide_next_lds), g.q[it], g.dst[it], g.rows[it], g.slab[it], wg0,
+                        g.first[it + 1] - wg0, bx - wg0, g.eps, ws, tag);
+    } else if (g.rows[it] <= 512) {
+        gsw_pieces_body<RP, 8, T>(g.qp[it], g.dst[it], g.rows[it], wide_next_lds, g.eps);
+    } else if constexpr (wide_next_rows(RP, T) > 512) {
+        gsw_pieces_body<RP, 16, T>(g.qp[it], g.dst[it], g.rows[it], wide_next_lds, g.eps);
+    }
+}
+
 // M = P Q^T at ranks 9 to 32 with the residuals sketched (conef_psgd_mfma_residual.h).
 template <int RP, bool LOOK, int T>
 __global__ void __launch_bounds__(T, 4)
-psgd_mfma_residual_batch_kernel(PsgdBatch<MfmaResidualItem<RP, LOOK, T>> b, double one_minus_beta)
+psgd_mfma_residual_batch_kernel(PsgdBatch<MfmaResidualItem<RP, LOOK, T>> b, double one_minus_beta, WideNext next, GsgWs* ws, unsigned tag)
 {
-    int local;
-    const MfmaResidualItem<RP, LOOK, T>& it = b.item[psgd_batch_locate(b, &local)];
+    if ((int)blockIdx.x < next.wgs) {
+        wide_next_body<RP, T>(next, (int)blockIdx.x, ws, tag);
+        return;
+    }
+    const int bx = (int)blockIdx.x - next.wgs;
+    const int i = psgd_batch_item(b, bx);
+    const MfmaResidualItem<RP, LOOK, T>& it = b.item[i];
     conef_rowlist_body<float, ListMfmaResidual<RP, LOOK, T>>(it.front, it.plan, it.cs_in, it.cs_out, it.n, it.d, it.w, it.rb,
-                                                             one_minus_beta, local);
+                                                             one_minus_beta, bx - b.first[i]);
 }
 
 // Rows a workgroup of the dense M = P Q^T takes: as many as leave the launch two thousand workgroups
@@ -4445,7 +4489,8 @@ bool wide_sketch_round(const ConefPsgdItem* items, int count, int32_t a, int32_t
 }
 
 template <int RP, bool LOOK, int T>
-int wide_sketch_launch(const PaddedRound& pr, const WideTiles& tiles, const std::vector<MfmaLook>& look, float beta, hipStream_t s)
+int wide_sketch_launch(const PaddedRound& pr, const WideTiles& tiles, const std::vector<MfmaLook>& look, const WideNext& next, float beta,
+                       void* workspace, hipStream_t s)
 {
     using Item = MfmaResidualItem<RP, LOOK, T>;
     std::vector<Item> table;
@@ -4458,25 +4503,61 @@ int wide_sketch_launch(const PaddedRound& pr, const WideTiles& tiles, const std:
         blocks.push_back((int)tiles.shapes[k].tiles);
     }
     auto kern = psgd_mfma_residual_batch_kernel<RP, LOOK, T>;
-    if (hipError_t e = conef_allow_lds((const void*)kern, tiles.lds); e != hipSuccess) return (int)e;
+    const size_t lds = next.wgs ? std::max(tiles.lds, wide_next_lds_bytes<RP>(next.gram)) : tiles.lds;
+    if (hipError_t e = conef_allow_lds((const void*)kern, lds); e != hipSuccess) return (int)e;
     const double omb = 1. - (double)beta;
+    GsgWs* ws = (GsgWs*)workspace;
+    const unsigned tag = 0u;      // drawn by conef_launch_tagged
     return run_batches(table, blocks, [&](const PsgdBatch<Item>& bt, int grid) {
-        conef_launch(kern, dim3((unsigned)grid), dim3(T), tiles.lds, s, bt, omb);
+        conef_launch_tagged<4>(g_gsg_launches, kern, dim3((unsigned)(grid + next.wgs)), dim3(T), lds, s, bt, omb, next, ws, tag);
     });
 }
 
 template <int RP>
-int wide_sketch_residual(const PaddedRound& pr, const WideTiles& tiles, const std::vector<MfmaLook>& look, float beta, hipStream_t s)
+int wide_sketch_residual(const PaddedRound& pr, const WideTiles& tiles, const std::vector<MfmaLook>& look, const WideNext& next, float beta,
+                         void* workspace, hipStream_t s)
 {
     auto go = [&](auto looked) {
         constexpr bool LOOK = decltype(looked)::value;
         switch (tiles.threads) {
-            case 256: return wide_sketch_launch<RP, LOOK, 256>(pr, tiles, look, beta, s);
-            case 512: return wide_sketch_launch<RP, LOOK, 512>(pr, tiles, look, beta, s);
-            default: return wide_sketch_launch<RP, LOOK, 1024>(pr, tiles, look, beta, s);
+            case 256: return wide_sketch_launch<RP, LOOK, 256>(pr, tiles, look, next, beta, workspace, s);
+            case 512: return wide_sketch_launch<RP, LOOK, 512>(pr, tiles, look, next, beta, workspace, s);
+            default: return wide_sketch_launch<RP, LOOK, 1024>(pr, tiles, look, next, beta, workspace, s);
         }
     };
     return look.empty() ? go(std::false_type()) : go(std::true_type());
+}
+
+// The workgroups that orthogonalise pr's new Q factors into q_next along with the last launch; *threads: that launch's,
+// which may have to be wider for them.  wgs 0: none, they are a launch of their own.
+inline WideNext wide_next(const PaddedRound& pr, float* const* q_next, float eps, const void* workspace, int64_t workspace_bytes, int* threads)
+{
+    WideNext g = {};
+    g.eps = eps;
+    g.count = (int)pr.items.size();
+    int64_t tallest = 0;
+    for (int k = 0; k < g.count; ++k) {
+        const ConefPsgdItem& it = pr.items[(size_t)k];
+        g.q[k] = it.q;
+        g.qp[k] = pr.qi[(size_t)k];
+        g.dst[k] = q_next[k];
+        g.rows[k] = (int)it.m;
+        g.gram = g.gram || gsg_wants(it.q, it.m, it.r);
+        if (!aligned16(q_next[k])) return WideNext{};
+        tallest = std::max(tallest, it.m);
+    }
+    int wgs = 0;
+    for (int k = 0; k < g.count; ++k) {
+        int w = 1;
+        if (g.gram) gsg_split(g.rows[k], pr.rp, &g.slab[k], &w);
+        g.first[k] = wgs;
+        wgs += w;
+    }
+    g.first[g.count] = wgs;
+    if (g.gram ? !gsg_workspace_ok(workspace, workspace_bytes) : tallest > wide_next_rows(pr.rp, 1024)) return WideNext{};
+    if (!g.gram && tallest > wide_next_rows(pr.rp, *threads)) *threads = 512;
+    g.wgs = wgs;
+    return g;
 }
 
 // The first product with X formed from the cells: two column splits of a row tile to a workgroup share its cells in LDS, four
@@ -4766,6 +4847,7 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
     // Above rank 8 the residual is sketched by the last launch of a deferred round
     WideTiles tiles;
     const bool wide_sketch = deferred && rp > 8 && pqt_mode == 2 && wide_sketch_round(items, count, a, b, workspace, workspace_bytes, &pr, &tiles);
+    WideNext next = {};
     std::vector<MfmaLook> look;
     if (wide_sketch && mq_mode == 2 && look_pays(items, count))
         for (int k = 0; k < count; ++k) look.push_back(MfmaLook{items[k].cs, item_pktab(items[k]), items[k].w, alpha});
@@ -4812,8 +4894,9 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
             if (rc == CONEF_OK && made && want_next) *made = by_quads && by_fold ? 5 : 1;
             return rc;
         }
+        if (want_next && wide_sketch && columns) next = wide_next(pr, q_next, eps, workspace, workspace_bytes, &tiles.threads);
         // the column kernels work in place: the fix launch leaves the new Q in q_next as well
-        if (want_next && rp > 8 && columns)
+        if (want_next && rp > 8 && columns && !next.wgs)
             for (int k = 0; k < count; ++k) pr.qt[(size_t)k] = q_next[k];
         GsAhead* qs = want_next && rp <= 8 ? &ahead : nullptr;
         rc = deferred_products(pr, r, q_in.data(), quads_ready ? q_next + count : nullptr, mq_mode, alpha, eps, a, b, workspace,
@@ -4862,13 +4945,15 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
     }
     bool used = false;
     if (wide_sketch)
-        rc = rp == 16 ? wide_sketch_residual<16>(pr, tiles, look, beta, hs) : wide_sketch_residual<32>(pr, tiles, look, beta, hs);
+        rc = rp == 16 ? wide_sketch_residual<16>(pr, tiles, look, next, beta, workspace, hs)
+                      : wide_sketch_residual<32>(pr, tiles, look, next, beta, workspace, hs);
     else
         rc = pqt_batch(its, count, pqt_mode == 3 ? 1 : pqt_mode, pqt_mode == 2 ? beta : 0.f, a, b, hs,
                        ahead.count ? &ahead : nullptr, &used, deferred && rp <= 8 ? &pr.qi : nullptr);
     if (rc != CONEF_OK) return rc;
     if (want_next && deferred && rp > 8) {
-        if (gs_wide_by_columns(pr)) {
+        if (next.wgs) {
+        } else if (gs_wide_by_columns(pr)) {
             rc = orthogonalise_by_columns(pr, items[0].r, q_next, eps, workspace, workspace_bytes, hs);
         } else {
             std::vector<const float*> src;
