@@ -71,9 +71,10 @@ int conef_cs_update_planned_f32(const float* vec, const float* cs_in, float* cs_
     const ConefPlanHeader* hp = (const ConefPlanHeader*)plan_host;
     if (!conef_plan_matches(hp, n, d, w, a, b) || !plan_dev || !vec || !cs_in || !cs_out) return CONEF_ERR_INVALID;
     if (hp->kind == kConefPlanRowlist) {
-        ConefListVec front = {vec, aligned16(vec) && d % 4 == 0};
-        return conef_launch_rowlist(front, conef_rowlist_view(hp, plan_dev), cs_in, cs_out, n, d, w, beta,
-                                    (hipStream_t)stream);
+        const bool vec_ok = aligned16(vec) && d % 4 == 0;
+        return conef_launch_rowlist_any<ConefListVecT>([&](auto t) { return ConefListVecT<decltype(t)::value>{vec, vec_ok}; },
+                                                       conef_rowlist_view(hp, plan_dev), cs_in, cs_out, n, d, w, beta,
+                                                       (hipStream_t)stream);
     }
     if (hp->kind == kConefPlanPanels) {
         ConefPanelVec front = {vec, aligned16(vec) && d % 4 == 0};
@@ -101,9 +102,10 @@ int conef_cs_update_planned_f16(const float* vec, const void* cs_in_half, void* 
                                    d, w, beta, (hipStream_t)stream);
     }
     if (hp->kind != kConefPlanRowlist) return CONEF_ERR_INVALID;
-    ConefListVec front = {vec, aligned16(vec) && d % 4 == 0};
-    return conef_launch_rowlist(front, conef_rowlist_view(hp, plan_dev), (const __half*)cs_in_half,
-                                (__half*)cs_out_half, n, d, w, beta, (hipStream_t)stream);
+    const bool vec_ok = aligned16(vec) && d % 4 == 0;
+    return conef_launch_rowlist_any<ConefListVecT>([&](auto t) { return ConefListVecT<decltype(t)::value>{vec, vec_ok}; },
+                                                   conef_rowlist_view(hp, plan_dev), (const __half*)cs_in_half,
+                                                   (__half*)cs_out_half, n, d, w, beta, (hipStream_t)stream);
 }
 
 // DenseCS.query with the buckets and signs of a plan's table instead of hashing (either kind of
@@ -153,9 +155,9 @@ int conef_randblock_conef_step_planned_f32(float* x, const float* cs_in, float* 
     if (!(start >= 0 && start < numel && block >= 1 && block <= numel)) return CONEF_ERR_INVALID;
     ConefBlock blk = conef_make_block(numel, start, block);
     if (hp->kind == kConefPlanRowlist) {
-        ConefListRandBlock front = {x, payload, blk, alpha};
-        return conef_launch_rowlist(front, conef_rowlist_view(hp, plan_dev), cs_in, cs_out, n, m, w, beta,
-                                    (hipStream_t)stream);
+        return conef_launch_rowlist_any<ConefListRandBlockT>(
+            [&](auto t) { return ConefListRandBlockT<decltype(t)::value>{x, payload, blk, alpha}; }, conef_rowlist_view(hp, plan_dev),
+            cs_in, cs_out, n, m, w, beta, (hipStream_t)stream);
     }
     if (hp->kind == kConefPlanPanels) {
         ConefPanelRandBlock front = {x, payload, blk, alpha, aligned16(x) && m % 4 == 0};

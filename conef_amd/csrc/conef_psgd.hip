@@ -1128,7 +1128,8 @@ psgd_cs_query_batch_kernel(PsgdBatch<QueryItem> b, float alpha, ConefSeeds hs)
 // DenseCS.update(vec, beta) (CountSketch.py:27-48) of the sketches of a bucket's matrices on
 // row-list plans, vec = the item's dense residual.
 struct RowlistVecItem {
-    ConefListVec front;
+    const float* vec;
+    bool vec_ok;
     ConefRowlistView plan;
     const float* cs_in;
     float* cs_out;
@@ -1136,13 +1137,14 @@ struct RowlistVecItem {
     int d, w, rb;
 };
 
-__global__ void __launch_bounds__(kConefRowlistThreads)
+template <int T>
+__global__ void __launch_bounds__(T)
 psgd_rowlist_vec_batch_kernel(PsgdBatch<RowlistVecItem> b, double one_minus_beta)
 {
     int local;
     const RowlistVecItem& it = b.item[psgd_batch_locate(b, &local)];
-    conef_rowlist_body<float, ConefListVec>(it.front, it.plan, it.cs_in, it.cs_out, it.n, it.d, it.w, it.rb, one_minus_beta,
-                                            local);
+    const ConefListVecT<T> front = {it.vec, it.vec_ok};
+    conef_rowlist_body<float, ConefListVecT<T>>(front, it.plan, it.cs_in, it.cs_out, it.n, it.d, it.w, it.rb, one_minus_beta, local);
 }
 
 // The general form: any rank up to RP, element by element.
@@ -4749,8 +4751,8 @@ int conef_psgd_sketch_update_batch_f32(const ConefPsgdItem* items, int32_t count
 {
     if (count < 0 || (count > 0 && !items)) return CONEF_ERR_INVALID;
     std::vector<RowlistVecItem> table;
+    std::vector<ConefRowlistShape> shapes, taller;
     std::vector<int> blocks;
-    size_t lds = 0;
     int64_t full_tiles = 0;     // as in pqt_sketch_group: full-height tiles when there are 600 of them
     for (int k = 0; k < count; ++k) {
         ConefRowlistShape shape;
@@ -4758,6 +4760,8 @@ int conef_psgd_sketch_update_batch_f32(const ConefPsgdItem* items, int32_t count
             full_tiles += shape.tiles;
     }
     const int companions = full_tiles >= 600 ? 0 : count;
+    size_t lds = 0;
+    double values = 0., large = 0.;
     for (int k = 0; k < count; ++k) {
         const ConefPsgdItem& it = items[k];
         const ConefPlanHeader* hp = (const ConefPlanHeader*)it.plan_host;
@@ -4766,18 +4770,41 @@ int conef_psgd_sketch_update_batch_f32(const ConefPsgdItem* items, int32_t count
             return CONEF_ERR_INVALID;
         ConefRowlistShape shape;
         if (!conef_rowlist_shape(it.n, it.m, it.w, ConefListVec::kNeedsCells, ConefListVec::halves(it.m), &shape, companions)) return CONEF_ERR_INVALID;
-        RowlistVecItem t = {{it.err, aligned16(it.err) && it.m % 4 == 0}, conef_rowlist_view(hp, it.plan_dev), it.cs, it.cs,
-                            it.n, (int)it.m, it.w, shape.rb};
-        table.push_back(t);
-        blocks.push_back((int)shape.tiles);
-        if (shape.lds > lds) lds = shape.lds;
+        shapes.push_back(shape);
+        conef_rowlist_taller(it.n, it.m, it.w, ConefListVec::kNeedsCells, &shape);
+        taller.push_back(shape);
+        table.push_back(RowlistVecItem{it.err, aligned16(it.err) && it.m % 4 == 0, conef_rowlist_view(hp, it.plan_dev), it.cs, it.cs,
+                                       it.n, (int)it.m, it.w, 0});
+        values += (double)it.n * (double)it.m;
+        lds = std::max(lds, shape.lds);
     }
-    if (hipError_t e = conef_allow_lds((const void*)psgd_rowlist_vec_batch_kernel, lds); e != hipSuccess) return (int)e;
+    // (a launch gives every tile the LDS of its largest)
+    for (int k = 0; k < count; ++k)
+        if (2 * taller[(size_t)k].lds >= lds) large += (double)items[k].n * (double)items[k].m;
+    if (2. * large >= values) shapes = taller;
+    lds = 0;
+    int64_t tiles = 0;
+    for (int k = 0; k < count; ++k) {
+        const ConefRowlistShape& shape = shapes[(size_t)k];
+        table[(size_t)k].rb = shape.rb;
+        blocks.push_back((int)shape.tiles);
+        tiles += shape.tiles;
+        lds = std::max(lds, shape.lds);
+    }
     const double omb = 1. - (double)beta;
     hipStream_t s = (hipStream_t)stream;
-    return run_batches(table, blocks, [&](const PsgdBatch<RowlistVecItem>& bt, int grid) {
-        conef_launch(psgd_rowlist_vec_batch_kernel, dim3((unsigned)grid), dim3(kConefRowlistThreads), lds, s, bt, omb);
-    });
+    auto with = [&](auto threads) {
+        constexpr int T = decltype(threads)::value;
+        if (hipError_t e = conef_allow_lds((const void*)psgd_rowlist_vec_batch_kernel<T>, lds); e != hipSuccess) return (int)e;
+        return run_batches(table, blocks, [&](const PsgdBatch<RowlistVecItem>& bt, int grid) {
+            conef_launch(psgd_rowlist_vec_batch_kernel<T>, dim3((unsigned)grid), dim3(T), lds, s, bt, omb);
+        });
+    };
+    switch (conef_rowlist_workgroup(lds, tiles, values, ConefListVec::kLeastValues)) {
+        case 256: return with(std::integral_constant<int, 256>());
+        case 512: return with(std::integral_constant<int, 512>());
+        default: return with(std::integral_constant<int, 1024>());
+    }
 }
 
 // One PowerSGD round over the matrices of a bucket in a single call (powerSGD_hook.py:473-564 at

@@ -70,7 +70,10 @@ __global__ void __launch_bounds__(256) randblock_ef_batch_kernel(RbBatch<DenseIt
 }
 
 struct ListItem {
-    ConefListRandBlock front;
+    float* x;
+    float* payload;
+    ConefBlock blk;
+    float alpha;
     ConefRowlistView plan;
     const float* cs_in;
     float* cs_out;
@@ -79,14 +82,15 @@ struct ListItem {
     bool pk_lds;
 };
 
-template <int CAP>
-__global__ void __launch_bounds__(kConefRowlistThreads)
+template <int CAP, int T>
+__global__ void __launch_bounds__(T)
 randblock_rowlist_batch_kernel(RbBatch<ListItem, CAP> b, double one_minus_beta)
 {
     int local, width;
     const ListItem& it = b.item[rb_locate(b, &local, &width)];
-    conef_rowlist_body<float, ConefListRandBlock>(it.front, it.plan, it.cs_in, it.cs_out, it.n, it.d, it.w, it.rb,
-                                                  one_minus_beta, local, it.pk_lds);
+    const ConefListRandBlockT<T> front = {it.x, it.payload, it.blk, it.alpha};
+    conef_rowlist_body<float, ConefListRandBlockT<T>>(front, it.plan, it.cs_in, it.cs_out, it.n, it.d, it.w, it.rb,
+                                                      one_minus_beta, local, it.pk_lds);
 }
 
 template <typename Item, int CAP, typename Go>
@@ -171,30 +175,59 @@ int conef_randblock_step_batch_f32(const ConefRandBlockItem* items, int32_t coun
     }
     // sketched error: row-list plans share launches, the rest go one by one
     std::vector<ListItem> table;
-    std::vector<int> blocks;
-    size_t lds = 0;
+    std::vector<ConefRowlistShape> shapes, taller;
     for (int k = 0; k < count; ++k) {
         const ConefRandBlockItem& it = items[k];
         const ConefPlanHeader* hp = (const ConefPlanHeader*)it.plan_host;
         if (!hp || hp->kind != kConefPlanRowlist) continue;
         ConefRowlistShape shape;
         if (!conef_rowlist_shape(it.n, it.m, it.w, ConefListRandBlock::kNeedsCells, ConefListRandBlock::halves(it.m), &shape)) return CONEF_ERR_INVALID;
-        ListItem t = {{it.x, it.payload, conef_make_block(it.n * it.m, it.start, it.block), alpha},
-                      conef_rowlist_view(hp, it.plan_dev), it.cs_in, it.cs_out, it.n, (int)it.m, it.w, shape.rb, shape.pk_lds};
-        table.push_back(t);
-        blocks.push_back((int)shape.tiles);
-        if (shape.lds > lds) lds = shape.lds;
+        shapes.push_back(shape);
+        conef_rowlist_taller(it.n, it.m, it.w, ConefListRandBlock::kNeedsCells, &shape);
+        taller.push_back(shape);
+        table.push_back(ListItem{it.x, it.payload, conef_make_block(it.n * it.m, it.start, it.block), alpha,
+                                 conef_rowlist_view(hp, it.plan_dev), it.cs_in, it.cs_out, it.n, (int)it.m, it.w, 0, false});
     }
     if (!table.empty()) {
-        const void* kern = table.size() <= (size_t)kRbFew ? (const void*)randblock_rowlist_batch_kernel<kRbFew>
-                                                          : (const void*)randblock_rowlist_batch_kernel<rb_batch_max<ListItem>()>;
-        hipError_t e = conef_allow_lds(kern, lds);
-        if (e != hipSuccess) return (int)e;
+        // A launch gives every tile the LDS of its largest: taller ones where half the values are in tiles of half of that.
+        // Steps with one row by 256 threads and so, us: WRN-28-10 with sketches of 0.05 and 0.5 192 and 172, 325 and 242,
+        // an LSTM of 500 and one of 300 66 and 53, 34 and 21, an encoder of 1024 with 0.2 327 and 302.
+        size_t lds = 0;
+        for (const ConefRowlistShape& t : taller) lds = std::max(lds, t.lds);
+        double values = 0., large = 0.;
+        for (size_t k = 0; k < table.size(); ++k) {
+            const double v = (double)table[k].n * (double)table[k].d;
+            values += v;
+            if (2 * taller[k].lds >= lds) large += v;
+        }
+        if (2. * large >= values) shapes = taller;
+        lds = 0;
+        int64_t tiles = 0;
+        std::vector<int> blocks;
+        for (size_t k = 0; k < table.size(); ++k) {
+            table[k].rb = shapes[k].rb;
+            table[k].pk_lds = shapes[k].pk_lds;
+            blocks.push_back((int)shapes[k].tiles);
+            tiles += shapes[k].tiles;
+            lds = std::max(lds, shapes[k].lds);
+        }
         const double omb = 1. - (double)beta;
-        int rc = rb_run(table, blocks, [&](const auto& bt, int grid) {
-            conef_launch((randblock_rowlist_batch_kernel<sizeof(bt.item) / sizeof(bt.item[0])>), dim3((unsigned)grid), dim3(kConefRowlistThreads), lds, s,
-                               bt, omb);
-        });
+        auto with = [&](auto threads) {
+            constexpr int T = decltype(threads)::value;
+            hipError_t e = hipSuccess;
+            const int rc = rb_run(table, blocks, [&](const auto& bt, int grid) {
+                auto kern = randblock_rowlist_batch_kernel<sizeof(bt.item) / sizeof(bt.item[0]), T>;
+                e = conef_allow_lds((const void*)kern, lds);
+                if (e == hipSuccess) conef_launch(kern, dim3((unsigned)grid), dim3(T), lds, s, bt, omb);
+            });
+            return e != hipSuccess ? (int)e : rc;
+        };
+        int rc;
+        switch (conef_rowlist_workgroup(lds, tiles, values, ConefListRandBlock::kLeastValues)) {
+            case 256: rc = with(std::integral_constant<int, 256>()); break;
+            case 512: rc = with(std::integral_constant<int, 512>()); break;
+            default: rc = with(std::integral_constant<int, 1024>()); break;
+        }
         if (rc != CONEF_OK) return rc;
     }
     for (int k = 0; k < count; ++k) {

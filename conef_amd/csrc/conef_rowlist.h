@@ -20,6 +20,7 @@
 #pragma once
 #include "conef_device.h"
 #include "conef_sketch_core.h"
+#include <algorithm>
 #include <type_traits>
 
 constexpr int kConefRowlistThreads = 256;
@@ -94,17 +95,55 @@ inline bool conef_rowlist_shape(int64_t n, int64_t d, int32_t w, bool cells, boo
     return s->tiles <= 0x7fffffff;
 }
 
+// Taller tiles for matrices of few or of long rows (the shapes above give those one row a tile), and the threads of a
+// workgroup: sixteen waves a CU with as many tiles as its LDS holds or the launch has, and at least `least` values each.
+// A tile is a chain - its rows, then the lists - that a CU with one or two of them in it waits for, and a thread that walks a
+// list for two rows reads it once.  One row by 256 threads against this, us, sketches of 0.1 and of 0.4:
+//                        update, half cells            update                        random-block step
+//   [300,1000]           4.8   4.6    4.6   4.4        4.6   4.3    4.6   4.3        6.1   6.2    6.0   6.2
+//   [2000,2000]          8.4   6.0   11.3   8.6        7.9   6.1   11.1   8.2       14.8  10.3   17.8  11.7
+//   [900,5700]           9.5   8.1   17.9   9.9        8.6   7.9   16.8  10.0       17.9  17.4   29.9  19.1
+//   [4096,5700]         41.1  29.0   71.3  44.5       38.7  28.1   68.3  40.9       63.7  46.8  115.4  72.3
+//   [2000,9000]         37.4  25.9   95.8  48.1       37.1  25.3   95.7  46.7       68.1  47.7  153.8  64.4
+//   [2000,12000]        71.4  34.8  124.2  73.7       71.3  34.2  124.8  71.5      138.6  60.3  194.7  93.5
+// Over 354 such shapes (rows of 600 to 20000, 64 to 4096 of them) a third less on average, one 7 % more (0.5 us).
+inline void conef_rowlist_taller(int64_t n, int64_t d, int32_t w, bool cells, ConefRowlistShape* s)
+{
+    for (int rb = 4; rb >= 2; rb -= 2) {
+        if (s->rb >= rb) return;
+        // (two rows of [640,5760] in a random-block step of WRN-28-10: 200 us, one row by 512 threads 186)
+        if (n < (int64_t)rb * (cells && (rb == 4 || d > 2048) ? 400 : rb == 4 ? 200 : 128)) continue;
+        const size_t lds = conef_rowlist_lds(rb, d, w, cells), pk = cells ? conef_rowlist_pk_bytes(d) : 0;
+        if (lds > kConefRowlistLdsLimit) continue;
+        s->rb = rb;
+        // (the column table stays out where it would leave a CU fewer tiles: [2000,7000] 35.0 us without, 37.7 with)
+        s->pk_lds = cells && lds + pk <= kConefRowlistLdsLimit && kConefRowlistLdsLimit / (lds + pk) == kConefRowlistLdsLimit / lds;
+        s->lds = s->pk_lds ? lds + pk : lds;
+        s->tiles = (n + rb - 1) / rb;
+        return;
+    }
+}
+
+inline int conef_rowlist_workgroup(size_t lds, int64_t tiles, double values, int least)
+{
+    const int64_t per_cu = std::min<int64_t>((int64_t)(kConefRowlistLdsLimit / std::max<size_t>(lds, 1)), (tiles + 255) / 256);
+    int threads = per_cu <= 1 ? 1024 : per_cu <= 3 ? 512 : 256;
+    while (threads > 256 && values < (double)least * threads * (double)tiles) threads /= 2;
+    return threads;
+}
+
 // ------------------------------------------------------------------ fronts ----
 // A front fills vals[row_in_tile * d + col] for the tile's rows.  `cells` (only when
 // kNeedsCells) holds the tile's old sketch rows, [rows][w]; a front with kParksCells puts them there itself
 // while it stages.
 
 // DenseCS.update: the value is the dense tensor itself.
-struct ConefListVec {
+template <int T>
+struct ConefListVecT {
     const float* vec;
     bool vec_ok;           // base 16-byte aligned and d % 4 == 0 (the tile copy works either way)
     static constexpr bool kNeedsCells = false, kParksCells = false, kCompact = false;
-    static constexpr int kThreads = kConefRowlistThreads;
+    static constexpr int kThreads = T, kLeastValues = 8;
     // whether a tensor with tiles to spare goes by half-height ones.  Full against half height: [50000,512] 40.2
     // and 29.9 us, [20000,2048] 49.0 and 45.9, [30522,1024] 37.0 and 36.2, [33278,650] 26.2 and 26.0, [60000,300]
     // and [33278,200] within 1 % either way.
@@ -122,16 +161,16 @@ struct ConefListVec {
         if (lead > total) lead = total;
         const int total4 = (total - lead) >> 2;
         const float4* src4 = reinterpret_cast<const float4*>(base + lead);
-        for (int q0 = threadIdx.x; q0 < total4; q0 += 8 * kConefRowlistThreads) {
+        for (int q0 = threadIdx.x; q0 < total4; q0 += 8 * T) {
             float4 t[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                int q = q0 + u * kConefRowlistThreads;
+                int q = q0 + u * T;
                 t[u] = src4[q < total4 ? q : total4 - 1];
             }
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                int q = q0 + u * kConefRowlistThreads;
+                int q = q0 + u * T;
                 if (q < total4) {
                     if (lead == 0) {
                         reinterpret_cast<float4*>(vals)[q] = t[u];
@@ -149,6 +188,7 @@ struct ConefListVec {
         }
     }
 };
+using ConefListVec = ConefListVecT<kConefRowlistThreads>;
 
 // RandomBlock + ConEF (reference: communication/RandomBlock_hook.py:190,216-243,272-280 at world
 // size 1): xq = x + alpha * unsketch(old cells); inside the wrap-around block xq goes to the
@@ -160,13 +200,14 @@ struct ConefListVec {
 // `stage` then works from LDS: row and column of a quad advance with it (no division per quad),
 // the block is a pair of tile-relative ranges, and a tile that does not touch the block at all -
 // most of them - runs without any of that.
-struct ConefListRandBlock {
+template <int T>
+struct ConefListRandBlockT {
     float* x;
     float* payload;
     ConefBlock blk;
     float alpha;
     static constexpr bool kNeedsCells = true, kParksCells = false, kCompact = false;
-    static constexpr int kThreads = kConefRowlistThreads;
+    static constexpr int kThreads = T, kLeastValues = 3;
     static bool halves(int64_t) { return true; }      // (the column table sits in LDS next to the tiles)
     static constexpr int kQuads = 4;
     struct Regs {          // a thread's first kQuads quads, by name: no array for the compiler to keep in memory
@@ -202,9 +243,9 @@ struct ConefListRandBlock {
         if (total4 > 0) {
             const int q = threadIdx.x, last = total4 - 1;      // past the end: a valid address, result unused
             r.g0 = base4[q < last ? q : last];
-            r.g1 = base4[q + kConefRowlistThreads < last ? q + kConefRowlistThreads : last];
-            r.g2 = base4[q + 2 * kConefRowlistThreads < last ? q + 2 * kConefRowlistThreads : last];
-            r.g3 = base4[q + 3 * kConefRowlistThreads < last ? q + 3 * kConefRowlistThreads : last];
+            r.g1 = base4[q + T < last ? q + T : last];
+            r.g2 = base4[q + 2 * T < last ? q + 2 * T : last];
+            r.g3 = base4[q + 3 * T < last ? q + 3 * T : last];
         }
         return r;
     }
@@ -257,7 +298,7 @@ struct ConefListRandBlock {
                                           int rest) const
     {
         float4* base4 = reinterpret_cast<float4*>(base + lead);
-        constexpr int kStep = 4 * kConefRowlistThreads;          // elements between a thread's quads
+        constexpr int kStep = 4 * T;          // elements between a thread's quads
         const int drow = kStep / d, dcol = kStep - drow * d;
         int q = threadIdx.x;
         int e = lead + (q << 2);
@@ -265,7 +306,7 @@ struct ConefListRandBlock {
         int roff = (e / d) * w;
         auto one = [&](float4 g) {
             if (q < total4) quad<BLOCK>(g, q, e, col, roff, base4, f0, lead, d, w, vals, cells, pk_l, lo, hi, rest);
-            q += kConefRowlistThreads;
+            q += T;
             e += kStep;
             col += dcol;
             roff += drow * w;
@@ -281,9 +322,9 @@ struct ConefListRandBlock {
         while (q < total4) {                 // taller tiles: four more quads a trip
             const int last = total4 - 1;
             const float4 g0 = base4[q];
-            const float4 g1 = base4[q + kConefRowlistThreads < last ? q + kConefRowlistThreads : last];
-            const float4 g2 = base4[q + 2 * kConefRowlistThreads < last ? q + 2 * kConefRowlistThreads : last];
-            const float4 g3 = base4[q + 3 * kConefRowlistThreads < last ? q + 3 * kConefRowlistThreads : last];
+            const float4 g1 = base4[q + T < last ? q + T : last];
+            const float4 g2 = base4[q + 2 * T < last ? q + 2 * T : last];
+            const float4 g3 = base4[q + 3 * T < last ? q + 3 * T : last];
             one(g0);
             one(g1);
             one(g2);
@@ -315,6 +356,7 @@ struct ConefListRandBlock {
         }
     }
 };
+using ConefListRandBlock = ConefListRandBlockT<kConefRowlistThreads>;
 
 // ------------------------------------------------------------------ kernel ----
 // count >= 1 words from global memory to LDS, eight loads in flight per thread
@@ -473,13 +515,14 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
     // bucket on neighbouring lanes: the lanes of a wave walk lists of about the same length (a wave
     // takes as many trips as its longest list).
     constexpr int kWalk = 4;
+    // (halves: update of [3000,200] with 80 buckets by 4 rows 4.6 us either way, [640,5760] by 2 rows 8.4 and 7.5)
     // A tile with more (bucket, row) pairs than threads: a thread walks a bucket's list for two rows, an entry
     // is taken apart once for both.  Update and random-block step, one row and two rows a thread: [33278,650]
     // 24.0 and 22.5, 38.5 and 37.3 us; [30522,1024] 33.1 and 31.9, 54.0 and 52.6; [6144,1024] 10.9 and 10.2, 17.5 and
     // 16.8; [9000,333] with 166 buckets 9.9 and 8.7, 13.3 and 12.2.  Four rows were slower than two everywhere
     // ([33278,650] 25.4), and two lose where they leave threads without work ([20000,300] with 15 buckets 9.0
     // and 9.7).
-    if (sizeof(CsT) == sizeof(float) && rows >= 2 && total > T) {
+    if (rows >= 2 && total > T) {
         constexpr int kTrip = 2;
         const int per = (rows + 1) >> 1, items = per * w;
         int jj = threadIdx.x / per, rg = threadIdx.x - jj * per;
@@ -558,11 +601,24 @@ conef_rowlist_body(const Front& front, ConefRowlistView plan, const CsT* cs_in, 
 }
 
 template <typename CsT, typename Front>
-__global__ void __launch_bounds__(kConefRowlistThreads)
+__global__ void __launch_bounds__(Front::kThreads)
 conef_rowlist_kernel(Front front, ConefRowlistView plan, const CsT* cs_in, CsT* cs_out, int64_t n, int d, int w,
                      int rb, double one_minus_beta, bool pk_lds)
 {
     conef_rowlist_body<CsT, Front>(front, plan, cs_in, cs_out, n, d, w, rb, one_minus_beta, (int)blockIdx.x, pk_lds);
+}
+
+template <typename CsT, typename Front>
+int conef_launch_rowlist_shape(Front front, const ConefRowlistShape& shape, ConefRowlistView plan, const CsT* cs_in, CsT* cs_out,
+                               int64_t n, int64_t d, int32_t w, float beta, hipStream_t s)
+{
+    auto k = conef_rowlist_kernel<CsT, Front>;
+    hipError_t e = conef_allow_lds((const void*)k, shape.lds);
+    if (e != hipSuccess) return (int)e;
+    const double omb = 1. - (double)beta;   // (1. - beta) with beta an fp32 value, CountSketch.py:38,63
+    conef_launch(k, dim3((unsigned)shape.tiles), dim3(Front::kThreads), shape.lds, s, front, plan, cs_in,
+                       cs_out, n, (int)d, (int)w, shape.rb, omb, shape.pk_lds);
+    return (int)hipGetLastError();
 }
 
 template <typename CsT, typename Front>
@@ -571,11 +627,22 @@ int conef_launch_rowlist(Front front, ConefRowlistView plan, const CsT* cs_in, C
 {
     ConefRowlistShape shape;
     if (!conef_rowlist_shape(n, d, w, Front::kNeedsCells, Front::halves(d), &shape)) return CONEF_ERR_INVALID;
-    auto k = conef_rowlist_kernel<CsT, Front>;
-    hipError_t e = conef_allow_lds((const void*)k, shape.lds);
-    if (e != hipSuccess) return (int)e;
-    const double omb = 1. - (double)beta;   // (1. - beta) with beta an fp32 value, CountSketch.py:38,63
-    conef_launch(k, dim3((unsigned)shape.tiles), dim3(kConefRowlistThreads), shape.lds, s, front, plan, cs_in,
-                       cs_out, n, (int)d, (int)w, shape.rb, omb, shape.pk_lds);
-    return (int)hipGetLastError();
+    return conef_launch_rowlist_shape(front, shape, plan, cs_in, cs_out, n, d, w, beta, s);
+}
+
+// The same for a front of any workgroup size, made by make(std::integral_constant<int, threads>).
+template <template <int> class FrontT, typename CsT, typename Make>
+int conef_launch_rowlist_any(Make make, ConefRowlistView plan, const CsT* cs_in, CsT* cs_out, int64_t n, int64_t d, int32_t w, float beta,
+                             hipStream_t s)
+{
+    using Front = FrontT<kConefRowlistThreads>;
+    ConefRowlistShape shape;
+    if (!conef_rowlist_shape(n, d, w, Front::kNeedsCells, Front::halves(d), &shape)) return CONEF_ERR_INVALID;
+    conef_rowlist_taller(n, d, w, Front::kNeedsCells, &shape);
+    auto go = [&](auto threads) { return conef_launch_rowlist_shape(make(threads), shape, plan, cs_in, cs_out, n, d, w, beta, s); };
+    switch (conef_rowlist_workgroup(shape.lds, shape.tiles, (double)n * (double)d, Front::kLeastValues)) {
+        case 256: return go(std::integral_constant<int, 256>());
+        case 512: return go(std::integral_constant<int, 512>());
+        default: return go(std::integral_constant<int, 1024>());
+    }
 }

@@ -415,3 +415,54 @@ def test_randblock_step_on_panels_and_row_groups_bit_exact(oracle, n, d, ss, kin
         np.testing.assert_array_equal(to_np(xd), x, err_msg="decompressed gradient, step %d" % step)
         np.testing.assert_array_equal(to_np(payload), opay, err_msg="payload, step %d" % step)
         np.testing.assert_array_equal(to_np(cs.cs), ocs, err_msg="sketch, step %d" % step)
+
+
+# Row lists around the tiles of one, two and four rows and the three workgroup sizes, rows of whole quads and others, with
+# and without the column table in LDS, the last tile with fewer rows, LDS of a quarter, a half and nearly all of a CU.
+TILES = [(255, 600, 0.1), (257, 601, 0.1), (801, 602, 0.4), (1601, 603, 0.1), (1603, 1400, 0.4), (257, 2048, 0.1), (258, 2051, 0.1),
+         (801, 2900, 0.3), (1602, 4001, 0.1), (640, 5760, 0.2), (1605, 5761, 0.4), (803, 7002, 0.1), (801, 12_001, 0.1), (130, 16_000, 0.3),
+         (33, 20_003, 0.1), (257, 24_000, 0.02)]
+
+
+@pytest.mark.parametrize("n,d,ss", TILES)
+def test_row_list_tiles_bit_exact(oracle, n, d, ss):
+    from conef_amd.compressors.CountSketch import DenseCS
+    from conef_amd.compressors.halfCountSketch import DenseCS as HalfCS
+    cs, half, step = DenseCS(n, d, ss), HalfCS(n, d, ss), DenseCS(n, d, ss)
+    assert cs.plan().kind == 1 and half.plan().kind == 1
+    o, oh, ocs = oracle.DenseCS(n, d, ss), oracle.HalfDenseCS(n, d, ss), np.zeros((n, step.range), np.float32)
+    rng = np.random.RandomState(n + d)
+    numel = n * d
+    block = max(1, int(0.1 * numel))
+    for start in (numel - block // 3, 3 * d + 1):
+        v = (rng.randn(n, d) * 1e-2).astype(np.float32)
+        for s, ref in ((cs, o), (half, oh)):
+            s.update(dev(v), 0.9)
+            ref.update(v, 0.9)
+            np.testing.assert_array_equal(to_np(s.cs), ref.cs)
+        xd, payload, opay = dev(v), torch.empty(block, device="cuda"), np.empty(block, np.float32)
+        step.randblock_step(xd, payload, start, block, 1 - 0.9, 0.9)
+        oracle.randblock_conef_step(v, ocs, opay, start, block, 1 - 0.9, 0.9)
+        np.testing.assert_array_equal(to_np(xd), v)
+        np.testing.assert_array_equal(to_np(payload), opay)
+        np.testing.assert_array_equal(to_np(step.cs), ocs)
+
+
+@pytest.mark.parametrize("shapes", [[(640, 5760), (10,), (64, 27), (300, 2880)], [(801, 3003), (900, 2002), (64, 64, 3, 3)],
+                                    [(1000, 650)] * 5 + [(1000, 7)], [(16, 16, 3, 3)] * 20 + [(600, 4001)]])
+def test_row_list_tiles_of_a_bucket(oracle, shapes):
+    """Tensors of several shapes in one launch, which has one workgroup size and one tile's LDS for all."""
+    from _helpers import FakeGradBucket
+    from conef_amd.RandomBlock_hook import RandomBlock_hook, RandomBlockState
+    args = dict(compression_ratio=0.1, use_error_compression=True, sketch_size=0.2, beta=0.9)
+    st, ost = RandomBlockState(None, start_compression_iter=2, **args), oracle.RandomBlockOracle(**args)
+    st.iter = 2
+    rng = np.random.RandomState(4)
+    for step in range(2):
+        flat = (rng.randn(sum(int(np.prod(s)) for s in shapes)) * 1e-3).astype(np.float32)
+        fd = dev(flat)
+        RandomBlock_hook(st, FakeGradBucket(fd, shapes)).wait()
+        ost.step(0, flat, shapes)
+        np.testing.assert_array_equal(to_np(fd), flat)
+        for e, oe in zip(st.error_dict[0], ost.error_dict[0]):
+            np.testing.assert_array_equal(to_np(e.cs), oe.cs)
