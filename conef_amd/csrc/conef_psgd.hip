@@ -1022,15 +1022,18 @@ psgd_mfma_mtp_batch_kernel(PsgdBatch<MfmaMtpItem> b)
 {
     int local;
     const MfmaMtpItem& it = b.item[psgd_batch_locate_near(b, &local)];
-    psgd_mfma_mtp_body<V>(it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, local % it.col_tiles, local / it.col_tiles);
+    __shared__ float red[kMfmaWaves][16][64];
+    psgd_mfma_mtp_body<V>(red, it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, local % it.col_tiles, local / it.col_tiles);
 }
 
 // the same with the workgroups in front that solve the matrices' Gram systems (deferred
 // orthogonalisation of P at ranks 16 and 32), and one launch for the matrices of every vector
 // width: the solving workgroups outlast the products of one width, and a launch per width would
-// each wait for its slowest workgroup
+// each wait for its slowest workgroup.  Four workgroups a CU (128 registers, 34 KB of LDS): a batch asks for 768 of them, which
+// two a CU - a place in LDS for every V, stages twice as long and 236 registers - took in a round and a half.  An encoder of
+// 1024 at rank 32 803 -> 765 us a step, its embedding's launch 54 -> 50.
 template <int RP, typename Item>
-__global__ void __launch_bounds__(kMfmaThreads)
+__global__ void __launch_bounds__(kMfmaThreads, 4)
 psgd_mfma_mtp_gram_batch_kernel(PsgdBatch<Item> b, GramTask g)
 {
     if ((int)blockIdx.x < g.count) {
@@ -1045,9 +1048,10 @@ psgd_mfma_mtp_gram_batch_kernel(PsgdBatch<Item> b, GramTask g)
     constexpr bool LOOK = std::is_same<Item, MfmaLookMtpItem>::value;
     MfmaLook look = {};
     if constexpr (LOOK) look = it.look;
-    if (it.v == 4) psgd_mfma_mtp_body<4, LOOK>(it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, ct, slab, look);
-    else if (it.v == 2) psgd_mfma_mtp_body<2, LOOK>(it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, ct, slab, look);
-    else psgd_mfma_mtp_body<1, LOOK>(it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, ct, slab, look);
+    __shared__ float red[kMfmaWaves][16][64];
+    if (it.v == 4) psgd_mfma_mtp_body<4, LOOK>(red, it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, ct, slab, look);
+    else if (it.v == 2) psgd_mfma_mtp_body<2, LOOK>(red, it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, ct, slab, look);
+    else psgd_mfma_mtp_body<1, LOOK>(red, it.x, it.p, it.out, it.n, it.m, it.r, it.rows_per_slab, ct, slab, look);
 }
 
 // the Gram systems alone (ranks 9 to 32): a workgroup a matrix

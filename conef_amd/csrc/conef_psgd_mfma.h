@@ -15,6 +15,7 @@
 #pragma once
 #include "conef_device.h"
 #include "conef_sketch_core.h"
+#include <type_traits>
 
 typedef float conef_f16v __attribute__((ext_vector_type(16)));
 
@@ -170,6 +171,7 @@ psgd_mfma_mq_kernel(float* __restrict__ x, const float* __restrict__ err, const 
 // Any alignment, any m >= V: the last run of V columns is moved back to end with the row (columns
 // two lanes then hold come out of both the same).
 // LOOK: X = M + alpha * unsketch(cs), formed here (conef_psgd_look.h).
+// red: the workgroup's place in LDS for the waves' tiles, given by the kernel: one that takes every V has one for all.
 struct MfmaLook {
     const float* cs;         // [n, w]
     const uint32_t* pk;      // bucket and sign of every column
@@ -179,11 +181,10 @@ struct MfmaLook {
 
 template <int V, bool LOOK = false>
 __device__ __forceinline__ void
-psgd_mfma_mtp_body(const float* __restrict__ x, const float* __restrict__ p, float* __restrict__ out, int64_t n, int m,
-                   int r, int rows_per_slab, int bx, int by, MfmaLook look = {})
+psgd_mfma_mtp_body(float (*red)[16][64], const float* __restrict__ x, const float* __restrict__ p, float* __restrict__ out, int64_t n,
+                   int m, int r, int rows_per_slab, int bx, int by, MfmaLook look = {})
 {
-    __shared__ float red[kMfmaWaves][16][64];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int lq = lane & 31, half = lane >> 5;
     const int c0 = bx * 32 * V;
     const int c = c0 + V * lq;
@@ -197,7 +198,9 @@ psgd_mfma_mtp_body(const float* __restrict__ x, const float* __restrict__ p, flo
     for (int t = 0; t < V; ++t)
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[t][v] = 0.f;
-    constexpr int U = V == 4 ? 4 : 8;                  // row pairs per stage
+    // A wave takes 2 UC rows, then those 2 UC kMfmaWaves on; a stage is half of them, which with the tiles of four column runs
+    // and LOOK's cells just fits the registers of four workgroups a CU.
+    constexpr int UC = V == 4 ? 4 : 8, U = UC / 2;
     struct Stage {
         float xv[U][V], pv[U], cv[U][LOOK ? V : 1];
     };
@@ -206,12 +209,17 @@ psgd_mfma_mtp_body(const float* __restrict__ x, const float* __restrict__ p, flo
 #pragma unroll
         for (int t = 0; t < V; ++t) pk[t] = look.pk[cc + t];
     }
+    // A pair of rows is the wave's, so its place is a scalar; a lane adds where it reads from there (rows with a plan of
+    // row lists, which LOOK asks for, are short: 32 bits do).
+    using Offset = std::conditional_t<LOOK, uint32_t, int64_t>;
+    const Offset xo = (Offset)half * (Offset)m + (Offset)cc, po = (Offset)half * (Offset)r + (Offset)(rank_ok ? lq : 0);
     auto load = [&](Stage& st, int64_t ib) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int64_t i = ib + 2 * u + half;
-            const int64_t ii = i < i1 ? i : i0;         // past the slab: a valid row, its products are zeroed
-            const float* src = x + ii * m + cc;
+            // past the slab: a valid row, its products are zeroed
+            const int64_t i = ib + 2 * u < i1 ? ib + 2 * u : i0;
+            const bool second = i + 1 < i1;
+            const float* src = x + i * m + (second ? xo : (Offset)cc);
             if constexpr (V == 4) {
                 conef_ld4u(src, st.xv[u]);
             } else if constexpr (V == 2) {
@@ -220,10 +228,12 @@ psgd_mfma_mtp_body(const float* __restrict__ x, const float* __restrict__ p, flo
             } else {
                 st.xv[u][0] = *src;
             }
-            st.pv[u] = p[ii * r + (rank_ok ? lq : 0)];
+            st.pv[u] = (p + i * r)[second ? po : (Offset)(rank_ok ? lq : 0)];
             if constexpr (LOOK) {
+                const float* cells = look.cs + i * look.w;
+                const uint32_t below = second && half ? (uint32_t)look.w : 0u;
 #pragma unroll
-                for (int t = 0; t < V; ++t) st.cv[u][t] = look.cs[ii * look.w + (pk[t] & 0x7fffffffu)];
+                for (int t = 0; t < V; ++t) st.cv[u][t] = cells[(pk[t] & 0x7fffffffu) + below];
             }
         }
     };
@@ -240,20 +250,17 @@ psgd_mfma_mtp_body(const float* __restrict__ x, const float* __restrict__ p, flo
             for (int t = 0; t < V; ++t) acc[t] = conef_mfma32((ok && col_ok) ? st.xv[u][t] : 0.f, b, acc[t]);
         }
     };
-    constexpr int kStep = 2 * kMfmaWaves * U;
-    int64_t ib = i0 + 2 * wave * U;
+    constexpr int kStep = 2 * kMfmaWaves * UC;
+    int64_t ib = i0 + 2 * wave * UC;
     if (ib < i1) {
         Stage s0, s1;
         load(s0, ib);
         while (true) {
-            int64_t nb = ib + kStep;
-            load(s1, nb < i1 ? nb : ib);
+            const int64_t nb = ib + kStep, hb = ib + 2 * U;
+            if (hb < i1) load(s1, hb);
             compute(s0, ib);
-            if (nb >= i1) break;
-            ib = nb;
-            nb = ib + kStep;
-            load(s0, nb < i1 ? nb : ib);
-            compute(s1, ib);
+            if (nb < i1) load(s0, nb);
+            if (hb < i1) compute(s1, hb);
             if (nb >= i1) break;
             ib = nb;
         }
@@ -282,7 +289,8 @@ __global__ void __launch_bounds__(kMfmaThreads)
 psgd_mfma_mtp_kernel(const float* __restrict__ x, const float* __restrict__ p, float* __restrict__ out, int64_t n, int m,
                      int r, int rows_per_slab)
 {
-    psgd_mfma_mtp_body<V>(x, p, out, n, m, r, rows_per_slab, (int)blockIdx.x, (int)blockIdx.y);
+    __shared__ float red[kMfmaWaves][16][64];
+    psgd_mfma_mtp_body<V>(red, x, p, out, n, m, r, rows_per_slab, (int)blockIdx.x, (int)blockIdx.y);
 }
 
 // ------------------------------------------------------------ M = P Q^T ----
