@@ -838,8 +838,8 @@ psgd_defer_fix_batch_kernel(PsgdBatch<DeferFixItem> b, float alpha)
 }
 
 // ---- ranks 16 and 32 ----
-// The shares of P^T P of a finished P (the matrix-core product leaves P in column splits that a
-// second kernel adds, so they cannot come out of the product itself): a workgroup per 256 rows,
+// The shares of P^T P of a finished P (the matrix-core product leaves P in column splits that another
+// kernel adds, so they cannot come out of the product itself): a workgroup per 256 rows,
 // on the matrix cores in double (the first phase of gsg_kernel).
 struct GramShareItem {
     const float* a;
@@ -860,6 +860,58 @@ psgd_gram_shares_batch_kernel(PsgdBatch<GramShareItem> b)
     gsg_gram_tiles<RP>(it.a, r0, r1, tiles);
     __syncthreads();
     for (int e = threadIdx.x; e < NG; e += kGsgThreads) {
+        int i, j;
+        gsg_entry(e, RP, &i, &j);
+        it.parts[(size_t)local * NG + e] = gsg_tiles_entry<RP>(tiles, i, j);
+    }
+}
+
+// The same where P still lies in column splits: a workgroup adds those of its 256 rows first (the order of
+// psgd_sum_partials_body, the same bits), into P and into LDS, and takes the share from there.  One launch of 9 to 11 us for
+// two of 4.6 and 10.6 with a boundary between them: an encoder of 1024 at rank 32 534 -> 522 us, [1000,2000] at rank 16
+// 60.4 -> 57.  What bounds it is the matrix cores' rate in double (5 us; a wave for each tile, three to a SIMD, took as long).
+constexpr int kSumShareThreads = 1024;
+struct SumShareItem {
+    const float* partial;    // [slabs][rows][RP], or P itself (slabs 1)
+    float* out;
+    int64_t rows;
+    int slabs;
+    double* parts;
+};
+
+template <int RP>
+__global__ void __launch_bounds__(kSumShareThreads)
+psgd_sum_shares_batch_kernel(PsgdBatch<SumShareItem> b)
+{
+    constexpr int NC = RP / 16, NT = NC * (NC + 1) / 2, NG = RP * (RP + 1) / 2, QPR = RP / 4;
+    __shared__ double tiles[kGsgThreads / 64][NT][256];
+    __shared__ __align__(16) float rows_l[256 * RP];
+    int local;
+    const SumShareItem& it = b.item[psgd_batch_locate(b, &local)];
+    const int64_t r0 = (int64_t)local * 256;
+    const int rows = r0 + 256 < it.rows ? 256 : (int)(it.rows - r0), slabs = it.slabs;
+    const float* src = it.partial + r0 * RP;
+    const int64_t step = it.rows * RP;
+    for (int e = threadIdx.x; e < rows * QPR; e += kSumShareThreads) {
+        float s[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int k0 = 0; k0 < slabs; k0 += 8) {             // eight loads in flight, added in slab order
+            float v[8][4];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) conef_ld4u(src + (k0 + u < slabs ? k0 + u : k0) * step + 4 * e, v[u]);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                if (k0 + u >= slabs) continue;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) s[j] += v[u][j];
+            }
+        }
+        if (slabs > 1) conef_st4u(it.out + r0 * RP + 4 * e, s);
+        *reinterpret_cast<float4*>(&rows_l[4 * e]) = make_float4(s[0], s[1], s[2], s[3]);
+    }
+    __syncthreads();
+    if (threadIdx.x < kGsgThreads) gsg_gram_tiles<RP>(rows_l, 0, rows, tiles);
+    __syncthreads();
+    for (int e = threadIdx.x; e < NG; e += kSumShareThreads) {
         int i, j;
         gsg_entry(e, RP, &i, &j);
         it.parts[(size_t)local * NG + e] = gsg_tiles_entry<RP>(tiles, i, j);
@@ -2918,9 +2970,16 @@ inline int rows_per_query_block(int64_t n, int64_t col_blocks)
 // once the batch as a whole has workgroups to spare
 inline int mq_rows_per_wg(int64_t total_rows) { return total_rows / 4 >= 256 ? 4 : 1; }
 
+// where a product lies in parts that are still to be added: [slabs][rows][RP], or the finished factor (one slab)
+struct MtpRaw {
+    const float* src;
+    int slabs;
+};
+
+// outs: the column splits of a product on the matrix cores are left there.
 template <int MODE>
 int mq_batch(const ConefPsgdItem* items, int count, float alpha, int32_t a, int32_t b, void* workspace,
-             int64_t workspace_bytes, hipStream_t s)
+             int64_t workspace_bytes, hipStream_t s, std::vector<MtpRaw>* outs = nullptr)
 {
     ConefSeeds hs = {a, b, a + 2, b + 3};
     std::vector<char> done((size_t)count, 0);
@@ -2969,7 +3028,8 @@ int mq_batch(const ConefPsgdItem* items, int count, float alpha, int32_t a, int3
                                 g.splits, conef_make_mod(1)};
                 table.push_back(t);
                 blocks.push_back(g.row_tiles * g.splits);
-                if (g.splits > 1) {
+                if (outs) (*outs)[(size_t)j] = MtpRaw{out, g.splits};
+                if (g.splits > 1 && !outs) {
                     const int64_t cnt = it.n * it.r;
                     SumItem si = {out, it.p, cnt, g.splits};
                     sums.push_back(si);
@@ -3091,11 +3151,6 @@ inline int64_t mtp_batch_layout(const ConefPsgdItem* items, int count, std::vect
 // matrices' Gram systems, and the row-slab partials are left for the caller's fix launch instead
 // of being added here; outs[k] then says where item k's raw Q is ([slabs][m][r]).  Only for a batch
 // that is one launch of this kernel (one rank below 16, all items 16-byte shaped or none).
-struct MtpRaw {
-    const float* src;
-    int slabs;
-};
-
 int mtp_batch(const ConefPsgdItem* items, int count, void* workspace, int64_t workspace_bytes, hipStream_t s,
               const GramTask* gram = nullptr, std::vector<MtpRaw>* outs = nullptr, const std::vector<MfmaLook>* look = nullptr)
 {
@@ -3486,11 +3541,33 @@ int round_products_deferred(const PaddedRound& pr, int r, float* const* q_in, fl
     return defer_fix(pr, r, raw, tmats, q_shares ? &qgrams : nullptr, s);
 }
 
+// conef_psgd_mq_batch_f32
+int mq_batch_any(const ConefPsgdItem* items, int count, int mode, float alpha, int32_t a, int32_t b, void* workspace,
+                 int64_t workspace_bytes, hipStream_t s, std::vector<MtpRaw>* outs = nullptr)
+{
+    if (count < 0 || (count > 0 && !items) || mode < 0 || mode > 2) return CONEF_ERR_INVALID;
+    for (int k = 0; k < count; ++k) {
+        const ConefPsgdItem& it = items[k];
+        if (!item_ok(it) || (mode == 1 && !it.err) || (mode == 2 && (!it.cs || it.w < 1 || it.w > (1 << 30))))
+            return CONEF_ERR_INVALID;
+        if (mode == 2 && it.plan_host && !conef_plan_matches((const ConefPlanHeader*)it.plan_host, it.n, it.m, it.w, a, b))
+            return CONEF_ERR_INVALID;
+    }
+    if (mode == 0) return mq_batch<0>(items, count, 0.f, a, b, workspace, workspace_bytes, s, outs);
+    if (mode == 1) return mq_batch<1>(items, count, 0.f, a, b, workspace, workspace_bytes, s, outs);
+    return mq_batch<2>(items, count, alpha, a, b, workspace, workspace_bytes, s, outs);
+}
+
+// The sums ride with the shares up to 16 splits, which is 512 KB for a workgroup of 256 rows; with 64 it would be 2 MB, and
+// the launch that adds them alone has the whole machine.
+constexpr int kSumShareSplits = 16;
+
 // The same for ranks 9 to 32, whose products run on the matrix cores: the shares of P^T P come
-// from a short launch of their own over the finished P, the systems ride in the second product's
+// from a short launch of their own, which also adds the column splits of P, the systems ride in the second product's
 // first launch, and the fix launch is the wide form.  `mq_mode` as in conef_psgd_mq_batch_f32.
 // look: X = M + alpha * unsketch(cs) is formed where it is read, and M stays as it is.
-int look_mq(const std::vector<ConefPsgdItem>& items, float alpha, void* workspace, int64_t workspace_bytes, hipStream_t s);
+int look_mq(const std::vector<ConefPsgdItem>& items, float alpha, void* workspace, int64_t workspace_bytes, hipStream_t s,
+            std::vector<MtpRaw>* outs);
 
 int round_products_deferred_mfma(const PaddedRound& pr, int r, float* const* q_in, int mq_mode, float alpha, float eps,
                                  int32_t a, int32_t b, void* workspace, int64_t workspace_bytes, hipStream_t s,
@@ -3500,10 +3577,17 @@ int round_products_deferred_mfma(const PaddedRound& pr, int r, float* const* q_i
     const int count = (int)pr.items.size(), rp = pr.rp;
     std::vector<ConefPsgdItem> first(pr.items);
     for (int k = 0; k < count; ++k) first[(size_t)k].q = q_in[k];
-    int rc = look ? look_mq(first, alpha, workspace, workspace_bytes, s)
-                  : conef_psgd_mq_batch_f32(first.data(), count, mq_mode, alpha, a, b, workspace, workspace_bytes, (void*)s);
+    int most = 1;
+    for (const ConefPsgdItem& it : first) most = std::max(most, mfma_mq_shape(it.n, it.m).splits);
+    std::vector<MtpRaw> splits;
+    if (most <= kSumShareSplits)
+        for (const ConefPsgdItem& it : first) splits.push_back(MtpRaw{it.p, 1});
+    std::vector<MtpRaw>* const left = splits.empty() ? nullptr : &splits;
+    int rc = look ? look_mq(first, alpha, workspace, workspace_bytes, s, left)
+                  : mq_batch_any(first.data(), count, mq_mode, alpha, a, b, workspace, workspace_bytes, s, left);
     if (rc != CONEF_OK) return rc;
     std::vector<GramShareItem> shares;
+    std::vector<SumShareItem> sum_shares;
     std::vector<int> share_blocks;
     std::vector<float*> tmats;
     GramTask gram;
@@ -3514,7 +3598,8 @@ int round_products_deferred_mfma(const PaddedRound& pr, int r, float* const* q_i
     for (int k = 0; k < count; ++k) {
         const ConefPsgdItem& it = items[k];
         const int nb = (int)((it.n + 255) / 256);
-        shares.push_back(GramShareItem{it.p, it.n, (double*)at});
+        if (left) sum_shares.push_back(SumShareItem{splits[(size_t)k].src, it.p, it.n, splits[(size_t)k].slabs, (double*)at});
+        else shares.push_back(GramShareItem{it.p, it.n, (double*)at});
         share_blocks.push_back(nb);
         gram.parts[k] = (const double*)at;
         gram.nparts[k] = nb;
@@ -3523,10 +3608,16 @@ int round_products_deferred_mfma(const PaddedRound& pr, int r, float* const* q_i
         gram.tmat[k] = (float*)at;
         at += defer_tmat_bytes(rp) + conef_align256(8 * defer_qgram_doubles(it));
     }
-    rc = run_batches(shares, share_blocks, [&](const PsgdBatch<GramShareItem>& bt, int grid) {
-        if (rp == 32) conef_launch(psgd_gram_shares_batch_kernel<32>, dim3((unsigned)grid), dim3(kGsgThreads), 0, s, bt);
-        else conef_launch(psgd_gram_shares_batch_kernel<16>, dim3((unsigned)grid), dim3(kGsgThreads), 0, s, bt);
-    });
+    if (left)
+        rc = run_batches(sum_shares, share_blocks, [&](const PsgdBatch<SumShareItem>& bt, int grid) {
+            if (rp == 32) conef_launch(psgd_sum_shares_batch_kernel<32>, dim3((unsigned)grid), dim3(kSumShareThreads), 0, s, bt);
+            else conef_launch(psgd_sum_shares_batch_kernel<16>, dim3((unsigned)grid), dim3(kSumShareThreads), 0, s, bt);
+        });
+    else
+        rc = run_batches(shares, share_blocks, [&](const PsgdBatch<GramShareItem>& bt, int grid) {
+            if (rp == 32) conef_launch(psgd_gram_shares_batch_kernel<32>, dim3((unsigned)grid), dim3(kGsgThreads), 0, s, bt);
+            else conef_launch(psgd_gram_shares_batch_kernel<16>, dim3((unsigned)grid), dim3(kGsgThreads), 0, s, bt);
+        });
     if (rc != CONEF_OK) return rc;
     std::vector<MtpRaw> raw((size_t)count);
     rc = mtp_batch(items, count, workspace, workspace_bytes, s, &gram, &raw, look);
@@ -4612,7 +4703,8 @@ inline bool look_pays(const ConefPsgdItem* items, int count)
     return widths <= 320. * values && (cells <= 0.35 * values || values <= 4e6) && look_mq_shape(items, count, &g);
 }
 
-int look_mq(const std::vector<ConefPsgdItem>& items, float alpha, void* workspace, int64_t workspace_bytes, hipStream_t s)
+int look_mq(const std::vector<ConefPsgdItem>& items, float alpha, void* workspace, int64_t workspace_bytes, hipStream_t s,
+            std::vector<MtpRaw>* outs)
 {
     const int count = (int)items.size();
     std::vector<int64_t> offs;
@@ -4629,7 +4721,8 @@ int look_mq(const std::vector<ConefPsgdItem>& items, float alpha, void* workspac
         float* out = g.splits > 1 ? partials + offs[(size_t)k] : it.p;
         table.push_back(LookMqItem{it.x, it.cs, item_pktab(it), it.q, out, it.n, (int)it.m, it.r, it.w, g.cols_per_split, g.splits});
         blocks.push_back(g.row_tiles * ((g.splits + shape.groups - 1) / shape.groups));
-        if (g.splits > 1) {
+        if (outs) (*outs)[(size_t)k] = MtpRaw{out, g.splits};
+        if (g.splits > 1 && !outs) {
             sums.push_back(SumItem{out, it.p, it.n * it.r, g.splits});
             sum_blocks.push_back((int)((it.n * it.r + 255) / 256));
         }
@@ -4715,18 +4808,7 @@ int64_t conef_psgd_batch_workspace_bytes(const ConefPsgdItem* items, int32_t cou
 int conef_psgd_mq_batch_f32(const ConefPsgdItem* items, int32_t count, int32_t mode, float alpha, int32_t a, int32_t b,
                             void* workspace, int64_t workspace_bytes, void* stream)
 {
-    if (count < 0 || (count > 0 && !items) || mode < 0 || mode > 2) return CONEF_ERR_INVALID;
-    for (int k = 0; k < count; ++k) {
-        const ConefPsgdItem& it = items[k];
-        if (!item_ok(it) || (mode == 1 && !it.err) || (mode == 2 && (!it.cs || it.w < 1 || it.w > (1 << 30))))
-            return CONEF_ERR_INVALID;
-        if (mode == 2 && it.plan_host && !conef_plan_matches((const ConefPlanHeader*)it.plan_host, it.n, it.m, it.w, a, b))
-            return CONEF_ERR_INVALID;
-    }
-    hipStream_t s = (hipStream_t)stream;
-    if (mode == 0) return mq_batch<0>(items, count, 0.f, a, b, workspace, workspace_bytes, s);
-    if (mode == 1) return mq_batch<1>(items, count, 0.f, a, b, workspace, workspace_bytes, s);
-    return mq_batch<2>(items, count, alpha, a, b, workspace, workspace_bytes, s);
+    return mq_batch_any(items, count, mode, alpha, a, b, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 int conef_psgd_mtp_batch_f32(const ConefPsgdItem* items, int32_t count, void* workspace, int64_t workspace_bytes,
