@@ -3558,9 +3558,11 @@ int mq_batch_any(const ConefPsgdItem* items, int count, int mode, float alpha, i
     return mq_batch<2>(items, count, alpha, a, b, workspace, workspace_bytes, s, outs);
 }
 
-// The sums ride with the shares up to 16 splits, which is 512 KB for a workgroup of 256 rows; with 64 it would be 2 MB, and
-// the launch that adds them alone has the whole machine.
-constexpr int kSumShareSplits = 16;
+// Whether the sums ride with the shares.  A workgroup adds the splits of its 256 rows alone: 512 KB for 32 splits of rank 16
+// or 16 of rank 32.  A launch of their own and this, us: rank 16 [512,4096] (32 splits) 73.5 and 71.0, [256,8192] (64) 77.3 and
+// 74.9, [128,20000] 78.1 and 74.3; rank 32 [1024,4096] (16) 108 and 105.9, [512,4096] (32) 101.1 and 102.6, [256,8192] (64)
+// 100.8 and 110.7.
+inline bool sums_with_shares(int splits, int rp) { return rp == 16 || splits <= 16; }
 
 // The same for ranks 9 to 32, whose products run on the matrix cores: the shares of P^T P come
 // from a short launch of their own, which also adds the column splits of P, the systems ride in the second product's
@@ -3580,7 +3582,7 @@ int round_products_deferred_mfma(const PaddedRound& pr, int r, float* const* q_i
     int most = 1;
     for (const ConefPsgdItem& it : first) most = std::max(most, mfma_mq_shape(it.n, it.m).splits);
     std::vector<MtpRaw> splits;
-    if (most <= kSumShareSplits)
+    if (sums_with_shares(most, rp))
         for (const ConefPsgdItem& it : first) splits.push_back(MtpRaw{it.p, 1});
     std::vector<MtpRaw>* const left = splits.empty() ? nullptr : &splits;
     int rc = look ? look_mq(first, alpha, workspace, workspace_bytes, s, left)
