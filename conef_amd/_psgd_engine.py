@@ -138,7 +138,7 @@ class _RoundPlan:
     arenas.  Built on the first step of a bucket and reused while the bucket keeps its buffer
     and layout, so that a step costs a handful of foreign calls however many tensors it has."""
     __slots__ = ("small", "layout", "cells", "cs_static", "env_ahead", "env_topk_side", "env_small", "check_gs", "tape", "key", "shapes", "work", "passthrough", "before", "after", "total_ps", "total_qs", "arena_key", "ps",
-                 "qs", "items", "count", "sketches", "fused_sketch", "batched_update", "residual_offsets",
+                 "qs", "items", "count", "sketches", "fused_sketch", "fused_order", "batched_update", "residual_offsets",
                  "topk_table", "q_next", "q_next_ptrs", "q_next_ready", "q_next_made", "made", "q_next_event", "aside_recorded",
                  "topk_event", "ws_need", "handoff_event", "topk_number", "q_next_number", "is_wide", "wide", "chunks", "runs", "ef_spans")
 
@@ -224,6 +224,7 @@ def _build_round(state, grads, shapes, key, error_mode):
     plan.small = None               # (mode1, mode3) -> whether the bucket's round runs as one launch (a bucket of small matrices)
     plan.sketches = []
     plan.fused_sketch = False
+    plan.fused_order = None         # the order of steps it was decided for
     plan.batched_update = False
     plan.topk_table = None
     plan.topk_event = None          # the side stream's top-k of this bucket's errors, to be waited for by its next round
@@ -474,11 +475,16 @@ def _run_round(state, bucket, input_tensor, error_mode, streams):
             plan.cells = _host.same_sketches(errs.values(), moves + [True] * (len(errs) - count))
             for cnt, (cs, _) in enumerate(plan.sketches):
                 items[cnt].cs = cs.cs.data_ptr()
-            plan.fused_sketch = plan.batched_update and (state.matrix_approximation_rank <= 8 or not plan.is_wide and all(
-                lib.conef_psgd_round_wide_sketch_fits(run, part, HASH_A, HASH_B) for run, part in plan.runs))
+            plan.fused_order = None
         if not plan.cs_static:
             for cnt, (cs, _) in enumerate(plan.sketches):
                 items[cnt].cs = cs.cs.data_ptr()
+        # above rank 8 also a matter of the order of steps, which may be switched from step to step
+        order = lib.conef_psgd_round_in_order() if state.matrix_approximation_rank > 8 else 0
+        if plan.fused_order != order:
+            plan.fused_order = order
+            plan.fused_sketch = plan.batched_update and (state.matrix_approximation_rank <= 8 or not plan.is_wide and all(
+                lib.conef_psgd_round_wide_sketch_fits(run, part, HASH_A, HASH_B) for run, part in plan.runs))
     elif error_mode == "conef_v2":
         for cnt, (matrix, n, m, rank) in enumerate(work):
             if cnt not in errs:

@@ -5109,6 +5109,8 @@ int conef_psgd_q_next_f32(const ConefPsgdItem* items, int32_t count, float eps, 
     return rc;
 }
 
+int conef_psgd_round_in_order(void) { return order_asked() ? 1 : 0; }
+
 // Whether a round with a sketched error at ranks 9 to 32 sketches the residuals in its last launch (pqt_mode 2).
 int conef_psgd_round_wide_sketch_fits(const ConefPsgdItem* items, int32_t count, int32_t a, int32_t b)
 {

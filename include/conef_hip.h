@@ -377,6 +377,9 @@ int conef_psgd_round_small_f32(const ConefPsgdItem* items, int32_t count, int32_
  * columns or more, a row-list plan per sketch for the seeds a and b, no CONEF_ROUND_DEFER=0), 0 where pqt_mode 3 with room for dense residuals is the
  * faster call.  conef_psgd_batch_workspace_bytes covers what it needs. */
 int conef_psgd_round_wide_sketch_fits(const ConefPsgdItem* items, int32_t count, int32_t a, int32_t b);
+/* 1 where CONEF_ROUND_DEFER=0 asks for the reference's order of steps as things stand, else 0: a caller that keeps the
+ * answer of conef_psgd_round_wide_sketch_fits asks again where this has changed. */
+int conef_psgd_round_in_order(void);
 
 /* The middle of that round as a call of its own, for a caller that splits the round: P = X Q with the Q
  * factors of `first` (a copy of `items` whose q may point elsewhere; null: items' own), P orthogonalised
