@@ -216,8 +216,14 @@ psgd_mfma_mtp_body(float (*red)[16][64], const float* __restrict__ x, const floa
     const int c = c0 + V * lq;
     const bool col_ok = c < m;
     const int cc = col_ok ? (c + V <= m ? c : m - V) : 0;
+    // Rows are counted from the slab's first, in 32 bits: a wave's place is a scalar, and 64-bit compares and selections of scalars
+    // are chains of instructions, ahead of a stage's loads.  Rank 32, us, with 64 bits and so: [1024,1024] 7.3 and 6.9, [300,9000]
+    // 11.6 and 11.0, [4096,4096] 24.5 and 23.5, [30522,1024] 39.3 and 37.6 (a lane's own 64-bit place: 6.9, 11.0, 25.3, 40.7).
     const int64_t i0 = (int64_t)by * rows_per_slab;
-    const int64_t i1 = i0 + rows_per_slab < n ? i0 + rows_per_slab : n;
+    const int rows = i0 + rows_per_slab < n ? rows_per_slab : (int)(n - i0);
+    x += i0 * m;
+    p += i0 * r;
+    const float* const slab_cells = LOOK ? look.cs + i0 * look.w : nullptr;
     const bool rank_ok = lq < r;
     conef_f16v acc[V];
 #pragma unroll
@@ -225,7 +231,7 @@ psgd_mfma_mtp_body(float (*red)[16][64], const float* __restrict__ x, const floa
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[t][v] = 0.f;
     // A wave takes 2 UC rows, then those 2 UC kMfmaWaves on; a stage is half of them, which with the tiles of four column runs
-    // and LOOK's cells just fits the registers of four workgroups a CU.
+    // and LOOK's cells fits the registers of four workgroups a CU (124 and 126 of 128 at ranks 16 and 32).
     constexpr int UC = V == 4 ? 4 : 8, U = UC / 2;
     struct Stage {
         float xv[U][V], pv[U], cv[U][LOOK ? V : 1];
@@ -239,13 +245,13 @@ psgd_mfma_mtp_body(float (*red)[16][64], const float* __restrict__ x, const floa
     // row lists, which LOOK asks for, are short: 32 bits do).
     using Offset = std::conditional_t<LOOK, uint32_t, int64_t>;
     const Offset xo = (Offset)half * (Offset)m + (Offset)cc, po = (Offset)half * (Offset)r + (Offset)(rank_ok ? lq : 0);
-    auto load = [&](Stage& st, int64_t ib) {
+    auto load = [&](Stage& st, int ib) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             // past the slab: a valid row, its products are zeroed
-            const int64_t i = ib + 2 * u < i1 ? ib + 2 * u : i0;
-            const bool second = i + 1 < i1;
-            const float* src = x + i * m + (second ? xo : (Offset)cc);
+            const int i = ib + 2 * u < rows ? ib + 2 * u : 0;
+            const bool second = i + 1 < rows;
+            const float* src = x + (int64_t)i * m + (second ? xo : (Offset)cc);
             if constexpr (V == 4) {
                 conef_ld4u(src, st.xv[u]);
             } else if constexpr (V == 2) {
@@ -254,19 +260,19 @@ psgd_mfma_mtp_body(float (*red)[16][64], const float* __restrict__ x, const floa
             } else {
                 st.xv[u][0] = *src;
             }
-            st.pv[u] = (p + i * r)[second ? po : (Offset)(rank_ok ? lq : 0)];
+            st.pv[u] = (p + (int64_t)i * r)[second ? po : (Offset)(rank_ok ? lq : 0)];
             if constexpr (LOOK) {
-                const float* cells = look.cs + i * look.w;
+                const float* cells = slab_cells + (int64_t)i * look.w;
                 const uint32_t below = second && half ? (uint32_t)look.w : 0u;
 #pragma unroll
                 for (int t = 0; t < V; ++t) st.cv[u][t] = cells[(pk[t] & 0x7fffffffu) + below];
             }
         }
     };
-    auto compute = [&](Stage& st, int64_t ib) {
+    auto compute = [&](Stage& st, int ib) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const bool ok = ib + 2 * u + half < i1;
+            const bool ok = ib + 2 * u + half < rows;
             if constexpr (LOOK) {
 #pragma unroll
                 for (int t = 0; t < V; ++t) st.xv[u][t] = __fadd_rn(st.xv[u][t], conef_query_term(st.cv[u][t], pk[t], look.alpha));
@@ -277,17 +283,17 @@ psgd_mfma_mtp_body(float (*red)[16][64], const float* __restrict__ x, const floa
         }
     };
     constexpr int kStep = 2 * kMfmaWaves * UC;
-    int64_t ib = i0 + 2 * wave * UC;
-    if (ib < i1) {
+    int ib = 2 * wave * UC;
+    if (ib < rows) {
         Stage s0, s1;
         load(s0, ib);
         while (true) {
-            const int64_t nb = ib + kStep, hb = ib + 2 * U;
-            if (hb < i1) load(s1, hb);
+            const int nb = ib + kStep, hb = ib + 2 * U;
+            if (hb < rows) load(s1, hb);
             compute(s0, ib);
-            if (nb < i1) load(s0, nb);
-            if (hb < i1) compute(s1, hb);
-            if (nb >= i1) break;
+            if (nb < rows) load(s0, nb);
+            if (hb < rows) compute(s1, hb);
+            if (nb >= rows) break;
             ib = nb;
         }
     }
