@@ -122,6 +122,54 @@ int rb_run(const std::vector<Item>& table, const std::vector<int>& blocks, Go go
     return rb_run_cap<Item, rb_batch_max<Item>()>(table, blocks, go);
 }
 
+inline bool by_row_list(const ConefRandBlockItem& it)
+{
+    const ConefPlanHeader* hp = (const ConefPlanHeader*)it.plan_host;
+    return hp && hp->kind == kConefPlanRowlist;
+}
+
+// How a launch takes the tensors on row lists of a sketched step.
+struct ListTiles {
+    std::vector<ConefRowlistShape> shapes;      // of those tensors, in order
+    size_t lds;
+    int threads;
+};
+
+inline bool list_tiles(const ConefRandBlockItem* items, int count, ListTiles* lt)
+{
+    std::vector<ConefRowlistShape> taller;
+    std::vector<double> values;
+    size_t lds = 0;
+    for (int k = 0; k < count; ++k) {
+        const ConefRandBlockItem& it = items[k];
+        if (!by_row_list(it)) continue;
+        ConefRowlistShape shape;
+        if (!conef_rowlist_shape(it.n, it.m, it.w, ConefListRandBlock::kNeedsCells, ConefListRandBlock::halves(it.m), &shape)) return false;
+        lt->shapes.push_back(shape);
+        conef_rowlist_taller(it.n, it.m, it.w, ConefListRandBlock::kNeedsCells, &shape);
+        taller.push_back(shape);
+        values.push_back((double)it.n * (double)it.m);
+        lds = std::max(lds, shape.lds);
+    }
+    // A launch gives every tile the LDS of its largest: taller ones where half the values are in tiles of half of that.
+    // Steps with one row by 256 threads and so, us: WRN-28-10 with sketches of 0.05 and 0.5 192 and 172, 325 and 242,
+    // an LSTM of 500 and one of 300 66 and 53, 34 and 21, an encoder of 1024 with 0.2 327 and 302.
+    double all = 0., large = 0.;
+    for (size_t k = 0; k < values.size(); ++k) {
+        all += values[k];
+        if (2 * taller[k].lds >= lds) large += values[k];
+    }
+    if (2. * large >= all) lt->shapes = taller;
+    lt->lds = 0;
+    int64_t tiles = 0;
+    for (const ConefRowlistShape& t : lt->shapes) {
+        tiles += t.tiles;
+        lt->lds = std::max(lt->lds, t.lds);
+    }
+    lt->threads = values.empty() ? 0 : conef_rowlist_workgroup(lt->lds, tiles, all, ConefListRandBlock::kLeastValues);
+    return true;
+}
+
 }  // namespace
 
 extern "C" {
@@ -175,49 +223,22 @@ int conef_randblock_step_batch_f32(const ConefRandBlockItem* items, int32_t coun
     }
     // sketched error: row-list plans share launches, the rest go one by one
     std::vector<ListItem> table;
-    std::vector<ConefRowlistShape> shapes, taller;
     for (int k = 0; k < count; ++k) {
         const ConefRandBlockItem& it = items[k];
-        const ConefPlanHeader* hp = (const ConefPlanHeader*)it.plan_host;
-        if (!hp || hp->kind != kConefPlanRowlist) continue;
-        ConefRowlistShape shape;
-        if (!conef_rowlist_shape(it.n, it.m, it.w, ConefListRandBlock::kNeedsCells, ConefListRandBlock::halves(it.m), &shape)) return CONEF_ERR_INVALID;
-        shapes.push_back(shape);
-        conef_rowlist_taller(it.n, it.m, it.w, ConefListRandBlock::kNeedsCells, &shape);
-        taller.push_back(shape);
+        if (!by_row_list(it)) continue;
         table.push_back(ListItem{it.x, it.payload, conef_make_block(it.n * it.m, it.start, it.block), alpha,
-                                 conef_rowlist_view(hp, it.plan_dev), it.cs_in, it.cs_out, it.n, (int)it.m, it.w, 0, false});
+                                 conef_rowlist_view((const ConefPlanHeader*)it.plan_host, it.plan_dev), it.cs_in, it.cs_out, it.n,
+                                 (int)it.m, it.w, 0, false});
     }
+    ListTiles tiles;
+    if (!list_tiles(items, count, &tiles)) return CONEF_ERR_INVALID;
     if (!table.empty()) {
-        // A launch gives every tile the LDS of its largest: taller ones where half the values are in tiles of half of that.
-        // Steps with one row by 256 threads and so, us: WRN-28-10 with sketches of 0.05 and 0.5 192 and 172, 325 and 242,
-        // an LSTM of 500 and one of 300 66 and 53, 34 and 21, an encoder of 1024 with 0.2 327 and 302.
-        size_t lds = 0;
-        for (const ConefRowlistShape& t : taller) lds = std::max(lds, t.lds);
-        double values = 0., large = 0.;
-        for (size_t k = 0; k < table.size(); ++k) {
-            const double v = (double)table[k].n * (double)table[k].d;
-            values += v;
-            if (2 * taller[k].lds >= lds) large += v;
-        }
-        // (and not where tiles of two rows fill the machine already: the LSTM's three [2600,650] 17.6 us by 3900 of those,
-        // 18.3 by 1950 of four)
-        int64_t flat = 0;
-        int least = shapes[0].rb;
-        for (const ConefRowlistShape& t : shapes) {
-            flat += t.tiles;
-            least = std::min(least, t.rb);
-        }
-        if (2. * large >= values && (least < 2 || flat < 2048)) shapes = taller;
-        lds = 0;
-        int64_t tiles = 0;
+        const size_t lds = tiles.lds;
         std::vector<int> blocks;
         for (size_t k = 0; k < table.size(); ++k) {
-            table[k].rb = shapes[k].rb;
-            table[k].pk_lds = shapes[k].pk_lds;
-            blocks.push_back((int)shapes[k].tiles);
-            tiles += shapes[k].tiles;
-            lds = std::max(lds, shapes[k].lds);
+            table[k].rb = tiles.shapes[k].rb;
+            table[k].pk_lds = tiles.shapes[k].pk_lds;
+            blocks.push_back((int)tiles.shapes[k].tiles);
         }
         const double omb = 1. - (double)beta;
         auto with = [&](auto threads) {
@@ -231,7 +252,7 @@ int conef_randblock_step_batch_f32(const ConefRandBlockItem* items, int32_t coun
             return e != hipSuccess ? (int)e : rc;
         };
         int rc;
-        switch (conef_rowlist_workgroup(lds, tiles, values, ConefListRandBlock::kLeastValues)) {
+        switch (tiles.threads) {
             case 256: rc = with(std::integral_constant<int, 256>()); break;
             case 512: rc = with(std::integral_constant<int, 512>()); break;
             default: rc = with(std::integral_constant<int, 1024>()); break;
@@ -240,10 +261,9 @@ int conef_randblock_step_batch_f32(const ConefRandBlockItem* items, int32_t coun
     }
     for (int k = 0; k < count; ++k) {
         const ConefRandBlockItem& it = items[k];
-        const ConefPlanHeader* hp = (const ConefPlanHeader*)it.plan_host;
-        if (hp && hp->kind == kConefPlanRowlist) continue;
+        if (by_row_list(it)) continue;
         int rc;
-        if (hp)
+        if (it.plan_host)
             rc = conef_randblock_conef_step_planned_f32(it.x, it.cs_in, it.cs_out, it.payload, it.plan_host, it.plan_dev,
                                                         it.staging, it.n, it.m, it.w, it.start, it.block, alpha, beta, a,
                                                         b, stream);
@@ -252,6 +272,23 @@ int conef_randblock_step_batch_f32(const ConefRandBlockItem* items, int32_t coun
                                                 it.block, alpha, beta, a, b, stream);
         if (rc != CONEF_OK) return rc;
     }
+    return CONEF_OK;
+}
+
+// Host only.
+int conef_randblock_step_tiles(const ConefRandBlockItem* items, int32_t count, int32_t a, int32_t b, int32_t* rows, int32_t* threads)
+{
+    if (count < 0 || (count > 0 && (!items || !rows)) || !threads) return CONEF_ERR_INVALID;
+    for (int k = 0; k < count; ++k) {
+        const ConefRandBlockItem& it = items[k];
+        if (it.n < 1 || it.m < 1 || it.m > 0x7fffffffLL || it.w < 1 || it.w > (1 << 30)) return CONEF_ERR_INVALID;
+        if (it.plan_host && !conef_plan_matches((const ConefPlanHeader*)it.plan_host, it.n, it.m, it.w, a, b)) return CONEF_ERR_INVALID;
+    }
+    ListTiles tiles;
+    if (!list_tiles(items, count, &tiles)) return CONEF_ERR_INVALID;
+    size_t at = 0;
+    for (int k = 0; k < count; ++k) rows[k] = by_row_list(items[k]) ? tiles.shapes[at++].rb : 0;
+    *threads = tiles.threads;
     return CONEF_OK;
 }
 

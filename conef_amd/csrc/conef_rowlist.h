@@ -107,11 +107,20 @@ inline bool conef_rowlist_shape(int64_t n, int64_t d, int32_t w, bool cells, boo
 //   [2000,9000]         37.4  25.9   95.8  48.1       37.1  25.3   95.7  46.7       68.1  47.7  153.8  64.4
 //   [2000,12000]        71.4  34.8  124.2  73.7       71.3  34.2  124.8  71.5      138.6  60.3  194.7  93.5
 // Over 354 such shapes (rows of 600 to 20000, 64 to 4096 of them) a third less on average, one 7 % more (0.5 us).
+// A random-block step (cells) whose tiles have two rows stays as it is: its old cells and the column table lie in LDS too, and four
+// rows of a long matrix leave a CU too few tiles.  Two or three rows and four, us, buffers out of the caches, sketches of 0.1 and of 0.4:
+//   [2600,650]    9.4   9.5   10.2  10.8      three of them  19.9  21.0   21.4  24.4
+//   [2600,1000]  11.4  12.4   12.3  13.4      [2048,2502]    17.3  19.4   21.0  20.8
+//   [3400,800]   11.4  13.9   13.3  15.8      [16000,1500]   56.9  71.4   87.6  93.0
+// (Over 110 shapes of 2048 to 16000 rows 3 % less than four rows, against one workgroup size for all 7 % less and 5 % more at
+// worst, where four rows were 26 % more.  Updates of such shapes by four rows are 3 % faster.)
 inline void conef_rowlist_taller(int64_t n, int64_t d, int32_t w, bool cells, ConefRowlistShape* s)
 {
+    if (cells && s->rb >= 2) return;
     for (int rb = 4; rb >= 2; rb -= 2) {
         if (s->rb >= rb) return;
-        // (two rows of [640,5760] in a random-block step of WRN-28-10: 200 us, one row by 512 threads 186)
+        // (cells, rows of more than 2048 columns: two rows of [640,5760] 15.8 us, one row by 512 threads 14.2, [640,4096] 12.2 and
+        // 11.2, [260,4096] 9.3 and 8.2; three [640,2880] in a launch 18.2 and 20.0, [640,9000] 21.1 and 24.0)
         if (n < (int64_t)rb * (cells && (rb == 4 || d > 2048) ? 400 : rb == 4 ? 200 : 128)) continue;
         const size_t lds = conef_rowlist_lds(rb, d, w, cells), pk = cells ? conef_rowlist_pk_bytes(d) : 0;
         if (lds > kConefRowlistLdsLimit) continue;

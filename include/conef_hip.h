@@ -226,6 +226,10 @@ typedef struct ConefRandBlockItem {
  * (and the query loop RandomBlock_hook.py:171-193) for a whole bucket. */
 int conef_randblock_step_batch_f32(const ConefRandBlockItem* items, int32_t count, int32_t mode, float alpha,
                                    float beta, int32_t a, int32_t b, void* stream);
+/* How that call (mode 2) would deal out the tensors whose sketches are on row lists: rows[k] rows of tensor k to a
+ * workgroup (0: another way) of *threads threads (0: no such tensor).  Reads the items' sizes and plan_host; host only. */
+int conef_randblock_step_tiles(const ConefRandBlockItem* items, int32_t count, int32_t a, int32_t b, int32_t* rows,
+                               int32_t* threads);
 
 /* ------------------------------------------------------------------ PowerSGD ---------- */
 /* M is [n,m], Q is [m,r], P is [n,r], 1 <= r <= 32. */

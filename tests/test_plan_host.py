@@ -238,3 +238,37 @@ def test_plan_argument_checks():
     buf = np.zeros(64, np.uint8)
     assert lib.conef_plan_build_host(buf.ctypes.data, 64, 5, 1000, 100, A, B, 0, 0) == -1   # buffer too small
     assert lib.conef_plan_workspace_bytes(buf.ctypes.data) == -1                            # not a plan
+
+
+def step_tiles(shapes, ss):
+    """(rows of a tile per tensor, threads of a workgroup) of a sketched random-block step over these tensors."""
+    import ctypes
+
+    from conef_amd import _lib
+    lib = _lib.load()
+    items, keep = (_lib.RandBlockItem * len(shapes))(), []
+    for it, (n, d) in zip(items, shapes):
+        it.n, it.m, it.w = n, d, max(1, int(ss * d))
+        buf = np.zeros(lib.conef_plan_bytes(n, d, it.w, 0, 0), np.uint8)
+        assert lib.conef_plan_build_host(buf.ctypes.data, buf.nbytes, n, d, it.w, A, B, 0, 0) == 0
+        it.plan_host = buf.ctypes.data
+        keep.append(buf)
+    rows, threads = (ctypes.c_int32 * len(shapes))(), ctypes.c_int32(-1)
+    assert lib.conef_randblock_step_tiles(items, len(shapes), A, B, rows, ctypes.byref(threads)) == 0
+    return list(rows), threads.value
+
+
+@pytest.mark.parametrize("shapes,ss,rows", [
+    # tiles of two and three rows stay, alone, next to others and next to a tensor of a few rows
+    ([(2600, 650)] * 3, 0.1, [2, 2, 2]), ([(2600, 650)] * 3 + [(10, 650)], 0.1, [2, 2, 2, 1]),
+    ([(2600, 650)] * 2 + [(64, 27)], 0.4, [2, 2, 1]), ([(2100, 700)], 0.1, [2]), ([(2600, 1000)] * 2 + [(10, 1000)], 0.2, [2, 2, 1]),
+    ([(16000, 1500)], 0.1, [3]), ([(16001, 1301)], 0.4, [3]), ([(3400, 800)], 0.1, [3]), ([(2048, 2502)], 0.1, [2]),
+    # one row a tile: four rows where they leave 400 tiles, else two, and one where there are few rows
+    ([(1600, 1500)] * 2, 0.1, [4, 4]), ([(1500, 1500)] * 2, 0.1, [2, 2]), ([(700, 1500)], 0.1, [2]), ([(255, 1500)], 0.1, [1]), ([(640, 5760)], 0.2, [1]),
+    ([(2000, 5000)], 0.1, [4]),
+    # nothing taller where most values are in tiles of little LDS, and nothing on row lists at all
+    ([(1600, 640), (2048, 600), (9000, 300), (300, 9000)], 0.1, [1, 2, 8, 1]), ([(5, 200_000)], 0.1, [0])])
+def test_rows_of_the_tiles_of_a_random_block_step(shapes, ss, rows):
+    got, threads = step_tiles(shapes, ss)
+    assert got == rows
+    assert threads in ((256, 512, 1024) if any(rows) else (0,))
