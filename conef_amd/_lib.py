@@ -60,6 +60,7 @@ SIGNATURES = {
     "conef_psgd_round_f32": [_P, _I32, _I32, _I32, _F32, _F32, _F32, _I32, _I32, _P, _I64, _P],
     "conef_psgd_round_small_fits": [_P, _I32, _I32, _I32, _I32, _I32],
     "conef_psgd_round_wide_sketch_fits": [_P, _I32, _I32, _I32],
+    "conef_psgd_round_wide_sketch_form": [_P, _I32, _I32, _I32, _P, _P, _P],
     "conef_psgd_round_in_order": [],
     "conef_psgd_round_small_workspace_bytes": [_P, _I32],
     "conef_psgd_round_small_f32": [_P, _I32, _I32, _I32, _F32, _F32, _F32, _I32, _I32, _P, _I64, _P],

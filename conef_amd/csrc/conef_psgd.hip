@@ -3884,6 +3884,14 @@ psgd_lin_residual_batch_kernel(PsgdBatch<RowlistResidualItem<RP, true, true, T>>
 // end of a bucket's round was 27 us (six factors [1024,32]) or 34 (with a [4096,32]) behind a residual launch of 20 to 25; the
 // two together take 37 and 35.5, and 89 where [30522,1024] took 76 + 27 with narrower workgroups.  (Without the raised
 // priority the second kind took 52; its chain of short steps otherwise waits its turn between streaming waves.)
+//
+// Several workgroups of one matrix wait for each other's records, here with as much LDS as the launch's largest tile, which can be a
+// whole CU's, and with rounds of other buckets on other streams.  That ends because they wait for nobody else: they are neighbours at
+// the front of the grid, started in order before any tile, so that all of a matrix are on the machine, or go to the next places that
+// come free, and everything else that runs (tiles, the workgroups of other matrices once all of theirs run) comes to its end by
+// itself.  Places may only run out where waiting workgroups hold them all: at most 15 a launch, of 256 at one a CU, which
+// wide_next keeps to.  (The waits are bounded besides.)
+constexpr int kWideNextWgsPerItem = 16;
 struct WideNext {
     const float* q[kPsgdBatchMax];       // row-major
     const float* qp[kPsgdBatchMax];      // by pieces
@@ -4627,35 +4635,50 @@ int wide_sketch_residual(const PaddedRound& pr, const WideTiles& tiles, const st
     return look.empty() ? go(std::false_type()) : go(std::true_type());
 }
 
-// The workgroups that orthogonalise pr's new Q factors into q_next along with the last launch; *threads: that launch's,
-// which may have to be wider for them.  wgs 0: none, they are a launch of their own.
-inline WideNext wide_next(const PaddedRound& pr, float* const* q_next, float eps, const void* workspace, int64_t workspace_bytes, int* threads)
+// Which workgroups orthogonalise the Q factors of pr along with the last launch; *threads: that launch's, which may have to be
+// wider for them.  wgs 0: none, they are a launch of their own.
+inline WideNext wide_next_split(const PaddedRound& pr, int* threads)
 {
     WideNext g = {};
-    g.eps = eps;
+    if (!gs_wide_by_columns(pr)) return g;
     g.count = (int)pr.items.size();
     int64_t tallest = 0;
     for (int k = 0; k < g.count; ++k) {
         const ConefPsgdItem& it = pr.items[(size_t)k];
-        g.q[k] = it.q;
-        g.qp[k] = pr.qi[(size_t)k];
-        g.dst[k] = q_next[k];
         g.rows[k] = (int)it.m;
         g.gram = g.gram || gsg_wants(it.q, it.m, it.r);
-        if (!aligned16(q_next[k])) return WideNext{};
         tallest = std::max(tallest, it.m);
     }
+    if (!g.gram && tallest > wide_next_rows(pr.rp, 1024)) return WideNext{};
     int wgs = 0;
     for (int k = 0; k < g.count; ++k) {
         int w = 1;
         if (g.gram) gsg_split(g.rows[k], pr.rp, &g.slab[k], &w);
+        if (w > kWideNextWgsPerItem) return WideNext{};
         g.first[k] = wgs;
         wgs += w;
     }
     g.first[g.count] = wgs;
-    if (g.gram ? !gsg_workspace_ok(workspace, workspace_bytes) : tallest > wide_next_rows(pr.rp, 1024)) return WideNext{};
     if (!g.gram && tallest > wide_next_rows(pr.rp, *threads)) *threads = 512;
     g.wgs = wgs;
+    return g;
+}
+
+// The same for a round: the new Q factors into q_next.
+inline WideNext wide_next(const PaddedRound& pr, float* const* q_next, float eps, const void* workspace, int64_t workspace_bytes, int* threads)
+{
+    for (size_t k = 0; k < pr.items.size(); ++k)
+        if (!aligned16(q_next[k])) return WideNext{};
+    int wider = *threads;
+    WideNext g = wide_next_split(pr, &wider);
+    if (!g.wgs || (g.gram && !gsg_workspace_ok(workspace, workspace_bytes))) return WideNext{};
+    *threads = wider;
+    g.eps = eps;
+    for (int k = 0; k < g.count; ++k) {
+        g.q[k] = pr.items[(size_t)k].q;
+        g.qp[k] = pr.qi[(size_t)k];
+        g.dst[k] = q_next[k];
+    }
     return g;
 }
 
@@ -5009,7 +5032,7 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
             if (rc == CONEF_OK && made && want_next) *made = by_quads && by_fold ? 5 : 1;
             return rc;
         }
-        if (want_next && wide_sketch && columns) next = wide_next(pr, q_next, eps, workspace, workspace_bytes, &tiles.threads);
+        if (want_next && wide_sketch) next = wide_next(pr, q_next, eps, workspace, workspace_bytes, &tiles.threads);
         // the column kernels work in place: the fix launch leaves the new Q in q_next as well
         if (want_next && rp > 8 && columns && !next.wgs)
             for (int k = 0; k < count; ++k) pr.qt[(size_t)k] = q_next[k];
@@ -5119,6 +5142,25 @@ int conef_psgd_round_wide_sketch_fits(const ConefPsgdItem* items, int32_t count,
         if (!item_ok(items[k])) return 0;
     WideTiles tiles;
     return wide_sketch_tiles(items, count, &tiles) && wide_sketch_plans(items, count, a, b) ? 1 : 0;
+}
+
+// How such a round runs, on the host alone.
+int conef_psgd_round_wide_sketch_form(const ConefPsgdItem* items, int32_t count, int32_t a, int32_t b, int32_t* threads, int32_t* groups,
+                                      int32_t* riders)
+{
+    if (!threads || !groups || !riders || conef_psgd_round_wide_sketch_fits(items, count, a, b) != 1) return CONEF_ERR_INVALID;
+    WideTiles tiles;
+    LookMqShape look;
+    if (!wide_sketch_tiles(items, count, &tiles)) return CONEF_ERR_INVALID;
+    PaddedRound pr;
+    pr.items = at_rank_bound(items, count);
+    pr.rp = rank_bound(items[0].r);
+    pr.padded = pr.rp != items[0].r;
+    const WideNext next = wide_next_split(pr, &tiles.threads);
+    *threads = tiles.threads;
+    *groups = look_pays(items, count) && look_mq_shape(items, count, &look) ? look.groups : 0;
+    *riders = !next.wgs ? 0 : next.gram ? 2 : 1;
+    return CONEF_OK;
 }
 
 // Whether conef_psgd_round_small_f32 takes this bucket: at most 24 matrices of at most 73728 elements

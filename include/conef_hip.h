@@ -381,6 +381,12 @@ int conef_psgd_round_small_f32(const ConefPsgdItem* items, int32_t count, int32_
  * columns or more, a row-list plan per sketch for the seeds a and b, no CONEF_ROUND_DEFER=0), 0 where pqt_mode 3 with room for dense residuals is the
  * faster call.  conef_psgd_batch_workspace_bytes covers what it needs. */
 int conef_psgd_round_wide_sketch_fits(const ConefPsgdItem* items, int32_t count, int32_t a, int32_t b);
+/* How such a round runs (host only; CONEF_ERR_INVALID where the answer above is 0): threads of a workgroup of the last
+ * launch; column splits of the first product that share a workgroup, or 0 where X = M + error is laid out first; and who
+ * orthogonalises the Q factors for the next round with CONEF_ROUND_MAKE_NEXT - a workgroup of the last launch a matrix (1), several
+ * a matrix (2), launches of their own (0). */
+int conef_psgd_round_wide_sketch_form(const ConefPsgdItem* items, int32_t count, int32_t a, int32_t b, int32_t* threads,
+                                      int32_t* groups, int32_t* riders);
 /* 1 where CONEF_ROUND_DEFER=0 asks for the reference's order of steps as things stand, else 0: a caller that keeps the
  * answer of conef_psgd_round_wide_sketch_fits asks again where this has changed. */
 int conef_psgd_round_in_order(void);

@@ -272,3 +272,36 @@ def test_rows_of_the_tiles_of_a_random_block_step(shapes, ss, rows):
     got, threads = step_tiles(shapes, ss)
     assert got == rows
     assert threads in ((256, 512, 1024) if any(rows) else (0,))
+
+
+def wide_sketch_form(shapes, rank, ss):
+    """(threads of the last launch, column splits of the first product that share a workgroup, kind of riders) of a round with
+    a sketched error over a bucket of these gradients, or None where the residuals go out dense."""
+    import ctypes
+
+    import torch
+    from conef_amd import _lib, _psgd_engine
+    from conef_amd.powerSGD_hook import PowerSGDState
+    lib = _lib.load()
+    grads = [torch.empty(s, device="meta") for s in shapes]
+    state = PowerSGDState(None, matrix_approximation_rank=rank)
+    work = [(n, m, r) for n, m, r in ((g.shape[0], g[0].numel(), min(g.shape[0], g[0].numel(), rank)) for g in grads if g.dim() > 1)
+            if _psgd_engine.should_compress(n, m, r, state.min_compression_rate)[0]]
+    items, keep = (_lib.PsgdItem * len(work))(), []
+    for it, (n, m, r) in zip(items, work):
+        it.x = it.p = it.q = it.cs = it.plan_dev = 256
+        it.n, it.m, it.r, it.w = n, m, r, max(1, int(ss * m))
+        buf = np.zeros(lib.conef_plan_bytes(n, m, it.w, 0, 0), np.uint8)
+        assert lib.conef_plan_build_host(buf.ctypes.data, buf.nbytes, n, m, it.w, A, B, 0, 0) == 0
+        it.plan_host = buf.ctypes.data
+        keep.append(buf)
+    out = [ctypes.c_int32(-1) for _ in range(3)]
+    rc = lib.conef_psgd_round_wide_sketch_form(items, len(work), A, B, *[ctypes.byref(v) for v in out])
+    assert (rc == 0) == (lib.conef_psgd_round_wide_sketch_fits(items, len(work), A, B) == 1)
+    return tuple(v.value for v in out) if rc == 0 else None
+
+
+@pytest.mark.parametrize("rank,height,riders", [(16, 1024, 1), (16, 1025, 2), (32, 1025, 2), (32, 4096, 2), (32, 4097, 0), (17, 1025, 0)])
+def test_workgroups_of_a_factor_that_wait_for_each_other_are_few(rank, height, riders):
+    """At most sixteen, in the last launch of a round: a taller factor is a launch of its own."""
+    assert wide_sketch_form([(3000, height)], rank, 0.1)[2] == riders
