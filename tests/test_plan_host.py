@@ -301,6 +301,17 @@ def wide_sketch_form(shapes, rank, ss):
     return tuple(v.value for v in out) if rc == 0 else None
 
 
+def test_sketched_rounds_of_the_gpu_tests_cover_every_form():
+    """Threads of the last launch, column splits that share a workgroup of the first product, and workgroups that
+    orthogonalise Q along with the last launch: all that there are, at rank 16 and at rank 32."""
+    from test_gpu_hooks import WIDE_SKETCH_ROUNDS
+    for rank in (16, 32):
+        forms = [wide_sketch_form(shapes, rank, ss) for shapes, ss in WIDE_SKETCH_ROUNDS]
+        assert None not in forms
+        assert {g for _, g, _ in forms} == {0, 1, 2, 4}
+        assert {(t, r) for t, _, r in forms} >= {(t, r) for t in (256, 512, 1024) for r in (1, 2)} | {(1024, 0)}
+
+
 @pytest.mark.parametrize("rank,height,riders", [(16, 1024, 1), (16, 1025, 2), (32, 1025, 2), (32, 4096, 2), (32, 4097, 0), (17, 1025, 0)])
 def test_workgroups_of_a_factor_that_wait_for_each_other_are_few(rank, height, riders):
     """At most sixteen, in the last launch of a round: a taller factor is a launch of its own."""
