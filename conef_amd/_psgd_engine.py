@@ -640,10 +640,11 @@ def _issue_round(state, plan, lib, errs, error_mode, mode1, mode3, alpha, beta3,
     elif count and state.warm_start and plan.env_ahead and (state.matrix_approximation_rank > 8 or mode3 in (0, 1, 2)):
         # The bucket's next round starts by orthogonalising the Q factors this round leaves
         # (powerSGD_hook.py:496-497): a few workgroups and an idle machine.  It is done at the end of
-        # this round instead, into a second buffer: by workgroups of the last launch at ranks up to 8, by
-        # short launches of their own above (CONEF_ROUND_AHEAD=0 keeps the reference's order, for
-        # comparisons).  Where the buckets do not run side by side (one stream), those launches go to a side
-        # stream, which the bucket's next round waits for, and overlap the next bucket.
+        # this round instead, into a second buffer: by workgroups of the last launch at ranks up to 8 and, with
+        # a sketched error, at ranks 16 and 32, by short launches of their own else (CONEF_ROUND_AHEAD=0 keeps the
+        # reference's order, for comparisons).  Where the buckets do not run side by side (one stream), the
+        # launches above rank 8 go to a side stream, which the bucket's next round waits for, and overlap the
+        # next bucket.
         if plan.q_next is None:
             # row-major factors first, then the same in the order the kernels of ranks up to 8 load them, and behind
             # that what a round with a sketched error keeps (CONEF_ROUND_NEXT_FOLD)

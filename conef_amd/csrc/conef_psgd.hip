@@ -3150,7 +3150,8 @@ inline int64_t mtp_batch_layout(const ConefPsgdItem* items, int count, std::vect
 // `gram` (deferred orthogonalisation of P): count workgroups in front of the launch solve the
 // matrices' Gram systems, and the row-slab partials are left for the caller's fix launch instead
 // of being added here; outs[k] then says where item k's raw Q is ([slabs][m][r]).  Only for a batch
-// that is one launch of this kernel (one rank below 16, all items 16-byte shaped or none).
+// that is one launch (padded_round: matrices of one rank, rows of four columns or more).  `look` (with `gram`, ranks 9 to 32): X is
+// formed from M and the cells.
 int mtp_batch(const ConefPsgdItem* items, int count, void* workspace, int64_t workspace_bytes, hipStream_t s,
               const GramTask* gram = nullptr, std::vector<MtpRaw>* outs = nullptr, const std::vector<MfmaLook>* look = nullptr)
 {
@@ -3564,13 +3565,14 @@ int mq_batch_any(const ConefPsgdItem* items, int count, int mode, float alpha, i
 // 100.8 and 110.7.
 inline bool sums_with_shares(int splits, int rp) { return rp == 16 || splits <= 16; }
 
-// The same for ranks 9 to 32, whose products run on the matrix cores: the shares of P^T P come
-// from a short launch of their own, which also adds the column splits of P, the systems ride in the second product's
-// first launch, and the fix launch is the wide form.  `mq_mode` as in conef_psgd_mq_batch_f32.
-// look: X = M + alpha * unsketch(cs) is formed where it is read, and M stays as it is.
+// P = X Q with X formed from M and the cells (below, with the rounds it belongs to)
 int look_mq(const std::vector<ConefPsgdItem>& items, float alpha, void* workspace, int64_t workspace_bytes, hipStream_t s,
             std::vector<MtpRaw>* outs);
 
+// The two products with the orthogonalisation of P deferred (round_products_deferred) for ranks 9 to 32, which run on the matrix
+// cores: the shares of P^T P come from a short launch of their own, which also adds the column splits of P, the systems ride in the
+// second product's first launch, and the fix launch is the wide form.  `mq_mode` as in conef_psgd_mq_batch_f32.
+// look: X = M + alpha * unsketch(cs) is formed where it is read, and M stays as it is.
 int round_products_deferred_mfma(const PaddedRound& pr, int r, float* const* q_in, int mq_mode, float alpha, float eps,
                                  int32_t a, int32_t b, void* workspace, int64_t workspace_bytes, hipStream_t s,
                                  const std::vector<MfmaLook>* look = nullptr)
@@ -5090,10 +5092,9 @@ int conef_psgd_round_ahead_f32(const ConefPsgdItem* items, int32_t count, int32_
                        ahead.count ? &ahead : nullptr, &used, deferred && rp <= 8 ? &pr.qi : nullptr);
     if (rc != CONEF_OK) return rc;
     if (want_next && deferred && rp > 8) {
-        if (next.wgs) {
-        } else if (gs_wide_by_columns(pr)) {
+        if (!next.wgs && gs_wide_by_columns(pr)) {
             rc = orthogonalise_by_columns(pr, items[0].r, q_next, eps, workspace, workspace_bytes, hs);
-        } else {
+        } else if (!next.wgs) {
             std::vector<const float*> src;
             for (int k = 0; k < count; ++k) src.push_back(its[k].q);
             rc = orthogonalise_by_gram_wide(pr, items[0].r, src, q_next, eps, workspace, hs);

@@ -346,8 +346,10 @@ int conef_psgd_sketch_update_batch_f32(const ConefPsgdItem* items, int32_t count
  * conef_psgd_pqt_batch_f32 (pqt_mode 0..2; 3 = mode 1, then conef_psgd_sketch_update_batch_f32 on the
  * residuals it wrote to err).  Replaces powerSGD_hook.py:473-564 at world size 1 (the all-reduces in
  * between are the identity there).  The launches are those of the separate calls, in the same order, only with
- * CONEF_ROUND_DEFER=0 in the environment: the orthogonalisation of P is deferred else where the batch allows, and a
- * sketched error (mq_mode 2, pqt_mode 2) up to rank 8 is added to the products instead of to the matrices. */
+ * CONEF_ROUND_DEFER=0 in the environment: the orthogonalisation of P is deferred else where the batch allows.  A sketched
+ * error (mq_mode 2, pqt_mode 2) is then, where that is faster, added to the products instead of to the matrices up to rank 8, and
+ * at ranks 9 to 32, where conef_psgd_round_wide_sketch_fits, looked up by whatever reads the matrices, the residual being
+ * sketched by the launch that forms it. */
 int conef_psgd_round_f32(const ConefPsgdItem* items, int32_t count, int32_t mq_mode, int32_t pqt_mode, float alpha,
                          float beta, float eps, int32_t a, int32_t b, void* workspace, int64_t workspace_bytes,
                          void* stream);
@@ -377,9 +379,11 @@ int conef_psgd_round_small_f32(const ConefPsgdItem* items, int32_t count, int32_
                                void* stream);
 
 /* Whether a round with a sketched error (mq_mode 2) at ranks 9 to 32 is to be asked for with pqt_mode 2: 1 where the
- * residuals of these matrices are sketched by the launch that forms them (at most 24 matrices of one rank, rows of four
- * columns or more, a row-list plan per sketch for the seeds a and b, no CONEF_ROUND_DEFER=0), 0 where pqt_mode 3 with room for dense residuals is the
- * faster call.  conef_psgd_batch_workspace_bytes covers what it needs. */
+ * residuals of these matrices are sketched by the launch that forms them, 0 where pqt_mode 3 with room for dense residuals
+ * is the faster call.  1 takes at most 24 matrices of one rank, rows of four columns or more, a row-list plan per sketch for the
+ * seeds a and b, a row with its lists and cells within a workgroup's LDS, and no CONEF_ROUND_DEFER=0; and it is a matter of speed,
+ * hence of the shapes: half of the values at least in matrices that go by three rows a workgroup or more.
+ * conef_psgd_batch_workspace_bytes covers what it needs. */
 int conef_psgd_round_wide_sketch_fits(const ConefPsgdItem* items, int32_t count, int32_t a, int32_t b);
 /* How such a round runs (host only; CONEF_ERR_INVALID where the answer above is 0): threads of a workgroup of the last
  * launch; column splits of the first product that share a workgroup, or 0 where X = M + error is laid out first; and who
