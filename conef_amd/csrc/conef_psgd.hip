@@ -3887,13 +3887,16 @@ psgd_lin_residual_batch_kernel(PsgdBatch<RowlistResidualItem<RP, true, true, T>>
 // two together take 37 and 35.5, and 89 where [30522,1024] took 76 + 27 with narrower workgroups.  (Without the raised
 // priority the second kind took 52; its chain of short steps otherwise waits its turn between streaming waves.)
 //
-// Several workgroups of one matrix wait for each other's records, here with as much LDS as the launch's largest tile, which can be a
-// whole CU's, and with rounds of other buckets on other streams.  That ends because they wait for nobody else: they are neighbours at
-// the front of the grid, started in order before any tile, so that all of a matrix are on the machine, or go to the next places that
-// come free, and everything else that runs (tiles, the workgroups of other matrices once all of theirs run) comes to its end by
-// itself.  Places may only run out where waiting workgroups hold them all: at most 15 a launch, of 256 at one a CU, which
-// wide_next keeps to.  (The waits are bounded besides.)
-constexpr int kWideNextWgsPerItem = 16;
+// Several workgroups of one matrix wait for each other's records, here with as much LDS as the launch's largest tile and with rounds
+// of other buckets on other streams, at most four launches side by side (HIP's hardware queues).  Each XCD starts its share of a
+// grid, every eighth workgroup, in order and without regard to the others', so a workgroup may wait for one that an XCD has yet to
+// find a place for: among waiting workgroups, as all else (tiles come behind them) ends by itself.  It finds one.  Workgroups of up
+// to 512 threads (half a CU's LDS and registers at most: wide_sketch_tiles) are up to 16 an XCD a launch, those of 1024, which may
+// want a CU each, are kept to 7.  One of the former lacks a place where a waiting one of 1024 threads or two others are: on
+// 7 k + (16 (4 - k) - 1) / 2 of 32 CUs at most, k of the launches having 1024 threads, which is 31.  So launches of the former kind
+// end, and after them 28 CUs at most are held.  conef_gs_gram.h's own launch (16 an XCD, a quarter of a CU's LDS) counts as one of the
+// former.  (The waits are bounded besides.)
+constexpr int wide_next_wgs(int threads) { return threads <= 512 ? kGsgMaxWgs : 56; }
 struct WideNext {
     const float* q[kPsgdBatchMax];       // row-major
     const float* qp[kPsgdBatchMax];      // by pieces
@@ -4656,10 +4659,10 @@ inline WideNext wide_next_split(const PaddedRound& pr, int* threads)
     for (int k = 0; k < g.count; ++k) {
         int w = 1;
         if (g.gram) gsg_split(g.rows[k], pr.rp, &g.slab[k], &w);
-        if (w > kWideNextWgsPerItem) return WideNext{};
         g.first[k] = wgs;
         wgs += w;
     }
+    if (g.gram && wgs > wide_next_wgs(*threads)) return WideNext{};
     g.first[g.count] = wgs;
     if (!g.gram && tallest > wide_next_rows(pr.rp, *threads)) *threads = 512;
     g.wgs = wgs;

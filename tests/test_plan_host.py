@@ -312,7 +312,13 @@ def test_sketched_rounds_of_the_gpu_tests_cover_every_form():
         assert {(t, r) for t, _, r in forms} >= {(t, r) for t in (256, 512, 1024) for r in (1, 2)} | {(1024, 0)}
 
 
-@pytest.mark.parametrize("rank,height,riders", [(16, 1024, 1), (16, 1025, 2), (32, 1025, 2), (32, 4096, 2), (32, 4097, 0), (17, 1025, 0)])
-def test_workgroups_of_a_factor_that_wait_for_each_other_are_few(rank, height, riders):
-    """At most sixteen, in the last launch of a round: a taller factor is a launch of its own."""
-    assert wide_sketch_form([(3000, height)], rank, 0.1)[2] == riders
+@pytest.mark.parametrize("rank,heights,ss,riders", [
+    (16, [1024], 0.1, 1), (16, [1025], 0.1, 2), (32, [1025], 0.1, 2), (32, [4096], 0.1, 2), (32, [4097], 0.1, 0), (17, [1025], 0.1, 0),
+    (32, [4096, 4096, 4096, 2048], 0.5, 2), (32, [4096, 4096, 4096, 2049], 0.5, 0), (16, [4096] * 7, 0.5, 2),
+    (16, [4096] * 7 + [512], 0.5, 0), (32, [2048] * 16, 0.1, 2), (32, [2048] * 16 + [128], 0.1, 0), (16, [1024] * 9, 0.5, 1)])
+def test_workgroups_of_a_factor_that_wait_for_each_other_are_few(rank, heights, ss, riders):
+    """At most 56 in a last launch of 1024 threads, 128 in one of fewer: with more, or a taller factor, they are a launch of
+    their own."""
+    threads, _, got = wide_sketch_form([(3000, h) for h in heights], rank, ss)
+    assert got == riders
+    assert (threads == 1024) == (ss == 0.5) or riders == 1 or len(heights) == 1
