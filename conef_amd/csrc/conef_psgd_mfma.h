@@ -74,7 +74,10 @@ psgd_mfma_mq_body(float* __restrict__ x, const float* __restrict__ err, const fl
     // products, so a wave always has a stage's worth of loads in flight while it multiplies.  A stage is the wave's, so its
     // place is a scalar; a whole one has no columns to leave out.  (Whole blocks with an address and a test a load: an encoder
     // of 1024 with dense errors 571 us a step at rank 16, now 557, the LSTM 554 and 536, WRN-16-5 95.5 and 90.4.)
-    constexpr int U = 2;
+    // MODE 2 looks up cells between its loads and its products and stays with whole blocks: half blocks and these, us, rank 32,
+    // with a plan and without, sketches of a tenth: [30522,1024] 101.2 and 89.4, 110.7 and 106.9; [33278,650] 88.5 and 76.9, 103.7
+    // and 87.9; [17000,1001] 78.1 and 73.7, 81.8 and 79.1 ([100000,130], a block and two columns, 36.5 and 40.4, 47.7 and 55.8).
+    constexpr int U = MODE == 2 ? 4 : 2;
     struct Stage {
         float xv[U][4], ev[MODE == 1 ? U : 1][4], qv[U][4];
         uint32_t pk[MODE == 2 ? U : 1][4];
@@ -156,7 +159,7 @@ psgd_mfma_mq_body(float* __restrict__ x, const float* __restrict__ err, const fl
         Stage s0, s1;
         load(s0, cb);
         while (true) {
-            const int nb = cb + kStep, hb = cb + 8 * U;
+            const int nb = cb + (MODE == 2 ? 2 : 1) * kStep, hb = cb + (MODE == 2 ? kStep : 8 * U);
             if (hb < c_end) load(s1, hb);
             compute(s0, cb);
             if (nb < c_end) load(s0, nb);
