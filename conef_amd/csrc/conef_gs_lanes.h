@@ -343,20 +343,37 @@ __device__ __forceinline__ void gsw_store_columns(float* __restrict__ a, int row
     }
 }
 
-// The r column steps on columns in registers (v[cc][t]: row lane + 64 t of column w * CW + cc); piv: two pivot columns in LDS.
+// gsw_publish_column for column `own` of a wave's CW.
+template <int RPT, int CW, int C = 0>
+__device__ __forceinline__ void gsw_publish_own(float (&v)[CW][RPT], int own, float* pb, float eps)
+{
+    if (CW == 1 || own == C) {
+        gsw_publish_column<RPT>(v[C], pb, eps);
+    } else if constexpr (C + 1 < CW) {
+        gsw_publish_own<RPT, CW, C + 1>(v, own, pb, eps);
+    }
+}
+
+// The r column steps on columns in registers (cols[cc][t]: row lane + 64 t of column w * CW + cc); piv: two pivot columns in LDS.
 // PRIO: the waves' priority when they come and go.
 template <int RP, int RPT, int CW, int PRIO = 0>
-__device__ __forceinline__ void gsw_steps(float (&v)[CW][RPT], float* piv, int lane, int w, float eps)
+__device__ __forceinline__ void gsw_steps(float (&cols)[CW][RPT], float* piv, int lane, int w, float eps)
 {
+    // A copy: the compiler sees the caller's columns through their address here and makes one of what the branches on a column's
+    // number do, which then moves columns about in every step.  Rank 32, us, so and by address: [64] 17.7 and 22.7, [512] 20.2 and
+    // 21.4, [1024] 26.0 and 28.8.
+    float v[CW][RPT];
+#pragma unroll
+    for (int cc = 0; cc < CW; ++cc)
+#pragma unroll
+        for (int t = 0; t < RPT; ++t) v[cc][t] = cols[cc][t];
     constexpr int PS = RPT + 4;      // a lane's slice of the pivot column: 16-byte accesses of 16 lanes then cover all banks once
     const int col0 = w * CW;
     // Normalises this wave's column i and publishes it: a lane's slice of the column is RPT words,
     // written and read 16 bytes at a time.
     auto publish = [&](int i) __attribute__((always_inline)) {
         float* pb = piv + (i & 1) * (64 * PS) + lane * PS;
-#pragma unroll
-        for (int cc = 0; cc < CW; ++cc)
-            if (i % CW == cc) gsw_publish_column<RPT>(v[cc], pb, eps);
+        gsw_publish_own<RPT, CW>(v, i % CW, pb, eps);
     };
 
     if (w == 0) publish(0);
@@ -410,6 +427,10 @@ __device__ __forceinline__ void gsw_steps(float (&v)[CW][RPT], float* piv, int l
         }
         __syncthreads();
     }
+#pragma unroll
+    for (int cc = 0; cc < CW; ++cc)
+#pragma unroll
+        for (int t = 0; t < RPT; ++t) cols[cc][t] = v[cc][t];
 }
 
 // The same steps on a workgroup of T threads among others: the [rows, RP] matrix by pieces of four columns (qp:
